@@ -3,16 +3,13 @@
 // Replaces FlashGS render<BX,BY> (csrc/cuda_rasterizer/render.cu:549-576): zero the ranges,
 // identifyTileRanges (:9-31) and renderCUDA (:199-547).
 //
-// Blend layout: one wave64 owns one tile.  A tile is made of 16x16-pixel sub-tiles (1 for 16x16,
-// 2 for 32x16, 4 for 32x32); lane l shades the 2x2 pixel quad at (2*(l%8), 2*(l/8)) of every
-// sub-tile.  Gaussians are staged 32 at a time: the staging lanes tabulate the two one-dimensional
-// parts of the exponent over the tile's columns and rows in LDS, while the loads of the following
-// batch are already in flight; the wave then walks the batch, every lane reading the table
-// entries of its own columns and rows.  After every second Gaussian one ballot tests whether all
-// pixels of the tile have T < 1e-4, which is the reference's stop rule (render.cu:394-408).  A
-// workgroup is a single wave, so no workgroup barrier is needed anywhere.  Every kernel exists in
+// Blend layout: one wave64 works on 16x16 pixels, four per lane; a wide tile (32x16, 32x32) is a workgroup
+// of two or four such waves.  Gaussians are taken 16 at a time: their exponents at all pixels come from the
+// matrix unit, while the loads of the following batch are already in flight; then the wave shades its pixels
+// Gaussian by Gaussian.  After every second Gaussian one ballot tests whether all pixels of the tile
+// have T < 1e-4, which is the reference's stop rule (render.cu:394-408).  Every kernel exists in
 // two forms: all fp32, operation for operation the reference's pixel shader (the default), and
-// with the colour sums on the matrix unit four Gaussians at a time (f16 operands, fp32
+// with the colour sums on the matrix unit too, four Gaussians at a time (f16 operands, fp32
 // accumulation), which a caller asks for per call (FGS_BLEND_MATRIX_F16) or per process
 // (fgs_set_colour_sums).
 #include "fgs_internal.h"
@@ -23,6 +20,10 @@
 #include <utility>
 
 namespace fgs {
+
+// v_mul_legacy_f32: a product in which zero times anything, infinity included, is zero
+__device__ float mul_zero_wins(float a, float b) __asm("llvm.amdgcn.fmul.legacy");
+
 namespace {
 
 
@@ -175,23 +176,88 @@ __device__ __forceinline__ uint8_t encode_u8(float x)
     return (uint8_t)v;
 }
 
-// The exponent of a Gaussian at a pixel, q = w + cx dx^2 + cz dy^2 + cy dx dy with (dx, dy) the
-// offset of the pixel from the Gaussian's centre (render.cu:42-45), is split over the tile's own
-// pixel grid.  With (X, Y) the pixel's integer offset from the tile centre and (ex, ey) the
-// Gaussian centre's offset from the tile centre, dx = ex - X, dy = ey - Y and
-//     q = F(X) + G(Y) + cy X Y,
-//     F(X) = (w - cy ex ey) + dx (cx dx + cy ey),      G(Y) = dy (cz dy + cy ex).
-// F and G depend on one coordinate only: for every staged Gaussian they are tabulated once per
-// tile column and row (kFx + kGy values) by the staging lanes, and a lane gets the exponents of
-// its 2x2 quad from two table reads, four additions and four FMAs with its own constants X*Y.
-// All terms are of the magnitude of the exponent itself or of cy*|X|*|Y| with |X|, |Y| <= 16, so
-// nothing is lost against the 2e-3 image tolerance.
-struct Quad {
-    float T[2][2], r[2][2], g[2][2], b[2][2];
+// How a wave shades 16x16 pixels.  Lane l holds a strip of four pixels, (l % 16, 4 (l / 16) + j) for
+// j = 0 .. 3.  The exponent of a Gaussian, q = w + cx dx^2 + cz dy^2 + cy dx dy with (dx, dy) the offset of
+// the pixel from the Gaussian's centre (render.cu:42-45), is a quadratic along the strip, so its
+// weights alpha_j = 2^q_j follow from the value and the slope at the strip's first pixel:
+//     alpha_{j+1} = alpha_j rho_j,   rho_{j+1} = rho_j E,   rho_0 = 2^(q_1 - q_0),   E = 2^(2 cz),
+// two exponentials and five multiplications for four pixels.  (v_exp_f32 takes the vector unit 8
+// cycles a wave, a multiplication 2.)
+//
+// Values and slopes are a matrix product.  With (X, Y) the strip's first pixel relative to the centre
+// of the square and (ex, ey) the Gaussian's centre relative to it,
+//     q_0       = [w + cx ex^2 + cz ey^2 + cy ex ey] + bx X + by Y + cx X^2 + cz Y^2 + cy XY,
+//     q_1 - q_0 = [by + cz] + cy X + 2 cz Y,     bx = -(2 cx ex + cy ey),  by = -(2 cz ey + cy ex),
+// Gaussians x coefficients times {1, X, X^2, Y, Y^2, XY} x strips, and go through the matrix unit, whose
+// bf16 instructions run beside the vector instructions of other waves (its fp32 ones do not: the same
+// product with v_mfma_f32_32x32x2_f32 made a 4K frame 9 % slower).  Nothing is lost by bf16: the
+// coordinates are small whole numbers, a coefficient is the sum of three bf16 numbers of eight bits of its
+// significand each, products are exact and sums are fp32.  A slope is as exact as a value; its error
+// counts up to three times in alpha_3, some 1e-6 of it.
+//
+// v_mfma_f32_32x32x16_bf16 multiplies 32 rows by 32 columns over 16 slots, of which lanes 0-31 supply
+// slots 0-7 and lanes 32-63 slots 8-15, and lane l receives rows 8 i + 4 (l / 32) + j of column l % 32.
+// Rows 8 i + 4 h + j, h = 0, 1, are Gaussian 4 i + j, with its coefficients in the slots of half h only
+// and zeros in the others, and the slots of half h hold the coordinates of the strips of lanes 32 h ..
+// 32 h + 31: so lane l receives all 16 Gaussians, in list order, at its own strip.  Two coefficients of
+// three parts fill six slots of a half; five instructions make 16 values and 16 slopes per lane.
+//
+// The recurrence starts at the strip's first weight, so that one must not be flushed to zero while a
+// later one matters.  With a curvature along the strip in [-3, 0] (preprocess adds 0.3 to the variances,
+// so its curvatures are above -2.41) it is not: where 2^q_0 < 2^-126, no weight of the strip is above
+// 2^-27 of the opacity.  64 Gaussians with one among them that is out of this range (or out of what
+// the parts hold) are blended by evaluating every exponent (walk_plain).
+//
+// What bounds the launch is the vector unit: 25 fp32 instructions at 2 cycles and two exponentials at 8
+// per Gaussian and wave, about 10 cycles of staging and stop tests on top.  Measured: 98 cycles per
+// Gaussian and 16x16 pixels in the middle of a launch.  4K frame of 3M Gaussians 336 -> 280 us, 8K of
+// 8M 762 -> 671, 1080p of 1M 147 -> 138, against a version that took the exponents from per-column and
+// per-row tables in LDS (four exponentials, 32 vector instructions).  (Two waves per 16x16 pixels with
+// two pixels per lane and staging shared over barriers: 357 us on the 4K frame.)
+typedef float float16_t __attribute__((ext_vector_type(16)));
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+
+constexpr int kBatch = 16;                  // Gaussians per matrix product
+constexpr int kChunk = kWave;               // Gaussians staged at a time, one per lane
+constexpr int kStopBelow = 0x38d1b717;      // 0.0001f: a pixel with less transmittance left is opaque
+constexpr int kNeverStop = -2147483647 - 1;
+
+// An fp32 number as the sum of three bf16 numbers: eight bits of the significand each.
+// (Each is the upper half of a float; the bits below are left to high_halves to drop.)
+struct Parts {
+    float hi, mid, lo;
+};
+__device__ __forceinline__ Parts parts_of(float x)
+{
+    Parts p;
+    p.hi = x;
+    p.mid = x - __uint_as_float(__float_as_uint(x) & 0xffff0000u);
+    p.lo = p.mid - __uint_as_float(__float_as_uint(p.mid) & 0xffff0000u);
+    return p;
+}
+
+// the upper halves of two floats, a's in the lower half of the word
+__device__ __forceinline__ float high_halves(float a, float b)
+{
+    return __uint_as_float(__builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u));
+}
+
+// six slots: the parts of two coefficients
+__device__ __forceinline__ float4 slots_of(const Parts& a, const Parts& b)
+{
+    return make_float4(high_halves(a.hi, b.hi), high_halves(a.mid, b.mid), high_halves(a.lo, b.lo), 0.0f);
+}
+
+// What a lane keeps of the 64 x 4 pixels of a wave.
+struct Pixels {
+    float T[4], r[4], g[4], b[4];
 };
 
-constexpr int kBatch = 32;        // Gaussians staged per round: lanes 0-31 tabulate F, lanes 32-63 G
-constexpr int kGroups = kBatch / 4;
+__device__ __forceinline__ void pixel_of(int lane, int j, int* x, int* y)
+{
+    *x = lane & 15;
+    *y = ((lane >> 4) << 2) + j;
+}
 
 // The colour sums C += (alpha T) c are a matrix product, pixels x Gaussians times Gaussians x
 // channels, and go through v_mfma_f32_4x4x4_16b_f16: sixteen independent 4x4 products with an
@@ -199,12 +265,12 @@ constexpr int kGroups = kBatch / 4;
 // pixel, its four f16 values that pixel's weights alpha T for four Gaussians; column j of B is
 // channel j of those Gaussians' colours (the same in every block; column 3 is zero); lane j of the
 // block accumulates, in fp32, channel j of the four lanes' pixels in its four result registers.
-// A lane shades four pixels per sub-tile, so four Gaussians cost it four such instructions where
-// the plain form costs 48 multiply-adds.  Weights and colours are rounded to f16 (to nearest),
-// products and sums are fp32: the colour of a pixel differs from the all-fp32 sum by at most
-// 2^-10 of itself.  The weights are scaled by 2^14 (added to the exponent when it is tabulated,
-// taken out again with the result), which keeps them in f16's normal range down to 4e-9.
-// T itself never leaves fp32.  This form is opt-in (FGS_BLEND_MATRIX_F16); walk_list_fp32 is the default.
+// A lane shades four pixels, so four Gaussians cost it four such instructions where the plain form
+// costs 48 multiply-adds.  Weights and colours are rounded to f16 (to nearest), products and sums
+// are fp32: the colour of a pixel differs from the all-fp32 sum by at most 2^-10 of itself.  The
+// weights are scaled by 2^14 (added to the exponent, taken out again with the result), which keeps
+// them in f16's normal range down to 4e-9.  T itself never leaves fp32.  This form is opt-in
+// (FGS_BLEND_MATRIX_F16); the default forms the sums by fp32 multiply-add, as the reference does.
 typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
 typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
 typedef float float2_t __attribute__((ext_vector_type(2)));
@@ -231,50 +297,6 @@ __device__ __forceinline__ void lds_write(char* p, float v)
     *(volatile __attribute__((address_space(3))) float*)p = v;
 }
 
-// what a lane reads of one staged Gaussian: F at its columns, G at its rows
-template <int SX, int SY>
-struct StagedT {
-    float2 f[SX], g[SY];
-};
-// ... and of a group of four: their cy, and this lane's channel of their colours as four f16
-struct StagedGroup {
-    float4 cy;
-    float2 colour;
-};
-
-// One Gaussian on one quad: the weights alpha T (scaled) of its four pixels, T updated.
-__device__ __forceinline__ void shade_quad(Quad& q, const float xy[2][2], const float2 f, const float2 g, const float cy, float (&w)[4])
-{
-    const float fx[2] = {f.x, f.y}, gy[2] = {g.x, g.y};
-#pragma unroll
-    for (int j = 0; j < 2; j++)
-#pragma unroll
-        for (int i = 0; i < 2; i++) {
-            const float alpha = __builtin_amdgcn_exp2f(__builtin_fmaf(cy, xy[j][i], fx[i] + gy[j]));
-            const float at = alpha * q.T[j][i];
-            q.T[j][i] = __builtin_fmaf(at, -kWeightUnscale, q.T[j][i]);
-            w[2 * j + i] = at;
-        }
-}
-
-// The all-fp32 form (render.cu:40-52 operation for operation): colour sums by multiply-add.
-__device__ __forceinline__ void shade_quad_fp32(Quad& q, const float xy[2][2], const float2 f, const float2 g, const float cy,
-                                                const float4 rgb)
-{
-    const float fx[2] = {f.x, f.y}, gy[2] = {g.x, g.y};
-#pragma unroll
-    for (int j = 0; j < 2; j++)
-#pragma unroll
-        for (int i = 0; i < 2; i++) {
-            const float alpha = __builtin_amdgcn_exp2f(__builtin_fmaf(cy, xy[j][i], fx[i] + gy[j]));
-            const float at = alpha * q.T[j][i];
-            q.r[j][i] += rgb.x * at;
-            q.g[j][i] += rgb.y * at;
-            q.b[j][i] += rgb.z * at;
-            q.T[j][i] -= at;
-        }
-}
-
 __device__ __forceinline__ uint32_t pack_f16(float a, float b)
 {
     const float2_t v = {a, b};
@@ -282,415 +304,388 @@ __device__ __forceinline__ uint32_t pack_f16(float a, float b)
     return __builtin_bit_cast(uint32_t, h);
 }
 
-// Lane-constant part of the walk: where this lane reads the staged records, what it stages.
-template <int SX, int SY>
-struct LaneRole {
-    static constexpr int kFx = 16 * SX, kGy = 16 * SY;
-    static constexpr int kRec = kFx + kGy + 4;  // floats per staged Gaussian: F table, G table; padded so that the
-                                                // staging lanes, one record apart, write to different LDS banks
-    static constexpr int kGroupRec = 12;        // floats per group of four: cy x 4, 4 channels x 4 f16
-    static constexpr int kStage = kBatch * kRec + kGroups * kGroupRec;      // floats of a wave's staging area
-    uint32_t off_f, off_g, off_cy, off_colour;  // byte offsets into the staging area
-    int stage_slot;                             // Gaussian lane%32 of the batch
-    bool stage_g;                               // lanes 0-31 tabulate F, 32-63 G
-    float xy[SX * SY][2][2];                    // X*Y of the quad's pixels, offsets from the tile centre
+// A wave's colour sums: in the lane of the pixel (fp32), or in the layout of the matrix instruction.
+template <bool kFp32>
+struct Sums {
+    float r[4], g[4], b[4];
+};
+template <>
+struct Sums<false> {
+    float4_t acc[4];
+};
 
-    __device__ __forceinline__ void init(int lane)
+// LDS of a wave, in bytes: a record of five times six slots per staged Gaussian and one of zeros behind them,
+// then per Gaussian (r, g, b, E), or with f16 operands its four f16 channels in groups of four
+// Gaussians and E by itself.  (With f16 operands the sums also go back to their pixels through it.)
+constexpr int kRecord = 5 * 16;
+constexpr int kColours = (kChunk + 1) * kRecord;
+constexpr int kRatios = kColours + 8 * kChunk;              // f16 operands only
+constexpr int kStageFloats = (kColours + 16 * kChunk) / 4;
+
+// Lane-constant part of the walk.
+struct LaneRole {
+    int lane;
+    // this lane's columns of the right-hand matrices, two coordinates each: (1, X), (Y, X^2), (Y^2, XY)
+    float right[3];
+    // which record it supplies to the left-hand matrix: Gaussian 4 i + j for row 8 i + 4 h + j of its own
+    // half h, the record of zeros for the rows of the other half
+    int record_at, record_step;
+
+    __device__ __forceinline__ void init(int lane_, float* stage)
     {
-        // lane -> 2x2 quad of every 16x16 sub-tile
-        const int qx = (lane & 7) * 2, qy = (lane >> 3) * 2;
-#pragma unroll
-        for (int s = 0; s < SX * SY; s++) {
-            const int lx = (s % SX) * 16 + qx, ly = (s / SX) * 16 + qy;
-#pragma unroll
-            for (int j = 0; j < 2; j++)
-#pragma unroll
-                for (int i = 0; i < 2; i++) xy[s][j][i] = (float)((lx + i - kFx / 2) * (ly + j - kGy / 2));
-        }
-        // The offsets are held in vector registers (the empty asm hides what the compiler could
-        // know about them) so that every LDS read of the unrolled batch is "register +
-        // immediate": no address arithmetic in the loop.
-        off_f = 4u * (uint32_t)qx; off_g = 4u * (uint32_t)(kFx + qy);
-        off_cy = 4u * (uint32_t)(kBatch * kRec); off_colour = off_cy + 16u + 8u * (uint32_t)(lane & 3);
-        asm volatile("" : "+v"(off_f), "+v"(off_g), "+v"(off_cy), "+v"(off_colour));
-        stage_slot = lane & (kBatch - 1);
-        stage_g = lane >= kBatch;
+        lane = lane_;
+        const float X = (float)((lane & 15) - 8), Y = (float)(4 * (lane >> 4) - 8);
+        right[0] = high_halves(1.0f, X);
+        right[1] = high_halves(Y, X * X);
+        right[2] = high_halves(Y * Y, X * Y);
+        const bool own = (lane >> 5) == ((lane >> 2) & 1);
+        record_at = own ? (((lane >> 1) & 12) | (lane & 3)) * kRecord : kChunk * kRecord;
+        record_step = own ? kBatch * kRecord : 0;
+        if (lane < kRecord / 4) stage[kChunk * (kRecord / 4) + lane] = 0.0f;
     }
 };
 
-__device__ __forceinline__ void clear_quad(Quad& q)
+template <bool kFp32>
+__device__ __forceinline__ void clear(float (&T)[4], Sums<kFp32>& sums)
 {
 #pragma unroll
-    for (int j = 0; j < 2; j++)
-#pragma unroll
-        for (int i = 0; i < 2; i++) {
-            q.T[j][i] = 1.0f;
-            q.r[j][i] = 0.0f; q.g[j][i] = 0.0f; q.b[j][i] = 0.0f;
-        }
+    for (int k = 0; k < 4; k++) {
+        T[k] = 1.0f;
+        if constexpr (kFp32) { sums.r[k] = 0.0f; sums.g[k] = 0.0f; sums.b[k] = 0.0f; }
+        else sums.acc[k] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    }
 }
 
-// One wave blends entries [begin, begin + n) of the sorted list into the quads of the tile whose
-// centre is given, front to back, starting from T = 1 and no colour; begin must be an even
-// distance from the start of the tile's list, so that the pairs are the reference's pairs.
-// Returns true when the walk ended at the tile-wide stop.  s_rec is this wave's staging area of
-// LaneRole::kStage floats.
-template <int SX, int SY>
-__device__ __forceinline__ bool walk_list(
-    const LaneRole<SX, SY>& role, float* s_rec,
-    const uint32_t* __restrict__ point_list, int begin, int n,
-    float centre_x, float centre_y,
-    const float2* __restrict__ points_xy,
-    const float4* __restrict__ rgb_depth,
-    const float4* __restrict__ conic_opacity,
-    Quad (&quad)[SX * SY])
+// Whether all 256 pixels have T < stop_below, by their bits, which order like the numbers (a negative T
+// counts as opaque either way).  Mostly the first comparison settles it.
+__device__ __forceinline__ bool all_stopped(const float (&T)[4], int stop_below)
 {
-    using Staged = StagedT<SX, SY>;
-    using Role = LaneRole<SX, SY>;
-    constexpr int kSub = SX * SY;
-    constexpr int kFx = 16 * SX, kGy = 16 * SY;
-    constexpr int kTab = kFx > kGy ? kFx : kGy;
-    constexpr int kRec = Role::kRec, kGroupRec = Role::kGroupRec;
-    const char* const rec_bytes = reinterpret_cast<const char*>(s_rec);
-    const uint32_t off_f = role.off_f, off_g = role.off_g, off_cy = role.off_cy, off_colour = role.off_colour;
-    const int stage_slot = role.stage_slot;
-    const bool stage_g = role.stage_g;
-    float* const stage_tab = s_rec + stage_slot * kRec + (stage_g ? kFx : 0);
-    float* const stage_group = s_rec + kBatch * kRec + (stage_slot >> 2) * kGroupRec;
-    const int stage_len = stage_g ? kGy : kFx;
-    const int last = begin + n - 1;
+    auto as_int = [](float t) { return (int)__float_as_uint(t); };
+    if (ballot(as_int(T[1]) >= stop_below) != 0) return false;
+    return ballot(max(max(as_int(T[0]), as_int(T[2])), as_int(T[3])) >= stop_below) == 0;
+}
 
-#pragma unroll
-    for (int s = 0; s < kSub; s++) clear_quad(quad[s]);
-    float4_t acc[kSub][4];                  // colour sums in the layout of the matrix instruction
-#pragma unroll
-    for (int s = 0; s < kSub; s++)
-#pragma unroll
-        for (int p = 0; p < 4; p++) acc[s][p] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+__device__ __forceinline__ float clamped_to_f16(float c)          // NaN stays NaN
+{
+    return c > kColourMax ? kColourMax : (c < -kColourMax ? -kColourMax : c);
+}
 
-    // registers hold the batch that is staged next; loads for it overlap the shading of the current one
-    float2 nxy = make_float2(0.f, 0.f);
-    float4 nco = make_float4(0.f, 0.f, 0.f, 0.f), nrgb = make_float4(0.f, 0.f, 0.f, 0.f);
-    // The list index is fetched two batches ahead and the attributes one batch ahead, so that no
-    // wave waits for an index only to start the loads that depend on it.  Positions past the end
-    // of the list are clamped to its last entry: those loads are valid and their result unused.
-    // (Attributes two batches ahead and indices four, in two alternating sets of registers, change
-    // nothing: 4K frame 0.312 ms either way.)
-    uint32_t g_ahead = 0;
-    if (n > 0) {
-        const uint32_t g = point_list[min(begin + stage_slot, last)];
-        g_ahead = point_list[min(begin + kBatch + stage_slot, last)];
-        nxy = points_xy[g]; nco = conic_opacity[g]; nrgb = rgb_depth[g];
+__device__ __forceinline__ void accumulate_f16(Sums<false>& sums, const uint32_t (&packed)[4][2], float2 colours)
+{
+    const half4_t colour = __builtin_bit_cast(half4_t, colours);
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const uint2 a = make_uint2(packed[k][0], packed[k][1]);
+        sums.acc[k] = __builtin_amdgcn_mfma_f32_4x4x4f16(__builtin_bit_cast(half4_t, a), colour, sums.acc[k], 0, 0, 0);
     }
+}
 
-    bool done = false;
-    for (int base = 0; base < n && !done; base += kBatch) {
-        const int cnt = min(kBatch, n - base);
-        __builtin_amdgcn_wave_barrier();
-        {
-            // conic_opacity = (cx, cy, cz, w) in the units of the exponent (see fgs_preprocess).
-            // With e the centre's offset from the first column (row) of the tile, the entry for
-            // column k is con + d (curv d + lin) at d = e - k, evaluated as a polynomial in k.
-            // A slot past the end of the list gets an exponent that makes every weight zero.
-            const bool unused = stage_slot >= cnt;
-            const float ex = nxy.x - centre_x, ey = nxy.y - centre_y;
-            const float e = stage_g ? ey + (float)(kGy / 2) : ex + (float)(kFx / 2);
-            const float curv = unused ? 0.0f : (stage_g ? nco.z : nco.x);
-            const float lin = unused ? 0.0f : nco.y * (stage_g ? ex : ey);
-            // (log2 of the opacity is held below 2 so that no scaled weight leaves f16's range)
-            const float w_log2 = (nco.w > 1.99f ? 1.99f : nco.w) + kWeightScaleLog2;
-            const float con = stage_g ? 0.0f : (unused ? -1.0e30f : w_log2 - (nco.y * ex) * ey);
-            const float c0 = con + e * (curv * e + lin);
-            const float c1 = -(2.0f * curv * e + lin);
-#pragma unroll
-            for (int k = 0; k < kTab; k += 4) {
-                float4 t;
-                float* tv = &t.x;
-#pragma unroll
-                for (int c = 0; c < 4; c++) tv[c] = c0 + (float)(k + c) * (c1 + curv * (float)(k + c));
-                if (k < stage_len) *reinterpret_cast<float4*>(stage_tab + k) = t;
-            }
-            if (stage_g) {
-                stage_group[stage_slot & 3] = unused ? 0.0f : nco.y;
-                _Float16* const colour = reinterpret_cast<_Float16*>(stage_group + 4) + (stage_slot & 3);
-                auto in_range = [&](float c) {          // NaN stays NaN; a slot past the end of the list holds no colour
-                    return unused ? 0.0f : (c > kColourMax ? kColourMax : (c < -kColourMax ? -kColourMax : c));
-                };
-                colour[0] = (_Float16)in_range(nrgb.x);
-                colour[4] = (_Float16)in_range(nrgb.y);
-                colour[8] = (_Float16)in_range(nrgb.z);
-                colour[12] = (_Float16)0.0f;
-            }
-        }
-        __builtin_amdgcn_wave_barrier();
-        nxy = points_xy[g_ahead]; nco = conic_opacity[g_ahead]; nrgb = rgb_depth[g_ahead];
-        g_ahead = point_list[min(begin + base + 2 * kBatch + stage_slot, last)];
-        // Gaussians go in pairs; the tile-wide stop is tested after each pair (render.cu:394-408)
-        // The table reads of a Gaussian are issued before the Gaussian ahead of it is shaded, so
-        // that a wave does not sit out the LDS latency once per Gaussian.
-        auto fetch = [&](int j) {
-            const int rec = j * kRec * 4;
-            Staged r;
-#pragma unroll
-            for (int c = 0; c < SX; c++) r.f[c] = lds_read<float2>(rec_bytes + off_f + rec + c * 64);
-#pragma unroll
-            for (int c = 0; c < SY; c++) r.g[c] = lds_read<float2>(rec_bytes + off_g + rec + c * 64);
-            return r;
-        };
-        auto fetch_group = [&](int g) {
-            StagedGroup r;
-            r.cy = lds_read<float4>(rec_bytes + off_cy + g * kGroupRec * 4);
-            r.colour = lds_read<float2>(rec_bytes + off_colour + g * kGroupRec * 4);
-            return r;
-        };
-        uint32_t packed[kSub][4][2];        // f16 weights of the group's Gaussians 0-1 and 2-3, per pixel
-        float w0[kSub][4], w1[kSub][4];
-        auto shade = [&](const Staged& r, float cy, float (&w)[kSub][4]) {
-#pragma unroll
-            for (int s = 0; s < kSub; s++) shade_quad(quad[s], role.xy[s], r.f[s % SX], r.g[s / SX], cy, w[s]);
-        };
-        auto pack = [&](int half) {
-#pragma unroll
-            for (int s = 0; s < kSub; s++)
-#pragma unroll
-                for (int p = 0; p < 4; p++) packed[s][p][half] = pack_f16(w0[s][p], w1[s][p]);
-        };
-        auto accumulate = [&](const StagedGroup& grp) {
-            const half4_t colour = __builtin_bit_cast(half4_t, grp.colour);
-#pragma unroll
-            for (int s = 0; s < kSub; s++)
-#pragma unroll
-                for (int p = 0; p < 4; p++) {
-                    const uint2 a = make_uint2(packed[s][p][0], packed[s][p][1]);
-                    acc[s][p] = __builtin_amdgcn_mfma_f32_4x4x4f16(__builtin_bit_cast(half4_t, a), colour, acc[s][p], 0, 0, 0);
-                }
-        };
-        auto all_stopped = [&]() {
-            float live = quad[0].T[1][1];           // the largest T of this lane's pixels
-#pragma unroll
-            for (int s = 0; s < kSub; s++) {
-                live = __builtin_fmaxf(__builtin_fmaxf(live, quad[s].T[0][0]), __builtin_fmaxf(quad[s].T[0][1], quad[s].T[1][0]));
-                if (s > 0) live = __builtin_fmaxf(live, quad[s].T[1][1]);
-            }
-            return ballot(!(live < 0.0001f)) == 0;
-        };
-        // written out for the whole batch so that every record offset is an immediate
-#define FGS_GROUP(G)                                                                         \
-        if (4 * (G) >= cnt) break;                                                           \
-        grp = next_grp;                                                                      \
-        next_grp = fetch_group(((G) + 1) % kGroups);    /* past the batch: read and dropped */\
-        second = fetch(4 * (G) + 1);                                                         \
-        shade(first, grp.cy.x, w0);                                                          \
-        first = fetch(4 * (G) + 2);                                                          \
-        shade(second, grp.cy.y, w1);                                                         \
-        pack(0);                                                                             \
-        stop_mid = all_stopped();                                                            \
-        if (!stop_mid) {                                                                     \
-            second = fetch(4 * (G) + 3);                                                     \
-            shade(first, grp.cy.z, w0);                                                      \
-            first = fetch((4 * (G) + 4) % kBatch);                                           \
-            shade(second, grp.cy.w, w1);                                                     \
-            pack(1);                                                                         \
-        } else {                                                                             \
-            _Pragma("unroll") for (int s = 0; s < kSub; s++)                                 \
-                _Pragma("unroll") for (int p = 0; p < 4; p++) packed[s][p][1] = 0u;          \
-        }                                                                                    \
-        accumulate(grp);                                                                     \
-        if (stop_mid || all_stopped()) { done = true; break; }
-        static_assert(kBatch == 32, "the groups below cover a batch of 32");
-        Staged first = fetch(0), second;
-        StagedGroup grp, next_grp = fetch_group(0);
-        bool stop_mid = false;
-        do {
-            FGS_GROUP(0) FGS_GROUP(1) FGS_GROUP(2) FGS_GROUP(3) FGS_GROUP(4) FGS_GROUP(5) FGS_GROUP(6) FGS_GROUP(7)
-        } while (0);
-#undef FGS_GROUP
-    }
-
-    // Lane 4b+j holds channel j of the pixels of lanes 4b .. 4b+3: handed back through the
-    // staging area (a block of 16 x 4 floats per four lanes, padded to 68 so that the stores of
-    // the 32 lanes served together fall into different banks).
-    static_assert(Role::kStage >= 16 * 68, "the staging area holds the 64 x 16 colour sums of a sub-tile");
+// The first cnt of the Gaussians that the lanes hold (lane i: the i-th), with every exponent evaluated as
+// render.cu:42-45 writes it.  Returns how many were walked, ~that when the stop ended it.
+template <bool kFp32>
+__device__ __forceinline__ int walk_plain(float2 xy, float4 co, float4 rgb, int cnt, float left, float top, int stop_below,
+                                                    float (&T)[4], Sums<kFp32>& sums)
+{
     const int lane = lane_id();
+    int x, y;
+    pixel_of(lane, 0, &x, &y);
+    for (int i = 0; i < cnt; i += 2) {
+        uint32_t packed[4][2] = {};
+        float w[2][4] = {};
+        float c[2][3] = {};
 #pragma unroll
-    for (int s = 0; s < kSub; s++) {
-        __builtin_amdgcn_wave_barrier();
-        char* const out = reinterpret_cast<char*>(s_rec) + 4 * ((lane >> 2) * 68 + (lane & 3));
+        for (int half = 0; half < 2; half++) {
+            const int src = i + half;
+            if (src >= cnt) break;
+            const float dx = bcast_f(xy.x, src) - (left + (float)x);
+            const float cx = bcast_f(co.x, src), cy = bcast_f(co.y, src), cz = bcast_f(co.z, src), lw = bcast_f(co.w, src);
+            c[half][0] = bcast_f(rgb.x, src); c[half][1] = bcast_f(rgb.y, src); c[half][2] = bcast_f(rgb.z, src);
 #pragma unroll
-        for (int p = 0; p < 4; p++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) lds_write(out + 4 * (r * 16 + p * 4), acc[s][p][r]);
-        __builtin_amdgcn_wave_barrier();
-        const char* const in = rec_bytes + 4 * ((lane >> 2) * 68 + (lane & 3) * 16);
-#pragma unroll
-        for (int p = 0; p < 4; p++) {
-            const float4 c = lds_read<float4>(in + 16 * p);
-            quad[s].r[p >> 1][p & 1] = c.x * kWeightUnscale;
-            quad[s].g[p >> 1][p & 1] = c.y * kWeightUnscale;
-            quad[s].b[p >> 1][p & 1] = c.z * kWeightUnscale;
+            for (int k = 0; k < 4; k++) {
+                const float dy = bcast_f(xy.y, src) - (top + (float)(y + k));
+                const float q = lw + cx * dx * dx + cz * dy * dy + cy * dx * dy;
+                const float at = __builtin_amdgcn_exp2f(q) * T[k];
+                if constexpr (kFp32) {
+                    sums.r[k] += c[half][0] * at;
+                    sums.g[k] += c[half][1] * at;
+                    sums.b[k] += c[half][2] * at;
+                    T[k] -= at;
+                } else {
+                    T[k] = __builtin_fmaf(at, -kWeightUnscale, T[k]);
+                    w[half][k] = at;
+                }
+            }
         }
+        if constexpr (!kFp32) {
+            // two of the four Gaussians of a matrix instruction; this lane's channel of their colours
+#pragma unroll
+            for (int k = 0; k < 4; k++) packed[k][0] = pack_f16(w[0][k], w[1][k]);
+            const int ch = lane & 3;
+            float a = 0.0f, b = 0.0f;
+#pragma unroll
+            for (int m = 0; m < 3; m++)
+                if (ch == m) { a = clamped_to_f16(c[0][m]); b = clamped_to_f16(c[1][m]); }
+            accumulate_f16(sums, packed, make_float2(__uint_as_float(pack_f16(a, b)), 0.0f));
+        }
+        if (i + 1 < cnt && all_stopped(T, stop_below)) return ~(i + 2);
     }
-    __builtin_amdgcn_wave_barrier();
-    return done;
+    return cnt;
 }
 
-// The same walk with every operation in fp32 (render.cu:40-52 operation for operation): the colour
-// sums are three multiply-adds per pixel, and a staged Gaussian is one record - F table, G table,
-// (cy, red, green, blue) - so a lane reads all it needs of a Gaussian with three LDS reads and
-// nothing is converted, packed or handed between lanes.  Same arguments and result as walk_list.
-template <int SX, int SY>
-__device__ __forceinline__ bool walk_list_fp32(
-    const LaneRole<SX, SY>& role, float* s_rec,
+// One wave blends entries [begin, begin + n) of the sorted list into the 16x16 pixels whose first pixel
+// is (left, top), front to back, on top of T and sums; begin must be an even distance from the start
+// of the tile's list, so that the pairs are the reference's pairs.  The walk ends after the pair behind
+// which all 256 pixels have T < stop_below (render.cu:394-408).  Returns the entries walked, or ~entries
+// when that stop ended the walk.  stage: this wave's kStageFloats of LDS.
+template <bool kFp32>
+__device__ __forceinline__ int walk_list(
+    const LaneRole& role, float* stage,
     const uint32_t* __restrict__ point_list, int begin, int n,
-    float centre_x, float centre_y,
+    float left, float top,
     const float2* __restrict__ points_xy,
     const float4* __restrict__ rgb_depth,
     const float4* __restrict__ conic_opacity,
-    Quad (&quad)[SX * SY])
+    float (&T)[4], Sums<kFp32>& sums, int stop_below = kStopBelow)
 {
-    constexpr int kSub = SX * SY;
-    constexpr int kFx = 16 * SX, kGy = 16 * SY;
-    constexpr int kTab = kFx > kGy ? kFx : kGy;
-    constexpr int kRec = LaneRole<SX, SY>::kRec;        // kFx + kGy + 4: the tables, then (cy, r, g, b)
-    struct Staged {
-        float4 u;
-        float2 f[SX], g[SY];
-    };
-    const char* const rec_bytes = reinterpret_cast<const char*>(s_rec);
-    const uint32_t off_f = role.off_f, off_g = role.off_g;
-    uint32_t off_u = 4u * (uint32_t)(kFx + kGy);
-    asm volatile("" : "+v"(off_u));                     // kept in a vector register: reads are "register + immediate"
-    const int stage_slot = role.stage_slot;
-    const bool stage_g = role.stage_g;
-    float* const stage_tab = s_rec + stage_slot * kRec + (stage_g ? kFx : 0);
-    const int stage_len = stage_g ? kGy : kFx;
     const int last = begin + n - 1;
-
-#pragma unroll
-    for (int s = 0; s < kSub; s++) clear_quad(quad[s]);
-
-    // registers hold the batch that is staged next; the list index is fetched two batches ahead
-    // and the attributes one batch ahead (see walk_list)
-    float2 nxy = make_float2(0.f, 0.f);
-    float4 nco = make_float4(0.f, 0.f, 0.f, 0.f), nrgb = make_float4(0.f, 0.f, 0.f, 0.f);
+    const int lane = role.lane;
+    char* const bytes = reinterpret_cast<char*>(stage);
+    // registers hold the chunk that is staged next; loads for it overlap the shading of the current
+    // one.  The list index is fetched two chunks ahead and the attributes one chunk ahead, so that no
+    // wave waits for an index only to start the loads that depend on it.  Positions past the end of the
+    // list are clamped to its last entry: those loads are valid and their result unused.
+    float2 xy = make_float2(0.f, 0.f);
+    float4 co = make_float4(0.f, 0.f, 0.f, 0.f), rgb = make_float4(0.f, 0.f, 0.f, 0.f);
     uint32_t g_ahead = 0;
     if (n > 0) {
-        const uint32_t g = point_list[min(begin + stage_slot, last)];
-        g_ahead = point_list[min(begin + kBatch + stage_slot, last)];
-        nxy = points_xy[g]; nco = conic_opacity[g]; nrgb = rgb_depth[g];
+        const uint32_t g = point_list[min(begin + lane, last)];
+        g_ahead = point_list[min(begin + kChunk + lane, last)];
+        xy = points_xy[g]; co = conic_opacity[g]; rgb = rgb_depth[g];
     }
 
-    bool done = false;
-    for (int base = 0; base < n && !done; base += kBatch) {
-        const int cnt = min(kBatch, n - base);
+    for (int base = 0; base < n; base += kChunk) {
+        const int cnt = min(kChunk, n - base);
+        // conic_opacity = (cx, cy, cz, w) in the units of the exponent (see fgs_preprocess).  With f16
+        // weights log2 of the opacity is held below 2 so that no scaled weight leaves f16's range.
+        if constexpr (!kFp32) co.w = (co.w > 1.99f ? 1.99f : co.w) + kWeightScaleLog2;
+        const float ex = xy.x - (left + 8.0f), ey = xy.y - (top + 8.0f);
+        const float bx = -__builtin_fmaf(2.0f * co.x, ex, co.y * ey), by = -__builtin_fmaf(2.0f * co.z, ey, co.y * ex);
+        float c = __builtin_fmaf(ex, __builtin_fmaf(co.x, ex, co.y * ey), __builtin_fmaf(co.z * ey, ey, co.w));
+        const bool fits = co.z <= 0.0f && co.z >= -3.0f &&
+                          __builtin_fabsf(c) + __builtin_fabsf(bx) + __builtin_fabsf(by) + __builtin_fabsf(co.x) < 1.0e9f;
+        if (ballot(!fits) != 0) {
+            const int walked = walk_plain<kFp32>(xy, co, rgb, cnt, left, top, stop_below, T, sums);
+            if (walked < 0) return ~(base + ~walked);
+            xy = points_xy[g_ahead]; co = conic_opacity[g_ahead]; rgb = rgb_depth[g_ahead];
+            g_ahead = point_list[min(begin + base + 2 * kChunk + lane, last)];
+            continue;
+        }
+        if (lane >= cnt) c = -1.0e30f;          // a slot past the end of the list: every weight is zero
+        const float ratio = __builtin_amdgcn_exp2f(2.0f * co.z);
         __builtin_amdgcn_wave_barrier();
         {
-            // the entry for column (row) k is con + d (curv d + lin) at d = e - k, as a polynomial in k
-            const float ex = nxy.x - centre_x, ey = nxy.y - centre_y;
-            const float e = stage_g ? ey + (float)(kGy / 2) : ex + (float)(kFx / 2);
-            const float curv = stage_g ? nco.z : nco.x;
-            const float lin = nco.y * (stage_g ? ex : ey);
-            const float con = stage_g ? 0.0f : nco.w - (nco.y * ex) * ey;
-            const float c0 = con + e * (curv * e + lin);
-            const float c1 = -(2.0f * curv * e + lin);
-#pragma unroll
-            for (int k = 0; k < kTab; k += 4) {
-                float4 t;
-                float* tv = &t.x;
-#pragma unroll
-                for (int c = 0; c < 4; c++) tv[c] = c0 + (float)(k + c) * (c1 + curv * (float)(k + c));
-                if (k < stage_len) *reinterpret_cast<float4*>(stage_tab + k) = t;
+            const Parts pcz = parts_of(co.z), pcy = parts_of(co.y);
+            float4* const record = reinterpret_cast<float4*>(bytes + lane * kRecord);
+            record[0] = slots_of(parts_of(c), parts_of(bx));
+            record[1] = slots_of(parts_of(by), parts_of(co.x));
+            record[2] = slots_of(pcz, pcy);
+            record[3] = slots_of(parts_of(by + co.z), pcy);
+            const Parts twice = {2.0f * pcz.hi, 2.0f * pcz.mid, 2.0f * pcz.lo}, none = {0.0f, 0.0f, 0.0f};
+            record[4] = slots_of(twice, none);
+            if constexpr (kFp32) {
+                *reinterpret_cast<float4*>(bytes + kColours + 16 * lane) = make_float4(rgb.x, rgb.y, rgb.z, ratio);
+            } else {
+                _Float16* const colour = reinterpret_cast<_Float16*>(bytes + kColours + 32 * (lane >> 2)) + (lane & 3);
+                const bool unused = lane >= cnt;        // holds no colour
+                colour[0] = (_Float16)(unused ? 0.0f : clamped_to_f16(rgb.x));
+                colour[4] = (_Float16)(unused ? 0.0f : clamped_to_f16(rgb.y));
+                colour[8] = (_Float16)(unused ? 0.0f : clamped_to_f16(rgb.z));
+                colour[12] = (_Float16)0.0f;
+                *reinterpret_cast<float*>(bytes + kRatios + 4 * lane) = ratio;
             }
-            if (stage_g) *reinterpret_cast<float4*>(s_rec + stage_slot * kRec + kFx + kGy) =
-                make_float4(nco.y, nrgb.x, nrgb.y, nrgb.z);
         }
         __builtin_amdgcn_wave_barrier();
-        nxy = points_xy[g_ahead]; nco = conic_opacity[g_ahead]; nrgb = rgb_depth[g_ahead];
-        g_ahead = point_list[min(begin + base + 2 * kBatch + stage_slot, last)];
-        // the reads of a Gaussian are issued before the Gaussian ahead of it is shaded
-        auto fetch = [&](int j) {
-            const int rec = j * kRec * 4;
-            Staged r;
-            r.u = lds_read<float4>(rec_bytes + off_u + rec);
+        xy = points_xy[g_ahead]; co = conic_opacity[g_ahead]; rgb = rgb_depth[g_ahead];
+        g_ahead = point_list[min(begin + base + 2 * kChunk + lane, last)];
+
+        const char* record = bytes + role.record_at;
+        uint32_t colour_off = kColours + (kFp32 ? 0 : 8 * (lane & 3));
+        asm volatile("" : "+v"(colour_off));            // a vector register: LDS addresses are not scalars
+        const char* colour_at = bytes + colour_off;
+        const char* ratio_at = bytes + kRatios;
+#pragma unroll 1
+        for (int from = 0; from < cnt; from += kBatch) {
+            float16_t q, d;
+            {
+                bf16x8_t slots[5], right[3];        // the same two coordinates for the three parts
 #pragma unroll
-            for (int c = 0; c < SX; c++) r.f[c] = lds_read<float2>(rec_bytes + off_f + rec + c * 64);
+                for (int m = 0; m < 3; m++) {
+                    float both = role.right[m];
+                    asm volatile("" : "+v"(both));      // copied here and not kept in three registers throughout
+                    right[m] = __builtin_bit_cast(bf16x8_t, make_float4(both, both, both, 0.0f));
+                }
 #pragma unroll
-            for (int c = 0; c < SY; c++) r.g[c] = lds_read<float2>(rec_bytes + off_g + rec + c * 64);
-            return r;
-        };
-        auto shade = [&](const Staged& r) {
+                for (int m = 0; m < 5; m++) slots[m] = __builtin_bit_cast(bf16x8_t, lds_read<float4>(record + 16 * m));
+                float16_t zero;
 #pragma unroll
-            for (int s = 0; s < kSub; s++)
-                shade_quad_fp32(quad[s], role.xy[s], r.f[s % SX], r.g[s / SX], r.u.x, make_float4(r.u.y, r.u.z, r.u.w, 0.f));
-        };
-        auto all_stopped = [&]() {
-            float live = quad[0].T[1][1];           // the largest T of this lane's pixels
-#pragma unroll
-            for (int s = 0; s < kSub; s++) {
-                live = __builtin_fmaxf(__builtin_fmaxf(live, quad[s].T[0][0]), __builtin_fmaxf(quad[s].T[0][1], quad[s].T[1][0]));
-                if (s > 0) live = __builtin_fmaxf(live, quad[s].T[1][1]);
+                for (int i = 0; i < 16; i++) zero[i] = 0.0f;
+                q = __builtin_amdgcn_mfma_f32_32x32x16_bf16(slots[0], right[0], zero, 0, 0, 0);
+                d = __builtin_amdgcn_mfma_f32_32x32x16_bf16(slots[3], right[0], zero, 0, 0, 0);
+                q = __builtin_amdgcn_mfma_f32_32x32x16_bf16(slots[1], right[1], q, 0, 0, 0);
+                d = __builtin_amdgcn_mfma_f32_32x32x16_bf16(slots[4], right[1], d, 0, 0, 0);
+                q = __builtin_amdgcn_mfma_f32_32x32x16_bf16(slots[2], right[2], q, 0, 0, 0);
             }
-            return ballot(!(live < 0.0001f)) == 0;
-        };
-        // Gaussians go in pairs, the tile-wide stop is tested after each pair (render.cu:394-408);
-        // written out for the whole batch so that every record offset is an immediate
-#define FGS_PAIR(J)                                                                   \
-        if ((J) >= cnt) break;                                                        \
-        second = fetch((J) + 1);                                                      \
-        shade(first);                                                                 \
-        if ((J) + 1 >= cnt) break;              /* odd tail (render.cu:486-487) */    \
-        first = fetch(((J) + 2) % kBatch);      /* past the batch: read and dropped */\
-        shade(second);                                                                \
-        if (all_stopped()) { done = true; break; }
-        static_assert(kBatch == 32, "the pairs below cover a batch of 32");
-        Staged first = fetch(0), second;
-        do {
-            FGS_PAIR(0) FGS_PAIR(2) FGS_PAIR(4) FGS_PAIR(6) FGS_PAIR(8) FGS_PAIR(10) FGS_PAIR(12) FGS_PAIR(14)
-            FGS_PAIR(16) FGS_PAIR(18) FGS_PAIR(20) FGS_PAIR(22) FGS_PAIR(24) FGS_PAIR(26) FGS_PAIR(28) FGS_PAIR(30)
-        } while (0);
+            const int left_over = cnt - from;
+            int upto;
+            bool stopped = false;
+            // the weights of Gaussian j of the batch along the strip
+            auto weights = [&](int j, float E, float (&alpha)[4]) {
+                alpha[0] = __builtin_amdgcn_exp2f(q[j]);
+                float rho = __builtin_amdgcn_exp2f(d[j]);
+                // (zero times anything is zero here: a slope beyond the range of fp32 belongs to a value of zero)
+                alpha[1] = mul_zero_wins(alpha[0], rho); rho *= E;
+                alpha[2] = mul_zero_wins(alpha[1], rho); rho *= E;
+                alpha[3] = mul_zero_wins(alpha[2], rho);
+            };
+            if constexpr (kFp32) {
+                // render.cu:40-52, operation for operation
+                auto shade = [&](int j, const float4& u) {
+                    float alpha[4];
+                    weights(j, u.w, alpha);
+#pragma unroll
+                    for (int k = 0; k < 4; k++) {
+                        const float at = alpha[k] * T[k];
+                        sums.r[k] += u.x * at;
+                        sums.g[k] += u.y * at;
+                        sums.b[k] += u.z * at;
+                        T[k] -= at;
+                    }
+                };
+                auto colour = [&](int j) { return lds_read<float4>(colour_at + 16 * j); };
+                // Gaussians go in pairs, the stop is tested after each pair; a colour is read while the
+                // Gaussian ahead of it is shaded.  The second half of an odd tail (render.cu:486-487) is an
+                // unused slot: its weights are zero.
+#define FGS_PAIR(J)                                                                    \
+                second = colour((J) + 1);                                                  \
+                shade((J), first);                                                         \
+                first = colour(((J) + 2) % kBatch);     /* past the batch: read and dropped */ \
+                shade((J) + 1, second);                                                    \
+                upto = (J) + 2;                                                            \
+                if (upto >= left_over || all_stopped(T, stop_below)) break;
+                static_assert(kBatch == 16, "the pairs below cover a batch of 16");
+                float4 first = colour(0), second;
+                do {
+                    FGS_PAIR(0) FGS_PAIR(2) FGS_PAIR(4) FGS_PAIR(6) FGS_PAIR(8) FGS_PAIR(10) FGS_PAIR(12) FGS_PAIR(14)
+                } while (0);
 #undef FGS_PAIR
+            } else {
+                uint32_t packed[4][2];        // f16 weights of the group's Gaussians 0-1 and 2-3, per pixel
+                float w0[4], w1[4];
+                auto shade = [&](int j, float E, float (&w)[4]) {
+                    float alpha[4];
+                    weights(j, E, alpha);
+#pragma unroll
+                    for (int k = 0; k < 4; k++) {
+                        w[k] = alpha[k] * T[k];
+                        T[k] = __builtin_fmaf(w[k], -kWeightUnscale, T[k]);
+                    }
+                };
+                auto pack = [&](int half) {
+#pragma unroll
+                    for (int k = 0; k < 4; k++) packed[k][half] = pack_f16(w0[k], w1[k]);
+                };
+                // a stop behind the first pair of a group: the second pair's weights are zero
+#define FGS_GROUP(G)                                                                         \
+                {                                                                            \
+                    const float2 colours = lds_read<float2>(colour_at + 32 * (G));           \
+                    const float4 E = lds_read<float4>(ratio_at + 16 * (G));                  \
+                    shade(4 * (G), E.x, w0);                                                 \
+                    shade(4 * (G) + 1, E.y, w1);                                             \
+                    pack(0);                                                                 \
+                    upto = 4 * (G) + 2;                                                      \
+                    _Pragma("unroll") for (int k = 0; k < 4; k++) packed[k][1] = 0u;         \
+                    if (upto < left_over && !all_stopped(T, stop_below)) {                   \
+                        shade(4 * (G) + 2, E.z, w0);                                         \
+                        shade(4 * (G) + 3, E.w, w1);                                         \
+                        pack(1);                                                             \
+                        upto = 4 * (G) + 4;                                                  \
+                    }                                                                        \
+                    accumulate_f16(sums, packed, colours);                                   \
+                    if (upto >= left_over || all_stopped(T, stop_below)) break;              \
+                }
+                do { FGS_GROUP(0) FGS_GROUP(1) FGS_GROUP(2) FGS_GROUP(3) } while (0);
+#undef FGS_GROUP
+            }
+            stopped = all_stopped(T, stop_below);
+            if (stopped) return ~min(base + from + upto, n);
+            record += role.record_step;
+            colour_at += kFp32 ? 16 * kBatch : 8 * kBatch;
+            ratio_at += 4 * kBatch;
+        }
     }
-    __builtin_amdgcn_wave_barrier();
-    return done;
+    return n;
 }
 
-template <int SX, int SY, bool kFp32, typename... Args>
-__device__ __forceinline__ bool walk(Args&&... args)
+// The wave's pixels out of T and the colour sums.
+template <bool kFp32>
+__device__ __forceinline__ void finish(float* stage, const float (&T)[4], const Sums<kFp32>& sums, Pixels& px)
 {
-    if constexpr (kFp32) return walk_list_fp32<SX, SY>(args...);
-    else return walk_list<SX, SY>(args...);
+#pragma unroll
+    for (int k = 0; k < 4; k++) px.T[k] = T[k];
+    if constexpr (kFp32) {
+#pragma unroll
+        for (int k = 0; k < 4; k++) { px.r[k] = sums.r[k]; px.g[k] = sums.g[k]; px.b[k] = sums.b[k]; }
+    } else {
+        // Lane 4b+j holds channel j of the pixels of lanes 4b .. 4b+3: handed back through the
+        // staging area (a block of 16 x 4 floats per four lanes, padded to 68 so that the stores of
+        // the 32 lanes served together fall into different banks).
+        const int lane = lane_id();
+        __builtin_amdgcn_wave_barrier();
+        char* const out = reinterpret_cast<char*>(stage) + 4 * ((lane >> 2) * 68 + (lane & 3));
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) lds_write(out + 4 * (r * 16 + k * 4), sums.acc[k][r]);
+        __builtin_amdgcn_wave_barrier();
+        const char* const in = reinterpret_cast<const char*>(stage) + 4 * ((lane >> 2) * 68 + (lane & 3) * 16);
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const float4 c = lds_read<float4>(in + 16 * k);
+            px.r[k] = c.x * kWeightUnscale;
+            px.g[k] = c.y * kWeightUnscale;
+            px.b[k] = c.z * kWeightUnscale;
+        }
+        __builtin_amdgcn_wave_barrier();
+    }
 }
 
-// render.cu:59-73
-template <int SX, int SY>
-__device__ __forceinline__ void write_tile(
-    int lane, int tile_x, int tile_y, int width, int height, const Quad (&quad)[SX * SY],
+// render.cu:59-73; (left, top): first pixel of the wave's 16x16 square
+__device__ __forceinline__ void write_square(
+    int lane, int left, int top, int width, int height, const Pixels& px,
     float bg_r, float bg_g, float bg_b, uint8_t* __restrict__ out_u8, float* __restrict__ out_f32)
 {
-    const int qx = (lane & 7) * 2, qy = (lane >> 3) * 2;
 #pragma unroll
-    for (int s = 0; s < SX * SY; s++)
-#pragma unroll
-        for (int j = 0; j < 2; j++)
-#pragma unroll
-            for (int i = 0; i < 2; i++) {
-                const int x = tile_x * 16 * SX + (s % SX) * 16 + qx + i, y = tile_y * 16 * SY + (s / SX) * 16 + qy + j;
-                if (x < width && y < height) {
-                    const size_t pid = (size_t)width * y + x;
-                    float t = quad[s].T[j][i];
-                    if (t < 0.0001f) t = 0.0f;
-                    const float r = quad[s].r[j][i] + t * bg_r, g = quad[s].g[j][i] + t * bg_g, b = quad[s].b[j][i] + t * bg_b;
-                    if (out_u8) {
-                        out_u8[3 * pid + 0] = encode_u8(r);
-                        out_u8[3 * pid + 1] = encode_u8(g);
-                        out_u8[3 * pid + 2] = encode_u8(b);
-                    }
-                    if (out_f32) {
-                        out_f32[3 * pid + 0] = r;
-                        out_f32[3 * pid + 1] = g;
-                        out_f32[3 * pid + 2] = b;
-                    }
-                }
+    for (int k = 0; k < 4; k++) {
+        int x, y;
+        pixel_of(lane, k, &x, &y);
+        x += left; y += top;
+        if (x < width && y < height) {
+            const size_t pid = (size_t)width * y + x;
+            float t = px.T[k];
+            if (t < 0.0001f) t = 0.0f;
+            const float r = px.r[k] + t * bg_r, g = px.g[k] + t * bg_g, b = px.b[k] + t * bg_b;
+            if (out_u8) {
+                out_u8[3 * pid + 0] = encode_u8(r);
+                out_u8[3 * pid + 1] = encode_u8(g);
+                out_u8[3 * pid + 2] = encode_u8(b);
             }
+            if (out_f32) {
+                out_f32[3 * pid + 0] = r;
+                out_f32[3 * pid + 1] = g;
+                out_f32[3 * pid + 2] = b;
+            }
+        }
+    }
 }
 
 // Position in the launch -> tile.  The hardware deals consecutive workgroups out to the 8 XCDs in
@@ -708,25 +703,42 @@ __device__ __forceinline__ bool tile_of_position(int group, int tiles_x, int til
     return *tile_x < tiles_x && *tile_y < tiles_y;
 }
 
-template <int SX, int SY, bool kFp32>
-__device__ __forceinline__ void blend_tile(
-    const int2* __restrict__ ranges,
-    const uint32_t* __restrict__ point_list,
-    int width, int height, int tiles_x, int tiles_y,
-    const float2* __restrict__ points_xy,
-    const float4* __restrict__ rgb_depth,
-    const float4* __restrict__ conic_opacity,
-    float bg_r, float bg_g, float bg_b,
-    uint8_t* __restrict__ out_u8,
-    float* __restrict__ out_f32)
-{
-    constexpr int kSub = SX * SY;              // 16x16 sub-tiles per tile = quads per lane
-    constexpr int kFx = 16 * SX, kGy = 16 * SY;
-    __shared__ __align__(16) float s_rec[LaneRole<SX, SY>::kStage];
+#define FGS_BLEND_PARAMS                                                                         \
+    const int2* __restrict__ ranges, const uint32_t* __restrict__ point_list,                   \
+    int width, int height, int tiles_x, int tiles_y,                                            \
+    const float2* __restrict__ points_xy, const float4* __restrict__ rgb_depth,                 \
+    const float4* __restrict__ conic_opacity, float bg_r, float bg_g, float bg_b,               \
+    uint8_t* __restrict__ out_u8, float* __restrict__ out_f32
 
-    const int lane = threadIdx.x;
+template <bool kFp32>
+constexpr int kBlendWaves = kFp32 ? 5 : 4;       // resident waves per SIMD
+
+// One workgroup per tile, one wave per 16x16 square of it (1 for 16x16 tiles, 2 for 32x16, 4 for
+// 32x32); the waves of a wide tile walk the same list and find its lines in their CU's cache.  (One
+// wave for a whole 32x32 tile needs 64 registers for its colour sums, leaves two waves per SIMD, and
+// a frame of 3600 such tiles ends with the longest lists on single waves: 1200 us for 1M Gaussians
+// at 2560x1440 against 377 us; 32x16 tiles at 1599x901 384 against 217.)  The stop is the tile's, not the
+// wave's: a wave that finds its own square stopped waits until all have, and those that stopped
+// earlier than the last one walk on to where it did.
+// Resident waves: 5 per SIMD is what 96 registers allow (4: the same time on the largest frames, 3 to 5 %
+// more on the others; 6 spills).
+template <int SX, int SY, bool kFp32>
+__global__ __launch_bounds__(kWave * SX * SY) __attribute__((amdgpu_waves_per_eu(kBlendWaves<kFp32>, kBlendWaves<kFp32>))) void blend_kernel(FGS_BLEND_PARAMS, const uint32_t* __restrict__ tile_order)
+{
+    constexpr int kSquares = SX * SY;
+    __shared__ __align__(16) float s_stage[kSquares][kStageFloats];
+    __shared__ int s_walked[kSquares];
+
+    const int lane = threadIdx.x & (kWave - 1);
+    const int wave = kSquares == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     int tile_x, tile_y;
-    if (!tile_of_position((int)blockIdx.x, tiles_x, tiles_y, &tile_x, &tile_y)) return;
+    if (kSquares > 1 && tile_order) {
+        const int tile = (int)tile_order[blockIdx.x];
+        tile_x = tile % tiles_x;
+        tile_y = tile / tiles_x;
+    } else if (!tile_of_position((int)blockIdx.x, tiles_x, tiles_y, &tile_x, &tile_y)) {
+        return;
+    }
     const int2 range = ranges[tile_y * tiles_x + tile_x];
     const int n = range.y - range.x;
     // A launch ends when its longest list ends, and a wave that shares its SIMD equally with the
@@ -736,48 +748,31 @@ __device__ __forceinline__ void blend_tile(
     else if (n > 512) __builtin_amdgcn_s_setprio(2);
     else if (n > 256) __builtin_amdgcn_s_setprio(1);
 
-    LaneRole<SX, SY> role;
-    role.init(lane);
-    Quad quad[kSub];
+    LaneRole role;
+    role.init(lane, s_stage[wave]);
+    float T[4];
+    Sums<kFp32> sums;
+    clear<kFp32>(T, sums);
+    const int left = (tile_x * SX + wave % SX) * 16, top = (tile_y * SY + wave / SX) * 16;
+    int done = 0, upto = n;
+    int stop_below = kStopBelow;
+    for (;;) {          // once, or for a wave of a wide tile that stopped before the others once more
+        const int walked = walk_list<kFp32>(role, s_stage[wave], point_list, range.x + done, upto - done, (float)left, (float)top,
+                                            points_xy, rgb_depth, conic_opacity, T, sums, stop_below);
+        if (kSquares == 1 || stop_below == kNeverStop) break;
+        done = walked < 0 ? ~walked : walked;
+        if (lane == 0) s_walked[wave] = done;
+        __syncthreads();
+        upto = 0;
 #pragma unroll
-    for (int s = 0; s < kSub; s++) clear_quad(quad[s]);
-    const float centre_x = (float)(tile_x * kFx + kFx / 2), centre_y = (float)(tile_y * kGy + kGy / 2);
-    walk<SX, SY, kFp32>(role, s_rec, point_list, range.x, n, centre_x, centre_y, points_xy, rgb_depth, conic_opacity, quad);
-    write_tile<SX, SY>(lane, tile_x, tile_y, width, height, quad, bg_r, bg_g, bg_b, out_u8, out_f32);
-}
-
-#define FGS_BLEND_PARAMS                                                                         \
-    const int2* __restrict__ ranges, const uint32_t* __restrict__ point_list,                   \
-    int width, int height, int tiles_x, int tiles_y,                                            \
-    const float2* __restrict__ points_xy, const float4* __restrict__ rgb_depth,                 \
-    const float4* __restrict__ conic_opacity, float bg_r, float bg_g, float bg_b,               \
-    uint8_t* __restrict__ out_u8, float* __restrict__ out_f32
-#define FGS_BLEND_ARGS                                                                           \
-    ranges, point_list, width, height, tiles_x, tiles_y, points_xy, rgb_depth, conic_opacity,   \
-    bg_r, bg_g, bg_b, out_u8, out_f32
-
-// Registers are budgeted for 6 resident waves per SIMD on 16x16 tiles, 3 and 2 on the wider ones
-// (their colour sums take 32 and 64 registers).
-template <int SX, int SY>
-constexpr int kFewWaves = SX * SY == 1 ? 4 : SX * SY == 2 ? 3 : 2;
-template <int SX, int SY>
-constexpr int kPlainWaves = SX * SY == 1 ? 6 : kFewWaves<SX, SY>;
-
-template <int SX, int SY, bool kFp32>
-__global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(kPlainWaves<SX, SY>))) void blend_kernel(FGS_BLEND_PARAMS)
-{
-    blend_tile<SX, SY, kFp32>(FGS_BLEND_ARGS);
-}
-
-// The same kernel held to 4 resident waves per SIMD (16 per CU; 3 and 2 for the wider tiles,
-// whose colour sums need more registers).  Every resident wave walks its own tile's list and the
-// lists of the tiles in flight compete for the 4 MB L2 of their XCD: when there are more tiles
-// than the chip holds at once, fewer resident waves mean fewer misses (a 4K frame takes the same
-// time at 4, 5 and 6 waves per SIMD and half as long again at 8).
-template <int SX, int SY, bool kFp32>
-__global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(kFewWaves<SX, SY>, kFewWaves<SX, SY>))) void blend_kernel_few_waves(FGS_BLEND_PARAMS)
-{
-    blend_tile<SX, SY, kFp32>(FGS_BLEND_ARGS);
+        for (int w = 0; w < kSquares; w++) upto = max(upto, s_walked[w]);
+        upto = __builtin_amdgcn_readfirstlane(upto);
+        stop_below = kNeverStop;       // whatever is left of it, to the common end
+        if (done >= upto) break;
+    }
+    Pixels px;
+    finish<kFp32>(s_stage[wave], T, sums, px);
+    write_square(lane, left, top, width, height, px, bg_r, bg_g, bg_b, out_u8, out_f32);
 }
 
 // A frame of few tiles is placed on the chip almost at once, one wave per tile: the launch then
@@ -796,12 +791,11 @@ constexpr int kMinRest = 512;               // a shorter rest is not worth two b
 constexpr int kSharedWaves = 4;
 
 template <bool kFp32>
-__global__ __launch_bounds__(kSharedWaves * kWave) __attribute__((amdgpu_waves_per_eu(6, 6))) void blend_kernel_shared(FGS_BLEND_PARAMS, const uint32_t* __restrict__ tile_order)
+__global__ __launch_bounds__(kSharedWaves * kWave) __attribute__((amdgpu_waves_per_eu(kBlendWaves<kFp32>, kBlendWaves<kFp32>))) void blend_kernel_shared(FGS_BLEND_PARAMS, const uint32_t* __restrict__ tile_order)
 {
-    using Role = LaneRole<1, 1>;
-    __shared__ __align__(16) float s_rec[kSharedWaves][Role::kStage];
+    constexpr int kHandOver = 4 * 4 * kWave;            // a run's result: 4 pixels x 4 floats per lane
+    __shared__ __align__(16) float s_stage[kSharedWaves][kStageFloats > kHandOver ? kStageFloats : kHandOver];
     __shared__ int s_rest[kSharedWaves], s_from[kSharedWaves], s_tile_x[kSharedWaves], s_tile_y[kSharedWaves];
-    static_assert(Role::kStage >= 4 * 4 * kWave, "a run's result (4 pixels x 4 floats per lane) is handed over in the staging area");
 
     const int lane = threadIdx.x & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     // Wave w takes rank g of quarter w of the tiles ranked by list length: the workgroups with
@@ -819,8 +813,8 @@ __global__ __launch_bounds__(kSharedWaves * kWave) __attribute__((amdgpu_waves_p
     const int n = range.y - range.x;
     if (n > 256) __builtin_amdgcn_s_setprio(1);
 
-    Role role;
-    role.init(lane);
+    LaneRole role;
+    role.init(lane, s_stage[wave]);
     if (lane == 0) {
         s_rest[wave] = n;               // job 0 of wave w: the head of its own list, in one run
         s_from[wave] = range.x;
@@ -830,7 +824,7 @@ __global__ __launch_bounds__(kSharedWaves * kWave) __attribute__((amdgpu_waves_p
     __builtin_amdgcn_wave_barrier();    // job 0 reads these back in the same wave; the others after the barrier below
     // job 0: own head; job 1 + v: this wave's run of what is left of tile v.  While a wave blends
     // runs, the result of its own head waits in its private memory, not in registers.
-    Quad part[1];
+    Pixels px;
     volatile float kept[16];
     bool shared_out = false;
     for (int job = 0; job <= kSharedWaves; job++) {
@@ -843,11 +837,14 @@ __global__ __launch_bounds__(kSharedWaves * kWave) __attribute__((amdgpu_waves_p
             skip = min(wave * run, rest);
             count = min(run, rest - skip);
         }
-        clear_quad(part[0]);
-        const bool stopped = walk<1, 1, kFp32>(role, s_rec[wave], point_list, __builtin_amdgcn_readfirstlane(s_from[v]) + skip, count,
-                                             (float)(__builtin_amdgcn_readfirstlane(s_tile_x[v]) * 16 + 8),
-                                             (float)(__builtin_amdgcn_readfirstlane(s_tile_y[v]) * 16 + 8),
-                                             points_xy, rgb_depth, conic_opacity, part);
+        float T[4];
+        Sums<kFp32> sums;
+        clear<kFp32>(T, sums);
+        const bool stopped = walk_list<kFp32>(role, s_stage[wave], point_list, __builtin_amdgcn_readfirstlane(s_from[v]) + skip, count,
+                                                    (float)(__builtin_amdgcn_readfirstlane(s_tile_x[v]) * 16),
+                                                    (float)(__builtin_amdgcn_readfirstlane(s_tile_y[v]) * 16),
+                                                    points_xy, rgb_depth, conic_opacity, T, sums) < 0;
+        finish<kFp32>(s_stage[wave], T, sums, px);
         if (job == 0) {
             if (lane == 0) {
                 s_rest[wave] = (!stopped && n > kOwnShare + kMinRest) ? n - kOwnShare : 0;
@@ -859,16 +856,14 @@ __global__ __launch_bounds__(kSharedWaves * kWave) __attribute__((amdgpu_waves_p
             __builtin_amdgcn_s_setprio(3);
 #pragma unroll
             for (int k = 0; k < 4; k++) {
-                kept[4 * k + 0] = part[0].r[k >> 1][k & 1]; kept[4 * k + 1] = part[0].g[k >> 1][k & 1];
-                kept[4 * k + 2] = part[0].b[k >> 1][k & 1]; kept[4 * k + 3] = part[0].T[k >> 1][k & 1];
+                kept[4 * k + 0] = px.r[k]; kept[4 * k + 1] = px.g[k];
+                kept[4 * k + 2] = px.b[k]; kept[4 * k + 3] = px.T[k];
             }
             continue;
         }
-        float4* const mine = reinterpret_cast<float4*>(s_rec[wave]);
+        float4* const mine = reinterpret_cast<float4*>(s_stage[wave]);
 #pragma unroll
-        for (int k = 0; k < 4; k++)
-            mine[k * kWave + lane] = make_float4(part[0].r[k >> 1][k & 1], part[0].g[k >> 1][k & 1],
-                                                 part[0].b[k >> 1][k & 1], part[0].T[k >> 1][k & 1]);
+        for (int k = 0; k < 4; k++) mine[k * kWave + lane] = make_float4(px.r[k], px.g[k], px.b[k], px.T[k]);
         __syncthreads();
         if (wave == v) {
 #pragma unroll
@@ -876,7 +871,7 @@ __global__ __launch_bounds__(kSharedWaves * kWave) __attribute__((amdgpu_waves_p
                 float r = kept[4 * k + 0], g = kept[4 * k + 1], b = kept[4 * k + 2], t = kept[4 * k + 3];
 #pragma unroll
                 for (int w = 0; w < kSharedWaves; w++) {
-                    const float4 p = reinterpret_cast<const float4*>(s_rec[w])[k * kWave + lane];
+                    const float4 p = reinterpret_cast<const float4*>(s_stage[w])[k * kWave + lane];
                     r += t * p.x; g += t * p.y; b += t * p.z;
                     t *= p.w;
                 }
@@ -888,14 +883,13 @@ __global__ __launch_bounds__(kSharedWaves * kWave) __attribute__((amdgpu_waves_p
     if (shared_out) {
 #pragma unroll
         for (int k = 0; k < 4; k++) {
-            part[0].r[k >> 1][k & 1] = kept[4 * k + 0]; part[0].g[k >> 1][k & 1] = kept[4 * k + 1];
-            part[0].b[k >> 1][k & 1] = kept[4 * k + 2]; part[0].T[k >> 1][k & 1] = kept[4 * k + 3];
+            px.r[k] = kept[4 * k + 0]; px.g[k] = kept[4 * k + 1];
+            px.b[k] = kept[4 * k + 2]; px.T[k] = kept[4 * k + 3];
         }
     }
-    if (active) write_tile<1, 1>(lane, tile_x, tile_y, width, height, part, bg_r, bg_g, bg_b, out_u8, out_f32);
+    if (active) write_square(lane, tile_x * 16, tile_y * 16, width, height, px, bg_r, bg_g, bg_b, out_u8, out_f32);
 }
 #undef FGS_BLEND_PARAMS
-#undef FGS_BLEND_ARGS
 
 // How the colour sums are formed by the entry points that do not say (see fgs_set_colour_sums).
 std::atomic<int> g_colour_sums{FGS_COLOUR_SUMS_FP32};
@@ -921,24 +915,11 @@ int check_tile(int block_x, int block_y, int* sx, int* sy, const char* who)
     return fail(FGS_E_INVALID, "%s: tile %dx%d unsupported (16x16, 32x16, 32x32)", who, block_x, block_y);
 }
 
-// How a frame is blended.  More tiles than the chip holds at 8 waves per SIMD: the variant with
-// fewer resident waves.  A frame of 16x16 tiles that is resident at once: workgroups of four tiles
-// that share out their long lists, which needs the tiles ranked by list length.
-struct BlendShape {
-    int cus;
-    bool few_waves, shared;
-};
-
-int blend_shape(int block_x, int block_y, int tiles_x, int tiles_y, BlendShape* shape)
-{
-    int dev = 0;
-    FGS_HIP_TRY(hipGetDevice(&dev));
-    FGS_HIP_TRY(hipDeviceGetAttribute(&shape->cus, hipDeviceAttributeMultiprocessorCount, dev));
-    const long long num_tiles = (long long)tiles_x * tiles_y;
-    shape->few_waves = num_tiles > 32LL * shape->cus;
-    shape->shared = !shape->few_waves && block_x == 16 && block_y == 16 && num_tiles <= kOrderCap && shape->cus > 0;
-    return FGS_OK;
-}
+// A frame of at most kOrderCap tiles is about resident at once: its tiles are ranked by the length of
+// their lists and the longest start first (16x16 tiles also share out their long lists).  In a
+// larger frame the short lists at any time fill in behind the long ones, and neighbouring tiles
+// finding each other's lines in the L2 counts for more.
+bool is_ranked(int tiles_x, int tiles_y) { return (long long)tiles_x * tiles_y <= kOrderCap; }
 
 // render.cu:556-563: zero the ranges, then mark where each tile starts and ends
 int ranges_impl(int block_x, int block_y, int num_rendered, int width, int height,
@@ -989,27 +970,24 @@ int blend_impl(int block_x, int block_y, int width, int height,
     const long long blocks = (long long)((tiles_x + 7) / 8) * ((tiles_y + 7) / 8);
     const long long groups = (blocks + 7) / 8 * 8 * 64;
     if (groups > 0x7fffffffLL) return fail(FGS_E_INVALID, "%s: image too large", who);
-    const dim3 grid((unsigned)groups);
-    BlendShape shape;
-    rc = blend_shape(block_x, block_y, tiles_x, tiles_y, &shape);
-    if (rc != FGS_OK) return rc;
-    const bool few_waves = shape.few_waves;
-    const bool fp32 = mode == FGS_COLOUR_SUMS_FP32;
-#define FGS_LAUNCH_BLEND(SX, SY)                                                                        \
-    do {                                                                                                \
-        auto kernel = fp32 ? (few_waves ? blend_kernel_few_waves<SX, SY, true> : blend_kernel<SX, SY, true>) \
-                           : (few_waves ? blend_kernel_few_waves<SX, SY, false> : blend_kernel<SX, SY, false>); \
-        hipLaunchKernelGGL(kernel, grid, dim3(kWave), 0, st,                                            \
-                           (const int2*)ranges, values_sorted, width, height, tiles_x, tiles_y,         \
-                           (const float2*)points_xy, (const float4*)rgb_depth, (const float4*)conic_opacity, \
-                           bg[0], bg[1], bg[2], out_u8, out_f32);                                       \
-    } while (0)
-    if (shape.shared) {
-        const int num_tiles = tiles_x * tiles_y;
-        uint32_t* tile_order = nullptr;
+    const int num_tiles = tiles_x * tiles_y;
+    uint32_t* tile_order = nullptr;
+    if (is_ranked(tiles_x, tiles_y)) {
         rc = tile_order_table(st, &tile_order);
         if (rc != FGS_OK) return rc;
         hipLaunchKernelGGL(tile_order_kernel, dim3(1), dim3(1024), 0, st, (const int2*)ranges, num_tiles, tile_order);
+    }
+    const dim3 grid((unsigned)(tile_order ? num_tiles : groups));
+    const bool fp32 = mode == FGS_COLOUR_SUMS_FP32;
+#define FGS_LAUNCH_BLEND(SX, SY)                                                                        \
+    do {                                                                                                \
+        auto kernel = fp32 ? blend_kernel<SX, SY, true> : blend_kernel<SX, SY, false>;                  \
+        hipLaunchKernelGGL(kernel, grid, dim3(kWave * SX * SY), 0, st,                                  \
+                           (const int2*)ranges, values_sorted, width, height, tiles_x, tiles_y,         \
+                           (const float2*)points_xy, (const float4*)rgb_depth, (const float4*)conic_opacity, \
+                           bg[0], bg[1], bg[2], out_u8, out_f32, (const uint32_t*)tile_order);          \
+    } while (0)
+    if (tile_order && sx == 1 && sy == 1) {
         hipLaunchKernelGGL(fp32 ? blend_kernel_shared<true> : blend_kernel_shared<false>, dim3((unsigned)((num_tiles + kSharedWaves - 1) / kSharedWaves)), dim3(kSharedWaves * kWave), 0, st,
                            (const int2*)ranges, values_sorted, width, height, tiles_x, tiles_y,
                            (const float2*)points_xy, (const float4*)rgb_depth, (const float4*)conic_opacity,
@@ -1095,14 +1073,13 @@ extern "C" const char* fgs_blend_kernel_name(int block_x, int block_y, int width
     int sx = 0, sy = 0, mode = 0;
     if (check_tile(block_x, block_y, &sx, &sy, "fgs_blend_kernel_name") != FGS_OK || width <= 0 || height <= 0) return "";
     if (colour_mode(flags, &mode, "fgs_blend_kernel_name") != FGS_OK) return "";
-    BlendShape shape;
-    if (blend_shape(block_x, block_y, (width + block_x - 1) / block_x, (height + block_y - 1) / block_y, &shape) != FGS_OK) return "";
+    const bool ranked = is_ranked((width + block_x - 1) / block_x, (height + block_y - 1) / block_y);
     const bool fp32 = mode == FGS_COLOUR_SUMS_FP32;
-#define FGS_NAME(few, plain) (shape.few_waves ? (fp32 ? few ", true>" : few ", false>") : (fp32 ? plain ", true>" : plain ", false>"))
-    if (shape.shared) return fp32 ? "tile_order_kernel + blend_kernel_shared<true>" : "tile_order_kernel + blend_kernel_shared<false>";
-    if (sx == 1 && sy == 1) return FGS_NAME("blend_kernel_few_waves<1, 1", "blend_kernel<1, 1");
-    if (sx == 2 && sy == 1) return FGS_NAME("blend_kernel_few_waves<2, 1", "blend_kernel<2, 1");
-    return FGS_NAME("blend_kernel_few_waves<2, 2", "blend_kernel<2, 2");
+#define FGS_NAME(ranked_name, name) (ranked ? (fp32 ? "tile_order_kernel + " ranked_name "true>" : "tile_order_kernel + " ranked_name "false>") \
+                                            : (fp32 ? name "true>" : name "false>"))
+    if (sx == 1 && sy == 1) return FGS_NAME("blend_kernel_shared<", "blend_kernel<1, 1, ");
+    if (sx == 2 && sy == 1) return FGS_NAME("blend_kernel<2, 1, ", "blend_kernel<2, 1, ");
+    return FGS_NAME("blend_kernel<2, 2, ", "blend_kernel<2, 2, ");
 #undef FGS_NAME
 }
 

@@ -148,9 +148,9 @@ size_t fgs_get_sort_buffer_size(int num_rendered);
  * scratch that holds the tile ranges afterwards.  bg_color is a host array of 3 floats.
  * All arithmetic is fp32, as in render.cu:40-52, unless the process default was changed with
  * fgs_set_colour_sums (fgs_render_ex / fgs_blend_ex choose per call).
- * A frame of at most 8192 16x16 tiles first ranks its tiles by list length into a table the
+ * A frame of at most 8192 tiles first ranks its tiles by list length into a table the
  * library keeps per (device, stream) (32 KB, allocated on the first such call on that stream),
- * and the rest of a list of more than 768 entries is blended in four runs that each stop on
+ * and with 16x16 tiles the rest of a list of more than 768 entries is blended in four runs that each stop on
  * their own transmittance: the colour can differ from the pair-by-pair walk of
  * render.cu:315-408 by what lies behind T < 1e-4, i.e. by less than 1e-4 of a colour.  Calls on
  * different streams may overlap in time; a stream that is being captured and has no table yet

@@ -831,6 +831,63 @@ def test_colour_sum_modes_per_call_and_by_default(oracle, W, H, block):
         cabi.set_colour_sums(prev)
 
 
+@pytest.mark.parametrize("block", [(16, 16), (32, 16), (32, 32)])
+@pytest.mark.parametrize("flags", ["fp32", "f16"])
+@pytest.mark.parametrize("size", [(96, 70), (4096, 1040)])        # with the tiles ranked by list length and without
+def test_blend_batch_edges_and_conics_beyond_the_recurrence(oracle, block, flags, size):
+    """List lengths around the batch of 16 and the chunk of 64 Gaussians, and conics on both sides of
+    what the recurrence along a pixel strip takes (curvature in [-3, 0]): needles, splats far narrower
+    than a pixel, saddles, centres far outside the tile, an opacity of zero.  One Gaussian out of range
+    sends its 64 through the plain evaluation.  Bound: the colour weights are exact to the exponent's
+    rounding, at most 6 terms of magnitude M with M 2^-24 each, times ln 2; M < 300 for everything that
+    reaches a pixel here, so 1e-4 of a colour per Gaussian at its most and far less on average; with f16
+    operands 2^-10 of the colour on top."""
+    import gpu_pipeline as gp
+    from flashgs_amd import cabi
+    import torch
+    W, H = size
+    gx, gy = (W + block[0] - 1) // block[0], (H + block[1] - 1) // block[1]
+    rng = np.random.default_rng(17)
+    lengths = [0, 1, 2, 3, 15, 16, 17, 31, 33, 63, 64, 65, 79, 127, 128, 129, 200]
+    xy, co, rgbd, ranges, at = [], [], [], np.zeros((gx * gy, 2), np.int32), 0
+    tiles = rng.permutation(gx * gy)[:51]
+    for i, t in enumerate(tiles):
+        n = lengths[i % len(lengths)]
+        tx, ty = t % gx, t // gx
+        c = np.stack([tx * block[0] + rng.uniform(-4, block[0] + 4, n), ty * block[1] + rng.uniform(-4, block[1] + 4, n)], 1)
+        cx, cz = -rng.uniform(0.005, 0.4, n), -rng.uniform(0.005, 0.4, n)
+        cy = rng.uniform(-0.9, 0.9, n) * 2 * np.sqrt(cx * cz)
+        w = np.log2(rng.uniform(0.01, 0.6, n))
+        kind = i // len(lengths)
+        if kind == 1 and n:         # at the edges of the range: sharp along the strip, flat along it
+            cz[::3], cy[::3] = -2.9, 0.0
+            cz[1::3], cy[1::3] = -0.0, 0.0
+        if kind == 2 and n:         # beyond it
+            k = rng.integers(0, n)
+            cz[k], cy[k] = [(-40.0, 0.0), (-3.1, 0.1), (0.0005, 0.0)][i % 3]
+            if n > 2:
+                w[0] = -np.inf
+                c[1] += (300.0, -200.0)
+        xy.append(c); co.append(np.stack([cx, cy, cz, w], 1))
+        rgbd.append(np.concatenate([rng.uniform(0, 1, (n, 3)), rng.uniform(1, 50, (n, 1))], 1))
+        ranges[t] = (at, at + n)
+        at += n
+    xy, co, rgbd = (np.concatenate(a).astype(np.float32) for a in (xy, co, rgbd))
+    vals = np.arange(at, dtype=np.uint32)
+    bg = np.array([0.25, 0.5, 0.75], np.float32)
+    _, ref, _ = oracle.render(W, H, block[0], block[1], xy, rgbd, co, vals, ranges, bg, want_u8=False)
+    out = torch.full((H, W, 3), -1.0, device=gp.DEV, dtype=torch.float32)
+    d = [gp.dev(a) for a in (xy, rgbd, co)]
+    dv, dr = gp.dev(vals.view(np.int32)), gp.dev(ranges)
+    cabi.blend(block[0], block[1], W, H, d[0].data_ptr(), d[1].data_ptr(), d[2].data_ptr(), dv.data_ptr(), dr.data_ptr(), bg,
+               0, out.data_ptr(), torch.cuda.current_stream().cuda_stream,
+               flags=cabi.BLEND_FP32 if flags == "fp32" else cabi.BLEND_MATRIX_F16)
+    torch.cuda.synchronize()
+    err = np.abs(out.cpu().numpy() - ref)
+    assert np.isfinite(err).all()
+    assert err.max() <= (2e-4 if flags == "fp32" else 2e-4 + 2.0 ** -10), "max abs image error %g" % err.max()
+
+
 def test_ranges_kernel_against_searchsorted():
     import gpu_pipeline as gp
     import torch
