@@ -1022,6 +1022,29 @@ def test_sort_segment_size_classes(seg, dense):
     _sort_case(tile, depth.view(np.uint32), W, H, seed=seg)
 
 
+@pytest.mark.parametrize("depths", ["all words", "positive floats", "tiny", "from 0x7ff00000 up"])
+@pytest.mark.parametrize("ascending", [True, False])
+def test_sort_depth_words_of_every_pattern(depths, ascending):
+    """The network of the short segments takes its words as doubles: depth words that make a negative,
+    infinite, denormal or not-a-number double of them, around the widths of the network, ties included."""
+    import gpu_pipeline as gp
+    rng = np.random.default_rng(len(depths) + ascending)
+    lengths = [1, 2, 3, 63, 64, 65, 127, 128, 129, 255, 256, 257, 500, 512, 513, 700, 1023, 1024]
+    lo, hi = {"all words": (0, 1 << 32), "positive floats": (0x3e4ccccd, 0x42c80000), "tiny": (0, 40),
+              "from 0x7ff00000 up": (0x7fefffff, 1 << 32)}[depths]
+    tile = np.repeat(np.arange(len(lengths)), lengths)
+    n = len(tile)
+    depth = rng.integers(lo, hi, n, dtype=np.uint64)
+    depth[rng.random(n) < 0.1] = hi - 1
+    keys = (tile.astype(np.uint64) << np.uint64(32)) | depth
+    vals = np.arange(n, dtype=np.uint32) * np.uint32(7) if ascending else rng.integers(0, 1 << 32, n, dtype=np.uint64).astype(np.uint32)
+    mix = rng.permutation(n) if not ascending else np.arange(n)
+    keys, vals = keys[mix], vals[mix]
+    ks, vs = gp.sort(n, 80, 64, gp.dev(keys.view(np.int64)), gp.dev(vals.view(np.int32)))
+    order = np.argsort(keys, kind="stable")
+    assert np.array_equal(gp.u64(ks), keys[order]) and np.array_equal(gp.u32(vs), vals[order])
+
+
 @pytest.mark.parametrize("ascending", [False, True])
 @pytest.mark.parametrize("W,H", [(1920, 1080), (3840, 2160)])
 def test_sort_every_segment_length_up_to_1100(W, H, ascending):
