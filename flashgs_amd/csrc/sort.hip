@@ -20,10 +20,11 @@
 //     size class.  Up to 1024 pairs one wave holds the segment in registers as 64-bit
 //     words depth << 32 | value (| position where the values of a segment do not ascend) and runs
 //     a bitonic network on them (the result is that of a stable sort by depth); lane exchanges inside a row of 16 lanes are
-//     data-parallel-primitive moves.  Up to 4096 (8 waves) and 8192 pairs (16 waves) a workgroup
-//     runs up to four stable 8-bit counting passes in LDS (in place: the pairs wait in registers
-//     while they are counted), skipping a pass in which all pairs share the digit.  Longer segments, and segments whose keys differ above the sorted bit
-//     range, go through the same passes with the ping-pong copy in HBM instead of LDS.
+//     data-parallel-primitive moves.  Up to 4096 (4 waves), 8192 (8) and 16384 pairs (16) every wave
+//     of a workgroup sorts its part like that and the parts are merged, the steps between two waves
+//     through LDS.  Longer segments, and segments whose keys differ above the sorted bit range, go
+//     through stable 8-bit counting passes with a ping-pong copy in HBM, skipping a pass in which all
+//     pairs share the digit.
 //
 // Bytes moved per pair: 8 (count) + 24 (scatter) per partition pass, 24 for the segment sort:
 // 88 for two partition passes, against 8 + 6 * 24 = 152 for a six-pass LSD sort of 47 bits.
@@ -603,7 +604,8 @@ template <int kWaves, typename KeyT>
 __device__ __forceinline__ bool counting_pass(const KeyT* src_k, const uint32_t* src_v, KeyT* dst_k, uint32_t* dst_v,
                                               int n, int shift, uint32_t (*cnt)[kBins], uint32_t* wave_sum, int* flag)
 {
-    const int tid = threadIdx.x;
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));
     const int lane = tid & (kWave - 1);
     const int wave = tid / kWave;
     const int per = ((n + kWaves - 1) / kWaves + kWave - 1) / kWave * kWave;   // a multiple of 64
@@ -687,201 +689,6 @@ __device__ __forceinline__ bool counting_pass(const KeyT* src_k, const uint32_t*
     return true;
 }
 
-// The same pass over a segment of depth words and values held in LDS, in place: every thread takes
-// its kPer pairs into registers (pair w_lo + it*64 + lane for it < kPer, so a wave still ranks its
-// contiguous part 64 pairs at a time in segment order), and once all of them are counted nobody
-// needs the arrays any more and the ranked pairs go back into them.  Half the LDS of a ping-pong
-// copy, and one read of every pair instead of two.  The counters are 16 bits wide (positions stay
-// below 65536), two to a word, counted with 32-bit atomic additions on the half that is meant.
-template <int kWaves, int kPer>
-__device__ __forceinline__ bool counting_pass_lds(uint32_t* s_k, uint32_t* s_v, int n, int shift,
-                                                  uint16_t (*cnt)[kBins], uint32_t* wave_sum, int* flag)
-{
-    static_assert(kWaves * kWave >= kBins, "one thread per digit in the scan");
-    const int tid = threadIdx.x;
-    const int lane = tid & (kWave - 1);
-    const int wave = tid / kWave;
-    const int per = ((n + kWaves - 1) / kWaves + kWave - 1) / kWave * kWave;   // a multiple of 64, at most 64 * kPer
-    const int w_lo = min(n, wave * per), w_hi = min(n, w_lo + per);
-
-    uint32_t* const cnt_words = (uint32_t*)cnt[wave];
-    cnt_words[lane] = 0;
-    cnt_words[lane + kWave] = 0;
-    if (tid == 0) *flag = 0;
-    __syncthreads();
-    uint32_t k[kPer], v[kPer];
-#pragma unroll
-    for (int it = 0; it < kPer; it++) {
-        const int i = w_lo + it * kWave + lane;
-        k[it] = 0; v[it] = 0;
-        if (i < w_hi) {
-            k[it] = s_k[i];
-            v[it] = s_v[i];
-            const uint32_t d = (k[it] >> shift) & 255u;
-            atomicAdd(&cnt_words[d >> 1], (d & 1u) ? 0x10000u : 1u);
-        }
-    }
-    __syncthreads();
-
-    uint32_t total = 0;
-    if (tid < kBins) {                   // thread t handles digit t
-        for (int w = 0; w < kWaves; w++) {
-            const uint32_t c = cnt[w][tid];
-            cnt[w][tid] = (uint16_t)total;          // offset of wave w inside digit tid
-            total += c;
-        }
-        if (total == (uint32_t)n) *flag = 1;
-        const uint32_t incl = wave_inclusive_sum(total);
-        if (lane == kWave - 1) wave_sum[wave] = incl;
-        total = incl - total;             // exclusive inside this wave's 64 digits
-    }
-    __syncthreads();
-    if (tid < kBins) {
-        uint32_t base = total;
-        for (int w = 0; w < wave; w++) base += wave_sum[w];
-        for (int w = 0; w < kWaves; w++) cnt[w][tid] = (uint16_t)(cnt[w][tid] + base);     // absolute start of (wave, digit)
-    }
-    __syncthreads();
-    if (*flag != 0) return false;        // every pair has the same digit: nothing to move
-
-    // stable ranking, 64 pairs at a time in segment order
-#pragma unroll
-    for (int it = 0; it < kPer; it++) {
-        if (w_lo + it * kWave >= w_hi) break;
-        const bool valid = w_lo + it * kWave + lane < w_hi;
-        const uint32_t d = (k[it] >> shift) & 255u;
-        uint64_t peers = ballot(valid);
-#pragma unroll
-        for (int b = 0; b < 8; b++) {
-            const bool bit = (d >> b) & 1u;
-            const uint64_t with_bit = ballot(bit);
-            peers &= bit ? with_bit : ~with_bit;
-        }
-        const int below = popc_below(peers);
-        uint32_t before = 0;
-        if (valid && below == 0) {
-            before = cnt[wave][d];
-            cnt[wave][d] = (uint16_t)(before + (uint32_t)__popcll(peers));
-        }
-        const int leader = valid ? __ffsll((long long)peers) - 1 : lane;
-        before = (uint32_t)__shfl((int)before, leader);
-        if (valid) {
-            s_k[before + (uint32_t)below] = k[it];
-            s_v[before + (uint32_t)below] = v[it];
-        }
-        __builtin_amdgcn_wave_barrier();
-    }
-    return true;
-}
-
-// Sorts the segment [lo, hi) of tile id v in LDS.  Called by all kWaves waves of a workgroup
-// with the same arguments; hi - lo <= kCap.  A segment whose keys differ above the depth word
-// cannot be rebuilt from depth words: it is flagged (or, without a flag array, left alone) for
-// the general kernel.
-// Returns true when that was the case (nothing is moved then).
-template <int kWaves, int kCap>
-__device__ __forceinline__ bool sort_segment_lds(uint64_t* __restrict__ keys, uint32_t* __restrict__ values,
-                                                 uint32_t v, int lo, int hi, uint32_t* __restrict__ seg_flags,
-                                                 uint32_t* s_k, uint32_t* s_v,
-                                                 uint16_t (*s_cnt)[kBins], uint32_t* s_wave_sum, int* s_flag)
-{
-    static_assert(kCap % (kWaves * kWave) == 0, "every thread holds the same number of pairs");
-    const int tid = threadIdx.x;
-    const int len = hi - lo;
-    const uint32_t upper = (uint32_t)(keys[lo] >> 32);
-    bool mixed = false;
-    if (tid == 0) *s_flag = 0;
-    __syncthreads();
-    for (int i = tid; i < len; i += kWaves * kWave) {
-        const uint64_t k = keys[lo + i];
-        s_k[i] = (uint32_t)k;
-        s_v[i] = values[lo + i];
-        mixed = mixed || (uint32_t)(k >> 32) != upper;
-    }
-    if (mixed) *s_flag = 1;
-    __syncthreads();
-    const bool any_mixed = *s_flag != 0;
-    __syncthreads();                             // the passes reuse the flag
-    if (any_mixed) {
-        if (seg_flags && tid == 0) atomicOr(&seg_flags[v >> 5], 1u << (v & 31));
-        return true;
-    }
-
-#pragma unroll 1
-    for (int shift = 0; shift < 32; shift += 8) {
-        counting_pass_lds<kWaves, kCap / (kWaves * kWave)>(s_k, s_v, len, shift, s_cnt, s_wave_sum, s_flag);
-        __syncthreads();
-    }
-    for (int i = tid; i < len; i += kWaves * kWave) {
-        keys[lo + i] = ((uint64_t)upper << 32) | s_k[i];
-        values[lo + i] = s_v[i];
-    }
-    __syncthreads();
-    return false;
-}
-
-// Segment sort in LDS for one size class: segments with min_len < length <= kCap.
-// With a table of segment starts, workgroup w looks at the kIds tile ids [w*kIds, (w+1)*kIds),
-// one per lane, and sorts those of its class one after the other.  Without a table (more tile ids
-// than the table holds) the grid has one workgroup per tile id and each searches for its bounds.
-template <int kWaves, int kCap, int kIds>
-__global__ __launch_bounds__(kWaves * kWave) void segment_sort_kernel(
-    uint64_t* __restrict__ keys, uint32_t* __restrict__ values, int n, uint32_t tile_mask, int min_len, uint32_t ids,
-    const int* __restrict__ seg_start, uint32_t* __restrict__ seg_flags,
-    const uint32_t* __restrict__ list, const uint32_t* __restrict__ list_count, uint32_t list_cap)
-{
-    __shared__ uint32_t s_k[kCap];
-    __shared__ uint32_t s_v[kCap];
-    __shared__ __align__(4) uint16_t s_cnt[kWaves][kBins];
-    __shared__ uint32_t s_wave_sum[kWaves];
-    __shared__ int s_bounds[2];
-    __shared__ int s_flag;
-    __shared__ uint64_t s_match;
-
-    const int tid = threadIdx.x;
-    const int lane = tid & (kWave - 1);
-
-    if (!seg_start) {
-        const uint32_t v = blockIdx.x;
-        if (tid < kWave) {
-            const int a = wave_lower_bound(keys, n, v, tile_mask);
-            const int b = v == tile_mask ? n : wave_lower_bound(keys, n, v + 1, tile_mask);
-            if (lane == 0) { s_bounds[0] = a; s_bounds[1] = b; }
-        }
-        __syncthreads();
-        const int lo = s_bounds[0], hi = s_bounds[1];
-        if (hi - lo <= min_len || hi - lo > kCap) return;
-        sort_segment_lds<kWaves, kCap>(keys, values, v, lo, hi, seg_flags, s_k, s_v, s_cnt, s_wave_sum, &s_flag);
-        return;
-    }
-
-    if (list) {      // the segments of this class were listed: deal them out round-robin, shard by shard
-        const uint32_t shard = blockIdx.x % kListShards;
-        const uint32_t count = list_count[shard];
-        for (uint32_t i = blockIdx.x / kListShards; i < count; i += gridDim.x / kListShards) {
-            const uint32_t v = list[(size_t)shard * list_cap + i];
-            sort_segment_lds<kWaves, kCap>(keys, values, v, seg_start[v], seg_start[v + 1], seg_flags,
-                                           s_k, s_v, s_cnt, s_wave_sum, &s_flag);
-        }
-        return;
-    }
-
-    const uint32_t first_id = blockIdx.x * (uint32_t)kIds;
-    if (tid < kWave) {
-        const uint32_t v = first_id + (uint32_t)lane;
-        int len = 0;
-        if (lane < kIds && v < ids) len = seg_start[v + 1] - seg_start[v];
-        const uint64_t m = ballot(len > min_len && len <= kCap);
-        if (lane == 0) s_match = m;
-    }
-    __syncthreads();
-    for (uint64_t todo = s_match; todo; todo &= todo - 1) {
-        const uint32_t v = first_id + (uint32_t)(__ffsll((long long)todo) - 1);
-        sort_segment_lds<kWaves, kCap>(keys, values, v, seg_start[v], seg_start[v + 1], seg_flags,
-                                       s_k, s_v, s_cnt, s_wave_sum, &s_flag);
-    }
-}
-
 // x of lane (l ^ kJ).  Within a row of 16 lanes the exchange is a data-parallel-primitive move
 // (no LDS traffic); across rows it goes through the lane crossbar.
 template <int kJ>
@@ -924,6 +731,53 @@ __device__ __forceinline__ void keep_min_negated(uint64_t& a, uint64_t b)       
     asm("v_min_f64 %0, %0, -%1" : "+v"(a) : "v"(b));
 }
 
+// Compare distance j < kT, between slots of a lane; k > 0: slots with t & k descend.
+template <int kT>
+__device__ __forceinline__ void compare_slots(uint64_t (&c)[kT], int j, int k)
+{
+#pragma unroll
+    for (int t = 0; t < kT; t++) {
+        if ((t & j) != 0) continue;
+        const int t2 = t | j;
+        const uint64_t lo = min_word(c[t], c[t2]), hi = max_word(c[t], c[t2]);
+        const bool descends = k > 0 && (t & k) != 0;
+        c[t] = descends ? hi : lo;
+        c[t2] = descends ? lo : hi;
+    }
+}
+
+// Changes the sign a lane's words are held with.
+template <int kT>
+__device__ __forceinline__ void hold(uint64_t (&c)[kT], uint32_t& held, uint32_t sign)
+{
+#pragma unroll
+    for (int t = 0; t < kT; t++) c[t] ^= (uint64_t)(held ^ sign) << 32;
+    held = sign;
+}
+
+// Merges the bitonic runs of width k (k >= kT) of the network below.  run: this lane's sign while its
+// run descends; held: the sign its words are held with, run when this returns.
+template <int kT>
+__device__ __forceinline__ void merge_slots(uint64_t (&c)[kT], int lane, int k, uint32_t run, uint32_t& held)
+{
+#pragma unroll
+    for (int jl = kWave / 2; jl > 0; jl >>= 1) {              // lane distances
+        if (jl * kT >= k) continue;
+        hold(c, held, run ^ ((lane & jl) != 0 ? 0x80000000u : 0u));
+#pragma unroll
+        for (int t = 0; t < kT; t++) {
+            const uint64_t mine = c[t];
+            const uint64_t other = jl == 1 ? from_lane_xor64<1>(mine) : jl == 2 ? from_lane_xor64<2>(mine)
+                                 : jl == 4 ? from_lane_xor64<4>(mine) : jl == 8 ? from_lane_xor64<8>(mine)
+                                 : jl == 16 ? from_lane_xor64<16>(mine) : from_lane_xor64<32>(mine);
+            keep_min_negated(c[t], other);                    // the other lane holds its words with the other sign
+        }
+    }
+    hold(c, held, run);
+#pragma unroll
+    for (int j = kT / 2; j > 0; j >>= 1) compare_slots(c, j, 0);
+}
+
 // The network over kT register slots of every lane, 64 * kT elements, element i in slot i % kT of
 // lane i / kT.  A compare distance below kT pairs two slots of one lane (registers only); a
 // larger one pairs the same slot of two lanes: 21 of the (log n)(log n + 1)/2 exchange steps
@@ -940,53 +794,17 @@ template <int kT>
 __device__ __forceinline__ void bitonic_network(uint64_t (&c)[kT], int lane)
 {
     constexpr int n = kT * kWave;
-    auto in_slots = [&](int j, int k) {       // compare distance j < kT; k > 0: slots with t & k descend
-#pragma unroll
-        for (int t = 0; t < kT; t++) {
-            if ((t & j) != 0) continue;
-            const int t2 = t | j;
-            const uint64_t lo = min_word(c[t], c[t2]), hi = max_word(c[t], c[t2]);
-            const bool descends = k > 0 && (t & k) != 0;
-            c[t] = descends ? hi : lo;
-            c[t2] = descends ? lo : hi;
-        }
-    };
-    auto flip = [&](uint32_t sign) {
-#pragma unroll
-        for (int t = 0; t < kT; t++) c[t] ^= (uint64_t)sign << 32;
-    };
     // runs shorter than a lane's slots: the direction is a matter of the slot
 #pragma unroll
     for (int k = 2; k < kT; k <<= 1)
 #pragma unroll
         for (int j = kT / 2; j > 0; j >>= 1)
-            if (j < k) in_slots(j, k);
+            if (j < k) compare_slots(c, j, k);
     // longer ones: of the lane
-    auto sign_of = [&](int bit) { return (lane & bit) != 0 ? 0x80000000u : 0u; };
     uint32_t held = 0;                          // the sign this lane's words are held with
 #pragma unroll 1
-    for (int k = kT > 1 ? kT : 2; k <= n; k <<= 1) {
-        const uint32_t run = k < n ? sign_of(k / kT) : 0u;        // the last merge ascends everywhere
-#pragma unroll
-        for (int jl = kWave / 2; jl > 0; jl >>= 1) {              // lane distances
-            if (jl * kT >= k) continue;
-            const uint32_t want = run ^ sign_of(jl);
-            flip(held ^ want);
-            held = want;
-#pragma unroll
-            for (int t = 0; t < kT; t++) {
-                const uint64_t mine = c[t];
-                const uint64_t other = jl == 1 ? from_lane_xor64<1>(mine) : jl == 2 ? from_lane_xor64<2>(mine)
-                                     : jl == 4 ? from_lane_xor64<4>(mine) : jl == 8 ? from_lane_xor64<8>(mine)
-                                     : jl == 16 ? from_lane_xor64<16>(mine) : from_lane_xor64<32>(mine);
-                keep_min_negated(c[t], other);                    // the other lane holds its words with the other sign
-            }
-        }
-        flip(held ^ run);
-        held = run;
-#pragma unroll
-        for (int j = kT / 2; j > 0; j >>= 1) in_slots(j, 0);
-    }
+    for (int k = kT > 1 ? kT : 2; k <= n; k <<= 1)
+        merge_slots(c, lane, k, k < n && (lane & (k / kT)) != 0 ? 0x80000000u : 0u, held);   // the last merge ascends everywhere
 }
 
 // Words of LDS a wave needs to sort up to n pairs with the network: one 64-bit word for every
@@ -1122,6 +940,230 @@ __device__ __forceinline__ void sort_segment_bitonic(uint64_t* __restrict__ keys
     else sort_segment_bitonic_of<kT>(keys, values, v, lo, hi, seg_flags, s_w);
 }
 
+// One step of the network between two waves: the wave's words against those of `partner`, in the same
+// slots and lanes or (kMirrored) in reverse order.  Both go through LDS, held with opposite signs; a
+// wave that takes no part only meets the barriers.
+template <int kT, bool kMirrored>
+__device__ __forceinline__ void compare_waves(uint64_t (&c)[kT], int lane, int wave, int partner, bool present, bool takes_part,
+                                              uint32_t& held, uint64_t* s_w)
+{
+    hold(c, held, wave < partner ? 0u : 0x80000000u);
+    if (present) {
+        uint64_t* const to = s_w + wave * (kT * kWave) + lane;
+#pragma unroll
+        for (int t = 0; t < kT; t++) to[t * kWave] = c[t];
+    }
+    __syncthreads();
+    if (takes_part) {
+        const uint64_t* const from = s_w + partner * (kT * kWave) + (kMirrored ? kWave - 1 - lane : lane);
+#pragma unroll
+        for (int t = 0; t < kT; t++) {
+            keep_min_negated(c[t], from[(kMirrored ? kT - 1 - t : t) * kWave]);
+            if (t % 4 == 3) __builtin_amdgcn_sched_barrier(0);       // no more words in registers than that
+        }
+    }
+    __syncthreads();
+}
+
+// Sorts the segment [lo, hi) of tile id v, 64 * kWaves * kUse >= hi - lo, with the network over kUse
+// slots per lane of kWaves waves.  Called by all waves of a workgroup with the same arguments.  s_w: 64 *
+// kWaves * kUse words of LDS; s_seen: one word per wave.  A segment whose keys differ above the depth word is
+// flagged (or, without a flag array, left alone) for the general kernel: returns true then.
+// Every wave sorts 64 * kUse words as above.  Runs are then merged in pairs: the first step compares
+// element i of the lower run with element i from the end of the upper one, the next ones halve the
+// distance, between waves through LDS and inside a wave as above.  All runs ascend, so the words
+// past the end of the segment stay behind it, and waves that hold nothing else have nothing to do.
+// The vector unit bounds it, as it does the network of one wave: 75 steps for 4096 pairs against 55
+// for 1024, and three exchanges through LDS at about twice the cost of a step.  Counting passes in LDS
+// (four of them, each a chain of atomics, a scan over digits and a ranking by ballots) took more than
+// twice as long per pair: 8K frame of 111M pairs 825 -> 475 us for the segments of 1025 .. 4096 pairs
+// and 343 -> 195 for those up to 8192, 179 -> 141 for the longer ones; 4K frame of 8M pairs 49 -> 33,
+// 1080p frame of 1.8M pairs 18.6 -> 13.6.
+template <int kWaves, int kUse>
+__device__ __forceinline__ bool sort_segment_waves_of(uint64_t* __restrict__ keys, uint32_t* __restrict__ values,
+                                                      uint32_t v, int lo, int hi, uint32_t* __restrict__ seg_flags,
+                                                      uint64_t* s_w, uint32_t* s_seen)
+{
+    static_assert(kUse >= 2, "the ranks leave in two halves of a wave's slots");
+    constexpr int kPart = kUse * kWave;                 // words of a wave
+    int lane = threadIdx.x & (kWave - 1);
+    asm volatile("" : "+v"(lane));
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
+    const int len = hi - lo;
+    const int first = wave * kPart;                     // this wave's part of the segment
+    const bool present = first < len;
+    const int mine = len - first;
+    uint64_t c[kUse];
+    uint32_t val[kUse];
+    const uint64_t* const key_at = keys + lo + first + lane;
+    const uint32_t* const value_at = values + lo + first + lane;
+#pragma unroll
+    for (int t = 0; t < kUse; t++) {
+        c[t] = ~0ull;
+        val[t] = ~0u;
+        if (t * kWave + lane < mine) {
+            c[t] = key_at[t * kWave];
+            val[t] = value_at[t * kWave];
+        }
+    }
+    asm volatile("" : "+v"(lane));
+    const uint32_t upper = (uint32_t)(keys[lo] >> 32);
+    const uint32_t behind = mine > kPart ? values[lo + first + kPart] : ~0u;       // the first value of the next wave's part
+    bool mixed = false, other_words = false;
+#pragma unroll
+    for (int t = 0; t < kUse; t++) {
+        const bool valid = t * kWave + lane < mine;
+        mixed = mixed || (valid && (uint32_t)(c[t] >> 32) != upper);
+        other_words = other_words || (valid && (uint32_t)c[t] >= 0x7ff00000u);
+    }
+    asm volatile("" : "+v"(lane));
+#pragma unroll
+    for (int t = 0; t < kUse; t++) {
+        uint32_t next = (uint32_t)__shfl_down((int)val[t], 1);
+        const uint32_t wrap = t + 1 < kUse ? (uint32_t)bcast_i((int)val[t + 1 < kUse ? t + 1 : t], 0) : behind;
+        if (lane == kWave - 1) next = wrap;
+        other_words = other_words || (t * kWave + lane + 1 < mine && next < val[t]);
+        if (t % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+    }
+    const uint32_t seen = (ballot(mixed) ? 1u : 0u) | (ballot(other_words) ? 2u : 0u);
+    if (lane == 0) s_seen[wave] = seen;
+    __syncthreads();
+    uint32_t any = 0;
+#pragma unroll
+    for (int w = 0; w < kWaves; w++) any |= s_seen[w];
+    any = (uint32_t)__builtin_amdgcn_readfirstlane((int)any);
+    if (any & 1u) {
+        if (seg_flags && threadIdx.x == 0) atomicOr(&seg_flags[v >> 5], 1u << (v & 31));
+        __syncthreads();                        // s_seen is written again for the next segment
+        return true;
+    }
+    const bool by_value = any == 0;
+#pragma unroll
+    for (int t = 0; t < kUse; t++) {
+        const uint32_t depth = (uint32_t)c[t], i = (uint32_t)(first + t * kWave + lane);
+        const uint32_t high = by_value ? min(depth, 0x7fefffffu) : depth >> 16, low = by_value ? val[t] : (depth << 16) | i;
+        c[t] = ((uint64_t)high << 32) | low;
+    }
+    if (present) bitonic_network<kUse>(c, lane);
+#pragma unroll 1
+    for (int group = 2; group <= kWaves && (group / 2) * kPart < len; group <<= 1) {      // waves of a merged run
+        int partner = wave ^ (group - 1);
+        uint32_t held = 0;
+        compare_waves<kUse, true>(c, lane, wave, partner, present, present && partner * kPart < len, held, s_w);
+#pragma unroll 1
+        for (int d = group / 4; d > 0; d >>= 1) {
+            partner = wave ^ d;
+            compare_waves<kUse, false>(c, lane, wave, partner, present, present && partner * kPart < len, held, s_w);
+        }
+        if (present) merge_slots(c, lane, kPart, 0u, held);
+    }
+    asm volatile("" : "+v"(lane));
+    // the values of the words that carry positions, before any is overwritten
+#pragma unroll
+    for (int t = 0; t < kUse; t++) {
+        const uint32_t high = (uint32_t)(c[t] >> 32), low = (uint32_t)c[t];
+        uint32_t value = low;
+        if (!by_value && (low & 0xffffu) < (uint32_t)len) value = values[lo + (int)(low & 0xffffu)];
+        c[t] = ((uint64_t)(by_value ? high : (high << 16) | (low >> 16)) << 32) | value;
+        if (t % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+    }
+    if (!by_value) __syncthreads();
+    // back to contiguous stores through this wave's part of the LDS, half of the ranks at a time
+    uint64_t* const s_mine = s_w + first;
+    uint64_t* const key_to = keys + lo + first + lane;
+    uint32_t* const value_to = values + lo + first + lane;
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        __builtin_amdgcn_wave_barrier();
+        if (lane / (kWave / 2) == h) {
+#pragma unroll
+            for (int t = 0; t < kUse; t++) s_mine[staged(lane * kUse + t - h * (kPart / 2))] = c[t];
+        }
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int t = h * (kUse / 2); t < (h + 1) * (kUse / 2); t++) {
+            const int i = t * kWave + lane;
+            if (i < mine) {
+                const uint64_t w = s_mine[staged(i - h * (kPart / 2))];
+                key_to[t * kWave] = ((uint64_t)upper << 32) | (w >> 32);
+                value_to[t * kWave] = (uint32_t)w;
+            }
+        }
+    }
+    __syncthreads();
+    return false;
+}
+
+// The smallest number of slots per lane, from kLeast on, that holds the segment: hi - lo <= kCap.
+template <int kWaves, int kCap, int kLeast>
+__device__ __forceinline__ bool sort_segment_waves(uint64_t* __restrict__ keys, uint32_t* __restrict__ values,
+                                                   uint32_t v, int lo, int hi, uint32_t* __restrict__ seg_flags,
+                                                   uint64_t* s_w, uint32_t* s_seen)
+{
+    constexpr int kMost = kCap / (kWaves * kWave);
+    if constexpr (kLeast < kMost)
+        if (hi - lo > kLeast * kWaves * kWave)
+            return sort_segment_waves<kWaves, kCap, 2 * kLeast>(keys, values, v, lo, hi, seg_flags, s_w, s_seen);
+    return sort_segment_waves_of<kWaves, kLeast>(keys, values, v, lo, hi, seg_flags, s_w, s_seen);
+}
+
+// Segment sort by the waves of a workgroup for one size class: segments with min_len < length <= kCap.
+// With a table of segment starts, workgroup w looks at the kIds tile ids [w*kIds, (w+1)*kIds),
+// one per lane, and sorts those of its class one after the other.  Without a table (more tile ids
+// than the table holds) the grid has one workgroup per tile id and each searches for its bounds.
+template <int kWaves, int kCap, int kLeast, int kIds>
+__global__ __launch_bounds__(kWaves * kWave) void segment_sort_kernel(
+    uint64_t* __restrict__ keys, uint32_t* __restrict__ values, int n, uint32_t tile_mask, int min_len, uint32_t ids,
+    const int* __restrict__ seg_start, uint32_t* __restrict__ seg_flags,
+    const uint32_t* __restrict__ list, const uint32_t* __restrict__ list_count, uint32_t list_cap)
+{
+    __shared__ uint64_t s_w[kCap];
+    __shared__ uint32_t s_seen[kWaves];
+    __shared__ int s_bounds[2];
+    __shared__ uint64_t s_match;
+
+    const int tid = threadIdx.x;
+    const int lane = tid & (kWave - 1);
+
+    if (!seg_start) {
+        const uint32_t v = blockIdx.x;
+        if (tid < kWave) {
+            const int a = wave_lower_bound(keys, n, v, tile_mask);
+            const int b = v == tile_mask ? n : wave_lower_bound(keys, n, v + 1, tile_mask);
+            if (lane == 0) { s_bounds[0] = a; s_bounds[1] = b; }
+        }
+        __syncthreads();
+        const int lo = s_bounds[0], hi = s_bounds[1];
+        if (hi - lo <= min_len || hi - lo > kCap) return;
+        sort_segment_waves<kWaves, kCap, kLeast>(keys, values, v, lo, hi, seg_flags, s_w, s_seen);
+        return;
+    }
+
+    if (list) {      // the segments of this class were listed: deal them out round-robin, shard by shard
+        const uint32_t shard = blockIdx.x % kListShards;
+        const uint32_t count = list_count[shard];
+        for (uint32_t i = blockIdx.x / kListShards; i < count; i += gridDim.x / kListShards) {
+            const uint32_t v = list[(size_t)shard * list_cap + i];
+            sort_segment_waves<kWaves, kCap, kLeast>(keys, values, v, seg_start[v], seg_start[v + 1], seg_flags, s_w, s_seen);
+        }
+        return;
+    }
+
+    const uint32_t first_id = blockIdx.x * (uint32_t)kIds;
+    if (tid < kWave) {
+        const uint32_t v = first_id + (uint32_t)lane;
+        int len = 0;
+        if (lane < kIds && v < ids) len = seg_start[v + 1] - seg_start[v];
+        const uint64_t m = ballot(len > min_len && len <= kCap);
+        if (lane == 0) s_match = m;
+    }
+    __syncthreads();
+    for (uint64_t todo = s_match; todo; todo &= todo - 1) {
+        const uint32_t v = first_id + (uint32_t)(__ffsll((long long)todo) - 1);
+        sort_segment_waves<kWaves, kCap, kLeast>(keys, values, v, seg_start[v], seg_start[v + 1], seg_flags, s_w, s_seen);
+    }
+}
+
 // One wave per workgroup; with a table of segment starts the workgroup looks at kIds tile ids
 // (one per lane) and sorts those with min_len < length <= 64*kT one after the other; without a
 // table the grid has one workgroup per tile id and each searches for its bounds.
@@ -1203,7 +1245,10 @@ __device__ __forceinline__ void sort_segment_general(uint64_t* __restrict__ keys
                                                      uint64_t* __restrict__ alt_keys, uint32_t* __restrict__ alt_values,
                                                      int lo, int hi, uint32_t (*s_cnt)[kBins], uint32_t* s_wave_sum, int* s_flag)
 {
-    const int tid = threadIdx.x;
+    // opaque, like the lane number of the networks: or the addresses of the copy below stay in
+    // registers beside a network's words in a workgroup that does both
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));
     const int len = hi - lo;
     uint64_t* kbuf[2] = { keys + lo, alt_keys + lo };
     uint32_t* vbuf[2] = { values + lo, alt_values + lo };
@@ -1226,9 +1271,9 @@ __device__ __forceinline__ void sort_segment_general(uint64_t* __restrict__ keys
 // ones longer than min_len: neighbouring tiles tend to be equally crowded, so they are dealt out
 // one segment at a time, round-robin), the workgroups behind them look at 64 tile ids each for
 // shorter segments that were flagged.
-// With a table (kLds) a listed segment of up to kCapHuge pairs is sorted in LDS like the classes
-// below it, sixteen pairs per thread in registers during a pass (a workgroup then has the LDS of
-// its CU to itself): the passes through memory take 7 us each for 12 000 pairs, those in LDS 2.
+// With a table (kLds) a listed segment of up to kCapHuge pairs is sorted by the network over the
+// sixteen waves (a workgroup then has the LDS of its CU to itself): the passes through memory take
+// 7 us each for 12 000 pairs.
 // The listed blocks first sort the listed segments of the classes below (first_class 1:
 // 1025 .. kCapLarge pairs, 2: only those above kCapMedium, 3: none; shard by shard like the
 // launches of those classes): a frame with a short list of pairs has few such segments or none,
@@ -1246,10 +1291,8 @@ __global__ __launch_bounds__(kGeneralWaves * kWave) void segment_sort_general_ke
     const uint32_t* __restrict__ list_medium, uint32_t cap_medium, const uint32_t* __restrict__ list_large, uint32_t cap_large,
     int first_class)
 {
-    constexpr int kLdsCap = kLds ? kCapHuge : 1;
-    __shared__ uint32_t s_k[kLdsCap];
-    __shared__ uint32_t s_v[kLdsCap];
-    __shared__ uint32_t s_cnt[kGeneralWaves][kBins];      // the passes in LDS use it as 16-bit counters
+    __shared__ uint64_t s_w[kLds ? kCapHuge : 1];
+    __shared__ uint32_t s_cnt[kGeneralWaves][kBins];
     __shared__ uint32_t s_wave_sum[kGeneralWaves];
     __shared__ int s_bounds[2];
     __shared__ int s_flag;
@@ -1298,8 +1341,7 @@ __global__ __launch_bounds__(kGeneralWaves * kWave) void segment_sort_general_ke
                     // keys that differ above the depth word: through memory right away (no flag: the
                     // workgroups that look at the flags run beside this one)
                     if (hi - lo <= kCapHuge)
-                        through_memory = sort_segment_lds<kGeneralWaves, kCapHuge>(keys, values, v, lo, hi, nullptr, s_k, s_v,
-                                                                                   (uint16_t (*)[kBins])s_cnt, s_wave_sum, &s_flag);
+                        through_memory = sort_segment_waves<kGeneralWaves, kCapHuge, 2>(keys, values, v, lo, hi, nullptr, s_w, s_wave_sum);
                 }
                 if (through_memory) sort_segment_general(keys, values, alt_keys, alt_values, lo, hi, s_cnt, s_wave_sum, &s_flag);
             }
@@ -1459,8 +1501,8 @@ extern "C" int fgs_sort_gaussian(int num_rendered,
             const unsigned g = most < limit ? most : limit;
             return (g + kListShards - 1) / kListShards * kListShards;
         };
-#define FGS_SEGMENT_CLASS(WAVES, CAP, IDS, MINLEN, GRID, LIST, COUNT, LISTCAP)                                \
-        hipLaunchKernelGGL((segment_sort_kernel<WAVES, CAP, IDS>), dim3(GRID), dim3((WAVES) * kWave), 0, st,  \
+#define FGS_SEGMENT_CLASS(WAVES, CAP, LEAST, IDS, MINLEN, GRID, LIST, COUNT, LISTCAP)                                \
+        hipLaunchKernelGGL((segment_sort_kernel<WAVES, CAP, LEAST, IDS>), dim3(GRID), dim3((WAVES) * kWave), 0, st,  \
                            ks, vs, n, tile_mask, MINLEN, ids, (const int*)seg_start, seg_flags,               \
                            (const uint32_t*)(LIST), (const uint32_t*)(COUNT), LISTCAP)
         // Up to 512 pairs: one wave, bitonic network in registers; one tile id per wave (neighbouring
@@ -1494,16 +1536,16 @@ extern "C" int fgs_sort_gaussian(int num_rendered,
                                    dim3(kWave), 0, st, ks, vs, (const int*)seg_start, seg_flags,
                                    (const uint32_t*)list_small, (const uint32_t*)seg_counts, cap_small);
             if (n > kCapSmall && !merged_tail) {
-                FGS_SEGMENT_CLASS(8, kCapMedium, 64, kCapSmall, list_grid((unsigned)(n / (kCapSmall + 1) + 1), 4096u),
+                FGS_SEGMENT_CLASS(4, kCapMedium, 8, 64, kCapSmall, list_grid((unsigned)(n / (kCapSmall + 1) + 1), 4096u),
                                   list_medium, seg_counts + kListShards, cap_medium);
                 if (n > kCapMedium && !merged_large)
-                    FGS_SEGMENT_CLASS(16, kCapLarge, 64, kCapMedium, list_grid((unsigned)(n / (kCapMedium + 1) + 1), 1024u),
+                    FGS_SEGMENT_CLASS(8, kCapLarge, 16, 64, kCapMedium, list_grid((unsigned)(n / (kCapMedium + 1) + 1), 1024u),
                                       list_large, seg_counts + 2 * kListShards, cap_large);
             }
         } else {
-            if (n > kCapTiny) FGS_SEGMENT_CLASS(4, kCapSmall, 1, kCapTiny, ids, no_list, no_list, 0u);
-            if (n > kCapSmall) FGS_SEGMENT_CLASS(8, kCapMedium, 64, kCapSmall, ids, no_list, no_list, 0u);
-            if (n > kCapMedium) FGS_SEGMENT_CLASS(16, kCapLarge, 64, kCapMedium, ids, no_list, no_list, 0u);
+            if (n > kCapTiny) FGS_SEGMENT_CLASS(4, kCapSmall, 4, 1, kCapTiny, ids, no_list, no_list, 0u);
+            if (n > kCapSmall) FGS_SEGMENT_CLASS(4, kCapMedium, 8, 64, kCapSmall, ids, no_list, no_list, 0u);
+            if (n > kCapMedium) FGS_SEGMENT_CLASS(8, kCapLarge, 16, 64, kCapMedium, ids, no_list, no_list, 0u);
         }
 #undef FGS_SEGMENT_CLASS
         // longer segments from their list, one workgroup per segment; behind them the shorter ones that were flagged

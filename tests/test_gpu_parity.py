@@ -1045,6 +1045,29 @@ def test_sort_depth_words_of_every_pattern(depths, ascending):
     assert np.array_equal(gp.u64(ks), keys[order]) and np.array_equal(gp.u32(vs), vals[order])
 
 
+@pytest.mark.parametrize("depths", ["all words", "positive floats", "few"])
+@pytest.mark.parametrize("ascending", [True, False])
+@pytest.mark.parametrize("copies", [1, 10, 40])
+def test_sort_segments_of_several_waves(depths, ascending, copies):
+    """Segments that several waves sort together: around the lengths where the slots per lane, the waves that
+    take part and the launches change; values that ascend everywhere but between two waves' parts."""
+    import gpu_pipeline as gp
+    rng = np.random.default_rng(copies + ascending)
+    lengths = [1025, 1535, 1537, 2047, 2048, 2049, 3071, 3073, 4095, 4096, 4097, 5120, 5121, 7169, 8191, 8192, 8193, 9217, 16383,
+               16384, 16385] * copies
+    lo, hi = {"all words": (0, 1 << 32), "positive floats": (0x3e4ccccd, 0x42c80000), "few": (0x40000000, 0x40000010)}[depths]
+    tile = np.repeat(np.arange(len(lengths)), lengths)
+    n = len(tile)
+    keys = (tile.astype(np.uint64) << np.uint64(32)) | rng.integers(lo, hi, n, dtype=np.uint64)
+    vals = np.arange(n, dtype=np.uint32)
+    if not ascending:       # one pair per segment is out of order: the first of a part of 64 .. 1024 pairs
+        first = np.concatenate([[0], np.cumsum(lengths)[:-1]])
+        vals[first + 64 * (1 << (np.arange(len(lengths)) % 5))] = 0
+    ks, vs = gp.sort(n, 1920, 1080, gp.dev(keys.view(np.int64)), gp.dev(vals.view(np.int32)))
+    order = np.argsort(keys, kind="stable")
+    assert np.array_equal(gp.u64(ks), keys[order]) and np.array_equal(gp.u32(vs), vals[order])
+
+
 @pytest.mark.parametrize("ascending", [False, True])
 @pytest.mark.parametrize("W,H", [(1920, 1080), (3840, 2160)])
 def test_sort_every_segment_length_up_to_1100(W, H, ascending):
