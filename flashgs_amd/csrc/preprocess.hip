@@ -34,13 +34,14 @@ namespace {
 
 constexpr int kBlock = 256;
 constexpr int kWavesPerBlock = kBlock / kWave;
-constexpr int kStashCap = 1024;         // flat candidates (and so stashed hits) per wave
+constexpr int kFlatCap = 1024;          // flat candidates per wave and round
+constexpr int kStashCap = 2048;         // stashed hits per wave
 constexpr int kHugeMin = 1024;          // rectangles with more tiles than this are tested by the whole workgroup
 // such rectangles per workgroup: as many as the LDS of 7 workgroups per CU leaves room for (a
 // rectangle beyond the list stays with its wave, 64 tiles a step, and everything behind this
 // workgroup waits for that count)
 constexpr int kHugeCap = 27;
-constexpr int kSpanWords = kWavesPerBlock * kStashCap / 4;   // column + row spans of one listed rectangle
+constexpr int kSpanWords = kWavesPerBlock * kFlatCap / 4;   // column + row spans of one listed rectangle
 static_assert(kSpanWords / kWave <= kWave, "one lane per group of 64 columns");
 constexpr unsigned kSpinLimit = 1u << 22;   // polls before a wait on the scan over workgroups gives up
 
@@ -479,11 +480,13 @@ __global__ __launch_bounds__(kBlock) void preprocess_kernel(
 {
     __shared__ uint32_t s_wave_total[kWavesPerBlock];
     __shared__ uint32_t s_block_base;
-    __shared__ uint32_t s_stash[kWavesPerBlock][kStashCap];     // hits of the flat candidates, in emission order
-    __shared__ uint64_t s_hits[kWavesPerBlock][kStashCap / kWave + 1];
+    // hits: tile of the rectangle << 6 | owner lane, an owner's hits together and in emission order
+    __shared__ uint16_t s_stash[kWavesPerBlock][kStashCap];
+    static_assert(kHugeMin << 6 <= 1 << 16, "a tile of a stashed rectangle in 10 bits");
+    __shared__ uint64_t s_hits[kWavesPerBlock][kFlatCap / kWave + 1];
     // flat candidate -> lane that owns it; free again after the flat tile tests, when the listed
     // rectangles use it for their column and row spans
-    __shared__ __align__(4) uint8_t s_owner[kWavesPerBlock][kStashCap];
+    __shared__ __align__(4) uint8_t s_owner[kWavesPerBlock][kFlatCap];
     // rectangles too big for one wave: parameters, per-wave hit counts, first key slot
     __shared__ float s_huge_f[kHugeCap][6];
     __shared__ int s_huge_i[kHugeCap][4];
@@ -608,13 +611,13 @@ __global__ __launch_bounds__(kBlock) void preprocess_kernel(
     // ---- count keys ----
     // Rectangles of up to 64 tiles are "flat": their candidates are laid end to end over the wave
     // (Gaussian-major, row-major inside a Gaussian - the order keys are emitted in), so every lane
-    // tests one candidate per step whatever the mix of rectangle sizes.  Hits are compacted into
-    // an LDS stash as (tile << 6 | owner lane) and written out once the slots are known.  A wave
-    // stashes at most kStashCap candidates; what does not fit, and every larger rectangle, is
-    // tested by the whole wave, 64 tiles a step, once to count and once more to emit.
+    // tests one candidate per step whatever the mix of rectangle sizes, in rounds of up to kFlatCap
+    // candidates.  Larger rectangles are tested by the whole wave, 64 tiles a step.  Hits are compacted
+    // into an LDS stash and written out once the slots are known.  The hits of a rectangle that the stash
+    // has no room for (or of more than kHugeMin tiles) are counted only, and tested once more to be emitted.
+    // (With one round of 1024 candidates, and larger rectangles tested twice, the launch took 1472 us on an 8K
+    // frame of 111M pairs and 308 on a 4K frame with 10 % needles; now 1330 and 275.)
     const bool flat_ok = has_tiles && area <= kWave && pack_ok;
-    uint32_t cand_incl = wave_inclusive_sum(flat_ok ? (uint32_t)area : 0u);
-    const bool flat = flat_ok && cand_incl <= (uint32_t)kStashCap;
     // A rectangle of thousands of tiles would keep one wave busy for a long time while every later
     // workgroup waits for this workgroup's count: such rectangles are put on a list and all waves
     // of the workgroup share the testing, a contiguous quarter of the tiles each.
@@ -636,53 +639,60 @@ __global__ __launch_bounds__(kBlock) void preprocess_kernel(
                               rw + rh <= kSpanWords;
         }
     }
-    const bool large = has_tiles && !flat && huge_slot < 0;
-    // lanes that drop out are at the end of the scan order, so the prefix of the others is unchanged
-    const uint32_t cand_excl = cand_incl - (uint32_t)area;
-    const uint64_t flat_lanes = ballot(flat);
-    const int last_flat = flat_lanes ? 63 - __builtin_clzll(flat_lanes) : 0;
-    const int n_cand = flat_lanes ? bcast_i((int)cand_incl, last_flat) : 0;
-
     uint8_t* owner_of = s_owner[wave];
-    uint32_t* stash = s_stash[wave];
+    uint16_t* stash = s_stash[wave];
     uint64_t* hit_words = s_hits[wave];
-    if (flat)
-        for (int k = 0; k < area; k++) owner_of[cand_excl + k] = (uint8_t)lane;
-    __builtin_amdgcn_wave_barrier();
-
     const uint32_t rect_pack = (uint32_t)rminx | ((uint32_t)rminy << 12) | ((uint32_t)(rw - 1) << 24);
     int n_stash = 0;
-    for (int c0 = 0; c0 < n_cand; c0 += kWave) {
-        const int c = c0 + lane;
-        const bool live = c < n_cand;
-        const int own = live ? (int)owner_of[c] : lane;
-        const float gcx = __shfl(cx, own), gcy = __shfl(cy, own);
-        const float gconx = __shfl(conx, own), gcony = __shfl(cony, own), gconz = __shfl(conz, own);
-        const float gpower = __shfl(power, own);
-        const uint32_t grect = (uint32_t)__shfl((int)rect_pack, own);
-        const int k = c - __shfl((int)cand_excl, own);
-        const int gminx = (int)(grect & 0xfffu), gminy = (int)((grect >> 12) & 0xfffu), grw = (int)(grect >> 24) + 1;
-        // k / grw for 0 <= k < 64, 1 <= grw <= 64: (k + 0.5) / grw is at least 1/128 away from an
-        // integer, far more than the error of the approximate reciprocal
-        const int ty = (int)(((float)k + 0.5f) * __builtin_amdgcn_rcpf((float)grw));
-        const int tx = k - ty * grw;
-        const bool hit = live && tile_hit(gminx + tx, gminy + ty, cam.bx, cam.by, gcx, gcy, gconx, gcony, gconz, gpower);
-        const uint64_t hits = ballot(hit);
-        if (hit) stash[n_stash + popc_below(hits)] = ((uint32_t)((gminy + ty) * cam.gx + gminx + tx) << 6) | (uint32_t)own;
-        if (lane == 0) hit_words[c0 / kWave] = hits;
-        n_stash += __popcll(hits);
-    }
-    __builtin_amdgcn_wave_barrier();
-
     uint32_t count = 0;
-    if (flat) {      // hits among this lane's candidates [cand_excl, cand_excl + area)
-        const int w0 = (int)(cand_excl >> 6), b0 = (int)(cand_excl & 63u);
-        uint64_t m = hit_words[w0] >> b0;
-        if (b0 + area > kWave) m |= hit_words[w0 + 1] << (kWave - b0);
-        if (area < kWave) m &= (1ull << area) - 1ull;
-        count = (uint32_t)__popcll(m);
+    bool waiting = flat_ok;      // flat and not tested yet
+    while (ballot(waiting) != 0) {
+        const uint32_t cand_incl = wave_inclusive_sum(waiting ? (uint32_t)area : 0u);
+        // (lanes that do not fit are at the end of the scan order, so the prefix of the others is unchanged)
+        const bool take = waiting && cand_incl <= (uint32_t)min(kFlatCap, kStashCap - n_stash);
+        const uint64_t takers = ballot(take);
+        if (takers == 0) break;
+        const uint32_t cand_excl = cand_incl - (uint32_t)area;
+        const int n_cand = bcast_i((int)cand_incl, 63 - __builtin_clzll(takers));
+        if (take)
+            for (int k = 0; k < area; k++) owner_of[cand_excl + k] = (uint8_t)lane;
+        __builtin_amdgcn_wave_barrier();
+        for (int c0 = 0; c0 < n_cand; c0 += kWave) {
+            const int c = c0 + lane;
+            const bool live = c < n_cand;
+            const int own = live ? (int)owner_of[c] : lane;
+            const float gcx = __shfl(cx, own), gcy = __shfl(cy, own);
+            const float gconx = __shfl(conx, own), gcony = __shfl(cony, own), gconz = __shfl(conz, own);
+            const float gpower = __shfl(power, own);
+            const uint32_t grect = (uint32_t)__shfl((int)rect_pack, own);
+            const int k = c - __shfl((int)cand_excl, own);
+            const int gminx = (int)(grect & 0xfffu), gminy = (int)((grect >> 12) & 0xfffu), grw = (int)(grect >> 24) + 1;
+            // k / grw for 0 <= k < 64, 1 <= grw <= 64: (k + 0.5) / grw is at least 1/128 away from an
+            // integer, far more than the error of the approximate reciprocal
+            const int ty = (int)(((float)k + 0.5f) * __builtin_amdgcn_rcpf((float)grw));
+            const int tx = k - ty * grw;
+            const bool hit = live && tile_hit(gminx + tx, gminy + ty, cam.bx, cam.by, gcx, gcy, gconx, gcony, gconz, gpower);
+            const uint64_t hits = ballot(hit);
+            if (hit) stash[n_stash + popc_below(hits)] = (uint16_t)((k << 6) | own);
+            if (lane == 0) hit_words[c0 / kWave] = hits;
+            n_stash += __popcll(hits);
+        }
+        __builtin_amdgcn_wave_barrier();
+        if (take) {      // hits among this lane's candidates [cand_excl, cand_excl + area)
+            const int w0 = (int)(cand_excl >> 6), b0 = (int)(cand_excl & 63u);
+            uint64_t m = hit_words[w0] >> b0;
+            if (b0 + area > kWave) m |= hit_words[w0 + 1] << (kWave - b0);
+            if (area < kWave) m &= (1ull << area) - 1ull;
+            count = (uint32_t)__popcll(m);
+            waiting = false;
+        }
+        __builtin_amdgcn_wave_barrier();
     }
-    const uint32_t flat_count = count;
+    const bool flat = flat_ok && !waiting;
+    const bool large = has_tiles && !flat && huge_slot < 0;
+    // stashed hits of a lane that come first; of a flat one, as many as the flat lanes in front of it have
+    uint32_t stash_at = wave_inclusive_sum(count) - count;
+    bool in_stash = flat;
     const uint64_t large_lanes = ballot(large);
     for (uint64_t todo = large_lanes; todo; todo &= todo - 1) {
         const int src = __ffsll((long long)todo) - 1;
@@ -692,6 +702,8 @@ __global__ __launch_bounds__(kBlock) void preprocess_kernel(
         const int gminx = bcast_i(rminx, src), gminy = bcast_i(rminy, src);
         const int grw = bcast_i(rw, src), garea = bcast_i(area, src);
         uint32_t total = 0;
+        const int at = n_stash;
+        bool keep = garea <= kHugeMin;
         for (int base = 0; base < garea; base += kWave) {
             const int j = base + lane;
             bool ok = false;
@@ -700,9 +712,17 @@ __global__ __launch_bounds__(kBlock) void preprocess_kernel(
                 div_mod(j, grw, ty, tx);
                 ok = tile_hit(gminx + tx, gminy + ty, cam.bx, cam.by, gcx, gcy, gconx, gcony, gconz, gpower);
             }
-            total += (uint32_t)__popcll(ballot(ok));
+            const uint64_t hits = ballot(ok);
+            const int n_hits = __popcll(hits);
+            keep = keep && n_stash + n_hits <= kStashCap;
+            if (keep) {
+                if (ok) stash[n_stash + popc_below(hits)] = (uint16_t)((j << 6) | src);
+                n_stash += n_hits;
+            }
+            total += (uint32_t)n_hits;
         }
-        if (lane == src) count = total;
+        if (!keep) n_stash = at;
+        if (lane == src) { count = total; stash_at = (uint32_t)at; in_stash = keep; }
     }
 
     // the listed rectangles: wave w counts tiles [w*part, (w+1)*part) of each
@@ -919,25 +939,33 @@ __global__ __launch_bounds__(kBlock) void preprocess_kernel(
         }
     }
     {
-        // stash entry e of owner o goes to slot(o) + (e - entries before o's first)
-        uint32_t before = wave_inclusive_sum(flat_count);
-        const uint32_t delta = my_slot - (before - flat_count);
+        // stash entry e of owner o goes to slot(o) + (e - o's first entry)
+        __builtin_amdgcn_wave_barrier();
+        const uint32_t delta = my_slot - stash_at;
         const uint32_t gidx_base = (uint32_t)(ticket * kBlock + wave * kWave);
+        const uint32_t first_tile = (uint32_t)rminy * (uint32_t)cam.gx + (uint32_t)rminx;
+        const int width = max(rw, 1);
         for (int e0 = 0; e0 < n_stash; e0 += kWave) {
             const int e = e0 + lane;
             const bool live = e < n_stash;
-            const uint32_t entry = live ? stash[e] : (uint32_t)lane;
-            const int own = (int)(entry & 63u);
+            const uint32_t entry = live ? (uint32_t)stash[e] : (uint32_t)lane;
+            const int own = (int)(entry & 63u), k = (int)(entry >> 6);
             const uint32_t odelta = (uint32_t)__shfl((int)delta, own);
             const uint32_t odepth = (uint32_t)__shfl((int)depth_bits, own);
+            const uint32_t ofirst = (uint32_t)__shfl((int)first_tile, own);
+            const int owidth = __shfl(width, own);
+            // k / owidth as above: k < 1024, so (k + 0.5) / owidth is 0.5 / owidth or more from an integer and
+            // off by less than a thousandth of that
+            const int ty = (int)(((float)k + 0.5f) * __builtin_amdgcn_rcpf((float)owidth));
+            const uint32_t tile = ofirst + (uint32_t)(ty * cam.gx + (k - ty * owidth));
             const uint64_t dst = (uint64_t)(odelta + (uint32_t)e);
             if (live && dst < cap) {
-                keys[dst] = ((uint64_t)(entry >> 6) << 32) | odepth;
+                keys[dst] = ((uint64_t)tile << 32) | odepth;
                 values[dst] = gidx_base + (uint32_t)own;
             }
         }
     }
-    for (uint64_t todo = large_lanes; todo; todo &= todo - 1) {
+    for (uint64_t todo = large_lanes & ~ballot(in_stash); todo; todo &= todo - 1) {
         const int src = __ffsll((long long)todo) - 1;
         if (bcast_i((int)count, src) == 0) continue;
         const float gcx = bcast_f(cx, src), gcy = bcast_f(cy, src);
