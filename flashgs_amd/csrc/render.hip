@@ -26,7 +26,6 @@ __device__ float mul_zero_wins(float a, float b) __asm("llvm.amdgcn.fmul.legacy"
 
 namespace {
 
-
 __global__ __launch_bounds__(256) void fill_i32_kernel(int* p, size_t n, int v)
 {
     size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -46,19 +45,28 @@ constexpr int kOrderBins = 128;            // everything from 2032 entries up sh
 // stream follow each other; blends on different streams may overlap and get a table each).  A
 // stream that is being captured and has no table yet cannot allocate one and uses this
 // per-device table instead, which captured blends on one device then share.
+// Wide tiles need no ranking to be blended (16x16 tiles share out their long lists by it), so theirs is
+// optional: under capture, where the table's address would stay in the graph and be shared by whatever
+// replays it beside this stream's own blends, and where no memory is left, they go unranked.
 __device__ uint32_t g_tile_order[kOrderCap];
 std::map<StreamKey, uint32_t*> g_order_tables;
 std::mutex g_order_mutex;
 
-int tile_order_table(hipStream_t stream, uint32_t** out)
+// *out is null only where the ranking is optional.
+int tile_order_table(hipStream_t stream, bool optional, uint32_t** out)
 {
     int device = 0;
+    *out = nullptr;
     FGS_HIP_TRY(hipGetDevice(&device));
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (optional && stream) {
+        FGS_HIP_TRY(hipStreamIsCapturing(stream, &capture));
+        if (capture != hipStreamCaptureStatusNone) return FGS_OK;
+    }
     std::lock_guard<std::mutex> lock(g_order_mutex);
     uint32_t*& table = g_order_tables[stream_key(device, stream)];
     if (!table) {
-        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-        if (stream) FGS_HIP_TRY(hipStreamIsCapturing(stream, &capture));
+        if (!optional && stream) FGS_HIP_TRY(hipStreamIsCapturing(stream, &capture));
         if (capture != hipStreamCaptureStatusNone) {
             void* shared = nullptr;
             FGS_HIP_TRY(hipGetSymbolAddress(&shared, HIP_SYMBOL(g_tile_order)));
@@ -68,7 +76,7 @@ int tile_order_table(hipStream_t stream, uint32_t** out)
         if (hipMalloc((void**)&table, kOrderCap * sizeof(uint32_t)) != hipSuccess) {
             (void)hipGetLastError();
             table = nullptr;
-            return fail(FGS_E_NOMEM, "cannot allocate the table of tile ranks");
+            return optional ? FGS_OK : fail(FGS_E_NOMEM, "cannot allocate the table of tile ranks");
         }
     }
     *out = table;
@@ -973,9 +981,9 @@ int blend_impl(int block_x, int block_y, int width, int height,
     const int num_tiles = tiles_x * tiles_y;
     uint32_t* tile_order = nullptr;
     if (is_ranked(tiles_x, tiles_y)) {
-        rc = tile_order_table(st, &tile_order);
+        rc = tile_order_table(st, sx * sy > 1, &tile_order);
         if (rc != FGS_OK) return rc;
-        hipLaunchKernelGGL(tile_order_kernel, dim3(1), dim3(1024), 0, st, (const int2*)ranges, num_tiles, tile_order);
+        if (tile_order) hipLaunchKernelGGL(tile_order_kernel, dim3(1), dim3(1024), 0, st, (const int2*)ranges, num_tiles, tile_order);
     }
     const dim3 grid((unsigned)(tile_order ? num_tiles : groups));
     const bool fp32 = mode == FGS_COLOUR_SUMS_FP32;

@@ -154,7 +154,8 @@ size_t fgs_get_sort_buffer_size(int num_rendered);
  * their own transmittance: the colour can differ from the pair-by-pair walk of
  * render.cu:315-408 by what lies behind T < 1e-4, i.e. by less than 1e-4 of a colour.  Calls on
  * different streams may overlap in time; a stream that is being captured and has no table yet
- * uses one table per device instead, so replays of such graphs on one device must not overlap.
+ * uses one table per device instead, so replays of such graphs on one device must not overlap
+ * (16x16 tiles only: the wide tiles go unranked under capture, and where the table cannot be allocated).
  */
 int fgs_render_16x16(int num_rendered, int width, int height,
                      const float* points_xy, const float* rgb_depth, const float* conic_opacity,

@@ -572,6 +572,54 @@ def test_sort_and_render_replayed_from_a_captured_graph():
         torch.cuda.synchronize()
 
 
+@pytest.mark.parametrize("block", [(32, 16), (32, 32)])
+def test_wide_tiles_replayed_beside_each_other(block):
+    """Blends of wide tiles hold no table of the library's in a captured graph: graphs of two frame sizes,
+    replayed side by side on two streams and beside eager blends on the stream they were captured on,
+    give the eager images."""
+    import gpu_pipeline as gp
+    from flashgs_amd import cabi
+    import torch
+    bx, by = block
+    side = torch.cuda.Stream()
+    frames = []
+    for W, H in ((640, 360), (1000, 700)):
+        sc = scenes.config0(n=30_000)
+        cam = scenes.look_at([0.0, 0.5, -15.0], [0.0, 0.0, 0.0], W, H, 50.0)
+        pre = gp.preprocess(gp.SceneOnDevice(sc), cam, 1 << 19, block=block)
+        K = pre["num_rendered"]
+        assert 0 < K <= 1 << 19
+        ks, vs = gp.sort(K, W, H, pre["keys"], pre["values"], block=block)
+        ranges, eager, _ = gp.render(K, W, H, pre["points_xy"], pre["rgb_depth"], pre["conic_opacity"], ks, vs,
+                                     (0.2, 0.4, 0.6), block=block, f32=False)
+        out = torch.zeros_like(eager)
+
+        def blend(stream, pre=pre, vs=vs, ranges=ranges, out=out, W=W, H=H):
+            cabi.blend(bx, by, W, H, pre["points_xy"].data_ptr(), pre["rgb_depth"].data_ptr(),
+                       pre["conic_opacity"].data_ptr(), vs.data_ptr(), ranges.data_ptr(),
+                       np.array([0.2, 0.4, 0.6], np.float32), out.data_ptr(), 0, stream)
+
+        torch.cuda.synchronize()
+        blend(side.cuda_stream)             # the stream has a table of its own before the capture
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            blend(torch.cuda.current_stream().cuda_stream)
+        frames.append((graph, blend, eager, out, (ks, pre)))
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    for replay in range(3):
+        for f in frames:
+            f[3].zero_()
+        torch.cuda.synchronize()
+        for f, s in zip(frames, streams):
+            with torch.cuda.stream(s):
+                f[0].replay()
+        frames[0][1](side.cuda_stream)
+        torch.cuda.synchronize()
+        for f in frames:
+            assert torch.equal(f[3], f[2]), "replay %d" % replay
+
+
 def test_repeated_frames_are_deterministic():
     import gpu_pipeline as gp
     sc = scenes.config0(n=50_000)
