@@ -38,9 +38,10 @@ if ROOT not in sys.path:
 HBM_PEAK_GBS = 8000.0            # MI355X HBM3E, published
 FP32_PEAK_TFLOPS = 157.3         # MI355X fp32 vector, published (packed FMA)
 FLOP_PER_EVAL = 19               # render.cu:40-52: 2 sub, 6 mul + 3 add, 1 mul, 3 FMA, 1 sub
-EXEC_SLOTS_PER_EVAL = 8.1        # non-transcendental VALU instructions the fp32 blend kernel issues per evaluation (SQ counters,
-                                 # profiles/frame_cfg2_3M_4K_sq_counters.txt): 2 for the exponent from its tables, alpha*T, T -=,
-                                 # 3 colour FMAs, 1.1 for staging, stop tests and loop; the v_exp_f32 issues beside them
+EXEC_SLOTS_PER_EVAL = 7.4        # non-transcendental VALU instructions the fp32 blend kernel issues per evaluation (SQ counters,
+                                 # profiles/frame_cfg2_3M_4K_sq_counters.txt, without the 0.08 matrix instructions): 1.25 for the weight
+                                 # from its recurrence, alpha*T, T -=, 3 colour FMAs, the rest staging, stop tests and loop; half a
+                                 # v_exp_f32 beside them.  Some of them issue faster than the v_fma_f32 of the calibration.
 ATTAINED_FMA_LANE_OPS = 38.05e12 # v_fma_f32 lane-operations/s measured on this part without packed math (bench.py --calibrate)
 CAPACITY = {0: 1 << 20, 1: 1 << 22, 2: 1 << 24, 3: 1 << 25, 4: 1 << 25, 5: 1 << 27, 6: 1 << 25}
 FAST_MODE_DTYPE = "f32 (colour sums: f16 operands on the matrix unit, fp32 products and sums)"
