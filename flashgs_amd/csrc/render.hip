@@ -201,7 +201,9 @@ __device__ __forceinline__ uint8_t encode_u8(float x)
 // product with v_mfma_f32_32x32x2_f32 made a 4K frame 9 % slower).  Nothing is lost by bf16: the
 // coordinates are small whole numbers, a coefficient is the sum of three bf16 numbers of eight bits of its
 // significand each, products are exact and sums are fp32.  A slope is as exact as a value; its error
-// counts up to three times in alpha_3, some 1e-6 of it.
+// counts up to three times in alpha_3, some 1e-6 of it.  Against a float64 blend of the same lists the
+// image of a 1080p frame of 1M is off by 4.0e-7 (2-norm), of the 4K orbit with its needles by 4.9e-6;
+// with the tables in LDS that were here before it was 1.0e-6 and 8.9e-6.
 //
 // v_mfma_f32_32x32x16_bf16 multiplies 32 rows by 32 columns over 16 slots, of which lanes 0-31 supply
 // slots 0-7 and lanes 32-63 slots 8-15, and lane l receives rows 8 i + 4 (l / 32) + j of column l % 32.
@@ -797,19 +799,27 @@ __global__ __launch_bounds__(kWave * SX * SY) __attribute__((amdgpu_waves_per_eu
 constexpr int kOwnShare = 256;
 constexpr int kMinRest = 512;               // a shorter rest is not worth two barriers: the owner walks it
 constexpr int kSharedWaves = 4;
+// Where every workgroup is resident at once even with one tile each (4 SIMDs of 256 CUs, four waves a
+// workgroup), a tile has a workgroup to itself: three waves of it have no list of their own and only take
+// runs, so a long list has all four instead of a share of them, and the cut into runs stays the same.  256x192
+// pixels, 300k clustered Gaussians 357 -> 245 us, 640x512 100 -> 81, 1M 228 -> 169, with lists too short to be
+// shared 14.8 -> 14.8.  Beyond that (1920x1080, 1M) waves without a list keep others off the chip: 138 -> 159.
+template <bool kFp32>
+constexpr int kSoloTiles = 256 * kBlendWaves<kFp32>;
 
 template <bool kFp32>
-__global__ __launch_bounds__(kSharedWaves * kWave) __attribute__((amdgpu_waves_per_eu(kBlendWaves<kFp32>, kBlendWaves<kFp32>))) void blend_kernel_shared(FGS_BLEND_PARAMS, const uint32_t* __restrict__ tile_order)
+__global__ __launch_bounds__(kSharedWaves * kWave) __attribute__((amdgpu_waves_per_eu(kBlendWaves<kFp32>, kBlendWaves<kFp32>))) void blend_kernel_shared(FGS_BLEND_PARAMS, const uint32_t* __restrict__ tile_order, int tiles_per_group)
 {
     constexpr int kHandOver = 4 * 4 * kWave;            // a run's result: 4 pixels x 4 floats per lane
     __shared__ __align__(16) float s_stage[kSharedWaves][kStageFloats > kHandOver ? kStageFloats : kHandOver];
     __shared__ int s_rest[kSharedWaves], s_from[kSharedWaves], s_tile_x[kSharedWaves], s_tile_y[kSharedWaves];
 
     const int lane = threadIdx.x & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-    // Wave w takes rank g of quarter w of the tiles ranked by list length: the workgroups with
-    // the longest lists come first in the launch, and a long list has three shorter ones beside it.
+    // Wave w takes rank g of quarter w of the tiles ranked by list length (with tiles_per_group 1, wave 0 takes
+    // rank g and the others none): the workgroups with the longest lists come first in the launch, and a
+    // long list has three shorter ones beside it.
     const int rank = wave * (int)gridDim.x + (int)blockIdx.x;
-    const bool active = rank < tiles_x * tiles_y;
+    const bool active = wave < tiles_per_group && rank < tiles_x * tiles_y;
     int tile_x = 0, tile_y = 0;
     if (active) {
         const int tile = (int)tile_order[rank];
@@ -996,10 +1006,11 @@ int blend_impl(int block_x, int block_y, int width, int height,
                            bg[0], bg[1], bg[2], out_u8, out_f32, (const uint32_t*)tile_order);          \
     } while (0)
     if (tile_order && sx == 1 && sy == 1) {
-        hipLaunchKernelGGL(fp32 ? blend_kernel_shared<true> : blend_kernel_shared<false>, dim3((unsigned)((num_tiles + kSharedWaves - 1) / kSharedWaves)), dim3(kSharedWaves * kWave), 0, st,
+        const int tiles_per_group = num_tiles <= (fp32 ? kSoloTiles<true> : kSoloTiles<false>) ? 1 : kSharedWaves;
+        hipLaunchKernelGGL(fp32 ? blend_kernel_shared<true> : blend_kernel_shared<false>, dim3((unsigned)((num_tiles + tiles_per_group - 1) / tiles_per_group)), dim3(kSharedWaves * kWave), 0, st,
                            (const int2*)ranges, values_sorted, width, height, tiles_x, tiles_y,
                            (const float2*)points_xy, (const float4*)rgb_depth, (const float4*)conic_opacity,
-                           bg[0], bg[1], bg[2], out_u8, out_f32, (const uint32_t*)tile_order);
+                           bg[0], bg[1], bg[2], out_u8, out_f32, (const uint32_t*)tile_order, tiles_per_group);
     } else if (sx == 1 && sy == 1) FGS_LAUNCH_BLEND(1, 1);
     else if (sx == 2 && sy == 1) FGS_LAUNCH_BLEND(2, 1);
     else FGS_LAUNCH_BLEND(2, 2);

@@ -712,6 +712,40 @@ def test_sort_full_size_properties():
     assert int(torch.bincount(vs.long(), minlength=n).max()) == 1     # a permutation
 
 
+@pytest.mark.parametrize("flags,rows", [("fp32", 32), ("f16", 25)])      # 40 tiles a row: 1280 and 1000 tiles
+def test_blend_one_tile_and_four_tiles_per_workgroup_agree(flags, rows):
+    """A frame whose workgroups are all resident at once gives each tile a workgroup of its own; one or two
+    rows of tiles more and four tiles share one.  Lists are cut into the same runs, so the common rows
+    of the two images are the same bits."""
+    import gpu_pipeline as gp
+    from flashgs_amd import cabi
+    import torch
+    W, gx = 640, 40
+    rng = np.random.default_rng(23)
+    n = rng.choice([0, 1, 63, 255, 256, 257, 767, 768, 769, 770, 1501, 3000], gx * rows, p=[0.3, 0.3] + [0.04] * 10)
+    ends = np.cumsum(n)
+    tile = np.repeat(np.arange(gx * rows), n)
+    K = len(tile)
+    xy = np.stack([(tile % gx) * 16 + rng.uniform(-4, 20, K), (tile // gx) * 16 + rng.uniform(-4, 20, K)], 1).astype(np.float32)
+    co = np.stack([-rng.uniform(0.005, 0.1, K), rng.uniform(-0.005, 0.005, K), -rng.uniform(0.005, 0.1, K),
+                   np.log2(rng.uniform(0.0005, 0.01, K))], 1).astype(np.float32)
+    rgbd = rng.uniform(0, 1, (K, 4)).astype(np.float32)
+    d = [gp.dev(a) for a in (xy, rgbd, co)]
+    dv = gp.dev(np.arange(K, dtype=np.int32))
+    images = []
+    for more in (0, 2):
+        ranges = np.zeros((gx * (rows + more), 2), np.int32)
+        ranges[:gx * rows] = np.stack([ends - n, ends], 1)
+        dr, H = gp.dev(ranges), 16 * (rows + more)
+        out = torch.full((H, W, 3), -1.0, device=gp.DEV, dtype=torch.float32)
+        cabi.blend(16, 16, W, H, d[0].data_ptr(), d[1].data_ptr(), d[2].data_ptr(), dv.data_ptr(), dr.data_ptr(),
+                   np.array([0.2, 0.4, 0.6], np.float32), 0, out.data_ptr(), torch.cuda.current_stream().cuda_stream,
+                   flags=cabi.BLEND_FP32 if flags == "fp32" else cabi.BLEND_MATRIX_F16)
+        torch.cuda.synchronize()
+        images.append(out.cpu().numpy()[:16 * rows])
+    assert np.array_equal(images[0], images[1])
+
+
 def test_blend_long_lists_shared_between_waves(oracle):
     """A small frame blends its long lists with four waves: the owner takes the head of the list,
     the rest is cut into four runs that start from T = 1 and are folded front to back.  Crafted
