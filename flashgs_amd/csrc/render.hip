@@ -41,19 +41,26 @@ __global__ __launch_bounds__(256) void fill_i32_kernel(int* p, size_t n, int v)
 constexpr int kOrderCap = 8192;            // tiles
 constexpr int kOrderBins = 128;            // everything from 2032 entries up shares the first bin
 // The ranking is written by one launch and read by the next, so it needs memory of its own: one
-// table per (device, stream), allocated on the first such blend on that stream (blends on one
-// stream follow each other; blends on different streams may overlap and get a table each).  A
-// stream that is being captured and has no table yet cannot allocate one and uses this
-// per-device table instead, which captured blends on one device then share.
+// table per (device, stream), allocated on the first such blend on that stream (blends on
+// different streams may overlap and get a table each).  Blends on one stream follow each other, and
+// its lock is held until both launches are enqueued: else another thread's ranking of another
+// frame, enqueued between them, would be the one the blend reads.  A stream that is being captured
+// and has no table yet cannot allocate one and uses the per-device table instead, which captured
+// blends on one device then share.
 // Wide tiles need no ranking to be blended (16x16 tiles share out their long lists by it), so theirs is
 // optional: under capture, where the table's address would stay in the graph and be shared by whatever
 // replays it beside this stream's own blends, and where no memory is left, they go unranked.
 __device__ uint32_t g_tile_order[kOrderCap];
-std::map<StreamKey, uint32_t*> g_order_tables;
+struct OrderTable {
+    std::mutex enqueue;
+    uint32_t* ranks = nullptr;
+};
+std::map<StreamKey, OrderTable> g_order_tables;      // (entries stay where they are)
 std::mutex g_order_mutex;
 
-// *out is null only where the ranking is optional.
-int tile_order_table(hipStream_t stream, bool optional, uint32_t** out)
+// *out is null only where the ranking is optional; enqueue is locked for as long as nobody else may
+// enqueue a launch that writes *out.
+int tile_order_table(hipStream_t stream, bool optional, uint32_t** out, std::unique_lock<std::mutex>* enqueue)
 {
     int device = 0;
     *out = nullptr;
@@ -63,8 +70,13 @@ int tile_order_table(hipStream_t stream, bool optional, uint32_t** out)
         FGS_HIP_TRY(hipStreamIsCapturing(stream, &capture));
         if (capture != hipStreamCaptureStatusNone) return FGS_OK;
     }
-    std::lock_guard<std::mutex> lock(g_order_mutex);
-    uint32_t*& table = g_order_tables[stream_key(device, stream)];
+    OrderTable* entry;
+    {
+        std::lock_guard<std::mutex> lock(g_order_mutex);
+        entry = &g_order_tables[stream_key(device, stream)];
+    }
+    *enqueue = std::unique_lock<std::mutex>(entry->enqueue);
+    uint32_t*& table = entry->ranks;
     if (!table) {
         if (!optional && stream) FGS_HIP_TRY(hipStreamIsCapturing(stream, &capture));
         if (capture != hipStreamCaptureStatusNone) {
@@ -990,8 +1002,9 @@ int blend_impl(int block_x, int block_y, int width, int height,
     if (groups > 0x7fffffffLL) return fail(FGS_E_INVALID, "%s: image too large", who);
     const int num_tiles = tiles_x * tiles_y;
     uint32_t* tile_order = nullptr;
+    std::unique_lock<std::mutex> enqueue;       // from the ranking to the blend that reads it
     if (is_ranked(tiles_x, tiles_y)) {
-        rc = tile_order_table(st, sx * sy > 1, &tile_order);
+        rc = tile_order_table(st, sx * sy > 1, &tile_order, &enqueue);
         if (rc != FGS_OK) return rc;
         if (tile_order) hipLaunchKernelGGL(tile_order_kernel, dim3(1), dim3(1024), 0, st, (const int2*)ranges, num_tiles, tile_order);
     }
