@@ -44,13 +44,10 @@ constexpr int kOrderBins = 128;            // everything from 2032 entries up sh
 // table per (device, stream), allocated on the first such blend on that stream (blends on
 // different streams may overlap and get a table each).  Blends on one stream follow each other, and
 // its lock is held until both launches are enqueued: else another thread's ranking of another
-// frame, enqueued between them, would be the one the blend reads.  A stream that is being captured
-// and has no table yet cannot allocate one and uses the per-device table instead, which captured
-// blends on one device then share.
-// Wide tiles need no ranking to be blended (16x16 tiles share out their long lists by it), so theirs is
-// optional: under capture, where the table's address would stay in the graph and be shared by whatever
-// replays it beside this stream's own blends, and where no memory is left, they go unranked.
-__device__ uint32_t g_tile_order[kOrderCap];
+// frame, enqueued between them, would be the one the blend reads.
+// No tile needs its rank to be blended, so there is none under capture, where the table's address
+// would stay in the graph and be shared by whatever replays it beside this stream's own blends, and
+// none where no memory is left.
 struct OrderTable {
     std::mutex enqueue;
     uint32_t* ranks = nullptr;
@@ -58,15 +55,15 @@ struct OrderTable {
 std::map<StreamKey, OrderTable> g_order_tables;      // (entries stay where they are)
 std::mutex g_order_mutex;
 
-// *out is null only where the ranking is optional; enqueue is locked for as long as nobody else may
-// enqueue a launch that writes *out.
-int tile_order_table(hipStream_t stream, bool optional, uint32_t** out, std::unique_lock<std::mutex>* enqueue)
+// *out is null where the tiles go unranked; enqueue is locked for as long as nobody else may enqueue a
+// launch that writes *out.
+int tile_order_table(hipStream_t stream, uint32_t** out, std::unique_lock<std::mutex>* enqueue)
 {
     int device = 0;
     *out = nullptr;
     FGS_HIP_TRY(hipGetDevice(&device));
-    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    if (optional && stream) {
+    if (stream) {
+        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
         FGS_HIP_TRY(hipStreamIsCapturing(stream, &capture));
         if (capture != hipStreamCaptureStatusNone) return FGS_OK;
     }
@@ -76,22 +73,11 @@ int tile_order_table(hipStream_t stream, bool optional, uint32_t** out, std::uni
         entry = &g_order_tables[stream_key(device, stream)];
     }
     *enqueue = std::unique_lock<std::mutex>(entry->enqueue);
-    uint32_t*& table = entry->ranks;
-    if (!table) {
-        if (!optional && stream) FGS_HIP_TRY(hipStreamIsCapturing(stream, &capture));
-        if (capture != hipStreamCaptureStatusNone) {
-            void* shared = nullptr;
-            FGS_HIP_TRY(hipGetSymbolAddress(&shared, HIP_SYMBOL(g_tile_order)));
-            *out = (uint32_t*)shared;
-            return FGS_OK;
-        }
-        if (hipMalloc((void**)&table, kOrderCap * sizeof(uint32_t)) != hipSuccess) {
-            (void)hipGetLastError();
-            table = nullptr;
-            return optional ? FGS_OK : fail(FGS_E_NOMEM, "cannot allocate the table of tile ranks");
-        }
+    if (!entry->ranks && hipMalloc((void**)&entry->ranks, kOrderCap * sizeof(uint32_t)) != hipSuccess) {
+        (void)hipGetLastError();
+        entry->ranks = nullptr;
     }
-    *out = table;
+    *out = entry->ranks;
     return FGS_OK;
 }
 
@@ -834,7 +820,7 @@ __global__ __launch_bounds__(kSharedWaves * kWave) __attribute__((amdgpu_waves_p
     const bool active = wave < tiles_per_group && rank < tiles_x * tiles_y;
     int tile_x = 0, tile_y = 0;
     if (active) {
-        const int tile = (int)tile_order[rank];
+        const int tile = tile_order ? (int)tile_order[rank] : rank;
         tile_x = tile % tiles_x;
         tile_y = tile / tiles_x;
     }
@@ -1004,7 +990,7 @@ int blend_impl(int block_x, int block_y, int width, int height,
     uint32_t* tile_order = nullptr;
     std::unique_lock<std::mutex> enqueue;       // from the ranking to the blend that reads it
     if (is_ranked(tiles_x, tiles_y)) {
-        rc = tile_order_table(st, sx * sy > 1, &tile_order, &enqueue);
+        rc = tile_order_table(st, &tile_order, &enqueue);
         if (rc != FGS_OK) return rc;
         if (tile_order) hipLaunchKernelGGL(tile_order_kernel, dim3(1), dim3(1024), 0, st, (const int2*)ranges, num_tiles, tile_order);
     }
@@ -1018,7 +1004,7 @@ int blend_impl(int block_x, int block_y, int width, int height,
                            (const float2*)points_xy, (const float4*)rgb_depth, (const float4*)conic_opacity, \
                            bg[0], bg[1], bg[2], out_u8, out_f32, (const uint32_t*)tile_order);          \
     } while (0)
-    if (tile_order && sx == 1 && sy == 1) {
+    if (is_ranked(tiles_x, tiles_y) && sx == 1 && sy == 1) {
         const int tiles_per_group = num_tiles <= (fp32 ? kSoloTiles<true> : kSoloTiles<false>) ? 1 : kSharedWaves;
         hipLaunchKernelGGL(fp32 ? blend_kernel_shared<true> : blend_kernel_shared<false>, dim3((unsigned)((num_tiles + tiles_per_group - 1) / tiles_per_group)), dim3(kSharedWaves * kWave), 0, st,
                            (const int2*)ranges, values_sorted, width, height, tiles_x, tiles_y,

@@ -153,9 +153,10 @@ size_t fgs_get_sort_buffer_size(int num_rendered);
  * and with 16x16 tiles the rest of a list of more than 768 entries is blended in four runs that each stop on
  * their own transmittance: the colour can differ from the pair-by-pair walk of
  * render.cu:315-408 by what lies behind T < 1e-4, i.e. by less than 1e-4 of a colour.  Calls on
- * different streams may overlap in time; a stream that is being captured and has no table yet
- * uses one table per device instead, so replays of such graphs on one device must not overlap
- * (16x16 tiles only: the wide tiles go unranked under capture, and where the table cannot be allocated).
+ * different streams may overlap in time, and several host threads may call on one stream.  Under
+ * stream capture, and where the table cannot be allocated, tiles go unranked: the image is the
+ * same, and a captured blend holds no memory of the library's, so its replays may overlap anything
+ * that leaves the caller's own buffers alone.
  */
 int fgs_render_16x16(int num_rendered, int width, int height,
                      const float* points_xy, const float* rgb_depth, const float* conic_opacity,
@@ -231,10 +232,10 @@ int fgs_blend_ex(int block_x, int block_y, int width, int height,
                  uint8_t* out_color_u8, float* out_color_f32, int flags, void* stream);
 
 /*
- * No counterpart in the reference.  Name of the kernel(s) a blend with these flags launches on
- * the current device for this tile and frame size (the choice depends on how many tiles the frame
- * has against what the chip holds at once), as a profiler lists them; "" for an unsupported tile
- * size or unknown flags.  Lets a benchmark attribute its figures to the kernel that ran.
+ * No counterpart in the reference.  Name of the kernel(s) a blend with these flags launches for this
+ * tile and frame size outside stream capture (frames of at most 8192 tiles have their tiles ranked
+ * first), as a profiler lists them; "" for an unsupported tile size or unknown flags.  Lets a
+ * benchmark attribute its figures to the kernel that ran.
  */
 const char* fgs_blend_kernel_name(int block_x, int block_y, int width, int height, int flags);
 

@@ -149,3 +149,15 @@ def test_blends_on_different_streams_have_tables_of_their_own(runtime, block):
     launches = enqueued(runtime, [[*block, 640, 360, 0x10000, 0x70, 2], [*block, 640, 360, 0x20000, 0x80, 2]])
     tables = {stream: {t for _, s, _, t in launches if s == stream} for stream in (0x70, 0x80)}
     assert len(launches) == 8 and all(len(t) == 1 for t in tables.values()) and tables[0x70] != tables[0x80]
+
+
+@pytest.mark.parametrize("block", [(16, 16), (32, 16), (32, 32)])
+def test_captured_blends_hold_no_table(runtime, block):
+    launches = enqueued(runtime, [[*block, 640, 360, 0x10000, 0x70, 2]], capturing=True)
+    assert launches == [[0, 0x70, 0x10000, None]] * 2
+
+
+@pytest.mark.parametrize("block", [(16, 16), (32, 16), (32, 32)])
+def test_blends_without_memory_for_a_table_go_unranked(runtime, block):
+    launches = enqueued(runtime, [[*block, 640, 360, 0x10000, 0x70, 2]], no_memory=True)
+    assert launches == [[0, 0x70, 0x10000, None]] * 2
