@@ -500,11 +500,12 @@ __device__ __forceinline__ int walk_list(
             record[3] = slots_of(parts_of(by + co.z), pcy);
             const Parts twice = {2.0f * pcz.hi, 2.0f * pcz.mid, 2.0f * pcz.lo}, none = {0.0f, 0.0f, 0.0f};
             record[4] = slots_of(twice, none);
+            const bool unused = lane >= cnt;            // holds no colour: a weight of zero would make NaN of an infinite one
             if constexpr (kFp32) {
-                *reinterpret_cast<float4*>(bytes + kColours + 16 * lane) = make_float4(rgb.x, rgb.y, rgb.z, ratio);
+                *reinterpret_cast<float4*>(bytes + kColours + 16 * lane) =
+                    make_float4(unused ? 0.0f : rgb.x, unused ? 0.0f : rgb.y, unused ? 0.0f : rgb.z, ratio);
             } else {
                 _Float16* const colour = reinterpret_cast<_Float16*>(bytes + kColours + 32 * (lane >> 2)) + (lane & 3);
-                const bool unused = lane >= cnt;        // holds no colour
                 colour[0] = (_Float16)(unused ? 0.0f : clamped_to_f16(rgb.x));
                 colour[4] = (_Float16)(unused ? 0.0f : clamped_to_f16(rgb.y));
                 colour[8] = (_Float16)(unused ? 0.0f : clamped_to_f16(rgb.z));
@@ -572,7 +573,7 @@ __device__ __forceinline__ int walk_list(
                 auto colour = [&](int j) { return lds_read<float4>(colour_at + 16 * j); };
                 // Gaussians go in pairs, the stop is tested after each pair; a colour is read while the
                 // Gaussian ahead of it is shaded.  The second half of an odd tail (render.cu:486-487) is an
-                // unused slot: its weights are zero.
+                // unused slot: its weights and its colour are zero.
 #define FGS_PAIR(J)                                                                    \
                 second = colour((J) + 1);                                                  \
                 shade((J), first);                                                         \

@@ -1,0 +1,84 @@
+"""Blends of hand-made tile lists through fgs_blend against the oracle's pair-by-pair walk: what a list may
+hold beyond what fgs_preprocess makes."""
+import numpy as np
+import pytest
+
+from flashgs_amd import cabi
+
+pytestmark = pytest.mark.gpu
+
+BLOCKS = [(16, 16), (32, 16), (32, 32)]
+
+
+def column_of_tiles(lists, tiles):
+    """Lists of (xy, conic_opacity, rgb) for tile 0, 1, ... of a frame one tile wide: (points_xy, rgb_depth,
+    conic_opacity, values, ranges), the list positions shuffled over the Gaussian indices."""
+    lengths = np.array([len(l[0]) for l in lists])
+    ends = np.cumsum(lengths)
+    ranges = np.zeros((tiles, 2), np.int32)
+    ranges[:len(lists)] = np.stack([ends - lengths, ends], 1)
+    xy, co, rgb = (np.concatenate([np.asarray(l[i], np.float64) for l in lists]) for i in range(3))
+    n = len(xy)
+    values = np.random.default_rng(n).permutation(n).astype(np.uint32)
+    at = np.empty(n, np.int64)
+    at[values] = np.arange(n)
+    rgbd = np.concatenate([rgb, np.ones((n, 1))], 1)
+    return tuple(np.ascontiguousarray(a[at], dtype=np.float32) for a in (xy, rgbd, co)) + (values, ranges)
+
+
+def gpu_blend(block, W, H, arrays, bg, flags=None):
+    """(float image, 8-bit image) of fgs_blend(_ex)."""
+    import gpu_pipeline as gp
+    import torch
+    xy, rgbd, co, values, ranges = arrays
+    d = [gp.dev(a) for a in (xy, rgbd, co, values.view(np.int32), ranges)]
+    out = torch.full((H, W, 3), -1.0, device=gp.DEV, dtype=torch.float32)
+    out_u8 = torch.full((H, W, 3), 77, device=gp.DEV, dtype=torch.uint8)
+    cabi.blend(block[0], block[1], W, H, d[0].data_ptr(), d[1].data_ptr(), d[2].data_ptr(), d[3].data_ptr(), d[4].data_ptr(),
+               bg, out_u8.data_ptr(), out.data_ptr(), torch.cuda.current_stream().cuda_stream, flags=flags)
+    torch.cuda.synchronize()
+    return out.cpu().numpy(), out_u8.cpu().numpy()
+
+
+def frame_height(block, W, ranked, lists):
+    """(tiles, height) of a frame one tile wide with room for the lists, whose tiles are ranked by list length or are too many
+    for that."""
+    import gpu_pipeline  # noqa: F401  (torch before the library)
+    tiles = lists if ranked else 8200
+    H = tiles * block[1]
+    assert ("tile_order_kernel" in cabi.blend_kernel_name(block[0], block[1], W, H)) == ranked
+    return tiles, H
+
+
+@pytest.mark.parametrize("ranked", [True, False])
+@pytest.mark.parametrize("block", BLOCKS)
+def test_last_of_an_odd_list_may_have_an_infinite_colour(oracle, block, ranked):
+    """A list ends behind its last Gaussian (render.cu:486-487), also where there is no second one of its pair: an infinite
+    colour of it stays infinite and does not meet a weight of zero.  The other colours: sums of weights
+    that are exact to some 1e-6 each, over at most 65 Gaussians of colours up to 1."""
+    rng = np.random.default_rng(5)
+    lists = []
+    for n in (1, 2, 3, 15, 16, 17, 31, 47, 63, 64, 65):
+        for kind in ("colour", "negative colour", "colour in front"):
+            c = rng.uniform(0, 16, (n, 2))
+            c[:, 1] += block[1] * len(lists)
+            co = np.stack([-rng.uniform(1e-4, 1e-3, n), np.zeros(n), -rng.uniform(1e-4, 1e-3, n), np.log2(rng.uniform(0.01, 0.05, n))], 1)
+            rgb = rng.uniform(0, 1, (n, 3))
+            if kind == "colour":
+                rgb[-1, 0] = np.inf
+            elif kind == "negative colour":
+                rgb[-1, 1] = -np.inf
+            else:
+                rgb[max(n - 2, 0), 2] = np.inf
+            lists.append((c, co, rgb))
+    W = 7
+    tiles, H = frame_height(block, W, ranked, len(lists))
+    arrays = column_of_tiles(lists, tiles)
+    bg = np.array([0.25, 0.5, 0.75], np.float32)
+    ref_u8, ref, _ = oracle.render(W, H, block[0], block[1], *arrays, bg)
+    out, out_u8 = gpu_blend(block, W, H, arrays, bg)
+    assert np.isinf(ref).any() and not np.isnan(ref).any()
+    finite = np.isfinite(ref)
+    assert np.array_equal(np.isfinite(out), finite) and np.array_equal(out[~finite], ref[~finite])
+    assert np.abs(out[finite] - ref[finite]).max() <= 1e-4
+    assert np.array_equal(out_u8[~finite], ref_u8[~finite])
