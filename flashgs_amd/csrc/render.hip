@@ -211,10 +211,12 @@ __device__ __forceinline__ uint8_t encode_u8(float x)
 // three parts fill six slots of a half; five instructions make 16 values and 16 slopes per lane.
 //
 // The recurrence starts at the strip's first weight, so that one must not be flushed to zero while a
-// later one matters.  With a curvature along the strip in [-3, 0] (preprocess adds 0.3 to the variances,
-// so its curvatures are above -2.41) it is not: where 2^q_0 < 2^-126, no weight of the strip is above
-// 2^-27 of the opacity.  64 Gaussians with one among them that is out of this range (or out of what
-// the parts hold) are blended by evaluating every exponent (walk_plain).
+// later one matters.  Along the strip q_t = Q + cz (t - t0)^2 with Q = w + dx^2 (cy^2 - 4 cx cz) / (-4 cz).
+// With cz in [-3, 0] and Q <= 20 it is not: q_0 < -126 means -cz t0^2 > 126 + Q, and then q_3 is below
+// Q - (sqrt(126 + Q) - 3 sqrt(3))^2, 2^-27 or less; a rho_0 with a first weight above zero is below 2^42.  A
+// semidefinite form, which fgs_preprocess makes up to roundings, has Q <= w and by the 0.3 it adds to the variances, in exact
+// arithmetic, cz > -2.41.  64 Gaussians with one among them that is out of this range (or out of what the parts
+// hold) are blended by evaluating every exponent (walk_plain).
 //
 // What bounds the launch is the vector unit: 25 fp32 instructions at 2 cycles and two exponentials at 8
 // per Gaussian and wave, about 10 cycles of staging and stop tests on top.  Measured: 98 cycles per
@@ -228,6 +230,7 @@ typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 constexpr int kBatch = 16;                  // Gaussians per matrix product
 constexpr int kChunk = kWave;               // Gaussians staged at a time, one per lane
 constexpr int kStopBelow = 0x38d1b717;      // 0.0001f: a pixel with less transmittance left is opaque
+constexpr float kMostExponent = 20.0f;      // of a Gaussian that the recurrence takes
 constexpr int kNeverStop = -2147483647 - 1;
 
 // An fp32 number as the sum of three bf16 numbers: eight bits of the significand each.
@@ -479,7 +482,9 @@ __device__ __forceinline__ int walk_list(
         const float ex = xy.x - (left + 8.0f), ey = xy.y - (top + 8.0f);
         const float bx = -__builtin_fmaf(2.0f * co.x, ex, co.y * ey), by = -__builtin_fmaf(2.0f * co.z, ey, co.y * ex);
         float c = __builtin_fmaf(ex, __builtin_fmaf(co.x, ex, co.y * ey), __builtin_fmaf(co.z * ey, ey, co.w));
-        const bool fits = co.z <= 0.0f && co.z >= -3.0f &&
+        const float reach = __builtin_fabsf(ex) + 8.0f;         // of the square's columns from the centre
+        const bool fits = co.z <= 0.0f && co.z >= -3.0f && co.w <= kMostExponent &&
+                          __builtin_fmaf(co.y, co.y, -4.0f * co.x * co.z) * (reach * reach) <= 4.0f * co.z * (co.w - kMostExponent) &&
                           __builtin_fabsf(c) + __builtin_fabsf(bx) + __builtin_fabsf(by) + __builtin_fabsf(co.x) < 1.0e9f;
         if (ballot(!fits) != 0) {
             const int walked = walk_plain<kFp32>(xy, co, rgb, cnt, left, top, stop_below, T, sums);

@@ -52,14 +52,14 @@ def frame_height(block, W, ranked, lists):
 
 @pytest.mark.parametrize("ranked", [True, False])
 @pytest.mark.parametrize("block", BLOCKS)
-def test_last_of_an_odd_list_may_have_an_infinite_colour(oracle, block, ranked):
+def test_last_of_an_odd_list_may_be_infinite(oracle, block, ranked):
     """A list ends behind its last Gaussian (render.cu:486-487), also where there is no second one of its pair: an infinite
-    colour of it stays infinite and does not meet a weight of zero.  The other colours: sums of weights
+    colour or weight of it stays infinite and does not meet a weight of zero.  The other colours: sums of weights
     that are exact to some 1e-6 each, over at most 65 Gaussians of colours up to 1."""
     rng = np.random.default_rng(5)
     lists = []
     for n in (1, 2, 3, 15, 16, 17, 31, 47, 63, 64, 65):
-        for kind in ("colour", "negative colour", "colour in front"):
+        for kind in ("colour", "negative colour", "weight", "colour in front"):
             c = rng.uniform(0, 16, (n, 2))
             c[:, 1] += block[1] * len(lists)
             co = np.stack([-rng.uniform(1e-4, 1e-3, n), np.zeros(n), -rng.uniform(1e-4, 1e-3, n), np.log2(rng.uniform(0.01, 0.05, n))], 1)
@@ -68,8 +68,10 @@ def test_last_of_an_odd_list_may_have_an_infinite_colour(oracle, block, ranked):
                 rgb[-1, 0] = np.inf
             elif kind == "negative colour":
                 rgb[-1, 1] = -np.inf
-            else:
+            elif kind == "colour in front":
                 rgb[max(n - 2, 0), 2] = np.inf
+            else:
+                co[-1, 3] = 300.0
             lists.append((c, co, rgb))
     W = 7
     tiles, H = frame_height(block, W, ranked, len(lists))
@@ -82,3 +84,45 @@ def test_last_of_an_odd_list_may_have_an_infinite_colour(oracle, block, ranked):
     assert np.array_equal(np.isfinite(out), finite) and np.array_equal(out[~finite], ref[~finite])
     assert np.abs(out[finite] - ref[finite]).max() <= 1e-4
     assert np.array_equal(out_u8[~finite], ref_u8[~finite])
+
+
+@pytest.mark.parametrize("ranked", [True, False])
+@pytest.mark.parametrize("flags", ["fp32", "f16"])
+@pytest.mark.parametrize("block", BLOCKS)
+def test_exponents_that_rise_steeply_along_a_column(oracle, block, flags, ranked):
+    """Conics whose exponent starts below -126 at the first pixel of a strip of four and is near zero at another one of
+    them: saddles (cx > 0, or cy^2 > 4 cx cz) with a curvature along the strip between -3 and 0, beside
+    needles that are semidefinite to a rounding.  Frames one pixel wide, so that no column has weights
+    above 1.  Bound: up to six terms of magnitude M < 2000, each rounded by M 2^-24, times ln 2 and a weight of
+    up to 0.9, over lists whose weights sum to less than 2; 2^-10 of a colour more with f16 operands."""
+    rng = np.random.default_rng(6)
+    lists = []
+    for i in range(48):
+        n = (1, 2, 7, 16, 33, 64)[i % 6]
+        rows = np.arange(block[1])
+        cz = -rng.uniform(0.3, 3.0, n)
+        dx = rng.uniform(2.0, 14.0, n) * rng.choice([-1, 1], n)
+        if i % 3 == 0:
+            cx, cy = rng.uniform(0.1, 1.0, n), np.zeros(n)
+        elif i % 3 == 1:
+            cx = -rng.uniform(0.1, 1.0, n)
+            cy = rng.choice([-1, 1], n) * rng.uniform(2.5, 6.0, n) * np.sqrt(cx * cz)
+        else:
+            cx = -rng.uniform(0.1, 3.0, n)
+            cy = rng.choice([-1, 1], n) * 2 * np.sqrt(cx * cz) * (1 + rng.uniform(-1e-6, 1e-6, n))
+        dy0 = rng.uniform(-4, block[1] + 4, n)              # centre's row
+        co = np.stack([cx, cy, cz, np.zeros(n)], 1)
+        d = dy0[:, None] - rows
+        peak = (cx * dx * dx)[:, None] + cz[:, None] * d * d + cy[:, None] * dx[:, None] * d
+        # (an opacity that the form with f16 operands does not hold down)
+        co[:, 3] = np.minimum(np.log2(rng.uniform(0.3, 0.9, n) / (1 if n < 3 else 0.5 * n)) - peak.max(1), 1.5)
+        lists.append((np.stack([dx, dy0 + block[1] * i], 1), co, rng.uniform(0, 1, (n, 3))))
+    W = 1
+    tiles, H = frame_height(block, W, ranked, len(lists))
+    arrays = column_of_tiles(lists, tiles)
+    bg = np.array([0.25, 0.5, 0.75], np.float32)
+    _, ref, _ = oracle.render(W, H, block[0], block[1], *arrays, bg, want_u8=False)
+    out, _ = gpu_blend(block, W, H, arrays, bg, cabi.BLEND_FP32 if flags == "fp32" else cabi.BLEND_MATRIX_F16)
+    err = np.abs(out - ref)
+    assert np.isfinite(err).all()
+    assert err.max() <= 6 * 2000 * 2.0 ** -24 * 0.69 * 2 + (2.0 ** -10 if flags == "f16" else 0.0), "max abs image error %g" % err.max()
