@@ -732,8 +732,8 @@ constexpr int kBlendWaves = kFp32 ? 5 : 4;       // resident waves per SIMD
 // wave for a whole 32x32 tile needs 64 registers for its colour sums, leaves two waves per SIMD, and
 // a frame of 3600 such tiles ends with the longest lists on single waves: 1200 us for 1M Gaussians
 // at 2560x1440 against 377 us; 32x16 tiles at 1599x901 384 against 217.)  The stop is the tile's, not the
-// wave's: a wave that finds its own square stopped waits until all have, and those that stopped
-// earlier than the last one walk on to where it did.
+// wave's: a wave that finds its own square stopped waits until all have, those that stopped
+// earlier than the last one walk on to where it did, and the tile stops there if all are still opaque.
 // Resident waves: 5 per SIMD is what 96 registers allow (4: the same time on the largest frames, 3 to 5 %
 // more on the others; 6 spills).
 template <int SX, int SY, bool kFp32>
@@ -741,7 +741,7 @@ __global__ __launch_bounds__(kWave * SX * SY) __attribute__((amdgpu_waves_per_eu
 {
     constexpr int kSquares = SX * SY;
     __shared__ __align__(16) float s_stage[kSquares][kStageFloats];
-    __shared__ int s_walked[kSquares];
+    __shared__ int s_walked[kSquares], s_stopped[kSquares];
 
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = kSquares == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
@@ -770,19 +770,33 @@ __global__ __launch_bounds__(kWave * SX * SY) __attribute__((amdgpu_waves_per_eu
     const int left = (tile_x * SX + wave % SX) * 16, top = (tile_y * SY + wave / SX) * 16;
     int done = 0, upto = n;
     int stop_below = kStopBelow;
-    for (;;) {          // once, or for a wave of a wide tile that stopped before the others once more
+    for (;;) {
         const int walked = walk_list<kFp32>(role, s_stage[wave], point_list, range.x + done, upto - done, (float)left, (float)top,
                                             points_xy, rgb_depth, conic_opacity, T, sums, stop_below);
-        if (kSquares == 1 || stop_below == kNeverStop) break;
-        done = walked < 0 ? ~walked : walked;
-        if (lane == 0) s_walked[wave] = done;
-        __syncthreads();
-        upto = 0;
+        if (kSquares == 1) break;
+        done += walked < 0 ? ~walked : walked;
+        if (stop_below == kStopBelow) {
+            if (lane == 0) s_walked[wave] = done;
+            __syncthreads();
+            upto = 0;
 #pragma unroll
-        for (int w = 0; w < kSquares; w++) upto = max(upto, s_walked[w]);
-        upto = __builtin_amdgcn_readfirstlane(upto);
-        stop_below = kNeverStop;       // whatever is left of it, to the common end
-        if (done >= upto) break;
+            for (int w = 0; w < kSquares; w++) upto = max(upto, s_walked[w]);
+            upto = __builtin_amdgcn_readfirstlane(upto);
+            stop_below = kNeverStop;        // to where the last one stopped
+            if (done < upto) continue;
+        }
+        // All waves are at the same pair, the first one behind which the tile can stop.  A weight above 1
+        // turns the sign of T: then a square that had stopped need not be opaque any more.
+        if (upto >= n) break;
+        const bool stopped = all_stopped(T, kStopBelow);
+        if (lane == 0) s_stopped[wave] = stopped;
+        __syncthreads();
+        bool all = true;
+#pragma unroll
+        for (int w = 0; w < kSquares; w++) all = all && s_stopped[w] != 0;
+        if (__builtin_amdgcn_readfirstlane(all)) break;
+        upto = n;
+        stop_below = kStopBelow;
     }
     Pixels px;
     finish<kFp32>(s_stage[wave], T, sums, px);

@@ -126,3 +126,83 @@ def test_exponents_that_rise_steeply_along_a_column(oracle, block, flags, ranked
     err = np.abs(out - ref)
     assert np.isfinite(err).all()
     assert err.max() <= 6 * 2000 * 2.0 ** -24 * 0.69 * 2 + (2.0 ** -10 if flags == "f16" else 0.0), "max abs image error %g" % err.max()
+
+
+def stops(T, squares, threshold):
+    """Transmittances [pairs, pixels] of a tile behind every pair, and the square of every pixel: (the pair behind which all
+    pixels have T < threshold, the last of the pairs behind which each square by itself first has)."""
+    below = T < threshold
+    first = [np.flatnonzero(b) for b in [below.all(1)] + [below[:, squares == s].all(1) for s in range(squares.max() + 1)]]
+    first = [f[0] if len(f) else len(T) for f in first]
+    return first[0], max(first[1:])
+
+
+@pytest.mark.parametrize("flags", ["fp32", "f16"])
+@pytest.mark.parametrize("block", [(32, 16), (32, 32)])
+def test_a_wide_tile_stops_where_all_of_it_is_opaque_at_once(oracle, block, flags):
+    """Weights above 1 (opacities up to 3) turn the sign of T, so a square of a wide tile that was opaque can be
+    transparent again before the other squares are opaque: the tile goes on (render.cu:394-408).  Lists are drawn until
+    some of them have such a history, none of it within a rounding of the threshold or with a product of weight and T that
+    f16 operands cannot hold (4).  The bound: some 1e-6 per weight, times up to 3.5, a dozen weights of colours up to 1; with
+    f16 operands 2^-10 of each weight's colour more."""
+    rng = np.random.default_rng(8)
+    y, x = np.mgrid[:block[1], :block[0]]
+    squares = (x // 16 + (block[0] // 16) * (y // 16)).ravel()
+    lists, late = [], 0
+    while late < 12:
+        n = int(rng.integers(6, 16))
+        c = rng.uniform(-2, 34, (n, 2)) * (1, block[1] / 32)
+        cx, cz = -rng.uniform(0.0002, 0.004, n), -rng.uniform(0.0002, 0.004, n)
+        op = rng.choice([1.2, 1.6, 2.2, 3.0, 0.99], n)
+        dx, dy = c[:, 0, None] - x.ravel(), c[:, 1, None] - y.ravel()
+        alpha = op[:, None] * 2.0 ** (cx[:, None] * dx * dx + cz[:, None] * dy * dy)
+        T = np.cumprod(1.0 - alpha, 0)
+        heaviest = np.abs(alpha[1:] * T[:-1]).max()
+        (together, alone), low, high = (stops(T[1::2], squares, t) for t in (1e-4, 0.95e-4, 1.05e-4))
+        if heaviest > 3.5 or not low == high == (together, alone) or (together == alone and len(lists) - late > 12):
+            continue
+        late += together > alone
+        c[:, 1] += block[1] * len(lists)
+        lists.append((c, np.stack([cx, np.zeros(n), cz, np.log2(op)], 1), rng.uniform(0, 1, (n, 3))))
+    W, H = block[0], block[1] * len(lists)
+    arrays = column_of_tiles(lists, len(lists))
+    bg = np.array([0.25, 0.5, 0.75], np.float32)
+    _, ref, _ = oracle.render(W, H, block[0], block[1], *arrays, bg, want_u8=False)
+    out, _ = gpu_blend(block, W, H, arrays, bg, cabi.BLEND_FP32 if flags == "fp32" else cabi.BLEND_MATRIX_F16)
+    for i in range(len(lists)):
+        rows = slice(i * block[1], (i + 1) * block[1])
+        assert np.abs(out[rows] - ref[rows]).max() <= 1e-4 + (15 * 3.5 * 2.0 ** -10 if flags == "f16" else 0.0), i
+
+
+@pytest.mark.parametrize("flags", ["fp32", "f16"])
+@pytest.mark.parametrize("block", [(32, 16), (32, 32)])
+def test_squares_of_a_wide_tile_walk_on_to_its_stop(oracle, block, flags):
+    """One square of a tile is opaque (T < 1e-4) early, the tile late, and Gaussians of colour 1e4 lie between the two and
+    behind the tile's stop: what lies between reaches the opaque square with up to 0.3, what lies behind reaches
+    nothing.  Bound: relative errors of some 1e-6 of the weights, and of 1e-4 of a T that is a product of ten
+    1 - 0.99; 2^-10 more with f16 operands."""
+    rng = np.random.default_rng(9)
+    lists, early = [], []
+    for square in range(block[0] // 16 * (block[1] // 16)):
+        for n_between in (2, 5, 18, 70):
+            left, top = square % 2 * 16, square // 2 * 16
+            head = [(left + 7.5, top + 7.5, -0.005, -0.005, 0.99, 1.0)] * 10
+            between = [(16.0, 16.0, -1e-6, -1e-6, 0.3 if n_between < 10 else 0.02, 1e4)] * n_between
+            close = [(16.0, 16.0, -1e-6, -1e-6, 0.99, 0.5)] * 12
+            behind = [(16.0, 16.0, -1e-6, -1e-6, 0.9, 1e4)] * 4
+            x, y, cx, cz, op, bright = np.array(head + between + close + behind).T
+            n = len(x)
+            early.append((len(lists) * block[1] + top, left, len(lists)))
+            lists.append((np.stack([x, y + block[1] * len(lists)], 1), np.stack([cx, np.zeros(n), cz, np.log2(op)], 1),
+                          bright[:, None] * rng.uniform(0.5, 1, (n, 3))))
+    W, H = block[0], block[1] * len(lists)
+    arrays = column_of_tiles(lists, len(lists))
+    bg = np.array([0.25, 0.5, 0.75], np.float32)
+    _, ref, walked = oracle.render(W, H, block[0], block[1], *arrays, bg, want_u8=False)
+    _, short, _ = oracle.render(W, H, block[0], block[1], *column_of_tiles([[a[:10] for a in l] for l in lists], len(lists)),
+                                bg, want_u8=False)
+    out, _ = gpu_blend(block, W, H, arrays, bg, cabi.BLEND_FP32 if flags == "fp32" else cabi.BLEND_MATRIX_F16)
+    bound = 1e-3 + (1e-5 + (2.0 ** -9 if flags == "f16" else 0.0)) * np.abs(ref)
+    for y, x, _ in early:
+        assert np.abs(ref - short)[y:y + 16, x:x + 16].max() > 0.02     # the lists are what the test is about
+    assert (np.abs(out - ref) <= bound).all(), np.abs(out - ref).max()
