@@ -458,8 +458,9 @@ __device__ __forceinline__ int walk_list(
     const float4* __restrict__ conic_opacity,
     float (&T)[4], Sums<kFp32>& sums, int stop_below = kStopBelow)
 {
-    const int last = begin + n - 1;
     const int lane = role.lane;
+    // the entry `ahead` of this lane's first (unsigned: behind the last entries of a list that ends near 2^31)
+    auto entry = [&](uint32_t ahead) { return point_list[min((uint32_t)begin + ahead + (uint32_t)lane, (uint32_t)begin + (uint32_t)n - 1u)]; };
     char* const bytes = reinterpret_cast<char*>(stage);
     // registers hold the chunk that is staged next; loads for it overlap the shading of the current
     // one.  The list index is fetched two chunks ahead and the attributes one chunk ahead, so that no
@@ -469,8 +470,8 @@ __device__ __forceinline__ int walk_list(
     float4 co = make_float4(0.f, 0.f, 0.f, 0.f), rgb = make_float4(0.f, 0.f, 0.f, 0.f);
     uint32_t g_ahead = 0;
     if (n > 0) {
-        const uint32_t g = point_list[min(begin + lane, last)];
-        g_ahead = point_list[min(begin + kChunk + lane, last)];
+        const uint32_t g = entry(0);
+        g_ahead = entry(kChunk);
         xy = points_xy[g]; co = conic_opacity[g]; rgb = rgb_depth[g];
     }
 
@@ -490,7 +491,7 @@ __device__ __forceinline__ int walk_list(
             const int walked = walk_plain<kFp32>(xy, co, rgb, cnt, left, top, stop_below, T, sums);
             if (walked < 0) return ~(base + ~walked);
             xy = points_xy[g_ahead]; co = conic_opacity[g_ahead]; rgb = rgb_depth[g_ahead];
-            g_ahead = point_list[min(begin + base + 2 * kChunk + lane, last)];
+            g_ahead = entry((uint32_t)base + 2 * kChunk);
             continue;
         }
         if (lane >= cnt) c = -1.0e30f;          // a slot past the end of the list: every weight is zero
@@ -520,7 +521,7 @@ __device__ __forceinline__ int walk_list(
         }
         __builtin_amdgcn_wave_barrier();
         xy = points_xy[g_ahead]; co = conic_opacity[g_ahead]; rgb = rgb_depth[g_ahead];
-        g_ahead = point_list[min(begin + base + 2 * kChunk + lane, last)];
+        g_ahead = entry((uint32_t)base + 2 * kChunk);
 
         const char* record = bytes + role.record_at;
         uint32_t colour_off = kColours + (kFp32 ? 0 : 8 * (lane & 3));

@@ -206,3 +206,40 @@ def test_squares_of_a_wide_tile_walk_on_to_its_stop(oracle, block, flags):
     for y, x, _ in early:
         assert np.abs(ref - short)[y:y + 16, x:x + 16].max() > 0.02     # the lists are what the test is about
     assert (np.abs(out - ref) <= bound).all(), np.abs(out - ref).max()
+
+
+@pytest.mark.parametrize("block", BLOCKS)
+def test_lists_that_end_with_the_last_pair_an_int_can_count(block):
+    """Indices of later entries are fetched ahead of the walk: at the end of 2^31 - 1 pairs they are not to leave the int's
+    range.  The same lists at the start of the pairs give the same bits."""
+    import gpu_pipeline as gp
+    import torch
+    most = 2 ** 31 - 1
+    if torch.cuda.mem_get_info()[0] < 4 * most + (1 << 30):
+        pytest.skip("no memory for 2^31 - 1 values")
+    rng = np.random.default_rng(10)
+    lengths = [1500, 769, 300, 129, 128, 127, 65, 64, 63, 2, 1]
+    lists = []
+    for i, n in enumerate(lengths):
+        c = rng.uniform(-4, 20, (n, 2)) + (0, block[1] * i)
+        co = np.stack([-rng.uniform(0.005, 0.1, n), np.zeros(n), -rng.uniform(0.005, 0.1, n), np.log2(rng.uniform(0.0005, 0.01, n))], 1)
+        lists.append((c, co, rng.uniform(0, 1, (n, 3))))
+    W, H = 16, block[1] * len(lists)
+    xy, rgbd, co, values, ranges = column_of_tiles(lists, len(lists))
+    bg = np.array([0.25, 0.5, 0.75], np.float32)
+    expected, _ = gpu_blend(block, W, H, (xy, rgbd, co, values, ranges), bg)
+    K = len(values)
+    d = [gp.dev(a) for a in (xy, rgbd, co)]
+    all_values = torch.empty(most, device=gp.DEV, dtype=torch.int32)
+    all_values[most - K:] = gp.dev(values.view(np.int32))
+    for last in range(len(lists)):          # every list in turn ends with the last pair
+        there = ranges.astype(np.int64) + most - ranges[last, 1]
+        there[last + 1:] = 0
+        all_values[most - ranges[last, 1]:] = gp.dev(values[:ranges[last, 1]].view(np.int32))
+        dr = gp.dev(there.astype(np.int32))
+        out = torch.full((H, W, 3), -1.0, device=gp.DEV, dtype=torch.float32)
+        cabi.blend(block[0], block[1], W, H, d[0].data_ptr(), d[1].data_ptr(), d[2].data_ptr(), all_values.data_ptr(),
+                   dr.data_ptr(), bg, 0, out.data_ptr(), torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        rows = (last + 1) * block[1]
+        assert np.array_equal(out.cpu().numpy()[:rows], expected[:rows]), lengths[last]
