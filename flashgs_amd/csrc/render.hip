@@ -215,8 +215,13 @@ __device__ __forceinline__ uint8_t encode_u8(float x)
 // With cz in [-3, 0] and Q <= 20 it is not: q_0 < -126 means -cz t0^2 > 126 + Q, and then q_3 is below
 // Q - (sqrt(126 + Q) - 3 sqrt(3))^2, 2^-27 or less; a rho_0 with a first weight above zero is below 2^42.  A
 // semidefinite form, which fgs_preprocess makes up to roundings, has Q <= w and by the 0.3 it adds to the variances, in exact
-// arithmetic, cz > -2.41.  64 Gaussians with one among them that is out of this range (or out of what the parts
-// hold) are blended by evaluating every exponent (walk_plain).
+// arithmetic, cz > -2.41.  From the 64 Gaussians with the first one beyond cz = -3 on, a list is walked with four
+// exponentials per strip, of exponents summed up from the same value and slope (walk_chunks<.., true>); 64 with
+// one among them that is out of what that takes too are blended by evaluating every exponent (walk_plain).  The
+// two forms are loops behind each other: side by side in one loop they cost the first 20 to 60 spilled registers.
+// A 4K frame of 3M with all its conics beyond -3: 900 us by walk_plain, 495 so (467 with exponents from tables over the
+// tile); with one in a hundred beyond 430, 323 (335); with none 295.  1080p of 1M: 283, 166 (150); 217, 161 (150); 143.
+// The same with 32x16 tiles: 700, 390 (760); 610, 466 (760); 447.
 //
 // What bounds the launch is the vector unit: 25 fp32 instructions at 2 cycles and two exponentials at 8
 // per Gaussian and wave, about 10 cycles of staging and stop tests on top.  Measured: 98 cycles per
@@ -230,7 +235,10 @@ typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 constexpr int kBatch = 16;                  // Gaussians per matrix product
 constexpr int kChunk = kWave;               // Gaussians staged at a time, one per lane
 constexpr int kStopBelow = 0x38d1b717;      // 0.0001f: a pixel with less transmittance left is opaque
-constexpr float kMostExponent = 20.0f;      // of a Gaussian that the recurrence takes
+constexpr float kMostExponent = 20.0f;      // of a Gaussian that the matrix product takes
+// Curvature along the strip up to which exponents are summed up: value and slopes are rounded at some 200 times it, to
+// 1e-3 at most (as from tables over the tile).
+constexpr float kSharpest = 64.0f;
 constexpr int kNeverStop = -2147483647 - 1;
 
 // An fp32 number as the sum of three bf16 numbers: eight bits of the significand each.
@@ -359,9 +367,11 @@ struct LaneRole {
 template <bool kFp32>
 __device__ __forceinline__ void clear(float (&T)[4], Sums<kFp32>& sums)
 {
+    float one = 1.0f;
+    asm volatile("" : "+v"(one));       // made here, not kept (in private memory, by then) from one job of a wave to the next
 #pragma unroll
     for (int k = 0; k < 4; k++) {
-        T[k] = 1.0f;
+        T[k] = one;
         if constexpr (kFp32) { sums.r[k] = 0.0f; sums.g[k] = 0.0f; sums.b[k] = 0.0f; }
         else sums.acc[k] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
     }
@@ -397,7 +407,8 @@ template <bool kFp32>
 __device__ __forceinline__ int walk_plain(float2 xy, float4 co, float4 rgb, int cnt, float left, float top, int stop_below,
                                                     float (&T)[4], Sums<kFp32>& sums)
 {
-    const int lane = lane_id();
+    int lane = lane_id();
+    asm volatile("" : "+v"(lane));      // as in write_square
     int x, y;
     pixel_of(lane, 0, &x, &y);
     for (int i = 0; i < cnt; i += 2) {
@@ -443,40 +454,40 @@ __device__ __forceinline__ int walk_plain(float2 xy, float4 co, float4 rgb, int 
     return cnt;
 }
 
-// One wave blends entries [begin, begin + n) of the sorted list into the 16x16 pixels whose first pixel
-// is (left, top), front to back, on top of T and sums; begin must be an even distance from the start
-// of the tile's list, so that the pairs are the reference's pairs.  The walk ends after the pair behind
-// which all 256 pixels have T < stop_below (render.cu:394-408).  Returns the entries walked, or ~entries
-// when that stop ended the walk.  stage: this wave's kStageFloats of LDS.
-template <bool kFp32>
-__device__ __forceinline__ int walk_list(
+// What a wave holds of a list ahead of its walk: the attributes of the chunk that comes next, one Gaussian per lane, and
+// the indices for the chunk behind it.  The list index is fetched two chunks ahead and the attributes one chunk ahead, so
+// that no wave waits for an index only to start the loads that depend on it.  Positions past the end of the list are
+// clamped to its last entry: those loads are valid and their result unused.  (Positions are unsigned: a list may end
+// with pair 2^31 - 1.)
+struct Ahead {
+    float2 xy;
+    float4 co, rgb;
+    uint32_t index;
+};
+
+// walk_list below from its entry base on, in chunks of 64: to the first chunk that the recurrence does not take, or
+// (kSteep) to the end.  Returns as walk_list does, or base of the chunk it ended in front of.
+template <bool kFp32, bool kSteep>
+__device__ __forceinline__ int walk_chunks(
     const LaneRole& role, float* stage,
     const uint32_t* __restrict__ point_list, int begin, int n,
     float left, float top,
     const float2* __restrict__ points_xy,
     const float4* __restrict__ rgb_depth,
     const float4* __restrict__ conic_opacity,
-    float (&T)[4], Sums<kFp32>& sums, int stop_below = kStopBelow)
+    float (&T)[4], Sums<kFp32>& sums, int stop_below, Ahead& next, int base)
 {
     const int lane = role.lane;
-    // the entry `ahead` of this lane's first (unsigned: behind the last entries of a list that ends near 2^31)
-    auto entry = [&](uint32_t ahead) { return point_list[min((uint32_t)begin + ahead + (uint32_t)lane, (uint32_t)begin + (uint32_t)n - 1u)]; };
     char* const bytes = reinterpret_cast<char*>(stage);
-    // registers hold the chunk that is staged next; loads for it overlap the shading of the current
-    // one.  The list index is fetched two chunks ahead and the attributes one chunk ahead, so that no
-    // wave waits for an index only to start the loads that depend on it.  Positions past the end of the
-    // list are clamped to its last entry: those loads are valid and their result unused.
-    float2 xy = make_float2(0.f, 0.f);
-    float4 co = make_float4(0.f, 0.f, 0.f, 0.f), rgb = make_float4(0.f, 0.f, 0.f, 0.f);
-    uint32_t g_ahead = 0;
-    if (n > 0) {
-        const uint32_t g = entry(0);
-        g_ahead = entry(kChunk);
-        xy = points_xy[g]; co = conic_opacity[g]; rgb = rgb_depth[g];
-    }
-
-    for (int base = 0; base < n; base += kChunk) {
+    auto fetch = [&]() {
+        next.xy = points_xy[next.index]; next.co = conic_opacity[next.index]; next.rgb = rgb_depth[next.index];
+        next.index = point_list[min((uint32_t)begin + (uint32_t)base + 2u * kChunk + (uint32_t)lane, (uint32_t)begin + (uint32_t)n - 1u)];
+    };
+    for (; base < n; base += kChunk) {
         const int cnt = min(kChunk, n - base);
+        const float2 xy = next.xy;
+        const float4 rgb = next.rgb;
+        float4 co = next.co;
         // conic_opacity = (cx, cy, cz, w) in the units of the exponent (see fgs_preprocess).  With f16
         // weights log2 of the opacity is held below 2 so that no scaled weight leaves f16's range.
         if constexpr (!kFp32) co.w = (co.w > 1.99f ? 1.99f : co.w) + kWeightScaleLog2;
@@ -484,18 +495,18 @@ __device__ __forceinline__ int walk_list(
         const float bx = -__builtin_fmaf(2.0f * co.x, ex, co.y * ey), by = -__builtin_fmaf(2.0f * co.z, ey, co.y * ex);
         float c = __builtin_fmaf(ex, __builtin_fmaf(co.x, ex, co.y * ey), __builtin_fmaf(co.z * ey, ey, co.w));
         const float reach = __builtin_fabsf(ex) + 8.0f;         // of the square's columns from the centre
-        const bool fits = co.z <= 0.0f && co.z >= -3.0f && co.w <= kMostExponent &&
+        const bool fits = co.z <= 0.0f && co.z >= -(kSteep ? kSharpest : 3.0f) && co.w <= kMostExponent &&
                           __builtin_fmaf(co.y, co.y, -4.0f * co.x * co.z) * (reach * reach) <= 4.0f * co.z * (co.w - kMostExponent) &&
                           __builtin_fabsf(c) + __builtin_fabsf(bx) + __builtin_fabsf(by) + __builtin_fabsf(co.x) < 1.0e9f;
         if (ballot(!fits) != 0) {
+            if constexpr (!kSteep) return base;
             const int walked = walk_plain<kFp32>(xy, co, rgb, cnt, left, top, stop_below, T, sums);
             if (walked < 0) return ~(base + ~walked);
-            xy = points_xy[g_ahead]; co = conic_opacity[g_ahead]; rgb = rgb_depth[g_ahead];
-            g_ahead = entry((uint32_t)base + 2 * kChunk);
+            fetch();
             continue;
         }
         if (lane >= cnt) c = -1.0e30f;          // a slot past the end of the list: every weight is zero
-        const float ratio = __builtin_amdgcn_exp2f(2.0f * co.z);
+        const float ratio = kSteep ? 2.0f * co.z : __builtin_amdgcn_exp2f(2.0f * co.z);
         __builtin_amdgcn_wave_barrier();
         {
             const Parts pcz = parts_of(co.z), pcy = parts_of(co.y);
@@ -520,8 +531,7 @@ __device__ __forceinline__ int walk_list(
             }
         }
         __builtin_amdgcn_wave_barrier();
-        xy = points_xy[g_ahead]; co = conic_opacity[g_ahead]; rgb = rgb_depth[g_ahead];
-        g_ahead = entry((uint32_t)base + 2 * kChunk);
+        fetch();
 
         const char* record = bytes + role.record_at;
         uint32_t colour_off = kColours + (kFp32 ? 0 : 8 * (lane & 3));
@@ -556,11 +566,19 @@ __device__ __forceinline__ int walk_list(
             // the weights of Gaussian j of the batch along the strip
             auto weights = [&](int j, float E, float (&alpha)[4]) {
                 alpha[0] = __builtin_amdgcn_exp2f(q[j]);
-                float rho = __builtin_amdgcn_exp2f(d[j]);
-                // (zero times anything is zero here: a slope beyond the range of fp32 belongs to a value of zero)
-                alpha[1] = mul_zero_wins(alpha[0], rho); rho *= E;
-                alpha[2] = mul_zero_wins(alpha[1], rho); rho *= E;
-                alpha[3] = mul_zero_wins(alpha[2], rho);
+                if constexpr (kSteep) {         // (E is the slope's step)
+                    float at = q[j] + d[j], slope = d[j] + E;
+                    alpha[1] = __builtin_amdgcn_exp2f(at);
+                    at += slope; slope += E;
+                    alpha[2] = __builtin_amdgcn_exp2f(at);
+                    alpha[3] = __builtin_amdgcn_exp2f(at + slope);
+                } else {
+                    float rho = __builtin_amdgcn_exp2f(d[j]);
+                    // (zero times anything is zero here: a slope beyond the range of fp32 belongs to a value of zero)
+                    alpha[1] = mul_zero_wins(alpha[0], rho); rho *= E;
+                    alpha[2] = mul_zero_wins(alpha[1], rho); rho *= E;
+                    alpha[3] = mul_zero_wins(alpha[2], rho);
+                }
             };
             if constexpr (kFp32) {
                 // render.cu:40-52, operation for operation
@@ -641,6 +659,36 @@ __device__ __forceinline__ int walk_list(
     return n;
 }
 
+// One wave blends entries [begin, begin + n) of the sorted list into the 16x16 pixels whose first pixel
+// is (left, top), front to back, on top of T and sums; begin must be an even distance from the start
+// of the tile's list, so that the pairs are the reference's pairs.  The walk ends after the pair behind
+// which all 256 pixels have T < stop_below (render.cu:394-408).  Returns the entries walked, or ~entries
+// when that stop ended the walk.  stage: this wave's kStageFloats of LDS.
+template <bool kFp32>
+__device__ __forceinline__ int walk_list(
+    const LaneRole& role, float* stage,
+    const uint32_t* __restrict__ point_list, int begin, int n,
+    float left, float top,
+    const float2* __restrict__ points_xy,
+    const float4* __restrict__ rgb_depth,
+    const float4* __restrict__ conic_opacity,
+    float (&T)[4], Sums<kFp32>& sums, int stop_below = kStopBelow)
+{
+    const int lane = role.lane;
+    Ahead next = {};
+    if (n > 0) {
+        const uint32_t last = (uint32_t)begin + (uint32_t)n - 1u;
+        const uint32_t g = point_list[min((uint32_t)begin + (uint32_t)lane, last)];
+        next.index = point_list[min((uint32_t)begin + kChunk + (uint32_t)lane, last)];
+        next.xy = points_xy[g]; next.co = conic_opacity[g]; next.rgb = rgb_depth[g];
+    }
+    const int walked = walk_chunks<kFp32, false>(role, stage, point_list, begin, n, left, top, points_xy, rgb_depth, conic_opacity,
+                                                 T, sums, stop_below, next, 0);
+    if (walked < 0 || walked >= n) return walked;
+    return walk_chunks<kFp32, true>(role, stage, point_list, begin, n, left, top, points_xy, rgb_depth, conic_opacity,
+                                    T, sums, stop_below, next, walked);
+}
+
 // The wave's pixels out of T and the colour sums.
 template <bool kFp32>
 __device__ __forceinline__ void finish(float* stage, const float (&T)[4], const Sums<kFp32>& sums, Pixels& px)
@@ -679,6 +727,7 @@ __device__ __forceinline__ void write_square(
     int lane, int left, int top, int width, int height, const Pixels& px,
     float bg_r, float bg_g, float bg_b, uint8_t* __restrict__ out_u8, float* __restrict__ out_f32)
 {
+    asm volatile("" : "+v"(lane));      // what follows from it is computed here, not kept through the walk
 #pragma unroll
     for (int k = 0; k < 4; k++) {
         int x, y;

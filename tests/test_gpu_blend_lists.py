@@ -243,3 +243,34 @@ def test_lists_that_end_with_the_last_pair_an_int_can_count(block):
         torch.cuda.synchronize()
         rows = (last + 1) * block[1]
         assert np.array_equal(out.cpu().numpy()[:rows], expected[:rows]), lengths[last]
+
+
+@pytest.mark.parametrize("ranked", [True, False])
+@pytest.mark.parametrize("flags", ["fp32", "f16"])
+@pytest.mark.parametrize("block", BLOCKS)
+def test_splats_sharper_than_a_pixel(oracle, block, flags, ranked):
+    """Conics with a curvature along the strip beyond the recurrence's -3 (splats that were not widened by 0.3): up to -64,
+    where exponents are summed up, and beyond, in lists around the chunk of 64, from the first Gaussian on, from later ones
+    on, or in turn with others.  Bound: with a centre within 12 pixels the exponent's terms are below 64 * 144 + the
+    like across, 18432, and are rounded three times, and slopes below 1536 up to three times each: 1.7e-3, times ln 2, on a
+    weight of up to 0.6; beyond -64 every exponent is evaluated.  The 2^-10 of f16 operands on top."""
+    rng = np.random.default_rng(11)
+    lists = []
+    for i in range(60):
+        n = (1, 2, 15, 17, 63, 64, 65, 128, 131, 200)[i % 10]
+        c = rng.uniform(-2, 18, (n, 2)) + (0, block[1] * i + rng.uniform(0, block[1] - 16))
+        cx, cz = -rng.uniform(0.02, 0.5, n), -rng.uniform(0.02, 0.5, n)
+        sharp = np.arange(n) >= (0, n // 2, 70)[i % 3] if i % 4 else np.arange(n) % 5 == 1
+        cz[sharp] = -np.exp(rng.uniform(np.log(3.0), np.log(64.0 if i % 5 else 1000.0), sharp.sum()))
+        cx[sharp] = -np.exp(rng.uniform(np.log(0.1), np.log(64.0), sharp.sum()))
+        cy = rng.uniform(-0.95, 0.95, n) * 2 * np.sqrt(cx * cz)
+        lists.append((c, np.stack([cx, cy, cz, np.log2(rng.uniform(0.05, 0.6, n))], 1), rng.uniform(0, 1, (n, 3))))
+    W = 16
+    tiles, H = frame_height(block, W, ranked, len(lists))
+    arrays = column_of_tiles(lists, tiles)
+    bg = np.array([0.25, 0.5, 0.75], np.float32)
+    _, ref, _ = oracle.render(W, H, block[0], block[1], *arrays, bg, want_u8=False)
+    out, _ = gpu_blend(block, W, H, arrays, bg, cabi.BLEND_FP32 if flags == "fp32" else cabi.BLEND_MATRIX_F16)
+    err = np.abs(out - ref)
+    assert np.isfinite(err).all()
+    assert err.max() <= 0.6 * 0.69 * 1.7e-3 + (2.0 ** -10 if flags == "f16" else 0.0), "max abs image error %g" % err.max()
