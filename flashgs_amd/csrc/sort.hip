@@ -1108,19 +1108,17 @@ __device__ __forceinline__ bool sort_segment_waves(uint64_t* __restrict__ keys, 
 }
 
 // Segment sort by the waves of a workgroup for one size class: segments with min_len < length <= kCap.
-// With a table of segment starts, workgroup w looks at the kIds tile ids [w*kIds, (w+1)*kIds),
-// one per lane, and sorts those of its class one after the other.  Without a table (more tile ids
-// than the table holds) the grid has one workgroup per tile id and each searches for its bounds.
-template <int kWaves, int kCap, int kLeast, int kIds>
+// With a table of segment starts, the first launch has listed the segments of the class.  Without a table
+// (more tile ids than it holds) the grid has one workgroup per tile id and each searches for its bounds.
+template <int kWaves, int kCap, int kLeast>
 __global__ __launch_bounds__(kWaves * kWave) void segment_sort_kernel(
-    uint64_t* __restrict__ keys, uint32_t* __restrict__ values, int n, uint32_t tile_mask, int min_len, uint32_t ids,
+    uint64_t* __restrict__ keys, uint32_t* __restrict__ values, int n, uint32_t tile_mask, int min_len,
     const int* __restrict__ seg_start, uint32_t* __restrict__ seg_flags,
     const uint32_t* __restrict__ list, const uint32_t* __restrict__ list_count, uint32_t list_cap)
 {
     __shared__ uint64_t s_w[kCap];
     __shared__ uint32_t s_seen[kWaves];
     __shared__ int s_bounds[2];
-    __shared__ uint64_t s_match;
 
     const int tid = threadIdx.x;
     const int lane = tid & (kWave - 1);
@@ -1139,27 +1137,11 @@ __global__ __launch_bounds__(kWaves * kWave) void segment_sort_kernel(
         return;
     }
 
-    if (list) {      // the segments of this class were listed: deal them out round-robin, shard by shard
-        const uint32_t shard = blockIdx.x % kListShards;
-        const uint32_t count = list_count[shard];
-        for (uint32_t i = blockIdx.x / kListShards; i < count; i += gridDim.x / kListShards) {
-            const uint32_t v = list[(size_t)shard * list_cap + i];
-            sort_segment_waves<kWaves, kCap, kLeast>(keys, values, v, seg_start[v], seg_start[v + 1], seg_flags, s_w, s_seen);
-        }
-        return;
-    }
-
-    const uint32_t first_id = blockIdx.x * (uint32_t)kIds;
-    if (tid < kWave) {
-        const uint32_t v = first_id + (uint32_t)lane;
-        int len = 0;
-        if (lane < kIds && v < ids) len = seg_start[v + 1] - seg_start[v];
-        const uint64_t m = ballot(len > min_len && len <= kCap);
-        if (lane == 0) s_match = m;
-    }
-    __syncthreads();
-    for (uint64_t todo = s_match; todo; todo &= todo - 1) {
-        const uint32_t v = first_id + (uint32_t)(__ffsll((long long)todo) - 1);
+    // the listed segments are dealt out round-robin, shard by shard
+    const uint32_t shard = blockIdx.x % kListShards;
+    const uint32_t count = list_count[shard];
+    for (uint32_t i = blockIdx.x / kListShards; i < count; i += gridDim.x / kListShards) {
+        const uint32_t v = list[(size_t)shard * list_cap + i];
         sort_segment_waves<kWaves, kCap, kLeast>(keys, values, v, seg_start[v], seg_start[v + 1], seg_flags, s_w, s_seen);
     }
 }
@@ -1501,9 +1483,9 @@ extern "C" int fgs_sort_gaussian(int num_rendered,
             const unsigned g = most < limit ? most : limit;
             return (g + kListShards - 1) / kListShards * kListShards;
         };
-#define FGS_SEGMENT_CLASS(WAVES, CAP, LEAST, IDS, MINLEN, GRID, LIST, COUNT, LISTCAP)                                \
-        hipLaunchKernelGGL((segment_sort_kernel<WAVES, CAP, LEAST, IDS>), dim3(GRID), dim3((WAVES) * kWave), 0, st,  \
-                           ks, vs, n, tile_mask, MINLEN, ids, (const int*)seg_start, seg_flags,               \
+#define FGS_SEGMENT_CLASS(WAVES, CAP, LEAST, MINLEN, GRID, LIST, COUNT, LISTCAP)                                \
+        hipLaunchKernelGGL((segment_sort_kernel<WAVES, CAP, LEAST>), dim3(GRID), dim3((WAVES) * kWave), 0, st,  \
+                           ks, vs, n, tile_mask, MINLEN, (const int*)seg_start, seg_flags,               \
                            (const uint32_t*)(LIST), (const uint32_t*)(COUNT), LISTCAP)
         // Up to 512 pairs: one wave, bitonic network in registers; one tile id per wave (neighbouring
         // tiles tend to be equally busy, so a wave that took several of them would become the tail
@@ -1536,16 +1518,16 @@ extern "C" int fgs_sort_gaussian(int num_rendered,
                                    dim3(kWave), 0, st, ks, vs, (const int*)seg_start, seg_flags,
                                    (const uint32_t*)list_small, (const uint32_t*)seg_counts, cap_small);
             if (n > kCapSmall && !merged_tail) {
-                FGS_SEGMENT_CLASS(4, kCapMedium, 8, 64, kCapSmall, list_grid((unsigned)(n / (kCapSmall + 1) + 1), 4096u),
+                FGS_SEGMENT_CLASS(4, kCapMedium, 8, kCapSmall, list_grid((unsigned)(n / (kCapSmall + 1) + 1), 4096u),
                                   list_medium, seg_counts + kListShards, cap_medium);
                 if (n > kCapMedium && !merged_large)
-                    FGS_SEGMENT_CLASS(8, kCapLarge, 16, 64, kCapMedium, list_grid((unsigned)(n / (kCapMedium + 1) + 1), 1024u),
+                    FGS_SEGMENT_CLASS(8, kCapLarge, 16, kCapMedium, list_grid((unsigned)(n / (kCapMedium + 1) + 1), 1024u),
                                       list_large, seg_counts + 2 * kListShards, cap_large);
             }
         } else {
-            if (n > kCapTiny) FGS_SEGMENT_CLASS(4, kCapSmall, 4, 1, kCapTiny, ids, no_list, no_list, 0u);
-            if (n > kCapSmall) FGS_SEGMENT_CLASS(4, kCapMedium, 8, 64, kCapSmall, ids, no_list, no_list, 0u);
-            if (n > kCapMedium) FGS_SEGMENT_CLASS(8, kCapLarge, 16, 64, kCapMedium, ids, no_list, no_list, 0u);
+            if (n > kCapTiny) FGS_SEGMENT_CLASS(4, kCapSmall, 4, kCapTiny, ids, no_list, no_list, 0u);
+            if (n > kCapSmall) FGS_SEGMENT_CLASS(4, kCapMedium, 8, kCapSmall, ids, no_list, no_list, 0u);
+            if (n > kCapMedium) FGS_SEGMENT_CLASS(8, kCapLarge, 16, kCapMedium, ids, no_list, no_list, 0u);
         }
 #undef FGS_SEGMENT_CLASS
         // longer segments from their list, one workgroup per segment; behind them the shorter ones that were flagged
