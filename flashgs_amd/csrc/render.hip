@@ -867,14 +867,11 @@ __global__ __launch_bounds__(kWave * SX * SY) __attribute__((amdgpu_waves_per_eu
 constexpr int kOwnShare = 256;
 constexpr int kMinRest = 512;               // a shorter rest is not worth two barriers: the owner walks it
 constexpr int kSharedWaves = 4;
-// Where every workgroup is resident at once even with one tile each (4 SIMDs of 256 CUs, four waves a
-// workgroup), a tile has a workgroup to itself: three waves of it have no list of their own and only take
-// runs, so a long list has all four instead of a share of them, and the cut into runs stays the same.  256x192
+// Where every workgroup is resident at once even with one tile each (a wave of it on each SIMD of a CU, so up to
+// kBlendWaves workgroups a CU), a tile has a workgroup to itself: three waves of it have no list of their own and
+// only take runs, so a long list has all four instead of a share of them, and the cut into runs stays the same.  256x192
 // pixels, 300k clustered Gaussians 357 -> 245 us, 640x512 100 -> 81, 1M 228 -> 169, with lists too short to be
 // shared 14.8 -> 14.8.  Beyond that (1920x1080, 1M) waves without a list keep others off the chip: 138 -> 159.
-template <bool kFp32>
-constexpr int kSoloTiles = 256 * kBlendWaves<kFp32>;
-
 template <bool kFp32>
 __global__ __launch_bounds__(kSharedWaves * kWave) __attribute__((amdgpu_waves_per_eu(kBlendWaves<kFp32>, kBlendWaves<kFp32>))) void blend_kernel_shared(FGS_BLEND_PARAMS, const uint32_t* __restrict__ tile_order, int tiles_per_group)
 {
@@ -1075,7 +1072,10 @@ int blend_impl(int block_x, int block_y, int width, int height,
                            bg[0], bg[1], bg[2], out_u8, out_f32, (const uint32_t*)tile_order);          \
     } while (0)
     if (is_ranked(tiles_x, tiles_y) && sx == 1 && sy == 1) {
-        const int tiles_per_group = num_tiles <= (fp32 ? kSoloTiles<true> : kSoloTiles<false>) ? 1 : kSharedWaves;
+        int device = 0, cus = 0;
+        FGS_HIP_TRY(hipGetDevice(&device));
+        FGS_HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
+        const int tiles_per_group = num_tiles <= cus * (fp32 ? kBlendWaves<true> : kBlendWaves<false>) ? 1 : kSharedWaves;
         hipLaunchKernelGGL(fp32 ? blend_kernel_shared<true> : blend_kernel_shared<false>, dim3((unsigned)((num_tiles + tiles_per_group - 1) / tiles_per_group)), dim3(kSharedWaves * kWave), 0, st,
                            (const int2*)ranges, values_sorted, width, height, tiles_x, tiles_y,
                            (const float2*)points_xy, (const float4*)rgb_depth, (const float4*)conic_opacity,

@@ -34,6 +34,7 @@ static __thread dim3 pushed_grid, pushed_block;
 static __thread void *pushed_stream;
 
 int hipGetDevice(int *device) { *device = 0; return 0; }
+int hipDeviceGetAttribute(int *value, int attribute, int device) { (void)attribute; (void)device; *value = 256; return 0; }
 int hipGetLastError(void) { return 0; }
 int hipMalloc(void **p, size_t bytes) { *p = no_memory ? NULL : malloc(bytes); return *p ? 0 : 2; }
 int hipGetSymbolAddress(void **p, const void *symbol) { *p = (void *)symbol; return 0; }
