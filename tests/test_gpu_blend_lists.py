@@ -274,3 +274,75 @@ def test_splats_sharper_than_a_pixel(oracle, block, flags, ranked):
     err = np.abs(out - ref)
     assert np.isfinite(err).all()
     assert err.max() <= 0.6 * 0.69 * 1.7e-3 + (2.0 ** -10 if flags == "f16" else 0.0), "max abs image error %g" % err.max()
+
+
+def exact_blend(block, W, H, arrays, bg):
+    """The pair-by-pair walk of every tile's list in float64: (image, T of every pixel)."""
+    xy, rgbd, co, values, ranges = arrays
+    xy, rgbd, co = (a.astype(np.float64) for a in (xy, rgbd, co))
+    gx = -(-W // block[0])
+    out = np.zeros((-(-H // block[1]) * block[1], gx * block[0], 3))
+    remaining = np.ones(out.shape[:2])
+    for t, (lo, hi) in enumerate(ranges):
+        y, x = np.mgrid[t // gx * block[1]:(t // gx + 1) * block[1], t % gx * block[0]:(t % gx + 1) * block[0]]
+        g = values[lo:hi]
+        dx, dy = xy[g, 0, None, None] - x, xy[g, 1, None, None] - y
+        cx, cy, cz, w = (co[g, i, None, None] for i in range(4))
+        alpha = np.exp2(w + cx * dx * dx + cz * dy * dy + cy * dx * dy)
+        T = np.concatenate([np.ones((1,) + x.shape), np.cumprod(1.0 - alpha, 0)])
+        stops = np.flatnonzero((T[2::2] < 1e-4).all((1, 2)))            # behind pair 0, 1, ...
+        n = 2 * (stops[0] + 1) if len(stops) else hi - lo
+        left = np.where(T[n] < 1e-4, 0.0, T[n])
+        remaining[y, x] = T[n]
+        out[y, x] = np.einsum("nyx,nc->yxc", alpha[:n] * T[:n], rgbd[g[:n], :3]) + left[..., None] * bg
+    return out[:H, :W], remaining[:H, :W]
+
+
+#: smallest and largest standard deviation of a splat along its axes in pixels, before it is widened by 0.3
+SPLATS = {"small": (0.1, 2.0), "medium": (3.0, 20.0), "wide": (20.0, 300.0), "needles": (0.1, 100.0)}
+
+
+@pytest.mark.parametrize("block", BLOCKS)
+@pytest.mark.parametrize("splats", sorted(SPLATS))
+def test_error_against_float64(oracle, block, splats):
+    """The fp32 blend of conics as fgs_preprocess makes them against a float64 evaluation, beside an fp32 evaluation of
+    render.cu:42-52 term by term (the oracle's).  Bound: half as much again as that, and twice as much at the
+    worst pixel, for the other order of the sums; on top, for splats of a pixel, whose exponent is a sum of terms of up to
+    2 * 2.4 * 12^2 = 700 where term by term it is small: two roundings of 700 * 2^-25 times ln 2 and a weight of up to 0.5, 1.4e-5 at
+    the worst pixel, and a twentieth of it over all."""
+    lo, hi = SPLATS[splats]
+    rng = np.random.default_rng(12)
+    lists = []
+    for i in range(24):
+        n = int(rng.integers(20, 250))
+        sigma = np.exp(rng.uniform(np.log(lo), np.log(hi), (n, 2)))
+        if splats == "needles":
+            sigma = np.stack([np.exp(rng.uniform(np.log(30.0), np.log(hi), n)), rng.uniform(lo, 0.5, n)], 1)
+        angle = rng.uniform(0, np.pi, n)
+        c, s = np.cos(angle), np.sin(angle)
+        a, b = sigma[:, 0] ** 2, sigma[:, 1] ** 2
+        xx, yy, xy = a * c * c + b * s * s + 0.3, a * s * s + b * c * c + 0.3, (a - b) * c * s
+        det = xx * yy - xy * xy
+        half_log2e = 0.5 * 1.4426950408889634
+        # a centre within two standard deviations of a pixel of the tile
+        r = 2 * np.sqrt(rng.uniform(0, 1, n))
+        phi = rng.uniform(0, 2 * np.pi, n)
+        u, v = r * np.cos(phi) * sigma[:, 0], r * np.sin(phi) * sigma[:, 1]
+        centre = rng.uniform(0, 1, (n, 2)) * block + np.stack([u * c - v * s, u * s + v * c], 1)
+        lists.append((centre + (0, block[1] * i),
+                      np.stack([-half_log2e * yy / det, 2 * half_log2e * xy / det, -half_log2e * xx / det,
+                                np.log2(rng.uniform(0.02, 0.5, n))], 1), rng.uniform(0, 1, (n, 3))))
+    W, H = block[0], block[1] * len(lists)
+    arrays = column_of_tiles(lists, len(lists))
+    bg = np.array([0.25, 0.5, 0.75], np.float32)
+    exact, T = exact_blend(block, W, H, arrays, bg.astype(np.float64))
+    _, plain, _ = oracle.render(W, H, block[0], block[1], *arrays, bg, want_u8=False)
+    out, _ = gpu_blend(block, W, H, arrays, bg)
+    scale = np.sqrt((exact ** 2).mean())
+    same = np.abs(T / 1e-4 - 1) > 0.05        # where T is 1e-4 but for a rounding, the background stays or goes
+    rms = [np.sqrt(((i - exact)[same] ** 2).mean()) / scale for i in (out, plain)]
+    worst = [np.abs(i - exact)[same].max() for i in (out, plain)]
+    print("%s %dx%d: rms error / rms value %.2e (term by term %.2e), largest error %.2e (%.2e)"
+          % (splats, block[0], block[1], rms[0], rms[1], worst[0], worst[1]))
+    assert same.mean() > 0.99
+    assert rms[0] <= 1.5 * rms[1] + 7e-7 and worst[0] <= 2 * worst[1] + 1.4e-5

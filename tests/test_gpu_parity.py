@@ -120,8 +120,8 @@ def test_large_splats_all_tile_sizes(oracle, block):
 
 @pytest.mark.parametrize("block", [(32, 16), (32, 32)])
 def test_wide_tiles_on_a_frame_with_many_tiles(oracle, block):
-    """5120x2880 has more tiles than the chip holds at once even at 32x32 (160x90 = 14 400):
-    the blend then runs its variant with fewer resident waves."""
+    """5120x2880 has more than 8192 tiles even at 32x32 (160x90 = 14 400): the blend then takes them in blocks of 8x8 per XCD
+    and does not rank them by list length."""
     sc = scenes.config0(n=40_000)
     cam = sc.cameras[0]
     scale = 2880 / cam.height
@@ -843,14 +843,16 @@ def _blend_lists(oracle, lists, W, H, bg, seed, colour_hi=1.5, flags=None):
     return out.cpu().numpy(), ref
 
 
-@pytest.mark.parametrize("W,H", [(320, 240), (3840, 400)])       # the kernel of small frames and the one of large frames
+@pytest.mark.parametrize("W,H", [(320, 240), (3840, 560)])       # the kernel of small frames and the one of large frames
 def test_blend_faint_weights_keep_their_relative_accuracy(oracle, W, H):
     """With FGS_BLEND_MATRIX_F16 the colour sums take their weights as f16.  Lists of thousands of Gaussians whose weights
     alpha*T lie between 1e-8 and 1e-5, far below f16's smallest normal number 6e-5, still add up to
     colours that are right to 2^-10 of themselves: the weights are scaled before the conversion."""
     gx = (W + 15) // 16
     lists = [(t, 1500 + 37 * (t % 5), op) for t, op in zip(range(0, 12 * gx, gx + 3), [1e-5, 3e-6, 1e-6, 3e-7, 1e-7, 1e-8] * 2)]
+    import torch  # noqa: F401  (before the library)
     from flashgs_amd import cabi
+    assert ("shared" in cabi.blend_kernel_name(16, 16, W, H)) == (W == 320)
     got, ref = _blend_lists(oracle, lists, W, H, (0.0, 0.0, 0.0), seed=5, flags=cabi.BLEND_MATRIX_F16)
     lit = ref > 0
     assert lit.any() and ref[lit].max() < 0.05                      # faint sums, nothing near 1
@@ -917,19 +919,19 @@ def test_colour_sum_modes_per_call_and_by_default(oracle, W, H, block):
 
 @pytest.mark.parametrize("block", [(16, 16), (32, 16), (32, 32)])
 @pytest.mark.parametrize("flags", ["fp32", "f16"])
-@pytest.mark.parametrize("size", [(96, 70), (4096, 1040)])        # with the tiles ranked by list length and without
-def test_blend_batch_edges_and_conics_beyond_the_recurrence(oracle, block, flags, size):
+@pytest.mark.parametrize("ranked", [True, False])         # with the tiles ranked by list length and without
+def test_blend_batch_edges_and_conics_beyond_the_recurrence(oracle, block, flags, ranked):
     """List lengths around the batch of 16 and the chunk of 64 Gaussians, and conics on both sides of
     what the recurrence along a pixel strip takes (curvature in [-3, 0]): needles, splats far narrower
-    than a pixel, saddles, centres far outside the tile, an opacity of zero.  One Gaussian out of range
-    sends its 64 through the plain evaluation.  Bound: the colour weights are exact to the exponent's
+    than a pixel, saddles, centres far outside the tile, an opacity of zero.  Bound: the colour weights are exact to the exponent's
     rounding, at most 6 terms of magnitude M with M 2^-24 each, times ln 2; M < 300 for everything that
     reaches a pixel here, so 1e-4 of a colour per Gaussian at its most and far less on average; with f16
     operands 2^-10 of the colour on top."""
     import gpu_pipeline as gp
     from flashgs_amd import cabi
     import torch
-    W, H = size
+    W, H = (96, 70) if ranked else (4096, 65 * block[1])
+    assert ("tile_order_kernel" in cabi.blend_kernel_name(block[0], block[1], W, H)) == ranked
     gx, gy = (W + block[0] - 1) // block[0], (H + block[1] - 1) // block[1]
     rng = np.random.default_rng(17)
     lengths = [0, 1, 2, 3, 15, 16, 17, 31, 33, 63, 64, 65, 79, 127, 128, 129, 200]
