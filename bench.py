@@ -40,8 +40,8 @@ FP32_PEAK_TFLOPS = 157.3         # MI355X fp32 vector, published (packed FMA)
 FLOP_PER_EVAL = 19               # render.cu:40-52: 2 sub, 6 mul + 3 add, 1 mul, 3 FMA, 1 sub
 EXEC_SLOTS_PER_EVAL = 7.4        # non-transcendental VALU instructions the fp32 blend kernel issues per evaluation (SQ counters,
                                  # profiles/frame_cfg2_3M_4K_sq_counters.txt, without the 0.08 matrix instructions): 1.25 for the weight
-                                 # from its recurrence, alpha*T, T -=, 3 colour FMAs, the rest staging, stop tests and loop; half a
-                                 # v_exp_f32 beside them.  Some of them issue faster than the v_fma_f32 of the calibration.
+                                 # from its recurrence, alpha*T, T -=, 3 colour FMAs, the rest staging, stop tests and loop.  Half a
+                                 # v_exp_f32 beside them is not priced.
 ATTAINED_FMA_LANE_OPS = 38.05e12 # v_fma_f32 lane-operations/s measured on this part without packed math (bench.py --calibrate)
 CAPACITY = {0: 1 << 20, 1: 1 << 22, 2: 1 << 24, 3: 1 << 25, 4: 1 << 25, 5: 1 << 27, 6: 1 << 25}
 FAST_MODE_DTYPE = "f32 (colour sums: f16 operands on the matrix unit, fp32 products and sums)"
@@ -68,6 +68,8 @@ def parse():
                     help="also run one 256 MiB device-to-device copy, as the known-size reference for FETCH_SIZE / WRITE_SIZE")
     ap.add_argument("--size", default=None, metavar="WxH",
                     help="frame size for the trajectory workload (config 4), e.g. 3840x2160; default 1920x1080")
+    ap.add_argument("--details", default=None, metavar="FILE",
+                    help="write the full report of every configuration, of which the printed line holds the main figures, to FILE as JSON")
     ap.add_argument("--calibrate", action="store_true",
                     help="also measure what this GPU attains on a stream copy, a stream read and fp32 FMA / exp2 issue "
                          "(libflashgs_calibrate.so) and report it under \"calibration\"")
@@ -100,10 +102,13 @@ def calibrate(torch, dev):
     mix4 = call(lib.fgs_cal_alu, C.c_int(1), C.c_void_p(sink.data_ptr()))
     mix8 = call(lib.fgs_cal_alu, C.c_int(2), C.c_void_p(sink.data_ptr()))
     exp = call(lib.fgs_cal_alu, C.c_int(3), C.c_void_p(sink.data_ptr()))
+    mul = call(lib.fgs_cal_alu, C.c_int(4), C.c_void_p(sink.data_ptr()))
+    sub = call(lib.fgs_cal_alu, C.c_int(5), C.c_void_p(sink.data_ptr()))
     torch.cuda.synchronize()
     return {
         "copy_GBs_read_plus_write": round(copy / 1e9, 1), "read_GBs": round(read / 1e9, 1),
         "fma_T_lane_ops_per_s": round(fma / 1e12, 2), "fma_TFLOPs": round(2 * fma / 1e12, 2),
+        "mul_T_lane_ops_per_s": round(mul / 1e12, 2), "sub_T_lane_ops_per_s": round(sub / 1e12, 2),
         "exp2_plus_sub_T_lane_ops_per_s": round(exp / 1e12, 2),
         "fma_and_exp2_4to1_T_lane_ops_per_s": round(mix4 / 1e12, 2),
         "fma_and_exp2_8to1_T_lane_ops_per_s": round(mix8 / 1e12, 2),
@@ -333,8 +338,9 @@ def stage_report(fr, stage_ms, K, counts, walked):
     tile_passes = (int(tiles).bit_length() + 7) // 8
     stages["sort"]["design_bytes"] = int(K * (32 * tile_passes + 8 + 24))   # count + scatter per tile digit, starts, segment sort
     hbm("ranges", 8 * K + 16 * tiles)
-    stages["readback"] = dict(ms=round(stage_ms["readback"], 4), bound="host latency: GPU time between the preprocess launch and the first sort launch (the host polls "
-                                   "the pair count in pinned memory and enqueues the sort while the launch still writes keys)")
+    # GPU time between the preprocess launch and the first sort launch (the host polls the pair count in pinned memory and
+    # enqueues the sort while the launch still writes keys)
+    stages["readback"] = dict(ms=round(stage_ms["readback"], 4), bound="host latency")
 
     blend_ms = stage_ms["blend"]
     kernel = fr.cabi.blend_kernel_name(16, 16, W, H)        # of the library default, which is what was timed
@@ -397,6 +403,22 @@ def ops_surface_ms(torch, np, fr, steps):
     return round(ms, 4), same, round(batch_ms, 4)
 
 
+def brief(rep):
+    """The main figures of a configuration's report: the printed line has to stay short enough to be kept whole."""
+    flight = rep["two_frames_in_flight"] or {}
+    out = {"ms_per_frame": rep["ms_per_frame"], "fps": rep["fps"], "pairs": rep["pairs"],
+           "stages_ms": {k: v["ms"] for k, v in rep["stages"].items()}, "blend_frac": rep["roofline"]["frac"],
+           "fast_mode_ms": rep["fast_mode"]["ms_per_frame"], "blocking_ms": rep["blocking_readback_ms_per_frame"],
+           "two_in_flight_ms": flight.get("ms_per_frame"), "cpu_ms": (rep["cpu_baseline"] or {}).get("ms_per_frame")}
+    if flight.get("images_identical") is False:
+        out["images_differ"] = True
+    if "trajectory" in rep:
+        t = rep["trajectory"]
+        out["trajectory_ms"] = {"p50": t["frame_ms_p50"], "p99": t["frame_ms_p99"],
+                                "batch": t.get("batch_two_frames_in_flight_ms_per_frame")}
+    return out
+
+
 def run_config(mods, config, size, steps, warmup, cpu_reps, with_cpu, with_ops, base=None, in_flight=True):
     torch, np, cabi, scenes = mods
     fr = Frame(torch, np, cabi, scenes, config, size, base)
@@ -417,14 +439,11 @@ def run_config(mods, config, size, steps, warmup, cpu_reps, with_cpu, with_ops, 
     rep = dict(workload=fr.sc.name, gaussians=fr.n, width=fr.W, height=fr.H, pairs=int(K), poses=len(fr.cams),
                ms_per_frame=round(ms_per_step, 4), fps=round(1000.0 / ms_per_step, 2), dtype="f32", stages=stages,
                roofline=roofline, cpu_baseline=cpu,
-               pair_count="stored into pinned host memory by the launch as soon as it is known and polled there "
-                          "(fgs_preprocess_mirrored / fgs_wait_count)",
+               pair_count="polled in pinned host memory (fgs_preprocess_mirrored / fgs_wait_count)",
                blocking_readback_ms_per_frame=round(blocking_ms, 4),
                two_frames_in_flight=None if flight_ms is None else dict(
-                   ms_per_frame=round(flight_ms, 4), fps=round(1000.0 / flight_ms, 2), images_identical=flight_same,
-                   what="the same frames sent in turn to two streams, each with work buffers and an image of its own: "
-                        "one frame's blend runs beside the next frame's preprocess and sort"),
-               stage_timing="a second pass over the same steps with a HIP event in front of every stage",
+                   ms_per_frame=round(flight_ms, 4), fps=round(1000.0 / flight_ms, 2), images_identical=flight_same),
+               stage_timing="second pass, HIP events",
                ms_per_frame_with_stage_events=round(instrumented_ms, 4),
                fast_mode=dict(dtype=FAST_MODE_DTYPE, ms_per_frame=round(fast_ms, 4), fps=round(1000.0 / fast_ms, 2),
                               blend_ms=round(fast_stage["blend"], 4),
@@ -489,8 +508,6 @@ def main():
         "n_gpus": 1, "steps": args.steps, "warmup": args.warmup,
         "ms_per_step": head["ms_per_frame"], "higher_is_better": True, "scaling": "weak",
         "vs_baseline": None, "dtype": head["dtype"],
-        "dtype_note": "every stage in fp32 as the reference (ndc2Pix in fp64 as its literals make it); the timed blend "
-                      "kernel is the one named in roofline.kernel",
         "data": "synthetic",
         "config": {"workload": head["workload"], "gaussians": head["gaussians"], "width": head["width"], "height": head["height"],
                    "tile": "16x16", "sh_degree": 3, "pairs": head["pairs"], "poses": head["poses"],
@@ -539,7 +556,10 @@ def main():
             big = fr_o.sc if config == 3 else (None if config == 5 else big)
             del fr_o
             torch.cuda.empty_cache()
-        result["configs"] = others
+        result["configs"] = {name: brief(rep) for name, rep in others.items()}
+    if args.details:
+        with open(args.details, "w") as f:
+            json.dump(dict(result, headline=head, configs=others if not args.headline_only else {}), f, indent=1)
     print(json.dumps(result))
 
 

@@ -30,7 +30,8 @@ __global__ __launch_bounds__(kThreads) void read_kernel(const float4* __restrict
 }
 
 // kChains independent dependency chains per lane, each `iters` long.
-// kExpEvery = 0: FMA only; k > 0: one exp2 after every k FMAs of a chain.
+// kExpEvery = 0: FMA only; k > 0: one exp2 after every k FMAs of a chain; kExpOnly, kMulOnly, kSubOnly: those only.
+constexpr int kExpOnly = -1, kMulOnly = -2, kSubOnly = -3;
 template <int kExpEvery>
 __global__ __launch_bounds__(kThreads) void alu_kernel(float* __restrict__ sink, int iters, float a, float b)
 {
@@ -41,8 +42,14 @@ __global__ __launch_bounds__(kThreads) void alu_kernel(float* __restrict__ sink,
     for (int it = 0; it < iters; it++) {
 #pragma unroll
         for (int c = 0; c < kChains; c++) {
-            if (kExpEvery < 0) {
+            if (kExpEvery == kExpOnly) {
                 x[c] = __builtin_amdgcn_exp2f(x[c]) - 1.0f;          // exp2 only (the subtraction keeps it bounded)
+            } else if (kExpEvery == kMulOnly || kExpEvery == kSubOnly) {
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    x[c] = kExpEvery == kMulOnly ? x[c] * a : x[c] - a;
+                    asm volatile("" : "+v"(x[c]));                   // one instruction each
+                }
             } else {
 #pragma unroll
                 for (int k = 0; k < (kExpEvery > 0 ? kExpEvery : 4); k++) x[c] = __builtin_fmaf(x[c], a, b);
@@ -108,7 +115,8 @@ extern "C" int fgs_cal_read(const void* src, float* sink, size_t bytes, double* 
 
 // Wave64 instructions per second, summed over the chip: mode 0 = v_fma_f32 only, mode 1 = one
 // v_exp_f32 after every four FMAs (reports FMA + exp instructions), mode 2 = the same after every
-// eight, mode 3 = v_exp_f32 + one subtraction only (reports exp instructions only).
+// eight, mode 3 = v_exp_f32 + one subtraction only (reports exp instructions only), mode 4 = v_mul_f32
+// only, mode 5 = v_sub_f32 only.
 extern "C" int fgs_cal_alu(int mode, float* sink, double* lane_ops_per_s, void* stream)
 {
     hipStream_t st = (hipStream_t)stream;
@@ -125,8 +133,14 @@ extern "C" int fgs_cal_alu(int mode, float* sink, double* lane_ops_per_s, void* 
     } else if (mode == 2) {
         rc = timed(st, 3, &ms, [&] { hipLaunchKernelGGL(alu_kernel<8>, dim3(blocks), dim3(kThreads), 0, st, sink, iters, 0.5f, -1.0f); });
         per_chain_iter = 9;
+    } else if (mode == 4) {
+        rc = timed(st, 3, &ms, [&] { hipLaunchKernelGGL(alu_kernel<kMulOnly>, dim3(blocks), dim3(kThreads), 0, st, sink, iters, 0.999f, 0.f); });
+        per_chain_iter = 4;
+    } else if (mode == 5) {
+        rc = timed(st, 3, &ms, [&] { hipLaunchKernelGGL(alu_kernel<kSubOnly>, dim3(blocks), dim3(kThreads), 0, st, sink, iters, 0.001f, 0.f); });
+        per_chain_iter = 4;
     } else {
-        rc = timed(st, 3, &ms, [&] { hipLaunchKernelGGL(alu_kernel<-1>, dim3(blocks), dim3(kThreads), 0, st, sink, iters, 0.f, 0.f); });
+        rc = timed(st, 3, &ms, [&] { hipLaunchKernelGGL(alu_kernel<kExpOnly>, dim3(blocks), dim3(kThreads), 0, st, sink, iters, 0.f, 0.f); });
         per_chain_iter = 1;
     }
     const double lane_ops = (double)blocks * kThreads * 8.0 * iters * per_chain_iter;

@@ -8,12 +8,33 @@ import pytest
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 BENCH = os.path.join(ROOT, "bench.py")
+LONGEST = 7000          # characters of the line that are sure to be kept whole
+CONFIG = 450            # ... and of one of the eight other configurations in it
 
 
 def test_more_than_one_gpu_is_refused_with_a_message():
     done = subprocess.run([sys.executable, BENCH, "--gpus", "2"], capture_output=True, text=True, timeout=120)
     assert done.returncode == 2
     assert "one GPU only" in done.stderr and done.stdout.strip() == ""
+
+
+def test_a_configuration_is_a_few_figures_in_the_line():
+    """The full report of a configuration is some 2500 characters, and a line with eight of them was cut off when it was stored:
+    the line holds their main figures."""
+    sys.path.insert(0, ROOT)
+    import bench
+    stages = {k: {"ms": 1234.5678, "bound": "hbm", "kernel": "x" * 60} for k in ("preprocess", "sort", "ranges", "readback", "blend")}
+    rep = {"ms_per_frame": 1234.5678, "fps": 12345.67, "pairs": 1234567890, "stages": stages,
+           "roofline": {"frac": 0.1234, "kernel": "x" * 60, "achieved_is": "y" * 80}, "fast_mode": {"ms_per_frame": 1234.5678, "dtype": "z" * 90},
+           "blocking_readback_ms_per_frame": 1234.5678, "cpu_baseline": {"ms_per_frame": 12345.67, "sample": "s" * 60},
+           "two_frames_in_flight": {"ms_per_frame": 1234.5678, "images_identical": False},
+           "trajectory": {"frame_ms_p50": 1234.5678, "frame_ms_p99": 1234.5678, "batch_two_frames_in_flight_ms_per_frame": 1234.5678}}
+    short = bench.brief(rep)
+    assert len(json.dumps({"cfg4_2M_orbit_3840x2160_needles_last": short})) <= CONFIG + 40
+    assert short["stages_ms"]["blend"] == 1234.5678 and short["images_differ"] is True
+    del rep["trajectory"]
+    rep.update(cpu_baseline=None, two_frames_in_flight=None)
+    assert bench.brief(rep)["cpu_ms"] is None and "trajectory_ms" not in bench.brief(rep)
 
 
 @pytest.mark.gpu
@@ -26,6 +47,7 @@ def test_the_line_of_a_small_workload_has_every_field():
     lines = [l for l in done.stdout.splitlines() if l.startswith("{")]
     assert len(lines) == 1
     d = json.loads(lines[0])
+    assert len(lines[0]) + 8 * CONFIG < LONGEST
     for key in ("metric", "value", "unit", "n_gpus", "steps", "warmup", "ms_per_step", "higher_is_better", "scaling",
                 "vs_baseline", "dtype", "data", "config", "roofline", "cpu_baseline"):
         assert key in d, key
