@@ -8,8 +8,8 @@
 // matrix unit, while the loads of the following batch are already in flight; then the wave shades its pixels
 // Gaussian by Gaussian.  After every second Gaussian one ballot tests whether all pixels of the tile
 // have T < 1e-4, which is the reference's stop rule (render.cu:394-408).  Every kernel exists in
-// two forms: all fp32, operation for operation the reference's pixel shader (the default), and
-// with the colour sums on the matrix unit too, four Gaussians at a time (f16 operands, fp32
+// two forms: all sums and products in fp32 (the default; from the weight on the operations of the reference's pixel
+// shader, the weight itself by other means than its formula: see below), and with the colour sums on the matrix unit too, four Gaussians at a time (f16 operands, fp32
 // accumulation), which a caller asks for per call (FGS_BLEND_MATRIX_F16) or per process
 // (fgs_set_colour_sums).
 #include "fgs_internal.h"
@@ -187,8 +187,8 @@ __device__ __forceinline__ uint8_t encode_u8(float x)
 // the pixel from the Gaussian's centre (render.cu:42-45), is a quadratic along the strip, so its
 // weights alpha_j = 2^q_j follow from the value and the slope at the strip's first pixel:
 //     alpha_{j+1} = alpha_j rho_j,   rho_{j+1} = rho_j E,   rho_0 = 2^(q_1 - q_0),   E = 2^(2 cz),
-// two exponentials and five multiplications for four pixels.  (v_exp_f32 takes the vector unit 8
-// cycles a wave, a multiplication 2.)
+// two exponentials and five multiplications for four pixels.  (v_exp_f32 takes the vector unit 7 to 8
+// cycles a wave, a multiplication 4.)
 //
 // Values and slopes are a matrix product.  With (X, Y) the strip's first pixel relative to the centre
 // of the square and (ex, ey) the Gaussian's centre relative to it,
@@ -219,14 +219,16 @@ __device__ __forceinline__ uint8_t encode_u8(float x)
 // exponentials per strip, of exponents summed up from the same value and slope (walk_chunks<.., true>); 64 with
 // one among them that is out of what that takes too are blended by evaluating every exponent (walk_plain).  The
 // two forms are loops behind each other: side by side in one loop they cost the first 20 to 60 spilled registers.
-// A 4K frame of 3M with all its conics beyond -3: 900 us by walk_plain, 495 so (467 with exponents from tables over the
-// tile); with one in a hundred beyond 430, 323 (335); with none 295.  1080p of 1M: 283, 166 (150); 217, 161 (150); 143.
-// The same with 32x16 tiles: 700, 390 (760); 610, 466 (760); 447.
+// A 4K frame of 3M with all its conics beyond -3: 900 us by walk_plain, 485 so (467 with exponents from tables over the
+// tile); with one in a hundred beyond 430, 320 (335); with none 300.  1080p of 1M: 282, 160 (150); 218, 157 (150); 142.
+// The same with 32x16 tiles: 700, 382 (760); 605, 461 (760); 443.
 //
-// What bounds the launch is the vector unit: 25 fp32 instructions at 2 cycles and two exponentials at 8
-// per Gaussian and wave, about 10 cycles of staging and stop tests on top.  Measured: 98 cycles per
-// Gaussian and 16x16 pixels in the middle of a launch.  4K frame of 3M Gaussians 336 -> 280 us, 8K of
-// 8M 762 -> 671, 1080p of 1M 147 -> 138, against a version that took the exponents from per-column and
+// What bounds the launch is the issue of vector instructions: 25 fp32 instructions (5 for the recurrence, 4 alpha T, 4 T -=,
+// 12 for the colour sums) and two exponentials per Gaussian and wave, and 4 more for staging, stop tests and loop.
+// Measured on the 4K frame of 3M: 108 cycles per Gaussian and 16x16 pixels, 98 in the middle of a launch.  Chains of
+// v_fma_f32, v_mul_f32 or v_sub_f32 take 4 cycles an instruction and a v_exp_f32 among them 7 to 8, which would be
+// 130: some of the instructions here issue faster than in those chains.  4K frame of 3M Gaussians 336 -> 276 us, 8K of
+// 8M 762 -> 671, 1080p of 1M 147 -> 140, against a version that took the exponents from per-column and
 // per-row tables in LDS (four exponentials, 32 vector instructions).  (Two waves per 16x16 pixels with
 // two pixels per lane and staging shared over barriers: 357 us on the 4K frame.)
 typedef float float16_t __attribute__((ext_vector_type(16)));
@@ -486,17 +488,20 @@ __device__ __forceinline__ int walk_chunks(
     for (; base < n; base += kChunk) {
         const int cnt = min(kChunk, n - base);
         const float2 xy = next.xy;
-        const float4 rgb = next.rgb;
-        float4 co = next.co;
+        float4 co = next.co, rgb = next.rgb;
         // conic_opacity = (cx, cy, cz, w) in the units of the exponent (see fgs_preprocess).  With f16
         // weights log2 of the opacity is held below 2 so that no scaled weight leaves f16's range.
         if constexpr (!kFp32) co.w = (co.w > 1.99f ? 1.99f : co.w) + kWeightScaleLog2;
         const float ex = xy.x - (left + 8.0f), ey = xy.y - (top + 8.0f);
         const float bx = -__builtin_fmaf(2.0f * co.x, ex, co.y * ey), by = -__builtin_fmaf(2.0f * co.z, ey, co.y * ex);
         float c = __builtin_fmaf(ex, __builtin_fmaf(co.x, ex, co.y * ey), __builtin_fmaf(co.z * ey, ey, co.w));
+        // Q over the columns of the square, multiplied out, and the other limits of the walk.  (These checks are made by every wave of
+        // a tile: as comparisons one by one they cost a 1599x901 frame of 32x16 tiles 1.3 %.  A NaN that max drops makes one of
+        // the sum.)
+        const float limit = kSteep ? kSharpest : 3.0f;
         const float reach = __builtin_fabsf(ex) + 8.0f;         // of the square's columns from the centre
-        const bool fits = co.z <= 0.0f && co.z >= -(kSteep ? kSharpest : 3.0f) && co.w <= kMostExponent &&
-                          __builtin_fmaf(co.y, co.y, -4.0f * co.x * co.z) * (reach * reach) <= 4.0f * co.z * (co.w - kMostExponent) &&
+        const float beyond = __builtin_fmaf(__builtin_fmaf(co.y, co.y, -4.0f * co.x * co.z) * reach, reach, 4.0f * co.z * (kMostExponent - co.w));
+        const bool fits = __builtin_fmaxf(__builtin_fmaxf(beyond, co.z), __builtin_fmaxf(-limit - co.z, co.w - kMostExponent)) <= 0.0f &&
                           __builtin_fabsf(c) + __builtin_fabsf(bx) + __builtin_fabsf(by) + __builtin_fabsf(co.x) < 1.0e9f;
         if (ballot(!fits) != 0) {
             if constexpr (!kSteep) return base;
@@ -505,7 +510,13 @@ __device__ __forceinline__ int walk_chunks(
             fetch();
             continue;
         }
-        if (lane >= cnt) c = -1.0e30f;          // a slot past the end of the list: every weight is zero
+        if (cnt < kChunk) {                     // (a branch, not selects for every chunk)
+            asm volatile("");
+            if (lane >= cnt) {                  // a slot past the end of the list: every weight is zero, and so is
+                c = -1.0e30f;                   // the colour, or the weight would make NaN of an infinite one
+                rgb = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            }
+        }
         const float ratio = kSteep ? 2.0f * co.z : __builtin_amdgcn_exp2f(2.0f * co.z);
         __builtin_amdgcn_wave_barrier();
         {
@@ -517,15 +528,13 @@ __device__ __forceinline__ int walk_chunks(
             record[3] = slots_of(parts_of(by + co.z), pcy);
             const Parts twice = {2.0f * pcz.hi, 2.0f * pcz.mid, 2.0f * pcz.lo}, none = {0.0f, 0.0f, 0.0f};
             record[4] = slots_of(twice, none);
-            const bool unused = lane >= cnt;            // holds no colour: a weight of zero would make NaN of an infinite one
             if constexpr (kFp32) {
-                *reinterpret_cast<float4*>(bytes + kColours + 16 * lane) =
-                    make_float4(unused ? 0.0f : rgb.x, unused ? 0.0f : rgb.y, unused ? 0.0f : rgb.z, ratio);
+                *reinterpret_cast<float4*>(bytes + kColours + 16 * lane) = make_float4(rgb.x, rgb.y, rgb.z, ratio);
             } else {
                 _Float16* const colour = reinterpret_cast<_Float16*>(bytes + kColours + 32 * (lane >> 2)) + (lane & 3);
-                colour[0] = (_Float16)(unused ? 0.0f : clamped_to_f16(rgb.x));
-                colour[4] = (_Float16)(unused ? 0.0f : clamped_to_f16(rgb.y));
-                colour[8] = (_Float16)(unused ? 0.0f : clamped_to_f16(rgb.z));
+                colour[0] = (_Float16)clamped_to_f16(rgb.x);
+                colour[4] = (_Float16)clamped_to_f16(rgb.y);
+                colour[8] = (_Float16)clamped_to_f16(rgb.z);
                 colour[12] = (_Float16)0.0f;
                 *reinterpret_cast<float*>(bytes + kRatios + 4 * lane) = ratio;
             }
@@ -581,7 +590,7 @@ __device__ __forceinline__ int walk_chunks(
                 }
             };
             if constexpr (kFp32) {
-                // render.cu:40-52, operation for operation
+                // render.cu:46-52, operation for operation
                 auto shade = [&](int j, const float4& u) {
                     float alpha[4];
                     weights(j, u.w, alpha);

@@ -146,8 +146,13 @@ size_t fgs_get_sort_buffer_size(int num_rendered);
  * csrc/cuda_rasterizer/render.cu:549-608): zero `ranges`, find each tile's [start,end) in the
  * sorted keys, blend front to back and write out_color u8[H,W,3].  `ranges` int32[tiles,2] is
  * scratch that holds the tile ranges afterwards.  bg_color is a host array of 3 floats.
- * All arithmetic is fp32, as in render.cu:40-52, unless the process default was changed with
- * fgs_set_colour_sums (fgs_render_ex / fgs_blend_ex choose per call).
+ * All sums are fp32, as in render.cu:40-52, unless the process default was changed with
+ * fgs_set_colour_sums (fgs_render_ex / fgs_blend_ex choose per call).  The weights of render.cu:42-45 come from
+ * exponents that are a matrix product of fp32 coefficients (each as three bf16 numbers, its whole significand) and from a
+ * recurrence along four pixels; they are as close to exact ones as the formula evaluated term by term in fp32 for
+ * splats of some pixels and more, and some 1e-6 of a colour away for splats of about a pixel.  Conics may be of any kind;
+ * those with a curvature along y beyond -3 (splats that were not widened by 0.3), saddles and non-finite ones take
+ * slower paths.
  * A frame of at most 8192 tiles first ranks its tiles by list length into a table the
  * library keeps per (device, stream) (32 KB, allocated on the first such call on that stream),
  * and with 16x16 tiles the rest of a list of more than 768 entries is blended in four runs that each stop on
@@ -199,7 +204,7 @@ int fgs_blend(int block_x, int block_y, int width, int height,
 /*
  * No counterpart in the reference.  How a blend forms its colour sums C += (alpha T) c.
  *   FGS_COLOUR_SUMS_FP32 (default): by fp32 multiply-add, operation for operation what
- *     render.cu:40-52 does.
+ *     render.cu:46-52 does.
  *   FGS_COLOUR_SUMS_MATRIX_F16 (opt-in, about a fifth faster in the blend of a 4K frame): on the
  *     matrix unit; the weights alpha T and the colours are rounded to f16, products and sums are
  *     fp32: a pixel's colour is within 2^-10 of itself of the all-fp32 sum.  Colours beyond
