@@ -38,7 +38,7 @@ if ROOT not in sys.path:
 HBM_PEAK_GBS = 8000.0            # MI355X HBM3E, published
 FP32_PEAK_TFLOPS = 157.3         # MI355X fp32 vector, published (packed FMA)
 FLOP_PER_EVAL = 19               # render.cu:40-52: 2 sub, 6 mul + 3 add, 1 mul, 3 FMA, 1 sub
-EXEC_SLOTS_PER_EVAL = 7.4        # non-transcendental VALU instructions the fp32 blend kernel issues per evaluation (SQ counters,
+EXEC_SLOTS_PER_EVAL = 7.3        # non-transcendental VALU instructions the fp32 blend kernel issues per evaluation (SQ counters,
                                  # profiles/frame_cfg2_3M_4K_sq_counters.txt, without the 0.08 matrix instructions): 1.25 for the weight
                                  # from its recurrence, alpha*T, T -=, 3 colour FMAs, the rest staging, stop tests and loop.  Half a
                                  # v_exp_f32 beside them is not priced.
