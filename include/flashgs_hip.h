@@ -150,7 +150,7 @@ size_t fgs_get_sort_buffer_size(int num_rendered);
  * fgs_set_colour_sums (fgs_render_ex / fgs_blend_ex choose per call).  The weights of render.cu:42-45 come from
  * exponents that are a matrix product of fp32 coefficients (each as three bf16 numbers, its whole significand) and from a
  * recurrence along four pixels; they are as close to exact ones as the formula evaluated term by term in fp32 for
- * splats of some pixels and more, and some 1e-6 of a colour away for splats of about a pixel.  Conics may be of any kind;
+ * splats of some pixels and more, and within some 6e-6 of a colour for splats of about a pixel.  Conics may be of any kind;
  * those with a curvature along y beyond -3 (splats that were not widened by 0.3), saddles and non-finite ones take
  * slower paths.
  * A frame of at most 8192 tiles first ranks its tiles by list length into a table the
