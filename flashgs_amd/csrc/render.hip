@@ -591,13 +591,17 @@ __device__ __forceinline__ int walk_chunks(
                 }
             };
             if constexpr (kFp32) {
-                // render.cu:46-52, operation for operation
+                // render.cu:46-52, operation for operation.  T -= at stays a subtraction: the product is there for the
+                // colours anyway, and v_fma_f32 with a negated and a repeated operand takes the issue of about two
+                // v_sub_f32 (4K frame of 3M 290 -> 283 us, 8K of 8M 693 -> 674, 1080p of 1M 141 -> 136; errors against
+                // float64 the same to three digits).
                 auto shade = [&](int j, const float4& u) {
                     float alpha[4];
                     weights(j, u.w, alpha);
 #pragma unroll
                     for (int k = 0; k < 4; k++) {
-                        const float at = alpha[k] * T[k];
+                        float at = alpha[k] * T[k];
+                        asm("" : "+v"(at));
                         sums.r[k] += u.x * at;
                         sums.g[k] += u.y * at;
                         sums.b[k] += u.z * at;
