@@ -9,10 +9,10 @@
 //  1. Partition by tile id: one stable counting pass per 8 bits of tile id (two passes for up to
 //     65536 tiles; above that digits of 9 bits, so an 8K frame of 129 600 tiles still takes two).
 //     A pass is count -> offsets -> scatter: `count_chunk_kernel` builds one digit histogram per
-//     block of 4096 pairs (3840 with 9-bit digits) and the sums of every chunk of blocks,
+//     block of 4096 pairs (fewer on shorter lists) and the sums of every chunk of blocks,
 //     `offsets_kernel` turns them into the exclusive start of every (block, digit) run, and
 //     `scatter_kernel` ranks its block in LDS (wave64 ballot matching, so equal digits keep
-//     their input order) and writes each run to its start.  A list of up to 64 blocks takes
+//     their input order) and writes each run to its start.  A short list takes
 //     count -> scatter.  No workgroup ever waits for another one.
 //  2. Sort every tile's segment by the 32 depth bits without touching memory in between: the
 //     last scatter pass also tabulates where each tile id's segment begins (with more than two
@@ -30,39 +30,56 @@
 // 88 for two partition passes, against 8 + 6 * 24 = 152 for a six-pass LSD sort of 47 bits.
 #include "fgs_internal.h"
 
+#include <algorithm>
+
 namespace fgs {
 namespace {
 
 constexpr int kBins = 256;                      // counters of a counting pass inside a segment (8-bit digits)
 constexpr int kSortBlock = 256;
-constexpr int kSortWaves = kSortBlock / kWave;
 constexpr int kXcds = 8;                        // accelerator dies of the device, workgroup i of a launch runs on die i % 8
 
-// Shape of a partition pass: digits of kBitsT bits, kItemsT pairs per thread.  Up to 65 536 tiles
-// two passes of 8 bits do; above that (an 8K frame has 129 600) digits of 9 bits keep it at two
-// passes up to 262 144 tiles, with 15 pairs per thread so that the workgroup's LDS still lets
-// three workgroups share a CU.
-template <int kBitsT, int kItemsT>
+// Shape of a partition pass: digits of kBitsT bits, kItemsT pairs per thread of a scatter workgroup of kThreadsT.
+// Up to 65 536 tiles two passes of 8 bits do; above that (an 8K frame has 129 600) digits of 9 bits keep
+// it at two passes up to 262 144 tiles.
+// A scatter workgroup has sixteen waves with a few pairs per lane each, not four waves with sixteen: ranking 64 pairs is a
+// chain of some hundred instructions that a wave goes through once per pair of its lanes, and with the one or two
+// waves per SIMD that the LDS of a block of 4096 pairs left, a SIMD issued an instruction every four to seven cycles.
+// Sort of the frame of 110M pairs 3160 -> 2690 us, 8K / 14.5M pairs 446 -> 416, 4K / 8M 216 -> 199, 1080p / 1.7M 98 -> 90,
+// 720p / 0.2M 38 -> 31.  (Blocks of 2048 pairs lose 2 % on 4K and 8K, of 3072 and 5120 no difference to 4096, of
+// 6144 to 8192 5 to 20 %: one workgroup per CU.)
+template <int kBitsT, int kItemsT, int kThreadsT>
 struct PassShape {
     static constexpr int kBits = kBitsT;
     static constexpr int kBinsP = 1 << kBitsT;
-    static constexpr int kItems = kItemsT;                  // pairs per thread in count/scatter
-    static constexpr int kTile = kSortBlock * kItemsT;      // pairs per count/scatter workgroup
-    static constexpr int kPerThread = kBinsP / kSortBlock;  // digits per thread where a thread stands for digits
-    static_assert(kBinsP % kSortBlock == 0 && kTile <= 65535, "16-bit counts per wave and digit");
+    static constexpr int kItems = kItemsT;                  // pairs per thread in scatter
+    static constexpr int kThreads = kThreadsT;              // of a scatter workgroup
+    static constexpr int kWaves = kThreadsT / kWave;
+    static constexpr int kTile = kThreadsT * kItemsT;       // pairs per count/scatter workgroup
+    static constexpr int kCountItems = kTile / kSortBlock;  // pairs per thread in count
+    static constexpr int kPerThread = kBinsP / kSortBlock;  // digits per thread of a count row
+    static constexpr int kDigits = kThreadsT < kBinsP ? kBinsP / kThreadsT : 1;     // digits per scatter thread that stands for digits
+    static constexpr int kGroups = kThreadsT < kBinsP ? 1 : kThreadsT / kBinsP;     // scatter threads per digit
+    static_assert(kBinsP % kSortBlock == 0 && kTile % kSortBlock == 0 && kTile <= 65535, "16-bit counts per wave and digit");
+    static_assert(kThreadsT < kBinsP ? kBinsP % kThreadsT == 0 : kThreadsT % kBinsP == 0, "whole digits per thread, or whole groups of threads");
 };
-using Narrow = PassShape<8, 16>;
-using Wide = PassShape<9, 15>;
+using Narrow = PassShape<8, 4, 1024>;
+using Wide = PassShape<9, 4, 1024>;
 constexpr int kNarrowMaxTileBits = 16;
-// A short list (the 0.2M pairs of a 720p frame are 49 blocks of 4096) leaves most CUs without a
-// block and every block ranking 16 rounds: there four pairs per thread, four times the blocks.
-using Short = PassShape<8, 4>;
+// The 0.2M pairs of a 720p frame are 49 blocks of 4096, which would leave four CUs in five without one: shorter lists
+// are cut into smaller blocks (0.2M pairs 36.7 us with 2048 a block, 30.6 with 1024; 0.4M 54.5 with 1024,
+// 50 with 1536, 44 with 2048; 1.2M 83 with 4096, 79 with 2048; 1.7M 92.5 and 90; 0.1M on an 8K frame 78 and, with 1024, 64).
+using Middle = PassShape<8, 2, 1024>;
+using Short = PassShape<8, 1, 1024>;
+using WideShort = PassShape<9, 1, 1024>;
+constexpr int kShortPairs = 1 << 18;
+constexpr int kMiddlePairs = 1 << 21;
 
-
-// A list of at most kSmallRows blocks needs no launch that turns the histogram rows into starts:
-// the scatter workgroups add the rows up themselves.
-constexpr int kSmallRows = 64;
-constexpr int kShortPairs = kSmallRows * Narrow::kTile;     // up to this many pairs: blocks of Short::kTile, still without that launch
+// A list with at most this many histogram entries (256 blocks, or 128 with 9-bit digits) needs no launch that turns
+// the histogram rows into starts: the scatter workgroups add the rows up themselves (0.4M pairs, 193 rows: 44 us against 50
+// with that launch; 0.6M, 295 rows: 78 and 72).
+constexpr int kMostRowWords = 65536;
+constexpr int kMaxChunks = 256;
 
 inline size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 
@@ -89,7 +106,7 @@ PassGrid pass_grid(int n, int tile)
 {
     PassGrid g;
     g.tiles = (n + tile - 1) / tile;
-    g.chunk = g.tiles > 256 ? (g.tiles + 255) / 256 : 1;     // at most 256 chunks, one count workgroup each: about one per CU
+    g.chunk = (g.tiles + kMaxChunks - 1) / kMaxChunks;       // one count workgroup each: about one per CU
     g.chunks = (g.tiles + g.chunk - 1) / g.chunk;
     return g;
 }
@@ -98,13 +115,14 @@ PassGrid pass_grid(int n, int tile)
 Workspace workspace_for(int n)
 {
     Workspace w;
-    const PassGrid a = pass_grid(n, Narrow::kTile), b = pass_grid(n, Wide::kTile);
-    size_t hist = (size_t)a.tiles * Narrow::kBinsP > (size_t)b.tiles * Wide::kBinsP ? (size_t)a.tiles * Narrow::kBinsP
-                                                                                     : (size_t)b.tiles * Wide::kBinsP;
-    if (n <= kShortPairs && (size_t)pass_grid(n, Short::kTile).tiles * Short::kBinsP > hist)
-        hist = (size_t)pass_grid(n, Short::kTile).tiles * Short::kBinsP;
-    const size_t sums = (size_t)a.chunks * Narrow::kBinsP > (size_t)b.chunks * Wide::kBinsP ? (size_t)a.chunks * Narrow::kBinsP
-                                                                                             : (size_t)b.chunks * Wide::kBinsP;
+    // (monotone in n: a workspace sized for more pairs serves fewer)
+    auto rows_of = [](auto shape, int pairs) {
+        using Shape = decltype(shape);
+        return (size_t)pass_grid(pairs, Shape::kTile).tiles * Shape::kBinsP;
+    };
+    const size_t hist = std::max({rows_of(Short(), std::min(n, kShortPairs)), rows_of(Middle(), std::min(n, kMiddlePairs)),
+                                  rows_of(WideShort(), std::min(n, kShortPairs)), rows_of(Narrow(), n), rows_of(Wide(), n)});
+    const size_t sums = (size_t)std::min(n, kMaxChunks) * Wide::kBinsP;
     w.alt_keys = 0;
     w.alt_values = align_up((size_t)n * 8, 256);
     w.hist = w.alt_values + align_up((size_t)n * 4, 256);
@@ -146,7 +164,7 @@ __global__ __launch_bounds__(kSortBlock) void count_kernel(const uint64_t* __res
     const uint32_t mask = (1u << nbits) - 1u;
     const int base = blockIdx.x * Shape::kTile;
 #pragma unroll
-    for (int i = 0; i < Shape::kItems; i++) {
+    for (int i = 0; i < Shape::kCountItems; i++) {
         const int idx = base + i * kSortBlock + tid;
         if (idx < n) atomicAdd(&h[digit_of(keys[idx], shift, mask)], 1u);
     }
@@ -156,7 +174,7 @@ __global__ __launch_bounds__(kSortBlock) void count_kernel(const uint64_t* __res
         hist[(size_t)blockIdx.x * kB + q * kSortBlock + tid] = h[q * kSortBlock + tid];
 }
 
-// The same for a list of more than kSmallRows blocks: one workgroup counts a whole chunk of
+// The same for a list of more than kMostRowWords histogram entries: one workgroup counts a whole chunk of
 // `chunk` consecutive blocks, blockDim.x / kSortBlock of them at a time, and so also has the
 // chunk's digit sums, which the offsets launch needs (a launch of their own would read the rows
 // back just to add them up).
@@ -187,14 +205,14 @@ __global__ __launch_bounds__(kCountGroups * kSortBlock) void count_chunk_kernel(
         const int row = first + group;
         if (row < t1) {
             const int base = row * Shape::kTile;
-            uint64_t k[Shape::kItems];
+            uint64_t k[Shape::kCountItems];
 #pragma unroll
-            for (int i = 0; i < Shape::kItems; i++) {
+            for (int i = 0; i < Shape::kCountItems; i++) {
                 const int idx = base + i * kSortBlock + tid;
                 k[i] = idx < n ? keys[idx] : 0ull;
             }
 #pragma unroll
-            for (int i = 0; i < Shape::kItems; i++)
+            for (int i = 0; i < Shape::kCountItems; i++)
                 if (base + i * kSortBlock + tid < n) atomicAdd(&h[group][digit_of(k[i], shift, mask)], 1u);
         }
         __syncthreads();
@@ -294,7 +312,7 @@ __global__ __launch_bounds__(kOffsetThreads) void offsets_kernel(uint32_t* __res
 // which is where the next workgroup's run of d begins.  Every entry has one writer, empty ids
 // included, and no launch has to read the keys again.
 template <class Shape, bool kTable>
-__global__ __launch_bounds__(kSortBlock) void scatter_kernel(
+__global__ __launch_bounds__(Shape::kThreads) void scatter_kernel(
     const uint64_t* __restrict__ keys_in, const uint32_t* __restrict__ values_in,
     uint64_t* __restrict__ keys_out, uint32_t* __restrict__ values_out,
     int n, int shift, int nbits,
@@ -302,13 +320,15 @@ __global__ __launch_bounds__(kSortBlock) void scatter_kernel(
     int raw_rows,                                // ... if > 0, the raw_rows histogram rows themselves (a short list)
     int* __restrict__ seg_start)                 // kTable: [2^(shift - 32 + nbits) + 1]
 {
-    constexpr int kB = Shape::kBinsP, kItems = Shape::kItems, kTile = Shape::kTile, kPer = Shape::kPerThread;
+    constexpr int kB = Shape::kBinsP, kItems = Shape::kItems, kTile = Shape::kTile, kPer = Shape::kDigits;
+    constexpr int kThreads = Shape::kThreads, kWaves = Shape::kWaves;
     // per-wave digit counts, then per-wave digit offsets: at most kTile, so 16 bits do, and with
-    // them the workgroup's LDS stays under a third of the CU's (three resident workgroups, not two)
-    __shared__ uint16_t s_count[kSortWaves][kB];
+    // them the workgroup's LDS stays under half of the CU's
+    __shared__ __align__(4) uint16_t s_count[kWaves][kB];
     __shared__ uint16_t s_bin_start[kB];              // where each digit starts in the ranked block
     __shared__ uint32_t s_global[kB];                 // destination of ranked slot p with digit d: s_global[d] + p
-    __shared__ uint32_t s_wave_sum[kPer * kSortWaves];
+    constexpr int kScanWaves = kB / kWave;           // waves' worth of digits
+    __shared__ uint32_t s_wave_sum[kScanWaves];
     __shared__ uint64_t s_keys[kTile];
     __shared__ uint32_t s_values[kTile];
 
@@ -349,42 +369,70 @@ __global__ __launch_bounds__(kSortBlock) void scatter_kernel(
         const int off = wave * (kWave * kItems) + i * kWave + lane;
         val[i] = off < in_tile ? values_in[tile_base + off] : 0u;
     }
-    uint32_t my_start[kPer];
+    // A thread stands for the digits tid, tid + kThreads, ...; with more threads than digits the first kB do.
+    const bool has_digits = tid < kB;
+    uint32_t my_start[kPer] = {};
     if (raw_rows == 0) {
+        if (has_digits) {
 #pragma unroll
-        for (int q = 0; q < kPer; q++) my_start[q] = start[(size_t)tile * kB + q * kSortBlock + tid];
+            for (int q = 0; q < kPer; q++) my_start[q] = start[(size_t)tile * kB + q * kThreads + tid];
+        }
     } else {
-        // A list of at most kSmallRows blocks: every workgroup adds up the histogram rows itself
+        // A list of at most kMostRowWords histogram entries: every workgroup adds up the histogram rows itself
         // (the digit totals, and what the blocks in front of it hold of each digit), which
         // saves the launch that would do it.
         uint32_t total[kPer], before[kPer], incl[kPer];
+        const int group = tid / kB;
 #pragma unroll
         for (int q = 0; q < kPer; q++) {
-            const int d = q * kSortBlock + tid;
+            const int d = (q * kThreads + tid) % kB;
             total[q] = 0; before[q] = 0;
 #pragma unroll 16
-            for (int b = 0; b < raw_rows; b++) {
+            for (int b = group; b < raw_rows; b += Shape::kGroups) {
                 const uint32_t c = start[(size_t)b * kB + d];
                 total[q] += c;
                 before[q] += b < tile ? c : 0u;
             }
-            incl[q] = wave_inclusive_sum(total[q]);
-            if (lane == kWave - 1) s_wave_sum[q * kSortWaves + wave] = incl[q];
+        }
+        if constexpr (Shape::kGroups > 1) {
+            uint32_t* const s_part = (uint32_t*)s_keys;
+            static_assert(sizeof(uint32_t) * 2 * Shape::kGroups * kB <= sizeof(uint64_t) * kTile, "the partial sums fit in the space of the keys");
+            s_part[2 * tid] = total[0];
+            s_part[2 * tid + 1] = before[0];
+            __syncthreads();
+            if (has_digits) {
+#pragma unroll
+                for (int g = 1; g < Shape::kGroups; g++) {
+                    total[0] += s_part[2 * (g * kB + tid)];
+                    before[0] += s_part[2 * (g * kB + tid) + 1];
+                }
+            }
+        }
+        if (has_digits) {
+#pragma unroll
+            for (int q = 0; q < kPer; q++) {
+                incl[q] = wave_inclusive_sum(total[q]);
+                if (lane == kWave - 1) s_wave_sum[q * kWaves + wave] = incl[q];
+            }
         }
         __syncthreads();
+        if (has_digits) {
 #pragma unroll
-        for (int q = 0; q < kPer; q++) {
-            uint32_t digit_base = incl[q] - total[q];
+            for (int q = 0; q < kPer; q++) {
+                uint32_t digit_base = incl[q] - total[q];
 #pragma unroll
-            for (int w = 0; w < kPer * kSortWaves; w++)
-                if (w < q * kSortWaves + wave) digit_base += s_wave_sum[w];
-            my_start[q] = digit_base + before[q];
+                for (int w = 0; w < kScanWaves; w++)
+                    if (w < q * kWaves + wave) digit_base += s_wave_sum[w];
+                my_start[q] = digit_base + before[q];
+            }
         }
     }
+    {
+        uint32_t* const words = (uint32_t*)&s_count[0][0];
 #pragma unroll
-    for (int w = 0; w < kSortWaves; w++)
-#pragma unroll
-        for (int q = 0; q < kPer; q++) s_count[w][q * kSortBlock + tid] = 0;
+        for (int w = 0; w < kWaves * kB / 2; w += kThreads)
+            if (w + tid < kWaves * kB / 2) words[w + tid] = 0;
+    }
     if (kTable && tid < 2) {
         const int low = (int)((uint32_t)(edge_key >> 32) & low_mask);
         s_own[tid] = tid == 0 ? (tile > 0 ? low + 1 : 0) : (tile == (int)gridDim.x - 1 ? (int)low_mask : low);
@@ -419,31 +467,34 @@ __global__ __launch_bounds__(kSortBlock) void scatter_kernel(
 
     // digit totals of the block; per-wave offsets inside each digit.  A thread stands for the
     // digits tid, tid + 256, ...; the scan runs over the digits in their order.
-    uint32_t total[kPer], incl[kPer];
+    uint32_t total[kPer] = {}, incl[kPer] = {};
+    if (has_digits) {
 #pragma unroll
-    for (int q = 0; q < kPer; q++) {
-        const int d = q * kSortBlock + tid;
-        total[q] = 0;
+        for (int q = 0; q < kPer; q++) {
+            const int d = q * kThreads + tid;
 #pragma unroll
-        for (int w = 0; w < kSortWaves; w++) {
-            const uint32_t c = s_count[w][d];
-            s_count[w][d] = (uint16_t)total[q];
-            total[q] += c;
+            for (int w = 0; w < kWaves; w++) {
+                const uint32_t c = s_count[w][d];
+                s_count[w][d] = (uint16_t)total[q];
+                total[q] += c;
+            }
+            incl[q] = wave_inclusive_sum(total[q]);
+            if (lane == kWave - 1) s_wave_sum[q * kWaves + wave] = incl[q];
         }
-        incl[q] = wave_inclusive_sum(total[q]);
-        if (lane == kWave - 1) s_wave_sum[q * kSortWaves + wave] = incl[q];
     }
     __syncthreads();
+    if (has_digits) {
 #pragma unroll
-    for (int q = 0; q < kPer; q++) {
-        const int d = q * kSortBlock + tid;
-        uint32_t before_wave = 0;
+        for (int q = 0; q < kPer; q++) {
+            const int d = q * kThreads + tid;
+            uint32_t before_wave = 0;
 #pragma unroll
-        for (int w = 0; w < kPer * kSortWaves; w++)
-            if (w < q * kSortWaves + wave) before_wave += s_wave_sum[w];
-        const uint32_t bin_start = before_wave + incl[q] - total[q];
-        s_bin_start[d] = (uint16_t)bin_start;
-        s_global[d] = my_start[q] - bin_start;
+            for (int w = 0; w < kScanWaves; w++)
+                if (w < q * kWaves + wave) before_wave += s_wave_sum[w];
+            const uint32_t bin_start = before_wave + incl[q] - total[q];
+            s_bin_start[d] = (uint16_t)bin_start;
+            s_global[d] = my_start[q] - bin_start;
+        }
     }
     __syncthreads();
 
@@ -469,16 +520,16 @@ __global__ __launch_bounds__(kSortBlock) void scatter_kernel(
         uint32_t out_value[kItems], out_at[kItems];
 #pragma unroll
         for (int i = 0; i < kItems; i++) {
-            const int p = min(i * kSortBlock + tid, in_tile - 1);
+            const int p = min(i * kThreads + tid, in_tile - 1);
             out_key[i] = s_keys[p];
             out_value[i] = s_values[p];
         }
 #pragma unroll
         for (int i = 0; i < kItems; i++)
-            out_at[i] = s_global[digit_of(out_key[i], shift, mask)] + (uint32_t)(i * kSortBlock + tid);
+            out_at[i] = s_global[digit_of(out_key[i], shift, mask)] + (uint32_t)(i * kThreads + tid);
 #pragma unroll
         for (int i = 0; i < kItems; i++) {
-            if (i * kSortBlock + tid < in_tile) {
+            if (i * kThreads + tid < in_tile) {
                 keys_out[out_at[i]] = out_key[i];
                 values_out[out_at[i]] = out_value[i];
             }
@@ -490,7 +541,7 @@ __global__ __launch_bounds__(kSortBlock) void scatter_kernel(
             // (a loop of its own: in the one above the LDS reads of all slots are in flight together)
 #pragma unroll 4
             for (int i = 0; i < kItems; i++) {
-                const int p = i * kSortBlock + tid;
+                const int p = i * kThreads + tid;
                 if (p >= in_tile) break;
                 const uint32_t field = (uint32_t)(s_keys[p] >> 32);
                 const uint32_t d = (field >> low_bits) & mask;
@@ -503,8 +554,8 @@ __global__ __launch_bounds__(kSortBlock) void scatter_kernel(
             // owned low parts above the last pair of a digit's run: the end of the run
 #pragma unroll
             for (int q = 0; q < kPer; q++) {
-                const uint32_t d = (uint32_t)(q * kSortBlock + tid);
-                if (d > mask) continue;
+                const uint32_t d = (uint32_t)(q * kThreads + tid);
+                if (d > mask) continue;         // (d is below kB then, a digit of this thread)
                 int last = own_lo - 1;
                 if (total[q]) last = (int)((uint32_t)(s_keys[(uint32_t)s_bin_start[d] + total[q] - 1u] >> 32) & low_mask);
                 const int end = (int)(my_start[q] + total[q]);
@@ -1419,7 +1470,7 @@ extern "C" int fgs_sort_gaussian(int num_rendered,
     auto partition = [&](auto shape) {
         using Shape = decltype(shape);
         const PassGrid g = pass_grid(n, Shape::kTile);
-        const bool small = n <= kShortPairs;         // the scatter workgroups add up the histogram rows themselves
+        const bool small = g.tiles * Shape::kBinsP <= kMostRowWords;     // the scatter workgroups add up the histogram rows themselves
         const int passes = (tile_bits + Shape::kBits - 1) / Shape::kBits;
         table_by_scatter = seg_start && passes <= 2;
         const uint64_t* src_k = gaussian_keys_unsorted;
@@ -1443,10 +1494,10 @@ extern "C" int fgs_sort_gaussian(int num_rendered,
                                    hist, g.tiles, g.chunk, chunk_sums, g.chunks);
             }
             if (last && table_by_scatter)
-                hipLaunchKernelGGL((scatter_kernel<Shape, true>), dim3(g.tiles), dim3(kSortBlock), 0, st,
+                hipLaunchKernelGGL((scatter_kernel<Shape, true>), dim3(g.tiles), dim3(Shape::kThreads), 0, st,
                                    src_k, src_v, dst_k, dst_v, n, shift, nbits, hist, small ? g.tiles : 0, seg_start);
             else
-                hipLaunchKernelGGL((scatter_kernel<Shape, false>), dim3(g.tiles), dim3(kSortBlock), 0, st,
+                hipLaunchKernelGGL((scatter_kernel<Shape, false>), dim3(g.tiles), dim3(Shape::kThreads), 0, st,
                                    src_k, src_v, dst_k, dst_v, n, shift, nbits, hist, small ? g.tiles : 0, (int*)nullptr);
             src_k = dst_k;
             src_v = dst_v;
@@ -1454,7 +1505,10 @@ extern "C" int fgs_sort_gaussian(int num_rendered,
     };
     if (tile_bits <= kNarrowMaxTileBits) {
         if (n <= kShortPairs) partition(Short());
+        else if (n <= kMiddlePairs) partition(Middle());
         else partition(Narrow());
+    } else if (n <= kShortPairs) {
+        partition(WideShort());
     } else {
         partition(Wide());
     }

@@ -34,6 +34,9 @@ def test_sort_buffer_size_is_monotonic_and_bounded():
     assert all(a <= b for a, b in zip(sizes, sizes[1:]))
     assert sizes[-1] >= 12 * 2 ** 27                     # room for the second key/value buffer
     assert sizes[-1] < 2.5 * 12 * 2 ** 27
+    edges = sorted(max(1, (1 << b) + d) for b in (8, 10, 11, 12, 17, 18, 19, 20, 21, 24) for d in (-1, 0, 1))
+    sizes = [cabi.get_sort_buffer_size(n) for n in edges]      # a space for more pairs serves fewer, whatever their blocks
+    assert all(a <= b for a, b in zip(sizes, sizes[1:]))
     assert cabi.get_sort_buffer_size(-1) == 0
     assert cabi.get_sort_buffer_size(cabi.FGS_MAX_RENDERED) > 0
 

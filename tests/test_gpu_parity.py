@@ -1195,6 +1195,23 @@ def test_sort_around_the_list_lengths_where_the_launches_change(n, W, H):
     _sort_case(tile, depth, W, H, seed=n % 97, ascending=True)
 
 
+@pytest.mark.parametrize("n,W,H", [(1023, 640, 480), (1024, 640, 480), (1025, 640, 480), (200_001, 640, 480), (400_003, 1920, 1080),
+                                   ((1 << 21) - 1, 1920, 1080), (1 << 21, 1920, 1080), ((1 << 21) + 1, 1920, 1080),
+                                   (777, 7680, 4320), (131_072, 7680, 4320), (131_073, 7680, 4320), (262_145, 7680, 4320),
+                                   (524_289, 7680, 4320)])
+def test_sort_around_the_list_lengths_where_the_partition_blocks_change(n, W, H):
+    """Blocks of 1024, 2048 or 4096 pairs (8-bit digits) and of 1024 or 4096 (9-bit), histogram rows added up by the scatter
+    workgroups or by a launch of their own: one block and its neighbours, ragged last blocks, the lengths around
+    each change, crowded tiles, all pairs of the first blocks in one tile."""
+    rng = np.random.default_rng(n % 1009 + W)
+    tiles = ((W + 15) // 16) * ((H + 15) // 16)
+    tile = (tiles * rng.random(n) ** 3).astype(np.uint32)
+    tile[:min(n // 3, 5000)] = tiles - 1
+    depth = rng.integers(0, 1 << 32, n, dtype=np.uint64).astype(np.uint32)
+    depth[::5] = depth[n // 2]
+    _sort_case(tile, depth, W, H, seed=n % 89, ascending=n % 2 == 0)
+
+
 def test_sort_bits_above_the_range_stay_with_their_pair():
     """Bits above 32 + bit_length(tiles) are outside the sorted range (sort.cu:34-39) but travel
     with the key; segments whose keys differ there take the general path."""
