@@ -14,6 +14,7 @@
 // (fgs_set_colour_sums).
 #include "fgs_internal.h"
 
+#include <algorithm>
 #include <atomic>
 #include <map>
 #include <mutex>
@@ -34,12 +35,14 @@ __global__ __launch_bounds__(256) void fill_i32_kernel(int* p, size_t n, int v)
 }
 
 
-// Tiles of a small frame ranked by the length of their lists, longest first (in steps of 16;
-// the order inside a step is whatever the atomics make it).  One workgroup.
+// Tiles of a small frame ranked by the length of their lists, longest first (in steps of kOrderStep;
+// the order inside a step is whatever the atomics make it), and behind the ranking how many of them are shared out and from
+// which length on.  One workgroup.
 // (Ranking in the last workgroup of tile_ranges_kernel instead costs more than this launch: every
 // workgroup then has to push its ranges out of its XCD's L2 before it counts itself done.)
 constexpr int kOrderCap = 8192;            // tiles
-constexpr int kOrderBins = 128;            // everything from 2032 entries up shares the first bin
+constexpr int kOrderBins = 256, kOrderStep = 32;       // bins of so many entries; everything from 8160 up shares the first one
+constexpr int kLeastShared = 128;          // entries of a list that is shared out (see blend_kernel_shared)
 // The ranking is written by one launch and read by the next, so it needs memory of its own: one
 // table per (device, stream), allocated on the first such blend on that stream (blends on
 // different streams may overlap and get a table each).  Blends on one stream follow each other, and
@@ -73,7 +76,7 @@ int tile_order_table(hipStream_t stream, uint32_t** out, std::unique_lock<std::m
         entry = &g_order_tables[stream_key(device, stream)];
     }
     *enqueue = std::unique_lock<std::mutex>(entry->enqueue);
-    if (!entry->ranks && hipMalloc((void**)&entry->ranks, kOrderCap * sizeof(uint32_t)) != hipSuccess) {
+    if (!entry->ranks && hipMalloc((void**)&entry->ranks, (kOrderCap + 2) * sizeof(uint32_t)) != hipSuccess) {
         (void)hipGetLastError();
         entry->ranks = nullptr;
     }
@@ -81,8 +84,26 @@ int tile_order_table(hipStream_t stream, uint32_t** out, std::unique_lock<std::m
     return FGS_OK;
 }
 
+// From which length on a tile's list is shared out (see blend_kernel_shared): three eighths of what a SIMD walks of the
+// whole frame, by the lists of 256 tiles spread over it, and at least kLeastShared; a multiple of kOrderStep.  Lists are cut alike whether
+// the tiles are ranked or not, so the image is the same.  Called by a whole wave.
+__device__ __forceinline__ int least_shared(const int2* __restrict__ ranges, int num_tiles, int squares, int simds)
+{
+    constexpr int kSamples = 256;
+    uint32_t sum = 0;
+#pragma unroll
+    for (int k = 0; k < kSamples / kWave; k++) {
+        const int2 r = ranges[(long long)(k * kWave + lane_id()) * num_tiles / kSamples];
+        sum += (uint32_t)max(0, r.y - r.x);
+    }
+    sum = (uint32_t)bcast_i((int)wave_inclusive_sum(sum), kWave - 1);
+    const uint64_t each = (uint64_t)sum * (uint32_t)num_tiles / kSamples * (uint32_t)squares / (uint32_t)simds;
+    const uint64_t least = each / 8 * 3 / kOrderStep * kOrderStep;
+    return least < kLeastShared ? kLeastShared : least > 0x40000000u ? 0x40000000 : (int)least;
+}
+
 __global__ __launch_bounds__(1024) void tile_order_kernel(const int2* __restrict__ ranges, int num_tiles,
-                                                          uint32_t* __restrict__ tile_order)
+                                                          uint32_t* __restrict__ tile_order, int squares, int simds)
 {
     constexpr int kPerThread = kOrderCap / 1024;
     __shared__ uint32_t s_count[kOrderBins];
@@ -96,29 +117,40 @@ __global__ __launch_bounds__(1024) void tile_order_kernel(const int2* __restrict
         bin[k] = 0; slot[k] = 0;
         if (t < num_tiles) {
             const int2 r = ranges[t];
-            bin[k] = (uint32_t)(kOrderBins - 1 - max(0, min((r.y - r.x) >> 4, kOrderBins - 1)));
+            bin[k] = (uint32_t)(kOrderBins - 1 - max(0, min((r.y - r.x) / kOrderStep, kOrderBins - 1)));
             slot[k] = atomicAdd(&s_count[bin[k]], 1u);
         }
     }
     __syncthreads();
     if (tid < kWave) {
-        // exclusive prefix over the bins, two per lane
-        const uint32_t a = s_count[2 * tid], b = s_count[2 * tid + 1];
-        uint32_t incl = a + b;
+        // exclusive prefix over the bins, four per lane
+        static_assert(kOrderBins == 4 * kWave, "four bins per lane");
+        const uint32_t a = s_count[4 * tid], b = s_count[4 * tid + 1], c = s_count[4 * tid + 2], d = s_count[4 * tid + 3];
+        const uint32_t all = a + b + c + d;
+        uint32_t incl = all;
 #pragma unroll
         for (int o = 1; o < kWave; o <<= 1) {
             const uint32_t up = (uint32_t)__shfl_up((int)incl, o);
             if (tid >= o) incl += up;
         }
-        const uint32_t excl = incl - (a + b);
-        s_count[2 * tid] = excl;
-        s_count[2 * tid + 1] = excl + a;
+        const uint32_t excl = incl - all;
+        s_count[4 * tid] = excl;
+        s_count[4 * tid + 1] = excl + a;
+        s_count[4 * tid + 2] = excl + a + b;
+        s_count[4 * tid + 3] = excl + a + b + c;
     }
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < kPerThread; k++) {
         const int t = tid + k * 1024;
         if (t < num_tiles) tile_order[s_count[bin[k]] + slot[k]] = (uint32_t)t;
+    }
+    if (tid < kWave) {
+        const int least = least_shared(ranges, num_tiles, squares, simds);
+        if (tid == 0) {
+            tile_order[kOrderCap] = least / kOrderStep < kOrderBins ? s_count[kOrderBins - least / kOrderStep] : 0u;
+            tile_order[kOrderCap + 1] = (uint32_t)least;
+        }
     }
 }
 
@@ -242,6 +274,8 @@ constexpr float kMostExponent = 20.0f;      // of a Gaussian that the matrix pro
 // 1e-3 at most (as from tables over the tile).
 constexpr float kSharpest = 64.0f;
 constexpr int kNeverStop = -2147483647 - 1;
+// Exponents up to this one count as none above zero: T that has turned negative stays below kStopBelow (2^0.01 - 1 of 1, at most).
+constexpr float kSlightlyAbove = 0.01f;
 
 // An fp32 number as the sum of three bf16 numbers: eight bits of the significand each.
 // (Each is the upper half of a float; the bits below are left to high_halves to drop.)
@@ -469,7 +503,7 @@ struct Ahead {
 
 // walk_list below from its entry base on, in chunks of 64: to the first chunk that the recurrence does not take, or
 // (kSteep) to the end.  Returns as walk_list does, or base of the chunk it ended in front of.
-template <bool kFp32, bool kSteep>
+template <bool kFp32, bool kSteep, bool kRun>
 __device__ __forceinline__ int walk_chunks(
     const LaneRole& role, float* stage,
     const uint32_t* __restrict__ point_list, int begin, int n,
@@ -477,7 +511,7 @@ __device__ __forceinline__ int walk_chunks(
     const float2* __restrict__ points_xy,
     const float4* __restrict__ rgb_depth,
     const float4* __restrict__ conic_opacity,
-    float (&T)[4], Sums<kFp32>& sums, int stop_below, Ahead& next, int base)
+    float (&T)[4], Sums<kFp32>& sums, int stop_below, Ahead& next, int base, bool& above)
 {
     const int lane = role.lane;
     char* const bytes = reinterpret_cast<char*>(stage);
@@ -504,6 +538,12 @@ __device__ __forceinline__ int walk_chunks(
         const float beyond = __builtin_fmaf(__builtin_fmaf(co.y, co.y, -4.0f * co.x * co.z) * reach, reach, 4.0f * co.z * (kMostExponent - co.w));
         const bool fits = __builtin_fmaxf(__builtin_fmaxf(beyond, co.z), __builtin_fmaxf(-limit - co.z, co.w - kMostExponent)) <= 0.0f &&
                           __builtin_fabsf(c) + __builtin_fabsf(bx) + __builtin_fabsf(by) + __builtin_fabsf(co.x) < 1.0e9f;
+        if constexpr (kRun) {
+            // any exponent above kSlightlyAbove
+            const float w = kFp32 ? co.w : co.w - kWeightScaleLog2;
+            const float over = __builtin_fmaf(__builtin_fmaf(co.y, co.y, -4.0f * co.x * co.z) * reach, reach, 4.0f * co.z * (kSlightlyAbove - w));
+            above = above || ballot(!(__builtin_fmaxf(over, w - kSlightlyAbove) <= 0.0f)) != 0;
+        }
         if (ballot(!fits) != 0) {
             if constexpr (!kSteep) return base;
             const int walked = walk_plain<kFp32>(xy, co, rgb, cnt, left, top, stop_below, T, sums);
@@ -678,7 +718,7 @@ __device__ __forceinline__ int walk_chunks(
 // of the tile's list, so that the pairs are the reference's pairs.  The walk ends after the pair behind
 // which all 256 pixels have T < stop_below (render.cu:394-408).  Returns the entries walked, or ~entries
 // when that stop ended the walk.  stage: this wave's kStageFloats of LDS.
-template <bool kFp32>
+template <bool kFp32, bool kRun>
 __device__ __forceinline__ int walk_list(
     const LaneRole& role, float* stage,
     const uint32_t* __restrict__ point_list, int begin, int n,
@@ -686,7 +726,7 @@ __device__ __forceinline__ int walk_list(
     const float2* __restrict__ points_xy,
     const float4* __restrict__ rgb_depth,
     const float4* __restrict__ conic_opacity,
-    float (&T)[4], Sums<kFp32>& sums, int stop_below = kStopBelow)
+    float (&T)[4], Sums<kFp32>& sums, int stop_below, bool& above)
 {
     const int lane = role.lane;
     Ahead next = {};
@@ -696,11 +736,11 @@ __device__ __forceinline__ int walk_list(
         next.index = point_list[min((uint32_t)begin + kChunk + (uint32_t)lane, last)];
         next.xy = points_xy[g]; next.co = conic_opacity[g]; next.rgb = rgb_depth[g];
     }
-    const int walked = walk_chunks<kFp32, false>(role, stage, point_list, begin, n, left, top, points_xy, rgb_depth, conic_opacity,
-                                                 T, sums, stop_below, next, 0);
+    const int walked = walk_chunks<kFp32, false, kRun>(role, stage, point_list, begin, n, left, top, points_xy, rgb_depth, conic_opacity,
+                                                 T, sums, stop_below, next, 0, above);
     if (walked < 0 || walked >= n) return walked;
-    return walk_chunks<kFp32, true>(role, stage, point_list, begin, n, left, top, points_xy, rgb_depth, conic_opacity,
-                                    T, sums, stop_below, next, walked);
+    return walk_chunks<kFp32, true, kRun>(role, stage, point_list, begin, n, left, top, points_xy, rgb_depth, conic_opacity,
+                                    T, sums, stop_below, next, walked, above);
 }
 
 // The wave's pixels out of T and the colour sums.
@@ -801,7 +841,7 @@ constexpr int kBlendWaves = kFp32 ? 5 : 4;       // resident waves per SIMD
 // Resident waves: 5 per SIMD is what 96 registers allow (4: the same time on the largest frames, 3 to 5 %
 // more on the others; 6 spills).
 template <int SX, int SY, bool kFp32>
-__global__ __launch_bounds__(kWave * SX * SY) __attribute__((amdgpu_waves_per_eu(kBlendWaves<kFp32>, kBlendWaves<kFp32>))) void blend_kernel(FGS_BLEND_PARAMS, const uint32_t* __restrict__ tile_order)
+__global__ __launch_bounds__(kWave * SX * SY) __attribute__((amdgpu_waves_per_eu(kBlendWaves<kFp32>, kBlendWaves<kFp32>))) void blend_kernel(FGS_BLEND_PARAMS)
 {
     constexpr int kSquares = SX * SY;
     __shared__ __align__(16) float s_stage[kSquares][kStageFloats];
@@ -810,13 +850,7 @@ __global__ __launch_bounds__(kWave * SX * SY) __attribute__((amdgpu_waves_per_eu
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = kSquares == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     int tile_x, tile_y;
-    if (kSquares > 1 && tile_order) {
-        const int tile = (int)tile_order[blockIdx.x];
-        tile_x = tile % tiles_x;
-        tile_y = tile / tiles_x;
-    } else if (!tile_of_position((int)blockIdx.x, tiles_x, tiles_y, &tile_x, &tile_y)) {
-        return;
-    }
+    if (!tile_of_position((int)blockIdx.x, tiles_x, tiles_y, &tile_x, &tile_y)) return;
     const int2 range = ranges[tile_y * tiles_x + tile_x];
     const int n = range.y - range.x;
     // A launch ends when its longest list ends, and a wave that shares its SIMD equally with the
@@ -835,8 +869,9 @@ __global__ __launch_bounds__(kWave * SX * SY) __attribute__((amdgpu_waves_per_eu
     int done = 0, upto = n;
     int stop_below = kStopBelow;
     for (;;) {
-        const int walked = walk_list<kFp32>(role, s_stage[wave], point_list, range.x + done, upto - done, (float)left, (float)top,
-                                            points_xy, rgb_depth, conic_opacity, T, sums, stop_below);
+        bool above;
+        const int walked = walk_list<kFp32, false>(role, s_stage[wave], point_list, range.x + done, upto - done, (float)left, (float)top,
+                                                   points_xy, rgb_depth, conic_opacity, T, sums, stop_below, above);
         if (kSquares == 1) break;
         done += walked < 0 ? ~walked : walked;
         if (stop_below == kStopBelow) {
@@ -867,124 +902,305 @@ __global__ __launch_bounds__(kWave * SX * SY) __attribute__((amdgpu_waves_per_eu
     write_square(lane, left, top, width, height, px, bg_r, bg_g, bg_b, out_u8, out_f32);
 }
 
-// A frame of few tiles is placed on the chip almost at once, one wave per tile: the launch then
-// lasts as long as the busiest SIMD (the sum of the lists placed on it) and at least as long as
-// the longest list walked by one wave.  Here the tiles are ranked by list length
-// (tile_order_kernel) and a workgroup of four waves takes one tile from each quarter of the
-// ranking: the workgroups with the longest lists are dispatched first, the short ones fill in
-// behind them, and a long list has three shorter ones beside it.  Every wave blends the first
-// kOwnShare entries of its own tile; what is left of a list of more than kOwnShare + kMinRest
-// entries after that is cut into four runs of pairs, one per wave.  A run is blended from T = 1, C = 0 and the owner folds the runs in front-to-back order,
-// C += T C_run, T *= T_run, which is the same sum in another order of additions.  A run stops
-// when its own T is below the threshold everywhere, so a tile can be walked a little further than
-// the reference walks it: what that adds is below 1e-4 of a colour.
-constexpr int kOwnShare = 256;
-constexpr int kMinRest = 512;               // a shorter rest is not worth two barriers: the owner walks it
-constexpr int kSharedWaves = 4;
-// Where every workgroup is resident at once even with one tile each (a wave of it on each SIMD of a CU, so up to
-// kBlendWaves workgroups a CU), a tile has a workgroup to itself: three waves of it have no list of their own and
-// only take runs, so a long list has all four instead of a share of them, and the cut into runs stays the same.  256x192
-// pixels, 300k clustered Gaussians 357 -> 245 us, 640x512 100 -> 81, 1M 228 -> 169, with lists too short to be
-// shared 14.8 -> 14.8.  Beyond that (1920x1080, 1M) waves without a list keep others off the chip: 138 -> 159.
+// Frames of at most kOrderCap tiles.  Such a frame is about resident at once, and a wave alone on its SIMD issues one
+// instruction in seven cycles, 104 ns per entry, where five waves issue one in 1.5: the launch lasted as long as its
+// longest lists on single waves (32x16 tiles, 1599x901: 60 us of issue, 236 us for 2465 entries).  So the tiles are ranked by list
+// length, the longest start first, and those that are long for this frame (tile_order_kernel) have a workgroup of kT teams, one wave per
+// 16x16 square each, to themselves; all other tiles have a team each, without a word to the others of the workgroup
+// (one wave per square: a wave for a whole 32x32 tile needs 64 registers for its colour sums).
+//
+// A long list is walked in rounds.  Its first kHead entries are walked by the first team, since what stops there (opaque
+// content mostly does) shall cost the others nothing.  Then every team takes a run of the entries that follow, from T = 1, C = 0, and
+// the owner folds them front to back, C += T C_run, T *= T_run.  A round is kRoundRuns runs, whatever the number of teams, so a
+// list is cut alike in every frame; they are kHead entries long at first and twice as long with every round, so that what
+// is walked past a stop stays a fraction of the list.  The tile's stop is looked for behind
+// every run, from the products of T.  The run that has it is walked once more by the owner, on top of what was in front of it and with
+// the stop tested behind every pair, so the image ends where the reference's walk ends.  (Weights do not exceed
+// 1, so T only falls and a stop shows at the end of the run that has it; a run with an exponent above zero in it, which can
+// turn the sign of T, is walked that way too.)
+//
+// Against a wave per square that shared (16x16 tiles only) from 768 entries on among the four tiles of a workgroup: 32x16 at 1599x901
+// 237 -> 115 us, 32x32 at 2560x1440 1M 321 -> 277, at 640x512 1M 1873 -> 943; 16x16 1080p 1M 145 -> 126, 700k 104 -> 92, 1365x767 300k
+// 80 -> 58, 1280x720 with long lists everywhere 224 -> 86, with short ones 30 -> 31, 256x192 300k 227 -> 181, 4K 32x32 city 789 -> 788,
+// needles that make every tile opaque 45 -> 45 at 1080p and 33 -> 40 at 1024x700.  (What a round costs beside its walk is some
+// 2 us; 15 with the owner's state in volatile private memory, whose loads wait for each other.)  Shared from a quarter or a half of the average on
+// instead of three eighths: 1080p 141 and 132, 32x32 276 and 325; heads of 128 or 256 entries: 1080p 127 and 123, 1280x720 98
+// and 148 (64: 121 and 98, all with rounds of as many runs as teams); rounds of four runs: 32x16 108, 1280x720 98, 256x192 206.
+//
+// Unranked (no table: stream capture, no memory) every team has a tile and long lists are shared with the others of the workgroup, cut as
+// they are with a table.  What a team has blended of its own tile waits in private memory meanwhile.
+constexpr int kHead = 64, kMostRun = 512, kRoundRuns = 8;
+// resident waves per SIMD: whole workgroups
 template <bool kFp32>
-__global__ __launch_bounds__(kSharedWaves * kWave) __attribute__((amdgpu_waves_per_eu(kBlendWaves<kFp32>, kBlendWaves<kFp32>))) void blend_kernel_shared(FGS_BLEND_PARAMS, const uint32_t* __restrict__ tile_order, int tiles_per_group)
+constexpr int shared_waves(int of_workgroup) { return of_workgroup > 8 ? of_workgroup / 4 : kBlendWaves<kFp32>; }
+
+template <int SX, int SY, int kT, bool kFp32>
+__global__ __launch_bounds__(kWave * SX * SY * kT) __attribute__((amdgpu_waves_per_eu(shared_waves<kFp32>(SX * SY * kT), shared_waves<kFp32>(SX * SY * kT))))
+void blend_kernel_shared(FGS_BLEND_PARAMS, const uint32_t* __restrict__ tile_order, int tiles_per_group, int simds)
 {
+    constexpr int kSquares = SX * SY, kWaves = kSquares * kT;
     constexpr int kHandOver = 4 * 4 * kWave;            // a run's result: 4 pixels x 4 floats per lane
-    __shared__ __align__(16) float s_stage[kSharedWaves][kStageFloats > kHandOver ? kStageFloats : kHandOver];
-    __shared__ int s_rest[kSharedWaves], s_from[kSharedWaves], s_tile_x[kSharedWaves], s_tile_y[kSharedWaves];
+    __shared__ __align__(16) float s_stage[kWaves][kStageFloats > kHandOver ? kStageFloats : kHandOver];
+    __shared__ int s_walked[kWaves], s_stopped[kWaves], s_above[2][kT];
+    __shared__ int s_tile[kT][4];                       // of every team: first pixel, first pair, pairs
+    __shared__ int s_rest[kT];                          // pairs left for all teams
 
     const int lane = threadIdx.x & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-    // Wave w takes rank g of quarter w of the tiles ranked by list length (with tiles_per_group 1, wave 0 takes
-    // rank g and the others none): the workgroups with the longest lists come first in the launch, and a
-    // long list has three shorter ones beside it.
-    const int rank = wave * (int)gridDim.x + (int)blockIdx.x;
-    const bool active = wave < tiles_per_group && rank < tiles_x * tiles_y;
+    const int team = wave / kSquares, square = wave % kSquares;
+    static_assert(kLeastShared >= 2 * kHead, "a rest worth sharing behind the head");
+    const int num_tiles = tiles_x * tiles_y, group = (int)blockIdx.x;
+    // Ranked: the tiles with long lists have a workgroup each, tiles_per_group teams of the others have a tile.
+    int rank = team * (int)gridDim.x + group, least, teams = kT;
+    bool active = team < tiles_per_group;
+    if (tile_order) {
+        const int alone = (int)tile_order[kOrderCap];
+        const int first = group < alone ? group : alone + (group - alone) * tiles_per_group;
+        if (first >= num_tiles) return;
+        if (group >= alone && team >= tiles_per_group) return;
+        teams = group < alone ? kT : tiles_per_group;
+        rank = first + team;
+        active = group >= alone || team == 0;
+        least = (int)tile_order[kOrderCap + 1];
+    } else {
+        least = least_shared(ranges, num_tiles, kSquares, simds);
+    }
+    active = active && rank < num_tiles;
     int tile_x = 0, tile_y = 0;
+    int2 range = make_int2(0, 0);
     if (active) {
         const int tile = tile_order ? (int)tile_order[rank] : rank;
         tile_x = tile % tiles_x;
         tile_y = tile / tiles_x;
+        range = ranges[tile];
     }
-    int2 range = make_int2(0, 0);
-    if (active) range = ranges[tile_y * tiles_x + tile_x];
-    const int n = range.y - range.x;
+    int n = range.y - range.x, begin = range.x;         // of the tile that is walked
+    if (lane == 0 && square == 0) {
+        s_tile[team][0] = tile_x * SX * 16;
+        s_tile[team][1] = tile_y * SY * 16;
+        s_tile[team][2] = begin;
+        s_tile[team][3] = n;
+        s_above[0][team] = 0;
+        s_above[1][team] = 0;
+        s_rest[team] = 0;
+    }
     if (n > 256) __builtin_amdgcn_s_setprio(1);
-
     LaneRole role;
     role.init(lane, s_stage[wave]);
-    if (lane == 0) {
-        s_rest[wave] = n;               // job 0 of wave w: the head of its own list, in one run
-        s_from[wave] = range.x;
-        s_tile_x[wave] = tile_x;
-        s_tile_y[wave] = tile_y;
-    }
-    __builtin_amdgcn_wave_barrier();    // job 0 reads these back in the same wave; the others after the barrier below
-    // job 0: own head; job 1 + v: this wave's run of what is left of tile v.  While a wave blends
-    // runs, the result of its own head waits in its private memory, not in registers.
-    Pixels px;
-    volatile float kept[16];
-    bool shared_out = false;
-    for (int job = 0; job <= kSharedWaves; job++) {
-        const int v = job == 0 ? wave : job - 1;
-        const int rest = __builtin_amdgcn_readfirstlane(s_rest[v]);
-        if (job != 0 && rest == 0) continue;
-        int skip = 0, count = rest > kOwnShare + kMinRest ? kOwnShare : rest;
-        if (job != 0) {
-            const int run = (((rest + kSharedWaves - 1) / kSharedWaves) + 1) & ~1;      // whole pairs
-            skip = min(wave * run, rest);
-            count = min(run, rest - skip);
-        }
-        float T[4];
-        Sums<kFp32> sums;
-        clear<kFp32>(T, sums);
-        const bool stopped = walk_list<kFp32>(role, s_stage[wave], point_list, __builtin_amdgcn_readfirstlane(s_from[v]) + skip, count,
-                                                    (float)(__builtin_amdgcn_readfirstlane(s_tile_x[v]) * 16),
-                                                    (float)(__builtin_amdgcn_readfirstlane(s_tile_y[v]) * 16),
-                                                    points_xy, rgb_depth, conic_opacity, T, sums) < 0;
+    __syncthreads();
+    bool share = false;                                 // some list of the workgroup is long
+#pragma unroll
+    for (int t = 0; t < kT; t++) share = share || (t < teams && s_tile[t][3] >= least);
+    share = __builtin_amdgcn_readfirstlane(share);
+
+    const int square_x = square % SX * 16, square_y = square / SX * 16;
+    int left = tile_x * SX * 16 + square_x, top = tile_y * SY * 16 + square_y;
+    float T[4];
+    Sums<kFp32> sums;
+    clear<kFp32>(T, sums);
+    // The wave's own square while it works on runs: in private memory (its address is given away), not in registers.
+    float4_t kept[4];
+    asm volatile("" : : "v"((__attribute__((address_space(5))) float4_t*)&kept[0]) : "memory");
+    auto result = [&](float4_t (&p)[4]) {               // of the walk
+        Pixels px;
         finish<kFp32>(s_stage[wave], T, sums, px);
-        if (job == 0) {
-            if (lane == 0) {
-                s_rest[wave] = (!stopped && n > kOwnShare + kMinRest) ? n - kOwnShare : 0;
-                s_from[wave] = range.x + kOwnShare;
+#pragma unroll
+        for (int k = 0; k < 4; k++) p[k] = float4_t{px.r[k], px.g[k], px.b[k], px.T[k]};
+    };
+    auto keep = [&](const float4_t (&p)[4]) {
+#pragma unroll
+        for (int k = 0; k < 4; k++) kept[k] = p[k];
+        asm volatile("" : : : "memory");
+    };
+    auto recall = [&](float4_t (&p)[4]) {
+#pragma unroll
+        for (int k = 0; k < 4; k++) p[k] = kept[k];
+    };
+    enum { kOwn, kRuns, kAgain };
+    int mode = kOwn, v = -1;                            // v: the team whose tile is shared
+    int end = n >= least ? kHead : n;                    // of the walk of entries one after the other
+    int from = 0, upto = end, stop_below = kStopBelow;
+    int pos = 0, cap = 0, len = 0, left_runs = 0, step = 0;         // runs start at pos and are len long, at most cap; left_runs of a round
+    for (;;) {
+        bool above = false;
+        int walked = 0;
+        if (upto > from)
+            walked = walk_list<kFp32, true>(role, s_stage[wave], point_list, begin + from, upto - from, (float)left, (float)top,
+                                            points_xy, rgb_depth, conic_opacity, T, sums, stop_below, above);
+        bool next_tile = false;
+        if (mode == kRuns) {
+            {
+                float4_t p[4];
+                result(p);
+                float4_t* const mine = reinterpret_cast<float4_t*>(s_stage[wave]);
+#pragma unroll
+                for (int k = 0; k < 4; k++) mine[k * kWave + lane] = p[k];
+            }
+            if (above && lane == 0) s_above[step & 1][team] = 1;
+            __syncthreads();
+            if (team == v) {
+                float t[4] = {kept[0][3], kept[1][3], kept[2][3], kept[3][3]};
+                int mask = 0;
+#pragma unroll
+                for (int j = 0; j < kT; j++) {
+                    const float4_t* const part = reinterpret_cast<const float4_t*>(s_stage[j * kSquares + square]);
+#pragma unroll
+                    for (int k = 0; k < 4; k++) t[k] *= part[k * kWave + lane][3];
+                    if (all_stopped(t, kStopBelow)) mask |= 1 << j;
+                }
+                if (lane == 0) s_stopped[square] = mask;
             }
             __syncthreads();
-            shared_out = (s_rest[0] | s_rest[1] | s_rest[2] | s_rest[3]) != 0;
-            if (!shared_out) break;
-            __builtin_amdgcn_s_setprio(3);
+            int mask = s_stopped[0];
 #pragma unroll
-            for (int k = 0; k < 4; k++) {
-                kept[4 * k + 0] = px.r[k]; kept[4 * k + 1] = px.g[k];
-                kept[4 * k + 2] = px.b[k]; kept[4 * k + 3] = px.T[k];
-            }
-            continue;
-        }
-        float4* const mine = reinterpret_cast<float4*>(s_stage[wave]);
+            for (int q = 1; q < kSquares; q++) mask &= s_stopped[q];
 #pragma unroll
-        for (int k = 0; k < 4; k++) mine[k * kWave + lane] = make_float4(px.r[k], px.g[k], px.b[k], px.T[k]);
-        __syncthreads();
-        if (wave == v) {
+            for (int j = 0; j < kT; j++) mask |= s_above[step & 1][j] != 0 ? 1 << j : 0;
+            mask = __builtin_amdgcn_readfirstlane(mask);
+            const int taken = mask ? __builtin_ctz(mask) : kT;
+            if (team == v) {
+                float4_t p[4];
+                recall(p);
+                for (int j = 0; j < taken; j++) {
+                    const float4_t* const part = reinterpret_cast<const float4_t*>(s_stage[j * kSquares + square]);
 #pragma unroll
-            for (int k = 0; k < 4; k++) {
-                float r = kept[4 * k + 0], g = kept[4 * k + 1], b = kept[4 * k + 2], t = kept[4 * k + 3];
-#pragma unroll
-                for (int w = 0; w < kSharedWaves; w++) {
-                    const float4 p = reinterpret_cast<const float4*>(s_stage[w])[k * kWave + lane];
-                    r += t * p.x; g += t * p.y; b += t * p.z;
-                    t *= p.w;
+                    for (int k = 0; k < 4; k++) {
+                        const float4_t run = part[k * kWave + lane];
+                        const float t = p[k][3];
+                        p[k] = float4_t{p[k][0] + t * run[0], p[k][1] + t * run[1], p[k][2] + t * run[2], t * run[3]};
+                    }
                 }
-                kept[4 * k + 0] = r; kept[4 * k + 1] = g; kept[4 * k + 2] = b; kept[4 * k + 3] = t;
+                keep(p);
+            }
+            step++;
+            if (lane == 0 && square == 0) s_above[step & 1][team] = 0;
+            const int runs = min(taken, left_runs);
+            pos = min(n, pos + runs * len);
+            left_runs -= runs;
+            if (taken == kT) {
+                next_tile = pos >= n;
+            } else {
+                // run `taken` has the tile's stop in it or weights above one: its team walks it
+                mode = kAgain;
+                clear<kFp32>(T, sums);
+                from = pos;
+                end = min(n, pos + len);
+                upto = team == v ? end : pos;
+                stop_below = kStopBelow;
+                if (team == v) {
+#pragma unroll
+                    for (int k = 0; k < 4; k++) T[k] = kept[k][3];
+                }
+            }
+            __syncthreads();                            // the parts have been read
+            if (mode == kAgain) continue;
+        } else {
+            // entries one after the other
+            from += walked < 0 ? ~walked : walked;
+            bool stopped = walked < 0;
+            const bool bystander = mode == kAgain && team != v;
+            if (kSquares == 1) {
+                if (mode == kOwn && !share) break;
+                if (mode == kAgain) {
+                    if (team == v && lane == 0) s_stopped[0] = stopped;
+                    __syncthreads();
+                    stopped = __builtin_amdgcn_readfirstlane(s_stopped[0]) != 0;
+                }
+            } else {
+                // The stop is the tile's: a square that has stopped waits until all have, those that stopped earlier than the last
+                // one walk on to where it did, and the tile stops there if all are still opaque (a weight above 1 turns
+                // the sign of T: then a square that had stopped need not be opaque any more).
+                const int first = (mode == kAgain ? v : team) * kSquares;      // the tile's waves
+                if (stop_below == kStopBelow) {
+                    if (lane == 0) s_walked[wave] = from;
+                    __syncthreads();
+                    int furthest = 0;
+#pragma unroll
+                    for (int q = 0; q < kSquares; q++) furthest = max(furthest, s_walked[first + q]);
+                    upto = __builtin_amdgcn_readfirstlane(furthest);
+                    if (bystander) from = upto;
+                    stop_below = kNeverStop;
+                    continue;
+                }
+                // 1: opaque, 2: at the end
+                const bool opaque = all_stopped(T, kStopBelow);
+                if (lane == 0) s_stopped[wave] = bystander ? 3 : (opaque ? 1 : 0) | (upto >= end ? 2 : 0);
+                __syncthreads();
+                int state = 3;
+                bool unfinished = false;
+#pragma unroll
+                for (int t = 0; t < kT; t++) {
+                    int of_team = 3;
+#pragma unroll
+                    for (int q = 0; q < kSquares; q++) of_team &= s_stopped[t * kSquares + q];
+                    unfinished = unfinished || (t < teams && of_team == 0);
+                    if (t * kSquares == first) state = of_team;
+                }
+                state = __builtin_amdgcn_readfirstlane(state);
+                __syncthreads();                        // read before they are written again
+                stopped = (state & 1) != 0;
+                stop_below = kStopBelow;
+                if (__builtin_amdgcn_readfirstlane(unfinished)) {
+                    upto = state != 0 || bystander ? from : end;        // (a finished tile stays where it is)
+                    continue;
+                }
+                if (mode == kOwn && !share) break;
+            }
+            if (mode == kOwn) {
+                if (lane == 0 && square == 0) s_rest[team] = !stopped && n >= least;
+                __syncthreads();
+                int rests = 0;
+#pragma unroll
+                for (int t = 0; t < kT; t++) rests |= s_rest[t];
+                if (__builtin_amdgcn_readfirstlane(rests) == 0) break;
+                float4_t p[4];
+                result(p);
+                keep(p);
+                next_tile = true;
+            } else {
+                if (team == v) {
+                    float4_t p[4], before[4];
+                    result(p);
+                    recall(before);
+#pragma unroll
+                    for (int k = 0; k < 4; k++) p[k] += float4_t{before[k][0], before[k][1], before[k][2], 0.0f};
+                    keep(p);
+                }
+                pos = end;
+                left_runs--;
+                next_tile = stopped || end >= n;
+                __syncthreads();                        // s_stopped has been read
             }
         }
-        __syncthreads();
-    }
-    if (shared_out) {
-#pragma unroll
-        for (int k = 0; k < 4; k++) {
-            px.r[k] = kept[4 * k + 0]; px.g[k] = kept[4 * k + 1];
-            px.b[k] = kept[4 * k + 2]; px.T[k] = kept[4 * k + 3];
+        if (next_tile) {
+            do v++; while (v < kT && __builtin_amdgcn_readfirstlane(s_rest[min(v, kT - 1)]) == 0);
+            if (v == kT) break;
+            __builtin_amdgcn_s_setprio(3);
+            left = __builtin_amdgcn_readfirstlane(s_tile[v][0]) + square_x;
+            top = __builtin_amdgcn_readfirstlane(s_tile[v][1]) + square_y;
+            begin = __builtin_amdgcn_readfirstlane(s_tile[v][2]);
+            n = __builtin_amdgcn_readfirstlane(s_tile[v][3]);
+            pos = kHead;
+            cap = kHead / 2;
+            left_runs = 0;
         }
+        mode = kRuns;
+        if (left_runs == 0) {
+            left_runs = kRoundRuns;
+            cap = min(2 * cap, kMostRun);
+            len = min(cap, ((n - pos + kRoundRuns - 1) / kRoundRuns + 15) & ~15);
+        }
+        from = team < left_runs ? min(n, pos + team * len) : n;
+        upto = min(n, from + len);
+        stop_below = kSquares == 1 ? kStopBelow : kNeverStop;
+        clear<kFp32>(T, sums);
     }
-    if (active) write_square(lane, tile_x * 16, tile_y * 16, width, height, px, bg_r, bg_g, bg_b, out_u8, out_f32);
+    float4_t p[4];
+    if (v >= 0) recall(p);
+    else result(p);
+    Pixels px;
+#pragma unroll
+    for (int k = 0; k < 4; k++) { px.r[k] = p[k][0]; px.g[k] = p[k][1]; px.b[k] = p[k][2]; px.T[k] = p[k][3]; }
+    if (active) write_square(lane, tile_x * SX * 16 + square_x, tile_y * SY * 16 + square_y, width, height, px, bg_r, bg_g, bg_b, out_u8, out_f32);
 }
 #undef FGS_BLEND_PARAMS
 
@@ -1013,7 +1229,7 @@ int check_tile(int block_x, int block_y, int* sx, int* sy, const char* who)
 }
 
 // A frame of at most kOrderCap tiles is about resident at once: its tiles are ranked by the length of
-// their lists and the longest start first (16x16 tiles also share out their long lists).  In a
+// their lists, the longest start first, and the long ones are shared out.  In a
 // larger frame the short lists at any time fill in behind the long ones, and neighbouring tiles
 // finding each other's lines in the L2 counts for more.
 bool is_ranked(int tiles_x, int tiles_y) { return (long long)tiles_x * tiles_y <= kOrderCap; }
@@ -1045,6 +1261,16 @@ int ranges_impl(int block_x, int block_y, int num_rendered, int width, int heigh
     return check_hip(hipGetLastError(), who);
 }
 
+// Teams of a workgroup of blend_kernel_shared, a divisor of kRoundRuns.  More of them where there are few tiles: 192 with
+// 1811 entries on average 208 us by 4, 183 by 8; 475 with 760 152, 112; 950 with 1320 184, 149.  32x32 tiles: 247 with 4372 1137 by 2,
+// 975 by 4.
+int teams_of(int sx, int sy, int num_tiles, int cus)
+{
+    if (sx == 1 && sy == 1) return num_tiles > 4 * cus ? 4 : 8;
+    if (sx == 2 && sy == 2) return num_tiles > cus ? 2 : 4;
+    return 4;
+}
+
 // render.cu:566-575
 int blend_impl(int block_x, int block_y, int width, int height,
                const float* points_xy, const float* rgb_depth, const float* conic_opacity,
@@ -1068,36 +1294,45 @@ int blend_impl(int block_x, int block_y, int width, int height,
     const long long groups = (blocks + 7) / 8 * 8 * 64;
     if (groups > 0x7fffffffLL) return fail(FGS_E_INVALID, "%s: image too large", who);
     const int num_tiles = tiles_x * tiles_y;
+    const bool fp32 = mode == FGS_COLOUR_SUMS_FP32;
+#define FGS_BLEND_ARGS (const int2*)ranges, values_sorted, width, height, tiles_x, tiles_y,                     \
+                       (const float2*)points_xy, (const float4*)rgb_depth, (const float4*)conic_opacity,        \
+                       bg[0], bg[1], bg[2], out_u8, out_f32
+    if (!is_ranked(tiles_x, tiles_y)) {
+        auto launch = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3((unsigned)groups), dim3(kWave * sx * sy), 0, st, FGS_BLEND_ARGS);
+        };
+        if (sx == 1 && sy == 1) launch(fp32 ? blend_kernel<1, 1, true> : blend_kernel<1, 1, false>);
+        else if (sx == 2 && sy == 1) launch(fp32 ? blend_kernel<2, 1, true> : blend_kernel<2, 1, false>);
+        else launch(fp32 ? blend_kernel<2, 2, true> : blend_kernel<2, 2, false>);
+        return check_hip(hipGetLastError(), who);
+    }
+    int device = 0, cus = 0;
+    FGS_HIP_TRY(hipGetDevice(&device));
+    FGS_HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
     uint32_t* tile_order = nullptr;
     std::unique_lock<std::mutex> enqueue;       // from the ranking to the blend that reads it
-    if (is_ranked(tiles_x, tiles_y)) {
-        rc = tile_order_table(st, &tile_order, &enqueue);
-        if (rc != FGS_OK) return rc;
-        if (tile_order) hipLaunchKernelGGL(tile_order_kernel, dim3(1), dim3(1024), 0, st, (const int2*)ranges, num_tiles, tile_order);
+    rc = tile_order_table(st, &tile_order, &enqueue);
+    if (rc != FGS_OK) return rc;
+    if (tile_order)
+        hipLaunchKernelGGL(tile_order_kernel, dim3(1), dim3(1024), 0, st, (const int2*)ranges, num_tiles, tile_order, sx * sy, 4 * cus);
+    auto launch = [&](auto kernel, int teams) {
+        const int waves = sx * sy * teams, resident = cus * std::max(1, 4 * (fp32 ? kBlendWaves<true> : kBlendWaves<false>) / waves);
+        const int per_group = num_tiles <= resident ? 1 : teams;
+        hipLaunchKernelGGL(kernel, dim3((unsigned)(tile_order ? num_tiles : (num_tiles + per_group - 1) / per_group)),
+                           dim3(kWave * waves), 0, st, FGS_BLEND_ARGS, (const uint32_t*)tile_order, per_group, 4 * cus);
+    };
+    const int teams = teams_of(sx, sy, num_tiles, cus);
+    if (sx == 1 && sy == 1) {
+        if (teams == 8) launch(fp32 ? blend_kernel_shared<1, 1, 8, true> : blend_kernel_shared<1, 1, 8, false>, 8);
+        else launch(fp32 ? blend_kernel_shared<1, 1, 4, true> : blend_kernel_shared<1, 1, 4, false>, 4);
+    } else if (sx == 2 && sy == 1) {
+        launch(fp32 ? blend_kernel_shared<2, 1, 4, true> : blend_kernel_shared<2, 1, 4, false>, 4);
+    } else {
+        if (teams == 4) launch(fp32 ? blend_kernel_shared<2, 2, 4, true> : blend_kernel_shared<2, 2, 4, false>, 4);
+        else launch(fp32 ? blend_kernel_shared<2, 2, 2, true> : blend_kernel_shared<2, 2, 2, false>, 2);
     }
-    const dim3 grid((unsigned)(tile_order ? num_tiles : groups));
-    const bool fp32 = mode == FGS_COLOUR_SUMS_FP32;
-#define FGS_LAUNCH_BLEND(SX, SY)                                                                        \
-    do {                                                                                                \
-        auto kernel = fp32 ? blend_kernel<SX, SY, true> : blend_kernel<SX, SY, false>;                  \
-        hipLaunchKernelGGL(kernel, grid, dim3(kWave * SX * SY), 0, st,                                  \
-                           (const int2*)ranges, values_sorted, width, height, tiles_x, tiles_y,         \
-                           (const float2*)points_xy, (const float4*)rgb_depth, (const float4*)conic_opacity, \
-                           bg[0], bg[1], bg[2], out_u8, out_f32, (const uint32_t*)tile_order);          \
-    } while (0)
-    if (is_ranked(tiles_x, tiles_y) && sx == 1 && sy == 1) {
-        int device = 0, cus = 0;
-        FGS_HIP_TRY(hipGetDevice(&device));
-        FGS_HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
-        const int tiles_per_group = num_tiles <= cus * (fp32 ? kBlendWaves<true> : kBlendWaves<false>) ? 1 : kSharedWaves;
-        hipLaunchKernelGGL(fp32 ? blend_kernel_shared<true> : blend_kernel_shared<false>, dim3((unsigned)((num_tiles + tiles_per_group - 1) / tiles_per_group)), dim3(kSharedWaves * kWave), 0, st,
-                           (const int2*)ranges, values_sorted, width, height, tiles_x, tiles_y,
-                           (const float2*)points_xy, (const float4*)rgb_depth, (const float4*)conic_opacity,
-                           bg[0], bg[1], bg[2], out_u8, out_f32, (const uint32_t*)tile_order, tiles_per_group);
-    } else if (sx == 1 && sy == 1) FGS_LAUNCH_BLEND(1, 1);
-    else if (sx == 2 && sy == 1) FGS_LAUNCH_BLEND(2, 1);
-    else FGS_LAUNCH_BLEND(2, 2);
-#undef FGS_LAUNCH_BLEND
+#undef FGS_BLEND_ARGS
     return check_hip(hipGetLastError(), who);
 }
 
@@ -1177,11 +1412,23 @@ extern "C" const char* fgs_blend_kernel_name(int block_x, int block_y, int width
     if (colour_mode(flags, &mode, "fgs_blend_kernel_name") != FGS_OK) return "";
     const bool ranked = is_ranked((width + block_x - 1) / block_x, (height + block_y - 1) / block_y);
     const bool fp32 = mode == FGS_COLOUR_SUMS_FP32;
-#define FGS_NAME(ranked_name, name) (ranked ? (fp32 ? "tile_order_kernel + " ranked_name "true>" : "tile_order_kernel + " ranked_name "false>") \
-                                            : (fp32 ? name "true>" : name "false>"))
-    if (sx == 1 && sy == 1) return FGS_NAME("blend_kernel_shared<", "blend_kernel<1, 1, ");
-    if (sx == 2 && sy == 1) return FGS_NAME("blend_kernel<2, 1, ", "blend_kernel<2, 1, ");
-    return FGS_NAME("blend_kernel<2, 2, ", "blend_kernel<2, 2, ");
+#define FGS_NAME(name) (fp32 ? name "true>" : name "false>")
+    if (ranked) {
+        const int tiles = ((width + block_x - 1) / block_x) * ((height + block_y - 1) / block_y);
+        int device = 0, cus = 0;
+        if (hipGetDevice(&device) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess) {
+            (void)hipGetLastError();
+            cus = 256;          // no device: what an MI355X would launch
+        }
+        const int teams = teams_of(sx, sy, tiles, cus);
+        if (sx == 1 && sy == 1)
+            return teams == 8 ? FGS_NAME("tile_order_kernel + blend_kernel_shared<1, 1, 8, ") : FGS_NAME("tile_order_kernel + blend_kernel_shared<1, 1, 4, ");
+        if (sx == 2 && sy == 1) return FGS_NAME("tile_order_kernel + blend_kernel_shared<2, 1, 4, ");
+        return teams == 4 ? FGS_NAME("tile_order_kernel + blend_kernel_shared<2, 2, 4, ") : FGS_NAME("tile_order_kernel + blend_kernel_shared<2, 2, 2, ");
+    }
+    if (sx == 1 && sy == 1) return FGS_NAME("blend_kernel<1, 1, ");
+    if (sx == 2 && sy == 1) return FGS_NAME("blend_kernel<2, 1, ");
+    return FGS_NAME("blend_kernel<2, 2, ");
 #undef FGS_NAME
 }
 

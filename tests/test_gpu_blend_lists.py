@@ -346,3 +346,43 @@ def test_error_against_float64(oracle, block, splats):
           % (splats, block[0], block[1], rms[0], rms[1], worst[0], worst[1]))
     assert same.mean() > 0.99
     assert rms[0] <= 1.5 * rms[1] + 7e-7 and worst[0] <= 2 * worst[1] + 1.4e-5
+
+
+@pytest.mark.parametrize("flags", ["fp32", "f16"])
+@pytest.mark.parametrize("tiles", [40, 300, 1100])
+@pytest.mark.parametrize("block", BLOCKS)
+def test_lists_shared_by_the_teams_of_a_workgroup(oracle, block, tiles, flags):
+    """Lists around the lengths where they are shared out and where rounds and runs end, odd ones among them, with opaque content
+    that ends the walk in the head, in one run or another, on a run's last pair, or never, and with weights above one in
+    some runs; workgroups of 16, 8, 4 and 2 teams.  The walk ends behind the reference's pair, so the bound is the one of a
+    whole walk: rounding of sums of up to 0.5 * 1500 weights of 1.5, some 1e-5, and twice that where weights above one turn T's sign."""
+    rng = np.random.default_rng(tiles + block[0] * block[1])
+    lengths = [1, 2, 63, 64, 65, 127, 128, 129, 191, 192, 193, 257, 319, 320, 321, 385, 511, 576, 577, 700, 832, 833, 1000, 1089, 1500, 1501]
+    stops = [None, 10, 60, 66, 100, 127, 128, 160, 190, 250, 300, 319, 400, 500, 650, 900]
+    lists = []
+    for i in range(min(tiles, 40)):
+        n = lengths[i % len(lengths)] if i < 30 else 1200
+        top = block[1] * i
+        xy = rng.uniform(0, 1, (n, 2)) * block + (0, top)
+        cx, cz = -rng.uniform(0.005, 0.3, n), -rng.uniform(0.005, 0.3, n)
+        w = np.log2(rng.uniform(0.002, 0.02, n))
+        cy = rng.uniform(-0.9, 0.9, n) * 2 * np.sqrt(cx * cz)
+        at = stops[(5 * i) % len(stops)]
+        if at is not None and at + 30 <= n:          # opaque for every pixel: alpha of 0.9 and more
+            o = slice(at, at + 30)
+            cx[o] = cz[o] = -1e-5
+            cy[o] = 0.0
+            w[o] = np.log2(0.92)
+            # (wide tiles: other squares stop at other pairs)
+            o = slice(at, at + 8)
+            cx[o] = cz[o] = -2e-2
+        if i % 7 == 3 and n > 150:                   # weights of up to 1.4
+            w[rng.integers(70, n, 3)] = 0.5
+        lists.append((xy, np.stack([cx, cy, cz, w], 1), rng.uniform(0, 1, (n, 3))))
+    W, H = block[0], block[1] * tiles
+    arrays = column_of_tiles(lists, tiles)
+    bg = np.array([0.25, 0.5, 0.75], np.float32)
+    _, ref, _ = oracle.render(W, H, block[0], block[1], *arrays, bg, want_u8=False)
+    out, _ = gpu_blend(block, W, H, arrays, bg, cabi.BLEND_FP32 if flags == "fp32" else cabi.BLEND_MATRIX_F16)
+    err = np.abs(out - ref)
+    assert err.max() <= (3e-5 if flags == "fp32" else 2.0 ** -10 * 1.5), "max abs image error %g at %r" % (err.max(), np.unravel_index(err.argmax(), err.shape))
