@@ -106,7 +106,7 @@ PassGrid pass_grid(int n, int tile)
 {
     PassGrid g;
     g.tiles = (n + tile - 1) / tile;
-    g.chunk = (g.tiles + kMaxChunks - 1) / kMaxChunks;       // one count workgroup each: about one per CU
+    g.chunk = g.tiles > kMaxChunks ? (g.tiles + kMaxChunks - 1) / kMaxChunks : 1;       // one count workgroup each: about one per CU
     g.chunks = (g.tiles + g.chunk - 1) / g.chunk;
     return g;
 }
