@@ -927,7 +927,7 @@ __global__ __launch_bounds__(kWave * SX * SY) __attribute__((amdgpu_waves_per_eu
 // instead of three eighths: 1080p 141 and 132, 32x32 276 and 325; heads of 128 or 256 entries: 1080p 127 and 123, 1280x720 98
 // and 148 (64: 121 and 98, all with rounds of as many runs as teams); rounds of four runs: 32x16 108, 1280x720 98, 256x192 206.
 //
-// Unranked (no table: stream capture, no memory) every team has a tile and long lists are shared with the others of the workgroup, cut as
+// Unranked (stream capture, no memory, all workgroups resident at once) every team has a tile and long lists are shared with the others of the workgroup, cut as
 // they are with a table.  What a team has blended of its own tile waits in private memory meanwhile.
 constexpr int kHead = 64, kMostRun = 512, kRoundRuns = 8;
 // resident waves per SIMD: whole workgroups
@@ -1272,7 +1272,11 @@ int teams_of(int sx, int sy, int num_tiles, int cus)
 }
 
 // render.cu:566-575
-int blend_impl(int block_x, int block_y, int width, int height,
+// rank: a blend by itself (fgs_blend) is two launches, the ranking and the blend.  Behind the ranges of the same call (fgs_render)
+// a frame whose workgroups are all resident at once even with one tile each goes unranked, since nothing starts later than
+// anything else there; the image is the same bits.  256x192 / 2.8k pairs 11.1 -> 8.7 us, 348k pairs 181 -> 178, 400x300 / 362k
+// 110 -> 107, opaque needles 110 -> 117, 700x600 in 32x32 tiles 114 -> 112.
+int blend_impl(bool rank, int block_x, int block_y, int width, int height,
                const float* points_xy, const float* rgb_depth, const float* conic_opacity,
                const uint32_t* values_sorted, const int* ranges, const float bg[3],
                uint8_t* out_u8, float* out_f32, int flags, void* stream, const char* who)
@@ -1312,25 +1316,27 @@ int blend_impl(int block_x, int block_y, int width, int height,
     FGS_HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
     uint32_t* tile_order = nullptr;
     std::unique_lock<std::mutex> enqueue;       // from the ranking to the blend that reads it
-    rc = tile_order_table(st, &tile_order, &enqueue);
-    if (rc != FGS_OK) return rc;
+    const int teams = teams_of(sx, sy, num_tiles, cus), waves = sx * sy * teams;
+    const int resident = cus * std::max(1, 4 * (fp32 ? kBlendWaves<true> : kBlendWaves<false>) / waves);
+    if (rank || num_tiles > resident) {
+        rc = tile_order_table(st, &tile_order, &enqueue);
+        if (rc != FGS_OK) return rc;
+    }
     if (tile_order)
         hipLaunchKernelGGL(tile_order_kernel, dim3(1), dim3(1024), 0, st, (const int2*)ranges, num_tiles, tile_order, sx * sy, 4 * cus);
-    auto launch = [&](auto kernel, int teams) {
-        const int waves = sx * sy * teams, resident = cus * std::max(1, 4 * (fp32 ? kBlendWaves<true> : kBlendWaves<false>) / waves);
+    auto launch = [&](auto kernel) {
         const int per_group = num_tiles <= resident ? 1 : teams;
         hipLaunchKernelGGL(kernel, dim3((unsigned)(tile_order ? num_tiles : (num_tiles + per_group - 1) / per_group)),
                            dim3(kWave * waves), 0, st, FGS_BLEND_ARGS, (const uint32_t*)tile_order, per_group, 4 * cus);
     };
-    const int teams = teams_of(sx, sy, num_tiles, cus);
     if (sx == 1 && sy == 1) {
-        if (teams == 8) launch(fp32 ? blend_kernel_shared<1, 1, 8, true> : blend_kernel_shared<1, 1, 8, false>, 8);
-        else launch(fp32 ? blend_kernel_shared<1, 1, 4, true> : blend_kernel_shared<1, 1, 4, false>, 4);
+        if (teams == 8) launch(fp32 ? blend_kernel_shared<1, 1, 8, true> : blend_kernel_shared<1, 1, 8, false>);
+        else launch(fp32 ? blend_kernel_shared<1, 1, 4, true> : blend_kernel_shared<1, 1, 4, false>);
     } else if (sx == 2 && sy == 1) {
-        launch(fp32 ? blend_kernel_shared<2, 1, 4, true> : blend_kernel_shared<2, 1, 4, false>, 4);
+        launch(fp32 ? blend_kernel_shared<2, 1, 4, true> : blend_kernel_shared<2, 1, 4, false>);
     } else {
-        if (teams == 4) launch(fp32 ? blend_kernel_shared<2, 2, 4, true> : blend_kernel_shared<2, 2, 4, false>, 4);
-        else launch(fp32 ? blend_kernel_shared<2, 2, 2, true> : blend_kernel_shared<2, 2, 2, false>, 2);
+        if (teams == 4) launch(fp32 ? blend_kernel_shared<2, 2, 4, true> : blend_kernel_shared<2, 2, 4, false>);
+        else launch(fp32 ? blend_kernel_shared<2, 2, 2, true> : blend_kernel_shared<2, 2, 2, false>);
     }
 #undef FGS_BLEND_ARGS
     return check_hip(hipGetLastError(), who);
@@ -1350,7 +1356,7 @@ int render_impl(int block_x, int block_y, int num_rendered, int width, int heigh
         return fail(FGS_E_INVALID, "%s: null buffer", who);
     rc = ranges_impl(block_x, block_y, num_rendered, width, height, keys_sorted, ranges, stream, who);
     if (rc != FGS_OK) return rc;
-    return blend_impl(block_x, block_y, width, height, points_xy, rgb_depth, conic_opacity, values_sorted, ranges,
+    return blend_impl(false, block_x, block_y, width, height, points_xy, rgb_depth, conic_opacity, values_sorted, ranges,
                       bg, out_u8, out_f32, flags, stream, who);
 }
 
@@ -1444,7 +1450,7 @@ extern "C" int fgs_blend(int block_x, int block_y, int width, int height,
                          const uint32_t* gaussian_values_sorted, const int* ranges, const float bg_color[3],
                          uint8_t* out_color_u8, float* out_color_f32, void* stream)
 {
-    return fgs::blend_impl(block_x, block_y, width, height, points_xy, rgb_depth, conic_opacity,
+    return fgs::blend_impl(true, block_x, block_y, width, height, points_xy, rgb_depth, conic_opacity,
                            gaussian_values_sorted, ranges, bg_color, out_color_u8, out_color_f32, 0, stream, "fgs_blend");
 }
 
@@ -1453,7 +1459,7 @@ extern "C" int fgs_blend_ex(int block_x, int block_y, int width, int height,
                             const uint32_t* gaussian_values_sorted, const int* ranges, const float bg_color[3],
                             uint8_t* out_color_u8, float* out_color_f32, int flags, void* stream)
 {
-    return fgs::blend_impl(block_x, block_y, width, height, points_xy, rgb_depth, conic_opacity,
+    return fgs::blend_impl(true, block_x, block_y, width, height, points_xy, rgb_depth, conic_opacity,
                            gaussian_values_sorted, ranges, bg_color, out_color_u8, out_color_f32, flags, stream, "fgs_blend_ex");
 }
 
