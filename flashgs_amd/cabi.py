@@ -24,6 +24,8 @@ SIGNATURES = {
                               + [C.c_void_p] * 6 + [C.c_int64, C.c_void_p]),
     "fgs_preprocess_mirrored": (C.c_int, [C.c_int] + [C.c_void_p] * 4 + [C.c_int] * 4 + [C.c_void_p] * 2 + [C.c_float] * 4
                                 + [C.c_void_p] * 6 + [C.c_int64, C.c_void_p, C.c_void_p]),
+    "fgs_preprocess_chained": (C.c_int, [C.c_int] + [C.c_void_p] * 4 + [C.c_int] * 4 + [C.c_void_p] * 2 + [C.c_float] * 4
+                               + [C.c_void_p] * 6 + [C.c_int64, C.c_void_p, C.c_void_p, C.c_void_p]),
     "fgs_wait_count": (C.c_int, [C.c_void_p, C.c_double, C.c_void_p]),
     "fgs_sort_gaussian": (C.c_int, [C.c_int] * 5 + [C.c_void_p, C.c_size_t] + [C.c_void_p] * 4 + [C.c_void_p]),
     "fgs_get_sort_buffer_size": (C.c_size_t, [C.c_int]),

@@ -160,6 +160,10 @@ void check_arguments()
                 "null count mirror");
         refused(fgs_preprocess_mirrored(-1, f, f, f, f, 64, 64, 16, 16, pos, rot, 1, 1, 100, 0.01f, f, f, f, k, v, i32, 16, &word, nullptr),
                 "negative P with a count mirror");
+        refused(fgs_preprocess_chained(16, f, f, f, f, 64, 64, 16, 16, pos, rot, 1, 1, 100, 0.01f, f, f, f, k, v, i32, 16, &word, nullptr, nullptr),
+                "null next offset");
+        refused(fgs_preprocess_chained(16, f, f, f, f, 64, 64, 16, 16, pos, rot, 1, 1, 100, 0.01f, f, f, f, k, v, i32, 16, &word, i32, nullptr),
+                "the current offset as the next one");
     }
 }
 

@@ -476,7 +476,8 @@ __global__ __launch_bounds__(kBlock) void preprocess_kernel(
     int status_capacity,
     int num_blocks,                        // workgroups that hold Gaussians; the grid has one more, the scanner's
     unsigned spin_limit,
-    int* __restrict__ count_mirror)        // pinned host memory that also receives the pair count, or null
+    int* __restrict__ count_mirror,        // pinned host memory that also receives the pair count, or null
+    int* __restrict__ next_offset)         // a word that is zero when the launch has ended (the start of a later one), or null
 {
     __shared__ uint32_t s_wave_total[kWavesPerBlock];
     __shared__ uint32_t s_block_base;
@@ -531,6 +532,8 @@ __global__ __launch_bounds__(kBlock) void preprocess_kernel(
             // generation can be handed to the next launch.  Gave up: workgroups may still be
             // dispatched; the generation stays and the words are marked unusable.
             if (lane == 0) publish(scan_words, gave_up ? (uint64_t)which | kControlAborted : (uint64_t)(which ^ 1u));
+        } else if (tid == kWave && next_offset) {
+            *next_offset = 0;           // (one launch less in a caller's frame than clearing it there)
         }
         return;
     }
@@ -1151,7 +1154,7 @@ int preprocess_impl(bool allocate, const char* who, int P,
                     float focal_x, float focal_y, float zFar, float zNear,
                     float* points_xy, float* rgb_depth, float* conic_opacity,
                     uint64_t* gaussian_keys_unsorted, uint32_t* gaussian_values_unsorted,
-                    int* curr_offset, int64_t key_capacity, int* count_mirror, void* stream)
+                    int* curr_offset, int64_t key_capacity, int* count_mirror, int* next_offset, void* stream)
 {
     if (P < 0) return fail(FGS_E_INVALID, "%s: P = %d is negative", who, P);
     if (width <= 0 || height <= 0 || block_x <= 0 || block_y <= 0)
@@ -1227,7 +1230,7 @@ int preprocess_impl(bool allocate, const char* who, int P,
     hipLaunchKernelGGL(preprocess_kernel, dim3(num_blocks + 1), dim3(kBlock), 0, st,
                        P, positions, shs, opacities, cov3Ds, cam, points_xy, rgb_depth, conic_opacity,
                        gaussian_keys_unsorted, gaussian_values_unsorted, curr_offset, key_capacity,
-                       words, status_capacity, num_blocks, g_spin_limit.load(), mirror_on_device);
+                       words, status_capacity, num_blocks, g_spin_limit.load(), mirror_on_device, next_offset);
     return check_hip(hipGetLastError(), "preprocess_kernel launch");
 }
 
@@ -1271,7 +1274,7 @@ extern "C" int fgs_preprocess(int P,
     return fgs::preprocess_impl(true, "fgs_preprocess", P, positions, shs, opacities, cov3Ds, width, height, block_x, block_y,
                                 cam_position, cam_rotation, focal_x, focal_y, zFar, zNear, points_xy, rgb_depth,
                                 conic_opacity, gaussian_keys_unsorted, gaussian_values_unsorted, curr_offset,
-                                key_capacity, nullptr, stream);
+                                key_capacity, nullptr, nullptr, stream);
 }
 
 extern "C" int fgs_preprocess_static(int P,
@@ -1286,7 +1289,7 @@ extern "C" int fgs_preprocess_static(int P,
     return fgs::preprocess_impl(false, "fgs_preprocess_static", P, positions, shs, opacities, cov3Ds, width, height,
                                 block_x, block_y, cam_position, cam_rotation, focal_x, focal_y, zFar, zNear, points_xy,
                                 rgb_depth, conic_opacity, gaussian_keys_unsorted, gaussian_values_unsorted, curr_offset,
-                                key_capacity, nullptr, stream);
+                                key_capacity, nullptr, nullptr, stream);
 }
 
 extern "C" int fgs_preprocess_mirrored(int P,
@@ -1302,7 +1305,24 @@ extern "C" int fgs_preprocess_mirrored(int P,
     return fgs::preprocess_impl(true, "fgs_preprocess_mirrored", P, positions, shs, opacities, cov3Ds, width, height,
                                 block_x, block_y, cam_position, cam_rotation, focal_x, focal_y, zFar, zNear, points_xy,
                                 rgb_depth, conic_opacity, gaussian_keys_unsorted, gaussian_values_unsorted, curr_offset,
-                                key_capacity, count_mirror, stream);
+                                key_capacity, count_mirror, nullptr, stream);
+}
+
+extern "C" int fgs_preprocess_chained(int P,
+                                      const float* positions, const float* shs, const float* opacities, const float* cov3Ds,
+                                      int width, int height, int block_x, int block_y,
+                                      const float cam_position[3], const float cam_rotation[9],
+                                      float focal_x, float focal_y, float zFar, float zNear,
+                                      float* points_xy, float* rgb_depth, float* conic_opacity,
+                                      uint64_t* gaussian_keys_unsorted, uint32_t* gaussian_values_unsorted,
+                                      int* curr_offset, int64_t key_capacity, int* count_mirror, int* next_offset, void* stream)
+{
+    if (!count_mirror || !next_offset) return fgs::fail(FGS_E_INVALID, "fgs_preprocess_chained: null count_mirror or next_offset");
+    if (next_offset == curr_offset) return fgs::fail(FGS_E_INVALID, "fgs_preprocess_chained: next_offset is curr_offset");
+    return fgs::preprocess_impl(true, "fgs_preprocess_chained", P, positions, shs, opacities, cov3Ds, width, height,
+                                block_x, block_y, cam_position, cam_rotation, focal_x, focal_y, zFar, zNear, points_xy,
+                                rgb_depth, conic_opacity, gaussian_keys_unsorted, gaussian_values_unsorted, curr_offset,
+                                key_capacity, count_mirror, next_offset, stream);
 }
 
 extern "C" int fgs_wait_count(const int* count_mirror, double timeout_seconds, int* count)

@@ -85,7 +85,7 @@ void preprocess_to(torch::Tensor& orig_points, torch::Tensor& shs, torch::Tensor
                    float focal_x, float focal_y, float zFar, float zNear,
                    torch::Tensor& points_xy, torch::Tensor& rgb_depth, torch::Tensor& conic_opacity,
                    torch::Tensor& gaussian_keys_unsorted, torch::Tensor& gaussian_values_unsorted,
-                   torch::Tensor& curr_offset, int* count_mirror)
+                   torch::Tensor& curr_offset, int* count_mirror, torch::Tensor* next_offset = nullptr)
 {
     need(opacities.dim() >= 1, "opacities must have at least one dimension");
     const int64_t P = opacities.size(0);
@@ -104,8 +104,23 @@ void preprocess_to(torch::Tensor& orig_points, torch::Tensor& shs, torch::Tensor
     const std::vector<float> rot = host_floats(rotation, "rotation", 9);
     const int64_t capacity = std::min(gaussian_keys_unsorted.numel(), gaussian_values_unsorted.numel());
     need(capacity > 0, "gaussian_keys_unsorted / gaussian_values_unsorted are empty");
+    if (next_offset) need_device(*next_offset, "next_offset", torch::kInt32, 1, opacities);
 
     DeviceScope scope(opacities);
+    if (next_offset) {
+        *count_mirror = FGS_COUNT_PENDING;
+        fgs_check(fgs_preprocess_chained((int)P,
+                                         orig_points.data_ptr<float>(), shs.data_ptr<float>(), opacities.data_ptr<float>(),
+                                         cov3Ds.data_ptr<float>(), width, height, block_x, block_y, pos.data(), rot.data(),
+                                         focal_x, focal_y, zFar, zNear,
+                                         points_xy.data_ptr<float>(), rgb_depth.data_ptr<float>(), conic_opacity.data_ptr<float>(),
+                                         (uint64_t*)gaussian_keys_unsorted.data_ptr<int64_t>(),
+                                         (uint32_t*)gaussian_values_unsorted.data_ptr<int>(),
+                                         curr_offset.data_ptr<int>(), capacity, count_mirror, next_offset->data_ptr<int>(),
+                                         current_stream(opacities)),
+                  "preprocess_chained");
+        return;
+    }
     if (count_mirror) {
         *count_mirror = FGS_COUNT_PENDING;
         fgs_check(fgs_preprocess_mirrored((int)P,
@@ -165,6 +180,20 @@ void preprocess_mirrored(torch::Tensor& orig_points, torch::Tensor& shs, torch::
     preprocess_to(orig_points, shs, opacities, cov3Ds, width, height, block_x, block_y, position, rotation,
                   focal_x, focal_y, zFar, zNear, points_xy, rgb_depth, conic_opacity,
                   gaussian_keys_unsorted, gaussian_values_unsorted, curr_offset, mirror_word(count_mirror));
+}
+
+// No counterpart in the reference: preprocess_mirrored that leaves zero in next_offset, for the next frame to start from.
+void preprocess_chained(torch::Tensor& orig_points, torch::Tensor& shs, torch::Tensor& opacities, torch::Tensor& cov3Ds,
+                        int width, int height, int block_x, int block_y,
+                        torch::Tensor& position, torch::Tensor& rotation,
+                        float focal_x, float focal_y, float zFar, float zNear,
+                        torch::Tensor& points_xy, torch::Tensor& rgb_depth, torch::Tensor& conic_opacity,
+                        torch::Tensor& gaussian_keys_unsorted, torch::Tensor& gaussian_values_unsorted,
+                        torch::Tensor& curr_offset, torch::Tensor& count_mirror, torch::Tensor& next_offset)
+{
+    preprocess_to(orig_points, shs, opacities, cov3Ds, width, height, block_x, block_y, position, rotation,
+                  focal_x, focal_y, zFar, zNear, points_xy, rgb_depth, conic_opacity,
+                  gaussian_keys_unsorted, gaussian_values_unsorted, curr_offset, mirror_word(count_mirror), &next_offset);
 }
 
 int wait_count(torch::Tensor& count_mirror, double timeout_seconds)
@@ -290,6 +319,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
     ops.def("render_32x32", &render<32, 32>, "tile ranges and alpha blending, 32x32 tiles");
     ops.def("preprocess_mirrored", &preprocess_mirrored,
             "preprocess that also stores the pair count into a pinned host tensor as soon as it is known");
+    ops.def("preprocess_chained", &preprocess_chained,
+            "preprocess_mirrored that also leaves zero in another offset tensor, for the next frame to start from");
     ops.def("wait_count", &wait_count, "poll the pinned host tensor of preprocess_mirrored for the pair count");
     ops.def("reset_scan", &reset_scan, "clear preprocess's scan status on the tensor's device and current stream");
 }

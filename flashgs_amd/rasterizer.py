@@ -4,8 +4,8 @@ through ``flash_gaussian_splatting.ops``, ``savePpm`` and ``render_scene``.
 
 Differences from the reference driver: the output image is allocated once instead of per frame,
 the pair count is polled in pinned host memory, where the preprocess launch stores it as soon as
-it is known (``ops.preprocess_mirrored`` / ``ops.wait_count``), instead of being copied back with
-a blocking read,
+it is known (``ops.preprocess_chained`` / ``ops.wait_count``), instead of being copied back with
+a blocking read, and that launch clears the offset the next frame starts from,
 the too-many-pairs condition raises a real exception (``example.py:82`` raises a string), a
 preprocess whose bounded waits gave up is launched once more after ``ops.reset_scan`` and raises
 ``ScanGaveUp`` if that fails too, and the tile size is a constructor argument.  ``BatchRasterizer``
@@ -109,7 +109,10 @@ class Rasterizer:
         self.SORT_BUFFER_SIZE = ops().get_sort_buffer_size(MAX_NUM_RENDERED)
         self.list_sorting_space = torch.zeros(self.SORT_BUFFER_SIZE, device=dev, dtype=torch.int8)
         self.ranges = torch.zeros((MAX_NUM_TILES, 2), device=dev, dtype=torch.int32)
-        self.curr_offset = torch.zeros(1, device=dev, dtype=torch.int32)
+        # two words in turn: a frame's preprocess leaves zero in the one that the next frame starts from
+        self._offsets = torch.zeros(2, device=dev, dtype=torch.int32).split(1)
+        self.curr_offset = self._offsets[0]
+        self._cleared = None
         self.points_xy = torch.zeros((scene.num_vertex, 2), device=dev, dtype=torch.float32)
         self.rgb_depth = torch.zeros((scene.num_vertex, 4), device=dev, dtype=torch.float32)
         self.conic_opacity = torch.zeros((scene.num_vertex, 4), device=dev, dtype=torch.float32)
@@ -141,17 +144,24 @@ class Rasterizer:
             raise ScanGaveUp("a workgroup of the previous frame's preprocess gave up waiting after the pair count "
                              "had been reported; that frame's image is not to be used")
         for attempt in range(2):
-            self.curr_offset.zero_()
-            o.preprocess_mirrored(scene.position, scene.shs, scene.opacity, scene.cov3d,
-                                  camera.width, camera.height, bx, by,
-                                  camera.position, camera.rotation,
-                                  camera.focal_x, camera.focal_y, camera.zFar, camera.zNear,
-                                  self.points_xy, self.rgb_depth, self.conic_opacity,
-                                  self.gaussian_keys_unsorted, self.gaussian_values_unsorted, self.curr_offset, self._count)
+            if self._cleared is not None and any(self.curr_offset is word for word in self._offsets):
+                self.curr_offset = self._cleared
+            else:
+                self.curr_offset.zero_()
+            self._cleared = None
+            other = self._offsets[1] if self.curr_offset is self._offsets[0] else self._offsets[0]
+            o.preprocess_chained(scene.position, scene.shs, scene.opacity, scene.cov3d,
+                                 camera.width, camera.height, bx, by,
+                                 camera.position, camera.rotation,
+                                 camera.focal_x, camera.focal_y, camera.zFar, camera.zNear,
+                                 self.points_xy, self.rgb_depth, self.conic_opacity,
+                                 self.gaussian_keys_unsorted, self.gaussian_values_unsorted, self.curr_offset, self._count,
+                                 other)
             # the count arrives while the launch is still writing keys; the sort below is enqueued
             # behind it on the same stream
             num_rendered = o.wait_count(self._count, 60.0)
             if num_rendered >= 0:
+                self._cleared = other if scene.num_vertex > 0 else None
                 break
             # a bounded wait of the launch gave up: clear the scan status and launch once more
             o.reset_scan(self.curr_offset)

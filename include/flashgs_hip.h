@@ -117,6 +117,21 @@ int fgs_preprocess_mirrored(int P,
                             int* curr_offset, int64_t key_capacity, int* count_mirror, void* stream);
 
 /*
+ * No counterpart in the reference.  fgs_preprocess_mirrored that also leaves zero in *next_offset (device memory, another
+ * word than *curr_offset): a caller with two words uses them in turn, one frame's launch clearing the start of the
+ * next, and needs no launch of its own to clear it.  Only a launch whose count came out at zero or more, with P > 0, has
+ * cleared the word for certain.
+ */
+int fgs_preprocess_chained(int P,
+                           const float* positions, const float* shs, const float* opacities, const float* cov3Ds,
+                           int width, int height, int block_x, int block_y,
+                           const float cam_position[3], const float cam_rotation[9],
+                           float focal_x, float focal_y, float zFar, float zNear,
+                           float* points_xy, float* rgb_depth, float* conic_opacity,
+                           uint64_t* gaussian_keys_unsorted, uint32_t* gaussian_values_unsorted,
+                           int* curr_offset, int64_t key_capacity, int* count_mirror, int* next_offset, void* stream);
+
+/*
  * Host only: polls *count_mirror until it differs from FGS_COUNT_PENDING and stores what it finds
  * in *count (negative: the launch gave up).  FGS_E_TIMEOUT after timeout_seconds without a count.
  */

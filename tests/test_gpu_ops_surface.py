@@ -87,6 +87,36 @@ def test_ops_errors_on_the_gpu():
                              torch.zeros((cam.height, cam.width, 3), device="cuda:0", dtype=torch.uint8))
 
 
+def test_frames_start_from_the_offset_that_the_frame_before_cleared():
+    """Frames of different pair counts in turn, a call of the operator on the rasterizer's offset and a tensor of the caller's
+    between them: every count is the one of a rasterizer that has rendered nothing else, and is in curr_offset."""
+    import flash_gaussian_splatting as fgs
+    sc, scene, cam, rast = _setup(n=5000)
+    _, _, cam2, fresh = _setup(n=5000)
+    cam2.width, cam2.height = cam.width // 2, cam.height // 2
+    bg = torch.zeros(3)
+    expected = []
+    for c in (cam, cam2):
+        _, _, _, once = _setup(n=5000)
+        image = once.forward(scene, c, bg).clone()
+        expected.append((once.num_rendered, image))
+    assert expected[0][0] != expected[1][0]
+    for i, c in enumerate((cam, cam2, cam2, cam, cam, cam2, cam)):
+        if i == 3:              # as the reference's driver does it
+            rast.curr_offset.fill_(0)
+            fgs.ops.preprocess(scene.position, scene.shs, scene.opacity, scene.cov3d, cam.width, cam.height, 16, 16,
+                               cam.position, cam.rotation, cam.focal_x, cam.focal_y, cam.zFar, cam.zNear,
+                               rast.points_xy, rast.rgb_depth, rast.conic_opacity,
+                               rast.gaussian_keys_unsorted, rast.gaussian_values_unsorted, rast.curr_offset)
+            assert int(rast.curr_offset.cpu()[0]) == expected[0][0]
+        if i == 5:
+            rast.curr_offset = torch.full((1,), 99, device="cuda:0", dtype=torch.int32)
+        image = rast.forward(scene, c, bg)
+        count, ref = expected[c is cam2]
+        assert rast.num_rendered == count == int(rast.curr_offset.cpu()[0])
+        assert torch.equal(image, ref)
+
+
 def _write_ply(path, recs):
     props = ["x", "y", "z", "nx", "ny", "nz"] + ["f_dc_%d" % i for i in range(3)] + ["f_rest_%d" % i for i in range(45)] \
         + ["opacity"] + ["scale_%d" % i for i in range(3)] + ["rot_%d" % i for i in range(4)]
