@@ -13,9 +13,9 @@
 //  * The candidate tiles of all Gaussians of a wave with rectangles of at most 64 tiles are laid
 //    end to end and tested one per lane per step, so lanes stay busy whatever the mix of sizes;
 //    larger rectangles are tested by the whole wave, 64 tiles a step, and rectangles of more than
-//    1024 tiles by the whole workgroup, which gets the passing tiles of every column and row as
-//    an interval found by bisection with the reference's own edge predicates: the tiles are
-//    counted from the intervals alone and visited only to write their keys.
+//    1024 tiles by the whole workgroup, which finds the passing tiles of every column and row as an
+//    interval by bisection with the reference's own edge predicates and joins these to one interval
+//    of columns per row: no tile of such a rectangle is visited but to write its key.
 //
 // THIS FILE MUST BE COMPILED WITH -ffp-contract=off.  Every fp32 expression that feeds a key is
 // written in the operand order of the reference and has to be evaluated one IEEE operation at a
@@ -42,7 +42,6 @@ constexpr int kHugeMin = 1024;          // rectangles with more tiles than this 
 // workgroup waits for that count)
 constexpr int kHugeCap = 27;
 constexpr int kSpanWords = kWavesPerBlock * kFlatCap / 4;   // column + row spans of one listed rectangle
-static_assert(kSpanWords / kWave <= kWave, "one lane per group of 64 columns");
 constexpr unsigned kSpinLimit = 1u << 22;   // polls before a wait on the scan over workgroups gives up
 
 struct Camera {
@@ -495,7 +494,7 @@ __global__ __launch_bounds__(kBlock) void preprocess_kernel(
     __shared__ uint32_t s_huge_cnt[kHugeCap][kWavesPerBlock];
     __shared__ int s_huge_spans[kHugeCap];                      // 1: the tiles that pass are found from column and row spans
     __shared__ int s_nhuge;
-    __shared__ int s_centre[2];                                 // column and row of a listed rectangle that hold its centre
+    __shared__ int s_centre;                                    // column of a listed rectangle that holds its centre, or -1
     __shared__ uint32_t s_control;
 
     const int tid = threadIdx.x;
@@ -728,143 +727,126 @@ __global__ __launch_bounds__(kBlock) void preprocess_kernel(
         if (lane == src) { count = total; stash_at = (uint32_t)at; in_stash = keep; }
     }
 
-    // the listed rectangles: wave w counts tiles [w*part, (w+1)*part) of each
+    // the listed rectangles, one after the other, by the whole workgroup
     __syncthreads();
     const int n_huge = min(s_nhuge, kHugeCap);
     uint32_t* const spans = reinterpret_cast<uint32_t*>(&s_owner[0][0]);
-    // Fills spans[0, rw) with the rows that pass the vertical-edge test in each column of the
-    // rectangle and spans[rw, rw + rh) with the columns that pass the horizontal-edge test in
-    // each row.  All threads of the workgroup call it; barriers before and after.
-    auto fill_spans = [&](int e) {
+    // Finds the passing tiles of listed rectangle e as one interval of columns per row and leaves them
+    // in spans[rw, rw + rh) as first | length << 16; returns the tiles of this thread's rows.  A tile
+    // passes if its column's span holds its row, or its row's span holds its column, or it is the tile
+    // of the centre.
+    //  * The spans of the columns are turned into intervals of columns per row by what changes from
+    //    one column to the next: a row that column x holds and column x - 1 does not begins at x,
+    //    one that column x + 1 does not hold ends at x, and a row that begins once is an interval.
+    //    An ellipse of any shape has a handful of such rows per column, where the tiles that it covers
+    //    are thousands.
+    //  * The ellipse is convex, so the interval by columns, the one by the row's own span and the
+    //    centre join up.  Where rounding leaves a gap or a second beginning, the entry is marked
+    //    (s_huge_spans) and tested tile by tile.
+    // All threads of the workgroup call it; barriers before and after.
+    // What bounds it is the workgroup's own time on a rectangle (everything behind it waits for the
+    // count).  With every column going down its span to count the rows whose own span does not hold
+    // it, and the tiles visited 64 columns of a row a step to write their keys, an 8K frame of 110M pairs
+    // and 20 567 such rectangles took 1309 us, now 916 (744 without these rectangles); 2M Gaussians
+    // with needles at 4K 262, now 215 (175 without), at 1080p 170, now 152.  From 513 tiles on instead
+    // of 1025: 939, 215 and 152; from 257 on: 1043, 241 and 151.
+    static_assert(kSpanWords <= 1024, "columns of a listed rectangle in 10 bits; 1 << 20 per row that begins");
+    auto fill_hulls = [&](int e) -> uint32_t {
+        constexpr int kOwn = kSpanWords / kBlock;
         const float gcx = s_huge_f[e][0], gcy = s_huge_f[e][1];
         const float gconx = s_huge_f[e][2], gcony = s_huge_f[e][3], gconz = s_huge_f[e][4];
         const float w = 2.0f * s_huge_f[e][5];
         const int gminx = s_huge_i[e][0], gminy = s_huge_i[e][1], grw = s_huge_i[e][2];
-        const int grh = s_huge_i[e][3] / grw;
+        const int grh = s_huge_i[e][3] / grw, words = grw + grh;
         __syncthreads();
-        for (int i = tid; i < grw + grh; i += kBlock)
-            spans[i] = i < grw ? edge_span(gconz, gcony, gconx, gcx, gcy, gminx + i, cam.bx, gminy, cam.by, grh, w)
-                               : edge_span(gconx, gcony, gconz, gcy, gcx, gminy + i - grw, cam.by, gminx, cam.bx, grw, w);
+        if (tid == 0) s_centre = -1;
+        for (int i = tid; i < words; i += kBlock) {
+            const bool col = i < grw;
+            spans[i] = edge_span(col ? gconz : gconx, gcony, col ? gconx : gconz, col ? gcx : gcy, col ? gcy : gcx,
+                                 col ? gminx + i : gminy + i - grw, col ? cam.bx : cam.by, col ? gminy : gminx,
+                                 col ? cam.by : cam.bx, col ? grh : grw, w);
+        }
+        uint32_t own[kOwn];             // the spans of this thread's rows; their words collect the columns now
+#pragma unroll
+        for (int k = 0; k < kOwn; k++) {
+            const int i = tid + k * kBlock;
+            if (i >= grw && i < words) { own[k] = spans[i]; spans[i] = 0; }
+        }
         __syncthreads();
+        for (int x = tid; x < grw; x += kBlock) {
+            const uint32_t col = spans[x];
+            const int lo = (int)(col & 0x7fffu), hi = (int)((col >> 15) & 0x7fffu);
+            if (col >> 30) s_centre = x;
+            auto changes = [&](int other, uint32_t what) {      // rows of this column that column `other` does not hold
+                int olo = hi + 1, ohi = hi;
+                if (other >= 0 && other < grw) {
+                    const uint32_t o = spans[other];
+                    if ((o & 0x7fffu) <= ((o >> 15) & 0x7fffu)) { olo = (int)(o & 0x7fffu); ohi = (int)((o >> 15) & 0x7fffu); }
+                }
+                for (int ty = lo; ty <= min(hi, olo - 1); ty++) atomicAdd(&spans[grw + ty], what);
+                for (int ty = max(lo, ohi + 1); ty <= hi; ty++) atomicAdd(&spans[grw + ty], what);
+            };
+            if (lo <= hi) {
+                changes(x - 1, (1u << 20) | (uint32_t)x);
+                changes(x + 1, (uint32_t)x << 10);
+            }
+        }
+        __syncthreads();
+        uint32_t tiles = 0;
+        bool whole = true;
+        const int centre = s_centre;
+#pragma unroll
+        for (int k = 0; k < kOwn; k++) {
+            const int i = tid + k * kBlock;
+            if (i >= grw && i < words) {
+                const uint32_t by_columns = spans[i];
+                // (sums of several beginnings carry upwards only: 2 or more stay 2 or more)
+                whole = whole && (by_columns >> 20) <= 1u;
+                int lo = (int)(own[k] & 0x7fffu), hi = (int)((own[k] >> 15) & 0x7fffu);
+                auto join = [&](int l, int h) {
+                    if (lo > hi) { lo = l; hi = h; return; }
+                    whole = whole && l <= hi + 1 && lo <= h + 1;
+                    lo = min(lo, l); hi = max(hi, h);
+                };
+                if (by_columns >> 20) join((int)(by_columns & 1023u), (int)((by_columns >> 10) & 1023u));
+                if ((own[k] >> 30) != 0 && centre >= 0) join(centre, centre);
+                const uint32_t n = lo <= hi ? (uint32_t)(hi - lo + 1) : 0u;
+                spans[i] = (uint32_t)lo | (n << 16);
+                tiles += n;
+            }
+        }
+        if (!whole) s_huge_spans[e] = 0;
+        __syncthreads();
+        return tiles;
     };
-    // Walks the tiles of listed rectangle e that are this wave's share, in row-major order, and
-    // calls visit(tx, ty, passes) once per step of 64 tiles with every lane's own tile.
-    //  * With spans the share is a quarter of the rows.  A step covers 64 columns of one row;
-    //    it is skipped when neither the column spans of those columns reach the row (their
-    //    union is kept per 64 columns) nor the row's own span reaches the columns.
-    //  * Without spans the share is a quarter of the tiles, each tested in full.
-    auto walk_listed = [&](int e, bool from_spans, auto&& visit) {
+    // Tests the tiles of listed rectangle e that are this wave's share, a contiguous quarter, in
+    // row-major order, and calls visit(tx, ty, passes) once per step of 64 tiles with every lane's own tile.
+    auto walk_listed = [&](int e, auto&& visit) {
         const int gminx = s_huge_i[e][0], gminy = s_huge_i[e][1], grw = s_huge_i[e][2], garea = s_huge_i[e][3];
-        if (from_spans) {
-            const int grh = garea / grw;
-            const int chunks = (grw + kWave - 1) / kWave;
-            // lane c keeps the union of the column spans of columns 64c .. 64c + 63 (first row, last row)
-            uint32_t chunk_lo = 0x7fffu, chunk_hi = 0;
-            for (int c = 0; c < chunks; c++) {
-                const int x = c * kWave + lane;
-                const uint32_t col = x < grw ? spans[x] : 1u;
-                uint32_t lo = col & 0x7fffu, hi = (col >> 15) & 0x7fffu;
-                if (lo > hi) { lo = 0x7fffu; hi = 0; }
-#pragma unroll
-                for (int o = 32; o > 0; o >>= 1) {
-                    lo = min(lo, (uint32_t)__shfl_xor((int)lo, o));
-                    hi = max(hi, (uint32_t)__shfl_xor((int)hi, o));
-                }
-                if (lane == c) { chunk_lo = lo; chunk_hi = hi; }
+        const int part = ((garea + kWavesPerBlock - 1) / kWavesPerBlock + kWave - 1) / kWave * kWave;
+        const int j_lo = min(garea, wave * part), j_hi = min(garea, j_lo + part);
+        for (int base = j_lo; base < j_hi; base += kWave) {
+            const int j = base + lane;
+            bool ok = false;
+            int tx = 0, ty = 0;
+            if (j < j_hi) {
+                div_mod(j, grw, ty, tx);
+                ok = tile_hit(gminx + tx, gminy + ty, cam.bx, cam.by, s_huge_f[e][0], s_huge_f[e][1],
+                              s_huge_f[e][2], s_huge_f[e][3], s_huge_f[e][4], s_huge_f[e][5]);
             }
-            const int rows = (grh + kWavesPerBlock - 1) / kWavesPerBlock;
-            const int y_lo = min(grh, wave * rows), y_hi = min(grh, y_lo + rows);
-            for (int ty = y_lo; ty < y_hi; ty++) {
-                const uint32_t row = spans[grw + ty];
-                const uint32_t rlo = row & 0x7fffu, rhi = (row >> 15) & 0x7fffu;
-                // one lane per chunk decides whether the step is needed; the wave walks the needed ones
-                const bool columns_reach = (uint32_t)ty >= chunk_lo && (uint32_t)ty <= chunk_hi;
-                const bool row_reaches = rlo <= rhi && rlo <= (uint32_t)(lane * kWave + kWave - 1) && rhi >= (uint32_t)(lane * kWave);
-                uint64_t needed = ballot(lane < chunks && (columns_reach || row_reaches || (row >> 30) != 0));
-                for (; needed; needed &= needed - 1) {
-                    const int c = __ffsll((long long)needed) - 1;
-                    const int tx = c * kWave + lane;
-                    bool ok = false;
-                    if (tx < grw) {
-                        const uint32_t col = spans[tx];
-                        const bool by_column = (uint32_t)ty >= (col & 0x7fffu) && (uint32_t)ty <= ((col >> 15) & 0x7fffu);
-                        const bool by_row = (uint32_t)tx >= rlo && (uint32_t)tx <= rhi;
-                        ok = by_column || by_row || ((col & row) >> 30) != 0;
-                    }
-                    visit(tx, ty, ok);
-                }
-            }
-        } else {
-            const int part = ((garea + kWavesPerBlock - 1) / kWavesPerBlock + kWave - 1) / kWave * kWave;
-            const int j_lo = min(garea, wave * part), j_hi = min(garea, j_lo + part);
-            for (int base = j_lo; base < j_hi; base += kWave) {
-                const int j = base + lane;
-                bool ok = false;
-                int tx = 0, ty = 0;
-                if (j < j_hi) {
-                    div_mod(j, grw, ty, tx);
-                    ok = tile_hit(gminx + tx, gminy + ty, cam.bx, cam.by, s_huge_f[e][0], s_huge_f[e][1],
-                                  s_huge_f[e][2], s_huge_f[e][3], s_huge_f[e][4], s_huge_f[e][5]);
-                }
-                visit(tx, ty, ok);
-            }
-        }
-    };
-    // How many tiles of listed rectangle e pass, per quarter of its rows (the quarters are the
-    // waves' shares when the keys are written).  From the spans no tile has to be visited: a tile
-    // passes if its row's span holds its column, or its column's span holds its row, or it is
-    // the tile of the centre.  The rows add up their spans; every column goes down its own span
-    // and counts the rows whose span does not hold it already.
-    auto count_from_spans = [&](int e) {
-        const int grw = s_huge_i[e][2];
-        const int grh = s_huge_i[e][3] / grw;
-        const int rows = (grh + kWavesPerBlock - 1) / kWavesPerBlock;
-        auto add = [&](int ty, uint32_t v) {
-            int q = 0;
-#pragma unroll
-            for (int k = 1; k < kWavesPerBlock; k++) q += ty >= k * rows ? 1 : 0;
-            atomicAdd(&s_huge_cnt[e][q], v);
-        };
-        for (int ty = tid; ty < grh; ty += kBlock) {
-            const uint32_t row = spans[grw + ty];
-            const uint32_t rlo = row & 0x7fffu, rhi = (row >> 15) & 0x7fffu;
-            if (rlo <= rhi) add(ty, rhi - rlo + 1u);
-            if (row >> 30) s_centre[1] = ty;
-        }
-        for (int tx = tid; tx < grw; tx += kBlock) {
-            const uint32_t col = spans[tx];
-            const uint32_t clo = col & 0x7fffu, chi = (col >> 15) & 0x7fffu;
-            if (col >> 30) s_centre[0] = tx;
-            for (uint32_t ty = clo; ty <= chi; ty++) {          // an empty span is 1 .. 0
-                const uint32_t row = spans[grw + (int)ty];
-                const uint32_t rlo = row & 0x7fffu, rhi = (row >> 15) & 0x7fffu;
-                if (!(rlo <= rhi && (uint32_t)tx >= rlo && (uint32_t)tx <= rhi)) add((int)ty, 1u);
-            }
-        }
-        __syncthreads();
-        if (tid == 0 && s_centre[0] >= 0 && s_centre[1] >= 0) {
-            // the tile of the centre, unless a span has counted it
-            const int tx = s_centre[0], ty = s_centre[1];
-            const uint32_t col = spans[tx], row = spans[grw + ty];
-            const bool by_column = (uint32_t)ty >= (col & 0x7fffu) && (uint32_t)ty <= ((col >> 15) & 0x7fffu);
-            const bool by_row = (uint32_t)tx >= (row & 0x7fffu) && (uint32_t)tx <= ((row >> 15) & 0x7fffu);
-            if (!by_column && !by_row) {
-                int q = 0;
-                while (ty >= (q + 1) * rows) q++;
-                atomicAdd(&s_huge_cnt[e][q], 1u);
-            }
+            visit(tx, ty, ok);
         }
     };
     for (int e = 0; e < n_huge; e++) {
         if (s_huge_spans[e] != 0) {
-            if (tid < kWavesPerBlock) s_huge_cnt[e][tid] = 0;
-            if (tid == 0) { s_centre[0] = -1; s_centre[1] = -1; }
-            fill_spans(e);
-            count_from_spans(e);
-            continue;
+            const uint32_t sum = wave_inclusive_sum(fill_hulls(e));
+            if (s_huge_spans[e] != 0) {
+                if (lane == kWave - 1) s_huge_cnt[e][wave] = sum;
+                continue;
+            }
         }
         uint32_t total = 0;
-        walk_listed(e, false, [&](int, int, bool ok) { total += (uint32_t)__popcll(ballot(ok)); });
+        walk_listed(e, [&](int, int, bool ok) { total += (uint32_t)__popcll(ballot(ok)); });
         if (lane == 0) s_huge_cnt[e][wave] = total;
     }
     if (n_huge > 0) {
@@ -920,15 +902,45 @@ __global__ __launch_bounds__(kBlock) void preprocess_kernel(
     if (n_huge > 0) {
         if (huge_slot >= 0) s_huge_u[huge_slot][2] = my_slot;
         __syncthreads();
-        for (int e = 0; e < n_huge; e++) {
-            const bool from_spans = s_huge_spans[e] != 0;
-            if (from_spans) fill_spans(e);
-            const int gminx = s_huge_i[e][0], gminy = s_huge_i[e][1];
+        // (downwards: the intervals of the last one counted are still there)
+        for (int e = n_huge - 1; e >= 0; e--) {
+            const bool hulls = s_huge_spans[e] != 0;
+            if (hulls && e != n_huge - 1) fill_hulls(e);
+            const int gminx = s_huge_i[e][0], gminy = s_huge_i[e][1], grw = s_huge_i[e][2];
             const uint32_t gdepth = s_huge_u[e][0], gidx = s_huge_u[e][1];
             uint64_t slot = s_huge_u[e][2];
+            if (hulls) {
+                // 64 rows at a time: 1 << shift lanes per row, as many as a row has tiles on average
+                const int grh = s_huge_i[e][3] / grw;
+                for (int r0 = 0; r0 < grh; r0 += kWave) {
+                    const int rows = min(kWave, grh - r0);
+                    const uint32_t word = lane < rows ? spans[grw + r0 + lane] : 0u;
+                    const uint32_t row_end = wave_inclusive_sum(word >> 16);
+                    const uint32_t tiles = (uint32_t)bcast_i((int)row_end, kWave - 1);
+                    int shift = 6;
+                    while (shift > 2 && tiles <= (uint32_t)rows << (shift - 1)) shift--;
+                    const int step = kWave >> shift;
+                    for (int r = wave * step; r < rows; r += kWavesPerBlock * step) {
+                        const int row = r + (lane >> shift);
+                        const uint32_t hull = (uint32_t)__shfl((int)word, row);
+                        const uint32_t n = hull >> 16;
+                        const uint64_t dst0 = slot + (uint64_t)((uint32_t)__shfl((int)row_end, row) - n);
+                        const uint32_t tile0 = (uint32_t)((gminy + r0 + row) * cam.gx + gminx) + (hull & 0xffffu);
+                        for (uint32_t k = (uint32_t)(lane & ((1 << shift) - 1)); k < n; k += 1u << shift) {
+                            const uint64_t dst = dst0 + k;
+                            if (dst < cap) {
+                                keys[dst] = ((uint64_t)(tile0 + k) << 32) | gdepth;
+                                values[dst] = gidx;
+                            }
+                        }
+                    }
+                    slot += tiles;
+                }
+                continue;
+            }
             for (int w = 0; w < wave; w++) slot += s_huge_cnt[e][w];
             if (s_huge_cnt[e][wave] == 0) continue;
-            walk_listed(e, from_spans, [&](int tx, int ty, bool ok) {
+            walk_listed(e, [&](int tx, int ty, bool ok) {
                 const uint64_t hits = ballot(ok);
                 if (ok) {
                     const uint64_t dst = slot + (uint64_t)popc_below(hits);

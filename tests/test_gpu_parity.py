@@ -1030,6 +1030,53 @@ def test_orbit_config_at_4k_with_the_needles_stored_last(oracle):
         assert ref["pre"]["counts"]["candidates"] > 5 * ref["K"]
 
 
+def _big_rectangles(n, width, height, longest, thinnest, thickest, seed):
+    """n Gaussians of 100 to `longest` pixels' length in any direction, the other two axes `thinnest` to
+    `thickest` times that, in and around the frame."""
+    rng = np.random.default_rng(seed)
+    sc = scenes.config0(n=n)
+    cam = sc.cameras[0]
+    cam.width, cam.height = width, height
+    cam.focal_x = cam.focal_y = 0.6 * max(width, height)
+    sc.position = sc.position.copy()
+    depth = rng.uniform(4.0, 8.0, n)
+    x, y = (rng.uniform(-0.6, 0.6, n) * depth * s / cam.focal_x for s in (width, height))
+    R = np.asarray(cam.rotation, np.float64).reshape(3, 3)
+    sc.position[:] = (np.stack([x, y, depth], 1) @ R.T + np.asarray(cam.position, np.float64)).astype(np.float32)
+    length = 10.0 ** rng.uniform(2.0, np.log10(longest), (n, 1)) * depth[:, None] / cam.focal_x / 3.3
+    scale = length * np.concatenate([np.ones((n, 1)), 10.0 ** rng.uniform(np.log10(thinnest), np.log10(thickest), (n, 2))], 1)
+    sc.cov3d = scenes.cov3d_from_scale_rotation(scale.astype(np.float32), scenes._unit_quats(rng, n))
+    return sc, cam
+
+
+def _rows_with_a_gap(keys, values, gx):
+    """Rows of a Gaussian whose tiles are not one interval of columns (an unsorted list: row-major per Gaussian)."""
+    tile, v = (keys >> np.uint64(32)).astype(np.int64), values.astype(np.int64)
+    together = (v[1:] == v[:-1]) & (tile[1:] // gx == tile[:-1] // gx)
+    return int((together & (tile[1:] != tile[:-1] + 1)).sum())
+
+
+# listed rectangles of 1022 + 2 columns and rows (the most that the intervals have room for) and one more, a landscape, a
+# portrait, wide tiles; and needles so thin that rounding leaves gaps in their rows, which are tested tile by tile
+@pytest.mark.parametrize("width, height, block, longest, thinnest, thickest", [
+    (16352, 32, (16, 16), 1e4, 1e-3, 1), (32, 16352, (16, 16), 1e4, 1e-3, 1), (16368, 32, (16, 16), 1e4, 1e-3, 1), (2111, 1303, (16, 16), 3e3, 1e-2, 1),
+    (1033, 3777, (16, 16), 1e4, 1e-3, 1), (5003, 2801, (32, 16), 1e4, 1e-3, 1), (4176, 2608, (16, 16), 2e4, 1e-7, 1e-5)])
+def test_rectangles_of_thousands_of_tiles(oracle, width, height, block, longest, thinnest, thickest):
+    import gpu_pipeline as gp
+    sc, cam = _big_rectangles(1500 if thickest == 1 else 6000, width, height, longest, thinnest, thickest, seed=width)
+    cap = 1 << 23
+    pre = oracle.preprocess(sc.position, sc.shs, sc.opacity, sc.cov3d, width, height, block[0], block[1],
+                            cam.position, cam.rotation, cam.focal_x, cam.focal_y, cam.zFar, cam.zNear, cap)
+    K = pre["num_rendered"]
+    assert 0 < K < cap and pre["counts"]["candidates"] > 1024 * 100
+    if thickest < 1:
+        assert _rows_with_a_gap(pre["keys"][:K], pre["values"][:K], (width + block[0] - 1) // block[0]) > 0
+    got = gp.preprocess(gp.SceneOnDevice(sc), cam, cap, block)
+    assert got["num_rendered"] == K
+    assert np.array_equal(gp.u64(got["keys"])[:K], pre["keys"][:K])
+    assert np.array_equal(gp.u32(got["values"])[:K], pre["values"][:K])
+
+
 @pytest.fixture(scope="module")
 def config3_scene():
     return scenes.make(3)
