@@ -154,29 +154,16 @@ __global__ __launch_bounds__(1024) void tile_order_kernel(const int2* __restrict
     }
 }
 
-// render.cu:9-31, with the tile index checked against the number of tiles.  A thread looks at
-// kRangesPerThread pairs, 256 apart so that the loads of a workgroup stay contiguous.
+// render.cu:9-31, with the tile index checked against the number of tiles: what the pair at idx, of tile cur (num_tiles:
+// outside the image) behind a pair of tile prev, says about the ranges.
 // Also writes (0, 0) for the tiles without pairs (the reference clears the whole table first,
 // render.cu:557): the pair that opens tile c clears the tiles between its predecessor's tile and
 // c, the first pair those before it and the last pair those behind it.  A run of up to 4 tiles is
-// cleared by the thread that found it, a longer one by its whole wave.
-constexpr int kRangesPerThread = 4;
-
-__global__ __launch_bounds__(256) void tile_ranges_kernel(int L, const uint64_t* __restrict__ keys,
-                                                          int2* __restrict__ ranges, uint32_t num_tiles)
+// cleared by the thread that found it, a longer one by its whole wave.  All lanes of a wave call it.
+__device__ __forceinline__ void mark_ranges(long long idx, bool valid, uint32_t cur, uint32_t prev, int L,
+                                            int2* __restrict__ ranges, uint32_t num_tiles)
 {
-    const long long base = (long long)blockIdx.x * (256 * kRangesPerThread) + threadIdx.x;
     const int lane = threadIdx.x & (kWave - 1);
-    uint32_t cur[kRangesPerThread], prev[kRangesPerThread];
-#pragma unroll
-    for (int k = 0; k < kRangesPerThread; k++) {
-        const long long idx = base + k * 256;
-        cur[k] = 0; prev[k] = 0;
-        if (idx < L) {
-            cur[k] = min((uint32_t)(keys[idx] >> 32), num_tiles);           // num_tiles: outside the image
-            if (idx > 0) prev[k] = min((uint32_t)(keys[idx - 1] >> 32), num_tiles);
-        }
-    }
     auto clear_by_wave = [&](bool mine, uint32_t lo, uint32_t hi) {         // tiles [lo, hi)
         for (uint64_t todo = ballot(mine); todo; todo &= todo - 1) {
             const int src = __ffsll((long long)todo) - 1;
@@ -184,24 +171,87 @@ __global__ __launch_bounds__(256) void tile_ranges_kernel(int L, const uint64_t*
             for (uint32_t t = from + (uint32_t)lane; t < to; t += kWave) ranges[t] = make_int2(0, 0);
         }
     };
+    const bool opens = valid && (idx == 0 || cur != prev);
+    if (opens) {
+        if (idx > 0 && prev < num_tiles) ranges[prev].y = (int)idx;
+        if (cur < num_tiles) ranges[cur].x = (int)idx;
+    }
+    if (valid && idx == L - 1 && cur < num_tiles) ranges[cur].y = L;
+    // empty tiles in front of this pair's tile
+    const uint32_t lo = idx == 0 ? 0u : min(prev + 1u, num_tiles);
+    const bool gap = opens && lo < cur;
+    const bool wide = gap && cur - lo > 4u;
+    if (gap && !wide)
+        for (uint32_t t = lo; t < cur; t++) ranges[t] = make_int2(0, 0);
+    clear_by_wave(wide, lo, cur);
+    clear_by_wave(valid && idx == L - 1 && cur + 1u < num_tiles, cur + 1u, num_tiles);
+}
+
+// A thread looks at kRangesPerThread pairs, 256 apart so that the loads of a workgroup stay contiguous.
+constexpr int kRangesPerThread = 4;
+
+__global__ __launch_bounds__(256) void tile_ranges_kernel(int L, const uint64_t* __restrict__ keys,
+                                                          int2* __restrict__ ranges, uint32_t num_tiles)
+{
+    const long long base = (long long)blockIdx.x * (256 * kRangesPerThread) + threadIdx.x;
+    uint32_t cur[kRangesPerThread], prev[kRangesPerThread];
 #pragma unroll
     for (int k = 0; k < kRangesPerThread; k++) {
         const long long idx = base + k * 256;
-        const bool valid = idx < L;
-        const bool opens = valid && (idx == 0 || cur[k] != prev[k]);
-        if (opens) {
-            if (idx > 0 && prev[k] < num_tiles) ranges[prev[k]].y = (int)idx;
-            if (cur[k] < num_tiles) ranges[cur[k]].x = (int)idx;
+        cur[k] = 0; prev[k] = 0;
+        if (idx < L) {
+            cur[k] = min((uint32_t)(keys[idx] >> 32), num_tiles);
+            if (idx > 0) prev[k] = min((uint32_t)(keys[idx - 1] >> 32), num_tiles);
         }
-        if (valid && idx == L - 1 && cur[k] < num_tiles) ranges[cur[k]].y = L;
-        // empty tiles in front of this pair's tile
-        const uint32_t lo = idx == 0 ? 0u : min(prev[k] + 1u, num_tiles);
-        const bool gap = opens && lo < cur[k];
-        const bool wide = gap && cur[k] - lo > 4u;
-        if (gap && !wide)
-            for (uint32_t t = lo; t < cur[k]; t++) ranges[t] = make_int2(0, 0);
-        clear_by_wave(wide, lo, cur[k]);
-        clear_by_wave(valid && idx == L - 1 && cur[k] + 1u < num_tiles, cur[k] + 1u, num_tiles);
+    }
+#pragma unroll
+    for (int k = 0; k < kRangesPerThread; k++) {
+        const long long idx = base + k * 256;
+        mark_ranges(idx, idx < L, cur[k], prev[k], L, ranges, num_tiles);
+    }
+}
+
+// The same for a long list of pairs, most of which say nothing: a wave takes kRangeRuns runs of 64 keys, looks at the last
+// key of each, and reads only the runs that end in another tile than they begin in (and the first and the last one of the
+// list), kRangesPerThread of them at a time.  Reading every key is bound by the memory, 881 MB for 110M pairs; this reads a
+// line of each run's four and the runs that hold a tile's border: 110M pairs in 129 600 tiles 185 us by the kernel above,
+// 66 by this one, 14.5M pairs there 22.1 and 18.2, 11.6M in 32 400 18.5 and 12.7, 8.0M 13.9 and 10.7, 5.2M in 8160 10.3 and 5.5.
+// (16 runs per wave: 51, 20.4, 12.0, 12.4 and 5.8.  A bisection by each lane where its 64 keys end in another tile: 41, 26.5, 5.6,
+// 7.4 and 4.3, but 19.6 in place of 4.4 where 1.7M pairs lie unevenly: one dependent chain per border.)
+constexpr int kRangeRuns = 8;
+
+__global__ __launch_bounds__(256) void tile_ranges_sampled_kernel(int L, const uint64_t* __restrict__ keys,
+                                                                  int2* __restrict__ ranges, uint32_t num_tiles)
+{
+    const int lane = threadIdx.x & (kWave - 1);
+    const long long base = ((long long)blockIdx.x * (256 / kWave) + threadIdx.x / kWave) * (kRangeRuns * kWave);
+    auto tile_at = [&](long long idx) { return min((uint32_t)(keys[idx] >> 32), num_tiles); };
+    const long long begin = base + lane * kWave, end = min((long long)L, begin + kWave);
+    const bool mine = lane < kRangeRuns && begin < L;
+    uint32_t last = 0, before = 0;
+    if (mine) last = tile_at(end - 1);
+    if (lane == 0 && mine && begin > 0) before = tile_at(begin - 1);
+    const uint32_t left = (uint32_t)__shfl_up((int)last, 1);
+    if (lane > 0) before = left;
+    uint64_t todo = ballot(mine && (last != before || begin == 0 || end == L));
+    while (todo) {
+        long long idx[kRangesPerThread];
+        uint32_t cur[kRangesPerThread], prev[kRangesPerThread];
+        bool valid[kRangesPerThread];
+#pragma unroll
+        for (int k = 0; k < kRangesPerThread; k++) {
+            const int run = todo ? __ffsll((long long)todo) - 1 : 0;
+            idx[k] = base + run * kWave + lane;
+            valid[k] = todo != 0 && idx[k] < L;
+            cur[k] = valid[k] ? tile_at(idx[k]) : 0u;
+            prev[k] = (uint32_t)__shfl((int)before, run);
+            todo &= todo - 1;           // (0 stays 0)
+        }
+#pragma unroll
+        for (int k = 0; k < kRangesPerThread; k++) {
+            const uint32_t left_key = (uint32_t)__shfl_up((int)cur[k], 1);
+            mark_ranges(idx[k], valid[k], cur[k], lane > 0 ? left_key : prev[k], L, ranges, num_tiles);
+        }
     }
 }
 
@@ -1234,6 +1284,11 @@ int check_tile(int block_x, int block_y, int* sx, int* sy, const char* who)
 // finding each other's lines in the L2 counts for more.
 bool is_ranked(int tiles_x, int tiles_y) { return (long long)tiles_x * tiles_y <= kOrderCap; }
 
+// Pairs from which on tile_ranges_sampled_kernel is the faster one, whatever the number of tiles and however unevenly the pairs
+// lie in them (its second trip to memory costs 1.3 us): 1.4M pairs 4.1 us by every key and 5.4 by samples, 1.7M 4.4 and 5.7,
+// 3.3M 6.0 and 5.3, 4.0M 7.2 and 5.8.
+constexpr int kSampledPairs = 3 << 20;
+
 // render.cu:556-563: zero the ranges, then mark where each tile starts and ends
 int ranges_impl(int block_x, int block_y, int num_rendered, int width, int height,
                 const uint64_t* keys_sorted, int* ranges, void* stream, const char* who)
@@ -1252,6 +1307,11 @@ int ranges_impl(int block_x, int block_y, int num_rendered, int width, int heigh
     if (fill_blocks > 1024) fill_blocks = 1024;
     if (num_rendered == 0)
         hipLaunchKernelGGL(fill_i32_kernel, dim3((unsigned)fill_blocks), dim3(256), 0, st, ranges, words, 0);
+    else if (num_rendered >= kSampledPairs)
+        hipLaunchKernelGGL(tile_ranges_sampled_kernel,
+                           dim3((unsigned)(((size_t)num_rendered + 4 * kRangeRuns * kWave - 1) / (4 * kRangeRuns * kWave))),
+                           dim3(256), 0, st, num_rendered, keys_sorted, (int2*)ranges,
+                           (uint32_t)(num_tiles > 0xffffffffu ? 0xffffffffu : num_tiles));
     else
         hipLaunchKernelGGL(tile_ranges_kernel,
                            dim3((unsigned)(((size_t)num_rendered + 256 * kRangesPerThread - 1) / (256 * kRangesPerThread))),

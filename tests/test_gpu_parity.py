@@ -1000,6 +1000,31 @@ def test_ranges_kernel_against_searchsorted():
         assert np.array_equal(rg.cpu().numpy(), want)
 
 
+# around the number of pairs from which on only the runs that hold a tile's border are read (a wave takes 8 runs of 64 keys)
+@pytest.mark.parametrize("n", [(3 << 20) - 1, 3 << 20, (3 << 20) + 1, (3 << 20) + 63, (3 << 20) + 65, (3 << 20) + 513])
+@pytest.mark.parametrize("W, H", [(16, 16), (400, 300), (7680, 4320)])
+def test_ranges_around_the_length_where_keys_are_sampled(n, W, H):
+    import gpu_pipeline as gp
+    import torch
+    from flashgs_amd import cabi
+    rng = np.random.default_rng(n + W)
+    tiles = ((W + 15) // 16) * ((H + 15) // 16)
+    # uneven lists, empty tiles in front, in between and behind, one list of half the pairs, pairs of tiles outside the image
+    tile = (tiles * rng.random(n) ** 3).astype(np.uint64)
+    tile[(tile < tiles // 100) | ((tile > tiles // 3) & (tile < tiles // 2)) | (tile > tiles * 9 // 10)] = tiles // 4
+    tile[: n // 2] = tiles // 5
+    tile[-70:] = tiles + 3
+    tile.sort()
+    keys = (tile << np.uint64(32)) | rng.integers(0, 1 << 32, n).astype(np.uint64)
+    dk = gp.dev(keys.view(np.int64))
+    rg = torch.full((tiles, 2), -9, device=gp.DEV, dtype=torch.int32)
+    cabi.tile_ranges(16, 16, n, W, H, dk.data_ptr(), rg.data_ptr(), 0)
+    torch.cuda.synchronize()
+    lo = np.searchsorted(tile, np.arange(tiles), side="left")
+    hi = np.searchsorted(tile, np.arange(tiles), side="right")
+    assert np.array_equal(rg.cpu().numpy(), np.where((lo == hi)[:, None], 0, np.stack([lo, hi], 1)).astype(np.int32))
+
+
 @pytest.mark.parametrize("config", [1, 2, 4])
 def test_full_size_configs(oracle, config):
     """The 1080p / 1M, the 4K / 3M and (every sixth pose of) the 2M orbit configurations end to
