@@ -307,9 +307,9 @@ __device__ __forceinline__ uint8_t encode_u8(float x)
 //
 // What bounds the launch is the issue of vector instructions: 25 fp32 instructions (5 for the recurrence, 4 alpha T, 4 T -=,
 // 12 for the colour sums) and two exponentials per Gaussian and wave, and 4 more for staging, stop tests and loop.
-// Measured on the 4K frame of 3M: 108 cycles per Gaussian and 16x16 pixels, 98 in the middle of a launch.  Chains of
-// v_fma_f32, v_mul_f32 or v_sub_f32 take 4 cycles an instruction and a v_exp_f32 among them 7 to 8, which would be
-// 130: some of the instructions here issue faster than in those chains.  4K frame of 3M Gaussians 336 -> 280 us, 8K of
+// The 4K frame of 3M takes some 105 cycles per Gaussian and 16x16 pixels.  With two or more waves on a SIMD v_fma_f32, v_mul_f32,
+// v_add_f32 and v_sub_f32 with vector registers as all operands take 2.4 to 2.9 cycles, with a scalar operand 4.3 like
+// comparisons, shifts and conversions, a v_exp_f32 8.5, and nothing issues beside it.  4K frame of 3M Gaussians 336 -> 280 us, 8K of
 // 8M 762 -> 671, 1080p of 1M 147 -> 139, against a version that took the exponents from per-column and
 // per-row tables in LDS (four exponentials, 32 vector instructions).  (Two waves per 16x16 pixels with
 // two pixels per lane and staging shared over barriers: 357 us on the 4K frame.)

@@ -168,11 +168,11 @@ size_t fgs_get_sort_buffer_size(int num_rendered);
  * splats of some pixels and more, and within some 6e-6 of a colour for splats of about a pixel.  Conics may be of any kind;
  * those with a curvature along y beyond -3 (splats that were not widened by 0.3), saddles and non-finite ones take
  * slower paths.
- * A frame of at most 8192 tiles first ranks its tiles by list length into a table the
- * library keeps per (device, stream) (32 KB, allocated on the first such call on that stream),
- * and with 16x16 tiles the rest of a list of more than 768 entries is blended in four runs that each stop on
- * their own transmittance: the colour can differ from the pair-by-pair walk of
- * render.cu:315-408 by what lies behind T < 1e-4, i.e. by less than 1e-4 of a colour.  Calls on
+ * A frame of at most 8192 tiles (unless it is so small that all its workgroups are resident at once) first ranks its
+ * tiles by list length into a table the library keeps per (device, stream) (32 KB, allocated on the first such call
+ * on that stream), and lists that are long for the frame are blended in runs by several waves and folded front to
+ * back.  The run that holds the stop of render.cu:394-408 is walked again pair by pair behind what
+ * precedes it, so the walk ends where the reference's does.  Calls on
  * different streams may overlap in time, and several host threads may call on one stream.  Under
  * stream capture, and where the table cannot be allocated, tiles go unranked: the image is the
  * same, and a captured blend holds no memory of the library's, so its replays may overlap anything
