@@ -13,6 +13,7 @@
 // accumulation), which a caller asks for per call (FGS_BLEND_MATRIX_F16) or per process
 // (fgs_set_colour_sums).
 #include "fgs_internal.h"
+#include "tile_order.h"
 
 #include <algorithm>
 #include <atomic>
@@ -41,8 +42,6 @@ __global__ __launch_bounds__(256) void fill_i32_kernel(int* p, size_t n, int v)
 // (Ranking in the last workgroup of tile_ranges_kernel instead costs more than this launch: every
 // workgroup then has to push its ranges out of its XCD's L2 before it counts itself done.)
 constexpr int kOrderCap = 8192;            // tiles
-constexpr int kOrderBins = 256, kOrderStep = 32;       // bins of so many entries; everything from 8160 up shares the first one
-constexpr int kLeastShared = 128;          // entries of a list that is shared out (see blend_kernel_shared)
 // The ranking is written by one launch and read by the next, so it needs memory of its own: one
 // table per (device, stream), allocated on the first such blend on that stream (blends on
 // different streams may overlap and get a table each).  Blends on one stream follow each other, and
@@ -84,8 +83,8 @@ int tile_order_table(hipStream_t stream, uint32_t** out, std::unique_lock<std::m
     return FGS_OK;
 }
 
-// From which length on a tile's list is shared out (see blend_kernel_shared): three eighths of what a SIMD walks of the
-// whole frame, by the lists of 256 tiles spread over it, and at least kLeastShared; a multiple of kOrderStep.  Lists are cut alike whether
+// From which length on a tile's list is shared out (see blend_kernel_shared): by what a SIMD walks of the
+// whole frame, as the lists of 256 tiles spread over it say.  Lists are cut alike whether
 // the tiles are ranked or not, so the image is the same.  Called by a whole wave.
 __device__ __forceinline__ int least_shared(const int2* __restrict__ ranges, int num_tiles, int squares, int simds)
 {
@@ -98,8 +97,7 @@ __device__ __forceinline__ int least_shared(const int2* __restrict__ ranges, int
     }
     sum = (uint32_t)bcast_i((int)wave_inclusive_sum(sum), kWave - 1);
     const uint64_t each = (uint64_t)sum * (uint32_t)num_tiles / kSamples * (uint32_t)squares / (uint32_t)simds;
-    const uint64_t least = each / 8 * 3 / kOrderStep * kOrderStep;
-    return least < kLeastShared ? kLeastShared : least > 0x40000000u ? 0x40000000 : (int)least;
+    return least_shared_of(each);
 }
 
 __global__ __launch_bounds__(1024) void tile_order_kernel(const int2* __restrict__ ranges, int num_tiles,
@@ -117,7 +115,7 @@ __global__ __launch_bounds__(1024) void tile_order_kernel(const int2* __restrict
         bin[k] = 0; slot[k] = 0;
         if (t < num_tiles) {
             const int2 r = ranges[t];
-            bin[k] = (uint32_t)(kOrderBins - 1 - max(0, min((r.y - r.x) / kOrderStep, kOrderBins - 1)));
+            bin[k] = (uint32_t)order_bin(r.y - r.x);
             slot[k] = atomicAdd(&s_count[bin[k]], 1u);
         }
     }
@@ -148,7 +146,7 @@ __global__ __launch_bounds__(1024) void tile_order_kernel(const int2* __restrict
     if (tid < kWave) {
         const int least = least_shared(ranges, num_tiles, squares, simds);
         if (tid == 0) {
-            tile_order[kOrderCap] = least / kOrderStep < kOrderBins ? s_count[kOrderBins - least / kOrderStep] : 0u;
+            tile_order[kOrderCap] = s_count[first_bin_below(least)];
             tile_order[kOrderCap + 1] = (uint32_t)least;
         }
     }
@@ -999,7 +997,8 @@ void blend_kernel_shared(FGS_BLEND_PARAMS, const uint32_t* __restrict__ tile_ord
     const int team = wave / kSquares, square = wave % kSquares;
     static_assert(kLeastShared >= 2 * kHead, "a rest worth sharing behind the head");
     const int num_tiles = tiles_x * tiles_y, group = (int)blockIdx.x;
-    // Ranked: the tiles with long lists have a workgroup each, tiles_per_group teams of the others have a tile.
+    // Ranked: the tiles with long lists have a workgroup each, tiles_per_group teams of the others have a tile, and nothing
+    // is shared where a team without one has left.
     int rank = team * (int)gridDim.x + group, least, teams = kT;
     bool active = team < tiles_per_group;
     if (tile_order) {
@@ -1040,7 +1039,7 @@ void blend_kernel_shared(FGS_BLEND_PARAMS, const uint32_t* __restrict__ tile_ord
     bool share = false;                                 // some list of the workgroup is long
 #pragma unroll
     for (int t = 0; t < kT; t++) share = share || (t < teams && s_tile[t][3] >= least);
-    share = __builtin_amdgcn_readfirstlane(share);
+    share = teams == kT && __builtin_amdgcn_readfirstlane(share);
 
     const int square_x = square % SX * 16, square_y = square / SX * 16;
     int left = tile_x * SX * 16 + square_x, top = tile_y * SY * 16 + square_y;
@@ -1067,7 +1066,7 @@ void blend_kernel_shared(FGS_BLEND_PARAMS, const uint32_t* __restrict__ tile_ord
     };
     enum { kOwn, kRuns, kAgain };
     int mode = kOwn, v = -1;                            // v: the team whose tile is shared
-    int end = n >= least ? kHead : n;                    // of the walk of entries one after the other
+    int end = share && n >= least ? kHead : n;           // of the walk of entries one after the other
     int from = 0, upto = end, stop_below = kStopBelow;
     int pos = 0, cap = 0, len = 0, left_runs = 0, step = 0;         // runs start at pos and are len long, at most cap; left_runs of a round
     for (;;) {

@@ -386,3 +386,46 @@ def test_lists_shared_by_the_teams_of_a_workgroup(oracle, block, tiles, flags):
     out, _ = gpu_blend(block, W, H, arrays, bg, cabi.BLEND_FP32 if flags == "fp32" else cabi.BLEND_MATRIX_F16)
     err = np.abs(out - ref)
     assert err.max() <= (3e-5 if flags == "fp32" else 2.0 ** -10 * 1.5), "max abs image error %g at %r" % (err.max(), np.unravel_index(err.argmax(), err.shape))
+
+
+@pytest.mark.parametrize("block, W, H, usual", [((32, 32), 640, 512, 22_000), ((32, 32), 512, 512, 27_000),
+                                                ((32, 16), 640, 400, 27_000), ((16, 16), 400, 320, 54_000)])
+def test_lists_of_tens_of_thousands_in_a_frame_of_few_tiles(oracle, block, W, H, usual):
+    """The length from which lists are shared out is at its limit, which the ranking still tells apart: fgs_blend, which ranks the
+    tiles, and fgs_render_f32, which does not rank so few, give the same bits.  Lists in front of, at and
+    behind that limit, most of them of `usual` entries.  Three tiles against the oracle; bound: every weight and T carries a
+    rounding for each entry in front of it, 2^-24 of a colour of at most 1 each."""
+    import gpu_pipeline as gp
+    import torch
+    gx, gy = -(-W // block[0]), -(-H // block[1])
+    tiles = gx * gy
+    rng = np.random.default_rng(tiles)
+    lengths = np.full(tiles, usual)
+    lengths[::7] = np.resize([0, 1, 100, 5000, 8159, 8160, 8161, 9000, 30_000], len(lengths[::7]))
+    K, squares = int(lengths.sum()), block[0] * block[1] // 256
+    assert K * squares / 1024 * 3 / 8 > 8192 and tiles <= 512
+    n = 60_000
+    xy = rng.uniform(0, 1, (n, 2)) * (W, H)
+    co = np.stack([np.full(n, -1e-6), np.zeros(n), np.full(n, -1e-6), np.log2(rng.uniform(0.1, 1.0, n) * 20.0 / usual)], 1)
+    rgbd = np.concatenate([rng.uniform(0, 1, (n, 3)), np.ones((n, 1))], 1)
+    xy, co, rgbd = (np.ascontiguousarray(a, dtype=np.float32) for a in (xy, co, rgbd))
+    ends = np.cumsum(lengths)
+    ranges = np.stack([ends - lengths, ends], 1).astype(np.int32)
+    ranges[lengths == 0] = 0
+    bg = np.array([0.25, 0.5, 0.75], np.float32)
+    # tile t's list: Gaussians t, t + 1, ... in turn
+    tile = np.repeat(np.arange(tiles), lengths)
+    values = ((np.arange(K) - (ends - lengths)[tile] + tile) % n).astype(np.uint32)
+    out, out_u8 = gpu_blend(block, W, H, (xy, rgbd, co, values, ranges), bg)
+    keys = gp.dev((tile.astype(np.uint64) << np.uint64(32)).view(np.int64))
+    found, ref_u8, ref = gp.render(K, W, H, *(gp.dev(a) for a in (xy, rgbd, co)), keys, gp.dev(values.view(np.int32)), bg, block)
+    assert np.array_equal(found.cpu().numpy(), ranges)
+    assert np.array_equal(out, ref.cpu().numpy()) and np.array_equal(out_u8, ref_u8.cpu().numpy())
+    few = np.zeros_like(ranges)
+    some = [1, 7 * 5, 7 * 8]                 # `usual`, 8160 and 30 000 entries
+    few[some] = ranges[some]
+    _, exact, _ = oracle.render(W, H, block[0], block[1], xy, rgbd, co, values, few, bg, want_u8=False)
+    for t in some:
+        y, x = t // gx * block[1], t % gx * block[0]
+        err = np.abs(out - exact)[y:y + block[1], x:x + block[0]]
+        assert lengths[t] >= 8160 and err.max() <= 30_000 * 2.0 ** -24, (t, err.max())
