@@ -109,10 +109,12 @@ class Rasterizer:
         self.SORT_BUFFER_SIZE = ops().get_sort_buffer_size(MAX_NUM_RENDERED)
         self.list_sorting_space = torch.zeros(self.SORT_BUFFER_SIZE, device=dev, dtype=torch.int8)
         self.ranges = torch.zeros((MAX_NUM_TILES, 2), device=dev, dtype=torch.int32)
-        # two words in turn: a frame's preprocess leaves zero in the one that the next frame starts from
-        self._offsets = torch.zeros(2, device=dev, dtype=torch.int32).split(1)
-        self.curr_offset = self._offsets[0]
-        self._cleared = None
+        # Two words in turn: a frame's preprocess leaves zero in the one that the next frame starts from.  That holds while
+        # nobody else has them; see curr_offset.
+        self._offsets = [torch.zeros(1, device=dev, dtype=torch.int32) for _ in range(2)]
+        self._turn = 0              # the word of the last frame
+        self._cleared = False       # the other one is zero
+        self._curr_offset = None    # the caller's word, once there is one
         self.points_xy = torch.zeros((scene.num_vertex, 2), device=dev, dtype=torch.float32)
         self.rgb_depth = torch.zeros((scene.num_vertex, 4), device=dev, dtype=torch.float32)
         self.conic_opacity = torch.zeros((scene.num_vertex, 4), device=dev, dtype=torch.float32)
@@ -123,6 +125,36 @@ class Rasterizer:
         if max_width and max_height:
             self._out = torch.zeros((max_height, max_width, 3), device=dev, dtype=torch.uint8)
         self.num_rendered = 0
+
+    @property
+    def curr_offset(self):
+        """The word on the device that the last frame counted its pairs in (example.py:47-64).  From the first look at it on every
+        frame counts in this one tensor and clears it first, whatever it holds: a caller may keep it and run the
+        operators on it between frames."""
+        if self._curr_offset is None:
+            self._curr_offset = self._offsets[self._turn]
+        return self._curr_offset
+
+    @curr_offset.setter
+    def curr_offset(self, word):
+        self._curr_offset = word
+
+    def _preprocess(self, scene, camera):
+        bx, by = self.tile
+        arguments = (scene.position, scene.shs, scene.opacity, scene.cov3d, camera.width, camera.height, bx, by,
+                     camera.position, camera.rotation, camera.focal_x, camera.focal_y, camera.zFar, camera.zNear,
+                     self.points_xy, self.rgb_depth, self.conic_opacity,
+                     self.gaussian_keys_unsorted, self.gaussian_values_unsorted)
+        cleared, self._cleared = self._cleared, False
+        if self._curr_offset is not None:
+            self._curr_offset.zero_()
+            ops().preprocess_mirrored(*arguments, self._curr_offset, self._count)
+            return
+        if cleared:
+            self._turn ^= 1
+        else:
+            self._offsets[self._turn].zero_()
+        ops().preprocess_chained(*arguments, self._offsets[self._turn], self._count, self._offsets[self._turn ^ 1])
 
     def _image(self, camera, device):
         if self._out is None or self._out.shape[0] != camera.height or self._out.shape[1] != camera.width:
@@ -140,31 +172,19 @@ class Rasterizer:
         if self.num_rendered >= 0 and int(self._count[0]) < 0:
             # the count of the last frame was good when it arrived, and a wait of one workgroup gave up after that
             self.num_rendered = -1
-            o.reset_scan(self.curr_offset)
+            o.reset_scan(self._offsets[0])
             raise ScanGaveUp("a workgroup of the previous frame's preprocess gave up waiting after the pair count "
                              "had been reported; that frame's image is not to be used")
         for attempt in range(2):
-            if self._cleared is not None and any(self.curr_offset is word for word in self._offsets):
-                self.curr_offset = self._cleared
-            else:
-                self.curr_offset.zero_()
-            self._cleared = None
-            other = self._offsets[1] if self.curr_offset is self._offsets[0] else self._offsets[0]
-            o.preprocess_chained(scene.position, scene.shs, scene.opacity, scene.cov3d,
-                                 camera.width, camera.height, bx, by,
-                                 camera.position, camera.rotation,
-                                 camera.focal_x, camera.focal_y, camera.zFar, camera.zNear,
-                                 self.points_xy, self.rgb_depth, self.conic_opacity,
-                                 self.gaussian_keys_unsorted, self.gaussian_values_unsorted, self.curr_offset, self._count,
-                                 other)
+            self._preprocess(scene, camera)
             # the count arrives while the launch is still writing keys; the sort below is enqueued
             # behind it on the same stream
             num_rendered = o.wait_count(self._count, 60.0)
             if num_rendered >= 0:
-                self._cleared = other if scene.num_vertex > 0 else None
+                self._cleared = self._curr_offset is None and scene.num_vertex > 0
                 break
             # a bounded wait of the launch gave up: clear the scan status and launch once more
-            o.reset_scan(self.curr_offset)
+            o.reset_scan(self._offsets[0])
         self.num_rendered = num_rendered
         if num_rendered < 0:
             raise ScanGaveUp("preprocess gave up waiting for its scan over workgroups twice in a row "

@@ -117,6 +117,40 @@ def test_frames_start_from_the_offset_that_the_frame_before_cleared():
         assert torch.equal(image, ref)
 
 
+@pytest.mark.parametrize("looked_at", [None, 0, 1, 2, 3])
+def test_a_caller_may_keep_the_word_of_the_pair_count(looked_at):
+    """The rasterizer's offset taken once, before the first frame or after some, and counted in by the operator between frames:
+    every frame's count and image are those of a rasterizer that has rendered nothing else, and the tensor holds the
+    count of what ran last.  Nobody looks at it: the frames start from the words that the launches before them cleared."""
+    import flash_gaussian_splatting as fgs
+    sc, scene, cam, rast = _setup(n=5000)
+    _, _, cam2, _ = _setup(n=5000)
+    cam2.width, cam2.height = cam.width // 2, cam.height // 2
+    bg = torch.zeros(3)
+    expected = []
+    for c in (cam, cam2):
+        _, _, _, once = _setup(n=5000)
+        image = once.forward(scene, c, bg).clone()
+        expected.append((once.num_rendered, image))
+    off = None
+    for i, c in enumerate((cam, cam2, cam2, cam, cam, cam2, cam, cam2)):
+        if i == looked_at:
+            off = rast.curr_offset
+            assert int(off.cpu()[0]) == rast.num_rendered
+        if off is not None:
+            off.fill_(0)
+            fgs.ops.preprocess(scene.position, scene.shs, scene.opacity, scene.cov3d, cam.width, cam.height, 16, 16,
+                               cam.position, cam.rotation, cam.focal_x, cam.focal_y, cam.zFar, cam.zNear,
+                               rast.points_xy, rast.rgb_depth, rast.conic_opacity,
+                               rast.gaussian_keys_unsorted, rast.gaussian_values_unsorted, off)
+            assert int(off.cpu()[0]) == expected[0][0]
+        image = rast.forward(scene, c, bg)
+        count, ref = expected[c is cam2]
+        assert rast.num_rendered == count and torch.equal(image, ref)
+        assert off is None or (off is rast.curr_offset and int(off.cpu()[0]) == count)
+    assert int(rast.curr_offset.cpu()[0]) == expected[1][0]
+
+
 def _write_ply(path, recs):
     props = ["x", "y", "z", "nx", "ny", "nz"] + ["f_dc_%d" % i for i in range(3)] + ["f_rest_%d" % i for i in range(45)] \
         + ["opacity"] + ["scale_%d" % i for i in range(3)] + ["rot_%d" % i for i in range(4)]
