@@ -586,14 +586,17 @@ __device__ __forceinline__ int walk_chunks(
         const float beyond = __builtin_fmaf(__builtin_fmaf(co.y, co.y, -4.0f * co.x * co.z) * reach, reach, 4.0f * co.z * (kMostExponent - co.w));
         const bool fits = __builtin_fmaxf(__builtin_fmaxf(beyond, co.z), __builtin_fmaxf(-limit - co.z, co.w - kMostExponent)) <= 0.0f &&
                           __builtin_fabsf(c) + __builtin_fabsf(bx) + __builtin_fabsf(by) + __builtin_fabsf(co.x) < 1.0e9f;
+        float over = 0.0f;
         if constexpr (kRun) {
-            // any exponent above kSlightlyAbove
+            // Any exponent above kSlightlyAbove: over the columns, multiplied out by 4 cz < 0.  cz = 0, where over is 0 too unless
+            // cy makes it more, is one; what does not fit is looked at below.
             const float w = kFp32 ? co.w : co.w - kWeightScaleLog2;
-            const float over = __builtin_fmaf(__builtin_fmaf(co.y, co.y, -4.0f * co.x * co.z) * reach, reach, 4.0f * co.z * (kSlightlyAbove - w));
-            above = above || ballot(!(__builtin_fmaxf(over, w - kSlightlyAbove) <= 0.0f)) != 0;
+            over = __builtin_fmaf(__builtin_fmaf(co.y, co.y, -4.0f * co.x * co.z) * reach, reach, 4.0f * co.z * (kSlightlyAbove - w));
+            above = above || ballot(!(__builtin_fmaxf(over, w - kSlightlyAbove) < 0.0f)) != 0;
         }
         if (ballot(!fits) != 0) {
             if constexpr (!kSteep) return base;
+            if constexpr (kRun) above = above || ballot(!(over < 0.0f && co.z < 0.0f)) != 0;     // (NaN too)
             const int walked = walk_plain<kFp32>(xy, co, rgb, cnt, left, top, stop_below, T, sums);
             if (walked < 0) return ~(base + ~walked);
             fetch();

@@ -429,3 +429,39 @@ def test_lists_of_tens_of_thousands_in_a_frame_of_few_tiles(oracle, block, W, H,
         y, x = t // gx * block[1], t % gx * block[0]
         err = np.abs(out - exact)[y:y + block[1], x:x + block[0]]
         assert lengths[t] >= 8160 and err.max() <= 30_000 * 2.0 ** -24, (t, err.max())
+
+
+@pytest.mark.parametrize("kind", ["flat along y", "growing along x and y", "growing along x"])
+@pytest.mark.parametrize("block", BLOCKS)
+def test_stop_in_a_run_that_conics_of_another_kind_undo(oracle, block, kind):
+    """A list that is shared out becomes opaque in a run (T of some 8e-5 everywhere), and behind that two Gaussians of that run,
+    whose exponents grow away from the centre, have weights of some 3.5 and turn the sign of T twice: at the run's end
+    T is above the stop.  The walk ends where the reference's does, and what lies behind, of colour 1e4, reaches nothing.  Bound:
+    relative errors of some 1e-6 of weights and 1e-4 of a T that is a product of 1 - 0.9, on colours of up to 1."""
+    rng = np.random.default_rng(13)
+    n, lists = 700, []
+    for at in (64, 70, 126, 128, 200, 254, 320, 500):
+        xy = rng.uniform(0, 1, (n, 2)) * block
+        co = np.stack([np.full(n, -1e-6), np.zeros(n), np.full(n, -1e-6), np.log2(rng.uniform(0.001, 0.002, n))], 1)
+        rgb = rng.uniform(0, 1, (n, 3))
+        co[10:13, 3] = np.log2(0.874)               # T 2e-3
+        co[at, 3] = np.log2(0.96)
+        rgb[at + 2:] = 1e4
+        turns = slice(at + 2, at + 4)
+        if kind == "flat along y":
+            xy[turns] = 1000.0, 5.0
+            co[turns] = 2.4e-6, 0.0, 0.0, -0.6
+        elif kind == "growing along x and y":
+            xy[turns] = 700.0, 700.0
+            co[turns] = 2.4e-6, 0.0, 2.4e-6, -0.6
+        else:                                       # (the one kind that the multiplied form tells by itself)
+            xy[turns] = 1000.0, 5.0
+            co[turns] = 2.4e-6, 0.0, -1e-6, -0.6
+        lists.append((xy + (0, block[1] * len(lists)), co, rgb))
+    W, H = block[0], block[1] * len(lists)
+    arrays = column_of_tiles(lists, len(lists))
+    bg = np.array([0.25, 0.5, 0.75], np.float32)
+    _, ref, _ = oracle.render(W, H, block[0], block[1], *arrays, bg, want_u8=False)
+    out, _ = gpu_blend(block, W, H, arrays, bg)
+    brightest, err = float(ref.max()), float(np.abs(out - ref).max())
+    assert 0.1 < brightest <= 1.0 and err <= 1e-4
