@@ -322,8 +322,9 @@ constexpr float kMostExponent = 20.0f;      // of a Gaussian that the matrix pro
 // 1e-3 at most (as from tables over the tile).
 constexpr float kSharpest = 64.0f;
 constexpr int kNeverStop = -2147483647 - 1;
-// Exponents up to this one count as none above zero: T that has turned negative stays below kStopBelow (2^0.01 - 1 of 1, at most).
-constexpr float kSlightlyAbove = 0.01f;
+// Exponents up to this one count as none above zero: T of kLeastInFront to 1 stays in there, and once below kStopBelow it stays
+// below it, since a weight turns the sign of T with a factor of at most 2^0.01 - 1 < 0.007.
+constexpr float kSlightlyAbove = 0.01f, kLeastInFront = -0.01f;
 
 // An fp32 number as the sum of three bf16 numbers: eight bits of the significand each.
 // (Each is the upper half of a float; the bits below are left to high_halves to drop.)
@@ -968,7 +969,8 @@ __global__ __launch_bounds__(kWave * SX * SY) __attribute__((amdgpu_waves_per_eu
 // every run, from the products of T.  The run that has it is walked once more by the owner, on top of what was in front of it and with
 // the stop tested behind every pair, so the image ends where the reference's walk ends.  (Weights do not exceed
 // 1, so T only falls and a stop shows at the end of the run that has it; a run with an exponent above zero in it, which can
-// turn the sign of T, is walked that way too.)
+// turn the sign of T, is walked that way too, and so is every run behind such weights while T of some pixel in front of it is
+// above 1 or below kLeastInFront: there a run's own stop is not the tile's, and the tile's need not last to the end of the run.)
 //
 // Against a wave per square that shared (16x16 tiles only) from 768 entries on among the four tiles of a workgroup: 32x16 at 1599x901
 // 237 -> 115 us, 32x32 at 2560x1440 1M 321 -> 277, at 640x512 1M 1873 -> 943; 16x16 1080p 1M 145 -> 126, 700k 104 -> 92, 1365x767 300k
@@ -1091,6 +1093,11 @@ void blend_kernel_shared(FGS_BLEND_PARAMS, const uint32_t* __restrict__ tile_ord
             __syncthreads();
             if (team == v) {
                 float t[4] = {kept[0][3], kept[1][3], kept[2][3], kept[3][3]};
+                bool outside = false;
+#pragma unroll
+                for (int k = 0; k < 4; k++) outside = outside || t[k] < kLeastInFront || t[k] > 1.0f;
+                const bool serial = ballot(outside) != 0;
+                if (serial && lane == 0) s_above[step & 1][0] = 1;
                 int mask = 0;
 #pragma unroll
                 for (int j = 0; j < kT; j++) {

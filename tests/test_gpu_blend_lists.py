@@ -465,3 +465,45 @@ def test_stop_in_a_run_that_conics_of_another_kind_undo(oracle, block, kind):
     out, _ = gpu_blend(block, W, H, arrays, bg)
     brightest, err = float(ref.max()), float(np.abs(out - ref).max())
     assert 0.1 < brightest <= 1.0 and err <= 1e-4
+
+
+@pytest.mark.parametrize("kind", ["above one", "negative"])
+@pytest.mark.parametrize("block", BLOCKS)
+def test_runs_behind_weights_that_turned_the_transmittance(oracle, block, kind):
+    """Weights of 4 at one pixel leave T of that pixel above 1, or far below zero, in front of a later run of the list.
+    Above one: the run is opaque (its own T below 1e-4), the pixel not yet, and what lies behind in the run counts.
+    Negative: the run has the tile's stop, and a weight of 1.005 behind that turns the pixel's T to above 1e-4: the walk ends at the
+    stop.  Bound: relative errors of 1e-4 of T on what colours of up to 1e4 the reference blends, a hundred times less than
+    what they are, and 1e-4."""
+    rng = np.random.default_rng(14)
+    n, lists = 900, []
+    for at in (140, 200, 330, 450, 640):
+        xy = rng.uniform(0, 1, (n, 2)) * block
+        co = np.stack([np.full(n, -1e-6), np.zeros(n), np.full(n, -1e-6), np.log2(rng.uniform(0.0005, 0.001, n))], 1)
+        rgb = rng.uniform(0, 1, (n, 3)) * 0.5
+        pixel = (5.0, 6.0)
+        if kind == "above one":
+            turned = slice(70, 72)                       # T 9
+            co[at:at + 8, 3] = np.log2(0.7)              # 6.6e-5
+            rgb[at + 8:] = 1e4
+        else:
+            co[10:13, 3] = np.log2(0.83)                 # T 5e-3 everywhere
+            turned = slice(70, 77)                       # T -10
+            co[at, 3] = np.log2(0.985)                   # the tile's stop
+            xy[at + 2] = pixel
+            co[at + 2] = -2.0, 0.0, -2.0, 0.0072
+            rgb[at] = 0.0
+            rgb[at + 2:] = 1e4
+        xy[turned] = pixel
+        co[turned] = -2.0, 0.0, -2.0, 2.0
+        rgb[turned] = 0.0
+        lists.append((xy + (0, block[1] * len(lists)), co, rgb))
+    W, H = block[0], block[1] * len(lists)
+    arrays = column_of_tiles(lists, len(lists))
+    bg = np.array([0.25, 0.5, 0.75], np.float32)
+    _, ref, _ = oracle.render(W, H, block[0], block[1], *arrays, bg, want_u8=False)
+    out, _ = gpu_blend(block, W, H, arrays, bg)
+    err, dark = np.abs(out - ref), np.minimum(np.abs(ref), 1.0)
+    assert (np.abs(ref) > 2.0).any() == (kind == "above one")
+    worst = float((err - 0.01 * (np.abs(ref) - dark)).max())
+    assert worst <= 1e-4
