@@ -507,8 +507,14 @@ __global__ __launch_bounds__(kBlock) void preprocess_kernel(
     __syncthreads();
     const uint32_t control = s_control;
     if (control & kControlAborted) {
-        // a scanner on these words gave up (in this launch or an earlier one): touch nothing
-        if (tid == 0) { atomicMin(curr_offset, kIntMin); if (blockIdx.x == 0) report_count(count_mirror, kIntMin); }
+        // a scanner on these words gave up (in this launch or an earlier one): nothing is made
+        if (tid == 0) {
+            atomicMin(curr_offset, kIntMin);
+            if (blockIdx.x == 0) {
+                if (next_offset) *next_offset = 0;
+                report_count(count_mirror, kIntMin);
+            }
+        }
         return;
     }
 
@@ -1154,8 +1160,9 @@ int static_scratch(int device, uint64_t** out)
     return FGS_OK;
 }
 
-__global__ void mirror_count_kernel(const int* curr_offset, int* count_mirror)
+__global__ void mirror_count_kernel(const int* curr_offset, int* count_mirror, int* next_offset)
 {
+    if (next_offset) *next_offset = 0;
     report_count(count_mirror, *curr_offset);
 }
 
@@ -1192,7 +1199,7 @@ int preprocess_impl(bool allocate, const char* who, int P,
     }
     if (P == 0) {
         if (mirror_on_device) {
-            hipLaunchKernelGGL(mirror_count_kernel, dim3(1), dim3(1), 0, (hipStream_t)stream, (const int*)curr_offset, mirror_on_device);
+            hipLaunchKernelGGL(mirror_count_kernel, dim3(1), dim3(1), 0, (hipStream_t)stream, (const int*)curr_offset, mirror_on_device, next_offset);
             return check_hip(hipGetLastError(), "mirror_count_kernel launch");
         }
         return FGS_OK;

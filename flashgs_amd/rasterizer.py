@@ -181,7 +181,7 @@ class Rasterizer:
             # behind it on the same stream
             num_rendered = o.wait_count(self._count, 60.0)
             if num_rendered >= 0:
-                self._cleared = self._curr_offset is None and scene.num_vertex > 0
+                self._cleared = self._curr_offset is None
                 break
             # a bounded wait of the launch gave up: clear the scan status and launch once more
             o.reset_scan(self._offsets[0])

@@ -119,8 +119,7 @@ int fgs_preprocess_mirrored(int P,
 /*
  * No counterpart in the reference.  fgs_preprocess_mirrored that also leaves zero in *next_offset (device memory, another
  * word than *curr_offset): a caller with two words uses them in turn, one frame's launch clearing the start of the
- * next, and needs no launch of its own to clear it.  Only a launch whose count came out at zero or more, with P > 0, has
- * cleared the word for certain.
+ * next, and needs no launch of its own to clear it.  The word is cleared whatever the count comes out at, with P = 0 too.
  */
 int fgs_preprocess_chained(int P,
                            const float* positions, const float* shs, const float* opacities, const float* cov3Ds,

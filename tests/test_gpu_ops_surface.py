@@ -151,6 +151,46 @@ def test_a_caller_may_keep_the_word_of_the_pair_count(looked_at):
     assert int(rast.curr_offset.cpu()[0]) == expected[1][0]
 
 
+def test_the_next_offset_is_cleared_whatever_the_count():
+    """preprocess_chained leaves zero in the other word: with Gaussians, without any, where the scan gives up and where an earlier one
+    on the stream has."""
+    import flash_gaussian_splatting as fgs
+    from flashgs_amd import cabi
+    sc, scene, cam, rast = _setup(n=5000)
+    big = scenes.config0(n=1_200_000)           # more workgroups than the chip holds at once
+    big_scene = Scene(torch.device("cuda:0")).from_arrays(big.position, big.shs, big.opacity, big.cov3d)
+    big_rast = Rasterizer(big_scene, 1 << 22, 1 << 14)
+    none = Scene(torch.device("cuda:0")).from_arrays(sc.position[:0], sc.shs[:0], sc.opacity[:0], sc.cov3d[:0])
+    no_rast = Rasterizer(none, 1 << 10, 1 << 14)
+
+    def count(r, s, start):
+        off, other = (torch.full((1,), v, device="cuda:0", dtype=torch.int32) for v in (start, 77))
+        fgs.ops.preprocess_chained(s.position, s.shs, s.opacity, s.cov3d, cam.width, cam.height, 16, 16,
+                                   cam.position, cam.rotation, cam.focal_x, cam.focal_y, cam.zFar, cam.zNear,
+                                   r.points_xy, r.rgb_depth, r.conic_opacity,
+                                   r.gaussian_keys_unsorted, r.gaussian_values_unsorted, off, r._count, other)
+        n = fgs.ops.wait_count(r._count, 60.0)
+        torch.cuda.synchronize()
+        assert int(other.cpu()[0]) == 0 and int(off.cpu()[0]) == n
+        return n
+
+    rast.forward(scene, cam, torch.zeros(3))
+    assert count(rast, scene, 0) == rast.num_rendered and count(rast, scene, 5) == rast.num_rendered + 5
+    assert count(no_rast, none, 0) == 0 and count(no_rast, none, 41) == 41
+    previous = cabi.set_scan_spin_limit(0)
+    try:
+        assert count(big_rast, big_scene, 0) < 0
+    finally:
+        cabi.set_scan_spin_limit(previous)
+    assert count(rast, scene, 0) < 0             # the scan status is marked
+    fgs.ops.reset_scan(rast.ranges)
+    assert count(rast, scene, 0) == rast.num_rendered
+    image = no_rast.forward(none, cam, torch.zeros(3))
+    for _ in range(3):
+        assert no_rast.num_rendered == 0 and int(image.max()) == 0
+        image = no_rast.forward(none, cam, torch.zeros(3))
+
+
 def _write_ply(path, recs):
     props = ["x", "y", "z", "nx", "ny", "nz"] + ["f_dc_%d" % i for i in range(3)] + ["f_rest_%d" % i for i in range(45)] \
         + ["opacity"] + ["scale_%d" % i for i in range(3)] + ["rot_%d" % i for i in range(4)]
