@@ -1073,6 +1073,7 @@ void blend_kernel_shared(FGS_BLEND_PARAMS, const uint32_t* __restrict__ tile_ord
     int mode = kOwn, v = -1;                            // v: the team whose tile is shared
     int end = share && n >= least ? kHead : n;           // of the walk of entries one after the other
     int from = 0, upto = end, stop_below = kStopBelow;
+    bool turned = false;                                // an exponent above zero in what the wave has walked of its own tile
     int pos = 0, cap = 0, len = 0, left_runs = 0, step = 0;         // runs start at pos and are len long, at most cap; left_runs of a round
     for (;;) {
         bool above = false;
@@ -1093,11 +1094,13 @@ void blend_kernel_shared(FGS_BLEND_PARAMS, const uint32_t* __restrict__ tile_ord
             __syncthreads();
             if (team == v) {
                 float t[4] = {kept[0][3], kept[1][3], kept[2][3], kept[3][3]};
-                bool outside = false;
+                if (turned) {
+                    bool outside = false;
 #pragma unroll
-                for (int k = 0; k < 4; k++) outside = outside || t[k] < kLeastInFront || t[k] > 1.0f;
-                const bool serial = ballot(outside) != 0;
-                if (serial && lane == 0) s_above[step & 1][0] = 1;
+                    for (int k = 0; k < 4; k++) outside = outside || t[k] < kLeastInFront || t[k] > 1.0f;
+                    const bool serial = ballot(outside) != 0;
+                    if (serial && lane == 0) s_above[step & 1][0] = 1;
+                }
                 int mask = 0;
 #pragma unroll
                 for (int j = 0; j < kT; j++) {
@@ -1154,6 +1157,7 @@ void blend_kernel_shared(FGS_BLEND_PARAMS, const uint32_t* __restrict__ tile_ord
             if (mode == kAgain) continue;
         } else {
             // entries one after the other
+            turned = turned || above;
             from += walked < 0 ? ~walked : walked;
             bool stopped = walked < 0;
             const bool bystander = mode == kAgain && team != v;
