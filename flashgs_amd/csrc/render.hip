@@ -969,8 +969,8 @@ __global__ __launch_bounds__(kWave * SX * SY) __attribute__((amdgpu_waves_per_eu
 // every run, from the products of T.  The run that has it is walked once more by the owner, on top of what was in front of it and with
 // the stop tested behind every pair, so the image ends where the reference's walk ends.  (Weights do not exceed
 // 1, so T only falls and a stop shows at the end of the run that has it; a run with an exponent above zero in it, which can
-// turn the sign of T, is walked that way too, and so is every run behind such weights while T of some pixel in front of it is
-// above 1 or below kLeastInFront: there a run's own stop is not the tile's, and the tile's need not last to the end of the run.)
+// turn the sign of T, is walked that way too, and so is a run behind T of some pixel above 1 or below
+// kLeastInFront: there a run's own stop is not the tile's, and the tile's need not last to the end of the run.)
 //
 // Against a wave per square that shared (16x16 tiles only) from 768 entries on among the four tiles of a workgroup: 32x16 at 1599x901
 // 237 -> 115 us, 32x32 at 2560x1440 1M 321 -> 277, at 640x512 1M 1873 -> 943; 16x16 1080p 1M 145 -> 126, 700k 104 -> 92, 1365x767 300k
@@ -996,7 +996,7 @@ void blend_kernel_shared(FGS_BLEND_PARAMS, const uint32_t* __restrict__ tile_ord
     __shared__ __align__(16) float s_stage[kWaves][kStageFloats > kHandOver ? kStageFloats : kHandOver];
     __shared__ int s_walked[kWaves], s_stopped[kWaves], s_above[2][kT];
     __shared__ int s_tile[kT][4];                       // of every team: first pixel, first pair, pairs
-    __shared__ int s_rest[kT];                          // pairs left for all teams
+    __shared__ int s_rest[kT];                          // 1: pairs left for all teams, 3: and T of the first run is outside
 
     const int lane = threadIdx.x & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int team = wave / kSquares, square = wave % kSquares;
@@ -1069,11 +1069,17 @@ void blend_kernel_shared(FGS_BLEND_PARAMS, const uint32_t* __restrict__ tile_ord
 #pragma unroll
         for (int k = 0; k < 4; k++) p[k] = kept[k];
     };
+    // Whether a pixel's T is outside what a run may start from (see above).  It can be only behind entries that were walked
+    // one after the other, and is looked at there: before every fold it was 2 % of the blend of frames of some thousand tiles.
+    auto outside = [&]() {
+        const float most = __builtin_fmaxf(__builtin_fmaxf(T[0], T[1]), __builtin_fmaxf(T[2], T[3]));
+        const float fewest = __builtin_fminf(__builtin_fminf(T[0], T[1]), __builtin_fminf(T[2], T[3]));
+        return ballot(most > 1.0f || fewest < kLeastInFront) != 0;
+    };
     enum { kOwn, kRuns, kAgain };
     int mode = kOwn, v = -1;                            // v: the team whose tile is shared
     int end = share && n >= least ? kHead : n;           // of the walk of entries one after the other
     int from = 0, upto = end, stop_below = kStopBelow;
-    bool turned = false;                                // an exponent above zero in what the wave has walked of its own tile
     int pos = 0, cap = 0, len = 0, left_runs = 0, step = 0;         // runs start at pos and are len long, at most cap; left_runs of a round
     for (;;) {
         bool above = false;
@@ -1094,13 +1100,6 @@ void blend_kernel_shared(FGS_BLEND_PARAMS, const uint32_t* __restrict__ tile_ord
             __syncthreads();
             if (team == v) {
                 float t[4] = {kept[0][3], kept[1][3], kept[2][3], kept[3][3]};
-                if (turned) {
-                    bool outside = false;
-#pragma unroll
-                    for (int k = 0; k < 4; k++) outside = outside || t[k] < kLeastInFront || t[k] > 1.0f;
-                    const bool serial = ballot(outside) != 0;
-                    if (serial && lane == 0) s_above[step & 1][0] = 1;
-                }
                 int mask = 0;
 #pragma unroll
                 for (int j = 0; j < kT; j++) {
@@ -1157,7 +1156,6 @@ void blend_kernel_shared(FGS_BLEND_PARAMS, const uint32_t* __restrict__ tile_ord
             if (mode == kAgain) continue;
         } else {
             // entries one after the other
-            turned = turned || above;
             from += walked < 0 ? ~walked : walked;
             bool stopped = walked < 0;
             const bool bystander = mode == kAgain && team != v;
@@ -1209,7 +1207,10 @@ void blend_kernel_shared(FGS_BLEND_PARAMS, const uint32_t* __restrict__ tile_ord
                 if (mode == kOwn && !share) break;
             }
             if (mode == kOwn) {
-                if (lane == 0 && square == 0) s_rest[team] = !stopped && n >= least;
+                if (!stopped && n >= least) {
+                    const int rest = outside() ? 3 : 1;
+                    if (lane == 0) atomicOr(&s_rest[team], rest);
+                }
                 __syncthreads();
                 int rests = 0;
 #pragma unroll
@@ -1227,6 +1228,8 @@ void blend_kernel_shared(FGS_BLEND_PARAMS, const uint32_t* __restrict__ tile_ord
 #pragma unroll
                     for (int k = 0; k < 4; k++) p[k] += float4_t{before[k][0], before[k][1], before[k][2], 0.0f};
                     keep(p);
+                    const bool serial = outside();
+                    if (serial && lane == 0 && end < n) s_above[step & 1][0] = 1;        // as if the next run had weights above 1
                 }
                 pos = end;
                 left_runs--;
@@ -1235,8 +1238,10 @@ void blend_kernel_shared(FGS_BLEND_PARAMS, const uint32_t* __restrict__ tile_ord
             }
         }
         if (next_tile) {
-            do v++; while (v < kT && __builtin_amdgcn_readfirstlane(s_rest[min(v, kT - 1)]) == 0);
+            int rest = 0;
+            while (++v < kT && (rest = __builtin_amdgcn_readfirstlane(s_rest[v])) == 0) {}
             if (v == kT) break;
+            if ((rest & 2) != 0 && wave == 0 && lane == 0) s_above[step & 1][0] = 1;
             __builtin_amdgcn_s_setprio(3);
             left = __builtin_amdgcn_readfirstlane(s_tile[v][0]) + square_x;
             top = __builtin_amdgcn_readfirstlane(s_tile[v][1]) + square_y;
