@@ -40,9 +40,9 @@ FP32_PEAK_TFLOPS = 157.3         # MI355X fp32 vector, published (packed FMA)
 FLOP_PER_EVAL = 19               # render.cu:40-52: 2 sub, 6 mul + 3 add, 1 mul, 3 FMA, 1 sub
 EXEC_SLOTS_PER_EVAL = 7.3        # non-transcendental VALU instructions the fp32 blend kernel issues per evaluation (SQ counters,
                                  # profiles/frame_cfg2_3M_4K_sq_counters.txt, without the 0.08 matrix instructions): 1.25 for the weight
-                                 # from its recurrence, alpha*T, T -=, 3 colour FMAs, the rest staging, stop tests and loop.  Half a
-                                 # v_exp_f32 beside them is not priced.
-ATTAINED_FMA_LANE_OPS = 38.05e12 # v_fma_f32 lane-operations/s measured on this part without packed math (bench.py --calibrate)
+                                 # from its recurrence, alpha*T, T -=, 3 colour FMAs, the rest staging, stop tests and loop; and half a
+                                 # v_exp_f32 beside them.
+ATTAINED_EVALS = 6.20e12         # evaluations/s of a loop of these instructions, its exponentials apart (bench.py --calibrate)
 CAPACITY = {0: 1 << 20, 1: 1 << 22, 2: 1 << 24, 3: 1 << 25, 4: 1 << 25, 5: 1 << 27, 6: 1 << 25}
 FAST_MODE_DTYPE = "f32 (colour sums: f16 operands on the matrix unit, fp32 products and sums)"
 
@@ -71,7 +71,7 @@ def parse():
     ap.add_argument("--details", default=None, metavar="FILE",
                     help="write the full report of every configuration, of which the printed line holds the main figures, to FILE as JSON")
     ap.add_argument("--calibrate", action="store_true",
-                    help="also measure what this GPU attains on a stream copy, a stream read and fp32 FMA / exp2 issue "
+                    help="also measure what this GPU attains on a stream copy, a stream read and the issue of vector instructions "
                          "(libflashgs_calibrate.so) and report it under \"calibration\"")
     return ap.parse_args()
 
@@ -98,22 +98,21 @@ def calibrate(torch, dev):
 
     copy = call(lib.fgs_cal_copy, C.c_void_p(src.data_ptr()), C.c_void_p(dst.data_ptr()), C.c_size_t(nbytes))
     read = call(lib.fgs_cal_read, C.c_void_p(src.data_ptr()), C.c_void_p(sink.data_ptr()), C.c_size_t(nbytes))
-    fma = call(lib.fgs_cal_alu, C.c_int(0), C.c_void_p(sink.data_ptr()))
-    mix4 = call(lib.fgs_cal_alu, C.c_int(1), C.c_void_p(sink.data_ptr()))
-    mix8 = call(lib.fgs_cal_alu, C.c_int(2), C.c_void_p(sink.data_ptr()))
-    exp = call(lib.fgs_cal_alu, C.c_int(3), C.c_void_p(sink.data_ptr()))
-    mul = call(lib.fgs_cal_alu, C.c_int(4), C.c_void_p(sink.data_ptr()))
-    sub = call(lib.fgs_cal_alu, C.c_int(5), C.c_void_p(sink.data_ptr()))
+    kinds = ("fma", "mul", "add", "sub", "fma_scalar_operand", "mul_scalar_operand", "fma_repeated_operand", "shift", "compare", "exp2")
+    rates = {}
+    for waves in (1, 2, 5, 8):
+        rates["%d_waves_per_simd" % waves] = {
+            k: round(call(lib.fgs_cal_issue, C.c_int(i), C.c_int(waves), C.c_void_p(sink.data_ptr())) / 1e12, 2) for i, k in enumerate(kinds)}
+    entry, apart = (call(lib.fgs_cal_issue, C.c_int(m), C.c_int(5), C.c_void_p(sink.data_ptr())) for m in (10, 11))
     torch.cuda.synchronize()
     return {
         "copy_GBs_read_plus_write": round(copy / 1e9, 1), "read_GBs": round(read / 1e9, 1),
-        "fma_T_lane_ops_per_s": round(fma / 1e12, 2), "fma_TFLOPs": round(2 * fma / 1e12, 2),
-        "mul_T_lane_ops_per_s": round(mul / 1e12, 2), "sub_T_lane_ops_per_s": round(sub / 1e12, 2),
-        "exp2_plus_sub_T_lane_ops_per_s": round(exp / 1e12, 2),
-        "fma_and_exp2_4to1_T_lane_ops_per_s": round(mix4 / 1e12, 2),
-        "fma_and_exp2_8to1_T_lane_ops_per_s": round(mix8 / 1e12, 2),
-        "note": "1 GiB buffers; lane-ops = wave64 instructions x 64; packed fp32 is switched off, so the FMA figure "
-                "is the non-packed issue rate (the published 157.3 TFLOP/s counts packed FMA)",
+        "T_lane_ops_per_s": rates,
+        "blend_entry_T_evaluations_per_s": round(4 * entry / 1e12, 3),
+        "blend_entry_exponentials_apart_T_evaluations_per_s": round(4 * apart / 1e12, 3),
+        "note": "1 GiB buffers; lane-ops = wave64 instructions x 64; packed fp32 is switched off (the published 157.3 TFLOP/s "
+                "counts packed FMA); a blend's list entry is 25 multiplications, subtractions and multiply-adds, two exponentials, "
+                "two comparisons and two shifts for 256 evaluations, with 5 waves per SIMD",
     }
 
 
@@ -353,8 +352,8 @@ def stage_report(fr, stage_ms, K, counts, walked):
         # reference-equivalent work: the 19 flop of render.cu:40-52 per pixel-Gaussian evaluation over the
         # published fp32 vector peak (which counts packed FMA; this library issues none)
         tflops = FLOP_PER_EVAL * evals / (blend_ms * 1e-3) / 1e12
-        # executed work: the kernel's own VALU instructions per evaluation over the v_fma_f32 rate this part attains
-        floor_ms = EXEC_SLOTS_PER_EVAL * evals / ATTAINED_FMA_LANE_OPS * 1e3
+        # executed work: the kernel's own vector instructions at the rate that a loop of the same mix attains on this part
+        floor_ms = evals / ATTAINED_EVALS * 1e3
         roofline.update(achieved=round(tflops, 2), frac=round(tflops / FP32_PEAK_TFLOPS, 4),
                         achieved_is="reference-equivalent flop (19 per evaluation, render.cu:40-52) per second",
                         evaluations=int(evals), flop_per_evaluation=FLOP_PER_EVAL,
