@@ -476,7 +476,7 @@ __global__ __launch_bounds__(kBlock) void preprocess_kernel(
     int num_blocks,                        // workgroups that hold Gaussians; the grid has one more, the scanner's
     unsigned spin_limit,
     int* __restrict__ count_mirror,        // pinned host memory that also receives the pair count, or null
-    int* __restrict__ next_offset)         // a word that is zero when the launch has ended (the start of a later one), or null
+    int* __restrict__ next_offset)         // a word that is zero when the launch has ended, whatever the count (the start of a later one), or null
 {
     __shared__ uint32_t s_wave_total[kWavesPerBlock];
     __shared__ uint32_t s_block_base;

@@ -267,8 +267,8 @@ __device__ __forceinline__ uint8_t encode_u8(float x)
 // the pixel from the Gaussian's centre (render.cu:42-45), is a quadratic along the strip, so its
 // weights alpha_j = 2^q_j follow from the value and the slope at the strip's first pixel:
 //     alpha_{j+1} = alpha_j rho_j,   rho_{j+1} = rho_j E,   rho_0 = 2^(q_1 - q_0),   E = 2^(2 cz),
-// two exponentials and five multiplications for four pixels.  (v_exp_f32 takes the vector unit 7 to 8
-// cycles a wave, a multiplication 4.)
+// two exponentials and five multiplications for four pixels.  (v_exp_f32 takes the vector unit 8.4
+// cycles a wave, a multiplication 2.6.)
 //
 // Values and slopes are a matrix product.  With (X, Y) the strip's first pixel relative to the centre
 // of the square and (ex, ey) the Gaussian's centre relative to it,
@@ -305,9 +305,10 @@ __device__ __forceinline__ uint8_t encode_u8(float x)
 //
 // What bounds the launch is the issue of vector instructions: 25 fp32 instructions (5 for the recurrence, 4 alpha T, 4 T -=,
 // 12 for the colour sums) and two exponentials per Gaussian and wave, and 4 more for staging, stop tests and loop.
-// The 4K frame of 3M takes some 105 cycles per Gaussian and 16x16 pixels.  With two or more waves on a SIMD v_fma_f32, v_mul_f32,
-// v_add_f32 and v_sub_f32 with vector registers as all operands take 2.4 to 2.9 cycles, with a scalar operand 4.3 like
-// comparisons, shifts and conversions, a v_exp_f32 8.5, and nothing issues beside it.  4K frame of 3M Gaussians 336 -> 280 us, 8K of
+// The 4K frame of 3M takes some 107 cycles of its 2.1 GHz per Gaussian and 16x16 pixels: 1.486e9 evaluations in 285 us, where a loop of
+// these instructions attains 6.2e12 a second, 240 us (5.2e12 with the two exponentials side by side; calibrate.hip).  With several waves on a
+// SIMD v_mul_f32, v_add_f32 and v_sub_f32 with vector registers as all operands take 2.6 cycles, v_fma_f32 3.0, with a scalar operand
+// 4.4 like comparisons, shifts and conversions, a v_exp_f32 8.4, and nothing issues beside it.  4K frame of 3M Gaussians 336 -> 280 us, 8K of
 // 8M 762 -> 671, 1080p of 1M 147 -> 139, against a version that took the exponents from per-column and
 // per-row tables in LDS (four exponentials, 32 vector instructions).  (Two waves per 16x16 pixels with
 // two pixels per lane and staging shared over barriers: 357 us on the 4K frame.)
@@ -955,7 +956,7 @@ __global__ __launch_bounds__(kWave * SX * SY) __attribute__((amdgpu_waves_per_eu
 }
 
 // Frames of at most kOrderCap tiles.  Such a frame is about resident at once, and a wave alone on its SIMD issues one
-// instruction in seven cycles, 104 ns per entry, where five waves issue one in 1.5: the launch lasted as long as its
+// instruction in seven cycles, 104 ns per entry, where five waves issue one in three: the launch lasted as long as its
 // longest lists on single waves (32x16 tiles, 1599x901: 60 us of issue, 236 us for 2465 entries).  So the tiles are ranked by list
 // length, the longest start first, and those that are long for this frame (tile_order_kernel) have a workgroup of kT teams, one wave per
 // 16x16 square each, to themselves; all other tiles have a team each, without a word to the others of the workgroup

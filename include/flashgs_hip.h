@@ -167,14 +167,17 @@ size_t fgs_get_sort_buffer_size(int num_rendered);
  * splats of some pixels and more, and within some 6e-6 of a colour for splats of about a pixel.  Conics may be of any kind;
  * those with a curvature along y beyond -3 (splats that were not widened by 0.3), saddles and non-finite ones take
  * slower paths.
- * A frame of at most 8192 tiles (unless it is so small that all its workgroups are resident at once) first ranks its
- * tiles by list length into a table the library keeps per (device, stream) (32 KB, allocated on the first such call
- * on that stream), and lists that are long for the frame are blended in runs by several waves and folded front to
- * back.  The run that holds the stop of render.cu:394-408 is walked again pair by pair behind what
- * precedes it, so the walk ends where the reference's does.  Calls on
+ * A frame of at most 8192 tiles first ranks its tiles by list length into a table the library keeps per
+ * (device, stream) (32 KB, allocated on the first such call on that stream); fgs_render_* leaves the ranking out where
+ * the frame is so small that all its workgroups are resident at once.  Lists that are long for the frame are blended in
+ * runs by several waves and folded front to back.  The run that holds the stop of render.cu:394-408 is walked again
+ * pair by pair behind what precedes it, and so is one with weights above 1 in it or behind a transmittance that
+ * such weights took out of 0 to 1, so the walk ends where the reference's does.  From which length on a list is cut
+ * into runs follows from the lists of the whole frame and from the device's number of compute units: the colours of one tile's
+ * list can differ by the rounding of that sum between two frames, or two devices, that hold it.  Calls on
  * different streams may overlap in time, and several host threads may call on one stream.  Under
  * stream capture, and where the table cannot be allocated, tiles go unranked: the image is the
- * same, and a captured blend holds no memory of the library's, so its replays may overlap anything
+ * same bits, and a captured blend holds no memory of the library's, so its replays may overlap anything
  * that leaves the caller's own buffers alone.
  */
 int fgs_render_16x16(int num_rendered, int width, int height,
@@ -251,9 +254,10 @@ int fgs_blend_ex(int block_x, int block_y, int width, int height,
                  uint8_t* out_color_u8, float* out_color_f32, int flags, void* stream);
 
 /*
- * No counterpart in the reference.  Name of the kernel(s) a blend with these flags launches for this
+ * No counterpart in the reference.  Name of the kernel(s) fgs_blend(_ex) launches with these flags for this
  * tile and frame size outside stream capture (frames of at most 8192 tiles have their tiles ranked
- * first), as a profiler lists them; "" for an unsupported tile size or unknown flags.  Lets a
+ * first, by tile_order_kernel, which fgs_render_* leaves out where all workgroups are resident at once), as a
+ * profiler lists them; "" for an unsupported tile size or unknown flags.  Lets a
  * benchmark attribute its figures to the kernel that ran.
  */
 const char* fgs_blend_kernel_name(int block_x, int block_y, int width, int height, int flags);

@@ -354,7 +354,7 @@ def test_error_against_float64(oracle, block, splats):
 def test_lists_shared_by_the_teams_of_a_workgroup(oracle, block, tiles, flags):
     """Lists around the lengths where they are shared out and where rounds and runs end, odd ones among them, with opaque content
     that ends the walk in the head, in one run or another, on a run's last pair, or never, and with weights above one in
-    some runs; workgroups of 16, 8, 4 and 2 teams.  The walk ends behind the reference's pair, so the bound is the one of a
+    some runs; workgroups of 8, 4 and 2 teams, ranked, and the same bits from fgs_render_f32, which does not rank frames that are resident at once.  The walk ends behind the reference's pair, so the bound is the one of a
     whole walk: rounding of sums of up to 0.5 * 1500 weights of 1.5, some 1e-5, and twice that where weights above one turn T's sign."""
     rng = np.random.default_rng(tiles + block[0] * block[1])
     lengths = [1, 2, 63, 64, 65, 127, 128, 129, 191, 192, 193, 257, 319, 320, 321, 385, 511, 576, 577, 700, 832, 833, 1000, 1089, 1500, 1501]
@@ -386,6 +386,12 @@ def test_lists_shared_by_the_teams_of_a_workgroup(oracle, block, tiles, flags):
     out, _ = gpu_blend(block, W, H, arrays, bg, cabi.BLEND_FP32 if flags == "fp32" else cabi.BLEND_MATRIX_F16)
     err = np.abs(out - ref)
     assert err.max() <= (3e-5 if flags == "fp32" else 2.0 ** -10 * 1.5), "max abs image error %g at %r" % (err.max(), np.unravel_index(err.argmax(), err.shape))
+    import gpu_pipeline as gp
+    xy, rgbd, co, values, ranges = arrays
+    keys = np.repeat(np.arange(tiles, dtype=np.uint64) << np.uint64(32), ranges[:, 1] - ranges[:, 0])
+    found, _, same = gp.render(len(values), W, H, gp.dev(xy), gp.dev(rgbd), gp.dev(co), gp.dev(keys.view(np.int64)), gp.dev(values.view(np.int32)),
+                               bg, block, flags=cabi.BLEND_FP32 if flags == "fp32" else cabi.BLEND_MATRIX_F16)
+    assert np.array_equal(found.cpu().numpy(), ranges) and np.array_equal(same.cpu().numpy(), out)
 
 
 @pytest.mark.parametrize("block, W, H, usual", [((32, 32), 640, 512, 22_000), ((32, 32), 512, 512, 27_000),

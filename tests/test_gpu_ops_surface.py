@@ -89,7 +89,8 @@ def test_ops_errors_on_the_gpu():
 
 def test_frames_start_from_the_offset_that_the_frame_before_cleared():
     """Frames of different pair counts in turn, a call of the operator on the rasterizer's offset and a tensor of the caller's
-    between them: every count is the one of a rasterizer that has rendered nothing else, and is in curr_offset."""
+    between them: every count is the one of a rasterizer that has rendered nothing else, and is in curr_offset.  (Looked at after
+    every frame; frames that nobody looks at are below.)"""
     import flash_gaussian_splatting as fgs
     sc, scene, cam, rast = _setup(n=5000)
     _, _, cam2, fresh = _setup(n=5000)

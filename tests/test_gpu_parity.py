@@ -749,9 +749,9 @@ def test_blend_one_tile_and_four_tiles_per_workgroup_agree(flags, rows):
 
 
 def test_blend_long_lists_shared_between_waves(oracle):
-    """A small frame blends its long lists with four waves: the owner takes the head of the list,
-    the rest is cut into four runs that start from T = 1 and are folded front to back.  Crafted
-    lists around the lengths where that sets in, with odd and even lengths, one that saturates in
+    """A small frame blends its long lists with several teams: one takes the head of the list,
+    the rest is cut into rounds of runs that start from T = 1 and are folded front to back.  Crafted
+    lists of hundreds to thousands of entries, with odd and even lengths, one that saturates in
     its head, one that saturates inside a run and faint ones that never do; blended through
     fgs_blend on ranges made here, against the oracle's blend of the same lists."""
     import gpu_pipeline as gp
