@@ -13,24 +13,26 @@
 //     `offsets_kernel` turns them into the exclusive start of every (block, digit) run, and
 //     `scatter_kernel` ranks its block in LDS (wave64 ballot matching, so equal digits keep
 //     their input order) and writes each run to its start.  A short list takes
-//     count -> scatter.  No workgroup ever waits for another one.
+//     count -> scatter.  No workgroup ever waits for another one.  With one or two passes the pairs leave the
+//     partition as 64-bit words depth << 32 | value, the tile known from the place.
 //  2. Sort every tile's segment by the 32 depth bits without touching memory in between: the
 //     last scatter pass also tabulates where each tile id's segment begins (with more than two
 //     passes `segment_starts_kernel` does, from the sorted keys), then segments are handled by
-//     size class.  Up to 1024 pairs one wave holds the segment in registers as 64-bit
-//     words depth << 32 | value (| position where the values of a segment do not ascend) and runs
+//     size class.  Up to 1024 pairs one wave holds the segment in registers as such
+//     words (depth << 16 | position where the values of a segment do not ascend) and runs
 //     a bitonic network on them (the result is that of a stable sort by depth); lane exchanges inside a row of 16 lanes are
 //     data-parallel-primitive moves.  Up to 4096 (4 waves), 8192 (8) and 16384 pairs (16) every wave
 //     of a workgroup sorts its part like that and the parts are merged, the steps between two waves
-//     through LDS.  Longer segments, and segments whose keys differ above the sorted bit range, go
+//     through LDS.  Longer segments go
 //     through stable 8-bit counting passes with a ping-pong copy in HBM, skipping a pass in which all
 //     pairs share the digit.
 //
-// Bytes moved per pair: 8 (count) + 24 (scatter) per partition pass, 24 for the segment sort:
-// 88 for two partition passes, against 8 + 6 * 24 = 152 for a six-pass LSD sort of 47 bits.
+// Bytes moved per pair with two partition passes of 8-bit digits: 8 (count) + 12 + 9 (scatter) + 1 + 9 + 8, and 8 + 12 for the
+// segment sort: 67 (70 with 9-bit digits), against 8 + 6 * 24 = 152 for a six-pass LSD sort of 47 bits.
 #include "fgs_internal.h"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace fgs {
 namespace {
@@ -66,6 +68,7 @@ struct PassShape {
 using Narrow = PassShape<8, 4, 1024>;
 using Wide = PassShape<9, 4, 1024>;
 constexpr int kNarrowMaxTileBits = 16;
+constexpr int kWordsMaxTileBits = 18;           // two passes of Wide: up to here pairs are carried as words (Form::kWords)
 // The 0.2M pairs of a 720p frame are 49 blocks of 4096, which would leave four CUs in five without one: shorter lists
 // are cut into smaller blocks (0.2M pairs 36.7 us with 2048 a block, 30.6 with 1024; 0.4M 54.5 with 1024,
 // 50 with 1536, 44 with 2048; 1.2M 83 with 4096, 79 with 2048; 1.7M 92.5 and 90; 0.1M on an 8K frame 78 and, with 1024, 64).
@@ -95,8 +98,14 @@ constexpr int kListClasses = 4;
 static_assert(kListClasses * kListShards * 4 <= 512, "the list counters fit in the 512 bytes in front of the lists");
 
 struct Workspace {
-    size_t alt_keys, alt_values, hist, chunk_sums, seg_start, seg_flags, seg_lists, total;
+    size_t alt_keys, alt_values, hist, chunk_sums, seg_start, marks, seg_lists, total;
 };
+
+// Words of the workspace that the launches of one sort hand to each other.
+constexpr int kMarkBeyond = 0;                  // one word per count workgroup of the first pass: some key has bits above the sorted range
+constexpr int kMarkByIndex = kMaxChunks;        // the same for the whole list: the launches behind the first scatter read this one
+constexpr int kMarkLowStart = kMaxChunks + 8;   // first index of every digit of the first of two passes
+constexpr int kMarks = kMarkLowStart + 512;
 
 struct PassGrid {
     int tiles, chunk, chunks;       // workgroups of a count/scatter launch; chunks of `chunk` histogram rows each
@@ -128,8 +137,8 @@ Workspace workspace_for(int n)
     w.hist = w.alt_values + align_up((size_t)n * 4, 256);
     w.chunk_sums = w.hist + hist * 4;
     w.seg_start = align_up(w.chunk_sums + sums * 4, 256);
-    w.seg_flags = w.seg_start + align_up(((size_t)kMaxTableIds + 1) * 4, 256);
-    w.seg_lists = w.seg_flags + kMaxTableIds / 8;
+    w.marks = w.seg_start + align_up(((size_t)kMaxTableIds + 1) * 4, 256);
+    w.seg_lists = align_up(w.marks + kMarks * 4, 256);
     // counters (kListClasses * kListShards words), then per class kListShards lists, each able to
     // hold every segment of its class
     w.total = w.seg_lists + 512 + (size_t)kListShards * (((size_t)n / 512 + 2) + ((size_t)n / 1024 + 2) + ((size_t)n / 4096 + 2) +
@@ -137,41 +146,97 @@ Workspace workspace_for(int n)
     return w;
 }
 
-__device__ __forceinline__ uint32_t digit_of(uint64_t key, int shift, uint32_t mask)
-{
-    return (uint32_t)(key >> shift) & mask;
-}
+// What a partition pass reads and writes.
+enum class Form {
+    kPairs,         // keys and values as the caller has them
+    kWords,         // depth << 32 | value, and of the tile field only the digit that the next pass needs (one or two bytes)
+    kSegments,      // depth << 32 | value: the last pass, the segment a pair stands in is its tile
+};
+
+// The part of the tile field that the second of two passes sorts by.
+template <class Shape>
+using NextDigit = std::conditional_t<(Shape::kBits > 8), uint16_t, uint8_t>;
 
 // ---- partition pass, step 1: hist[block][digit] ---------------------------------------------------
 
-template <class Shape>
-__global__ __launch_bounds__(kSortBlock) void count_kernel(const uint64_t* __restrict__ keys, int n,
+// The kCountItems digits of a thread, from keys (kSortBlock apart) or from the bytes or half words that the pass before left (consecutive
+// ones, loaded together: the bytes behind the last digit are inside the buffer, their counts are not taken).
+template <class Shape, class In>
+struct Digits {
+    static constexpr bool kKeys = sizeof(In) == 8;
+    static constexpr int kItems = Shape::kCountItems;
+    static constexpr int kWords = kKeys ? 2 * kItems : kItems * (int)sizeof(In) / 4;
+    uint32_t w[kWords];
+
+    __device__ __forceinline__ int index(int i, int tid) const { return kKeys ? i * kSortBlock + tid : tid * kItems + i; }
+
+    __device__ __forceinline__ void load(const In* __restrict__ in, int base, int tid, int n)
+    {
+        if constexpr (kKeys) {
+#pragma unroll
+            for (int i = 0; i < kItems; i++) {
+                const int idx = base + i * kSortBlock + tid;
+                const uint64_t k = idx < n ? in[idx] : 0ull;
+                w[2 * i] = (uint32_t)k;
+                w[2 * i + 1] = (uint32_t)(k >> 32);
+            }
+        } else {
+            const int first = base + tid * kItems;
+            constexpr int kVector = kWords < 4 ? kWords : 4;
+            typedef uint32_t Vector __attribute__((ext_vector_type(kVector)));
+            const Vector* const at = (const Vector*)(in + first);
+#pragma unroll
+            for (int v = 0; v < kWords / kVector; v++) {
+                Vector x = 0;
+                if (first + v * (kItems / (kWords / kVector)) < n) x = at[v];
+#pragma unroll
+                for (int j = 0; j < kVector; j++) w[v * kVector + j] = kVector == 1 ? ((const uint32_t*)&x)[0] : x[j];
+            }
+        }
+    }
+    __device__ __forceinline__ uint32_t digit(int i, int shift, uint32_t mask) const
+    {
+        if constexpr (kKeys) return (w[2 * i + 1] >> shift) & mask;
+        constexpr int kPer = 4 / (sizeof(In) < 4 ? (int)sizeof(In) : 4);
+        return (w[i / kPer] >> (i % kPer * (32 / kPer))) & mask;
+    }
+    __device__ __forceinline__ uint32_t field(int i) const { return kKeys ? w[2 * i + 1] : 0u; }
+};
+
+template <class Shape, class In>
+__global__ __launch_bounds__(kSortBlock) void count_kernel(const In* __restrict__ in, int n,
                                                            int shift, int nbits, uint32_t* __restrict__ hist,
-                                                           uint32_t* __restrict__ seg_flags, uint32_t flag_words,
+                                                           uint32_t above, uint32_t* __restrict__ beyond,
                                                            uint32_t* __restrict__ seg_counts)
 {
     constexpr int kB = Shape::kBinsP;
     __shared__ uint32_t h[kB];
+    __shared__ uint32_t s_beyond;
     const int tid = threadIdx.x;
-    if (seg_flags) {        // the last pass also clears what the segment launches append to
+    if (seg_counts) {       // the last pass also clears what the segment launches append to
         const uint32_t gid = blockIdx.x * kSortBlock + tid;
-        for (uint32_t w = gid; w < flag_words; w += gridDim.x * kSortBlock) seg_flags[w] = 0;
         if (gid < (uint32_t)(kListClasses * kListShards)) seg_counts[gid] = 0;
     }
 #pragma unroll
     for (int q = 0; q < Shape::kPerThread; q++) h[q * kSortBlock + tid] = 0;
+    if (tid == 0) s_beyond = 0;
     __syncthreads();
     const uint32_t mask = (1u << nbits) - 1u;
     const int base = blockIdx.x * Shape::kTile;
+    Digits<Shape, In> digits;
+    digits.load(in, base, tid, n);
+    uint32_t seen = 0;
 #pragma unroll
     for (int i = 0; i < Shape::kCountItems; i++) {
-        const int idx = base + i * kSortBlock + tid;
-        if (idx < n) atomicAdd(&h[digit_of(keys[idx], shift, mask)], 1u);
+        if (base + digits.index(i, tid) < n) atomicAdd(&h[digits.digit(i, shift, mask)], 1u);
+        seen |= digits.field(i);
     }
+    if (beyond && (seen & above) != 0) s_beyond = 1;
     __syncthreads();
 #pragma unroll
     for (int q = 0; q < Shape::kPerThread; q++)
         hist[(size_t)blockIdx.x * kB + q * kSortBlock + tid] = h[q * kSortBlock + tid];
+    if (beyond && tid == 0) beyond[blockIdx.x] = s_beyond;
 }
 
 // The same for a list of more than kMostRowWords histogram entries: one workgroup counts a whole chunk of
@@ -180,19 +245,19 @@ __global__ __launch_bounds__(kSortBlock) void count_kernel(const uint64_t* __res
 // back just to add them up).
 constexpr int kCountGroups = 4;
 
-template <class Shape>
+template <class Shape, class In>
 __global__ __launch_bounds__(kCountGroups * kSortBlock) void count_chunk_kernel(
-    const uint64_t* __restrict__ keys, int n, int shift, int nbits, uint32_t* __restrict__ hist,
+    const In* __restrict__ in, int n, int shift, int nbits, uint32_t* __restrict__ hist,
     int tiles, int chunk, uint32_t* __restrict__ chunk_sums,
-    uint32_t* __restrict__ seg_flags, uint32_t flag_words, uint32_t* __restrict__ seg_counts)
+    uint32_t above, uint32_t* __restrict__ beyond, uint32_t* __restrict__ seg_counts)
 {
     constexpr int kB = Shape::kBinsP, kPer = Shape::kPerThread;
     __shared__ uint32_t h[kCountGroups][kB];
+    __shared__ uint32_t s_beyond;
     const int tid = threadIdx.x % kSortBlock, group = threadIdx.x / kSortBlock;
     const int groups = (int)blockDim.x / kSortBlock;
-    if (seg_flags) {        // the last pass also clears what the segment launches append to
+    if (seg_counts) {       // the last pass also clears what the segment launches append to
         const uint32_t gid = blockIdx.x * blockDim.x + threadIdx.x;
-        for (uint32_t w = gid; w < flag_words; w += gridDim.x * blockDim.x) seg_flags[w] = 0;
         if (gid < (uint32_t)(kListClasses * kListShards)) seg_counts[gid] = 0;
     }
     const uint32_t mask = (1u << nbits) - 1u;
@@ -200,20 +265,20 @@ __global__ __launch_bounds__(kCountGroups * kSortBlock) void count_chunk_kernel(
     uint32_t sum[kPer];
 #pragma unroll
     for (int q = 0; q < kPer; q++) { sum[q] = 0; h[group][q * kSortBlock + tid] = 0; }
+    if (threadIdx.x == 0) s_beyond = 0;
     __syncthreads();
+    uint32_t seen = 0;
     for (int first = t0; first < t1; first += groups) {      // the same trips for every group
         const int row = first + group;
         if (row < t1) {
             const int base = row * Shape::kTile;
-            uint64_t k[Shape::kCountItems];
+            Digits<Shape, In> digits;
+            digits.load(in, base, tid, n);
 #pragma unroll
             for (int i = 0; i < Shape::kCountItems; i++) {
-                const int idx = base + i * kSortBlock + tid;
-                k[i] = idx < n ? keys[idx] : 0ull;
+                if (base + digits.index(i, tid) < n) atomicAdd(&h[group][digits.digit(i, shift, mask)], 1u);
+                seen |= digits.field(i);
             }
-#pragma unroll
-            for (int i = 0; i < Shape::kCountItems; i++)
-                if (base + i * kSortBlock + tid < n) atomicAdd(&h[group][digit_of(k[i], shift, mask)], 1u);
         }
         __syncthreads();
         if (row < t1) {
@@ -227,6 +292,7 @@ __global__ __launch_bounds__(kCountGroups * kSortBlock) void count_chunk_kernel(
         }
         __syncthreads();
     }
+    if (beyond && (seen & above) != 0) s_beyond = 1;
 #pragma unroll
     for (int q = 0; q < kPer; q++) h[group][q * kSortBlock + tid] = sum[q];
     __syncthreads();
@@ -238,6 +304,7 @@ __global__ __launch_bounds__(kCountGroups * kSortBlock) void count_chunk_kernel(
             chunk_sums[(size_t)blockIdx.x * kB + q * kSortBlock + tid] = total;
         }
     }
+    if (beyond && threadIdx.x == 0) beyond[blockIdx.x] = s_beyond;
 }
 
 // ---- step 2: exclusive start of every (block, digit) run ----------------------------------------
@@ -250,7 +317,8 @@ constexpr int kOffsetThreads = 1024;
 
 template <class Shape>
 __global__ __launch_bounds__(kOffsetThreads) void offsets_kernel(uint32_t* __restrict__ hist, int tiles, int chunk,
-                                                                 const uint32_t* __restrict__ chunk_sums, int chunks)
+                                                                 const uint32_t* __restrict__ chunk_sums, int chunks,
+                                                                 uint32_t* marks)       // of the first pass, else null
 {
     constexpr int kB = Shape::kBinsP;
     constexpr int kMaxGroups = kOffsetThreads / kB;
@@ -260,6 +328,12 @@ __global__ __launch_bounds__(kOffsetThreads) void offsets_kernel(uint32_t* __res
     const int lane = d & (kWave - 1), wave = d / kWave;
     const int mine = (int)blockIdx.x;
     const int groups = (int)blockDim.x / kB;
+    if (marks && mine == 0) {       // one word out of the count workgroups' words
+        uint32_t seen = 0;
+        for (int c = (int)threadIdx.x; c < chunks; c += (int)blockDim.x) seen |= marks[kMarkBeyond + c];
+        const int any = __syncthreads_or(seen != 0);
+        if (threadIdx.x == 0) marks[kMarkByIndex] = any ? 1u : 0u;
+    }
     uint32_t total = 0, before = 0;
     for (int c0 = group * 16; c0 < chunks; c0 += 16 * groups) {
         uint32_t v[16];
@@ -303,25 +377,40 @@ __global__ __launch_bounds__(kOffsetThreads) void offsets_kernel(uint32_t* __res
 
 // ---- step 3: stable scatter ---------------------------------------------------------------------------
 
-// With kTable (the last pass of at most two) the launch also writes the table of segment starts,
+// With at most two passes the pairs leave the first one as 64-bit words depth << 32 | value beside the one digit that the
+// second pass needs, and the last one as words alone: the segment sort works on such words anyhow and knows the
+// tile from the segment, and it writes the pairs in full.  10 bytes (9 with 8-bit digits) in place of 12 are written, 8 in
+// place of 12 by the last pass, and the second count reads a byte or two per pair in place of its key.  With pairs carried
+// in full, and nine instructions per bit of the ranking in place of four: 8K frame of 110M pairs scatter 541 + 533 -> 519 + 425 us,
+// second count 213 -> 79; 4K / 8M 48 + 46 -> 43 + 40, 14.4 -> 8; 8K / 14.5M 82 + 83 -> 80 + 71, 27 -> 18.
+// A list with a key that has bits above the sorted range carries every pair's index in place of its value (the partition is stable, so
+// equal depths keep their order by it as well), and the segment sort fetches the pairs from the input.
+//
+// The last pass of at most two (Form::kSegments) also writes the table of segment starts,
 // seg_start[v] = first index of the output whose tile field is >= v, v in [0, ids], ids = 2^(bits of
 // the tile field).  The input of that pass is ordered by the low part of the tile field (the bits
 // below this pass's digit), so the first pair with low part >= L lies in exactly one workgroup's
 // block, and that workgroup writes the entries (d, L) of every digit d: the destination of its
 // first pair with digit d and low part >= L, or, if it has none, the end of its run of digit d,
 // which is where the next workgroup's run of d begins.  Every entry has one writer, empty ids
-// included, and no launch has to read the keys again.
-template <class Shape, bool kTable>
+// included, and no launch has to read the keys again.  Where the low parts begin is what the first pass
+// began with, left by its workgroup of block 0.
+template <class Shape, Form kIn, Form kOut>
 __global__ __launch_bounds__(Shape::kThreads) void scatter_kernel(
-    const uint64_t* __restrict__ keys_in, const uint32_t* __restrict__ values_in,
-    uint64_t* __restrict__ keys_out, uint32_t* __restrict__ values_out,
-    int n, int shift, int nbits,
+    const uint64_t* __restrict__ keys_in, const void* __restrict__ values_in,       // the digits of Form::kWords stand where the values do
+    uint64_t* __restrict__ keys_out, void* __restrict__ values_out,
+    int n, int shift, int nbits, int low_bits,   // kSegments: low_bits tile bits below this pass's digit
     const uint32_t* __restrict__ start,          // [blocks][bins] from offsets_kernel, or ...
     int raw_rows,                                // ... if > 0, the raw_rows histogram rows themselves (a short list)
-    int* __restrict__ seg_start)                 // kTable: [2^(shift - 32 + nbits) + 1]
+    uint32_t* marks, const uint32_t* beyond, int beyond_rows,       // beyond_rows > 0: the first pass
+    int* __restrict__ seg_start)                 // kSegments: [2^(low_bits + nbits) + 1]
 {
+    constexpr bool kTable = kOut == Form::kSegments;
     constexpr int kB = Shape::kBinsP, kItems = Shape::kItems, kTile = Shape::kTile, kPer = Shape::kDigits;
     constexpr int kThreads = Shape::kThreads, kWaves = Shape::kWaves;
+    typedef NextDigit<Shape> Next;
+    // what is staged beside a word: the tile field (pairs: all of it, else up to 16 or 18 bits)
+    typedef std::conditional_t<kOut == Form::kPairs || (Shape::kBits > 8), uint32_t, uint16_t> Field;
     // per-wave digit counts, then per-wave digit offsets: at most kTile, so 16 bits do, and with
     // them the workgroup's LDS stays under half of the CU's
     __shared__ __align__(4) uint16_t s_count[kWaves][kB];
@@ -329,8 +418,9 @@ __global__ __launch_bounds__(Shape::kThreads) void scatter_kernel(
     __shared__ uint32_t s_global[kB];                 // destination of ranked slot p with digit d: s_global[d] + p
     constexpr int kScanWaves = kB / kWave;           // waves' worth of digits
     __shared__ uint32_t s_wave_sum[kScanWaves];
-    __shared__ uint64_t s_keys[kTile];
-    __shared__ uint32_t s_values[kTile];
+    __shared__ uint64_t s_words[kTile];
+    __shared__ Field s_field[kTile];
+    __shared__ int s_low_start[kIn == Form::kWords ? kB : 1];
 
     const int tid = threadIdx.x;
     const int lane = tid & (kWave - 1);
@@ -345,29 +435,47 @@ __global__ __launch_bounds__(Shape::kThreads) void scatter_kernel(
     const int tile_base = tile * kTile;
     const int in_tile = min(kTile, n - tile_base);
 
-    // The low parts L whose first pair (the first of the input with low part >= L) lies in this
-    // block: those above the low part of the pair in front of the block, up to that of the
-    // block's last pair; the last block also takes the ones no pair reaches.
-    const int low_bits = shift - 32;
-    const uint32_t low_mask = (1u << low_bits) - 1u;
-    __shared__ int s_own[2];
-    uint64_t edge_key = 0;          // thread 0: the pair in front of the block, thread 1: the block's last pair
-    if (kTable && tid < 2 && (tid == 1 || tile > 0)) edge_key = keys_in[tid == 0 ? tile_base - 1 : tile_base + in_tile - 1];
-
     // wave w owns slots [w*64*kItems, (w+1)*64*kItems) of the block, item-major; everything is
     // requested before the first use so the latencies overlap
-    uint64_t key[kItems];
-    uint32_t val[kItems];
+    uint64_t word[kItems];          // depth << 32 | value
+    uint32_t field[kItems];         // (kWords: this pass's digit)
     uint32_t slot[kItems];
+    if constexpr (kIn == Form::kWords) {
 #pragma unroll
-    for (int i = 0; i < kItems; i++) {
-        const int off = wave * (kWave * kItems) + i * kWave + lane;
-        key[i] = off < in_tile ? keys_in[tile_base + off] : ~0ull;
-    }
+        for (int i = 0; i < kItems; i++) {
+            const int off = wave * (kWave * kItems) + i * kWave + lane;
+            word[i] = off < in_tile ? keys_in[tile_base + off] : ~0ull;
+        }
 #pragma unroll
-    for (int i = 0; i < kItems; i++) {
-        const int off = wave * (kWave * kItems) + i * kWave + lane;
-        val[i] = off < in_tile ? values_in[tile_base + off] : 0u;
+        for (int i = 0; i < kItems; i++) {
+            const int off = wave * (kWave * kItems) + i * kWave + lane;
+            field[i] = off < in_tile ? (uint32_t)((const Next*)values_in)[tile_base + off] : ~0u;
+        }
+    } else {
+        uint32_t val[kItems];
+#pragma unroll
+        for (int i = 0; i < kItems; i++) {
+            const int off = wave * (kWave * kItems) + i * kWave + lane;
+            word[i] = off < in_tile ? keys_in[tile_base + off] : ~0ull;
+        }
+#pragma unroll
+        for (int i = 0; i < kItems; i++) {
+            const int off = wave * (kWave * kItems) + i * kWave + lane;
+            val[i] = off < in_tile ? ((const uint32_t*)values_in)[tile_base + off] : 0u;
+        }
+        bool by_index = false;
+        if (beyond_rows > 0) {
+            uint32_t seen = 0;
+            for (int r = lane; r < beyond_rows; r += kWave) seen |= beyond[r];
+            by_index = ballot(seen != 0) != 0;
+            if (blockIdx.x == 0 && tid == 0) marks[kMarkByIndex] = by_index ? 1u : 0u;
+        }
+#pragma unroll
+        for (int i = 0; i < kItems; i++) {
+            const int off = wave * (kWave * kItems) + i * kWave + lane;
+            field[i] = (uint32_t)(word[i] >> 32);
+            word[i] = (word[i] << 32) | (by_index ? (uint32_t)(tile_base + off) : val[i]);
+        }
     }
     // A thread stands for the digits tid, tid + kThreads, ...; with more threads than digits the first kB do.
     const bool has_digits = tid < kB;
@@ -395,8 +503,8 @@ __global__ __launch_bounds__(Shape::kThreads) void scatter_kernel(
             }
         }
         if constexpr (Shape::kGroups > 1) {
-            uint32_t* const s_part = (uint32_t*)s_keys;
-            static_assert(sizeof(uint32_t) * 2 * Shape::kGroups * kB <= sizeof(uint64_t) * kTile, "the partial sums fit in the space of the keys");
+            uint32_t* const s_part = (uint32_t*)s_words;
+            static_assert(sizeof(uint32_t) * 2 * Shape::kGroups * kB <= sizeof(uint64_t) * kTile, "the partial sums fit in the space of the words");
             s_part[2 * tid] = total[0];
             s_part[2 * tid + 1] = before[0];
             __syncthreads();
@@ -433,34 +541,57 @@ __global__ __launch_bounds__(Shape::kThreads) void scatter_kernel(
         for (int w = 0; w < kWaves * kB / 2; w += kThreads)
             if (w + tid < kWaves * kB / 2) words[w + tid] = 0;
     }
-    if (kTable && tid < 2) {
-        const int low = (int)((uint32_t)(edge_key >> 32) & low_mask);
-        s_own[tid] = tid == 0 ? (tile > 0 ? low + 1 : 0) : (tile == (int)gridDim.x - 1 ? (int)low_mask : low);
+    if (kOut == Form::kWords && tile == 0 && has_digits) {
+#pragma unroll
+        for (int q = 0; q < kPer; q++) marks[kMarkLowStart + q * kThreads + tid] = my_start[q];
+    }
+    if (kIn == Form::kWords) {
+        for (int l = tid; l < kB; l += kThreads) s_low_start[l] = (int)marks[kMarkLowStart + l];
     }
     __syncthreads();
+    // The low parts L whose first pair (the first of the input with low part >= L) lies in this
+    // block: those above the low part of the pair in front of the block, up to that of the
+    // block's last pair; the last block also takes the ones no pair reaches.
+    // (a pair's low part: the last one that begins at its index or in front of it)
+    auto low_part = [&](int index) {
+        int low = 0;
+#pragma unroll
+        for (int step = kB / 2; step > 0; step >>= 1)
+            if (s_low_start[low + step] <= index) low += step;
+        return low;
+    };
+    int own_lo = 0, own_hi = -1;
+    if constexpr (kIn == Form::kWords) {
+        own_lo = tile > 0 ? low_part(tile_base - 1) + 1 : 0;
+        own_hi = tile == (int)gridDim.x - 1 ? kB - 1 : low_part(tile_base + in_tile - 1);
+    } else if (kTable) {
+        own_hi = tile == 0 ? 0 : -1;
+    }
 
-    // rank inside the wave: lanes with equal digits find each other with one ballot per digit bit
+    // rank inside the wave: lanes with equal digits find each other with one ballot per digit bit.  The pass issues instructions
+    // 77 % of its time on long lists, most of them here: a bit is taken as 0 or all ones, so that four instructions a bit do (the
+    // field, the comparison, and the peers of either half as one three-operand function), and every lane reads its
+    // digit's counter itself in place of a move from the lane that will update it.
 #pragma unroll
     for (int i = 0; i < kItems; i++) {
         const int off = wave * (kWave * kItems) + i * kWave + lane;
         const bool valid = off < in_tile;
-        const uint32_t d = digit_of(key[i], shift, mask);
-        uint64_t peers = ballot(valid);
+        const uint32_t d = (field[i] >> shift) & mask;
+        const uint64_t all = ballot(valid);
+        uint32_t peers_lo = (uint32_t)all, peers_hi = (uint32_t)(all >> 32);
 #pragma unroll
         for (int b = 0; b < Shape::kBits; b++) {
-            const bool bit = (d >> b) & 1u;
-            const uint64_t with_bit = ballot(bit);
-            peers &= bit ? with_bit : ~with_bit;
+            uint32_t bit = (uint32_t)__builtin_amdgcn_sbfe((int)d, b, 1);
+            asm("" : "+v"(bit));                                                            // one instruction, or every use makes a field of its own
+            const uint64_t with_bit = ballot(bit != 0);
+            peers_lo = __builtin_amdgcn_bitop3_b32(peers_lo, (uint32_t)with_bit, bit, 0x90);          // peers & ~(with_bit ^ bit)
+            peers_hi = __builtin_amdgcn_bitop3_b32(peers_hi, (uint32_t)(with_bit >> 32), bit, 0x90);
         }
-        const int below = popc_below(peers);
-        uint32_t before = 0;
-        if (valid && below == 0) {      // lowest lane of each group updates the wave's counter
-            before = s_count[wave][d];
-            s_count[wave][d] = (uint16_t)(before + (uint32_t)__popcll(peers));
-        }
-        const int leader = valid ? __ffsll((long long)peers) - 1 : lane;
-        before = (uint32_t)__shfl((int)before, leader);
-        slot[i] = before + (uint32_t)below;
+        const uint32_t below = __builtin_amdgcn_mbcnt_hi(peers_hi, __builtin_amdgcn_mbcnt_lo(peers_lo, 0u));
+        const uint32_t before = s_count[wave][d];
+        if (valid && below == 0)        // the lowest lane of each group updates the wave's counter
+            s_count[wave][d] = (uint16_t)(before + (uint32_t)__popc(peers_lo) + (uint32_t)__popc(peers_hi));
+        slot[i] = before + below;
         __builtin_amdgcn_wave_barrier();
     }
     __syncthreads();
@@ -503,51 +634,59 @@ __global__ __launch_bounds__(Shape::kThreads) void scatter_kernel(
     for (int i = 0; i < kItems; i++) {
         const int off = wave * (kWave * kItems) + i * kWave + lane;
         if (off < in_tile) {
-            const uint32_t dg = digit_of(key[i], shift, mask);
+            const uint32_t dg = (field[i] >> shift) & mask;
             const uint32_t p = (uint32_t)s_bin_start[dg] + s_count[wave][dg] + slot[i];
-            s_keys[p] = key[i];
-            s_values[p] = val[i];
+            s_words[p] = word[i];
+            // the whole tile field again where the table needs it
+            if (kIn == Form::kWords && own_lo <= own_hi) field[i] = (dg << low_bits) | (uint32_t)low_part(tile_base + off);
+            s_field[p] = (Field)field[i];
         }
     }
     __syncthreads();
-
-    const int own_lo = kTable ? s_own[0] : 0, own_hi = kTable ? s_own[1] : -1;
+    const bool whole_fields = kIn != Form::kWords || own_lo <= own_hi;
+    const int field_shift = kIn == Form::kWords && whole_fields ? low_bits : shift;
 
     // write out: neighbouring threads hold neighbouring ranked slots.  All LDS reads first (a slot
     // past the end reads the last pair and stores nothing), so their latencies overlap.
     {
-        uint64_t out_key[kItems];
-        uint32_t out_value[kItems], out_at[kItems];
+        uint64_t out_word[kItems];
+        uint32_t out_field[kItems], out_at[kItems];
 #pragma unroll
         for (int i = 0; i < kItems; i++) {
             const int p = min(i * kThreads + tid, in_tile - 1);
-            out_key[i] = s_keys[p];
-            out_value[i] = s_values[p];
+            out_word[i] = s_words[p];
+            out_field[i] = s_field[p];
         }
 #pragma unroll
         for (int i = 0; i < kItems; i++)
-            out_at[i] = s_global[digit_of(out_key[i], shift, mask)] + (uint32_t)(i * kThreads + tid);
+            out_at[i] = s_global[(out_field[i] >> field_shift) & mask] + (uint32_t)(i * kThreads + tid);
 #pragma unroll
         for (int i = 0; i < kItems; i++) {
             if (i * kThreads + tid < in_tile) {
-                keys_out[out_at[i]] = out_key[i];
-                values_out[out_at[i]] = out_value[i];
+                if constexpr (kOut == Form::kPairs) {
+                    keys_out[out_at[i]] = ((uint64_t)out_field[i] << 32) | (out_word[i] >> 32);
+                    ((uint32_t*)values_out)[out_at[i]] = (uint32_t)out_word[i];
+                } else {
+                    keys_out[out_at[i]] = out_word[i];
+                    if (kOut == Form::kWords) ((Next*)values_out)[out_at[i]] = (Next)(out_field[i] >> Shape::kBits);
+                }
             }
         }
     }
     if (kTable) {
         if (own_lo <= own_hi) {
+            const uint32_t low_mask = (1u << low_bits) - 1u;
             // the first pair of digit d with a low part >= L, for every owned L up to its own
             // (a loop of its own: in the one above the LDS reads of all slots are in flight together)
 #pragma unroll 4
             for (int i = 0; i < kItems; i++) {
                 const int p = i * kThreads + tid;
                 if (p >= in_tile) break;
-                const uint32_t field = (uint32_t)(s_keys[p] >> 32);
-                const uint32_t d = (field >> low_bits) & mask;
-                const int low = (int)(field & low_mask);
+                const uint32_t f = s_field[p];
+                const uint32_t d = (f >> low_bits) & mask;
+                const int low = (int)(f & low_mask);
                 int prev = own_lo - 1;
-                if (p > (int)s_bin_start[d]) prev = (int)((uint32_t)(s_keys[p - 1] >> 32) & low_mask);
+                if (p > (int)s_bin_start[d]) prev = (int)(s_field[p - 1] & low_mask);
                 for (int l = max(prev + 1, own_lo); l <= low; l++)
                     seg_start[(d << low_bits) | (uint32_t)l] = (int)(s_global[d] + (uint32_t)p);
             }
@@ -557,7 +696,7 @@ __global__ __launch_bounds__(Shape::kThreads) void scatter_kernel(
                 const uint32_t d = (uint32_t)(q * kThreads + tid);
                 if (d > mask) continue;         // (d is below kB then, a digit of this thread)
                 int last = own_lo - 1;
-                if (total[q]) last = (int)((uint32_t)(s_keys[(uint32_t)s_bin_start[d] + total[q] - 1u] >> 32) & low_mask);
+                if (total[q]) last = (int)(s_field[(uint32_t)s_bin_start[d] + total[q] - 1u] & low_mask);
                 const int end = (int)(my_start[q] + total[q]);
                 for (int l = max(last + 1, own_lo); l <= own_hi; l++) seg_start[(d << low_bits) | (uint32_t)l] = end;
             }
@@ -572,7 +711,6 @@ __global__ __launch_bounds__(Shape::kThreads) void scatter_kernel(
 constexpr int kCapTiny = 512, kCapSmall = 1024, kCapMedium = 4096, kCapLarge = 8192;
 constexpr int kMergedLargeMax = 1 << 24;     // up to this many pairs the last launch also takes the class of 4097 .. 8192 pairs
 constexpr int kMergedTailMax = 1 << 19;      // up to this many pairs the last launch also takes the classes of 1025 .. 8192 pairs
-constexpr uint32_t kOneLaunchIds = 262144;   // up to this many tile ids one launch sorts every segment of up to kCapSmall pairs
 
 // First index in [0, n) whose tile field is >= v (n if none), found by the whole wave probing 64
 // evenly spaced positions per step.  `keys` is ordered by tile field.  All lanes return the same.
@@ -599,16 +737,14 @@ __device__ __forceinline__ int wave_lower_bound(const uint64_t* __restrict__ key
 // seg_start[v] = first index whose tile field is >= v, for v in [0, ids]; seg_start[ids] = n.
 // A thread looks at kStartsPerThread pairs, 256 apart so that the loads of a workgroup stay
 // contiguous: where the tile field changes, it fills the entries of the ids in between (empty ids
-// get the same start as the next non-empty one).  Also clears the flag words and list counters.
+// get the same start as the next non-empty one).  Also clears the list counters.
 constexpr int kStartsPerThread = 8;
 
 __global__ __launch_bounds__(256) void segment_starts_kernel(const uint64_t* __restrict__ keys, int n, uint32_t tile_mask,
                                                              uint32_t ids, int* __restrict__ seg_start,
-                                                             uint32_t* __restrict__ seg_flags, uint32_t flag_words,
                                                              uint32_t* __restrict__ seg_counts)
 {
     const uint32_t gid = blockIdx.x * blockDim.x + threadIdx.x;
-    for (uint32_t w = gid; w < flag_words; w += gridDim.x * blockDim.x) seg_flags[w] = 0;
     if (gid < (uint32_t)(kListClasses * kListShards)) seg_counts[gid] = 0;
     const long long base = (long long)blockIdx.x * (256 * kStartsPerThread) + threadIdx.x;
     uint32_t cur[kStartsPerThread], before[kStartsPerThread];
@@ -647,14 +783,15 @@ __global__ __launch_bounds__(256) void segment_starts_kernel(const uint64_t* __r
     }
 }
 
-// One stable counting pass of a segment over bits shift..shift+7 of the sort word, by the kWaves
+// One stable counting pass of a segment over bits shift..shift+7 of its keys or words, by the kWaves
 // waves of one workgroup.  Wave w owns the contiguous part [w*per, (w+1)*per) of the segment.
 // Returns false (and moves nothing) when every pair has the same digit.  All threads of the
-// workgroup must call it.  KeyT is uint32_t for depth words in LDS, uint64_t for whole keys in HBM.
-template <int kWaves, typename KeyT>
-__device__ __forceinline__ bool counting_pass(const KeyT* src_k, const uint32_t* src_v, KeyT* dst_k, uint32_t* dst_v,
+// workgroup must call it.  src_v null: words, without values beside them.
+template <int kWaves>
+__device__ __forceinline__ bool counting_pass(const uint64_t* src_k, const uint32_t* src_v, uint64_t* dst_k, uint32_t* dst_v,
                                               int n, int shift, uint32_t (*cnt)[kBins], uint32_t* wave_sum, int* flag)
 {
+    static_assert(kWaves > 1 && kWaves * kWave >= kBins, "one thread per digit");
     int tid = threadIdx.x;
     asm volatile("" : "+v"(tid));
     const int lane = tid & (kWave - 1);
@@ -663,58 +800,41 @@ __device__ __forceinline__ bool counting_pass(const KeyT* src_k, const uint32_t*
     const int w_lo = min(n, wave * per), w_hi = min(n, w_lo + per);
 
     for (int d = lane; d < kBins; d += kWave) cnt[wave][d] = 0;
-    if (kWaves > 1) { if (tid == 0) *flag = 0; __syncthreads(); } else __builtin_amdgcn_wave_barrier();
+    if (tid == 0) *flag = 0;
+    __syncthreads();
     for (int i = w_lo + lane; i < w_hi; i += kWave)
         atomicAdd(&cnt[wave][(uint32_t)(src_k[i] >> shift) & 255u], 1u);
-    if (kWaves > 1) __syncthreads(); else __builtin_amdgcn_wave_barrier();
-
-    bool uniform;
-    if (kWaves == 1) {
-        // lane handles digits lane, lane+64, lane+128, lane+192; scan in digit order
-        uint32_t base = 0;
-        bool any_full = false;
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const uint32_t c = cnt[0][q * kWave + lane];
-            any_full = any_full || c == (uint32_t)n;
-            uint32_t incl = wave_inclusive_sum(c);
-            cnt[0][q * kWave + lane] = base + incl - c;
-            base += (uint32_t)bcast_i((int)incl, kWave - 1);
+    __syncthreads();
+    // thread t < 256 handles digit t
+    uint32_t total = 0;
+    if (tid < kBins) {
+        for (int w = 0; w < kWaves; w++) {
+            const uint32_t c = cnt[w][tid];
+            cnt[w][tid] = total;          // offset of wave w inside digit tid
+            total += c;
         }
-        uniform = ballot(any_full) != 0;
-        __builtin_amdgcn_wave_barrier();
-    } else {
-        // thread t < 256 handles digit t
-        uint32_t total = 0;
-        if (tid < kBins) {
-            for (int w = 0; w < kWaves; w++) {
-                const uint32_t c = cnt[w][tid];
-                cnt[w][tid] = total;          // offset of wave w inside digit tid
-                total += c;
-            }
-            if (total == (uint32_t)n) *flag = 1;
-            uint32_t incl = wave_inclusive_sum(total);
-            if (lane == kWave - 1) wave_sum[wave] = incl;
-            total = incl - total;             // exclusive inside this wave's 64 digits
-        }
-        __syncthreads();
-        if (tid < kBins) {
-            uint32_t base = total;
-            for (int w = 0; w < wave; w++) base += wave_sum[w];
-            for (int w = 0; w < kWaves; w++) cnt[w][tid] += base;     // absolute start of (wave, digit)
-        }
-        __syncthreads();
-        uniform = *flag != 0;
+        if (total == (uint32_t)n) *flag = 1;
+        uint32_t incl = wave_inclusive_sum(total);
+        if (lane == kWave - 1) wave_sum[wave] = incl;
+        total = incl - total;             // exclusive inside this wave's 64 digits
     }
+    __syncthreads();
+    if (tid < kBins) {
+        uint32_t base = total;
+        for (int w = 0; w < wave; w++) base += wave_sum[w];
+        for (int w = 0; w < kWaves; w++) cnt[w][tid] += base;     // absolute start of (wave, digit)
+    }
+    __syncthreads();
+    const bool uniform = *flag != 0;
     if (uniform) return false;
 
     // stable ranking, 64 pairs at a time in segment order
     for (int base = w_lo; base < w_hi; base += kWave) {
         const int i = base + lane;
         const bool valid = i < w_hi;
-        KeyT k = 0;
+        uint64_t k = 0;
         uint32_t v = 0;
-        if (valid) { k = src_k[i]; v = src_v[i]; }
+        if (valid) { k = src_k[i]; if (src_v) v = src_v[i]; }
         const uint32_t d = (uint32_t)(k >> shift) & 255u;
         uint64_t peers = ballot(valid);
 #pragma unroll
@@ -733,7 +853,7 @@ __device__ __forceinline__ bool counting_pass(const KeyT* src_k, const uint32_t*
         before = (uint32_t)__shfl((int)before, leader);
         if (valid) {
             dst_k[before + (uint32_t)below] = k;
-            dst_v[before + (uint32_t)below] = v;
+            if (src_v) dst_v[before + (uint32_t)below] = v;
         }
         __builtin_amdgcn_wave_barrier();
     }
@@ -858,6 +978,41 @@ __device__ __forceinline__ void bitonic_network(uint64_t (&c)[kT], int lane)
         merge_slots(c, lane, k, k < n && (lane & (k / kT)) != 0 ? 0x80000000u : 0u, held);   // the last merge ascends everywhere
 }
 
+// A list as the segment sort finds and leaves it.  kWords: keys holds depth << 32 | value words and values nothing yet.
+struct Lists {
+    uint64_t* keys;
+    uint32_t* values;
+    const uint64_t* keys_in;            // the caller's unsorted list
+    const uint32_t* values_in;
+    const uint32_t* by_index;           // one word: not zero where the values are indices into that list
+};
+
+template <bool kWords>
+__device__ __forceinline__ uint64_t word_at(const Lists& l, int i)
+{
+    if (kWords) return l.keys[i];
+    return (l.keys[i] << 32) | l.values[i];
+}
+
+template <bool kWords>
+__device__ __forceinline__ uint32_t value_at(const Lists& l, int i)
+{
+    return kWords ? (uint32_t)l.keys[i] : l.values[i];
+}
+
+// Stores a pair of tile id v.
+__device__ __forceinline__ void store_pair(const Lists& l, bool by_index, int i, uint32_t v, uint64_t word)
+{
+    uint64_t key = ((uint64_t)v << 32) | (word >> 32);
+    uint32_t value = (uint32_t)word;
+    if (by_index) {
+        key = l.keys_in[value];
+        value = l.values_in[value];
+    }
+    l.keys[i] = key;
+    l.values[i] = value;
+}
+
 // Words of LDS a wave needs to sort up to n pairs with the network: one 64-bit word for every
 // second pair (the sorted pairs go through it in two halves), one word of padding after every 16 (lane l puts its kUse consecutive ranks down at once; without
 // the padding the lanes of a wave would all start in the same bank).
@@ -871,13 +1026,13 @@ __device__ __forceinline__ int staged(int i) { return i + (i >> 4); }
 // stored contiguously again.  Equal depths have to stay in input order.  The pairs of one tile
 // come out of the preprocess in ascending order of their values (Gaussian indices) and their depths are
 // positive floats: then the value itself is the tie-break, the sorted word is the pair, and the word
-// is a positive finite double.  A segment whose values do not ascend, or with a depth word from
+// is a positive finite double (values that are indices ascend as well).  A segment whose values do not ascend, or with a depth word from
 // 0x7ff00000 up, carries depth << 16 | position instead (a small positive double whatever the depth)
 // and looks its values up afterwards.
-template <int kUse>
-__device__ __forceinline__ void sort_segment_bitonic_of(uint64_t* __restrict__ keys, uint32_t* __restrict__ values,
-                                                        uint32_t v, int lo, int hi, uint32_t* __restrict__ seg_flags,
-                                                        uint64_t* s_w)
+constexpr uint64_t kLastWord = 0x7fefffffffffffffull;       // the largest finite double
+
+template <int kUse, bool kWords>
+__device__ __forceinline__ void sort_segment_bitonic_of(const Lists& lists, uint32_t v, int lo, int hi, uint64_t* s_w)
 {
     // The lane number is made opaque here and again behind the network: otherwise every index and
     // address derived from it, for every width of the network, is computed once in front of the loop
@@ -886,56 +1041,45 @@ __device__ __forceinline__ void sort_segment_bitonic_of(uint64_t* __restrict__ k
     asm volatile("" : "+v"(lane));
     const int len = hi - lo;
     uint64_t c[kUse];
-    uint32_t val[kUse];
     // Every load is issued before the first one is looked at (nothing but the load stands under
     // the condition: a use in there would be waited for before the next slot's load goes out).  A
-    // slot past the end of the segment keeps all ones.
-    const uint64_t* const key_at = keys + lo + lane;
-    const uint32_t* const value_at = values + lo + lane;
+    // slot past the end of the segment holds the largest finite double and sorts behind every pair.
 #pragma unroll
     for (int t = 0; t < kUse; t++) {
-        c[t] = ~0ull;
-        val[t] = ~0u;
-        if (t * kWave + lane < len) {
-            c[t] = key_at[t * kWave];
-            val[t] = value_at[t * kWave];
+        c[t] = kWords ? kLastWord : ~0ull;
+        if (t * kWave + lane < len) c[t] = lists.keys[lo + t * kWave + lane];
+    }
+    if constexpr (!kWords) {
+        uint32_t val[kUse];
+#pragma unroll
+        for (int t = 0; t < kUse; t++) {
+            val[t] = ~0u;
+            if (t * kWave + lane < len) val[t] = lists.values[lo + t * kWave + lane];
         }
+#pragma unroll
+        for (int t = 0; t < kUse; t++) c[t] = t * kWave + lane < len ? (c[t] << 32) | val[t] : kLastWord;
     }
-    const uint32_t upper = (uint32_t)bcast_i((int)(uint32_t)(c[0] >> 32), 0);
-    bool mixed = false;
-    bool beyond = false;
+    bool other_words = false;   // a depth word from 0x7ff00000 up, or position i + 1 holds a smaller value than position i
 #pragma unroll
     for (int t = 0; t < kUse; t++) {
-        mixed = mixed || (t * kWave + lane < len && (uint32_t)(c[t] >> 32) != upper);
-        beyond = beyond || (t * kWave + lane < len && (uint32_t)c[t] >= 0x7ff00000u);
-    }
-    bool descends = false;   // position i + 1 holds a smaller value than position i
-#pragma unroll
-    for (int t = 0; t < kUse; t++) {
-        uint32_t next = (uint32_t)__shfl_down((int)val[t], 1);
+        uint32_t next = (uint32_t)__shfl_down((int)(uint32_t)c[t], 1);
         if (t + 1 < kUse) {
-            const uint32_t wrap = (uint32_t)bcast_i((int)val[t + 1 < kUse ? t + 1 : t], 0);
+            const uint32_t wrap = (uint32_t)bcast_i((int)(uint32_t)c[t + 1 < kUse ? t + 1 : t], 0);
             if (lane == kWave - 1) next = wrap;
         }
-        descends = descends || (t * kWave + lane + 1 < len && next < val[t]);
+        other_words = other_words || (t * kWave + lane + 1 < len && next < (uint32_t)c[t]) || (uint32_t)(c[t] >> 32) >= 0x7ff00000u;
     }
-    // (looked at behind the values on purpose: in front of them, their loads would wait for it)
-    if (ballot(mixed)) {     // keys differ above the depth word: left to the general kernel
-        if (seg_flags && lane == 0) atomicOr(&seg_flags[v >> 5], 1u << (v & 31));
-        return;
-    }
-    const bool by_value = ballot(descends || beyond) == 0;
+    const bool by_value = ballot(other_words) == 0;
     // (no branches around the slots: where two paths meet, the sixteen words are copied from the
     // registers one path left them in to those of the other)
     uint32_t* const s_val = (uint32_t*)s_w;
 #pragma unroll
     for (int t = 0; t < kUse; t++) {
         const int i = t * kWave + lane;
-        if (!by_value && i < len) s_val[i] = val[t];
-        const uint32_t depth = (uint32_t)c[t];
-        // a slot past the end of the segment has a depth of all ones and sorts behind every pair: as the
-        // largest finite double, or by its position
-        const uint32_t high = by_value ? min(depth, 0x7fefffffu) : depth >> 16, low = by_value ? val[t] : (depth << 16) | (uint32_t)i;
+        const uint32_t depth = (uint32_t)(c[t] >> 32), value = (uint32_t)c[t];
+        if (!by_value && i < len) s_val[i] = value;
+        // (a slot past the end by its position)
+        const uint32_t high = by_value ? depth : i < len ? depth >> 16 : 0xffffu, low = by_value ? value : (depth << 16) | (uint32_t)i;
         c[t] = ((uint64_t)high << 32) | low;
     }
     bitonic_network<kUse>(c, lane);
@@ -950,8 +1094,7 @@ __device__ __forceinline__ void sort_segment_bitonic_of(uint64_t* __restrict__ k
     // back to contiguous stores through LDS, the lower half of the ranks (lanes 0..31) first, then
     // the upper half through the same words: half the LDS, twice the waves per CU
     constexpr int kRounds = kUse >= 2 ? 2 : 1, kPart = kUse * kWave / kRounds;
-    uint64_t* const key_to = keys + lo + lane;
-    uint32_t* const value_to = values + lo + lane;
+    const bool by_index = *lists.by_index != 0;
 #pragma unroll
     for (int h = 0; h < kRounds; h++) {
         __builtin_amdgcn_wave_barrier();
@@ -966,11 +1109,7 @@ __device__ __forceinline__ void sort_segment_bitonic_of(uint64_t* __restrict__ k
 #pragma unroll
         for (int t = h * (kUse / kRounds); t < (h + 1) * (kUse / kRounds); t++) {
             const int i = t * kWave + lane;
-            if (i < len) {
-                const uint64_t w = s_w[staged(i - h * kPart)];
-                key_to[t * kWave] = ((uint64_t)upper << 32) | (w >> 32);
-                value_to[t * kWave] = (uint32_t)w;
-            }
+            if (i < len) store_pair(lists, by_index, lo + i, v, s_w[staged(i - h * kPart)]);
         }
     }
     __builtin_amdgcn_wave_barrier();
@@ -978,17 +1117,15 @@ __device__ __forceinline__ void sort_segment_bitonic_of(uint64_t* __restrict__ k
 
 // The network over the smallest power of two of register slots (at most kT) that holds the segment.
 // s_w: staging_words(64 * kT) 64-bit words.
-template <int kT>
-__device__ __forceinline__ void sort_segment_bitonic(uint64_t* __restrict__ keys, uint32_t* __restrict__ values,
-                                                     uint32_t v, int lo, int hi, uint32_t* __restrict__ seg_flags,
-                                                     uint64_t* s_w)
+template <int kT, bool kWords>
+__device__ __forceinline__ void sort_segment_bitonic(const Lists& lists, uint32_t v, int lo, int hi, uint64_t* s_w)
 {
     const int len = hi - lo;
-    if (len <= kWave) sort_segment_bitonic_of<1>(keys, values, v, lo, hi, seg_flags, s_w);
-    else if (kT >= 2 && len <= 2 * kWave) sort_segment_bitonic_of<(kT >= 2 ? 2 : 1)>(keys, values, v, lo, hi, seg_flags, s_w);
-    else if (kT >= 4 && len <= 4 * kWave) sort_segment_bitonic_of<(kT >= 4 ? 4 : 1)>(keys, values, v, lo, hi, seg_flags, s_w);
-    else if (kT >= 8 && len <= 8 * kWave) sort_segment_bitonic_of<(kT >= 8 ? 8 : 1)>(keys, values, v, lo, hi, seg_flags, s_w);
-    else sort_segment_bitonic_of<kT>(keys, values, v, lo, hi, seg_flags, s_w);
+    if (len <= kWave) sort_segment_bitonic_of<1, kWords>(lists, v, lo, hi, s_w);
+    else if (kT >= 2 && len <= 2 * kWave) sort_segment_bitonic_of<(kT >= 2 ? 2 : 1), kWords>(lists, v, lo, hi, s_w);
+    else if (kT >= 4 && len <= 4 * kWave) sort_segment_bitonic_of<(kT >= 4 ? 4 : 1), kWords>(lists, v, lo, hi, s_w);
+    else if (kT >= 8 && len <= 8 * kWave) sort_segment_bitonic_of<(kT >= 8 ? 8 : 1), kWords>(lists, v, lo, hi, s_w);
+    else sort_segment_bitonic_of<kT, kWords>(lists, v, lo, hi, s_w);
 }
 
 // One step of the network between two waves: the wave's words against those of `partner`, in the same
@@ -1018,8 +1155,7 @@ __device__ __forceinline__ void compare_waves(uint64_t (&c)[kT], int lane, int w
 
 // Sorts the segment [lo, hi) of tile id v, 64 * kWaves * kUse >= hi - lo, with the network over kUse
 // slots per lane of kWaves waves.  Called by all waves of a workgroup with the same arguments.  s_w: 64 *
-// kWaves * kUse words of LDS; s_seen: one word per wave.  A segment whose keys differ above the depth word is
-// flagged (or, without a flag array, left alone) for the general kernel: returns true then.
+// kWaves * kUse words of LDS; s_seen: one word per wave.
 // Every wave sorts 64 * kUse words as above.  Runs are then merged in pairs: the first step compares
 // element i of the lower run with element i from the end of the upper one, the next ones halve the
 // distance, between waves through LDS and inside a wave as above.  All runs ascend, so the words
@@ -1030,10 +1166,8 @@ __device__ __forceinline__ void compare_waves(uint64_t (&c)[kT], int lane, int w
 // twice as long per pair: 8K frame of 111M pairs 825 -> 475 us for the segments of 1025 .. 4096 pairs
 // and 343 -> 195 for those up to 8192, 179 -> 141 for the longer ones; 4K frame of 8M pairs 49 -> 33,
 // 1080p frame of 1.8M pairs 18.6 -> 13.6.
-template <int kWaves, int kUse>
-__device__ __forceinline__ bool sort_segment_waves_of(uint64_t* __restrict__ keys, uint32_t* __restrict__ values,
-                                                      uint32_t v, int lo, int hi, uint32_t* __restrict__ seg_flags,
-                                                      uint64_t* s_w, uint32_t* s_seen)
+template <int kWaves, int kUse, bool kWords>
+__device__ __forceinline__ void sort_segment_waves_of(const Lists& lists, uint32_t v, int lo, int hi, uint64_t* s_w, uint32_t* s_seen)
 {
     static_assert(kUse >= 2, "the ranks leave in two halves of a wave's slots");
     constexpr int kPart = kUse * kWave;                 // words of a wave
@@ -1045,54 +1179,43 @@ __device__ __forceinline__ bool sort_segment_waves_of(uint64_t* __restrict__ key
     const bool present = first < len;
     const int mine = len - first;
     uint64_t c[kUse];
-    uint32_t val[kUse];
-    const uint64_t* const key_at = keys + lo + first + lane;
-    const uint32_t* const value_at = values + lo + first + lane;
 #pragma unroll
     for (int t = 0; t < kUse; t++) {
-        c[t] = ~0ull;
-        val[t] = ~0u;
-        if (t * kWave + lane < mine) {
-            c[t] = key_at[t * kWave];
-            val[t] = value_at[t * kWave];
+        c[t] = kWords ? kLastWord : ~0ull;
+        if (t * kWave + lane < mine) c[t] = lists.keys[lo + first + t * kWave + lane];
+    }
+    if constexpr (!kWords) {
+        uint32_t val[kUse];
+#pragma unroll
+        for (int t = 0; t < kUse; t++) {
+            val[t] = ~0u;
+            if (t * kWave + lane < mine) val[t] = lists.values[lo + first + t * kWave + lane];
         }
+#pragma unroll
+        for (int t = 0; t < kUse; t++) c[t] = t * kWave + lane < mine ? (c[t] << 32) | val[t] : kLastWord;
     }
     asm volatile("" : "+v"(lane));
-    const uint32_t upper = (uint32_t)(keys[lo] >> 32);
-    const uint32_t behind = mine > kPart ? values[lo + first + kPart] : ~0u;       // the first value of the next wave's part
-    bool mixed = false, other_words = false;
+    const uint32_t behind = mine > kPart ? value_at<kWords>(lists, lo + first + kPart) : ~0u;       // the first value of the next wave's part
+    bool other_words = false;
 #pragma unroll
     for (int t = 0; t < kUse; t++) {
-        const bool valid = t * kWave + lane < mine;
-        mixed = mixed || (valid && (uint32_t)(c[t] >> 32) != upper);
-        other_words = other_words || (valid && (uint32_t)c[t] >= 0x7ff00000u);
-    }
-    asm volatile("" : "+v"(lane));
-#pragma unroll
-    for (int t = 0; t < kUse; t++) {
-        uint32_t next = (uint32_t)__shfl_down((int)val[t], 1);
-        const uint32_t wrap = t + 1 < kUse ? (uint32_t)bcast_i((int)val[t + 1 < kUse ? t + 1 : t], 0) : behind;
+        uint32_t next = (uint32_t)__shfl_down((int)(uint32_t)c[t], 1);
+        const uint32_t wrap = t + 1 < kUse ? (uint32_t)bcast_i((int)(uint32_t)c[t + 1 < kUse ? t + 1 : t], 0) : behind;
         if (lane == kWave - 1) next = wrap;
-        other_words = other_words || (t * kWave + lane + 1 < mine && next < val[t]);
+        other_words = other_words || (t * kWave + lane + 1 < mine && next < (uint32_t)c[t]) || (uint32_t)(c[t] >> 32) >= 0x7ff00000u;
         if (t % 4 == 3) __builtin_amdgcn_sched_barrier(0);
     }
-    const uint32_t seen = (ballot(mixed) ? 1u : 0u) | (ballot(other_words) ? 2u : 0u);
+    const uint32_t seen = ballot(other_words) ? 1u : 0u;
     if (lane == 0) s_seen[wave] = seen;
     __syncthreads();
     uint32_t any = 0;
 #pragma unroll
     for (int w = 0; w < kWaves; w++) any |= s_seen[w];
-    any = (uint32_t)__builtin_amdgcn_readfirstlane((int)any);
-    if (any & 1u) {
-        if (seg_flags && threadIdx.x == 0) atomicOr(&seg_flags[v >> 5], 1u << (v & 31));
-        __syncthreads();                        // s_seen is written again for the next segment
-        return true;
-    }
-    const bool by_value = any == 0;
+    const bool by_value = __builtin_amdgcn_readfirstlane((int)any) == 0;
 #pragma unroll
     for (int t = 0; t < kUse; t++) {
-        const uint32_t depth = (uint32_t)c[t], i = (uint32_t)(first + t * kWave + lane);
-        const uint32_t high = by_value ? min(depth, 0x7fefffffu) : depth >> 16, low = by_value ? val[t] : (depth << 16) | i;
+        const uint32_t depth = (uint32_t)(c[t] >> 32), value = (uint32_t)c[t], i = (uint32_t)(first + t * kWave + lane);
+        const uint32_t high = by_value ? depth : (int)i < len ? depth >> 16 : 0xffffu, low = by_value ? value : (depth << 16) | i;
         c[t] = ((uint64_t)high << 32) | low;
     }
     if (present) bitonic_network<kUse>(c, lane);
@@ -1114,15 +1237,14 @@ __device__ __forceinline__ bool sort_segment_waves_of(uint64_t* __restrict__ key
     for (int t = 0; t < kUse; t++) {
         const uint32_t high = (uint32_t)(c[t] >> 32), low = (uint32_t)c[t];
         uint32_t value = low;
-        if (!by_value && (low & 0xffffu) < (uint32_t)len) value = values[lo + (int)(low & 0xffffu)];
+        if (!by_value && (low & 0xffffu) < (uint32_t)len) value = value_at<kWords>(lists, lo + (int)(low & 0xffffu));
         c[t] = ((uint64_t)(by_value ? high : (high << 16) | (low >> 16)) << 32) | value;
         if (t % 4 == 3) __builtin_amdgcn_sched_barrier(0);
     }
     if (!by_value) __syncthreads();
     // back to contiguous stores through this wave's part of the LDS, half of the ranks at a time
     uint64_t* const s_mine = s_w + first;
-    uint64_t* const key_to = keys + lo + first + lane;
-    uint32_t* const value_to = values + lo + first + lane;
+    const bool by_index = *lists.by_index != 0;
 #pragma unroll
     for (int h = 0; h < 2; h++) {
         __builtin_amdgcn_wave_barrier();
@@ -1134,37 +1256,29 @@ __device__ __forceinline__ bool sort_segment_waves_of(uint64_t* __restrict__ key
 #pragma unroll
         for (int t = h * (kUse / 2); t < (h + 1) * (kUse / 2); t++) {
             const int i = t * kWave + lane;
-            if (i < mine) {
-                const uint64_t w = s_mine[staged(i - h * (kPart / 2))];
-                key_to[t * kWave] = ((uint64_t)upper << 32) | (w >> 32);
-                value_to[t * kWave] = (uint32_t)w;
-            }
+            if (i < mine) store_pair(lists, by_index, lo + first + i, v, s_mine[staged(i - h * (kPart / 2))]);
         }
     }
     __syncthreads();
-    return false;
 }
 
 // The smallest number of slots per lane, from kLeast on, that holds the segment: hi - lo <= kCap.
-template <int kWaves, int kCap, int kLeast>
-__device__ __forceinline__ bool sort_segment_waves(uint64_t* __restrict__ keys, uint32_t* __restrict__ values,
-                                                   uint32_t v, int lo, int hi, uint32_t* __restrict__ seg_flags,
-                                                   uint64_t* s_w, uint32_t* s_seen)
+template <int kWaves, int kCap, int kLeast, bool kWords>
+__device__ __forceinline__ void sort_segment_waves(const Lists& lists, uint32_t v, int lo, int hi, uint64_t* s_w, uint32_t* s_seen)
 {
     constexpr int kMost = kCap / (kWaves * kWave);
     if constexpr (kLeast < kMost)
         if (hi - lo > kLeast * kWaves * kWave)
-            return sort_segment_waves<kWaves, kCap, 2 * kLeast>(keys, values, v, lo, hi, seg_flags, s_w, s_seen);
-    return sort_segment_waves_of<kWaves, kLeast>(keys, values, v, lo, hi, seg_flags, s_w, s_seen);
+            return sort_segment_waves<kWaves, kCap, 2 * kLeast, kWords>(lists, v, lo, hi, s_w, s_seen);
+    sort_segment_waves_of<kWaves, kLeast, kWords>(lists, v, lo, hi, s_w, s_seen);
 }
 
 // Segment sort by the waves of a workgroup for one size class: segments with min_len < length <= kCap.
 // With a table of segment starts, the first launch has listed the segments of the class.  Without a table
 // (more tile ids than it holds) the grid has one workgroup per tile id and each searches for its bounds.
-template <int kWaves, int kCap, int kLeast>
+template <int kWaves, int kCap, int kLeast, bool kWords>
 __global__ __launch_bounds__(kWaves * kWave) void segment_sort_kernel(
-    uint64_t* __restrict__ keys, uint32_t* __restrict__ values, int n, uint32_t tile_mask, int min_len,
-    const int* __restrict__ seg_start, uint32_t* __restrict__ seg_flags,
+    Lists lists, int n, uint32_t tile_mask, int min_len, const int* __restrict__ seg_start,
     const uint32_t* __restrict__ list, const uint32_t* __restrict__ list_count, uint32_t list_cap)
 {
     __shared__ uint64_t s_w[kCap];
@@ -1177,14 +1291,14 @@ __global__ __launch_bounds__(kWaves * kWave) void segment_sort_kernel(
     if (!seg_start) {
         const uint32_t v = blockIdx.x;
         if (tid < kWave) {
-            const int a = wave_lower_bound(keys, n, v, tile_mask);
-            const int b = v == tile_mask ? n : wave_lower_bound(keys, n, v + 1, tile_mask);
+            const int a = wave_lower_bound(lists.keys, n, v, tile_mask);
+            const int b = v == tile_mask ? n : wave_lower_bound(lists.keys, n, v + 1, tile_mask);
             if (lane == 0) { s_bounds[0] = a; s_bounds[1] = b; }
         }
         __syncthreads();
         const int lo = s_bounds[0], hi = s_bounds[1];
         if (hi - lo <= min_len || hi - lo > kCap) return;
-        sort_segment_waves<kWaves, kCap, kLeast>(keys, values, v, lo, hi, seg_flags, s_w, s_seen);
+        sort_segment_waves<kWaves, kCap, kLeast, kWords>(lists, v, lo, hi, s_w, s_seen);
         return;
     }
 
@@ -1193,67 +1307,55 @@ __global__ __launch_bounds__(kWaves * kWave) void segment_sort_kernel(
     const uint32_t count = list_count[shard];
     for (uint32_t i = blockIdx.x / kListShards; i < count; i += gridDim.x / kListShards) {
         const uint32_t v = list[(size_t)shard * list_cap + i];
-        sort_segment_waves<kWaves, kCap, kLeast>(keys, values, v, seg_start[v], seg_start[v + 1], seg_flags, s_w, s_seen);
+        sort_segment_waves<kWaves, kCap, kLeast, kWords>(lists, v, seg_start[v], seg_start[v + 1], s_w, s_seen);
     }
 }
 
-// One wave per workgroup; with a table of segment starts the workgroup looks at kIds tile ids
-// (one per lane) and sorts those with min_len < length <= 64*kT one after the other; without a
-// table the grid has one workgroup per tile id and each searches for its bounds.
-template <int kT, int kIds>
+// One wave per workgroup, and one workgroup per tile id: it sorts that id's segment of up to 64*kT pairs.  Its bounds come from
+// the table of segment starts or, without one, from a search.
+template <int kT, bool kWords>
 __global__ __launch_bounds__(kWave) void segment_sort_wave_kernel(
-    uint64_t* __restrict__ keys, uint32_t* __restrict__ values, int n, uint32_t tile_mask, int min_len, uint32_t ids,
-    const int* __restrict__ seg_start, uint32_t* __restrict__ seg_flags,
+    Lists lists, int n, uint32_t tile_mask, const int* __restrict__ seg_start,
     int list_max0, int list_max1, int list_max2,
     uint32_t* __restrict__ seg_counts, uint32_t* __restrict__ list0, uint32_t* __restrict__ list1,
     uint32_t* __restrict__ list2, uint32_t* __restrict__ list3,
     uint32_t list_cap0, uint32_t list_cap1, uint32_t list_cap2, uint32_t list_cap3)
 {
     __shared__ uint64_t s_w[staging_words(kT * kWave)];
-    const int lane = threadIdx.x;
-    uint32_t first_id = blockIdx.x;
-    uint64_t todo = 0;
-    int lo_found = 0, hi_found = 0;
+    const uint32_t v = blockIdx.x;
+    int lo, hi;
     if (!seg_start) {
-        lo_found = wave_lower_bound(keys, n, first_id, tile_mask);
-        hi_found = first_id == tile_mask ? n : wave_lower_bound(keys, n, first_id + 1, tile_mask);
-        todo = hi_found - lo_found > min_len && hi_found - lo_found <= kT * kWave ? 1u : 0u;
+        lo = wave_lower_bound(lists.keys, n, v, tile_mask);
+        hi = v == tile_mask ? n : wave_lower_bound(lists.keys, n, v + 1, tile_mask);
     } else {
-        first_id = blockIdx.x * (uint32_t)kIds;
-        const uint32_t mine = first_id + (uint32_t)lane;
-        int len = 0;
-        if (lane < kIds && mine < ids) len = seg_start[mine + 1] - seg_start[mine];
+        lo = seg_start[v];
+        hi = seg_start[v + 1];
         // This launch sees every tile id once: it also lists the ids of the longer segments by class
         // (lengths up to list_max0, list_max1, list_max2, and everything longer), so that those
         // fewer, longer-running segments can be dealt out evenly by the launches that follow.
-        if (list0) {
+        const int len = hi - lo;
+        if (len > kT * kWave && threadIdx.x == 0) {
             // neighbouring tiles tend to be equally busy: mix the index so that every list gets its share
-            const uint32_t shard = (blockIdx.x ^ (blockIdx.x >> 5) ^ (blockIdx.x >> 10) ^ (blockIdx.x >> 15)) % kListShards;
-            if (len > kT * kWave && len <= list_max0)
-                list0[(size_t)shard * list_cap0 + atomicAdd(&seg_counts[0 * kListShards + shard], 1u)] = mine;
-            else if (len > list_max0 && len <= list_max1)
-                list1[(size_t)shard * list_cap1 + atomicAdd(&seg_counts[1 * kListShards + shard], 1u)] = mine;
-            else if (len > list_max1 && len <= list_max2)
-                list2[(size_t)shard * list_cap2 + atomicAdd(&seg_counts[2 * kListShards + shard], 1u)] = mine;
-            else if (len > list_max2)
-                list3[(size_t)shard * list_cap3 + atomicAdd(&seg_counts[3 * kListShards + shard], 1u)] = mine;
+            const uint32_t shard = (v ^ (v >> 5) ^ (v >> 10) ^ (v >> 15)) % kListShards;
+            if (len <= list_max0)
+                list0[(size_t)shard * list_cap0 + atomicAdd(&seg_counts[0 * kListShards + shard], 1u)] = v;
+            else if (len <= list_max1)
+                list1[(size_t)shard * list_cap1 + atomicAdd(&seg_counts[1 * kListShards + shard], 1u)] = v;
+            else if (len <= list_max2)
+                list2[(size_t)shard * list_cap2 + atomicAdd(&seg_counts[2 * kListShards + shard], 1u)] = v;
+            else
+                list3[(size_t)shard * list_cap3 + atomicAdd(&seg_counts[3 * kListShards + shard], 1u)] = v;
         }
-        todo = ballot(len > min_len && len <= kT * kWave);
     }
-    for (; todo; todo &= todo - 1) {
-        const uint32_t v = first_id + (uint32_t)(__ffsll((long long)todo) - 1);
-        const int lo = seg_start ? seg_start[v] : lo_found, hi = seg_start ? seg_start[v + 1] : hi_found;
-        sort_segment_bitonic<kT>(keys, values, v, lo, hi, seg_flags, s_w);
-        __builtin_amdgcn_wave_barrier();
-    }
+    // (words become pairs here, and indices values, also where there is nothing to sort)
+    if (hi > lo && hi - lo <= kT * kWave) sort_segment_bitonic<kT, kWords>(lists, v, lo, hi, s_w);
 }
 
 // The listed segments of one class (at most 64*kT pairs each), dealt out round-robin to
 // single-wave workgroups.
-template <int kT>
+template <int kT, bool kWords>
 __global__ __launch_bounds__(kWave) void segment_sort_wave_list_kernel(
-    uint64_t* __restrict__ keys, uint32_t* __restrict__ values, const int* __restrict__ seg_start,
-    uint32_t* __restrict__ seg_flags, const uint32_t* __restrict__ list, const uint32_t* __restrict__ list_count,
+    Lists lists, const int* __restrict__ seg_start, const uint32_t* __restrict__ list, const uint32_t* __restrict__ list_count,
     uint32_t list_cap)
 {
     __shared__ uint64_t s_w[staging_words(kT * kWave)];
@@ -1261,145 +1363,103 @@ __global__ __launch_bounds__(kWave) void segment_sort_wave_list_kernel(
     const uint32_t count = list_count[shard];
     for (uint32_t i = blockIdx.x / kListShards; i < count; i += gridDim.x / kListShards) {
         const uint32_t v = list[(size_t)shard * list_cap + i];
-        sort_segment_bitonic<kT>(keys, values, v, seg_start[v], seg_start[v + 1], seg_flags, s_w);
+        sort_segment_bitonic<kT, kWords>(lists, v, seg_start[v], seg_start[v + 1], s_w);
         __builtin_amdgcn_wave_barrier();
     }
 }
 
-// The same passes with whole keys and the ping-pong copy in HBM: for segments longer than
-// min_len and for shorter segments whose keys differ above the depth word.  General and slow;
-// inputs produced by fgs_preprocess only reach it with more than min_len pairs in one tile.
+// Stable counting passes with a ping-pong copy in HBM: for segments of more than min_len pairs.
 // Sixteen waves per workgroup: such a segment has thousands of pairs, every pass reads them from
 // memory 64 per wave and step, and the workgroup has the CU almost to itself (a frame of 109M
 // pairs with 534 such segments: 0.55 ms for the launch with four waves).
 constexpr int kGeneralWaves = 16;
 
-__device__ __forceinline__ void sort_segment_general(uint64_t* __restrict__ keys, uint32_t* __restrict__ values,
-                                                     uint64_t* __restrict__ alt_keys, uint32_t* __restrict__ alt_values,
-                                                     int lo, int hi, uint32_t (*s_cnt)[kBins], uint32_t* s_wave_sum, int* s_flag)
+template <bool kWords>
+__device__ __forceinline__ void sort_segment_general(const Lists& lists, uint64_t* __restrict__ alt_keys, uint32_t* __restrict__ alt_values,
+                                                     uint32_t v, int lo, int hi, uint32_t (*s_cnt)[kBins], uint32_t* s_wave_sum, int* s_flag)
 {
     // opaque, like the lane number of the networks: or the addresses of the copy below stay in
     // registers beside a network's words in a workgroup that does both
     int tid = threadIdx.x;
     asm volatile("" : "+v"(tid));
     const int len = hi - lo;
-    uint64_t* kbuf[2] = { keys + lo, alt_keys + lo };
-    uint32_t* vbuf[2] = { values + lo, alt_values + lo };
+    uint64_t* kbuf[2] = { lists.keys + lo, alt_keys + lo };
+    uint32_t* vbuf[2] = { kWords ? nullptr : lists.values + lo, kWords ? nullptr : alt_values + lo };
     int cur = 0;
+    constexpr int kDepth = kWords ? 32 : 0;             // where the depth bits begin
 #pragma unroll 1
-    for (int shift = 0; shift < 32; shift += 8) {
-        const bool moved = counting_pass<kGeneralWaves, uint64_t>(kbuf[cur], vbuf[cur], kbuf[cur ^ 1], vbuf[cur ^ 1], len,
-                                                                  shift, s_cnt, s_wave_sum, s_flag);
+    for (int shift = kDepth; shift < kDepth + 32; shift += 8) {
+        const bool moved = counting_pass<kGeneralWaves>(kbuf[cur], vbuf[cur], kbuf[cur ^ 1], vbuf[cur ^ 1], len, shift, s_cnt, s_wave_sum, s_flag);
         __threadfence_block();
         __syncthreads();
         if (moved) cur ^= 1;
     }
-    if (cur == 1)
-        for (int i = tid; i < len; i += kGeneralWaves * kWave) { kbuf[0][i] = kbuf[1][i]; vbuf[0][i] = vbuf[1][i]; }
+    const bool by_index = *lists.by_index != 0;
+    if (kWords || cur == 1 || by_index)
+        for (int i = tid; i < len; i += kGeneralWaves * kWave)
+            store_pair(lists, by_index, lo + i, v, kWords ? kbuf[cur][i] : (kbuf[cur][i] << 32) | vbuf[cur][i]);
     __threadfence_block();
     __syncthreads();
 }
 
-// With a table of segment starts the first list_blocks workgroups take the listed segments (the
+// With a table of segment starts the workgroups take the listed segments (the
 // ones longer than min_len: neighbouring tiles tend to be equally crowded, so they are dealt out
-// one segment at a time, round-robin), the workgroups behind them look at 64 tile ids each for
-// shorter segments that were flagged.
-// With a table (kLds) a listed segment of up to kCapHuge pairs is sorted by the network over the
+// one segment at a time, round-robin).
+// With a table (kTable) a listed segment of up to kCapHuge pairs is sorted by the network over the
 // sixteen waves (a workgroup then has the LDS of its CU to itself): the passes through memory take
 // 7 us each for 12 000 pairs.
-// The listed blocks first sort the listed segments of the classes below (first_class 1:
+// The workgroups first sort the listed segments of the classes below (first_class 1:
 // 1025 .. kCapLarge pairs, 2: only those above kCapMedium, 3: none; shard by shard like the
 // launches of those classes): a frame with a short list of pairs has few such segments or none,
 // and one launch instead of three is what counts there; up to kMergedLargeMax pairs the class
 // above kCapMedium still has few.
 constexpr int kCapHuge = 16384;
 
-template <bool kLds>
+template <bool kTable, bool kWords>
 __global__ __launch_bounds__(kGeneralWaves * kWave) void segment_sort_general_kernel(
-    uint64_t* __restrict__ keys, uint32_t* __restrict__ values,
-    uint64_t* __restrict__ alt_keys, uint32_t* __restrict__ alt_values,
-    int n, uint32_t tile_mask, int min_len, uint32_t ids,
-    const int* __restrict__ seg_start, const uint32_t* __restrict__ seg_flags,
-    const uint32_t* __restrict__ list, const uint32_t* __restrict__ list_count, uint32_t list_cap, uint32_t list_blocks,
+    Lists lists, uint64_t* __restrict__ alt_keys, uint32_t* __restrict__ alt_values,
+    int n, uint32_t tile_mask, int min_len, const int* __restrict__ seg_start,
+    const uint32_t* __restrict__ list, const uint32_t* __restrict__ list_count, uint32_t list_cap,
     const uint32_t* __restrict__ list_medium, uint32_t cap_medium, const uint32_t* __restrict__ list_large, uint32_t cap_large,
     int first_class)
 {
-    __shared__ uint64_t s_w[kLds ? kCapHuge : 1];
+    __shared__ uint64_t s_w[kTable ? kCapHuge : 1];
     __shared__ uint32_t s_cnt[kGeneralWaves][kBins];
     __shared__ uint32_t s_wave_sum[kGeneralWaves];
     __shared__ int s_bounds[2];
     __shared__ int s_flag;
-    __shared__ uint64_t s_match;
 
     const int tid = threadIdx.x;
     const int lane = tid & (kWave - 1);
 
-    if (!seg_start) {
+    if constexpr (!kTable) {
         const uint32_t v = blockIdx.x;
         if (tid < kWave) {
-            const int a = wave_lower_bound(keys, n, v, tile_mask);
-            const int b = v == tile_mask ? n : wave_lower_bound(keys, n, v + 1, tile_mask);
-            if (lane == 0) { s_bounds[0] = a; s_bounds[1] = b; s_flag = 0; }
+            const int a = wave_lower_bound(lists.keys, n, v, tile_mask);
+            const int b = v == tile_mask ? n : wave_lower_bound(lists.keys, n, v + 1, tile_mask);
+            if (lane == 0) { s_bounds[0] = a; s_bounds[1] = b; }
         }
         __syncthreads();
         const int lo = s_bounds[0], hi = s_bounds[1];
-        const int len = hi - lo;
-        if (len < 2) return;
-        if (len <= min_len) {       // without flags the shorter segments are re-examined here
-            const uint32_t upper = (uint32_t)(keys[lo] >> 32);
-            bool mixed = false;
-            for (int i = tid; i < len; i += kGeneralWaves * kWave) mixed = mixed || (uint32_t)(keys[lo + i] >> 32) != upper;
-            if (mixed) s_flag = 1;
-            __syncthreads();
-            const bool any_mixed = s_flag != 0;
-            __syncthreads();
-            if (!any_mixed) return;
-        }
-        sort_segment_general(keys, values, alt_keys, alt_values, lo, hi, s_cnt, s_wave_sum, &s_flag);
-        return;
-    }
-
-    if (blockIdx.x < list_blocks) {
+        if (hi - lo > min_len) sort_segment_general<kWords>(lists, alt_keys, alt_values, v, lo, hi, s_cnt, s_wave_sum, &s_flag);
+    } else {
         const uint32_t shard = blockIdx.x % kListShards;
         // list_count: the counters of all classes, class c at c * kListShards (1: medium, 2: large, 3: long)
         for (int c = first_class; c <= 3; c++) {
             const uint32_t* const ids_of = c == 1 ? list_medium : c == 2 ? list_large : list;
             const uint32_t cap = c == 1 ? cap_medium : c == 2 ? cap_large : list_cap;
             const uint32_t count = list_count[c * kListShards + shard];
-            for (uint32_t i = blockIdx.x / kListShards; i < count; i += list_blocks / kListShards) {
+            for (uint32_t i = blockIdx.x / kListShards; i < count; i += gridDim.x / kListShards) {
                 const uint32_t v = ids_of[(size_t)shard * cap + i];
                 const int lo = seg_start[v], hi = seg_start[v + 1];
-                bool through_memory = true;
-                if constexpr (kLds) {
-                    // keys that differ above the depth word: through memory right away (no flag: the
-                    // workgroups that look at the flags run beside this one)
-                    if (hi - lo <= kCapHuge)
-                        through_memory = sort_segment_waves<kGeneralWaves, kCapHuge, 2>(keys, values, v, lo, hi, nullptr, s_w, s_wave_sum);
-                }
-                if (through_memory) sort_segment_general(keys, values, alt_keys, alt_values, lo, hi, s_cnt, s_wave_sum, &s_flag);
+                if (hi - lo <= kCapHuge)
+                    sort_segment_waves<kGeneralWaves, kCapHuge, 2, kWords>(lists, v, lo, hi, s_w, s_wave_sum);
+                else
+                    sort_segment_general<kWords>(lists, alt_keys, alt_values, v, lo, hi, s_cnt, s_wave_sum, &s_flag);
             }
         }
-        return;
-    }
-    const uint32_t first_id = (blockIdx.x - list_blocks) * (uint32_t)kWave;
-    if (tid < kWave) {
-        const uint32_t v = first_id + (uint32_t)lane;
-        bool take = false;
-        if (v < ids) {
-            const int len = seg_start[v + 1] - seg_start[v];
-            take = len > 1 && len <= min_len && ((seg_flags[v >> 5] >> (v & 31)) & 1u);
-        }
-        const uint64_t m = ballot(take);
-        if (lane == 0) s_match = m;
-    }
-    __syncthreads();
-    for (uint64_t todo = s_match; todo; todo &= todo - 1) {
-        const uint32_t v = first_id + (uint32_t)(__ffsll((long long)todo) - 1);
-        sort_segment_general(keys, values, alt_keys, alt_values, seg_start[v], seg_start[v + 1], s_cnt, s_wave_sum, &s_flag);
     }
 }
-
-
 
 } // namespace
 } // namespace fgs
@@ -1450,55 +1510,65 @@ extern "C" int fgs_sort_gaussian(int num_rendered,
     uint32_t* hist = (uint32_t*)(list_sorting_space + ws.hist);
     uint32_t* chunk_sums = (uint32_t*)(list_sorting_space + ws.chunk_sums);
 
-    // The table of segment starts (with it the flag words and the lists of the longer segments)
+    uint32_t* marks = (uint32_t*)(list_sorting_space + ws.marks);
+
+    // The table of segment starts (with it the lists of the longer segments)
     // exists up to kMaxTableIds tile ids.  The last partition pass writes it when there are at
     // most two passes: with more, one workgroup could own 2^18 and more entries of a sparse frame.
     const uint32_t ids = 1u << tile_bits;
     int* seg_start = nullptr;
-    uint32_t* seg_flags = nullptr;
     uint32_t* seg_counts = nullptr;
-    if (n > 1 && ids <= kMaxTableIds) {
+    if (ids <= kMaxTableIds) {
         seg_start = (int*)(list_sorting_space + ws.seg_start);
-        seg_flags = (uint32_t*)(list_sorting_space + ws.seg_flags);
         seg_counts = (uint32_t*)(list_sorting_space + ws.seg_lists);
     }
-    bool table_by_scatter = false;
-    const bool one_wave_launch = seg_start && ids <= kOneLaunchIds;
-    const uint32_t flag_words = (ids + 31) / 32;
+    const bool words = tile_bits <= kWordsMaxTileBits;              // at most two passes
 
     // 1. stable partition by tile id, least significant tile digit first
     auto partition = [&](auto shape) {
         using Shape = decltype(shape);
+        using Next = NextDigit<Shape>;
         const PassGrid g = pass_grid(n, Shape::kTile);
         const bool small = g.tiles * Shape::kBinsP <= kMostRowWords;     // the scatter workgroups add up the histogram rows themselves
         const int passes = (tile_bits + Shape::kBits - 1) / Shape::kBits;
-        table_by_scatter = seg_start && passes <= 2;
         const uint64_t* src_k = gaussian_keys_unsorted;
-        const uint32_t* src_v = gaussian_values_unsorted;
+        const void* src_v = gaussian_values_unsorted;
         for (int p = 0; p < passes; p++) {
             const bool to_sorted = ((passes - p) & 1) != 0;      // the last pass lands in the caller's sorted buffers
             uint64_t* dst_k = to_sorted ? gaussian_keys_sorted : alt_keys;
             uint32_t* dst_v = to_sorted ? gaussian_values_sorted : alt_values;
-            const int shift = 32 + Shape::kBits * p;
             const int nbits = tile_bits - Shape::kBits * p < Shape::kBits ? tile_bits - Shape::kBits * p : Shape::kBits;
-            const bool last = p == passes - 1;
-            if (small) {
-                hipLaunchKernelGGL((count_kernel<Shape>), dim3(g.tiles), dim3(kSortBlock), 0, st, src_k, n, shift, nbits, hist,
-                                   last ? seg_flags : nullptr, flag_words, seg_counts);
-            } else {
-                const int groups = g.chunk < kCountGroups ? g.chunk : kCountGroups;
-                hipLaunchKernelGGL((count_chunk_kernel<Shape>), dim3(g.chunks), dim3(groups * kSortBlock), 0, st,
-                                   src_k, n, shift, nbits, hist, g.tiles, g.chunk, chunk_sums,
-                                   last ? seg_flags : nullptr, flag_words, seg_counts);
-                hipLaunchKernelGGL((offsets_kernel<Shape>), dim3(g.chunks), dim3(g.chunks > 16 ? kOffsetThreads : Shape::kBinsP), 0, st,
-                                   hist, g.tiles, g.chunk, chunk_sums, g.chunks);
-            }
-            if (last && table_by_scatter)
-                hipLaunchKernelGGL((scatter_kernel<Shape, true>), dim3(g.tiles), dim3(Shape::kThreads), 0, st,
-                                   src_k, src_v, dst_k, dst_v, n, shift, nbits, hist, small ? g.tiles : 0, seg_start);
-            else
-                hipLaunchKernelGGL((scatter_kernel<Shape, false>), dim3(g.tiles), dim3(Shape::kThreads), 0, st,
-                                   src_k, src_v, dst_k, dst_v, n, shift, nbits, hist, small ? g.tiles : 0, (int*)nullptr);
+            const bool first = p == 0, last = p == passes - 1;
+            const bool from_words = words && !first;
+            const int shift = from_words ? 0 : Shape::kBits * p;            // of the digit in what is read
+            uint32_t* const beyond = first ? marks + kMarkBeyond : nullptr;
+            uint32_t* const clear = last ? seg_counts : nullptr;
+            auto count = [&](auto* in) {
+                using In = std::remove_cv_t<std::remove_pointer_t<decltype(in)>>;
+                if (small) {
+                    hipLaunchKernelGGL((count_kernel<Shape, In>), dim3(g.tiles), dim3(kSortBlock), 0, st,
+                                       in, n, shift, nbits, hist, ~tile_mask, beyond, clear);
+                } else {
+                    const int groups = g.chunk < kCountGroups ? g.chunk : kCountGroups;
+                    hipLaunchKernelGGL((count_chunk_kernel<Shape, In>), dim3(g.chunks), dim3(groups * kSortBlock), 0, st,
+                                       in, n, shift, nbits, hist, g.tiles, g.chunk, chunk_sums, ~tile_mask, beyond, clear);
+                    hipLaunchKernelGGL((offsets_kernel<Shape>), dim3(g.chunks), dim3(g.chunks > 16 ? kOffsetThreads : Shape::kBinsP), 0, st,
+                                       hist, g.tiles, g.chunk, chunk_sums, g.chunks, first ? marks : nullptr);
+                }
+            };
+            if (from_words) count((const Next*)src_v);
+            else count(src_k);
+            const uint32_t* const beyond_at = marks + (small ? kMarkBeyond : kMarkByIndex);
+            const int beyond_rows = !first ? 0 : small ? g.tiles : 1;
+#define FGS_SCATTER(IN, OUT)                                                                                                \
+            hipLaunchKernelGGL((scatter_kernel<Shape, Form::IN, Form::OUT>), dim3(g.tiles), dim3(Shape::kThreads), 0, st,   \
+                               src_k, src_v, dst_k, (void*)dst_v, n, shift, nbits, last && passes == 2 ? Shape::kBits : 0,  \
+                               (const uint32_t*)hist, small ? g.tiles : 0, marks, beyond_at, beyond_rows, seg_start)
+            if (!words) FGS_SCATTER(kPairs, kPairs);
+            else if (first && last) FGS_SCATTER(kPairs, kSegments);
+            else if (first) FGS_SCATTER(kPairs, kWords);
+            else FGS_SCATTER(kWords, kSegments);
+#undef FGS_SCATTER
             src_k = dst_k;
             src_v = dst_v;
         }
@@ -1514,92 +1584,86 @@ extern "C" int fgs_sort_gaussian(int num_rendered,
     }
 
     // 2. every tile id's segment by depth, in place in the sorted buffers
-    if (n > 1) {
-        if (seg_start && !table_by_scatter) {
-            const unsigned blocks = (unsigned)(((size_t)n + 256 * kStartsPerThread - 1) / (256 * kStartsPerThread));
-            hipLaunchKernelGGL(segment_starts_kernel, dim3(blocks), dim3(256), 0, st,
-                               (const uint64_t*)gaussian_keys_sorted, n, tile_mask, ids, seg_start, seg_flags, flag_words, seg_counts);
-        }
-        uint64_t* ks = gaussian_keys_sorted;
-        uint32_t* vs = gaussian_values_sorted;
-        seg_counts = (uint32_t*)(list_sorting_space + ws.seg_lists);
-        const uint32_t cap_small = (uint32_t)(n / 512 + 2), cap_medium = (uint32_t)(n / 1024 + 2), cap_large = (uint32_t)(n / 4096 + 2),
-                       cap_long = (uint32_t)(n / 8192 + 2);
-        uint32_t* list_small = seg_counts + 128;
-        uint32_t* list_medium = list_small + (size_t)kListShards * cap_small;
-        uint32_t* list_large = list_medium + (size_t)kListShards * cap_medium;
-        uint32_t* list_long = list_large + (size_t)kListShards * cap_large;
-        const uint32_t* no_list = nullptr;
-        // grids of the list-driven launches: a multiple of kListShards, enough for every listed segment
-        // (the limits are several times what is resident at once: a workgroup takes every
-        // (grid / kListShards)-th segment of its shard, and the shards are not equally long)
-        auto list_grid = [](unsigned most, unsigned limit) {
-            const unsigned g = most < limit ? most : limit;
-            return (g + kListShards - 1) / kListShards * kListShards;
-        };
-#define FGS_SEGMENT_CLASS(WAVES, CAP, LEAST, MINLEN, GRID, LIST, COUNT, LISTCAP)                                \
-        hipLaunchKernelGGL((segment_sort_kernel<WAVES, CAP, LEAST>), dim3(GRID), dim3((WAVES) * kWave), 0, st,  \
-                           ks, vs, n, tile_mask, MINLEN, (const int*)seg_start, seg_flags,               \
-                           (const uint32_t*)(LIST), (const uint32_t*)(COUNT), LISTCAP)
-        // Up to 512 pairs: one wave, bitonic network in registers; one tile id per wave (neighbouring
+    const Lists lists = { gaussian_keys_sorted, gaussian_values_sorted, gaussian_keys_unsorted, gaussian_values_unsorted, marks + kMarkByIndex };
+    if (seg_start && !words) {
+        const unsigned blocks = (unsigned)(((size_t)n + 256 * kStartsPerThread - 1) / (256 * kStartsPerThread));
+        hipLaunchKernelGGL(segment_starts_kernel, dim3(blocks), dim3(256), 0, st,
+                           (const uint64_t*)gaussian_keys_sorted, n, tile_mask, ids, seg_start, seg_counts);
+    }
+    seg_counts = (uint32_t*)(list_sorting_space + ws.seg_lists);
+    const uint32_t cap_small = (uint32_t)(n / 512 + 2), cap_medium = (uint32_t)(n / 1024 + 2), cap_large = (uint32_t)(n / 4096 + 2),
+                   cap_long = (uint32_t)(n / 8192 + 2);
+    uint32_t* list_small = seg_counts + 128;
+    uint32_t* list_medium = list_small + (size_t)kListShards * cap_small;
+    uint32_t* list_large = list_medium + (size_t)kListShards * cap_medium;
+    uint32_t* list_long = list_large + (size_t)kListShards * cap_large;
+    const uint32_t* no_list = nullptr;
+    // grids of the list-driven launches: a multiple of kListShards, enough for every listed segment
+    // (the limits are several times what is resident at once: a workgroup takes every
+    // (grid / kListShards)-th segment of its shard, and the shards are not equally long)
+    auto list_grid = [](unsigned most, unsigned limit) {
+        const unsigned g = most < limit ? most : limit;
+        return (g + kListShards - 1) / kListShards * kListShards;
+    };
+#define FGS_SEGMENT_WAVE(CAP, WORDS)                                                                          \
+    hipLaunchKernelGGL((segment_sort_wave_kernel<(CAP) / kWave, WORDS>), dim3(ids), dim3(kWave),              \
+                       0, st, lists, n, tile_mask, (const int*)seg_start,                                     \
+                       kCapSmall, kCapMedium, kCapLarge, seg_counts, list_small, list_medium,                 \
+                       list_large, list_long, cap_small, cap_medium, cap_large, cap_long)
+#define FGS_SEGMENT_CLASS(WAVES, CAP, LEAST, WORDS, MINLEN, GRID, LIST, COUNT, LISTCAP)                         \
+    hipLaunchKernelGGL((segment_sort_kernel<WAVES, CAP, LEAST, WORDS>), dim3(GRID), dim3((WAVES) * kWave), 0, st,  \
+                       lists, n, tile_mask, MINLEN, (const int*)seg_start,                                    \
+                       (const uint32_t*)(LIST), (const uint32_t*)(COUNT), LISTCAP)
+#define FGS_SEGMENT_GENERAL(TABLE, WORDS, GRID, FIRST)                                                                  \
+    hipLaunchKernelGGL((segment_sort_general_kernel<TABLE, WORDS>), dim3(GRID), dim3(kGeneralWaves * kWave), 0, st,     \
+                       lists, alt_keys, alt_values, n, tile_mask, kCapLarge, (const int*)seg_start,                    \
+                       (const uint32_t*)list_long, (const uint32_t*)seg_counts, cap_long,                              \
+                       (const uint32_t*)list_medium, cap_medium, (const uint32_t*)list_large, cap_large, FIRST)
+    // A short list of pairs has few segments of more than 1024 pairs, or none: there the one
+    // launch below takes those classes too (720p, 0.2M pairs: two launches less).
+    const bool merged_tail = seg_start && n <= kMergedTailMax;
+    const bool merged_large = seg_start && !merged_tail && n <= kMergedLargeMax;
+    const int smallest = merged_tail ? kCapSmall : merged_large ? kCapMedium : kCapLarge;
+    const unsigned tail_blocks = n > smallest ? list_grid((unsigned)(n / (smallest + 1) + 1), n > kMergedLargeMax ? 2048u : 256u) : 0u;
+    const int first_class = merged_tail ? 1 : merged_large ? 2 : 3;
+    const unsigned medium_blocks = list_grid((unsigned)(n / (kCapSmall + 1) + 1), 4096u), large_blocks = list_grid((unsigned)(n / (kCapMedium + 1) + 1), 1024u);
+    if (words) {
+        // Up to 1024 pairs: one wave, bitonic network in registers; one tile id per wave (neighbouring
         // tiles tend to be equally busy, so a wave that took several of them would become the tail
-        // of the launch).  With a table the launch also lists the longer segments.
-        // Up to kOneLaunchIds tile ids the first launch takes the segments of 513..1024 pairs too,
-        // with 16 register slots: on a frame of few tiles there are few of them, about one wave per
-        // SIMD, and a launch of their own lasts as long as one such sort (1080p: -15 us, 4K: -8 us).
-        // While the 16-slot code needed 145 registers, the launch over the 131 072 ids of an 8K
-        // frame, most of them under 128 pairs, lost more to the three waves per SIMD than the
-        // second launch cost (+40 us); at 75 registers it wins there as well (-12 us, and -0.28 ms
-        // on the 8K frame of 109M pairs).
-        if (one_wave_launch)
-            hipLaunchKernelGGL((segment_sort_wave_kernel<kCapSmall / kWave, 1>), dim3(ids), dim3(kWave),
-                               0, st, ks, vs, n, tile_mask, 1, ids, (const int*)seg_start, seg_flags,
-                               kCapSmall, kCapMedium, kCapLarge, seg_counts, list_small, list_medium,
-                               list_large, list_long, cap_small, cap_medium, cap_large, cap_long);
-        else
-            hipLaunchKernelGGL((segment_sort_wave_kernel<kCapTiny / kWave, 1>), dim3(ids), dim3(kWave),
-                               0, st, ks, vs, n, tile_mask, 1, ids, (const int*)seg_start, seg_flags,
-                               kCapSmall, kCapMedium, kCapLarge, seg_counts, seg_start ? list_small : nullptr, list_medium,
-                               list_large, list_long, cap_small, cap_medium, cap_large, cap_long);
-        // A short list of pairs has few segments of more than 1024 pairs, or none: there the one
-        // launch below takes those classes too (720p, 0.2M pairs: two launches less).
-        const bool merged_tail = seg_start && n <= kMergedTailMax;
-        const bool merged_large = seg_start && !merged_tail && n <= kMergedLargeMax;
+        // of the launch).  The launch also lists the longer segments.  Segments of 513..1024 pairs in a launch of
+        // their own last as long as one such sort on a frame of few tiles, which has about one per SIMD (1080p: -15 us, 4K:
+        // -8 us, 8K -12 us without it, and -0.28 ms on the 8K frame of 109M pairs).
+        FGS_SEGMENT_WAVE(kCapSmall, true);
+        if (n > kCapSmall && !merged_tail) {
+            FGS_SEGMENT_CLASS(4, kCapMedium, 8, true, kCapSmall, medium_blocks, list_medium, seg_counts + kListShards, cap_medium);
+            if (n > kCapMedium && !merged_large)
+                FGS_SEGMENT_CLASS(8, kCapLarge, 16, true, kCapMedium, large_blocks, list_large, seg_counts + 2 * kListShards, cap_large);
+        }
+        // longer segments from their list, one workgroup per segment
+        if (tail_blocks) FGS_SEGMENT_GENERAL(true, true, tail_blocks, first_class);
+    } else {
+        FGS_SEGMENT_WAVE(kCapTiny, false);
         if (seg_start) {
-            if (n > kCapTiny && !one_wave_launch)       // 513..1024: the same network over 16 register slots, from the lists
-                hipLaunchKernelGGL((segment_sort_wave_list_kernel<kCapSmall / kWave>),
+            if (n > kCapTiny)       // 513..1024: the same network over 16 register slots, from the lists
+                hipLaunchKernelGGL((segment_sort_wave_list_kernel<kCapSmall / kWave, false>),
                                    dim3(list_grid((unsigned)(n / (kCapTiny + 1) + 1), 8192u)),
-                                   dim3(kWave), 0, st, ks, vs, (const int*)seg_start, seg_flags,
+                                   dim3(kWave), 0, st, lists, (const int*)seg_start,
                                    (const uint32_t*)list_small, (const uint32_t*)seg_counts, cap_small);
             if (n > kCapSmall && !merged_tail) {
-                FGS_SEGMENT_CLASS(4, kCapMedium, 8, kCapSmall, list_grid((unsigned)(n / (kCapSmall + 1) + 1), 4096u),
-                                  list_medium, seg_counts + kListShards, cap_medium);
+                FGS_SEGMENT_CLASS(4, kCapMedium, 8, false, kCapSmall, medium_blocks, list_medium, seg_counts + kListShards, cap_medium);
                 if (n > kCapMedium && !merged_large)
-                    FGS_SEGMENT_CLASS(8, kCapLarge, 16, kCapMedium, list_grid((unsigned)(n / (kCapMedium + 1) + 1), 1024u),
-                                      list_large, seg_counts + 2 * kListShards, cap_large);
+                    FGS_SEGMENT_CLASS(8, kCapLarge, 16, false, kCapMedium, large_blocks, list_large, seg_counts + 2 * kListShards, cap_large);
             }
+            if (tail_blocks) FGS_SEGMENT_GENERAL(true, false, tail_blocks, first_class);
         } else {
-            if (n > kCapTiny) FGS_SEGMENT_CLASS(4, kCapSmall, 4, kCapTiny, ids, no_list, no_list, 0u);
-            if (n > kCapSmall) FGS_SEGMENT_CLASS(4, kCapMedium, 8, kCapSmall, ids, no_list, no_list, 0u);
-            if (n > kCapMedium) FGS_SEGMENT_CLASS(8, kCapLarge, 16, kCapMedium, ids, no_list, no_list, 0u);
-        }
-#undef FGS_SEGMENT_CLASS
-        // longer segments from their list, one workgroup per segment; behind them the shorter ones that were flagged
-        if (seg_start) {
-            const int smallest = merged_tail ? kCapSmall : merged_large ? kCapMedium : kCapLarge;
-            const unsigned blocks = n > smallest ? list_grid((unsigned)(n / (smallest + 1) + 1), n > kMergedLargeMax ? 2048u : 256u) : 0u;
-            hipLaunchKernelGGL(segment_sort_general_kernel<true>, dim3(blocks + (ids + kWave - 1) / kWave),
-                               dim3(kGeneralWaves * kWave), 0, st, ks, vs, alt_keys, alt_values, n, tile_mask, kCapLarge, ids,
-                               (const int*)seg_start, (const uint32_t*)seg_flags,
-                               (const uint32_t*)list_long, (const uint32_t*)seg_counts, cap_long, blocks,
-                               (const uint32_t*)list_medium, cap_medium, (const uint32_t*)list_large, cap_large,
-                               merged_tail ? 1 : merged_large ? 2 : 3);
-        } else {
-            hipLaunchKernelGGL(segment_sort_general_kernel<false>, dim3(ids),
-                               dim3(kGeneralWaves * kWave), 0, st, ks, vs, alt_keys, alt_values, n, tile_mask, kCapLarge, ids,
-                               (const int*)seg_start, (const uint32_t*)seg_flags,
-                               no_list, no_list, 0u, 0u, no_list, 0u, no_list, 0u, 0);
+            if (n > kCapTiny) FGS_SEGMENT_CLASS(4, kCapSmall, 4, false, kCapTiny, ids, no_list, no_list, 0u);
+            if (n > kCapSmall) FGS_SEGMENT_CLASS(4, kCapMedium, 8, false, kCapSmall, ids, no_list, no_list, 0u);
+            if (n > kCapMedium) FGS_SEGMENT_CLASS(8, kCapLarge, 16, false, kCapMedium, ids, no_list, no_list, 0u);
+            if (n > kCapLarge) FGS_SEGMENT_GENERAL(false, false, ids, 0);
         }
     }
+#undef FGS_SEGMENT_WAVE
+#undef FGS_SEGMENT_CLASS
+#undef FGS_SEGMENT_GENERAL
     return check_hip(hipGetLastError(), "sort launch");
 }

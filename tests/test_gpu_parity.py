@@ -1286,7 +1286,7 @@ def test_sort_around_the_list_lengths_where_the_partition_blocks_change(n, W, H)
 
 def test_sort_bits_above_the_range_stay_with_their_pair():
     """Bits above 32 + bit_length(tiles) are outside the sorted range (sort.cu:34-39) but travel
-    with the key; segments whose keys differ there take the general path."""
+    with the key."""
     rng = np.random.default_rng(77)
     W, H = 640, 480                                   # 1200 tiles -> 11 tile bits
     n = 60000
@@ -1309,6 +1309,27 @@ def test_sort_bits_above_the_range_stay_with_their_pair():
     junk = rng.integers(0, 1 << 10, n).astype(np.uint32)
     junk[30000:] = 0
     _sort_case(tile, depth, W, H, junk=junk, seed=2)
+
+
+@pytest.mark.parametrize("W,H,n", [(64, 64, 1), (64, 64, 3000), (640, 480, 5000), (1920, 1080, 700_000), (3840, 2160, 2_200_000),
+                                   (7680, 4320, 900), (7680, 4320, 500_000), (8208, 8208, 1), (8208, 8208, 50_000),
+                                   (16400, 16400, 20_000)])
+def test_sort_one_key_with_bits_above_the_range(W, H, n):
+    """A single key has bits above the sorted range: then every pair's index is carried through the partition in place of its
+    value and the pairs are fetched from the input at the end.  One, two and three passes, with and without the
+    launch that turns histogram rows into starts, with the table of segment starts and without, tiles of one pair and of
+    more than 16 384, values that ascend and values that do not, the key in the first block and in the last."""
+    rng = np.random.default_rng(n)
+    tiles = ((W + 15) // 16) * ((H + 15) // 16)
+    for at in (0, n - 1):
+        tile = rng.integers(0, tiles, n).astype(np.uint32)
+        tile[:n // 3] = tiles - 1
+        tile[n // 2:n // 2 + 700] = 0
+        depth = rng.uniform(0.2, 90.0, n).astype(np.float32).view(np.uint32)
+        depth[::5] = depth[0]
+        junk = np.zeros(n, np.uint32)
+        junk[at] = 1
+        _sort_case(tile, depth, W, H, junk=junk, seed=n, ascending=n > 3 and at == 0)
 
 
 @pytest.mark.parametrize("W,H,n", [(16, 16, 5000), (256, 16, 9000), (160, 128, 70_000), (3840, 2160, 300),
