@@ -18,9 +18,9 @@
 //  2. Sort every tile's segment by the 32 depth bits without touching memory in between: the
 //     last scatter pass also tabulates where each tile id's segment begins (with more than two
 //     passes `segment_starts_kernel` does, from the sorted keys), then segments are handled by
-//     size class.  Up to 1024 pairs one wave holds the segment in registers as such
-//     words (depth << 16 | position where the values of a segment do not ascend) and runs
-//     a bitonic network on them (the result is that of a stable sort by depth); lane exchanges inside a row of 16 lanes are
+//     size class.  Up to 1024 pairs one wave holds a 32-bit word per pair, the upper bits of its depth in front of its place,
+//     in registers and runs a merging network on them, then fetches the pairs in that order and puts the few that the
+//     bits left out tell apart in order (the result is that of a stable sort by depth); lane exchanges inside a row of 16 lanes are
 //     data-parallel-primitive moves.  Up to 4096 (4 waves), 8192 (8) and 16384 pairs (16) every wave
 //     of a workgroup sorts its part like that and the parts are merged, the steps between two waves
 //     through LDS.  Longer segments go
@@ -33,6 +33,7 @@
 
 #include <algorithm>
 #include <type_traits>
+#include <utility>
 
 namespace fgs {
 namespace {
@@ -710,6 +711,7 @@ __global__ __launch_bounds__(Shape::kThreads) void scatter_kernel(
 // size classes of the segments: pairs per segment
 constexpr int kCapTiny = 512, kCapSmall = 1024, kCapMedium = 4096, kCapLarge = 8192;
 constexpr int kMergedLargeMax = 1 << 24;     // up to this many pairs the last launch also takes the class of 4097 .. 8192 pairs
+constexpr int kManyPairs = 1 << 26;
 constexpr int kMergedTailMax = 1 << 19;      // up to this many pairs the last launch also takes the classes of 1025 .. 8192 pairs
 
 // First index in [0, n) whose tile field is >= v (n if none), found by the whole wave probing 64
@@ -860,122 +862,132 @@ __device__ __forceinline__ bool counting_pass(const uint64_t* src_k, const uint3
     return true;
 }
 
-// x of lane (l ^ kJ).  Within a row of 16 lanes the exchange is a data-parallel-primitive move
-// (no LDS traffic); across rows it goes through the lane crossbar.
-template <int kJ>
-__device__ __forceinline__ uint32_t from_lane_xor(uint32_t x)
+// x of lane (l ^ kMask).  Within a row of 16 lanes most exchanges are one data-parallel-primitive move; the others go
+// through the lane crossbar, which is idle otherwise: two moves in its place cost the vector unit more than the crossbar delays.
+template <int kMask>
+__device__ __forceinline__ uint32_t from_lane_xor(uint32_t x, int lane)
 {
-    constexpr int kQuadXor1 = 0xB1, kQuadXor2 = 0x4E, kQuadReverse = 0x1B, kRowHalfMirror = 0x141, kRowRor8 = 0x128;
-    if (kJ == 1) return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, kQuadXor1, 0xf, 0xf, true);
-    if (kJ == 2) return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, kQuadXor2, 0xf, 0xf, true);
-    if (kJ == 4) {      // reverse the 8 lanes, then each quad: lane l reads lane l ^ 4
-        const int t = __builtin_amdgcn_mov_dpp((int)x, kRowHalfMirror, 0xf, 0xf, true);
-        return (uint32_t)__builtin_amdgcn_mov_dpp(t, kQuadReverse, 0xf, 0xf, true);
+    constexpr int kQuadXor1 = 0xB1, kQuadXor2 = 0x4E, kQuadReverse = 0x1B, kRowHalfMirror = 0x141, kRowMirror = 0x140, kRowRor8 = 0x128;
+    constexpr int kMove = kMask == 1 ? kQuadXor1 : kMask == 2 ? kQuadXor2 : kMask == 3 ? kQuadReverse : kMask == 7 ? kRowHalfMirror
+                        : kMask == 8 ? kRowRor8 : kMask == 15 ? kRowMirror : 0;
+    if constexpr (kMove != 0) return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, kMove, 0xf, 0xf, true);
+    else if constexpr (kMask < 32) return (uint32_t)__builtin_amdgcn_ds_swizzle((int)x, kMask << 10 | 0x1f);
+    else return (uint32_t)__builtin_amdgcn_ds_bpermute((lane ^ kMask) * 4, (int)x);
+}
+
+// The smaller word with limit 0, the larger one with limit ~0: one instruction (v_med3_u32), whichever a lane keeps.
+__device__ __forceinline__ uint32_t keep_word(uint32_t a, uint32_t b, uint32_t limit)
+{
+    return max(min(a, b), min(max(a, b), limit));
+}
+
+__device__ __forceinline__ void order_words(uint32_t& a, uint32_t& b)
+{
+    const uint32_t lo = min(a, b), hi = max(a, b);
+    a = lo;
+    b = hi;
+}
+
+// Comparators of Batcher's odd-even merge sort (63 for 16 slots, where a bitonic network has 80).
+template <int kT>
+struct SlotNetwork {
+    int first[kT * kT], second[kT * kT], count;
+    constexpr SlotNetwork() : first(), second(), count(0)
+    {
+        for (int p = 1; p < kT; p *= 2)
+            for (int k = p; k >= 1; k /= 2)
+                for (int j = k % p; j + k < kT; j += 2 * k)
+                    for (int i = 0; i < k && i + j + k < kT; i++)
+                        if ((i + j) / (2 * p) == (i + j + k) / (2 * p)) {
+                            first[count] = i + j;
+                            second[count] = i + j + k;
+                            count++;
+                        }
     }
-    if (kJ == 8) return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, kRowRor8, 0xf, 0xf, true);
-    return (uint32_t)__shfl_xor((int)x, kJ);
+};
+
+template <int kT, int... kI>
+__device__ __forceinline__ void sort_slots_by(uint32_t (&c)[kT], std::integer_sequence<int, kI...>)
+{
+    constexpr SlotNetwork<kT> net;
+    (order_words(c[net.first[kI]], c[net.second[kI]]), ...);
 }
 
-template <int kJ>
-__device__ __forceinline__ uint64_t from_lane_xor64(uint64_t x)
-{
-    return ((uint64_t)from_lane_xor<kJ>((uint32_t)(x >> 32)) << 32) | from_lane_xor<kJ>((uint32_t)x);
-}
-
-// The smaller and the larger of two words taken as doubles.  A positive double orders like its bits, so one
-// instruction takes the place of a 64-bit comparison and two selects (4 cycles of the vector unit
-// against 12); written out because fmin would first quiet signalling NaNs, which the words are not.
-__device__ __forceinline__ uint64_t min_word(uint64_t a, uint64_t b)
-{
-    uint64_t r;
-    asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
-    return r;
-}
-__device__ __forceinline__ uint64_t max_word(uint64_t a, uint64_t b)
-{
-    uint64_t r;
-    asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
-    return r;
-}
-__device__ __forceinline__ void keep_min_negated(uint64_t& a, uint64_t b)       // a = min(a, -b)
-{
-    asm("v_min_f64 %0, %0, -%1" : "+v"(a) : "v"(b));
-}
-
-// Compare distance j < kT, between slots of a lane; k > 0: slots with t & k descend.
 template <int kT>
-__device__ __forceinline__ void compare_slots(uint64_t (&c)[kT], int j, int k)
+__device__ __forceinline__ void sort_slots(uint32_t (&c)[kT])
 {
-#pragma unroll
-    for (int t = 0; t < kT; t++) {
-        if ((t & j) != 0) continue;
-        const int t2 = t | j;
-        const uint64_t lo = min_word(c[t], c[t2]), hi = max_word(c[t], c[t2]);
-        const bool descends = k > 0 && (t & k) != 0;
-        c[t] = descends ? hi : lo;
-        c[t2] = descends ? lo : hi;
-    }
+    constexpr SlotNetwork<kT> net;
+    sort_slots_by<kT>(c, std::make_integer_sequence<int, net.count>());
 }
 
-// Changes the sign a lane's words are held with.
-template <int kT>
-__device__ __forceinline__ void hold(uint64_t (&c)[kT], uint32_t& held, uint32_t sign)
+// One step of a merge across lanes: against the same slot of lane (l ^ kMask) or, kMirrored, the slots in reverse order.
+template <int kMask, bool kMirrored, int kT>
+__device__ __forceinline__ void compare_lanes(uint32_t (&c)[kT], int lane)
 {
+    constexpr int kTop = kMask >= 32 ? 5 : kMask >= 16 ? 4 : kMask >= 8 ? 3 : kMask >= 4 ? 2 : kMask >= 2 ? 1 : 0;
+    const uint32_t limit = (uint32_t)__builtin_amdgcn_sbfe(lane, kTop, 1);          // the upper lane keeps the larger word
+    // (eight slots at a time, with their mirror images: what is in flight stays in few registers)
+    constexpr int kHalf = kT / 2, kGroup = kHalf < 4 ? kHalf : 4;
+    if constexpr (kT == 1) {
+        c[0] = keep_word(c[0], from_lane_xor<kMask>(c[0], lane), limit);
+    } else {
 #pragma unroll
-    for (int t = 0; t < kT; t++) c[t] ^= (uint64_t)(held ^ sign) << 32;
-    held = sign;
-}
-
-// Merges the bitonic runs of width k (k >= kT) of the network below.  run: this lane's sign while its
-// run descends; held: the sign its words are held with, run when this returns.
-template <int kT>
-__device__ __forceinline__ void merge_slots(uint64_t (&c)[kT], int lane, int k, uint32_t run, uint32_t& held)
-{
+        for (int g = 0; g < kHalf; g += kGroup) {
+            uint32_t other[2 * kGroup];
 #pragma unroll
-    for (int jl = kWave / 2; jl > 0; jl >>= 1) {              // lane distances
-        if (jl * kT >= k) continue;
-        hold(c, held, run ^ ((lane & jl) != 0 ? 0x80000000u : 0u));
+            for (int i = 0; i < kGroup; i++) {
+                const int t = g + i, u = kT - 1 - t;
+                other[2 * i] = from_lane_xor<kMask>(c[kMirrored ? u : t], lane);
+                other[2 * i + 1] = from_lane_xor<kMask>(c[kMirrored ? t : u], lane);
+            }
 #pragma unroll
-        for (int t = 0; t < kT; t++) {
-            const uint64_t mine = c[t];
-            const uint64_t other = jl == 1 ? from_lane_xor64<1>(mine) : jl == 2 ? from_lane_xor64<2>(mine)
-                                 : jl == 4 ? from_lane_xor64<4>(mine) : jl == 8 ? from_lane_xor64<8>(mine)
-                                 : jl == 16 ? from_lane_xor64<16>(mine) : from_lane_xor64<32>(mine);
-            keep_min_negated(c[t], other);                    // the other lane holds its words with the other sign
+            for (int i = 0; i < kGroup; i++) {
+                const int t = g + i, u = kT - 1 - t;
+                c[t] = keep_word(c[t], other[2 * i], limit);
+                c[u] = keep_word(c[u], other[2 * i + 1], limit);
+            }
+            __builtin_amdgcn_sched_barrier(0);
         }
     }
-    hold(c, held, run);
-#pragma unroll
-    for (int j = kT / 2; j > 0; j >>= 1) compare_slots(c, j, 0);
 }
 
-// The network over kT register slots of every lane, 64 * kT elements, element i in slot i % kT of
-// lane i / kT.  A compare distance below kT pairs two slots of one lane (registers only); a
-// larger one pairs the same slot of two lanes: 21 of the (log n)(log n + 1)/2 exchange steps
-// cross lanes whatever kT is, where the slot-major layout (element i in lane i % 64) makes it
-// 33 of 36 for 256 elements and 45 of 55 for 1024.  The merge width k runs in a loop; the compare
-// distances j are written out, so the code holds every exchange pattern once whatever the number
-// of stages.
-// The words are positive doubles.  A lane that has to keep the larger of two words, or whose run
-// descends, holds its words negated (one exclusive-or of the sign where that changes): then every
-// step is the smaller word, or the smaller and the larger one of two slots.  Against integer
-// comparisons and selects the launch over the segments of up to 1024 pairs went from 66 to 48 us on a
-// 4K frame of 8.4M pairs, from 46 to 29 at 1080p (1.8M) and from 493 to 363 on 8K with 111M.
+// The steps of a merge whose lanes differ in one bit, from 2^(kFrom) down, as far as the run has them (below `bits`), then those inside a lane.
 template <int kT>
-__device__ __forceinline__ void bitonic_network(uint64_t (&c)[kT], int lane)
+__device__ __forceinline__ void merge_lanes(uint32_t (&c)[kT], int lane, int bits)
 {
-    constexpr int n = kT * kWave;
-    // runs shorter than a lane's slots: the direction is a matter of the slot
+    if (bits > 5) compare_lanes<32, false>(c, lane);
+    if (bits > 4) compare_lanes<16, false>(c, lane);
+    if (bits > 3) compare_lanes<8, false>(c, lane);
+    if (bits > 2) compare_lanes<4, false>(c, lane);
+    if (bits > 1) compare_lanes<2, false>(c, lane);
+    if (bits > 0) compare_lanes<1, false>(c, lane);
 #pragma unroll
-    for (int k = 2; k < kT; k <<= 1)
+    for (int j = kT / 2; j > 0; j >>= 1)
 #pragma unroll
-        for (int j = kT / 2; j > 0; j >>= 1)
-            if (j < k) compare_slots(c, j, k);
-    // longer ones: of the lane
-    uint32_t held = 0;                          // the sign this lane's words are held with
+        for (int t = 0; t < kT; t++)
+            if ((t & j) == 0) order_words(c[t], c[t | j]);
+}
+
+// Sorts 64 * kT words, element i in slot i % kT of lane i / kT: every lane its slots, then runs are merged two by two.  A merge
+// begins with element i of the lower run against element i from the end of the upper one, so that all runs ascend, and
+// goes on with halved distances.  A distance below kT pairs two slots of one lane (registers only); a larger one the same slot of
+// two lanes: 21 steps cross lanes whatever kT is, where the slot-major layout (element i in lane i % 64) makes it 33 of 36 for 256
+// elements and 45 of 55 for 1024.  The merges run in a loop and the distances are written out, so the code holds every exchange
+// pattern once.
+template <int kT>
+__device__ __forceinline__ void sort_words(uint32_t (&c)[kT], int lane)
+{
+    if constexpr (kT > 1) sort_slots(c);
 #pragma unroll 1
-    for (int k = kT > 1 ? kT : 2; k <= n; k <<= 1)
-        merge_slots(c, lane, k, k < n && (lane & (k / kT)) != 0 ? 0x80000000u : 0u, held);   // the last merge ascends everywhere
+    for (int m = 0; m < 6; m++) {               // runs of 2^m lanes
+        if (m == 0) compare_lanes<1, true>(c, lane);
+        else if (m == 1) compare_lanes<3, true>(c, lane);
+        else if (m == 2) compare_lanes<7, true>(c, lane);
+        else if (m == 3) compare_lanes<15, true>(c, lane);
+        else if (m == 4) compare_lanes<31, true>(c, lane);
+        else compare_lanes<63, true>(c, lane);
+        merge_lanes(c, lane, m);
+    }
 }
 
 // A list as the segment sort finds and leaves it.  kWords: keys holds depth << 32 | value words and values nothing yet.
@@ -986,19 +998,6 @@ struct Lists {
     const uint32_t* values_in;
     const uint32_t* by_index;           // one word: not zero where the values are indices into that list
 };
-
-template <bool kWords>
-__device__ __forceinline__ uint64_t word_at(const Lists& l, int i)
-{
-    if (kWords) return l.keys[i];
-    return (l.keys[i] << 32) | l.values[i];
-}
-
-template <bool kWords>
-__device__ __forceinline__ uint32_t value_at(const Lists& l, int i)
-{
-    return kWords ? (uint32_t)l.keys[i] : l.values[i];
-}
 
 // Stores a pair of tile id v.
 __device__ __forceinline__ void store_pair(const Lists& l, bool by_index, int i, uint32_t v, uint64_t word)
@@ -1013,282 +1012,464 @@ __device__ __forceinline__ void store_pair(const Lists& l, bool by_index, int i,
     l.values[i] = value;
 }
 
-// Words of LDS a wave needs to sort up to n pairs with the network: one 64-bit word for every
+// A segment [lo, hi) as buffers with their lengths: a load past the end gives 0, a store there is dropped, without a comparison.
+typedef uint32_t Pair2 __attribute__((ext_vector_type(2)));
+struct Segment {
+    __amdgpu_buffer_rsrc_t keys, values;
+    __device__ __forceinline__ Segment(const Lists& l, int lo, int len)
+    {
+        constexpr int kRawDwords = 0x00020000;      // word 3 of the descriptor: 32-bit data, no swizzle
+        keys = __builtin_amdgcn_make_buffer_rsrc(l.keys + lo, 0, len * 8, kRawDwords);
+        values = __builtin_amdgcn_make_buffer_rsrc(l.values + lo, 0, len * 4, kRawDwords);
+    }
+    template <bool kWords>
+    __device__ __forceinline__ void load(int i, uint32_t& depth, uint32_t& value) const
+    {
+        if constexpr (kWords) {
+            const Pair2 w = __builtin_amdgcn_raw_buffer_load_b64(keys, i * 8, 0, 0);
+            value = w.x;
+            depth = w.y;
+        } else {
+            depth = __builtin_amdgcn_raw_buffer_load_b32(keys, i * 8, 0, 0);
+            value = __builtin_amdgcn_raw_buffer_load_b32(values, i * 4, 0, 0);
+        }
+    }
+    template <bool kWords>
+    __device__ __forceinline__ uint32_t load_depth(int i) const
+    {
+        return __builtin_amdgcn_raw_buffer_load_b32(keys, i * 8 + (kWords ? 4 : 0), 0, 0);
+    }
+    // a pair as load() finds it
+    template <bool kWords>
+    __device__ __forceinline__ void put_back(int i, uint64_t word) const
+    {
+        if constexpr (kWords) {
+            __builtin_amdgcn_raw_buffer_store_b64(Pair2{ (uint32_t)word, (uint32_t)(word >> 32) }, keys, i * 8, 0, 0);
+        } else {
+            __builtin_amdgcn_raw_buffer_store_b32((uint32_t)(word >> 32), keys, i * 8, 0, 0);
+            __builtin_amdgcn_raw_buffer_store_b32((uint32_t)word, values, i * 4, 0, 0);
+        }
+    }
+    __device__ __forceinline__ void store(int i, uint32_t v, uint64_t word) const
+    {
+        const Pair2 key = { (uint32_t)(word >> 32), v };
+        __builtin_amdgcn_raw_buffer_store_b64(key, keys, i * 8, 0, 0);
+        __builtin_amdgcn_raw_buffer_store_b32((uint32_t)word, values, i * 4, 0, 0);
+    }
+};
+
+// Words of LDS a wave needs to sort up to n pairs: a 32-bit word for every pair or one 64-bit word for every
 // second pair (the sorted pairs go through it in two halves), one word of padding after every 16 (lane l puts its kUse consecutive ranks down at once; without
 // the padding the lanes of a wave would all start in the same bank).
 __host__ __device__ constexpr int staging_words(int n) { return n <= 64 ? n + n / 16 : n / 2 + n / 32; }
 __device__ __forceinline__ int staged(int i) { return i + (i >> 4); }
 
-// Sorts the segment [lo, hi) of tile id v with the network over kUse slots per lane, 64 * kUse >= hi - lo.
-// The network orders 64-bit words, depth above and a tie-break below, and it does not matter
-// which slot a word starts in: the loads are the contiguous ones (element t*64 + lane in slot t),
-// the network leaves rank lane*kUse + t in slot t, and the sorted words go through LDS to be
-// stored contiguously again.  Equal depths have to stay in input order.  The pairs of one tile
-// come out of the preprocess in ascending order of their values (Gaussian indices) and their depths are
-// positive floats: then the value itself is the tie-break, the sorted word is the pair, and the word
-// is a positive finite double (values that are indices ascend as well).  A segment whose values do not ascend, or with a depth word from
-// 0x7ff00000 up, carries depth << 16 | position instead (a small positive double whatever the depth)
-// and looks its values up afterwards.
-constexpr uint64_t kLastWord = 0x7fefffffffffffffull;       // the largest finite double
-
-template <int kUse, bool kWords>
-__device__ __forceinline__ void sort_segment_bitonic_of(const Lists& lists, uint32_t v, int lo, int hi, uint64_t* s_w)
+// (two 32-bit words: as one of 64 bits the pairs of all slots would have to sit in neighbouring registers)
+__device__ __forceinline__ void stage(uint64_t* at, uint32_t depth, uint32_t value)
 {
+    ((uint32_t*)at)[0] = value;
+    ((uint32_t*)at)[1] = depth;
+}
+
+__host__ __device__ constexpr int log2_of(int n) { return n <= 1 ? 0 : 1 + log2_of(n / 2); }
+
+__device__ __forceinline__ uint32_t wave_least(uint32_t x)
+{
+    constexpr int kRowShr1 = 0x111, kRowShr2 = 0x112, kRowShr4 = 0x114, kRowShr8 = 0x118, kRowBcast15 = 0x142, kRowBcast31 = 0x143;
+    x = min(x, (uint32_t)__builtin_amdgcn_update_dpp(~0, (int)x, kRowShr1, 0xf, 0xf, false));
+    x = min(x, (uint32_t)__builtin_amdgcn_update_dpp(~0, (int)x, kRowShr2, 0xf, 0xf, false));
+    x = min(x, (uint32_t)__builtin_amdgcn_update_dpp(~0, (int)x, kRowShr4, 0xf, 0xf, false));
+    x = min(x, (uint32_t)__builtin_amdgcn_update_dpp(~0, (int)x, kRowShr8, 0xf, 0xf, false));
+    x = min(x, (uint32_t)__builtin_amdgcn_update_dpp(~0, (int)x, kRowBcast15, 0xa, 0xf, false));
+    x = min(x, (uint32_t)__builtin_amdgcn_update_dpp(~0, (int)x, kRowBcast31, 0xc, 0xf, false));
+    return (uint32_t)__builtin_amdgcn_readlane((int)x, kWave - 1);
+}
+__device__ __forceinline__ uint32_t wave_most(uint32_t x) { return ~wave_least(~x); }
+
+// How the words of a segment are made.  The network orders 32-bit words: the depth above the segment's least one, without the low
+// `shift` bits that do not fit, in front of the pair's place in the segment, which keeps equal depths in input order and tells where the
+// pair's depth and value are fetched from afterwards.  64-bit words of depth and value (min and max of doubles) took four
+// instructions per word for a step across lanes, where these take two, twice the registers and twice the LDS between waves.
+// Where bits were left out (depths that span more than 2^22 of their units for 1024 pairs, i.e. more than a few octaves of
+// distances apart: most segments) pairs that agree in the others, a few in a thousand, can stand in the wrong order:
+// neighbours are exchanged until none does.  A segment that kRepairs rounds of that leave unsorted is sorted by the bits left
+// out and then, from that order, by the others.
+// (The bits that fit: 32 - log2 of the capacity; the shift is at most log2 of the capacity, so two such sorts cover every depth.)
+struct WordBits {
+    uint32_t least, range;
+    int shift, stage;
+    template <int kPlace>
+    __device__ __forceinline__ void span(uint32_t lo, uint32_t hi)
+    {
+        least = (uint32_t)__builtin_amdgcn_readfirstlane((int)lo);
+        range = (uint32_t)__builtin_amdgcn_readfirstlane((int)hi) - least;
+        shift = max(0, kPlace - __builtin_clz(range | 1u));
+    }
+    __device__ __forceinline__ bool complete() const { return shift == 0 || stage == 2; }
+    // stage 0 and 2: the bits from `shift` up; 1: those below
+    template <int kPlace>
+    __device__ __forceinline__ uint32_t word(uint32_t depth, bool valid, uint32_t place) const
+    {
+        const uint32_t above = valid ? depth - least : stage == 1 ? ~0u : range;         // (a place past the end sorts behind every pair)
+        return __builtin_amdgcn_ubfe(above, stage == 1 ? 0 : shift, stage == 1 ? shift : 32 - kPlace) << kPlace | place;
+    }
+};
+constexpr int kRepairs = 8;
+
+// Exchanges neighbours whose depths descend, ranks lane * kT + t: slots 0 and 1, 2 and 3, ... (first 0) or 1 and 2, 3 and 4, ...
+template <int kT>
+__device__ __forceinline__ void exchange_slots(uint32_t (&depth)[kT], uint32_t (&value)[kT], int first)
+{
+#pragma unroll
+    for (int t = 0; t + 1 < kT; t++) {
+        if (t % 2 != first) continue;
+        const bool swap = depth[t] > depth[t + 1];
+        const uint32_t v = value[t];
+        order_words(depth[t], depth[t + 1]);
+        value[t] = swap ? value[t + 1] : v;
+        value[t + 1] = swap ? v : value[t + 1];
+        __builtin_amdgcn_sched_barrier(0);      // one pair after the other: a copy of all of them would set the registers of the kernel
+    }
+}
+
+// The last slot of every lane against the first of the next one; what stands in front of lane 0 and behind lane 63 is given.
+template <int kT>
+__device__ __forceinline__ void exchange_ends(uint32_t (&depth)[kT], uint32_t (&value)[kT], int lane,
+                                              uint32_t depth_before, uint32_t value_before, uint32_t depth_behind, uint32_t value_behind)
+{
+    static_assert(kT >= 2, "a slot for either end of a lane");
+    uint32_t db = (uint32_t)__shfl_up((int)depth[kT - 1], 1), vb = (uint32_t)__shfl_up((int)value[kT - 1], 1);
+    uint32_t dn = (uint32_t)__shfl_down((int)depth[0], 1), vn = (uint32_t)__shfl_down((int)value[0], 1);
+    if (lane == 0) { db = depth_before; vb = value_before; }
+    if (lane == kWave - 1) { dn = depth_behind; vn = value_behind; }
+    value[0] = db > depth[0] ? vb : value[0];
+    depth[0] = max(db, depth[0]);
+    value[kT - 1] = depth[kT - 1] > dn ? vn : value[kT - 1];
+    depth[kT - 1] = min(dn, depth[kT - 1]);
+}
+
+// Whether any depth of the wave is larger than the next one; behind: the depth behind lane 63.
+template <int kT>
+__device__ __forceinline__ bool descends(const uint32_t (&depth)[kT], int lane, uint32_t behind)
+{
+    uint32_t next = (uint32_t)__shfl_down((int)depth[0], 1);
+    if (lane == kWave - 1) next = behind;
+    bool any = depth[kT - 1] > next;
+#pragma unroll
+    for (int t = 0; t + 1 < kT; t++) any |= depth[t] > depth[t + 1];
+    return ballot(any) != 0;
+}
+
+// Sorts the segment [lo, hi) of tile id v with the network over kUse slots per lane, 64 * kUse >= hi - lo.
+// The network does not care which slot a word starts in: the loads are the contiguous ones (element t*64 + lane in slot t),
+// the network leaves rank lane*kUse + t in slot t, depths and values are fetched from LDS by the place in the word, one
+// after the other through the same space, and the sorted pairs go through LDS to be stored contiguously again.
+template <int kUse, bool kWords>
+__device__ __forceinline__ void sort_segment_wave_of(const Lists& lists, uint32_t v, int lo, int hi, uint64_t* s_w)
+{
+    constexpr int kCap = kUse * kWave, kPlace = log2_of(kCap);
+    uint32_t* const s_one = (uint32_t*)s_w;
     // The lane number is made opaque here and again behind the network: otherwise every index and
     // address derived from it, for every width of the network, is computed once in front of the loop
-    // over the segments and kept in registers through all of it (80 registers of a 16-slot network).
+    // over the segments and kept in registers through all of it.
     int lane = threadIdx.x & (kWave - 1);
     asm volatile("" : "+v"(lane));
     const int len = hi - lo;
-    uint64_t c[kUse];
-    // Every load is issued before the first one is looked at (nothing but the load stands under
-    // the condition: a use in there would be waited for before the next slot's load goes out).  A
-    // slot past the end of the segment holds the largest finite double and sorts behind every pair.
+    const Segment segment(lists, lo, len);
+    const bool by_index = *lists.by_index != 0;
+    constexpr int kRounds = kUse >= 2 ? 2 : 1, kHalf = kCap / kRounds;
+    WordBits bits;
+    bits.stage = 0;
+#pragma unroll 1
+    for (;;) {
+        asm volatile("" : "+v"(lane));
+        uint32_t depth[kUse], value[kUse], c[kUse];
 #pragma unroll
-    for (int t = 0; t < kUse; t++) {
-        c[t] = kWords ? kLastWord : ~0ull;
-        if (t * kWave + lane < len) c[t] = lists.keys[lo + t * kWave + lane];
-    }
-    if constexpr (!kWords) {
-        uint32_t val[kUse];
+        for (int t = 0; t < kUse; t++) segment.load<kWords>(t * kWave + lane, depth[t], value[t]);
+        uint32_t least = ~0u, most = 0;
 #pragma unroll
         for (int t = 0; t < kUse; t++) {
-            val[t] = ~0u;
-            if (t * kWave + lane < len) val[t] = lists.values[lo + t * kWave + lane];
+            most = max(most, depth[t]);                                         // 0 past the end
+            depth[t] = t * kWave + lane < len ? depth[t] : ~0u;
+            least = min(least, depth[t]);
         }
+        bits.span<kPlace>(wave_least(least), wave_most(most));
 #pragma unroll
-        for (int t = 0; t < kUse; t++) c[t] = t * kWave + lane < len ? (c[t] << 32) | val[t] : kLastWord;
-    }
-    bool other_words = false;   // a depth word from 0x7ff00000 up, or position i + 1 holds a smaller value than position i
-#pragma unroll
-    for (int t = 0; t < kUse; t++) {
-        uint32_t next = (uint32_t)__shfl_down((int)(uint32_t)c[t], 1);
-        if (t + 1 < kUse) {
-            const uint32_t wrap = (uint32_t)bcast_i((int)(uint32_t)c[t + 1 < kUse ? t + 1 : t], 0);
-            if (lane == kWave - 1) next = wrap;
+        for (int t = 0; t < kUse; t++) {
+            s_one[t * kWave + lane] = value[t];
+            c[t] = bits.word<kPlace>(depth[t], t * kWave + lane < len, (uint32_t)(t * kWave + lane));
         }
-        other_words = other_words || (t * kWave + lane + 1 < len && next < (uint32_t)c[t]) || (uint32_t)(c[t] >> 32) >= 0x7ff00000u;
-    }
-    const bool by_value = ballot(other_words) == 0;
-    // (no branches around the slots: where two paths meet, the sixteen words are copied from the
-    // registers one path left them in to those of the other)
-    uint32_t* const s_val = (uint32_t*)s_w;
-#pragma unroll
-    for (int t = 0; t < kUse; t++) {
-        const int i = t * kWave + lane;
-        const uint32_t depth = (uint32_t)(c[t] >> 32), value = (uint32_t)c[t];
-        if (!by_value && i < len) s_val[i] = value;
-        // (a slot past the end by its position)
-        const uint32_t high = by_value ? depth : i < len ? depth >> 16 : 0xffffu, low = by_value ? value : (depth << 16) | (uint32_t)i;
-        c[t] = ((uint64_t)high << 32) | low;
-    }
-    bitonic_network<kUse>(c, lane);
-    asm volatile("" : "+v"(lane));
-    __builtin_amdgcn_wave_barrier();
-#pragma unroll
-    for (int t = 0; t < kUse; t++) {
-        const uint32_t high = (uint32_t)(c[t] >> 32), low = (uint32_t)c[t];
-        const uint32_t looked_up = s_val[by_value ? 0u : min(low & 0xffffu, (uint32_t)(kUse * kWave - 1))];
-        c[t] = ((uint64_t)(by_value ? high : (high << 16) | (low >> 16)) << 32) | (by_value ? low : looked_up);
-    }
-    // back to contiguous stores through LDS, the lower half of the ranks (lanes 0..31) first, then
-    // the upper half through the same words: half the LDS, twice the waves per CU
-    constexpr int kRounds = kUse >= 2 ? 2 : 1, kPart = kUse * kWave / kRounds;
-    const bool by_index = *lists.by_index != 0;
-#pragma unroll
-    for (int h = 0; h < kRounds; h++) {
+        sort_words(c, lane);
         __builtin_amdgcn_wave_barrier();
-        if (lane / (kWave / kRounds) == h) {
+        asm volatile("" : "+v"(lane));
 #pragma unroll
-            for (int t = 0; t < kUse; t++) {
-                const int r = lane * kUse + t;
-                if (r < len) s_w[staged(r - h * kPart)] = c[t];
+        for (int t = 0; t < kUse; t++) {
+            c[t] &= (uint32_t)(kCap - 1);
+            value[t] = s_one[c[t]];
+        }
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int t = 0; t < kUse; t++) s_one[t * kWave + lane] = depth[t];
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int t = 0; t < kUse; t++) depth[t] = s_one[c[t]];
+        __builtin_amdgcn_wave_barrier();
+        bool sorted = bits.complete() || !descends(depth, lane, ~0u);
+        if constexpr (kUse >= 2) {
+#pragma unroll 1
+            for (int r = 0; !sorted && r < kRepairs && bits.stage == 0; r++) {
+                exchange_slots(depth, value, 0);
+                exchange_slots(depth, value, 1);
+                exchange_ends(depth, value, lane, 0u, 0u, ~0u, 0u);
+                sorted = !descends(depth, lane, ~0u);
+            }
+        }
+        asm volatile("" : "+v"(lane));
+        // back to contiguous stores through LDS, the lower half of the ranks (lanes 0..31) first, then
+        // the upper half through the same words: half the LDS, twice the waves per CU
+#pragma unroll
+        for (int h = 0; h < kRounds; h++) {
+            __builtin_amdgcn_wave_barrier();
+            if (lane / (kWave / kRounds) == h) {
+#pragma unroll
+                for (int t = 0; t < kUse; t++) stage(s_w + staged(lane * kUse + t - h * kHalf), depth[t], value[t]);
+            }
+            __builtin_amdgcn_wave_barrier();
+            if (!sorted) {
+#pragma unroll
+                for (int t = h * (kUse / kRounds); t < (h + 1) * (kUse / kRounds); t++)
+                    segment.put_back<kWords>(t * kWave + lane, s_w[staged(t * kWave + lane - h * kHalf)]);
+            } else if (!by_index) {
+#pragma unroll
+                for (int t = h * (kUse / kRounds); t < (h + 1) * (kUse / kRounds); t++)
+                    segment.store(t * kWave + lane, v, s_w[staged(t * kWave + lane - h * kHalf)]);
+            } else {
+#pragma unroll
+                for (int t = h * (kUse / kRounds); t < (h + 1) * (kUse / kRounds); t++)
+                    if (t * kWave + lane < len) store_pair(lists, true, lo + t * kWave + lane, v, s_w[staged(t * kWave + lane - h * kHalf)]);
             }
         }
         __builtin_amdgcn_wave_barrier();
-#pragma unroll
-        for (int t = h * (kUse / kRounds); t < (h + 1) * (kUse / kRounds); t++) {
-            const int i = t * kWave + lane;
-            if (i < len) store_pair(lists, by_index, lo + i, v, s_w[staged(i - h * kPart)]);
-        }
+        if (sorted) break;
+        __threadfence_block();          // (other lanes read it back)
+        bits.stage++;
     }
-    __builtin_amdgcn_wave_barrier();
 }
 
 // The network over the smallest power of two of register slots (at most kT) that holds the segment.
 // s_w: staging_words(64 * kT) 64-bit words.
 template <int kT, bool kWords>
-__device__ __forceinline__ void sort_segment_bitonic(const Lists& lists, uint32_t v, int lo, int hi, uint64_t* s_w)
+__device__ __forceinline__ void sort_segment_wave(const Lists& lists, uint32_t v, int lo, int hi, uint64_t* s_w)
 {
     const int len = hi - lo;
-    if (len <= kWave) sort_segment_bitonic_of<1, kWords>(lists, v, lo, hi, s_w);
-    else if (kT >= 2 && len <= 2 * kWave) sort_segment_bitonic_of<(kT >= 2 ? 2 : 1), kWords>(lists, v, lo, hi, s_w);
-    else if (kT >= 4 && len <= 4 * kWave) sort_segment_bitonic_of<(kT >= 4 ? 4 : 1), kWords>(lists, v, lo, hi, s_w);
-    else if (kT >= 8 && len <= 8 * kWave) sort_segment_bitonic_of<(kT >= 8 ? 8 : 1), kWords>(lists, v, lo, hi, s_w);
-    else sort_segment_bitonic_of<kT, kWords>(lists, v, lo, hi, s_w);
+    if (len <= kWave) sort_segment_wave_of<1, kWords>(lists, v, lo, hi, s_w);
+    else if (kT >= 2 && len <= 2 * kWave) sort_segment_wave_of<(kT >= 2 ? 2 : 1), kWords>(lists, v, lo, hi, s_w);
+    else if (kT >= 4 && len <= 4 * kWave) sort_segment_wave_of<(kT >= 4 ? 4 : 1), kWords>(lists, v, lo, hi, s_w);
+    else if (kT >= 8 && len <= 8 * kWave) sort_segment_wave_of<(kT >= 8 ? 8 : 1), kWords>(lists, v, lo, hi, s_w);
+    else sort_segment_wave_of<kT, kWords>(lists, v, lo, hi, s_w);
 }
 
 // One step of the network between two waves: the wave's words against those of `partner`, in the same
-// slots and lanes or (kMirrored) in reverse order.  Both go through LDS, held with opposite signs; a
-// wave that takes no part only meets the barriers.
+// slots and lanes or (kMirrored) in reverse order, through LDS; a wave that takes no part only meets the barriers.
 template <int kT, bool kMirrored>
-__device__ __forceinline__ void compare_waves(uint64_t (&c)[kT], int lane, int wave, int partner, bool present, bool takes_part,
-                                              uint32_t& held, uint64_t* s_w)
+__device__ __forceinline__ void compare_waves(uint32_t (&c)[kT], int lane, int wave, int partner, bool present, bool takes_part, uint32_t* s_one)
 {
-    hold(c, held, wave < partner ? 0u : 0x80000000u);
     if (present) {
-        uint64_t* const to = s_w + wave * (kT * kWave) + lane;
+        uint32_t* const to = s_one + wave * (kT * kWave) + lane;
 #pragma unroll
         for (int t = 0; t < kT; t++) to[t * kWave] = c[t];
     }
     __syncthreads();
     if (takes_part) {
-        const uint64_t* const from = s_w + partner * (kT * kWave) + (kMirrored ? kWave - 1 - lane : lane);
+        const uint32_t* const from = s_one + partner * (kT * kWave) + (kMirrored ? kWave - 1 - lane : lane);
+        const uint32_t limit = wave < partner ? 0u : ~0u;
 #pragma unroll
-        for (int t = 0; t < kT; t++) {
-            keep_min_negated(c[t], from[(kMirrored ? kT - 1 - t : t) * kWave]);
-            if (t % 4 == 3) __builtin_amdgcn_sched_barrier(0);       // no more words in registers than that
-        }
+        for (int t = 0; t < kT; t++) c[t] = keep_word(c[t], from[(kMirrored ? kT - 1 - t : t) * kWave], limit);
     }
     __syncthreads();
 }
 
+// What the waves that sort one segment tell each other.
+template <int kWaves>
+struct Between {
+    uint32_t least[kWaves], most[kWaves], wrong[kWaves];
+    uint32_t first_depth[kWaves], first_value[kWaves], last_depth[kWaves], last_value[kWaves];
+};
+
 // Sorts the segment [lo, hi) of tile id v, 64 * kWaves * kUse >= hi - lo, with the network over kUse
-// slots per lane of kWaves waves.  Called by all waves of a workgroup with the same arguments.  s_w: 64 *
-// kWaves * kUse words of LDS; s_seen: one word per wave.
+// slots per lane of kWaves waves.  Called by all waves of a workgroup with the same arguments.  s_w: kWaves times the
+// staging words of 64 * kUse.
 // Every wave sorts 64 * kUse words as above.  Runs are then merged in pairs: the first step compares
 // element i of the lower run with element i from the end of the upper one, the next ones halve the
 // distance, between waves through LDS and inside a wave as above.  All runs ascend, so the words
 // past the end of the segment stay behind it, and waves that hold nothing else have nothing to do.
-// The vector unit bounds it, as it does the network of one wave: 75 steps for 4096 pairs against 55
-// for 1024, and three exchanges through LDS at about twice the cost of a step.  Counting passes in LDS
-// (four of them, each a chain of atomics, a scan over digits and a ranking by ballots) took more than
-// twice as long per pair: 8K frame of 111M pairs 825 -> 475 us for the segments of 1025 .. 4096 pairs
-// and 343 -> 195 for those up to 8192, 179 -> 141 for the longer ones; 4K frame of 8M pairs 49 -> 33,
-// 1080p frame of 1.8M pairs 18.6 -> 13.6.
 template <int kWaves, int kUse, bool kWords>
-__device__ __forceinline__ void sort_segment_waves_of(const Lists& lists, uint32_t v, int lo, int hi, uint64_t* s_w, uint32_t* s_seen)
+__device__ __forceinline__ void sort_segment_waves_of(const Lists& lists, uint32_t v, int lo, int hi, uint64_t* s_w, Between<kWaves>& s_between)
 {
     static_assert(kUse >= 2, "the ranks leave in two halves of a wave's slots");
     constexpr int kPart = kUse * kWave;                 // words of a wave
+    constexpr int kCap = kPart * kWaves, kPlace = log2_of(kCap);
+    static_assert(kCap * 4 <= kWaves * staging_words(kPart) * 8, "a word for every pair");
+    uint32_t* const s_one = (uint32_t*)s_w;
     int lane = threadIdx.x & (kWave - 1);
     asm volatile("" : "+v"(lane));
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
     const int len = hi - lo;
     const int first = wave * kPart;                     // this wave's part of the segment
     const bool present = first < len;
-    const int mine = len - first;
-    uint64_t c[kUse];
+    const Segment segment(lists, lo, len);
+    const bool by_index = *lists.by_index != 0;
+    uint64_t* const s_mine = s_w + wave * staging_words(kPart);
+    WordBits bits;
+    bits.stage = 0;
+#pragma unroll 1
+    for (;;) {
+        asm volatile("" : "+v"(lane));
+        uint32_t c[kUse];
+        {
+            uint32_t depth[kUse], least = ~0u, most = 0;
 #pragma unroll
-    for (int t = 0; t < kUse; t++) {
-        c[t] = kWords ? kLastWord : ~0ull;
-        if (t * kWave + lane < mine) c[t] = lists.keys[lo + first + t * kWave + lane];
-    }
-    if constexpr (!kWords) {
-        uint32_t val[kUse];
+            for (int t = 0; t < kUse; t++) depth[t] = segment.load_depth<kWords>(first + t * kWave + lane);
+#pragma unroll
+            for (int t = 0; t < kUse; t++) {
+                most = max(most, depth[t]);                                     // 0 past the end
+                depth[t] = first + t * kWave + lane < len ? depth[t] : ~0u;
+                least = min(least, depth[t]);
+            }
+            least = wave_least(least);
+            most = wave_most(most);
+            if (lane == 0) { s_between.least[wave] = least; s_between.most[wave] = most; }
+            __syncthreads();
+#pragma unroll
+            for (int w = 0; w < kWaves; w++) {
+                least = min(least, s_between.least[w]);
+                most = max(most, s_between.most[w]);
+            }
+            bits.span<kPlace>(least, most);
+#pragma unroll
+            for (int t = 0; t < kUse; t++)
+                c[t] = bits.word<kPlace>(depth[t], first + t * kWave + lane < len, (uint32_t)(first + t * kWave + lane));
+        }
+        if (present) sort_words(c, lane);
+#pragma unroll 1
+        for (int group = 2; group <= kWaves && (group / 2) * kPart < len; group <<= 1) {      // waves of a merged run
+            int partner = wave ^ (group - 1);
+            compare_waves<kUse, true>(c, lane, wave, partner, present, present && partner * kPart < len, s_one);
+#pragma unroll 1
+            for (int d = group / 4; d > 0; d >>= 1) {
+                partner = wave ^ d;
+                compare_waves<kUse, false>(c, lane, wave, partner, present, present && partner * kPart < len, s_one);
+            }
+            if (present) merge_lanes(c, lane, 6);
+        }
+        asm volatile("" : "+v"(lane));
+        // The pairs come from memory a second time: held through the merges they would take half of the registers, and with them the
+        // waves that another segment's merges need.
+        uint32_t depth[kUse], value[kUse];
+#pragma unroll
+        for (int t = 0; t < kUse; t++) segment.load<kWords>(first + t * kWave + lane, depth[t], value[t]);
 #pragma unroll
         for (int t = 0; t < kUse; t++) {
-            val[t] = ~0u;
-            if (t * kWave + lane < mine) val[t] = lists.values[lo + first + t * kWave + lane];
+            s_one[first + t * kWave + lane] = value[t];
+            depth[t] = first + t * kWave + lane < len ? depth[t] : ~0u;
+            c[t] &= (uint32_t)(kCap - 1);
         }
+        __syncthreads();
 #pragma unroll
-        for (int t = 0; t < kUse; t++) c[t] = t * kWave + lane < mine ? (c[t] << 32) | val[t] : kLastWord;
-    }
-    asm volatile("" : "+v"(lane));
-    const uint32_t behind = mine > kPart ? value_at<kWords>(lists, lo + first + kPart) : ~0u;       // the first value of the next wave's part
-    bool other_words = false;
+        for (int t = 0; t < kUse; t++) value[t] = s_one[c[t]];
+        __syncthreads();
 #pragma unroll
-    for (int t = 0; t < kUse; t++) {
-        uint32_t next = (uint32_t)__shfl_down((int)(uint32_t)c[t], 1);
-        const uint32_t wrap = t + 1 < kUse ? (uint32_t)bcast_i((int)(uint32_t)c[t + 1 < kUse ? t + 1 : t], 0) : behind;
-        if (lane == kWave - 1) next = wrap;
-        other_words = other_words || (t * kWave + lane + 1 < mine && next < (uint32_t)c[t]) || (uint32_t)(c[t] >> 32) >= 0x7ff00000u;
-        if (t % 4 == 3) __builtin_amdgcn_sched_barrier(0);
-    }
-    const uint32_t seen = ballot(other_words) ? 1u : 0u;
-    if (lane == 0) s_seen[wave] = seen;
-    __syncthreads();
-    uint32_t any = 0;
+        for (int t = 0; t < kUse; t++) s_one[first + t * kWave + lane] = depth[t];
+        __syncthreads();
 #pragma unroll
-    for (int w = 0; w < kWaves; w++) any |= s_seen[w];
-    const bool by_value = __builtin_amdgcn_readfirstlane((int)any) == 0;
-#pragma unroll
-    for (int t = 0; t < kUse; t++) {
-        const uint32_t depth = (uint32_t)(c[t] >> 32), value = (uint32_t)c[t], i = (uint32_t)(first + t * kWave + lane);
-        const uint32_t high = by_value ? depth : (int)i < len ? depth >> 16 : 0xffffu, low = by_value ? value : (depth << 16) | i;
-        c[t] = ((uint64_t)high << 32) | low;
-    }
-    if (present) bitonic_network<kUse>(c, lane);
+        for (int t = 0; t < kUse; t++) depth[t] = s_one[c[t]];
+        bool sorted = bits.complete();
+        if (!sorted) {
+            const int next = min(wave + 1, kWaves - 1), previous = max(wave - 1, 0);
 #pragma unroll 1
-    for (int group = 2; group <= kWaves && (group / 2) * kPart < len; group <<= 1) {      // waves of a merged run
-        int partner = wave ^ (group - 1);
-        uint32_t held = 0;
-        compare_waves<kUse, true>(c, lane, wave, partner, present, present && partner * kPart < len, held, s_w);
-#pragma unroll 1
-        for (int d = group / 4; d > 0; d >>= 1) {
-            partner = wave ^ d;
-            compare_waves<kUse, false>(c, lane, wave, partner, present, present && partner * kPart < len, held, s_w);
+            for (int r = 0; ; r++) {
+                if (lane == 0) { s_between.first_depth[wave] = depth[0]; s_between.first_value[wave] = value[0]; }
+                __syncthreads();
+                const uint32_t wrong = descends(depth, lane, wave == kWaves - 1 ? ~0u : s_between.first_depth[next]) ? 1u : 0u;
+                if (lane == 0) s_between.wrong[wave] = wrong;
+                __syncthreads();
+                uint32_t any = 0;
+#pragma unroll
+                for (int w = 0; w < kWaves; w++) any |= s_between.wrong[w];
+                sorted = __builtin_amdgcn_readfirstlane((int)any) == 0;
+                if (sorted || r == kRepairs || bits.stage != 0) break;
+                exchange_slots(depth, value, 0);
+                if (lane == 0) { s_between.first_depth[wave] = depth[0]; s_between.first_value[wave] = value[0]; }
+                if (lane == kWave - 1) { s_between.last_depth[wave] = depth[kUse - 1]; s_between.last_value[wave] = value[kUse - 1]; }
+                __syncthreads();
+                exchange_slots(depth, value, 1);
+                exchange_ends(depth, value, lane, wave == 0 ? 0u : s_between.last_depth[previous], s_between.last_value[previous],
+                              wave == kWaves - 1 ? ~0u : s_between.first_depth[next], s_between.first_value[next]);
+                __syncthreads();
+            }
         }
-        if (present) merge_slots(c, lane, kPart, 0u, held);
-    }
-    asm volatile("" : "+v"(lane));
-    // the values of the words that carry positions, before any is overwritten
+        __syncthreads();
+        asm volatile("" : "+v"(lane));
+        // back to contiguous stores through this wave's part of the LDS, half of the ranks at a time
 #pragma unroll
-    for (int t = 0; t < kUse; t++) {
-        const uint32_t high = (uint32_t)(c[t] >> 32), low = (uint32_t)c[t];
-        uint32_t value = low;
-        if (!by_value && (low & 0xffffu) < (uint32_t)len) value = value_at<kWords>(lists, lo + (int)(low & 0xffffu));
-        c[t] = ((uint64_t)(by_value ? high : (high << 16) | (low >> 16)) << 32) | value;
-        if (t % 4 == 3) __builtin_amdgcn_sched_barrier(0);
-    }
-    if (!by_value) __syncthreads();
-    // back to contiguous stores through this wave's part of the LDS, half of the ranks at a time
-    uint64_t* const s_mine = s_w + first;
-    const bool by_index = *lists.by_index != 0;
+        for (int h = 0; h < 2; h++) {
+            __builtin_amdgcn_wave_barrier();
+            if (lane / (kWave / 2) == h) {
 #pragma unroll
-    for (int h = 0; h < 2; h++) {
-        __builtin_amdgcn_wave_barrier();
-        if (lane / (kWave / 2) == h) {
+                for (int t = 0; t < kUse; t++) stage(s_mine + staged(lane * kUse + t - h * (kPart / 2)), depth[t], value[t]);
+            }
+            __builtin_amdgcn_wave_barrier();
+            if (!sorted) {
 #pragma unroll
-            for (int t = 0; t < kUse; t++) s_mine[staged(lane * kUse + t - h * (kPart / 2))] = c[t];
+                for (int t = h * (kUse / 2); t < (h + 1) * (kUse / 2); t++)
+                    segment.put_back<kWords>(first + t * kWave + lane, s_mine[staged(t * kWave + lane - h * (kPart / 2))]);
+            } else if (!by_index) {
+#pragma unroll
+                for (int t = h * (kUse / 2); t < (h + 1) * (kUse / 2); t++)
+                    segment.store(first + t * kWave + lane, v, s_mine[staged(t * kWave + lane - h * (kPart / 2))]);
+            } else {
+#pragma unroll
+                for (int t = h * (kUse / 2); t < (h + 1) * (kUse / 2); t++) {
+                    const int i = first + t * kWave + lane;
+                    if (i < len) store_pair(lists, true, lo + i, v, s_mine[staged(t * kWave + lane - h * (kPart / 2))]);
+                }
+            }
         }
-        __builtin_amdgcn_wave_barrier();
-#pragma unroll
-        for (int t = h * (kUse / 2); t < (h + 1) * (kUse / 2); t++) {
-            const int i = t * kWave + lane;
-            if (i < mine) store_pair(lists, by_index, lo + first + i, v, s_mine[staged(i - h * (kPart / 2))]);
-        }
+        if (!sorted) __threadfence_block();         // (other waves read it back)
+        __syncthreads();
+        if (sorted) break;
+        bits.stage++;
     }
-    __syncthreads();
 }
 
 // The smallest number of slots per lane, from kLeast on, that holds the segment: hi - lo <= kCap.
 template <int kWaves, int kCap, int kLeast, bool kWords>
-__device__ __forceinline__ void sort_segment_waves(const Lists& lists, uint32_t v, int lo, int hi, uint64_t* s_w, uint32_t* s_seen)
+__device__ __forceinline__ void sort_segment_waves(const Lists& lists, uint32_t v, int lo, int hi, uint64_t* s_w, Between<kWaves>& s_between)
 {
     constexpr int kMost = kCap / (kWaves * kWave);
     if constexpr (kLeast < kMost)
         if (hi - lo > kLeast * kWaves * kWave)
-            return sort_segment_waves<kWaves, kCap, 2 * kLeast, kWords>(lists, v, lo, hi, s_w, s_seen);
-    sort_segment_waves_of<kWaves, kLeast, kWords>(lists, v, lo, hi, s_w, s_seen);
+            return sort_segment_waves<kWaves, kCap, 2 * kLeast, kWords>(lists, v, lo, hi, s_w, s_between);
+    sort_segment_waves_of<kWaves, kLeast, kWords>(lists, v, lo, hi, s_w, s_between);
 }
 
-// Segment sort by the waves of a workgroup for one size class: segments with min_len < length <= kCap.
+// Segment sort by the waves of a workgroup for one size class: segments with min_len < length <= kCap.  Seven waves per SIMD cost a few spilled
+// registers: 110M pairs 328 -> 308 us against five of 82 registers, eight 357.
 // With a table of segment starts, the first launch has listed the segments of the class.  Without a table
 // (more tile ids than it holds) the grid has one workgroup per tile id and each searches for its bounds.
 template <int kWaves, int kCap, int kLeast, bool kWords>
-__global__ __launch_bounds__(kWaves * kWave) void segment_sort_kernel(
+__global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(7))) void segment_sort_kernel(
     Lists lists, int n, uint32_t tile_mask, int min_len, const int* __restrict__ seg_start,
     const uint32_t* __restrict__ list, const uint32_t* __restrict__ list_count, uint32_t list_cap)
 {
-    __shared__ uint64_t s_w[kCap];
-    __shared__ uint32_t s_seen[kWaves];
+    __shared__ uint64_t s_w[kWaves * staging_words(kCap / kWaves)];
+    __shared__ Between<kWaves> s_between;
     __shared__ int s_bounds[2];
 
     const int tid = threadIdx.x;
     const int lane = tid & (kWave - 1);
 
-    if (!seg_start) {
+    if (!kWords && !seg_start) {        // (words have a table)
         const uint32_t v = blockIdx.x;
         if (tid < kWave) {
             const int a = wave_lower_bound(lists.keys, n, v, tile_mask);
@@ -1298,7 +1479,7 @@ __global__ __launch_bounds__(kWaves * kWave) void segment_sort_kernel(
         __syncthreads();
         const int lo = s_bounds[0], hi = s_bounds[1];
         if (hi - lo <= min_len || hi - lo > kCap) return;
-        sort_segment_waves<kWaves, kCap, kLeast, kWords>(lists, v, lo, hi, s_w, s_seen);
+        sort_segment_waves<kWaves, kCap, kLeast, kWords>(lists, v, lo, hi, s_w, s_between);
         return;
     }
 
@@ -1307,11 +1488,11 @@ __global__ __launch_bounds__(kWaves * kWave) void segment_sort_kernel(
     const uint32_t count = list_count[shard];
     for (uint32_t i = blockIdx.x / kListShards; i < count; i += gridDim.x / kListShards) {
         const uint32_t v = list[(size_t)shard * list_cap + i];
-        sort_segment_waves<kWaves, kCap, kLeast, kWords>(lists, v, seg_start[v], seg_start[v + 1], s_w, s_seen);
+        sort_segment_waves<kWaves, kCap, kLeast, kWords>(lists, v, seg_start[v], seg_start[v + 1], s_w, s_between);
     }
 }
 
-// One wave per workgroup, and one workgroup per tile id: it sorts that id's segment of up to 64*kT pairs.  Its bounds come from
+// One wave per workgroup: it sorts the segments of up to 64*kT pairs of one tile id or of several, a grid apart.  Their bounds come from
 // the table of segment starts or, without one, from a search.
 template <int kT, bool kWords>
 __global__ __launch_bounds__(kWave) void segment_sort_wave_kernel(
@@ -1322,33 +1503,34 @@ __global__ __launch_bounds__(kWave) void segment_sort_wave_kernel(
     uint32_t list_cap0, uint32_t list_cap1, uint32_t list_cap2, uint32_t list_cap3)
 {
     __shared__ uint64_t s_w[staging_words(kT * kWave)];
-    const uint32_t v = blockIdx.x;
-    int lo, hi;
-    if (!seg_start) {
-        lo = wave_lower_bound(lists.keys, n, v, tile_mask);
-        hi = v == tile_mask ? n : wave_lower_bound(lists.keys, n, v + 1, tile_mask);
-    } else {
-        lo = seg_start[v];
-        hi = seg_start[v + 1];
-        // This launch sees every tile id once: it also lists the ids of the longer segments by class
-        // (lengths up to list_max0, list_max1, list_max2, and everything longer), so that those
-        // fewer, longer-running segments can be dealt out evenly by the launches that follow.
-        const int len = hi - lo;
-        if (len > kT * kWave && threadIdx.x == 0) {
-            // neighbouring tiles tend to be equally busy: mix the index so that every list gets its share
-            const uint32_t shard = (v ^ (v >> 5) ^ (v >> 10) ^ (v >> 15)) % kListShards;
-            if (len <= list_max0)
-                list0[(size_t)shard * list_cap0 + atomicAdd(&seg_counts[0 * kListShards + shard], 1u)] = v;
-            else if (len <= list_max1)
-                list1[(size_t)shard * list_cap1 + atomicAdd(&seg_counts[1 * kListShards + shard], 1u)] = v;
-            else if (len <= list_max2)
-                list2[(size_t)shard * list_cap2 + atomicAdd(&seg_counts[2 * kListShards + shard], 1u)] = v;
-            else
-                list3[(size_t)shard * list_cap3 + atomicAdd(&seg_counts[3 * kListShards + shard], 1u)] = v;
+    for (uint32_t v = blockIdx.x; v <= tile_mask; v += gridDim.x) {
+        int lo, hi;
+        if (!kWords && !seg_start) {
+            lo = wave_lower_bound(lists.keys, n, v, tile_mask);
+            hi = v == tile_mask ? n : wave_lower_bound(lists.keys, n, v + 1, tile_mask);
+        } else {
+            lo = seg_start[v];
+            hi = seg_start[v + 1];
+            // This launch sees every tile id once: it also lists the ids of the longer segments by class
+            // (lengths up to list_max0, list_max1, list_max2, and everything longer), so that those
+            // fewer, longer-running segments can be dealt out evenly by the launches that follow.
+            const int len = hi - lo;
+            if (len > kT * kWave && threadIdx.x == 0) {
+                // neighbouring tiles tend to be equally busy: mix the index so that every list gets its share
+                const uint32_t shard = (v ^ (v >> 5) ^ (v >> 10) ^ (v >> 15)) % kListShards;
+                if (len <= list_max0)
+                    list0[(size_t)shard * list_cap0 + atomicAdd(&seg_counts[0 * kListShards + shard], 1u)] = v;
+                else if (len <= list_max1)
+                    list1[(size_t)shard * list_cap1 + atomicAdd(&seg_counts[1 * kListShards + shard], 1u)] = v;
+                else if (len <= list_max2)
+                    list2[(size_t)shard * list_cap2 + atomicAdd(&seg_counts[2 * kListShards + shard], 1u)] = v;
+                else
+                    list3[(size_t)shard * list_cap3 + atomicAdd(&seg_counts[3 * kListShards + shard], 1u)] = v;
+            }
         }
+        // (words become pairs here, and indices values, also where there is nothing to sort)
+        if (hi > lo && hi - lo <= kT * kWave) sort_segment_wave<kT, kWords>(lists, v, lo, hi, s_w);
     }
-    // (words become pairs here, and indices values, also where there is nothing to sort)
-    if (hi > lo && hi - lo <= kT * kWave) sort_segment_bitonic<kT, kWords>(lists, v, lo, hi, s_w);
 }
 
 // The listed segments of one class (at most 64*kT pairs each), dealt out round-robin to
@@ -1363,7 +1545,7 @@ __global__ __launch_bounds__(kWave) void segment_sort_wave_list_kernel(
     const uint32_t count = list_count[shard];
     for (uint32_t i = blockIdx.x / kListShards; i < count; i += gridDim.x / kListShards) {
         const uint32_t v = list[(size_t)shard * list_cap + i];
-        sort_segment_bitonic<kT, kWords>(lists, v, seg_start[v], seg_start[v + 1], s_w);
+        sort_segment_wave<kT, kWords>(lists, v, seg_start[v], seg_start[v + 1], s_w);
         __builtin_amdgcn_wave_barrier();
     }
 }
@@ -1406,8 +1588,8 @@ __device__ __forceinline__ void sort_segment_general(const Lists& lists, uint64_
 // ones longer than min_len: neighbouring tiles tend to be equally crowded, so they are dealt out
 // one segment at a time, round-robin).
 // With a table (kTable) a listed segment of up to kCapHuge pairs is sorted by the network over the
-// sixteen waves (a workgroup then has the LDS of its CU to itself): the passes through memory take
-// 7 us each for 12 000 pairs.
+// sixteen waves: the passes through memory take 7 us each for 12 000 pairs.  (A workgroup has a CU to itself; two of
+// 64 registers a lane, the counters in the space of the words: 113 -> 145 us on the frame of 110M pairs.)
 // The workgroups first sort the listed segments of the classes below (first_class 1:
 // 1025 .. kCapLarge pairs, 2: only those above kCapMedium, 3: none; shard by shard like the
 // launches of those classes): a frame with a short list of pairs has few such segments or none,
@@ -1423,7 +1605,8 @@ __global__ __launch_bounds__(kGeneralWaves * kWave) void segment_sort_general_ke
     const uint32_t* __restrict__ list_medium, uint32_t cap_medium, const uint32_t* __restrict__ list_large, uint32_t cap_large,
     int first_class)
 {
-    __shared__ uint64_t s_w[kTable ? kCapHuge : 1];
+    __shared__ uint64_t s_w[kTable ? kGeneralWaves * staging_words(kCapHuge / kGeneralWaves) : 1];
+    __shared__ Between<kGeneralWaves> s_between;
     __shared__ uint32_t s_cnt[kGeneralWaves][kBins];
     __shared__ uint32_t s_wave_sum[kGeneralWaves];
     __shared__ int s_bounds[2];
@@ -1453,7 +1636,7 @@ __global__ __launch_bounds__(kGeneralWaves * kWave) void segment_sort_general_ke
                 const uint32_t v = ids_of[(size_t)shard * cap + i];
                 const int lo = seg_start[v], hi = seg_start[v + 1];
                 if (hi - lo <= kCapHuge)
-                    sort_segment_waves<kGeneralWaves, kCapHuge, 2, kWords>(lists, v, lo, hi, s_w, s_wave_sum);
+                    sort_segment_waves<kGeneralWaves, kCapHuge, 2, kWords>(lists, v, lo, hi, s_w, s_between);
                 else
                     sort_segment_general<kWords>(lists, alt_keys, alt_values, v, lo, hi, s_cnt, s_wave_sum, &s_flag);
             }
@@ -1606,7 +1789,7 @@ extern "C" int fgs_sort_gaussian(int num_rendered,
         return (g + kListShards - 1) / kListShards * kListShards;
     };
 #define FGS_SEGMENT_WAVE(CAP, WORDS)                                                                          \
-    hipLaunchKernelGGL((segment_sort_wave_kernel<(CAP) / kWave, WORDS>), dim3(ids), dim3(kWave),              \
+    hipLaunchKernelGGL((segment_sort_wave_kernel<(CAP) / kWave, WORDS>), dim3((ids + ids_per_wave - 1) / ids_per_wave), dim3(kWave),              \
                        0, st, lists, n, tile_mask, (const int*)seg_start,                                     \
                        kCapSmall, kCapMedium, kCapLarge, seg_counts, list_small, list_medium,                 \
                        list_large, list_long, cap_small, cap_medium, cap_large, cap_long)
@@ -1622,13 +1805,17 @@ extern "C" int fgs_sort_gaussian(int num_rendered,
     // A short list of pairs has few segments of more than 1024 pairs, or none: there the one
     // launch below takes those classes too (720p, 0.2M pairs: two launches less).
     const bool merged_tail = seg_start && n <= kMergedTailMax;
+    // On a long list a wave takes several tile ids (a grid apart): its successor would start some 3 us after its end.  The segments of up
+    // to 1024 pairs with 1, 2, 4 and 8 ids a wave: 110M pairs of an 8K frame 279, 256, 232, 224 us, 29M 113, 107, 109, 118, 36M of a 4K frame
+    // 93, 76, 85, 103; below, the last waves' second segments count for more: 14.5M 82, 77, 80, 8M 34.7, 39.7, 41.1.
+    const uint32_t ids_per_wave = n > kManyPairs ? 4 : n > kMergedLargeMax ? 2 : 1;
     const bool merged_large = seg_start && !merged_tail && n <= kMergedLargeMax;
     const int smallest = merged_tail ? kCapSmall : merged_large ? kCapMedium : kCapLarge;
     const unsigned tail_blocks = n > smallest ? list_grid((unsigned)(n / (smallest + 1) + 1), n > kMergedLargeMax ? 2048u : 256u) : 0u;
     const int first_class = merged_tail ? 1 : merged_large ? 2 : 3;
     const unsigned medium_blocks = list_grid((unsigned)(n / (kCapSmall + 1) + 1), 4096u), large_blocks = list_grid((unsigned)(n / (kCapMedium + 1) + 1), 1024u);
     if (words) {
-        // Up to 1024 pairs: one wave, bitonic network in registers; one tile id per wave (neighbouring
+        // Up to 1024 pairs: one wave, network in registers; one tile id per wave on all but long lists (neighbouring
         // tiles tend to be equally busy, so a wave that took several of them would become the tail
         // of the launch).  The launch also lists the longer segments.  Segments of 513..1024 pairs in a launch of
         // their own last as long as one such sort on a frame of few tiles, which has about one per SIMD (1080p: -15 us, 4K:

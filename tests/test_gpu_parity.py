@@ -1183,8 +1183,8 @@ def test_sort_segment_size_classes(seg, dense):
 @pytest.mark.parametrize("depths", ["all words", "positive floats", "tiny", "from 0x7ff00000 up"])
 @pytest.mark.parametrize("ascending", [True, False])
 def test_sort_depth_words_of_every_pattern(depths, ascending):
-    """The network of the short segments takes its words as doubles: depth words that make a negative,
-    infinite, denormal or not-a-number double of them, around the widths of the network, ties included."""
+    """Depth words that are no positive floats (negative, infinite, denormal, not a number, every bit set, which is
+    what stands past the end of a segment), around the widths of the network, ties included."""
     import gpu_pipeline as gp
     rng = np.random.default_rng(len(depths) + ascending)
     lengths = [1, 2, 3, 63, 64, 65, 127, 128, 129, 255, 256, 257, 500, 512, 513, 700, 1023, 1024]
@@ -1222,6 +1222,32 @@ def test_sort_segments_of_several_waves(depths, ascending, copies):
         first = np.concatenate([[0], np.cumsum(lengths)[:-1]])
         vals[first + 64 * (1 << (np.arange(len(lengths)) % 5))] = 0
     ks, vs = gp.sort(n, 1920, 1080, gp.dev(keys.view(np.int64)), gp.dev(vals.view(np.int32)))
+    order = np.argsort(keys, kind="stable")
+    assert np.array_equal(gp.u64(ks), keys[order]) and np.array_equal(gp.u32(vs), vals[order])
+
+
+@pytest.mark.parametrize("span", [1 << 20, 1 << 24, 0x7f7fffff, 0xffffffff])
+@pytest.mark.parametrize("group", [1, 2, 5, 9, 40, 1 << 30])
+def test_sort_depths_that_differ_in_the_bits_a_word_leaves_out(span, group):
+    """A network orders 32-bit words of the upper bits of the depths above the segment's least one.  Every
+    segment here spans `span`, and its other depths come in groups of up to `group` that differ in the
+    lowest ten bits only: in order behind the network alone, after a few exchanges of neighbours, and only after a
+    second sort; some depths are equal and have to keep their order."""
+    import gpu_pipeline as gp
+    rng = np.random.default_rng(group % 1000 + span % 1000)
+    lengths = [2, 3, 63, 64, 65, 127, 128, 129, 255, 256, 257, 511, 512, 513, 1000, 1023, 1024, 1025, 2047, 2049, 4096, 4097, 8192, 8193, 16384]
+    parts = []
+    for n in lengths:
+        base = rng.integers(0, max(1, span >> 10), (n + group - 1) // group).astype(np.uint64) << np.uint64(10)
+        low = rng.integers(0, 1 << int(rng.integers(1, 11)), n).astype(np.uint64)
+        depth = np.minimum(np.repeat(base, min(group, n))[:n] + low, span)
+        depth[rng.integers(0, n)] = 0
+        depth[rng.integers(0, n)] = span
+        parts.append(rng.permutation(depth))
+    tile = np.repeat(np.arange(len(lengths)), lengths).astype(np.uint64)
+    keys = (tile << np.uint64(32)) | np.concatenate(parts)
+    vals = rng.integers(0, 1 << 32, keys.size, dtype=np.uint64).astype(np.uint32)
+    ks, vs = gp.sort(keys.size, 80, 80, gp.dev(keys.view(np.int64)), gp.dev(vals.view(np.int32)))
     order = np.argsort(keys, kind="stable")
     assert np.array_equal(gp.u64(ks), keys[order]) and np.array_equal(gp.u32(vs), vals[order])
 
