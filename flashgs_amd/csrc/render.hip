@@ -36,6 +36,18 @@ __global__ __launch_bounds__(256) void fill_i32_kernel(int* p, size_t n, int v)
 }
 
 
+// The lists of a large frame that are long for it (see long_table) start first: one that starts late ends late, and the launch with
+// it (8K / 8M: lists of 2400 entries that start after a third of the launch end 50 us behind everything else: blend 695 -> 639 us).  The launch that marks the
+// ranges lists them, the first kLongLists workgroups of the blend take them from there, and a tile that finds itself listed leaves itself to
+// them.  A tile is looked for where it would be listed, so whatever the table holds every tile is blended, and what is no such
+// tile is passed over: the table needs no initial value, a list it has no room for starts where it would otherwise.
+// There are two tables: a launch that reads one clears the counts of the other one for the frame that follows.
+constexpr int kLongShards = 32, kLongPerShard = 16, kLongLists = kLongShards * kLongPerShard;
+struct LongLists {
+    uint32_t count[kLongShards], tiles[kLongShards][kLongPerShard];
+};
+__device__ __forceinline__ uint32_t long_shard(uint32_t tile) { return (tile ^ (tile >> 5) ^ (tile >> 10)) % kLongShards; }
+
 // Tiles of a small frame ranked by the length of their lists, longest first (in steps of kOrderStep;
 // the order inside a step is whatever the atomics make it), and behind the ranking how many of them are shared out and from
 // which length on.  One workgroup.
@@ -52,14 +64,15 @@ constexpr int kOrderCap = 8192;            // tiles
 // none where no memory is left.
 struct OrderTable {
     std::mutex enqueue;
-    uint32_t* ranks = nullptr;
+    uint32_t* ranks = nullptr;          // kOrderCap + 2 words, then two LongLists
+    int turn = 0;                       // which of those the next large frame uses
 };
 std::map<StreamKey, OrderTable> g_order_tables;      // (entries stay where they are)
 std::mutex g_order_mutex;
 
 // *out is null where the tiles go unranked; enqueue is locked for as long as nobody else may enqueue a
 // launch that writes *out.
-int tile_order_table(hipStream_t stream, uint32_t** out, std::unique_lock<std::mutex>* enqueue)
+int tile_order_table(hipStream_t stream, uint32_t** out, std::unique_lock<std::mutex>* enqueue, OrderTable** table = nullptr)
 {
     int device = 0;
     *out = nullptr;
@@ -75,11 +88,12 @@ int tile_order_table(hipStream_t stream, uint32_t** out, std::unique_lock<std::m
         entry = &g_order_tables[stream_key(device, stream)];
     }
     *enqueue = std::unique_lock<std::mutex>(entry->enqueue);
-    if (!entry->ranks && hipMalloc((void**)&entry->ranks, (kOrderCap + 2) * sizeof(uint32_t)) != hipSuccess) {
+    if (!entry->ranks && hipMalloc((void**)&entry->ranks, (kOrderCap + 2) * sizeof(uint32_t) + 2 * sizeof(LongLists)) != hipSuccess) {
         (void)hipGetLastError();
         entry->ranks = nullptr;
     }
     *out = entry->ranks;
+    if (table) *table = entry;
     return FGS_OK;
 }
 
@@ -219,7 +233,8 @@ __global__ __launch_bounds__(256) void tile_ranges_kernel(int L, const uint64_t*
 constexpr int kRangeRuns = 8;
 
 __global__ __launch_bounds__(256) void tile_ranges_sampled_kernel(int L, const uint64_t* __restrict__ keys,
-                                                                  int2* __restrict__ ranges, uint32_t num_tiles)
+                                                                  int2* __restrict__ ranges, uint32_t num_tiles,
+                                                                  LongLists* __restrict__ longer, int long_list)
 {
     const int lane = threadIdx.x & (kWave - 1);
     const long long base = ((long long)blockIdx.x * (256 / kWave) + threadIdx.x / kWave) * (kRangeRuns * kWave);
@@ -229,8 +244,15 @@ __global__ __launch_bounds__(256) void tile_ranges_sampled_kernel(int L, const u
     uint32_t last = 0, before = 0;
     if (mine) last = tile_at(end - 1);
     if (lane == 0 && mine && begin > 0) before = tile_at(begin - 1);
+    uint32_t ahead = num_tiles;
+    if (longer && mine && end - 1 + long_list < L) ahead = tile_at(end - 1 + long_list);
     const uint32_t left = (uint32_t)__shfl_up((int)last, 1);
     if (lane > 0) before = left;
+    // the tile that begins in this run and goes on behind it: still there long_list pairs further on?
+    if (mine && (last != before || begin == 0) && last < num_tiles && ahead == last) {
+        const uint32_t shard = long_shard(last), at = atomicAdd(&longer->count[shard], 1u);
+        if (at < (uint32_t)kLongPerShard) longer->tiles[shard][at] = last;
+    }
     uint64_t todo = ballot(mine && (last != before || begin == 0 || end == L));
     while (todo) {
         long long idx[kRangesPerThread];
@@ -861,16 +883,23 @@ __device__ __forceinline__ void write_square(
 
 // Position in the launch -> tile.  The hardware deals consecutive workgroups out to the 8 XCDs in
 // turn, and every XCD has its own L2.  Neighbouring tiles share most of their Gaussians, so each
-// XCD is given whole 8x8 blocks of tiles (its positions g = 8*slot + xcd walk blocks xcd, xcd+8,
-// ... 64 tiles at a time): a Gaussian's attribute lines are then fetched into one L2 once instead
-// of into several L2s once per tile.  False for the padding positions.
+// XCD is given whole blocks of 4x4 tiles (its positions g = 8*slot + xcd walk blocks xcd, xcd+8,
+// ... 16 tiles at a time): a Gaussian's attribute lines are then fetched into one L2 once instead
+// of into several L2s once per tile.  Every row of blocks begins further right, so that the blocks below each other
+// belong to XCDs five apart whatever the width of the frame: with blocks of 8x8 row after row from the left, an XCD had the same columns of
+// blocks in every second row of a frame of 60 blocks, in every row of one of 24, and 2 to 14 % more to blend than the average, and
+// the launch ends when the last XCD does (3000x2200 / 2M 231 -> 215 us, 8K / 8M 704 -> 683, 5120x2880 448 -> 438, 4K 320 -> 319; blocks of
+// 8x8 five apart 213, 685, 435, 322, 4x4 three apart 216, 691, 443, 316).  False for the padding positions.
+constexpr int kBlockLog2 = 2, kBlock = 1 << kBlockLog2;
 __device__ __forceinline__ bool tile_of_position(int group, int tiles_x, int tiles_y, int* tile_x, int* tile_y)
 {
     const int xcd = group & 7, slot = group >> 3;
-    const int blocks_x = (tiles_x + 7) >> 3;
-    const int block = (slot >> 6) * 8 + xcd, inner = slot & 63;
-    *tile_x = (block % blocks_x) * 8 + (inner & 7);
-    *tile_y = (block / blocks_x) * 8 + (inner >> 3);
+    const int blocks_x = (tiles_x + kBlock - 1) >> kBlockLog2;
+    const int block = (slot >> (2 * kBlockLog2)) * 8 + xcd, inner = slot & (kBlock * kBlock - 1);
+    const int row = block / blocks_x;
+    const int column = (block - row * blocks_x + ((blocks_x - 5) & 7) * row) % blocks_x;
+    *tile_x = column * kBlock + (inner & (kBlock - 1));
+    *tile_y = row * kBlock + (inner >> kBlockLog2);
     return *tile_x < tiles_x && *tile_y < tiles_y;
 }
 
@@ -894,7 +923,8 @@ constexpr int kBlendWaves = kFp32 ? 5 : 4;       // resident waves per SIMD
 // Resident waves: 5 per SIMD is what 96 registers allow (4: the same time on the largest frames, 3 to 5 %
 // more on the others; 6 spills).
 template <int SX, int SY, bool kFp32>
-__global__ __launch_bounds__(kWave * SX * SY) __attribute__((amdgpu_waves_per_eu(kBlendWaves<kFp32>, kBlendWaves<kFp32>))) void blend_kernel(FGS_BLEND_PARAMS)
+__global__ __launch_bounds__(kWave * SX * SY) __attribute__((amdgpu_waves_per_eu(kBlendWaves<kFp32>, kBlendWaves<kFp32>))) void blend_kernel(FGS_BLEND_PARAMS,
+    const LongLists* __restrict__ longer, LongLists* __restrict__ next_longer, int long_list)
 {
     constexpr int kSquares = SX * SY;
     __shared__ __align__(16) float s_stage[kSquares][kStageFloats];
@@ -903,9 +933,25 @@ __global__ __launch_bounds__(kWave * SX * SY) __attribute__((amdgpu_waves_per_eu
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = kSquares == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     int tile_x, tile_y;
-    if (!tile_of_position((int)blockIdx.x, tiles_x, tiles_y, &tile_x, &tile_y)) return;
-    const int2 range = ranges[tile_y * tiles_x + tile_x];
+    const bool first = longer && blockIdx.x < (unsigned)kLongLists;
+    if (first) {
+        const uint32_t shard = blockIdx.x % kLongShards, at = blockIdx.x / kLongShards;
+        if (at == 0 && threadIdx.x == 0) next_longer->count[shard] = 0;
+        const uint32_t tile = longer->tiles[shard][at];
+        if (at >= longer->count[shard] || tile >= (uint32_t)(tiles_x * tiles_y) || long_shard(tile) != shard) return;
+        tile_x = (int)(tile % (uint32_t)tiles_x);
+        tile_y = (int)(tile / (uint32_t)tiles_x);
+    } else if (!tile_of_position((int)blockIdx.x - (longer ? kLongLists : 0), tiles_x, tiles_y, &tile_x, &tile_y)) {
+        return;
+    }
+    const uint32_t tile = (uint32_t)(tile_y * tiles_x + tile_x);
+    const int2 range = ranges[tile];
     const int n = range.y - range.x;
+    if (longer && !first && n >= long_list) {       // left to one of the first workgroups?
+        const uint32_t shard = long_shard(tile), at = (uint32_t)lane;
+        const bool listed = at < min(longer->count[shard], (uint32_t)kLongPerShard) && longer->tiles[shard][at % kLongPerShard] == tile;
+        if (ballot(listed) != 0) return;
+    }
     // A launch ends when its longest list ends, and a wave that shares its SIMD equally with the
     // waves of short lists gets to its own end late: waves with long lists ask for a higher
     // issue priority.
@@ -1308,9 +1354,42 @@ bool is_ranked(int tiles_x, int tiles_y) { return (long long)tiles_x * tiles_y <
 // 3.3M 6.0 and 5.3, 4.0M 7.2 and 5.8.
 constexpr int kSampledPairs = 3 << 20;
 
+// The table of the long lists of a frame whose tiles are not ranked; no list where there is none.
+struct LongTable {
+    LongLists *list = nullptr, *next = nullptr;
+    int least = 0;
+};
+
+// A list is long for its frame if it has a seventh of the entries that a SIMD has on average: it takes 166 ns per entry beside others
+// where a SIMD takes 50, so half of the launch.
+// Only frames of kLongTiles tiles and more have such lists often enough (8K / 8M Gaussians, 129 600 tiles: blend 695 -> 639 us, ranges
+// 18.2 -> 22.6; 57 600 tiles 444 -> 441 and 16.5 -> 19.1, 32 400 319 -> 320 and 12.3 -> 16.8), and none where a seventh is more than
+// kLongMost entries: lists that long are opaque long before their end (110M pairs: 477 -> 479 and 88 -> 128).
+constexpr int kLongTiles = 1 << 16, kLongMost = 8192;
+int long_table(hipStream_t stream, int num_rendered, int block_x, int block_y, int width, int height, LongTable* out, std::unique_lock<std::mutex>* enqueue)
+{
+    const int tiles_x = (width + block_x - 1) / block_x, tiles_y = (height + block_y - 1) / block_y;
+    if ((long long)tiles_x * tiles_y < kLongTiles || num_rendered < kSampledPairs) return FGS_OK;        // (ranges marked from every key list none)
+    int device = 0, cus = 0;
+    FGS_HIP_TRY(hipGetDevice(&device));
+    FGS_HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
+    const long long seventh = (long long)num_rendered * (block_x / 16) * (block_y / 16) / (4 * cus) / 7;
+    if (seventh > kLongMost) return FGS_OK;
+    uint32_t* ranks = nullptr;
+    OrderTable* entry = nullptr;
+    int rc = tile_order_table(stream, &ranks, enqueue, &entry);
+    if (rc != FGS_OK || !ranks) return rc;
+    LongLists* const both = (LongLists*)(ranks + kOrderCap + 2);
+    out->list = both + entry->turn;
+    out->next = both + (entry->turn ^ 1);
+    entry->turn ^= 1;
+    out->least = (int)std::max(seventh, 1024LL);
+    return FGS_OK;
+}
+
 // render.cu:556-563: zero the ranges, then mark where each tile starts and ends
 int ranges_impl(int block_x, int block_y, int num_rendered, int width, int height,
-                const uint64_t* keys_sorted, int* ranges, void* stream, const char* who)
+                const uint64_t* keys_sorted, int* ranges, const LongTable& longer, void* stream, const char* who)
 {
     if (num_rendered < 0) return fail(FGS_E_INVALID, "%s: num_rendered = %d is negative", who, num_rendered);
     if (width <= 0 || height <= 0 || block_x <= 0 || block_y <= 0)
@@ -1330,7 +1409,7 @@ int ranges_impl(int block_x, int block_y, int num_rendered, int width, int heigh
         hipLaunchKernelGGL(tile_ranges_sampled_kernel,
                            dim3((unsigned)(((size_t)num_rendered + 4 * kRangeRuns * kWave - 1) / (4 * kRangeRuns * kWave))),
                            dim3(256), 0, st, num_rendered, keys_sorted, (int2*)ranges,
-                           (uint32_t)(num_tiles > 0xffffffffu ? 0xffffffffu : num_tiles));
+                           (uint32_t)(num_tiles > 0xffffffffu ? 0xffffffffu : num_tiles), longer.list, longer.least);
     else
         hipLaunchKernelGGL(tile_ranges_kernel,
                            dim3((unsigned)(((size_t)num_rendered + 256 * kRangesPerThread - 1) / (256 * kRangesPerThread))),
@@ -1355,7 +1434,7 @@ int teams_of(int sx, int sy, int num_tiles, int cus)
 // a frame whose workgroups are all resident at once even with one tile each goes unranked, since nothing starts later than
 // anything else there; the image is the same bits.  256x192 / 2.8k pairs 11.1 -> 8.7 us, 348k pairs 181 -> 178, 400x300 / 362k
 // 110 -> 107, opaque needles 110 -> 117, 700x600 in 32x32 tiles 114 -> 112.
-int blend_impl(bool rank, int block_x, int block_y, int width, int height,
+int blend_impl(bool rank, const LongTable& longer, int block_x, int block_y, int width, int height,
                const float* points_xy, const float* rgb_depth, const float* conic_opacity,
                const uint32_t* values_sorted, const int* ranges, const float bg[3],
                uint8_t* out_u8, float* out_f32, int flags, void* stream, const char* who)
@@ -1372,10 +1451,10 @@ int blend_impl(bool rank, int block_x, int block_y, int width, int height,
         return fail(FGS_E_INVALID, "%s: rgb_depth/conic_opacity must be 16-byte aligned, points_xy/ranges 8-byte aligned", who);
     const int tiles_x = (width + block_x - 1) / block_x, tiles_y = (height + block_y - 1) / block_y;
     hipStream_t st = (hipStream_t)stream;
-    // one workgroup per tile of the image padded to whole 8x8 blocks of tiles, blocks padded to a multiple of 8
-    const long long blocks = (long long)((tiles_x + 7) / 8) * ((tiles_y + 7) / 8);
-    const long long groups = (blocks + 7) / 8 * 8 * 64;
-    if (groups > 0x7fffffffLL) return fail(FGS_E_INVALID, "%s: image too large", who);
+    // one workgroup per tile of the image padded to whole blocks of tiles, blocks padded to a multiple of 8
+    const long long blocks = (long long)((tiles_x + kBlock - 1) / kBlock) * ((tiles_y + kBlock - 1) / kBlock);
+    const long long groups = (blocks + 7) / 8 * 8 * (kBlock * kBlock);
+    if (groups > 0x7fffffffLL - kLongLists) return fail(FGS_E_INVALID, "%s: image too large", who);
     const int num_tiles = tiles_x * tiles_y;
     const bool fp32 = mode == FGS_COLOUR_SUMS_FP32;
 #define FGS_BLEND_ARGS (const int2*)ranges, values_sorted, width, height, tiles_x, tiles_y,                     \
@@ -1383,7 +1462,8 @@ int blend_impl(bool rank, int block_x, int block_y, int width, int height,
                        bg[0], bg[1], bg[2], out_u8, out_f32
     if (!is_ranked(tiles_x, tiles_y)) {
         auto launch = [&](auto kernel) {
-            hipLaunchKernelGGL(kernel, dim3((unsigned)groups), dim3(kWave * sx * sy), 0, st, FGS_BLEND_ARGS);
+            hipLaunchKernelGGL(kernel, dim3((unsigned)(groups + (longer.list ? kLongLists : 0))), dim3(kWave * sx * sy), 0, st, FGS_BLEND_ARGS,
+                               (const LongLists*)longer.list, longer.next, longer.least);
         };
         if (sx == 1 && sy == 1) launch(fp32 ? blend_kernel<1, 1, true> : blend_kernel<1, 1, false>);
         else if (sx == 2 && sy == 1) launch(fp32 ? blend_kernel<2, 1, true> : blend_kernel<2, 1, false>);
@@ -1433,9 +1513,15 @@ int render_impl(int block_x, int block_y, int num_rendered, int width, int heigh
     if (rc != FGS_OK) return rc;
     if (num_rendered > 0 && (!points_xy || !rgb_depth || !conic_opacity || !keys_sorted || !values_sorted))
         return fail(FGS_E_INVALID, "%s: null buffer", who);
-    rc = ranges_impl(block_x, block_y, num_rendered, width, height, keys_sorted, ranges, stream, who);
+    LongTable longer;
+    std::unique_lock<std::mutex> enqueue;       // from the launch that lists them to the blend that reads the table
+    if (width > 0 && height > 0) {
+        rc = long_table((hipStream_t)stream, num_rendered, block_x, block_y, width, height, &longer, &enqueue);
+        if (rc != FGS_OK) return rc;
+    }
+    rc = ranges_impl(block_x, block_y, num_rendered, width, height, keys_sorted, ranges, longer, stream, who);
     if (rc != FGS_OK) return rc;
-    return blend_impl(false, block_x, block_y, width, height, points_xy, rgb_depth, conic_opacity, values_sorted, ranges,
+    return blend_impl(false, longer, block_x, block_y, width, height, points_xy, rgb_depth, conic_opacity, values_sorted, ranges,
                       bg, out_u8, out_f32, flags, stream, who);
 }
 
@@ -1520,7 +1606,7 @@ extern "C" const char* fgs_blend_kernel_name(int block_x, int block_y, int width
 extern "C" int fgs_tile_ranges(int block_x, int block_y, int num_rendered, int width, int height,
                                const uint64_t* gaussian_keys_sorted, int* ranges, void* stream)
 {
-    return fgs::ranges_impl(block_x, block_y, num_rendered, width, height, gaussian_keys_sorted, ranges, stream,
+    return fgs::ranges_impl(block_x, block_y, num_rendered, width, height, gaussian_keys_sorted, ranges, fgs::LongTable(), stream,
                             "fgs_tile_ranges");
 }
 
@@ -1529,7 +1615,7 @@ extern "C" int fgs_blend(int block_x, int block_y, int width, int height,
                          const uint32_t* gaussian_values_sorted, const int* ranges, const float bg_color[3],
                          uint8_t* out_color_u8, float* out_color_f32, void* stream)
 {
-    return fgs::blend_impl(true, block_x, block_y, width, height, points_xy, rgb_depth, conic_opacity,
+    return fgs::blend_impl(true, fgs::LongTable(), block_x, block_y, width, height, points_xy, rgb_depth, conic_opacity,
                            gaussian_values_sorted, ranges, bg_color, out_color_u8, out_color_f32, 0, stream, "fgs_blend");
 }
 
@@ -1538,7 +1624,7 @@ extern "C" int fgs_blend_ex(int block_x, int block_y, int width, int height,
                             const uint32_t* gaussian_values_sorted, const int* ranges, const float bg_color[3],
                             uint8_t* out_color_u8, float* out_color_f32, int flags, void* stream)
 {
-    return fgs::blend_impl(true, block_x, block_y, width, height, points_xy, rgb_depth, conic_opacity,
+    return fgs::blend_impl(true, fgs::LongTable(), block_x, block_y, width, height, points_xy, rgb_depth, conic_opacity,
                            gaussian_values_sorted, ranges, bg_color, out_color_u8, out_color_f32, flags, stream, "fgs_blend_ex");
 }
 

@@ -748,6 +748,43 @@ def test_blend_one_tile_and_four_tiles_per_workgroup_agree(flags, rows):
     assert np.array_equal(images[0], images[1])
 
 
+@pytest.mark.parametrize("W,H,block", [(4096, 4111, (16, 16)), (8200, 4096, (32, 16)), (8192, 8223, (32, 32))])
+@pytest.mark.parametrize("long_tiles", [0, 3, 2000])      # none, a few, more than there are places for
+def test_long_lists_of_large_frames_start_first(W, H, block, long_tiles):
+    """From 65536 tiles on the launch that marks the ranges lists tiles with long lists (1024 entries here), which the
+    first workgroups of the blend take.  The image is that of fgs_blend, which lists none, bit for bit, in every one of
+    several frames on the two tables, with the first one finding whatever is in fresh memory."""
+    import gpu_pipeline as gp
+    from flashgs_amd import cabi
+    import torch
+    gx, gy = (W + block[0] - 1) // block[0], (H + block[1] - 1) // block[1]
+    assert gx * gy >= 1 << 16
+    rng = np.random.default_rng(long_tiles)
+    bg = np.array([0.2, 0.4, 0.6], np.float32)
+    st = torch.cuda.current_stream().cuda_stream
+    for frame in range(3):
+        n = rng.integers(30, 80, gx * gy)
+        n[rng.permutation(gx * gy)[:long_tiles]] = rng.choice([1023, 1024, 1025, 1087, 1088, 1500, 2600], long_tiles)
+        n[rng.permutation(gx * gy)[:200]] = 0
+        ends = np.cumsum(n)
+        K = int(ends[-1])
+        assert K >= 3 << 20
+        tile = np.repeat(np.arange(gx * gy), n)
+        V = 5000                                        # attributes of a few Gaussians, placed around every tile's corner
+        xy = rng.uniform(0, [W, H], (V, 2)).astype(np.float32)
+        co = np.stack([-rng.uniform(1e-7, 1e-6, V), rng.uniform(-1e-8, 1e-8, V), -rng.uniform(1e-7, 1e-6, V),
+                       np.log2(rng.uniform(0.0005, 0.01, V))], 1).astype(np.float32)
+        d = [gp.dev(a) for a in (xy, rng.uniform(0, 1, (V, 4)).astype(np.float32), co)]
+        ks, vs = gp.dev((tile.astype(np.int64) << 32) | 1), gp.dev(rng.integers(0, V, K).astype(np.int32))
+        ranges, _, listed = gp.render(K, W, H, d[0], d[1], d[2], ks, vs, bg, block)
+        assert np.array_equal(ranges.cpu().numpy()[n > 0], np.stack([ends - n, ends], 1)[n > 0])
+        out = torch.full((H, W, 3), -1.0, device=gp.DEV, dtype=torch.float32)
+        cabi.blend(block[0], block[1], W, H, d[0].data_ptr(), d[1].data_ptr(), d[2].data_ptr(), vs.data_ptr(), ranges.data_ptr(),
+                   bg, 0, out.data_ptr(), st)
+        torch.cuda.synchronize()
+        assert torch.equal(listed, out)
+
+
 def test_blend_long_lists_shared_between_waves(oracle):
     """A small frame blends its long lists with several teams: one takes the head of the list,
     the rest is cut into rounds of runs that start from T = 1 and are folded front to back.  Crafted
