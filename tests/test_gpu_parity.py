@@ -1139,6 +1139,25 @@ def test_rectangles_of_thousands_of_tiles(oracle, width, height, block, longest,
     assert np.array_equal(gp.u32(got["values"])[:K], pre["values"][:K])
 
 
+# tile sizes that are no powers of two, tiles of one pixel, and frames on either side of 2^23 pixels, up to where pixel coordinates
+# and their sums are exact floats and tiles are tested without integer products; rectangles of 1 to some thousand tiles
+@pytest.mark.parametrize("width, height, block, longest", [
+    (1999, 1003, (17, 23), 500), (96, 64, (1, 1), 101), (1999, 1003, (16, 16), 130), (3001, 1999, (32, 16), 2e3),
+    ((1 << 23) - 8192, 64, (4093, 16), 3e5), ((1 << 23) + 8192, 64, (4096, 16), 3e5), (64, (1 << 23) + 9000, (16, 4100), 3e5)])
+def test_tile_tests_of_any_tile_size(oracle, width, height, block, longest):
+    import gpu_pipeline as gp
+    sc, cam = _big_rectangles(3000, width, height, longest, 1e-2, 1, seed=width % 1000)
+    cap = 1 << 23
+    pre = oracle.preprocess(sc.position, sc.shs, sc.opacity, sc.cov3d, width, height, block[0], block[1],
+                            cam.position, cam.rotation, cam.focal_x, cam.focal_y, cam.zFar, cam.zNear, cap)
+    K = pre["num_rendered"]
+    assert 1000 < K < cap
+    got = gp.preprocess(gp.SceneOnDevice(sc), cam, cap, block)
+    assert got["num_rendered"] == K
+    assert np.array_equal(gp.u64(got["keys"])[:K], pre["keys"][:K])
+    assert np.array_equal(gp.u32(got["values"])[:K], pre["values"][:K])
+
+
 @pytest.fixture(scope="module")
 def config3_scene():
     return scenes.make(3)
