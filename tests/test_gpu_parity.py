@@ -1349,6 +1349,21 @@ def test_sort_around_the_list_lengths_where_the_launches_change(n, W, H):
     _sort_case(tile, depth, W, H, seed=n % 97, ascending=True)
 
 
+@pytest.mark.parametrize("n", [1, 64, 65, 1023, 1024, 1025, 2049, 4096, 4097])
+@pytest.mark.parametrize("W,H", [(16, 16), (256, 192), (496, 528), (512, 512), (4096, 4080)])     # 1, 1023, 1024 and 65280 tiles, a frame of a thumbnail
+def test_sort_of_lists_of_one_block(n, W, H):
+    """Lists of at most 4096 pairs in at most 1023 tiles, and of at most 1024 pairs in at most 65535, go through the partition as one
+    block, which counts its own digits; a segment of more than 1024 pairs is sorted beside the others.  All of them in any
+    tile, in one tile, in two, and with bits above the sorted range."""
+    rng = np.random.default_rng(n + W)
+    T = ((W + 15) // 16) * ((H + 15) // 16)
+    for tile in (rng.integers(0, T, n), np.full(n, T - 1), np.where(rng.random(n) < 0.4, 0, T - 1)):
+        depth = rng.integers(0x3e4ccccd, 0x42c80000, n).astype(np.uint32)
+        depth[::3] = depth[0]
+        for junk in (None, (rng.random(n) < 0.01).astype(np.uint32)):
+            _sort_case(tile.astype(np.uint32), depth, W, H, junk, seed=n)
+
+
 @pytest.mark.parametrize("n,W,H", [(1023, 640, 480), (1024, 640, 480), (1025, 640, 480), (200_001, 640, 480), (400_003, 1920, 1080),
                                    ((1 << 21) - 1, 1920, 1080), (1 << 21, 1920, 1080), ((1 << 21) + 1, 1920, 1080),
                                    (777, 7680, 4320), (131_072, 7680, 4320), (131_073, 7680, 4320), (262_145, 7680, 4320),
