@@ -1768,33 +1768,31 @@ extern "C" int fgs_sort_gaussian(int num_rendered,
                 if (first && last) FGS_SCATTER(kPairs, kSegments, , true);
                 else if (first) FGS_SCATTER(kPairs, kWords, , true);
                 else FGS_SCATTER(kWords, kSegments, , true);
-                src_k = dst_k;
-                src_v = dst_v;
-                continue;
+            } else {
+                uint32_t* const beyond = first ? marks + kMarkBeyond : nullptr;
+                uint32_t* const clear = last ? seg_counts : nullptr;
+                auto count = [&](auto* in) {
+                    using In = std::remove_cv_t<std::remove_pointer_t<decltype(in)>>;
+                    if (small) {
+                        hipLaunchKernelGGL((count_kernel<Shape, In>), dim3(g.tiles), dim3(kSortBlock), 0, st,
+                                           in, n, shift, nbits, hist, ~tile_mask, beyond, clear);
+                    } else {
+                        const int groups = g.chunk < kCountGroups ? g.chunk : kCountGroups;
+                        hipLaunchKernelGGL((count_chunk_kernel<Shape, In>), dim3(g.chunks), dim3(groups * kSortBlock), 0, st,
+                                           in, n, shift, nbits, hist, g.tiles, g.chunk, chunk_sums, ~tile_mask, beyond, clear);
+                        hipLaunchKernelGGL((offsets_kernel<Shape>), dim3(g.chunks), dim3(g.chunks > 16 ? kOffsetThreads : Shape::kBinsP), 0, st,
+                                           hist, g.tiles, g.chunk, chunk_sums, g.chunks, first ? marks : nullptr);
+                    }
+                };
+                if (from_words) count((const Next*)src_v);
+                else count(src_k);
+                const uint32_t* const beyond_at = marks + (small ? kMarkBeyond : kMarkByIndex);
+                const int beyond_rows = !first ? 0 : small ? g.tiles : 1;
+                if (!words) FGS_SCATTER(kPairs, kPairs);
+                else if (first && last) FGS_SCATTER(kPairs, kSegments);
+                else if (first) FGS_SCATTER(kPairs, kWords);
+                else FGS_SCATTER(kWords, kSegments);
             }
-            uint32_t* const beyond = first ? marks + kMarkBeyond : nullptr;
-            uint32_t* const clear = last ? seg_counts : nullptr;
-            auto count = [&](auto* in) {
-                using In = std::remove_cv_t<std::remove_pointer_t<decltype(in)>>;
-                if (small) {
-                    hipLaunchKernelGGL((count_kernel<Shape, In>), dim3(g.tiles), dim3(kSortBlock), 0, st,
-                                       in, n, shift, nbits, hist, ~tile_mask, beyond, clear);
-                } else {
-                    const int groups = g.chunk < kCountGroups ? g.chunk : kCountGroups;
-                    hipLaunchKernelGGL((count_chunk_kernel<Shape, In>), dim3(g.chunks), dim3(groups * kSortBlock), 0, st,
-                                       in, n, shift, nbits, hist, g.tiles, g.chunk, chunk_sums, ~tile_mask, beyond, clear);
-                    hipLaunchKernelGGL((offsets_kernel<Shape>), dim3(g.chunks), dim3(g.chunks > 16 ? kOffsetThreads : Shape::kBinsP), 0, st,
-                                       hist, g.tiles, g.chunk, chunk_sums, g.chunks, first ? marks : nullptr);
-                }
-            };
-            if (from_words) count((const Next*)src_v);
-            else count(src_k);
-            const uint32_t* const beyond_at = marks + (small ? kMarkBeyond : kMarkByIndex);
-            const int beyond_rows = !first ? 0 : small ? g.tiles : 1;
-            if (!words) FGS_SCATTER(kPairs, kPairs);
-            else if (first && last) FGS_SCATTER(kPairs, kSegments);
-            else if (first) FGS_SCATTER(kPairs, kWords);
-            else FGS_SCATTER(kWords, kSegments);
 #undef FGS_SCATTER
             src_k = dst_k;
             src_v = dst_v;
