@@ -334,8 +334,11 @@ def stage_report(fr, stage_ms, K, counts, walked):
     else:
         stages["preprocess"] = dict(ms=round(stage_ms["preprocess"], 4), bound="hbm")
     hbm("sort", K * (8 + 24 * passes))
-    tile_passes = (int(tiles).bit_length() + 7) // 8
-    stages["sort"]["design_bytes"] = int(K * (32 * tile_passes + 8 + 24))   # count + scatter per tile digit, starts, segment sort
+    # counts, scatters and the segment sort; with one or two passes pairs travel as words beside `digit` bytes of the tile id
+    bits = int(tiles).bit_length()
+    digit = 1 if bits <= 16 else 2
+    per_pair = 48 if bits <= 8 else 64 + 3 * digit if bits <= 18 else 32 * ((bits + 7) // 8) + 8 + 24
+    stages["sort"]["design_bytes"] = int(K * per_pair)
     hbm("ranges", 8 * K + 16 * tiles)
     # GPU time between the preprocess launch and the first sort launch (the host polls the pair count in pinned memory and
     # enqueues the sort while the launch still writes keys)
