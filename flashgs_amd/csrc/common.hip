@@ -25,6 +25,15 @@ int check_hip(hipError_t st, const char* what)
     return fail(FGS_E_HIP, "%s: %s", what, hipGetErrorString(st));
 }
 
+hipError_t malloc_kept(void** out, size_t bytes)
+{
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    const bool relaxed = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+    const hipError_t st = hipMalloc(out, bytes);
+    if (relaxed) (void)hipThreadExchangeStreamCaptureMode(&mode);      // (mode: what this thread had before)
+    return st;
+}
+
 } // namespace fgs
 
 extern "C" const char* fgs_last_error(void) { return fgs::g_last_error; }

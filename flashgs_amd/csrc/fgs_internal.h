@@ -18,6 +18,10 @@ int fail(int code, const char* fmt, ...);
 // Maps a HIP status to FGS_OK / FGS_E_HIP (recording the HIP error text).
 int check_hip(hipError_t st, const char* what);
 
+// hipMalloc for memory that the library keeps, beside captures of other threads: one that was begun in the global mode, as captures are by
+// default, fails once a thread that has not asked for the relaxed mode allocates.  (A caller whose own stream is being captured does not come here.)
+hipError_t malloc_kept(void** out, size_t bytes);
+
 #define FGS_HIP_TRY(expr)                                  \
     do {                                                   \
         int _rc = ::fgs::check_hip((expr), #expr);         \

@@ -1137,7 +1137,7 @@ int acquire_scratch(int device, int num_blocks, hipStream_t stream, Scratch** ou
         while (cap < (size_t)num_blocks) cap <<= 1;
         const size_t words = kControlWords + 4 * cap;
         uint64_t* fresh = nullptr;
-        if (hipMalloc((void**)&fresh, words * sizeof(uint64_t)) != hipSuccess) {
+        if (malloc_kept((void**)&fresh, words * sizeof(uint64_t)) != hipSuccess) {
             (void)hipGetLastError();
             return fail(FGS_E_NOMEM, "cannot allocate %zu bytes of scan status", words * sizeof(uint64_t));
         }

@@ -88,7 +88,7 @@ int tile_order_table(hipStream_t stream, uint32_t** out, std::unique_lock<std::m
         entry = &g_order_tables[stream_key(device, stream)];
     }
     *enqueue = std::unique_lock<std::mutex>(entry->enqueue);
-    if (!entry->ranks && hipMalloc((void**)&entry->ranks, (kOrderCap + 2) * sizeof(uint32_t) + 2 * sizeof(LongLists)) != hipSuccess) {
+    if (!entry->ranks && malloc_kept((void**)&entry->ranks, (kOrderCap + 2) * sizeof(uint32_t) + 2 * sizeof(LongLists)) != hipSuccess) {
         (void)hipGetLastError();
         entry->ranks = nullptr;
     }

@@ -622,6 +622,69 @@ def test_blends_replayed_beside_each_other(block):
             assert torch.equal(f[3], f[2]), "replay %d" % replay
 
 
+def test_first_calls_on_a_stream_beside_a_capture():
+    """The first calls on a stream allocate what the library keeps for it (scan words, the table of ranked tiles and of the long lists of
+    a frame of 65536 tiles and more).  A capture that another thread has begun meanwhile, in the default mode, goes on and replays."""
+    import threading
+    import gpu_pipeline as gp
+    import torch
+    from flashgs_amd import cabi
+    sc = scenes.config0(n=20_000)
+    cam = sc.cameras[0]
+    sd = gp.SceneOnDevice(sc)
+    pre = gp.preprocess(sd, cam, 1 << 18)
+    K, W, H = pre["num_rendered"], cam.width, cam.height
+    bg = np.array([0.2, 0.4, 0.6], np.float32)
+    ks, vs = gp.sort(K, W, H, pre["keys"], pre["values"])
+    ranges, eager, _ = gp.render(K, W, H, pre["points_xy"], pre["rgb_depth"], pre["conic_opacity"], ks, vs, bg, f32=False)
+    # a frame of 65792 tiles with 48 entries each, two lists of 3000 among them
+    LW, LH, V = 4096, 4111, 1000
+    n = np.full(256 * 257, 48)
+    n[[77, 40_000]] = 3000
+    rng = np.random.default_rng(1)
+    large = [gp.dev(a) for a in (rng.uniform(0, [LW, LH], (V, 2)).astype(np.float32), rng.uniform(0, 1, (V, 4)).astype(np.float32),
+                                 np.stack([-rng.uniform(1e-7, 1e-6, V), rng.uniform(-1e-8, 1e-8, V), -rng.uniform(1e-7, 1e-6, V),
+                                           np.log2(rng.uniform(0.0005, 0.01, V))], 1).astype(np.float32),
+                                 np.repeat(np.arange(n.size), n).astype(np.int64) << 32, rng.integers(0, V, n.sum()).astype(np.int32))]
+    large_ranges, large_eager, _ = gp.render(int(n.sum()), LW, LH, *large, bg, f32=False)
+    keys, values = torch.zeros_like(pre["keys"]), torch.zeros_like(pre["values"])
+    offset = torch.zeros(1, device=gp.DEV, dtype=torch.int32)
+    image, large_image = torch.zeros_like(eager), torch.zeros_like(large_eager)
+    x = torch.zeros(1024, device=gp.DEV)
+    fresh, side, failed = torch.cuda.Stream(), torch.cuda.Stream(), []
+    torch.cuda.synchronize()
+
+    def first_calls():
+        try:
+            st = fresh.cuda_stream
+            cabi.preprocess(sd.n, sd.position.data_ptr(), sd.shs.data_ptr(), sd.opacity.data_ptr(), sd.cov3d.data_ptr(), W, H, 16, 16,
+                            cam.position, cam.rotation, cam.focal_x, cam.focal_y, cam.zFar, cam.zNear, pre["points_xy"].data_ptr(),
+                            pre["rgb_depth"].data_ptr(), pre["conic_opacity"].data_ptr(), keys.data_ptr(), values.data_ptr(), offset.data_ptr(),
+                            1 << 18, st)
+            cabi.render(16, 16, int(n.sum()), LW, LH, *[t.data_ptr() for t in large], large_ranges.data_ptr(), bg, large_image.data_ptr(), st)
+            cabi.blend(16, 16, W, H, pre["points_xy"].data_ptr(), pre["rgb_depth"].data_ptr(), pre["conic_opacity"].data_ptr(), vs.data_ptr(),
+                       ranges.data_ptr(), bg, image.data_ptr(), 0, st)
+        except Exception as error:
+            failed.append(error)
+
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        x += 1
+        other = threading.Thread(target=first_calls)
+        other.start()
+        other.join()
+        x += 1
+    assert not failed, failed
+    x.zero_()
+    torch.cuda.synchronize()
+    for replay in range(1, 4):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert bool((x == 2 * replay).all())
+    assert np.array_equal(gp.u64(keys)[:K], gp.u64(pre["keys"])[:K]) and int(offset[0]) == K
+    assert torch.equal(large_image, large_eager) and torch.equal(image, eager)
+
+
 def test_repeated_frames_are_deterministic():
     import gpu_pipeline as gp
     sc = scenes.config0(n=50_000)
