@@ -230,8 +230,12 @@ __global__ __launch_bounds__(256) void tile_ranges_kernel(int L, const uint64_t*
 // 66 by this one, 14.5M pairs there 22.1 and 18.2, 11.6M in 32 400 18.5 and 12.7, 8.0M 13.9 and 10.7, 5.2M in 8160 10.3 and 5.5.
 // (16 runs per wave: 51, 20.4, 12.0, 12.4 and 5.8.  A bisection by each lane where its 64 keys end in another tile: 41, 26.5, 5.6,
 // 7.4 and 4.3, but 19.6 in place of 4.4 where 1.7M pairs lie unevenly: one dependent chain per border.)
+//
+// kList: it also lists the tiles whose lists are long (LongLists): the one tile of the wave that begins in its runs and goes on behind them is looked
+// for again long_list pairs (more than the wave's) further on.  That is a line of its own, and it is waited for behind the borders.
 constexpr int kRangeRuns = 8;
 
+template <bool kList>
 __global__ __launch_bounds__(256) void tile_ranges_sampled_kernel(int L, const uint64_t* __restrict__ keys,
                                                                   int2* __restrict__ ranges, uint32_t num_tiles,
                                                                   LongLists* __restrict__ longer, int long_list)
@@ -244,15 +248,12 @@ __global__ __launch_bounds__(256) void tile_ranges_sampled_kernel(int L, const u
     uint32_t last = 0, before = 0;
     if (mine) last = tile_at(end - 1);
     if (lane == 0 && mine && begin > 0) before = tile_at(begin - 1);
-    uint32_t ahead = num_tiles;
-    if (longer && mine && end - 1 + long_list < L) ahead = tile_at(end - 1 + long_list);
     const uint32_t left = (uint32_t)__shfl_up((int)last, 1);
     if (lane > 0) before = left;
-    // the tile that begins in this run and goes on behind it: still there long_list pairs further on?
-    if (mine && (last != before || begin == 0) && last < num_tiles && ahead == last) {
-        const uint32_t shard = long_shard(last), at = atomicAdd(&longer->count[shard], 1u);
-        if (at < (uint32_t)kLongPerShard) longer->tiles[shard][at] = last;
-    }
+    const bool goes_on = last == (uint32_t)__shfl((int)last, kRangeRuns - 1) && end - 1 + long_list < L;
+    const bool begins = kList && mine && goes_on && (last != before || begin == 0) && last < num_tiles;
+    uint32_t ahead = ~0u;
+    if (begins) ahead = ((const uint32_t*)keys)[2 * (end - 1 + long_list) + 1];     // (nothing but the load: a use in here would be waited for)
     uint64_t todo = ballot(mine && (last != before || begin == 0 || end == L));
     while (todo) {
         long long idx[kRangesPerThread];
@@ -272,6 +273,10 @@ __global__ __launch_bounds__(256) void tile_ranges_sampled_kernel(int L, const u
             const uint32_t left_key = (uint32_t)__shfl_up((int)cur[k], 1);
             mark_ranges(idx[k], valid[k], cur[k], lane > 0 ? left_key : prev[k], L, ranges, num_tiles);
         }
+    }
+    if (begins && ahead == last) {
+        const uint32_t shard = long_shard(last), at = atomicAdd(&longer->count[shard], 1u);
+        if (at < (uint32_t)kLongPerShard) longer->tiles[shard][at] = last;
     }
 }
 
@@ -1362,10 +1367,12 @@ struct LongTable {
 
 // A list is long for its frame if it has a seventh of the entries that a SIMD has on average: it takes 166 ns per entry beside others
 // where a SIMD takes 50, so half of the launch.
-// Only frames of kLongTiles tiles and more have such lists often enough (8K / 8M Gaussians, 129 600 tiles: blend 695 -> 639 us, ranges
-// 18.2 -> 22.6; 57 600 tiles 444 -> 441 and 16.5 -> 19.1, 32 400 319 -> 320 and 12.3 -> 16.8), and none where a seventh is more than
+// Only frames of kLongTiles tiles and more have such lists often enough (8K / 8M Gaussians, 129 600 tiles: ranges and blend 675 -> 625 us, 3 of the
+// ranges' 23 for the listing; 6620x4058 / 29.6M pairs and 4797x3666 / 15.5M, where none ends late: 1 % more; before the listing cost that little:
+// 57 600 tiles blend 444 -> 441 us and ranges 16.5 -> 19.1, 32 400 319 -> 320 and 12.3 -> 16.8), and none where a seventh is more than
 // kLongMost entries: lists that long are opaque long before their end (110M pairs: 477 -> 479 and 88 -> 128).
-constexpr int kLongTiles = 1 << 16, kLongMost = 8192;
+constexpr int kLongTiles = 1 << 16, kLongLeast = 1024, kLongMost = 8192;
+static_assert(kLongLeast > kRangeRuns * kWave, "a tile that tile_ranges_sampled_kernel lists goes on behind the wave's runs");
 int long_table(hipStream_t stream, int num_rendered, int block_x, int block_y, int width, int height, LongTable* out, std::unique_lock<std::mutex>* enqueue)
 {
     const int tiles_x = (width + block_x - 1) / block_x, tiles_y = (height + block_y - 1) / block_y;
@@ -1383,7 +1390,7 @@ int long_table(hipStream_t stream, int num_rendered, int block_x, int block_y, i
     out->list = both + entry->turn;
     out->next = both + (entry->turn ^ 1);
     entry->turn ^= 1;
-    out->least = (int)std::max(seventh, 1024LL);
+    out->least = (int)std::max(seventh, (long long)kLongLeast);
     return FGS_OK;
 }
 
@@ -1406,7 +1413,7 @@ int ranges_impl(int block_x, int block_y, int num_rendered, int width, int heigh
     if (num_rendered == 0)
         hipLaunchKernelGGL(fill_i32_kernel, dim3((unsigned)fill_blocks), dim3(256), 0, st, ranges, words, 0);
     else if (num_rendered >= kSampledPairs)
-        hipLaunchKernelGGL(tile_ranges_sampled_kernel,
+        hipLaunchKernelGGL(longer.list ? tile_ranges_sampled_kernel<true> : tile_ranges_sampled_kernel<false>,
                            dim3((unsigned)(((size_t)num_rendered + 4 * kRangeRuns * kWave - 1) / (4 * kRangeRuns * kWave))),
                            dim3(256), 0, st, num_rendered, keys_sorted, (int2*)ranges,
                            (uint32_t)(num_tiles > 0xffffffffu ? 0xffffffffu : num_tiles), longer.list, longer.least);
