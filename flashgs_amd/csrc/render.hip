@@ -886,28 +886,6 @@ __device__ __forceinline__ void write_square(
     }
 }
 
-// Position in the launch -> tile.  The hardware deals consecutive workgroups out to the 8 XCDs in
-// turn, and every XCD has its own L2.  Neighbouring tiles share most of their Gaussians, so each
-// XCD is given whole blocks of 4x4 tiles (its positions g = 8*slot + xcd walk blocks xcd, xcd+8,
-// ... 16 tiles at a time): a Gaussian's attribute lines are then fetched into one L2 once instead
-// of into several L2s once per tile.  Every row of blocks begins further right, so that the blocks below each other
-// belong to XCDs five apart whatever the width of the frame: with blocks of 8x8 row after row from the left, an XCD had the same columns of
-// blocks in every second row of a frame of 60 blocks, in every row of one of 24, and 2 to 14 % more to blend than the average, and
-// the launch ends when the last XCD does (3000x2200 / 2M 231 -> 215 us, 8K / 8M 704 -> 683, 5120x2880 448 -> 438, 4K 320 -> 319; blocks of
-// 8x8 five apart 213, 685, 435, 322, 4x4 three apart 216, 691, 443, 316).  False for the padding positions.
-constexpr int kBlockLog2 = 2, kBlock = 1 << kBlockLog2;
-__device__ __forceinline__ bool tile_of_position(int group, int tiles_x, int tiles_y, int* tile_x, int* tile_y)
-{
-    const int xcd = group & 7, slot = group >> 3;
-    const int blocks_x = (tiles_x + kBlock - 1) >> kBlockLog2;
-    const int block = (slot >> (2 * kBlockLog2)) * 8 + xcd, inner = slot & (kBlock * kBlock - 1);
-    const int row = block / blocks_x;
-    const int column = (block - row * blocks_x + ((blocks_x - 5) & 7) * row) % blocks_x;
-    *tile_x = column * kBlock + (inner & (kBlock - 1));
-    *tile_y = row * kBlock + (inner >> kBlockLog2);
-    return *tile_x < tiles_x && *tile_y < tiles_y;
-}
-
 #define FGS_BLEND_PARAMS                                                                         \
     const int2* __restrict__ ranges, const uint32_t* __restrict__ point_list,                   \
     int width, int height, int tiles_x, int tiles_y,                                            \
@@ -1459,8 +1437,7 @@ int blend_impl(bool rank, const LongTable& longer, int block_x, int block_y, int
     const int tiles_x = (width + block_x - 1) / block_x, tiles_y = (height + block_y - 1) / block_y;
     hipStream_t st = (hipStream_t)stream;
     // one workgroup per tile of the image padded to whole blocks of tiles, blocks padded to a multiple of 8
-    const long long blocks = (long long)((tiles_x + kBlock - 1) / kBlock) * ((tiles_y + kBlock - 1) / kBlock);
-    const long long groups = (blocks + 7) / 8 * 8 * (kBlock * kBlock);
+    const long long groups = positions_of(tiles_x, tiles_y);
     if (groups > 0x7fffffffLL - kLongLists) return fail(FGS_E_INVALID, "%s: image too large", who);
     const int num_tiles = tiles_x * tiles_y;
     const bool fp32 = mode == FGS_COLOUR_SUMS_FP32;
