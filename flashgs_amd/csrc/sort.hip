@@ -1673,7 +1673,7 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(7))) void
             if (len > kT * kWave && threadIdx.x == 0) {
                 // neighbouring tiles tend to be equally busy: mix the index so that every list gets its share
                 const uint32_t shard = (v ^ (v >> 5) ^ (v >> 10) ^ (v >> 15)) % kListShards;
-                if (len <= list_max0)
+                if (kT * kWave < kCapSmall && len <= list_max0)
                     list0[(size_t)shard * list_cap0 + atomicAdd(&seg_counts[0 * kListShards + shard], 1u)] = v;
                 else if (len <= list_max1)
                     list1[(size_t)shard * list_cap1 + atomicAdd(&seg_counts[1 * kListShards + shard], 1u)] = v;
@@ -1894,6 +1894,11 @@ extern "C" int fgs_sort_gaussian(int num_rendered,
     auto partition = [&](auto shape) {
         using Shape = decltype(shape);
         using Next = NextDigit<Shape>;
+        // (what the forms below are compiled for: digits of 8 bits take one or two passes, which carry words, digits of 9 bits two or more)
+        constexpr bool kOnePass = Shape::kBits == 8;
+        static_assert(kNarrowMaxTileBits <= 16 && kNarrowMaxTileBits <= kWordsMaxTileBits && kNarrowMaxTileBits >= 9, "digits of 8 and 9 bits");
+        constexpr bool kAlwaysSmall = std::is_same_v<Shape, Short>;
+        static_assert(kShortPairs / Short::kTile * Short::kBinsP <= kMostRowWords, "a list of such blocks has few rows");
         const PassGrid g = pass_grid(n, Shape::kTile);
         const bool small = g.tiles * Shape::kBinsP <= kMostRowWords;     // the scatter workgroups add up the histogram rows themselves
         const int passes = (tile_bits + Shape::kBits - 1) / Shape::kBits;
@@ -1925,7 +1930,7 @@ extern "C" int fgs_sort_gaussian(int num_rendered,
                     if (small) {
                         hipLaunchKernelGGL((count_kernel<Shape, In>), dim3(g.tiles), dim3(kSortBlock), 0, st,
                                            in, n, shift, nbits, hist, ~tile_mask, beyond, clear);
-                    } else {
+                    } else if constexpr (!kAlwaysSmall) {
                         const int groups = g.chunk < kCountGroups ? g.chunk : kCountGroups;
                         hipLaunchKernelGGL((count_chunk_kernel<Shape, In>), dim3(g.chunks), dim3(groups * kSortBlock), 0, st,
                                            in, n, shift, nbits, hist, g.tiles, g.chunk, chunk_sums, ~tile_mask, beyond, clear);
@@ -1937,10 +1942,13 @@ extern "C" int fgs_sort_gaussian(int num_rendered,
                 else count(src_k);
                 const uint32_t* const beyond_at = marks + (small ? kMarkBeyond : kMarkByIndex);
                 const int beyond_rows = !first ? 0 : small ? g.tiles : 1;
-                if (!words) FGS_SCATTER(kPairs, kPairs);
-                else if (first && last) FGS_SCATTER(kPairs, kSegments);
-                else if (first) FGS_SCATTER(kPairs, kWords);
-                else FGS_SCATTER(kWords, kSegments);
+                if constexpr (kOnePass) {
+                    if (first && last) FGS_SCATTER(kPairs, kSegments);
+                } else {
+                    if (!words) FGS_SCATTER(kPairs, kPairs);
+                }
+                if (words && first && !last) FGS_SCATTER(kPairs, kWords);
+                if (words && !first) FGS_SCATTER(kWords, kSegments);
             }
 #undef FGS_SCATTER
             src_k = dst_k;
