@@ -811,41 +811,167 @@ def test_blend_one_tile_and_four_tiles_per_workgroup_agree(flags, rows):
     assert np.array_equal(images[0], images[1])
 
 
+def _long_lists_frame(W, H, block, long_lists, seed, each=(30, 80), opacity=(0.0005, 0.01)):
+    """A frame of 65536 tiles and more: (tensors as render() takes them, ranges, how many of its lists each of the table's 32 shards
+    lists).  Most lists have `each` entries; the long ones follow the length from which a list is long for the frame."""
+    import gpu_pipeline as gp
+    import torch
+    gx, gy = (W + block[0] - 1) // block[0], (H + block[1] - 1) // block[1]
+    T = gx * gy
+    assert T >= 1 << 16
+    rng = np.random.default_rng(seed)
+    shard = lambda t: (t ^ (t >> 5) ^ (t >> 10)) % 32
+    n = rng.integers(*each, T)
+    n[rng.permutation(T)[:200]] = 0
+    places, lengths = long_lists(rng, T, shard)
+    least = 1024
+    for _ in range(50):                     # (longer lists make more pairs, of which the length is a share)
+        n[places] = lengths(least)
+        now = max(1024, int(n.sum()) * (block[0] // 16) * (block[1] // 16) // (4 * torch.cuda.get_device_properties(0).multi_processor_count) // 7)
+        if now == least: break
+        least = now
+    else:
+        assert False, "no such lengths"
+    K = int(n.sum())
+    assert 3 << 20 <= K and least <= 8192
+    ends = np.cumsum(n)
+    begins = ends - n
+    listed = np.flatnonzero((begins // 64 + 1) * 64 - 1 + least < ends)       # still there so many pairs behind the run of 64 it begins in
+    V = 5000                                        # attributes of a few Gaussians
+    xy = rng.uniform(0, [W, H], (V, 2)).astype(np.float32)
+    co = np.stack([-rng.uniform(1e-7, 1e-6, V), rng.uniform(-1e-8, 1e-8, V), -rng.uniform(1e-7, 1e-6, V),
+                   np.log2(rng.uniform(*opacity, V))], 1).astype(np.float32)
+    tensors = [gp.dev(t) for t in (xy, rng.uniform(0, 1, (V, 4)).astype(np.float32), co, np.repeat(np.arange(T, dtype=np.int64), n) << 32,
+                                   rng.integers(0, V, K).astype(np.int32))]
+    return K, tensors, np.stack([begins, ends], 1), n, np.bincount(shard(listed), minlength=32)
+
+
+def _fresh_stream():
+    """A stream that no call has used, with a handle that none had (it is never destroyed)."""
+    import ctypes as C
+    import torch
+    hip = C.CDLL("libamdhip64.so")
+    handle = C.c_void_p()
+    assert hip.hipStreamCreate(C.byref(handle)) == 0
+    return torch.cuda.ExternalStream(handle.value)
+
+
+def _no_long_lists(rng, T, shard):
+    return np.arange(7, 13), lambda least: np.array([least - 64, least - 1, least, 1000, 700, 1])
+
+
+def _a_few_long_lists(rng, T, shard):
+    return rng.permutation(T)[:8], lambda least: least + np.array([-1, 0, 1, 63, 64, 65, 400, 2 * least])
+
+
+def _more_long_lists_than_places(rng, T, shard):
+    places = rng.permutation(T)
+    crowded = np.concatenate([places[shard(places) == k][:40] for k in (0, 13, 31)] + [places[shard(places) == 5][:16], places[shard(places) == 6][:17]])
+    return crowded, lambda least: least + 65 + np.arange(crowded.size) * 5
+
+
 @pytest.mark.parametrize("W,H,block", [(4096, 4111, (16, 16)), (8200, 4096, (32, 16)), (8192, 8223, (32, 32))])
-@pytest.mark.parametrize("long_tiles", [0, 3, 2000])      # none, a few, more than there are places for
-def test_long_lists_of_large_frames_start_first(W, H, block, long_tiles):
-    """From 65536 tiles on the launch that marks the ranges lists tiles with long lists (1024 entries here), which the
-    first workgroups of the blend take.  The image is that of fgs_blend, which lists none, bit for bit, in every one of
-    several frames on the two tables, with the first one finding whatever is in fresh memory."""
+@pytest.mark.parametrize("long_lists, fewest, most", [(_no_long_lists, 0, 0), (_a_few_long_lists, 3, 8), (_more_long_lists_than_places, 16, 40)])
+def test_long_lists_of_large_frames_start_first(W, H, block, long_lists, fewest, most):
+    """From 65536 tiles on the launch that marks the ranges lists tiles with long lists, which the
+    first workgroups of the blend take: none, a few around the length from which a list is long, and more than a shard of the table has
+    room for (16).  The image is that of fgs_blend, which lists none, bit for bit, in every one of
+    several frames on the two tables of a stream of its own, with the first one finding whatever is in fresh memory."""
     import gpu_pipeline as gp
     from flashgs_amd import cabi
     import torch
-    gx, gy = (W + block[0] - 1) // block[0], (H + block[1] - 1) // block[1]
-    assert gx * gy >= 1 << 16
-    rng = np.random.default_rng(long_tiles)
     bg = np.array([0.2, 0.4, 0.6], np.float32)
-    st = torch.cuda.current_stream().cuda_stream
+    stream = _fresh_stream()
     for frame in range(3):
-        n = rng.integers(30, 80, gx * gy)
-        n[rng.permutation(gx * gy)[:long_tiles]] = rng.choice([1023, 1024, 1025, 1087, 1088, 1500, 2600], long_tiles)
-        n[rng.permutation(gx * gy)[:200]] = 0
-        ends = np.cumsum(n)
-        K = int(ends[-1])
-        assert K >= 3 << 20
-        tile = np.repeat(np.arange(gx * gy), n)
-        V = 5000                                        # attributes of a few Gaussians, placed around every tile's corner
-        xy = rng.uniform(0, [W, H], (V, 2)).astype(np.float32)
-        co = np.stack([-rng.uniform(1e-7, 1e-6, V), rng.uniform(-1e-8, 1e-8, V), -rng.uniform(1e-7, 1e-6, V),
-                       np.log2(rng.uniform(0.0005, 0.01, V))], 1).astype(np.float32)
-        d = [gp.dev(a) for a in (xy, rng.uniform(0, 1, (V, 4)).astype(np.float32), co)]
-        ks, vs = gp.dev((tile.astype(np.int64) << 32) | 1), gp.dev(rng.integers(0, V, K).astype(np.int32))
-        ranges, _, listed = gp.render(K, W, H, d[0], d[1], d[2], ks, vs, bg, block)
-        assert np.array_equal(ranges.cpu().numpy()[n > 0], np.stack([ends - n, ends], 1)[n > 0])
-        out = torch.full((H, W, 3), -1.0, device=gp.DEV, dtype=torch.float32)
-        cabi.blend(block[0], block[1], W, H, d[0].data_ptr(), d[1].data_ptr(), d[2].data_ptr(), vs.data_ptr(), ranges.data_ptr(),
-                   bg, 0, out.data_ptr(), st)
+        K, d, ranges_of, n, in_shard = _long_lists_frame(W, H, block, long_lists, 10 * frame + block[1])
+        if fewest < 16:
+            assert fewest <= in_shard.sum() <= most
+        else:
+            assert in_shard[[0, 13, 31]].min() > 16 and in_shard[5] == 16 and in_shard[6] == 17 and in_shard.max() == most
         torch.cuda.synchronize()
+        with torch.cuda.stream(stream):
+            ranges, _, listed = gp.render(K, W, H, *d, bg, block)
+            out = torch.full((H, W, 3), -1.0, device=gp.DEV, dtype=torch.float32)
+            cabi.blend(block[0], block[1], W, H, d[0].data_ptr(), d[1].data_ptr(), d[2].data_ptr(), d[4].data_ptr(), ranges.data_ptr(),
+                       bg, 0, out.data_ptr(), stream.cuda_stream)
+            torch.cuda.synchronize()
+        assert np.array_equal(ranges.cpu().numpy()[n > 0], ranges_of[n > 0])
         assert torch.equal(listed, out)
+
+
+def test_a_long_list_of_the_last_tile_starts_first():
+    """300 entries in 65 792 tiles and some 6000, never opaque, in the last three: fgs_render starts those with the first workgroups, fgs_blend,
+    which lists none, with the last ones, behind which they are walked alone."""
+    import gpu_pipeline as gp
+    from flashgs_amd import cabi
+    import torch
+    W, H, bg = 4096, 4111, np.zeros(3, np.float32)
+    K, d, _, _, in_shard = _long_lists_frame(W, H, (16, 16), lambda rng, T, shard: (np.arange(T - 3, T), lambda least: np.full(3, 6000)), 1,
+                                             each=(295, 305), opacity=(0.0002, 0.0003))
+    assert in_shard.sum() == 3
+    ranges = torch.zeros((256 * 257, 2), device=gp.DEV, dtype=torch.int32)
+    out = torch.zeros((H, W, 3), device=gp.DEV, dtype=torch.uint8)
+    st = torch.cuda.current_stream().cuda_stream
+
+    def by_render():
+        cabi.render(16, 16, K, W, H, *[t.data_ptr() for t in d], ranges.data_ptr(), bg, out.data_ptr(), st)
+
+    def by_operators():
+        cabi.tile_ranges(16, 16, K, W, H, d[3].data_ptr(), ranges.data_ptr(), st)
+        cabi.blend(16, 16, W, H, d[0].data_ptr(), d[1].data_ptr(), d[2].data_ptr(), d[4].data_ptr(), ranges.data_ptr(), bg, out.data_ptr(), 0, st)
+
+    times = {by_render: [], by_operators: []}
+    for _ in range(12):
+        for f in times:
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            f()
+            b.record()
+            b.synchronize()
+            times[f].append(a.elapsed_time(b))
+    assert min(times[by_render]) < 0.85 * min(times[by_operators]), {f.__name__: min(t) for f, t in times.items()}
+
+
+def test_large_frames_captured_and_from_two_threads():
+    """Two frames with long lists: one captured and replayed beside eager renders of the other on the stream it was captured on (captured
+    frames have no table), then each from a thread of its own, on one stream and on one each."""
+    import threading
+    import gpu_pipeline as gp
+    from flashgs_amd import cabi
+    import torch
+    W, H, bg = 4096, 4111, np.array([0.2, 0.4, 0.6], np.float32)
+    frames = []
+    for seed in (3, 4):
+        K, d, _, _, in_shard = _long_lists_frame(W, H, (16, 16), _more_long_lists_than_places, seed)
+        ranges, _, want = gp.render(K, W, H, *d, bg)
+        out = torch.zeros_like(want)
+
+        def render(stream, K=K, d=d, ranges=ranges, out=out):
+            cabi.render_f32(16, 16, K, W, H, *[t.data_ptr() for t in d], ranges.data_ptr(), bg, 0, out.data_ptr(), stream)
+
+        frames.append((render, out, want))
+    assert not torch.equal(frames[0][2], frames[1][2])
+    side, other = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        frames[0][0](torch.cuda.current_stream().cuda_stream)
+    for replay in range(3):
+        for f in frames: f[1].zero_()
+        torch.cuda.synchronize()
+        with torch.cuda.stream(side):
+            graph.replay()
+        frames[1][0](side.cuda_stream)
+        torch.cuda.synchronize()
+        for f in frames: assert torch.equal(f[1], f[2]), "replay %d" % replay
+    for streams in ((side, side), (side, other)):
+        for f in frames: f[1].zero_()
+        torch.cuda.synchronize()
+        threads = [threading.Thread(target=lambda f=f, s=s: [f[0](s.cuda_stream) for _ in range(20)]) for f, s in zip(frames, streams)]
+        for t in threads: t.start()
+        for t in threads: t.join()
+        torch.cuda.synchronize()
+        for f in frames: assert torch.equal(f[1], f[2])
 
 
 def test_blend_long_lists_shared_between_waves(oracle):
