@@ -1608,12 +1608,13 @@ __device__ __forceinline__ void sort_segment_waves(const Lists& lists, uint32_t 
         if (sort_segment_waves_once<kWaves, kCap, kLeast, kWords, true>(lists, v, lo, hi, at_stage, s_w, s_between)) break;
 }
 
-// Segment sort by the waves of a workgroup for one size class: segments with min_len < length <= kCap.  Seven waves per SIMD cost a few spilled
-// registers: 110M pairs 328 -> 308 us against five of 82 registers, eight 357.
+// Segment sort by the waves of a workgroup for one size class: segments with min_len < length <= kCap.  Seven waves per SIMD: 110M pairs
+// 328 -> 308 us against five of 82 registers, eight, with spilled registers, 357.  Of pairs eight: on frames of more than 2^20 tile ids most of the workgroups
+// search for bounds that enclose nothing and end (16400x16400 pixels, 50 000 pairs: the sort 13.0 ms with seven, 12.3 with eight, 14.0 with five).
 // With a table of segment starts, the first launch has listed the segments of the class.  Without a table
 // (more tile ids than it holds) the grid has one workgroup per tile id and each searches for its bounds.
 template <int kWaves, int kCap, int kLeast, bool kWords>
-__global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(7))) void segment_sort_kernel(
+__global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(kWords ? 7 : 8))) void segment_sort_kernel(
     Lists lists, int n, uint32_t tile_mask, int min_len, const int* __restrict__ seg_start,
     const uint32_t* __restrict__ list, const uint32_t* __restrict__ list_count, uint32_t list_cap)
 {
