@@ -108,8 +108,9 @@ struct Workspace {
 };
 
 // Words of the workspace that the launches of one sort hand to each other.
-constexpr int kMarkBeyond = 0;                  // one word per count workgroup of the first pass: some key has bits above the sorted range
+constexpr int kMarkBeyond = 0;                  // one word per count workgroup of the first pass: some key differs from the first one above the sorted range
 constexpr int kMarkByIndex = kMaxChunks;        // the same for the whole list: the launches behind the first scatter read this one
+constexpr int kMarkAbove = kMarkByIndex + 1;    // the bits above the sorted range, the same in every key where that word is 0
 constexpr int kMarkLowStart = kMaxChunks + 8;   // first index of every digit of the first of two passes
 constexpr int kMarks = kMarkLowStart + 512;
 
@@ -209,6 +210,14 @@ struct Digits {
     __device__ __forceinline__ uint32_t field(int i) const { return kKeys ? w[2 * i + 1] : 0u; }
 };
 
+// The tile field of the list's first key, whose bits above the sorted range are those of every key unless marked (kMarkBeyond).
+template <class In>
+__device__ __forceinline__ uint32_t first_field(const In* in)
+{
+    if constexpr (sizeof(In) == 8) return (uint32_t)(in[0] >> 32);
+    return 0;
+}
+
 template <class Shape, class In>
 __global__ __launch_bounds__(kSortBlock) void count_kernel(const In* __restrict__ in, int n,
                                                            int shift, int nbits, uint32_t* __restrict__ hist,
@@ -232,10 +241,11 @@ __global__ __launch_bounds__(kSortBlock) void count_kernel(const In* __restrict_
     Digits<Shape, In> digits;
     digits.load(in, base, tid, n);
     uint32_t seen = 0;
+    const uint32_t field_of_first = beyond ? first_field(in) : 0u;
 #pragma unroll
     for (int i = 0; i < Shape::kCountItems; i++) {
         if (base + digits.index(i, tid) < n) atomicAdd(&h[digits.digit(i, shift, mask)], 1u);
-        seen |= digits.field(i);
+        if (base + digits.index(i, tid) < n) seen |= digits.field(i) ^ field_of_first;
     }
     if (beyond && (seen & above) != 0) s_beyond = 1;
     __syncthreads();
@@ -274,6 +284,7 @@ __global__ __launch_bounds__(kCountGroups * kSortBlock) void count_chunk_kernel(
     if (threadIdx.x == 0) s_beyond = 0;
     __syncthreads();
     uint32_t seen = 0;
+    const uint32_t field_of_first = beyond ? first_field(in) : 0u;
     for (int first = t0; first < t1; first += groups) {      // the same trips for every group
         const int row = first + group;
         if (row < t1) {
@@ -283,7 +294,7 @@ __global__ __launch_bounds__(kCountGroups * kSortBlock) void count_chunk_kernel(
 #pragma unroll
             for (int i = 0; i < Shape::kCountItems; i++) {
                 if (base + digits.index(i, tid) < n) atomicAdd(&h[group][digits.digit(i, shift, mask)], 1u);
-                seen |= digits.field(i);
+                if (base + digits.index(i, tid) < n) seen |= digits.field(i) ^ field_of_first;
             }
         }
         __syncthreads();
@@ -389,8 +400,9 @@ __global__ __launch_bounds__(kOffsetThreads) void offsets_kernel(uint32_t* __res
 // place of 12 by the last pass, and the second count reads a byte or two per pair in place of its key.  With pairs carried
 // in full, and nine instructions per bit of the ranking in place of four: 8K frame of 110M pairs scatter 541 + 533 -> 519 + 425 us,
 // second count 213 -> 79; 4K / 8M 48 + 46 -> 43 + 40, 14.4 -> 8; 8K / 14.5M 82 + 83 -> 80 + 71, 27 -> 18.
-// A list with a key that has bits above the sorted range carries every pair's index in place of its value (the partition is stable, so
-// equal depths keep their order by it as well), and the segment sort fetches the pairs from the input.
+// A list whose keys differ in bits above the sorted range carries every pair's index in place of its value (the partition is stable, so
+// equal depths keep their order by it as well), and the segment sort fetches the pairs from the input.  (8M pairs of a 4K frame 145 -> 417 us;
+// bits that every key has in common there are set again by the segment sort, 145.)
 //
 // The last pass of at most two (Form::kSegments) also writes the table of segment starts,
 // seg_start[v] = first index of the output whose tile field is >= v, v in [0, ids], ids = 2^(bits of
@@ -409,7 +421,7 @@ __global__ __launch_bounds__(Shape::kThreads) void scatter_kernel(
     int n, int shift, int nbits, int low_bits,   // kSegments: low_bits tile bits below this pass's digit
     const uint32_t* __restrict__ start,          // [blocks][bins] from offsets_kernel, or ...
     int raw_rows,                                // ... if > 0, the raw_rows histogram rows themselves (a short list)
-    uint32_t above,                              // kAlone: the bits of the tile field above the sorted range
+    uint32_t above,                              // the bits of the tile field above the sorted range
     uint32_t* marks, const uint32_t* beyond, int beyond_rows,       // beyond_rows > 0: the first pass
     int* __restrict__ seg_start)                 // kSegments: [2^(low_bits + nbits) + 1]
 {
@@ -474,16 +486,17 @@ __global__ __launch_bounds__(Shape::kThreads) void scatter_kernel(
         bool by_index = false;
         if constexpr (kAlone) {
             uint32_t seen = 0;
+            const uint32_t field_of_first = first_field(keys_in);
 #pragma unroll
             for (int i = 0; i < kItems; i++)
-                if (wave * (kWave * kItems) + i * kWave + lane < in_tile) seen |= (uint32_t)(word[i] >> 32) & above;
+                if (wave * (kWave * kItems) + i * kWave + lane < in_tile) seen |= ((uint32_t)(word[i] >> 32) ^ field_of_first) & above;
             by_index = __syncthreads_or(seen != 0) != 0;
-            if (tid == 0) marks[kMarkByIndex] = by_index ? 1u : 0u;
+            if (tid == 0) { marks[kMarkByIndex] = by_index ? 1u : 0u; marks[kMarkAbove] = field_of_first & above; }
         } else if (beyond_rows > 0) {
             uint32_t seen = 0;
             for (int r = lane; r < beyond_rows; r += kWave) seen |= beyond[r];
             by_index = ballot(seen != 0) != 0;
-            if (blockIdx.x == 0 && tid == 0) marks[kMarkByIndex] = by_index ? 1u : 0u;
+            if (blockIdx.x == 0 && tid == 0) { marks[kMarkByIndex] = by_index ? 1u : 0u; marks[kMarkAbove] = first_field(keys_in) & above; }
         }
 #pragma unroll
         for (int i = 0; i < kItems; i++) {
@@ -1016,10 +1029,13 @@ struct Lists {
     uint32_t* values;
     const uint64_t* keys_in;            // the caller's unsorted list
     const uint32_t* values_in;
-    const uint32_t* by_index;           // one word: not zero where the values are indices into that list
+    const uint32_t* by_index;           // not zero where the values are indices into that list; behind it, what is above every key's sorted range where not
 };
 
-// Stores a pair of tile id v.
+// The tile field of tile id v's pairs, where they are not indices.
+__device__ __forceinline__ uint32_t field_of(const Lists& l, uint32_t v) { return v | l.by_index[1]; }
+
+// Stores a pair of tile field v.
 __device__ __forceinline__ void store_pair(const Lists& l, bool by_index, int i, uint32_t v, uint64_t word)
 {
     uint64_t key = ((uint64_t)v << 32) | (word >> 32);
@@ -1070,9 +1086,9 @@ struct Segment {
             __builtin_amdgcn_raw_buffer_store_b32((uint32_t)word, values, i * 4, 0, 0);
         }
     }
-    __device__ __forceinline__ void store(int i, uint32_t v, uint64_t word) const
+    __device__ __forceinline__ void store(int i, uint32_t field, uint64_t word) const
     {
-        const Pair2 key = { (uint32_t)(word >> 32), v };
+        const Pair2 key = { (uint32_t)(word >> 32), field };
         __builtin_amdgcn_raw_buffer_store_b64(key, keys, i * 8, 0, 0);
         __builtin_amdgcn_raw_buffer_store_b32((uint32_t)word, values, i * 4, 0, 0);
     }
@@ -1281,7 +1297,6 @@ __device__ __forceinline__ bool sort_segment_wave_of(const Lists& lists, uint32_
     asm volatile("" : "+v"(lane));
     const int len = hi - lo;
     const Segment segment(lists, lo, len);
-    const bool by_index = *lists.by_index != 0;
     constexpr int kRounds = kUse >= 2 ? 2 : 1, kHalf = kCap / kRounds;
     WordBits bits;
     bits.stage = kAgain ? 1 : 0;
@@ -1346,6 +1361,11 @@ __device__ __forceinline__ bool sort_segment_wave_of(const Lists& lists, uint32_
         }
     }
     asm volatile("" : "+v"(lane));
+    // (looked at here: through the network they would take scalar registers that it needs)
+    const uint32_t* mark = lists.by_index;
+    asm volatile("" : "+s"(mark));
+    const bool by_index = mark[0] != 0;
+    const uint32_t field = v | mark[1];
     // back to contiguous stores through LDS, the lower half of the ranks (lanes 0..31) first, then
     // the upper half through the same words: half the LDS, twice the waves per CU
 #pragma unroll
@@ -1363,11 +1383,11 @@ __device__ __forceinline__ bool sort_segment_wave_of(const Lists& lists, uint32_
         } else if (!by_index) {
 #pragma unroll
             for (int t = h * (kUse / kRounds); t < (h + 1) * (kUse / kRounds); t++)
-                segment.store(t * kWave + lane, v, s_w[staged(t * kWave + lane - h * kHalf)]);
+                segment.store(t * kWave + lane, field, s_w[staged(t * kWave + lane - h * kHalf)]);
         } else {
 #pragma unroll
             for (int t = h * (kUse / kRounds); t < (h + 1) * (kUse / kRounds); t++)
-                if (t * kWave + lane < len) store_pair(lists, true, lo + t * kWave + lane, v, s_w[staged(t * kWave + lane - h * kHalf)]);
+                if (t * kWave + lane < len) store_pair(lists, true, lo + t * kWave + lane, field, s_w[staged(t * kWave + lane - h * kHalf)]);
         }
     }
     __builtin_amdgcn_wave_barrier();
@@ -1444,7 +1464,6 @@ __device__ __forceinline__ bool sort_segment_waves_of(const Lists& lists, uint32
     const int first = wave * kPart;                     // this wave's part of the segment
     const bool present = first < len;
     const Segment segment(lists, lo, len);
-    const bool by_index = *lists.by_index != 0;
     uint64_t* const s_mine = s_w + wave * staging_words(kPart);
     WordBits bits;
     bits.stage = kAgain ? at_stage : 0;
@@ -1558,6 +1577,11 @@ __device__ __forceinline__ bool sort_segment_waves_of(const Lists& lists, uint32
     }
     __syncthreads();
     asm volatile("" : "+v"(lane));
+    // (looked at here: through the network they would take scalar registers that it needs)
+    const uint32_t* mark = lists.by_index;
+    asm volatile("" : "+s"(mark));
+    const bool by_index = mark[0] != 0;
+    const uint32_t field = v | mark[1];
     // back to contiguous stores through this wave's part of the LDS, half of the ranks at a time
 #pragma unroll
     for (int h = 0; h < 2; h++) {
@@ -1574,12 +1598,12 @@ __device__ __forceinline__ bool sort_segment_waves_of(const Lists& lists, uint32
         } else if (!by_index) {
 #pragma unroll
             for (int t = h * (kUse / 2); t < (h + 1) * (kUse / 2); t++)
-                segment.store(first + t * kWave + lane, v, s_mine[staged(t * kWave + lane - h * (kPart / 2))]);
+                segment.store(first + t * kWave + lane, field, s_mine[staged(t * kWave + lane - h * (kPart / 2))]);
         } else {
 #pragma unroll
             for (int t = h * (kUse / 2); t < (h + 1) * (kUse / 2); t++) {
                 const int i = first + t * kWave + lane;
-                if (i < len) store_pair(lists, true, lo + i, v, s_mine[staged(t * kWave + lane - h * (kPart / 2))]);
+                if (i < len) store_pair(lists, true, lo + i, field, s_mine[staged(t * kWave + lane - h * (kPart / 2))]);
             }
         }
     }
@@ -1794,7 +1818,7 @@ __global__ __launch_bounds__(kGeneralWaves * kWave) void segment_sort_general_ke
         }
         __syncthreads();
         const int lo = s_bounds[0], hi = s_bounds[1];
-        if (hi - lo > min_len) sort_segment_general<kWords>(lists, alt_keys, alt_values, v, lo, hi, s_cnt, s_wave_sum, &s_flag);
+        if (hi - lo > min_len) sort_segment_general<kWords>(lists, alt_keys, alt_values, field_of(lists, v), lo, hi, s_cnt, s_wave_sum, &s_flag);
     } else {
         const uint32_t shard = blockIdx.x % kListShards;
         // list_count: the counters of all classes, class c at c * kListShards (1: medium, 2: large, 3: long)
@@ -1808,7 +1832,7 @@ __global__ __launch_bounds__(kGeneralWaves * kWave) void segment_sort_general_ke
                 if (hi - lo <= kCapHuge)
                     sort_segment_waves<kGeneralWaves, kCapHuge, 2, kWords>(lists, v, lo, hi, s_w, s_between);
                 else
-                    sort_segment_general<kWords>(lists, alt_keys, alt_values, v, lo, hi, s_cnt, s_wave_sum, &s_flag);
+                    sort_segment_general<kWords>(lists, alt_keys, alt_values, field_of(lists, v), lo, hi, s_cnt, s_wave_sum, &s_flag);
             }
         }
     }

@@ -1684,6 +1684,37 @@ def test_sort_one_key_with_bits_above_the_range(W, H, n):
         _sort_case(tile, depth, W, H, junk=junk, seed=n, ascending=n > 3 and at == 0)
 
 
+@pytest.mark.parametrize("W,H,n", [(64, 64, 2), (64, 64, 3000), (640, 480, 5000), (1920, 1080, 700_000), (3840, 2160, 2_200_000), (7680, 4320, 900),
+                                   (7680, 4320, 500_000), (8208, 8208, 50_000), (16400, 16400, 20_000)])
+def test_sort_keys_that_share_bits_above_the_range(W, H, n):
+    """The same bits above the sorted range in every key, and all but the first, the last, or one in the middle: the forms of a list that
+    test_sort_one_key_with_bits_above_the_range goes through."""
+    rng = np.random.default_rng(n)
+    tiles = ((W + 15) // 16) * ((H + 15) // 16)
+    tile = rng.integers(0, tiles, n).astype(np.uint32)
+    tile[:n // 3] = tiles - 1
+    depth = rng.uniform(0.2, 90.0, n).astype(np.float32).view(np.uint32)
+    depth[::5] = depth[0]
+    for other in (None, 0, n // 2, n - 1):
+        junk = np.full(n, 0x25, np.uint32)
+        if other is not None:
+            junk[other] = 0x21
+        _sort_case(tile, depth, W, H, junk=junk, seed=n, ascending=n > 3 and other == 0)
+
+
+def test_sort_of_keys_that_share_bits_above_the_range_in_time():
+    """8M pairs of a 4K frame: the same bits above the sorted range in every key cost nothing."""
+    import torch
+    g = torch.Generator(device="cuda")
+    g.manual_seed(5)
+    n = 8_000_000
+    rand = lambda: torch.rand(n, generator=g, device="cuda")
+    keys = ((rand() * 32400).long().clamp_(max=32399) << 32) | (0.5 + 89.5 * rand()).view(torch.int32).long()
+    values = torch.arange(n, device="cuda", dtype=torch.int32)
+    times = [_sort_time(n, 3840, 2160, k, values) for k in (keys, keys | (5 << 56))]
+    assert times[1] < 1.2 * times[0]
+
+
 @pytest.mark.parametrize("W,H,n", [(16, 16, 5000), (256, 16, 9000), (160, 128, 70_000), (3840, 2160, 300),
                                    (7680, 4320, 40), (8208, 8208, 200_000), (8208, 8208, 90)])
 def test_sort_segment_table_shapes(W, H, n):
