@@ -334,7 +334,8 @@ def stage_report(fr, stage_ms, K, counts, walked):
     else:
         stages["preprocess"] = dict(ms=round(stage_ms["preprocess"], 4), bound="hbm")
     hbm("sort", K * (8 + 24 * passes))
-    # counts, scatters and the segment sort; with one or two passes pairs travel as words beside `digit` bytes of the tile id
+    # counts, scatters and the segment sort; with one or two passes pairs travel as words beside `digit` bytes of the tile id.
+    # A lower bound: segments of more than 1024 pairs are read a second time
     bits = int(tiles).bit_length()
     digit = 1 if bits <= 16 else 2
     per_pair = 48 if bits <= 8 else 64 + 3 * digit if bits <= 18 else 32 * ((bits + 7) // 8) + 8 + 24

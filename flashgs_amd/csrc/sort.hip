@@ -20,7 +20,7 @@
 //     passes `segment_starts_kernel` does, from the sorted keys), then segments are handled by
 //     size class.  Up to 1024 pairs one wave holds a 32-bit word per pair, the upper bits of its depth in front of its place,
 //     in registers and runs a merging network on them, then fetches the pairs in that order and puts the few that the
-//     bits left out tell apart in order (the result is that of a stable sort by depth); lane exchanges inside a row of 16 lanes are
+//     bits left out tell apart in order, or sorts again by those (the result is that of a stable sort by depth); lane exchanges inside a row of 16 lanes are
 //     data-parallel-primitive moves.  Up to 4096 (4 waves), 8192 (8) and 16384 pairs (16) every wave
 //     of a workgroup sorts its part like that and the parts are merged, the steps between two waves
 //     through LDS.  Longer segments go
@@ -28,7 +28,8 @@
 //     pairs share the digit.
 //
 // Bytes moved per pair with two partition passes of 8-bit digits: 8 (count) + 12 + 9 (scatter) + 1 + 9 + 8, and 8 + 12 for the
-// segment sort: 67 (70 with 9-bit digits), against 8 + 6 * 24 = 152 for a six-pass LSD sort of 47 bits.
+// segment sort of up to 1024 pairs: 67 (70 with 9-bit digits), against 8 + 6 * 24 = 152 for a six-pass LSD sort of 47 bits.  Segments of 1025 to
+// 16384 pairs are read a second time, behind the merges; what sorts again is written and read twice more, and the longest segments are read twice and written once per counting pass.
 #include "fgs_internal.h"
 
 #include <algorithm>

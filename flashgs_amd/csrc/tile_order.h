@@ -8,33 +8,38 @@ namespace fgs {
 
 // Position in the launch of a frame that is not ranked -> tile.  The hardware deals consecutive workgroups out to the 8 XCDs in
 // turn, and every XCD has its own L2.  Neighbouring tiles share most of their Gaussians, so each
-// XCD is given whole 8x8 blocks of tiles (its positions g = 8*slot + xcd walk blocks xcd, xcd+8,
+// XCD is given whole blocks of tiles (of 8x8: its positions g = 8*slot + xcd walk blocks xcd, xcd+8,
 // ... 64 tiles at a time): a Gaussian's attribute lines are then fetched into one L2 once instead
 // of into several L2s once per tile.  Every row of blocks begins further right, so that a block's XCD is five behind that of the one above
 // it or, in rows of other than a multiple of 8 blocks, where the rotation wraps, 5 + blocks_x: row after row from the left, an XCD would
 // have the same columns of blocks in every second row of a frame of 60 blocks, in every row of one of 24, and 2 to 14 % more to blend
-// than the average, and the launch ends when the last XCD does.  Behind the sort, in us (row after row, five apart): 3000x2200 / 2M 207, 199;
-// 5120x2880 / 5M 383, 370; 4K / 3M 265, 260; 8K / 8M 650, 652; orbit at 4K 89.3, 89.3; 2720x1700 / 3M 261, 260; 110M pairs 596, 598.  With
-// blocks of 4x4, five apart: 192, 373, 261, 644, 91.8, 264, 600, and 8 to 21 % more bytes read.  Over 28 frames of 14 000 to 105 000 tiles the
-// orders are within 1 % of each other on average (8x8 0.997 of row after row, 4x4 0.992), single ones within 7 %.
+// than the average, and the launch ends when the last XCD does.  Blocks are of 4x4 tiles where of 8x8 an XCD would have some 55 or fewer,
+// which no order deals evenly, and of 8x8 above, where smaller ones cost more in bytes (8 to 21 %) than they even out.  Behind the
+// sort, in us (8x8 row after row; 8x8 and 4x4 five apart): 3000x2200 / 2M (25 944 tiles) 207; 199, 192; 3047x1725 / 1.1M clusters 180; 172, 164;
+// 2720x1700 / 3M 261; 260, 264; orbit at 4K (32 400) 89.3; 89.3, 91.8; 4K / 3M 265; 260, 261; 5120x2880 / 5M 383; 370, 373; orbit at 4961x3641 178;
+// 180, 183; 8K / 8M 650; 652, 644; 110M pairs 596; 598, 600.  Over 28 frames of 14 000 to 105 000 tiles the three are within 1 % of
+// each other on average, single ones within 7 %.
 // False for the padding positions.
-constexpr int kBlockLog2 = 3, kBlock = 1 << kBlockLog2;
+constexpr int kFineTiles = 28 << 10;
+constexpr int block_log2_of(int tiles_x, int tiles_y) { return (long long)tiles_x * tiles_y < kFineTiles ? 2 : 3; }
 
 constexpr long long positions_of(int tiles_x, int tiles_y)
 {
-    const long long blocks = (long long)((tiles_x + kBlock - 1) / kBlock) * ((tiles_y + kBlock - 1) / kBlock);
-    return (blocks + 7) / 8 * 8 * (kBlock * kBlock);
+    const int block_log2 = block_log2_of(tiles_x, tiles_y), size = 1 << block_log2;
+    const long long blocks = (long long)((tiles_x + size - 1) / size) * ((tiles_y + size - 1) / size);
+    return (blocks + 7) / 8 * 8 * (size * size);
 }
 
 constexpr bool tile_of_position(int group, int tiles_x, int tiles_y, int* tile_x, int* tile_y)
 {
+    const int block_log2 = block_log2_of(tiles_x, tiles_y), size = 1 << block_log2;
     const int xcd = group & 7, slot = group >> 3;
-    const int blocks_x = (tiles_x + kBlock - 1) >> kBlockLog2;
-    const int block = (slot >> (2 * kBlockLog2)) * 8 + xcd, inner = slot & (kBlock * kBlock - 1);
+    const int blocks_x = (tiles_x + size - 1) >> block_log2;
+    const int block = (slot >> (2 * block_log2)) * 8 + xcd, inner = slot & (size * size - 1);
     const int row = block / blocks_x;
     const int column = (block - row * blocks_x + ((blocks_x - 5) & 7) * row) % blocks_x;
-    *tile_x = column * kBlock + (inner & (kBlock - 1));
-    *tile_y = row * kBlock + (inner >> kBlockLog2);
+    *tile_x = (column << block_log2) + (inner & (size - 1));
+    *tile_y = (row << block_log2) + (inner >> block_log2);
     return *tile_x < tiles_x && *tile_y < tiles_y;
 }
 

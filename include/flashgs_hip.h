@@ -168,15 +168,16 @@ size_t fgs_get_sort_buffer_size(int num_rendered);
  * those with a curvature along y beyond -3 (splats that were not widened by 0.3), saddles and non-finite ones take
  * slower paths.
  * A frame of at most 8192 tiles first ranks its tiles by list length into a table the library keeps per
- * (device, stream) (32 KB, allocated on the first such call on that stream); fgs_render_* leaves the ranking out where
- * the frame is so small that all its workgroups are resident at once.  Lists that are long for the frame are blended in
+ * (device, stream) (37 KB, allocated on the first call on that stream that uses it); fgs_render_* leaves the ranking out where
+ * the frame is so small that all its workgroups are resident at once, and lists the long lists of a frame of 65536 tiles and 3 * 2^20 pairs or more
+ * in the same memory, so that they are blended first.  Lists that are long for the frame are blended in
  * runs by several waves and folded front to back.  The run that holds the stop of render.cu:394-408 is walked again
  * pair by pair behind what precedes it, and so is one with weights above 1 in it or behind a transmittance that
  * such weights took out of 0 to 1, so the walk ends where the reference's does.  From which length on a list is cut
  * into runs follows from the lists of the whole frame and from the device's number of compute units: the colours of one tile's
  * list can differ by the rounding of that sum between two frames, or two devices, that hold it.  Calls on
  * different streams may overlap in time, and several host threads may call on one stream.  Under
- * stream capture, and where the table cannot be allocated, tiles go unranked: the image is the
+ * stream capture, and where the table cannot be allocated, tiles go unranked and long lists unlisted: the image is the
  * same bits, and a captured blend holds no memory of the library's, so its replays may overlap anything
  * that leaves the caller's own buffers alone.
  */

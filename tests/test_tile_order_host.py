@@ -14,7 +14,7 @@ extern "C" void least_of(const uint64_t* each, int n, int* out) { for (int i = 0
 extern "C" void bin_of(const int* length, int n, int* out) { for (int i = 0; i < n; i++) out[i] = fgs::order_bin(length[i]); }
 extern "C" int first_bin(int least) { return fgs::first_bin_below(least); }
 extern "C" long long positions(int tiles_x, int tiles_y) { return fgs::positions_of(tiles_x, tiles_y); }
-extern "C" int block_size(void) { return fgs::kBlock; }
+extern "C" int block_size(int tiles_x, int tiles_y) { return 1 << fgs::block_log2_of(tiles_x, tiles_y); }
 extern "C" void tiles_of(int tiles_x, int tiles_y, int n, int* out)
 {
     for (int g = 0; g < n; g++) {
@@ -60,12 +60,12 @@ def test_the_ranking_counts_every_list_that_is_shared_out(lib):
 
 
 @pytest.mark.parametrize("tiles_x, tiles_y", [(1, 1), (1, 9000), (9000, 1), (7, 1200), (8, 1025), (85, 107), (91, 91), (170, 107), (188, 138), (240, 135),
-                                              (320, 180), (300, 225), (341, 513), (415, 254), (480, 270), (513, 513), (856, 12)])
+                                              (320, 180), (300, 225), (224, 127), (224, 128), (224, 129), (341, 513), (415, 254), (480, 270), (513, 513), (856, 12)])
 def test_every_tile_of_a_large_frame_has_one_position(lib, tiles_x, tiles_y):
     """Every tile once, a block of tiles on one XCD, and blocks below each other on XCDs five apart, or five and
     the blocks of a row where the rotation of the row wraps (never, where these are a multiple of 8)."""
     lib.positions.restype = C.c_longlong
-    n, size = lib.positions(tiles_x, tiles_y), lib.block_size()
+    n, size = lib.positions(tiles_x, tiles_y), lib.block_size(tiles_x, tiles_y)
     tiles = np.empty(n, np.int32)
     lib.tiles_of(tiles_x, tiles_y, n, tiles.ctypes.data_as(C.c_void_p))
     found = tiles[tiles >= 0]
