@@ -13,7 +13,8 @@
 //     `offsets_kernel` turns them into the exclusive start of every (block, digit) run, and
 //     `scatter_kernel` ranks its block in LDS (wave64 ballot matching, so equal digits keep
 //     their input order) and writes each run to its start.  A short list takes
-//     count -> scatter.  No workgroup ever waits for another one.  With one or two passes the pairs leave the
+//     count -> scatter.  Up to 8191 tiles and some millions of pairs the tile id is one digit instead (see tile_scatter_kernel).
+//     No workgroup ever waits for another one.  With one or two passes the pairs leave the
 //     partition as 64-bit words depth << 32 | value, the tile known from the place.
 //  2. Sort every tile's segment by the 32 depth bits without touching memory in between: the
 //     last scatter pass also tabulates where each tile id's segment begins (with more than two
@@ -737,6 +738,281 @@ __global__ __launch_bounds__(Shape::kThreads) void scatter_kernel(
             }
         }
         if (tile == 0 && tid == 0) seg_start[(size_t)1 << (low_bits + nbits)] = n;
+    }
+}
+
+// ---- the partition in one pass ---------------------------------------------------------------------
+//
+// In frames of up to 2^kOnePassBits tile ids, and lists that are not too long for them, the whole tile id is one digit: `tile_count_kernel` writes
+// a row of counts per block, 16 bits for every tile id, `tile_offsets_kernel` turns every column of the rows into what the blocks in front
+// hold of that tile, and `tile_scatter_kernel` sorts its block by tile id in LDS (two stable passes, seven bits first) and writes every pair's
+// word to its place.  The pairs travel once and there are three launches, where two passes of 8 bits take four to six, each of which lasts 3 to 14 us on
+// such a list whatever it moves: 3 + 4 + 8 us for 22 in all on 0.2M pairs of a 720p frame, 5 + 8 + 21 for 52 on 1.7M of a 1080p frame (that one reads 35 MB, of which
+// 14 are offsets, and writes 14 in runs of one or two pairs).  The whole sort, two passes -> one: 3600 tiles 0.1M pairs 27 -> 22 us, 0.4M 41 -> 35,
+// 1.6M 97 -> 77, 6.4M 275 -> 255; 8160 tiles 0.1M 28 -> 25, 0.8M 59 -> 48, 1.6M 78 -> 62, 3.2M 121 -> 113; 300 tiles 25k 27 -> 22, 0.8M 117 -> 96.
+// A block's rows cost 6 bytes per tile id, so it stops paying where blocks x ids do: 8160 tiles 6.4M pairs 170 -> 180 us, 14 400 tiles 0.2M 32 -> 34, 0.8M
+// 53 -> 48, 3.2M 100 -> 133.
+// (Instead of the two passes in LDS, pairs that put their places down by tile and count the smaller ones there, words written from
+// registers in any order: the scatter 21 -> 28 us, 12 -> 18 where some tiles are crowded.  Counters in memory in place of the rows, by atomic additions
+// of a block's counts and of bases taken from them: 0.4M and 1.7M pairs 17 and 45 us in all for 20 and 34, and an order to be mended behind it.)
+// Rows and offsets stand in the space of the copy that longer segments go through later, or behind what the sort needs if there is more.
+constexpr int kOnePassBits = 13, kOnePassIds = 1 << kOnePassBits, kOnePassLeastBits = 9;
+constexpr int kOnePassThreads = 1024, kOnePassWaves = kOnePassThreads / kWave;
+constexpr int kOnePassLow = 7;                  // bits of the tile id that the first sort of a block takes
+// Blocks of 2048 pairs up to this many pairs, of 4096 above: 3600 tiles 0.2M pairs 25 and 28 us, 0.8M 50 and 48; 8160 tiles 0.2M 26 and 28, 0.4M 32 and 31, 1.6M 73 and 62.
+// (Of 8192: 0.2M 33, 1.7M 1 % more.)
+constexpr int kOnePassShort = 1 << 19;
+constexpr size_t kOnePassCells = (size_t)1 << 23;       // the most cells of rows: 4.2M pairs with 8192 ids, 8.4M with 4096
+
+// rows[block][tile]: 16-bit counts, two in a word.
+template <int kItems>
+__global__ __launch_bounds__(kOnePassThreads) void tile_count_kernel(const uint64_t* __restrict__ keys, int n, uint32_t ids,
+                                                                     uint32_t* __restrict__ rows, uint32_t* __restrict__ beyond,
+                                                                     uint32_t* __restrict__ seg_counts)
+{
+    static_assert(kOnePassThreads * kItems <= 65535, "16-bit counts");
+    __shared__ uint32_t s_counts[kOnePassIds / 2];
+    __shared__ uint32_t s_beyond;
+    const int tid = threadIdx.x;
+    if (blockIdx.x == 0 && tid < kListClasses * kListShards) seg_counts[tid] = 0;       // what the segment launches append to
+    uint32_t field[kItems];
+    const int base = (int)blockIdx.x * (kOnePassThreads * kItems) + tid;
+#pragma unroll
+    for (int i = 0; i < kItems; i++) {
+        field[i] = 0;
+        if (base + i * kOnePassThreads < n) field[i] = ((const uint32_t*)keys)[2 * (size_t)(base + i * kOnePassThreads) + 1];
+    }
+    const uint32_t field_of_first = first_field(keys);
+    for (uint32_t t = tid; t < ids / 2; t += kOnePassThreads) s_counts[t] = 0;
+    if (tid == 0) s_beyond = 0;
+    __syncthreads();
+    uint32_t seen = 0;
+#pragma unroll
+    for (int i = 0; i < kItems; i++) {
+        if (base + i * kOnePassThreads < n) {
+            const uint32_t tile = field[i] & (ids - 1u);
+            atomicAdd(&s_counts[tile >> 1], tile & 1u ? 0x10000u : 1u);
+            seen |= field[i] ^ field_of_first;
+        }
+    }
+    if ((seen & ~(ids - 1u)) != 0) s_beyond = 1;
+    __syncthreads();
+    for (uint32_t t = tid; t < ids / 2; t += kOnePassThreads) rows[(size_t)blockIdx.x * (ids / 2) + t] = s_counts[t];
+    if (tid == 0) beyond[blockIdx.x] = s_beyond;
+}
+
+// offsets[block][tile] = pairs of the tile in the blocks in front; totals[tile].  A workgroup takes kColumnTiles tiles, in as many parts of the rows
+// as it has threads for.
+constexpr int kColumnTiles = 32, kColumnParts = kOnePassThreads / kColumnTiles;
+__global__ __launch_bounds__(kOnePassThreads) void tile_offsets_kernel(const uint16_t* __restrict__ rows, int blocks, uint32_t ids,
+                                                                       uint32_t* __restrict__ offsets, uint32_t* __restrict__ totals,
+                                                                       const uint64_t* __restrict__ keys, const uint32_t* __restrict__ beyond,
+                                                                       uint32_t* __restrict__ marks)
+{
+    constexpr int kAtOnce = 16;
+    __shared__ uint32_t s_sum[kColumnParts][kColumnTiles];
+    const int column = threadIdx.x % kColumnTiles, part = threadIdx.x / kColumnTiles;
+    const uint32_t tile = blockIdx.x * kColumnTiles + column;
+    const int per = (blocks + kColumnParts - 1) / kColumnParts;
+    const int r0 = min(blocks, part * per), r1 = min(blocks, r0 + per);
+    if (blockIdx.x == 0) {          // one word out of the count workgroups' words
+        uint32_t seen = 0;
+        for (int b = (int)threadIdx.x; b < blocks; b += kOnePassThreads) seen |= beyond[b];
+        const int any = __syncthreads_or(seen != 0);
+        if (threadIdx.x == 0) { marks[kMarkByIndex] = any ? 1u : 0u; marks[kMarkAbove] = first_field(keys) & ~(ids - 1u); }
+    }
+    uint32_t c[kAtOnce], sum = 0;
+    auto load = [&](int r) {
+#pragma unroll
+        for (int j = 0; j < kAtOnce; j++) c[j] = r + j < r1 ? rows[(size_t)(r + j) * ids + tile] : 0u;
+    };
+    for (int r = r0; r < r1; r += kAtOnce) {
+        load(r);
+#pragma unroll
+        for (int j = 0; j < kAtOnce; j++) sum += c[j];
+    }
+    s_sum[part][column] = sum;
+    __syncthreads();
+    uint32_t run = 0, total = 0;
+#pragma unroll
+    for (int p = 0; p < kColumnParts; p++) {
+        const uint32_t s = s_sum[p][column];
+        run += p < part ? s : 0u;
+        total += s;
+    }
+    if (part == 0) totals[tile] = total;
+    for (int r = r0; r < r1; r += kAtOnce) {
+        if (per > kAtOnce) load(r);
+#pragma unroll
+        for (int j = 0; j < kAtOnce; j++) {
+            if (r + j < r1) offsets[(size_t)(r + j) * ids + tile] = run;
+            run += c[j];
+        }
+    }
+}
+
+// Where the pairs of a block stand when it is stably sorted by kBits bits of their fields from `shift` up.  Slot i of lane l of wave w is place
+// w * 64 * kItems + i * 64 + l; places from in_tile on are none.
+template <int kItems, int kBits>
+__device__ __forceinline__ void rank_block(const uint32_t (&field)[kItems], int shift, int in_tile, uint32_t (&place)[kItems],
+                                           uint16_t (*s_count)[1 << kBits], uint16_t* s_start, uint32_t* s_wave_sum)
+{
+    constexpr int kB = 1 << kBits;
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
+    for (int w = tid; w < kOnePassWaves * kB / 2; w += kOnePassThreads) ((uint32_t*)&s_count[0][0])[w] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kItems; i++) {          // (the ranking of scatter_kernel)
+        const bool valid = wave * (kWave * kItems) + i * kWave + lane < in_tile;
+        const uint32_t d = __builtin_amdgcn_ubfe(field[i], shift, kBits);
+        const uint64_t all = ballot(valid);
+        uint32_t peers_lo = (uint32_t)all, peers_hi = (uint32_t)(all >> 32);
+#pragma unroll
+        for (int b = 0; b < kBits; b++) {
+            uint32_t bit = (uint32_t)__builtin_amdgcn_sbfe((int)d, b, 1);
+            asm("" : "+v"(bit));
+            const uint64_t with_bit = ballot(bit != 0);
+            peers_lo = __builtin_amdgcn_bitop3_b32(peers_lo, (uint32_t)with_bit, bit, 0x90);
+            peers_hi = __builtin_amdgcn_bitop3_b32(peers_hi, (uint32_t)(with_bit >> 32), bit, 0x90);
+        }
+        const uint32_t below = __builtin_amdgcn_mbcnt_hi(peers_hi, __builtin_amdgcn_mbcnt_lo(peers_lo, 0u));
+        const uint32_t before = s_count[wave][d];
+        if (valid && below == 0)
+            s_count[wave][d] = (uint16_t)(before + (uint32_t)__popc(peers_lo) + (uint32_t)__popc(peers_hi));
+        place[i] = before + below;
+        __builtin_amdgcn_wave_barrier();
+    }
+    __syncthreads();
+    uint32_t total = 0, incl = 0;
+    if (tid < kB) {
+#pragma unroll
+        for (int w = 0; w < kOnePassWaves; w++) {
+            const uint32_t c = s_count[w][tid];
+            s_count[w][tid] = (uint16_t)total;
+            total += c;
+        }
+        incl = wave_inclusive_sum(total);
+        if (lane == kWave - 1) s_wave_sum[wave] = incl;
+    }
+    __syncthreads();
+    if (tid < kB) {
+        uint32_t start = incl - total;
+        for (int w = 0; w < wave; w++) start += s_wave_sum[w];
+        s_start[tid] = (uint16_t)start;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kItems; i++) {
+        const uint32_t d = __builtin_amdgcn_ubfe(field[i], shift, kBits);
+        place[i] += (uint32_t)s_start[d] + s_count[wave][d];
+    }
+}
+
+// words: depth << 32 | value, every tile's pairs together and in input order; seg_start as in scatter_kernel.
+template <int kItems>
+__global__ __launch_bounds__(kOnePassThreads) void tile_scatter_kernel(const uint64_t* __restrict__ keys, const uint32_t* __restrict__ values,
+                                                                       uint64_t* __restrict__ words, int n, uint32_t ids,
+                                                                       const uint32_t* __restrict__ offsets, const uint32_t* __restrict__ totals,
+                                                                       const uint32_t* __restrict__ marks, int* __restrict__ seg_start)
+{
+    constexpr int kTile = kOnePassThreads * kItems, kPer = kOnePassIds / kOnePassThreads, kHigh = kOnePassBits - kOnePassLow;
+    typedef uint32_t Four __attribute__((ext_vector_type(4)));
+    static_assert(kPer % 4 == 0, "whole vectors");
+    __shared__ uint64_t s_words[kTile];
+    __shared__ uint16_t s_field[kTile];
+    __shared__ __align__(16) uint32_t s_to[kOnePassIds];        // place of the pair at place p of the sorted block, of tile t: s_to[t] + p
+    __shared__ __align__(4) uint16_t s_count[kOnePassWaves][1 << kOnePassLow];
+    __shared__ uint16_t s_start[1 << kOnePassLow];
+    __shared__ uint32_t s_wave_sum[kOnePassWaves];
+    static_assert(kHigh <= kOnePassLow, "the counts of either pass");
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
+    // (neighbouring blocks on one XCD, as in scatter_kernel)
+    const int xcd = (int)blockIdx.x % kXcds, each = (int)gridDim.x / kXcds, rest = (int)gridDim.x % kXcds;
+    const int block = xcd * each + min(xcd, rest) + (int)blockIdx.x / kXcds;
+    const int base = block * kTile, in_tile = min(kTile, n - base);
+    const int first = wave * (kWave * kItems) + lane;
+    uint64_t word[kItems];
+    uint32_t field[kItems], place[kItems];
+    {
+        uint32_t value[kItems];
+#pragma unroll
+        for (int i = 0; i < kItems; i++) word[i] = first + i * kWave < in_tile ? keys[base + first + i * kWave] : ~0ull;
+#pragma unroll
+        for (int i = 0; i < kItems; i++) value[i] = first + i * kWave < in_tile ? values[base + first + i * kWave] : 0u;
+        // where every tile's pairs begin, and this block's among them
+        Four total[kPer / 4], before[kPer / 4];
+        const uint32_t t0 = (uint32_t)(tid * kPer);
+        uint32_t sum = 0;
+#pragma unroll
+        for (int q = 0; q < kPer / 4; q++) {
+            total[q] = 0; before[q] = 0;
+            if (t0 < ids) {
+                total[q] = ((const Four*)(totals + t0))[q];
+                before[q] = ((const Four*)(offsets + (size_t)block * ids + t0))[q];
+            }
+        }
+        const bool by_index = marks[kMarkByIndex] != 0;
+#pragma unroll
+        for (int q = 0; q < kPer / 4; q++) sum += total[q].x + total[q].y + total[q].z + total[q].w;
+        const uint32_t incl = wave_inclusive_sum(sum);
+        if (lane == kWave - 1) s_wave_sum[wave] = incl;
+        __syncthreads();
+        uint32_t start = incl - sum;
+#pragma unroll
+        for (int w = 0; w < kOnePassWaves; w++) start += w < wave ? s_wave_sum[w] : 0u;
+        if (t0 < ids) {
+#pragma unroll
+            for (int q = 0; q < kPer / 4; q++) {
+                Four at;
+                at.x = start; at.y = at.x + total[q].x; at.z = at.y + total[q].y; at.w = at.z + total[q].z;
+                start = at.w + total[q].w;
+                if (block == 0) ((Four*)(seg_start + t0))[q] = at;
+                *(Four*)(s_to + t0 + 4 * q) = at + before[q];
+            }
+        }
+        if (block == 0 && tid == 0) seg_start[ids] = n;
+#pragma unroll
+        for (int i = 0; i < kItems; i++) {
+            field[i] = (uint32_t)(word[i] >> 32) & (ids - 1u);
+            word[i] = (word[i] << 32) | (by_index ? (uint32_t)(base + first + i * kWave) : value[i]);
+        }
+    }
+    rank_block<kItems, kOnePassLow>(field, 0, in_tile, place, s_count, s_start, s_wave_sum);
+#pragma unroll
+    for (int i = 0; i < kItems; i++) {
+        if (first + i * kWave < in_tile) {
+            s_words[place[i]] = word[i];
+            s_field[place[i]] = (uint16_t)field[i];
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kItems; i++) {
+        const int p = min(first + i * kWave, in_tile - 1);
+        word[i] = s_words[p];
+        field[i] = s_field[p];
+    }
+    rank_block<kItems, kHigh>(field, kOnePassLow, in_tile, place, (uint16_t(*)[1 << kHigh])s_count, s_start, s_wave_sum);
+#pragma unroll
+    for (int i = 0; i < kItems; i++) {
+        if (first + i * kWave < in_tile) {
+            s_words[place[i]] = word[i];
+            s_field[place[i]] = (uint16_t)field[i];
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kItems; i++) {
+        const int p = min(i * kOnePassThreads + tid, in_tile - 1);
+        word[i] = s_words[p];
+        field[i] = s_field[p];
+        if (i * kOnePassThreads + tid < in_tile && (p == 0 || s_field[p - 1] != field[i])) s_to[field[i]] -= (uint32_t)p;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kItems; i++) {
+        const int p = i * kOnePassThreads + tid;
+        if (p < in_tile) words[s_to[field[i]] + (uint32_t)p] = word[i];
     }
 }
 
@@ -1983,10 +2259,34 @@ extern "C" int fgs_sort_gaussian(int num_rendered,
     };
     // (the launches that sort longer segments from lists need counters that the counting launches clear)
     const bool few_ids = n <= kAlonePairs && ids <= (uint32_t)kAloneIds;
+    // (false where there is no room for the rows, or they are too many)
+    auto one_pass = [&](auto items) {
+        constexpr int kItems = decltype(items)::value;
+        const int blocks = (n + kOnePassThreads * kItems - 1) / (kOnePassThreads * kItems);
+        const size_t cells = (size_t)blocks * ids, bytes = cells * 6 + ((size_t)ids + blocks) * 4;
+        if (cells > kOnePassCells) return false;
+        const size_t behind = align_up(ws.total, 256);
+        char* const at = bytes <= ws.seg_start - ws.alt_keys ? (char*)alt_keys
+                       : behind < sorting_size && bytes <= sorting_size - behind ? list_sorting_space + behind : nullptr;
+        if (!at) return false;
+        uint32_t* const offsets = (uint32_t*)at;
+        uint32_t* const rows = offsets + cells;
+        uint32_t* const totals = rows + cells / 2;
+        uint32_t* const beyond = totals + ids;
+        hipLaunchKernelGGL((tile_count_kernel<kItems>), dim3(blocks), dim3(kOnePassThreads), 0, st, gaussian_keys_unsorted, n, ids, rows, beyond, seg_counts);
+        hipLaunchKernelGGL(tile_offsets_kernel, dim3(ids / kColumnTiles), dim3(kOnePassThreads), 0, st, (const uint16_t*)rows, blocks, ids, offsets, totals,
+                           gaussian_keys_unsorted, (const uint32_t*)beyond, marks);
+        hipLaunchKernelGGL((tile_scatter_kernel<kItems>), dim3(blocks), dim3(kOnePassThreads), 0, st, gaussian_keys_unsorted, gaussian_values_unsorted,
+                           gaussian_keys_sorted, n, ids, (const uint32_t*)offsets, (const uint32_t*)totals, (const uint32_t*)marks, seg_start);
+        return true;
+    };
+    const bool one_digit = tile_bits >= kOnePassLeastBits && tile_bits <= kOnePassBits;         // (up to 8 bits are one pass of that digit)
     if (n <= Short::kTile && tile_bits <= kNarrowMaxTileBits) {
         partition(Alone<Short>());
     } else if (few_ids) {
         partition(Alone<Narrow>());
+    } else if (one_digit && ((n <= kOnePassShort && one_pass(std::integral_constant<int, 2>())) || one_pass(std::integral_constant<int, 4>()))) {
+        // (done)
     } else if (tile_bits <= kNarrowMaxTileBits) {
         if (n <= kShortPairs) partition(Short());
         else if (n <= kMiddlePairs) partition(Middle());

@@ -1382,7 +1382,7 @@ def test_config3_more_than_100M_pairs(oracle, config3_scene):
     assert not gp.u64(got["keys"])[cap:].any() and not gp.u32(got["values"])[cap:].any()
 
 
-def _sort_case(tile, depth_bits, W, H, junk=None, seed=0, ascending=False):
+def _sort_case(tile, depth_bits, W, H, junk=None, seed=0, ascending=False, space_for=None):
     """`ascending`: the values are the input positions, as the pairs of a tile leave the preprocess
     (ascending Gaussian indices): the sorting networks then break ties of depth by the value itself.
     Otherwise a random permutation, where they have to carry positions."""
@@ -1399,7 +1399,7 @@ def _sort_case(tile, depth_bits, W, H, junk=None, seed=0, ascending=False):
         vals = np.arange(n, dtype=np.uint32)
         far = rng.integers(0, n, 3)                      # three tiles' segments that do not ascend among all that do
         vals[far] = vals[far][::-1] + np.uint32(1 << 30)
-    ks, vs = gp.sort(n, W, H, gp.dev(keys.view(np.int64)), gp.dev(vals.view(np.int32)))
+    ks, vs = gp.sort(n, W, H, gp.dev(keys.view(np.int64)), gp.dev(vals.view(np.int32)), space_for=space_for)
     masked = keys & np.uint64((1 << end_bit) - 1)
     order = np.argsort(masked, kind="stable")
     assert np.array_equal(gp.u64(ks)[:n], keys[order])
@@ -1634,6 +1634,33 @@ def test_sort_around_the_list_lengths_where_the_partition_blocks_change(n, W, H)
     depth = rng.integers(0, 1 << 32, n, dtype=np.uint64).astype(np.uint32)
     depth[::5] = depth[n // 2]
     _sort_case(tile, depth, W, H, seed=n % 89, ascending=n % 2 == 0)
+
+
+@pytest.mark.parametrize("W,H,n", [(256, 255, 5000), (512, 254, 2048), (512, 254, 2049), (1000, 400, 1025), (1000, 400, 4097), (1280, 720, 150_001),
+                                   (1920, 1080, 3000), (1920, 1080, 300_000), (1920, 1080, (1 << 19) - 1), (1920, 1080, (1 << 19) + 1),
+                                   (1280, 720, 1_300_003), (1920, 1080, 1 << 22), (1920, 1080, (1 << 22) + 1), (2048, 1024, 100_000)])
+@pytest.mark.parametrize("crowd", ["spread", "one tile", "last ids", "bits above"])
+@pytest.mark.parametrize("spare", [False, True])
+def test_sort_by_the_whole_tile_id(W, H, n, crowd, spare):
+    """Tile ids of 9 to 13 bits as one digit (and 8 and 14 bits, which are not): blocks of 2048 and of 4096 pairs, ragged last ones, the
+    longest lists that have rows, rows in the space of the copy and behind what the sort needs; every pair of most blocks in one tile,
+    ids up to the largest that the bits hold, beyond the frame's tiles; keys that differ in bits above them."""
+    rng = np.random.default_rng(n % 1013 + W + len(crowd))
+    tiles = ((W + 15) // 16) * ((H + 15) // 16)
+    ids = 1 << int(tiles).bit_length()
+    if crowd in ("spread", "bits above"):
+        tile = rng.integers(0, tiles, n)
+    elif crowd == "one tile":
+        tile = np.where(rng.random(n) < 0.9, tiles // 2, rng.integers(0, tiles, n))
+    else:
+        tile = ids - 1 - (ids * rng.random(n) ** 4).astype(np.int64)
+    if n > 1 << 21 and crowd == "one tile":     # (a segment of millions goes through memory for long)
+        tile = rng.integers(0, tiles, n)
+        tile[:n // 64] = tiles // 2
+    depth = rng.integers(0, 1 << 31, n, dtype=np.uint64).astype(np.uint32)
+    depth[::3] = depth[n // 2]                  # equal depths keep their order
+    junk = (rng.random(n) < 0.01).astype(np.uint32) if crowd == "bits above" else None
+    _sort_case(tile.astype(np.uint32), depth, W, H, junk, seed=n % 97, space_for=max(n, 1 << 24) if spare else None)
 
 
 def test_sort_bits_above_the_range_stay_with_their_pair():
