@@ -39,6 +39,7 @@ SIGNATURES = {
     "fgs_blend_ex": (C.c_int, [C.c_int] * 4 + [C.c_void_p] * 8 + [C.c_int, C.c_void_p]),
     "fgs_blend_kernel_name": (C.c_char_p, [C.c_int] * 5),
     "fgs_camera_matrices": (None, [C.c_void_p] * 2 + [C.c_int] * 2 + [C.c_float] * 4 + [C.c_void_p] * 2),
+    "fgs_sort_render": (C.c_int, [C.c_int] * 5 + [C.c_void_p, C.c_size_t] + [C.c_void_p] * 11 + [C.c_int, C.c_void_p]),
     "fgs_set_scan_spin_limit": (C.c_uint, [C.c_uint]),
     "fgs_reset_scan": (C.c_int, [C.c_void_p]),
     "fgs_set_colour_sums": (C.c_int, [C.c_int]),
@@ -173,6 +174,16 @@ def render_f32(block_x, block_y, num_rendered, width, height, points_xy, rgb_dep
         rc = load().fgs_render_ex(block_x, block_y, num_rendered, width, height, points_xy, rgb_depth, conic_opacity,
                                   keys_sorted, values_sorted, ranges, bg.ctypes.data, out_u8, out_f32, int(flags), stream)
         _check(rc, "fgs_render_ex")
+
+
+def sort_render(block_x, block_y, num_rendered, width, height, sorting_space, sorting_size, keys_unsorted, values_unsorted,
+                keys_sorted, values_sorted, points_xy, rgb_depth, conic_opacity, ranges, bg_color, out_u8, out_f32, stream=0,
+                flags=BLEND_DEFAULT):
+    """sort_gaussian and render_f32 of a frame whose keys preprocess made, in one call."""
+    bg = _host_f32(bg_color, 3)
+    _check(load().fgs_sort_render(block_x, block_y, num_rendered, width, height, sorting_space, sorting_size, keys_unsorted,
+                                  values_unsorted, keys_sorted, values_sorted, points_xy, rgb_depth, conic_opacity, ranges,
+                                  bg.ctypes.data, out_u8, out_f32, int(flags), stream), "fgs_sort_render")
 
 
 def blend_kernel_name(block_x, block_y, width, height, flags=BLEND_DEFAULT):

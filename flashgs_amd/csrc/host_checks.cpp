@@ -130,6 +130,12 @@ void check_arguments()
     expect(fgs_sort_gaussian(100000, 64, 64, 16, 16, ws, 1000, k, v, k, v, nullptr) == FGS_E_WORKSPACE, "workspace too small");
     expect(fgs_sort_gaussian(0, 64, 64, 16, 16, nullptr, 0, nullptr, nullptr, nullptr, nullptr, nullptr) == FGS_OK, "no pairs: nothing to do");
 
+    refused(fgs_sort_render(16, 16, -1, 64, 64, ws, 1 << 20, k, v, k, v, f, f, f, i32, bg, u8, nullptr, 0, nullptr), "negative pair count in sort_render");
+    refused(fgs_sort_render(16, 16, 5, 64, 64, ws, 1 << 20, k, v, k, v, nullptr, f, f, i32, bg, u8, nullptr, 0, nullptr), "null attributes in sort_render");
+    refused(fgs_sort_render(16, 16, 5, 64, 64, ws, 1 << 20, k, v, k, v, f, f, f, i32, bg, nullptr, nullptr, 0, nullptr), "null image in sort_render");
+    refused(fgs_sort_render(16, 32, 5, 64, 64, ws, 1 << 20, k, v, k, v, f, f, f, i32, bg, u8, nullptr, 0, nullptr), "tile shape in sort_render");
+    refused(fgs_sort_render(16, 16, 5, 64, 64, ws, 1 << 20, k, v, k, v, f, f, f, i32, bg, u8, nullptr, 7, nullptr), "flags in sort_render");
+    expect(fgs_sort_render(16, 16, 100000, 64, 64, ws, 1000, k, v, k, v, f, f, f, i32, bg, u8, nullptr, 0, nullptr) < 0, "workspace too small in sort_render");
     refused(fgs_render_16x16(-1, 64, 64, f, f, f, k, v, i32, bg, u8, nullptr), "negative pair count in render");
     refused(fgs_render_16x16(5, 64, 64, nullptr, f, f, k, v, i32, bg, u8, nullptr), "null attributes in render");
     refused(fgs_render_32x16(0, 64, 64, f, f, f, k, v, i32, bg, nullptr, nullptr), "null image");

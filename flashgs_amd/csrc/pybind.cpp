@@ -205,11 +205,9 @@ int wait_count(torch::Tensor& count_mirror, double timeout_seconds)
     return count;
 }
 
-// pybind.cpp:152-163
-void sort_gaussian(int num_rendered, int width, int height, int block_x, int block_y,
-                   torch::Tensor& list_sorting_space,
-                   torch::Tensor& gaussian_keys_unsorted, torch::Tensor& gaussian_values_unsorted,
-                   torch::Tensor& gaussian_keys_sorted, torch::Tensor& gaussian_values_sorted)
+void check_sort(int num_rendered, const torch::Tensor& list_sorting_space,
+                const torch::Tensor& gaussian_keys_unsorted, const torch::Tensor& gaussian_values_unsorted,
+                const torch::Tensor& gaussian_keys_sorted, const torch::Tensor& gaussian_values_sorted)
 {
     need(num_rendered >= 0, "num_rendered is negative");
     need(list_sorting_space.is_cuda() && list_sorting_space.is_contiguous() && list_sorting_space.element_size() == 1,
@@ -218,7 +216,15 @@ void sort_gaussian(int num_rendered, int width, int height, int block_x, int blo
     need_device(gaussian_values_unsorted, "gaussian_values_unsorted", torch::kInt32, num_rendered, list_sorting_space);
     need_device(gaussian_keys_sorted, "gaussian_keys_sorted", torch::kInt64, num_rendered, list_sorting_space);
     need_device(gaussian_values_sorted, "gaussian_values_sorted", torch::kInt32, num_rendered, list_sorting_space);
+}
 
+// pybind.cpp:152-163
+void sort_gaussian(int num_rendered, int width, int height, int block_x, int block_y,
+                   torch::Tensor& list_sorting_space,
+                   torch::Tensor& gaussian_keys_unsorted, torch::Tensor& gaussian_values_unsorted,
+                   torch::Tensor& gaussian_keys_sorted, torch::Tensor& gaussian_values_sorted)
+{
+    check_sort(num_rendered, list_sorting_space, gaussian_keys_unsorted, gaussian_values_unsorted, gaussian_keys_sorted, gaussian_values_sorted);
     DeviceScope scope(list_sorting_space);
     fgs_check(fgs_sort_gaussian(num_rendered, width, height, block_x, block_y,
                                 (char*)list_sorting_space.data_ptr(), (size_t)list_sorting_space.numel(),
@@ -237,12 +243,11 @@ size_t get_sort_buffer_size(int num_rendered)
     return fgs_get_sort_buffer_size(num_rendered);
 }
 
-// pybind.cpp:170-228
 template <int BX, int BY>
-void render(int num_rendered, int width, int height,
-            torch::Tensor& points_xy, torch::Tensor& rgb_depth, torch::Tensor& conic_opacity,
-            torch::Tensor& gaussian_keys_sorted, torch::Tensor& gaussian_values_sorted,
-            torch::Tensor& ranges, torch::Tensor& bg_color, torch::Tensor& out_color)
+std::vector<float> check_render(int num_rendered, int width, int height,
+                                const torch::Tensor& points_xy, const torch::Tensor& rgb_depth, const torch::Tensor& conic_opacity,
+                                const torch::Tensor& gaussian_keys_sorted, const torch::Tensor& gaussian_values_sorted,
+                                const torch::Tensor& ranges, const torch::Tensor& bg_color, const torch::Tensor& out_color)
 {
     need(num_rendered >= 0, "num_rendered is negative");
     need(width > 0 && height > 0, "width and height must be positive");
@@ -258,7 +263,18 @@ void render(int num_rendered, int width, int height,
     need_device(gaussian_keys_sorted, "gaussian_keys_sorted", torch::kInt64, num_rendered, out_color);
     need_device(gaussian_values_sorted, "gaussian_values_sorted", torch::kInt32, num_rendered, out_color);
     need_device(ranges, "ranges", torch::kInt32, 2 * tiles, out_color);
-    const std::vector<float> bg = host_floats(bg_color, "bg_color", 3);
+    return host_floats(bg_color, "bg_color", 3);
+}
+
+// pybind.cpp:170-228
+template <int BX, int BY>
+void render(int num_rendered, int width, int height,
+            torch::Tensor& points_xy, torch::Tensor& rgb_depth, torch::Tensor& conic_opacity,
+            torch::Tensor& gaussian_keys_sorted, torch::Tensor& gaussian_values_sorted,
+            torch::Tensor& ranges, torch::Tensor& bg_color, torch::Tensor& out_color)
+{
+    const std::vector<float> bg = check_render<BX, BY>(num_rendered, width, height, points_xy, rgb_depth, conic_opacity, gaussian_keys_sorted,
+                                                       gaussian_values_sorted, ranges, bg_color, out_color);
 
     DeviceScope scope(out_color);
     auto fn = BX == 16 ? fgs_render_16x16 : (BY == 16 ? fgs_render_32x16 : fgs_render_32x32);
@@ -268,6 +284,31 @@ void render(int num_rendered, int width, int height,
                  (const uint32_t*)gaussian_values_sorted.data_ptr<int>(),
                  ranges.data_ptr<int>(), bg.data(), (uint8_t*)out_color.data_ptr(), current_stream(out_color)),
               "render");
+}
+
+// No counterpart in the reference: sort_gaussian and then render of one frame whose keys preprocess made, in one call (fgs_sort_render).
+template <int BX, int BY>
+void sort_render(int num_rendered, int width, int height, torch::Tensor& list_sorting_space,
+                 torch::Tensor& gaussian_keys_unsorted, torch::Tensor& gaussian_values_unsorted,
+                 torch::Tensor& gaussian_keys_sorted, torch::Tensor& gaussian_values_sorted,
+                 torch::Tensor& points_xy, torch::Tensor& rgb_depth, torch::Tensor& conic_opacity,
+                 torch::Tensor& ranges, torch::Tensor& bg_color, torch::Tensor& out_color)
+{
+    check_sort(num_rendered, list_sorting_space, gaussian_keys_unsorted, gaussian_values_unsorted, gaussian_keys_sorted, gaussian_values_sorted);
+    const std::vector<float> bg = check_render<BX, BY>(num_rendered, width, height, points_xy, rgb_depth, conic_opacity, gaussian_keys_sorted,
+                                                       gaussian_values_sorted, ranges, bg_color, out_color);
+    need(list_sorting_space.device() == out_color.device(), "list_sorting_space is on a different device");
+
+    DeviceScope scope(out_color);
+    fgs_check(fgs_sort_render(BX, BY, num_rendered, width, height,
+                              (char*)list_sorting_space.data_ptr(), (size_t)list_sorting_space.numel(),
+                              (const uint64_t*)gaussian_keys_unsorted.data_ptr<int64_t>(),
+                              (const uint32_t*)gaussian_values_unsorted.data_ptr<int>(),
+                              (uint64_t*)gaussian_keys_sorted.data_ptr<int64_t>(),
+                              (uint32_t*)gaussian_values_sorted.data_ptr<int>(),
+                              points_xy.data_ptr<float>(), rgb_depth.data_ptr<float>(), conic_opacity.data_ptr<float>(),
+                              ranges.data_ptr<int>(), bg.data(), (uint8_t*)out_color.data_ptr(), nullptr, 0, current_stream(out_color)),
+              "sort_render");
 }
 
 // ---- loadPly (pybind.cpp:12-120) --------------------------------------------------------------------
@@ -317,6 +358,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
     ops.def("render_16x16", &render<16, 16>, "tile ranges and alpha blending, 16x16 tiles");
     ops.def("render_32x16", &render<32, 16>, "tile ranges and alpha blending, 32x16 tiles");
     ops.def("render_32x32", &render<32, 32>, "tile ranges and alpha blending, 32x32 tiles");
+    ops.def("sort_render_16x16", &sort_render<16, 16>, "sort_gaussian and render_16x16 of a frame whose keys preprocess made");
+    ops.def("sort_render_32x16", &sort_render<32, 16>, "sort_gaussian and render_32x16 of a frame whose keys preprocess made");
+    ops.def("sort_render_32x32", &sort_render<32, 32>, "sort_gaussian and render_32x32 of a frame whose keys preprocess made");
     ops.def("preprocess_mirrored", &preprocess_mirrored,
             "preprocess that also stores the pair count into a pinned host tensor as soon as it is known");
     ops.def("preprocess_chained", &preprocess_chained,

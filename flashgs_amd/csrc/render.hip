@@ -13,7 +13,9 @@
 // accumulation), which a caller asks for per call (FGS_BLEND_MATRIX_F16) or per process
 // (fgs_set_colour_sums).
 #include "fgs_internal.h"
+#include "sort.h"
 #include "tile_order.h"
+#include "tile_rank.h"
 
 #include <algorithm>
 #include <atomic>
@@ -36,24 +38,9 @@ __global__ __launch_bounds__(256) void fill_i32_kernel(int* p, size_t n, int v)
 }
 
 
-// The lists of a large frame that are long for it (see long_table) start first: one that starts late ends late, and the launch with
-// it (8K / 8M: lists of 2400 entries that start after a third of the launch end 50 us behind everything else: blend 695 -> 639 us).  The launch that marks the
-// ranges lists them, the first kLongLists workgroups of the blend take them from there, and a tile that finds itself listed leaves itself to
-// them.  A tile is looked for where it would be listed, so whatever the table holds every tile is blended, and what is no such
-// tile is passed over: the table needs no initial value, a list it has no room for starts where it would otherwise.
-// There are two tables: a launch that reads one clears the counts of the other one for the frame that follows.
-constexpr int kLongShards = 32, kLongPerShard = 16, kLongLists = kLongShards * kLongPerShard;
-struct LongLists {
-    uint32_t count[kLongShards], tiles[kLongShards][kLongPerShard];
-};
-__device__ __forceinline__ uint32_t long_shard(uint32_t tile) { return (tile ^ (tile >> 5) ^ (tile >> 10)) % kLongShards; }
-
-// Tiles of a small frame ranked by the length of their lists, longest first (in steps of kOrderStep;
-// the order inside a step is whatever the atomics make it), and behind the ranking how many of them are shared out and from
-// which length on.  One workgroup.
+// The ranking (rank_tiles) is a launch of one workgroup behind the ranges, or a workgroup of the sort's in front of them (fgs_sort_render).
 // (Ranking in the last workgroup of tile_ranges_kernel instead costs more than this launch: every
 // workgroup then has to push its ranges out of its XCD's L2 before it counts itself done.)
-constexpr int kOrderCap = 8192;            // tiles
 // The ranking is written by one launch and read by the next, so it needs memory of its own: one
 // table per (device, stream), allocated on the first such blend on that stream (blends on
 // different streams may overlap and get a table each).  Blends on one stream follow each other, and
@@ -97,73 +84,16 @@ int tile_order_table(hipStream_t stream, uint32_t** out, std::unique_lock<std::m
     return FGS_OK;
 }
 
-// From which length on a tile's list is shared out (see blend_kernel_shared): by what a SIMD walks of the
-// whole frame, as the lists of 256 tiles spread over it say.  Lists are cut alike whether
-// the tiles are ranked or not, so the image is the same.  Called by a whole wave.
-__device__ __forceinline__ int least_shared(const int2* __restrict__ ranges, int num_tiles, int squares, int simds)
-{
-    constexpr int kSamples = 256;
-    uint32_t sum = 0;
-#pragma unroll
-    for (int k = 0; k < kSamples / kWave; k++) {
-        const int2 r = ranges[(long long)(k * kWave + lane_id()) * num_tiles / kSamples];
-        sum += (uint32_t)max(0, r.y - r.x);
-    }
-    sum = (uint32_t)bcast_i((int)wave_inclusive_sum(sum), kWave - 1);
-    const uint64_t each = (uint64_t)sum * (uint32_t)num_tiles / kSamples * (uint32_t)squares / (uint32_t)simds;
-    return least_shared_of(each);
-}
+struct RangeLength {
+    const int2* ranges;
+    __device__ __forceinline__ int operator()(int tile) const { const int2 r = ranges[tile]; return r.y - r.x; }
+};
 
 __global__ __launch_bounds__(1024) void tile_order_kernel(const int2* __restrict__ ranges, int num_tiles,
                                                           uint32_t* __restrict__ tile_order, int squares, int simds)
 {
-    constexpr int kPerThread = kOrderCap / 1024;
     __shared__ uint32_t s_count[kOrderBins];
-    const int tid = threadIdx.x;
-    if (tid < kOrderBins) s_count[tid] = 0;
-    __syncthreads();
-    uint32_t bin[kPerThread], slot[kPerThread];
-#pragma unroll
-    for (int k = 0; k < kPerThread; k++) {
-        const int t = tid + k * 1024;
-        bin[k] = 0; slot[k] = 0;
-        if (t < num_tiles) {
-            const int2 r = ranges[t];
-            bin[k] = (uint32_t)order_bin(r.y - r.x);
-            slot[k] = atomicAdd(&s_count[bin[k]], 1u);
-        }
-    }
-    __syncthreads();
-    if (tid < kWave) {
-        // exclusive prefix over the bins, four per lane
-        static_assert(kOrderBins == 4 * kWave, "four bins per lane");
-        const uint32_t a = s_count[4 * tid], b = s_count[4 * tid + 1], c = s_count[4 * tid + 2], d = s_count[4 * tid + 3];
-        const uint32_t all = a + b + c + d;
-        uint32_t incl = all;
-#pragma unroll
-        for (int o = 1; o < kWave; o <<= 1) {
-            const uint32_t up = (uint32_t)__shfl_up((int)incl, o);
-            if (tid >= o) incl += up;
-        }
-        const uint32_t excl = incl - all;
-        s_count[4 * tid] = excl;
-        s_count[4 * tid + 1] = excl + a;
-        s_count[4 * tid + 2] = excl + a + b;
-        s_count[4 * tid + 3] = excl + a + b + c;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < kPerThread; k++) {
-        const int t = tid + k * 1024;
-        if (t < num_tiles) tile_order[s_count[bin[k]] + slot[k]] = (uint32_t)t;
-    }
-    if (tid < kWave) {
-        const int least = least_shared(ranges, num_tiles, squares, simds);
-        if (tid == 0) {
-            tile_order[kOrderCap] = s_count[first_bin_below(least)];
-            tile_order[kOrderCap + 1] = (uint32_t)least;
-        }
-    }
+    rank_tiles(RangeLength{ranges}, num_tiles, tile_order, squares, simds, s_count);
 }
 
 // render.cu:9-31, with the tile index checked against the number of tiles: what the pair at idx, of tile cur (num_tiles:
@@ -907,7 +837,7 @@ constexpr int kBlendWaves = kFp32 ? 5 : 4;       // resident waves per SIMD
 // more on the others; 6 spills).
 template <int SX, int SY, bool kFp32>
 __global__ __launch_bounds__(kWave * SX * SY) __attribute__((amdgpu_waves_per_eu(kBlendWaves<kFp32>, kBlendWaves<kFp32>))) void blend_kernel(FGS_BLEND_PARAMS,
-    const LongLists* __restrict__ longer, LongLists* __restrict__ next_longer, int long_list)
+    const LongLists* __restrict__ longer, LongLists* __restrict__ next_longer, int long_list, int long_per_shard)
 {
     constexpr int kSquares = SX * SY;
     __shared__ __align__(16) float s_stage[kSquares][kStageFloats];
@@ -916,7 +846,8 @@ __global__ __launch_bounds__(kWave * SX * SY) __attribute__((amdgpu_waves_per_eu
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = kSquares == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     int tile_x, tile_y;
-    const bool first = longer && blockIdx.x < (unsigned)kLongLists;
+    const int long_lists = longer ? kLongShards * long_per_shard : 0;
+    const bool first = (int)blockIdx.x < long_lists;
     if (first) {
         const uint32_t shard = blockIdx.x % kLongShards, at = blockIdx.x / kLongShards;
         if (at == 0 && threadIdx.x == 0) next_longer->count[shard] = 0;
@@ -924,7 +855,7 @@ __global__ __launch_bounds__(kWave * SX * SY) __attribute__((amdgpu_waves_per_eu
         if (at >= longer->count[shard] || tile >= (uint32_t)(tiles_x * tiles_y) || long_shard(tile) != shard) return;
         tile_x = (int)(tile % (uint32_t)tiles_x);
         tile_y = (int)(tile / (uint32_t)tiles_x);
-    } else if (!tile_of_position((int)blockIdx.x - (longer ? kLongLists : 0), tiles_x, tiles_y, &tile_x, &tile_y)) {
+    } else if (!tile_of_position((int)blockIdx.x - long_lists, tiles_x, tiles_y, &tile_x, &tile_y)) {
         return;
     }
     const uint32_t tile = (uint32_t)(tile_y * tiles_x + tile_x);
@@ -932,7 +863,7 @@ __global__ __launch_bounds__(kWave * SX * SY) __attribute__((amdgpu_waves_per_eu
     const int n = range.y - range.x;
     if (longer && !first && n >= long_list) {       // left to one of the first workgroups?
         const uint32_t shard = long_shard(tile), at = (uint32_t)lane;
-        const bool listed = at < min(longer->count[shard], (uint32_t)kLongPerShard) && longer->tiles[shard][at % kLongPerShard] == tile;
+        const bool listed = at < min(longer->count[shard], (uint32_t)long_per_shard) && longer->tiles[shard][at % kLongPerShard] == tile;
         if (ballot(listed) != 0) return;
     }
     // A launch ends when its longest list ends, and a wave that shares its SIMD equally with the
@@ -1046,7 +977,7 @@ void blend_kernel_shared(FGS_BLEND_PARAMS, const uint32_t* __restrict__ tile_ord
         active = group >= alone || team == 0;
         least = (int)tile_order[kOrderCap + 1];
     } else {
-        least = least_shared(ranges, num_tiles, kSquares, simds);
+        least = least_shared(RangeLength{ranges}, num_tiles, kSquares, simds);
     }
     active = active && rank < num_tiles;
     int tile_x = 0, tile_y = 0;
@@ -1341,6 +1272,7 @@ constexpr int kSampledPairs = 3 << 20;
 struct LongTable {
     LongLists *list = nullptr, *next = nullptr;
     int least = 0;
+    int per_shard = kLongPerShard / 2;
 };
 
 // A list is long for its frame if it has a seventh of the entries that a SIMD has on average: it takes 166 ns per entry beside others
@@ -1414,31 +1346,56 @@ int teams_of(int sx, int sy, int num_tiles, int cus)
     return 4;
 }
 
-// render.cu:566-575
-// rank: a blend by itself (fgs_blend) is two launches, the ranking and the blend.  Behind the ranges of the same call (fgs_render)
-// a frame whose workgroups are all resident at once even with one tile each goes unranked, since nothing starts later than
-// anything else there; the image is the same bits.  256x192 / 2.8k pairs 11.1 -> 8.7 us, 348k pairs 181 -> 178, 400x300 / 362k
-// 110 -> 107, opaque needles 110 -> 117, 700x600 in 32x32 tiles 114 -> 112.
-int blend_impl(bool rank, const LongTable& longer, int block_x, int block_y, int width, int height,
-               const float* points_xy, const float* rgb_depth, const float* conic_opacity,
-               const uint32_t* values_sorted, const int* ranges, const float bg[3],
-               uint8_t* out_u8, float* out_f32, int flags, void* stream, const char* who)
+// What a blend takes, checked before anything is launched for it.
+int check_blend(int block_x, int block_y, int width, int height, const float* points_xy, const float* rgb_depth, const float* conic_opacity,
+                const int* ranges, const float* bg, const uint8_t* out_u8, const float* out_f32, int flags, int* sx, int* sy, int* mode, const char* who)
 {
-    int sx = 0, sy = 0, mode = 0;
-    int rc = check_tile(block_x, block_y, &sx, &sy, who);
+    int rc = check_tile(block_x, block_y, sx, sy, who);
     if (rc != FGS_OK) return rc;
-    rc = colour_mode(flags, &mode, who);
+    rc = colour_mode(flags, mode, who);
     if (rc != FGS_OK) return rc;
     if (width <= 0 || height <= 0) return fail(FGS_E_INVALID, "%s: width/height must be positive", who);
     if (!ranges || !bg || (!out_u8 && !out_f32)) return fail(FGS_E_INVALID, "%s: null ranges, bg_color or output", who);
     if (((uintptr_t)rgb_depth | (uintptr_t)conic_opacity) % 16 != 0 ||
         ((uintptr_t)points_xy | (uintptr_t)ranges) % 8 != 0)
         return fail(FGS_E_INVALID, "%s: rgb_depth/conic_opacity must be 16-byte aligned, points_xy/ranges 8-byte aligned", who);
+    if (positions_of((width + block_x - 1) / block_x, (height + block_y - 1) / block_y) > 0x7fffffffLL - kLongShards * kLongPerShard)
+        return fail(FGS_E_INVALID, "%s: image too large", who);
+    return FGS_OK;
+}
+
+// How the blend of a ranked frame is launched.
+struct SharedGrid {
+    int cus = 0, teams = 0, resident = 0;       // teams of a workgroup, workgroups that are resident at once
+};
+int shared_grid(int sx, int sy, int num_tiles, bool fp32, SharedGrid* out)
+{
+    int device = 0;
+    FGS_HIP_TRY(hipGetDevice(&device));
+    FGS_HIP_TRY(hipDeviceGetAttribute(&out->cus, hipDeviceAttributeMultiprocessorCount, device));
+    out->teams = teams_of(sx, sy, num_tiles, out->cus);
+    out->resident = out->cus * std::max(1, 4 * (fp32 ? kBlendWaves<true> : kBlendWaves<false>) / (sx * sy * out->teams));
+    return FGS_OK;
+}
+
+// render.cu:566-575
+// ranked: the table of ranks of a frame that is ranked already, whose lock the caller holds, or null.
+// rank: a blend by itself (fgs_blend) is two launches, the ranking and the blend.  Behind the ranges of the same call (fgs_render)
+// a frame whose workgroups are all resident at once even with one tile each goes unranked, since nothing starts later than
+// anything else there; the image is the same bits.  256x192 / 2.8k pairs 11.1 -> 8.7 us, 348k pairs 181 -> 178, 400x300 / 362k
+// 110 -> 107, opaque needles 110 -> 117, 700x600 in 32x32 tiles 114 -> 112.
+int blend_impl(bool rank, uint32_t* ranked, const LongTable& longer, int block_x, int block_y, int width, int height,
+               const float* points_xy, const float* rgb_depth, const float* conic_opacity,
+               const uint32_t* values_sorted, const int* ranges, const float bg[3],
+               uint8_t* out_u8, float* out_f32, int flags, void* stream, const char* who)
+{
+    int sx = 0, sy = 0, mode = 0;
+    int rc = check_blend(block_x, block_y, width, height, points_xy, rgb_depth, conic_opacity, ranges, bg, out_u8, out_f32, flags, &sx, &sy, &mode, who);
+    if (rc != FGS_OK) return rc;
     const int tiles_x = (width + block_x - 1) / block_x, tiles_y = (height + block_y - 1) / block_y;
     hipStream_t st = (hipStream_t)stream;
     // one workgroup per tile of the image padded to whole blocks of tiles, blocks padded to a multiple of 8
     const long long groups = positions_of(tiles_x, tiles_y);
-    if (groups > 0x7fffffffLL - kLongLists) return fail(FGS_E_INVALID, "%s: image too large", who);
     const int num_tiles = tiles_x * tiles_y;
     const bool fp32 = mode == FGS_COLOUR_SUMS_FP32;
 #define FGS_BLEND_ARGS (const int2*)ranges, values_sorted, width, height, tiles_x, tiles_y,                     \
@@ -1446,26 +1403,25 @@ int blend_impl(bool rank, const LongTable& longer, int block_x, int block_y, int
                        bg[0], bg[1], bg[2], out_u8, out_f32
     if (!is_ranked(tiles_x, tiles_y)) {
         auto launch = [&](auto kernel) {
-            hipLaunchKernelGGL(kernel, dim3((unsigned)(groups + (longer.list ? kLongLists : 0))), dim3(kWave * sx * sy), 0, st, FGS_BLEND_ARGS,
-                               (const LongLists*)longer.list, longer.next, longer.least);
+            hipLaunchKernelGGL(kernel, dim3((unsigned)(groups + (longer.list ? kLongShards * longer.per_shard : 0))), dim3(kWave * sx * sy), 0, st, FGS_BLEND_ARGS,
+                               (const LongLists*)longer.list, longer.next, longer.least, longer.per_shard);
         };
         if (sx == 1 && sy == 1) launch(fp32 ? blend_kernel<1, 1, true> : blend_kernel<1, 1, false>);
         else if (sx == 2 && sy == 1) launch(fp32 ? blend_kernel<2, 1, true> : blend_kernel<2, 1, false>);
         else launch(fp32 ? blend_kernel<2, 2, true> : blend_kernel<2, 2, false>);
         return check_hip(hipGetLastError(), who);
     }
-    int device = 0, cus = 0;
-    FGS_HIP_TRY(hipGetDevice(&device));
-    FGS_HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
-    uint32_t* tile_order = nullptr;
+    SharedGrid grid;
+    rc = shared_grid(sx, sy, num_tiles, fp32, &grid);
+    if (rc != FGS_OK) return rc;
+    const int cus = grid.cus, teams = grid.teams, waves = sx * sy * teams, resident = grid.resident;
+    uint32_t* tile_order = ranked;
     std::unique_lock<std::mutex> enqueue;       // from the ranking to the blend that reads it
-    const int teams = teams_of(sx, sy, num_tiles, cus), waves = sx * sy * teams;
-    const int resident = cus * std::max(1, 4 * (fp32 ? kBlendWaves<true> : kBlendWaves<false>) / waves);
-    if (rank || num_tiles > resident) {
+    if (!ranked && (rank || num_tiles > resident)) {
         rc = tile_order_table(st, &tile_order, &enqueue);
         if (rc != FGS_OK) return rc;
     }
-    if (tile_order)
+    if (tile_order && !ranked)
         hipLaunchKernelGGL(tile_order_kernel, dim3(1), dim3(1024), 0, st, (const int2*)ranges, num_tiles, tile_order, sx * sy, 4 * cus);
     auto launch = [&](auto kernel) {
         const int per_group = num_tiles <= resident ? 1 : teams;
@@ -1505,7 +1461,50 @@ int render_impl(int block_x, int block_y, int num_rendered, int width, int heigh
     }
     rc = ranges_impl(block_x, block_y, num_rendered, width, height, keys_sorted, ranges, longer, stream, who);
     if (rc != FGS_OK) return rc;
-    return blend_impl(false, longer, block_x, block_y, width, height, points_xy, rgb_depth, conic_opacity, values_sorted, ranges,
+    return blend_impl(false, nullptr, longer, block_x, block_y, width, height, points_xy, rgb_depth, conic_opacity, values_sorted, ranges,
+                      bg, out_u8, out_f32, flags, stream, who);
+}
+
+// Sort and render of one frame.  The sort knows where every tile's pairs stand: its segment launches write the ranges and list the long lists,
+// and a workgroup of the scatter ranks the tiles of a small frame, so the launches that would find all this in the sorted keys are left out (720p / 0.2M
+// pairs: two of ten, 9 us of 77).  Where the sort has no such table (one pair, more than 2^18 tile ids) they follow it as in render_impl.
+int sort_render_impl(int block_x, int block_y, int num_rendered, int width, int height, char* list_sorting_space, size_t sorting_size,
+                     const uint64_t* keys_unsorted, const uint32_t* values_unsorted, uint64_t* keys_sorted, uint32_t* values_sorted,
+                     const float* points_xy, const float* rgb_depth, const float* conic_opacity, int* ranges, const float bg[3],
+                     uint8_t* out_u8, float* out_f32, int flags, void* stream, const char* who)
+{
+    int sx = 0, sy = 0, mode = 0;
+    int rc = check_blend(block_x, block_y, width, height, points_xy, rgb_depth, conic_opacity, ranges, bg, out_u8, out_f32, flags, &sx, &sy, &mode, who);
+    if (rc != FGS_OK) return rc;
+    if (num_rendered > 0 && (!points_xy || !rgb_depth || !conic_opacity)) return fail(FGS_E_INVALID, "%s: null buffer", who);
+    const int tiles_x = (width + block_x - 1) / block_x, tiles_y = (height + block_y - 1) / block_y, num_tiles = tiles_x * tiles_y;
+    LongTable longer;
+    std::unique_lock<std::mutex> enqueue, ranking;      // from the launch that writes a table to the blend that reads it
+    rc = long_table((hipStream_t)stream, num_rendered, block_x, block_y, width, height, &longer, &enqueue);
+    if (rc != FGS_OK) return rc;
+    FrameTables frame = { { (int2*)ranges, longer.list, (uint32_t)num_tiles, longer.least }, { nullptr, num_tiles, sx * sy, 0 } };
+    if (num_rendered > 0 && is_ranked(tiles_x, tiles_y)) {
+        SharedGrid grid;
+        rc = shared_grid(sx, sy, num_tiles, mode == FGS_COLOUR_SUMS_FP32, &grid);
+        if (rc != FGS_OK) return rc;
+        frame.ranking.simds = 4 * grid.cus;
+        if (num_tiles > grid.resident) {
+            rc = tile_order_table((hipStream_t)stream, &frame.ranking.order, &ranking);
+            if (rc != FGS_OK) return rc;
+        }
+    }
+    rc = sort_impl(num_rendered, width, height, block_x, block_y, list_sorting_space, sorting_size, keys_unsorted, values_unsorted,
+                   keys_sorted, values_sorted, &frame, stream, who);
+    if (rc != FGS_OK) return rc;
+    // The segment launch comes by the tiles in their order, and with half of the places the last ones of a horizon found none: frames of 763 and 793 long
+    // lists (8K / 8M, 6620x4058 / 6M) take 1.00 and 0.98 of the time behind a launch of their own with half of the places, 0.988 and 0.93 with all.
+    if (frame.notes.longer) longer.per_shard = kLongPerShard;
+    if (!frame.notes.ranges) {
+        rc = ranges_impl(block_x, block_y, num_rendered, width, height, keys_sorted, ranges, longer, stream, who);
+        if (rc != FGS_OK) return rc;
+    }
+    if (!frame.ranking.order && ranking.owns_lock()) ranking.unlock();          // (the blend ranks by itself)
+    return blend_impl(false, frame.ranking.order, longer, block_x, block_y, width, height, points_xy, rgb_depth, conic_opacity, values_sorted, ranges,
                       bg, out_u8, out_f32, flags, stream, who);
 }
 
@@ -1548,6 +1547,19 @@ extern "C" int fgs_render_ex(int block_x, int block_y, int num_rendered, int wid
     return fgs::render_impl(block_x, block_y, num_rendered, width, height, points_xy, rgb_depth,
                             conic_opacity, gaussian_keys_sorted, gaussian_values_sorted, ranges, bg_color,
                             out_color_u8, out_color_f32, flags, stream, "fgs_render_ex");
+}
+
+extern "C" int fgs_sort_render(int block_x, int block_y, int num_rendered, int width, int height,
+                               char* list_sorting_space, size_t sorting_size,
+                               const uint64_t* gaussian_keys_unsorted, const uint32_t* gaussian_values_unsorted,
+                               uint64_t* gaussian_keys_sorted, uint32_t* gaussian_values_sorted,
+                               const float* points_xy, const float* rgb_depth, const float* conic_opacity,
+                               int* ranges, const float bg_color[3], uint8_t* out_color_u8, float* out_color_f32,
+                               int flags, void* stream)
+{
+    return fgs::sort_render_impl(block_x, block_y, num_rendered, width, height, list_sorting_space, sorting_size, gaussian_keys_unsorted,
+                                 gaussian_values_unsorted, gaussian_keys_sorted, gaussian_values_sorted, points_xy, rgb_depth, conic_opacity,
+                                 ranges, bg_color, out_color_u8, out_color_f32, flags, stream, "fgs_sort_render");
 }
 
 extern "C" int fgs_set_colour_sums(int mode)
@@ -1599,7 +1611,7 @@ extern "C" int fgs_blend(int block_x, int block_y, int width, int height,
                          const uint32_t* gaussian_values_sorted, const int* ranges, const float bg_color[3],
                          uint8_t* out_color_u8, float* out_color_f32, void* stream)
 {
-    return fgs::blend_impl(true, fgs::LongTable(), block_x, block_y, width, height, points_xy, rgb_depth, conic_opacity,
+    return fgs::blend_impl(true, nullptr, fgs::LongTable(), block_x, block_y, width, height, points_xy, rgb_depth, conic_opacity,
                            gaussian_values_sorted, ranges, bg_color, out_color_u8, out_color_f32, 0, stream, "fgs_blend");
 }
 
@@ -1608,7 +1620,7 @@ extern "C" int fgs_blend_ex(int block_x, int block_y, int width, int height,
                             const uint32_t* gaussian_values_sorted, const int* ranges, const float bg_color[3],
                             uint8_t* out_color_u8, float* out_color_f32, int flags, void* stream)
 {
-    return fgs::blend_impl(true, fgs::LongTable(), block_x, block_y, width, height, points_xy, rgb_depth, conic_opacity,
+    return fgs::blend_impl(true, nullptr, fgs::LongTable(), block_x, block_y, width, height, points_xy, rgb_depth, conic_opacity,
                            gaussian_values_sorted, ranges, bg_color, out_color_u8, out_color_f32, flags, stream, "fgs_blend_ex");
 }
 

@@ -32,6 +32,7 @@
 // segment sort of up to 1024 pairs: 67 (70 with 9-bit digits), against 8 + 6 * 24 = 152 for a six-pass LSD sort of 47 bits.  Segments of 1025 to
 // 16384 pairs are read a second time, behind the merges; what sorts again is written and read twice more, and the longest segments are read twice and written once per counting pass.
 #include "fgs_internal.h"
+#include "sort.h"
 
 #include <algorithm>
 #include <type_traits>
@@ -913,7 +914,7 @@ template <int kItems>
 __global__ __launch_bounds__(kOnePassThreads) void tile_scatter_kernel(const uint64_t* __restrict__ keys, const uint32_t* __restrict__ values,
                                                                        uint64_t* __restrict__ words, int n, uint32_t ids,
                                                                        const uint32_t* __restrict__ offsets, const uint32_t* __restrict__ totals,
-                                                                       const uint32_t* __restrict__ marks, int* __restrict__ seg_start)
+                                                                       const uint32_t* __restrict__ marks, int* __restrict__ seg_start, TileRanking ranks)
 {
     constexpr int kTile = kOnePassThreads * kItems, kPer = kOnePassIds / kOnePassThreads, kHigh = kOnePassBits - kOnePassLow;
     typedef uint32_t Four __attribute__((ext_vector_type(4)));
@@ -926,9 +927,15 @@ __global__ __launch_bounds__(kOnePassThreads) void tile_scatter_kernel(const uin
     __shared__ uint32_t s_wave_sum[kOnePassWaves];
     static_assert(kHigh <= kOnePassLow, "the counts of either pass");
     const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
+    // The first workgroup of a launch with one more than there are blocks ranks the frame's tiles meanwhile.
+    const int ranking = ranks.order ? 1 : 0, blocks = (int)gridDim.x - ranking, index = (int)blockIdx.x - ranking;
+    if (index < 0) {
+        rank_tiles([&](int t) { return (int)totals[t]; }, ranks.num_tiles, ranks.order, ranks.squares, ranks.simds, s_to);
+        return;
+    }
     // (neighbouring blocks on one XCD, as in scatter_kernel)
-    const int xcd = (int)blockIdx.x % kXcds, each = (int)gridDim.x / kXcds, rest = (int)gridDim.x % kXcds;
-    const int block = xcd * each + min(xcd, rest) + (int)blockIdx.x / kXcds;
+    const int xcd = index % kXcds, each = blocks / kXcds, rest = blocks % kXcds;
+    const int block = xcd * each + min(xcd, rest) + index / kXcds;
     const int base = block * kTile, in_tile = min(kTile, n - base);
     const int first = wave * (kWave * kItems) + lane;
     uint64_t word[kItems];
@@ -1957,7 +1964,7 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(7))) void
     int list_max0, int list_max1, int list_max2,
     uint32_t* __restrict__ seg_counts, uint32_t* __restrict__ list0, uint32_t* __restrict__ list1,
     uint32_t* __restrict__ list2, uint32_t* __restrict__ list3,
-    uint32_t list_cap0, uint32_t list_cap1, uint32_t list_cap2, uint32_t list_cap3)
+    uint32_t list_cap0, uint32_t list_cap1, uint32_t list_cap2, uint32_t list_cap3, TileNotes notes)
 {
     __shared__ uint64_t s_w[staging_words(kT * kWave)];
     for (uint32_t v = blockIdx.x; v <= tile_mask; v += gridDim.x) {
@@ -1972,6 +1979,7 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(7))) void
             // (lengths up to list_max0, list_max1, list_max2, and everything longer), so that those
             // fewer, longer-running segments can be dealt out evenly by the launches that follow.
             const int len = hi - lo;
+            if (kWords && threadIdx.x == 0) note_tile(notes, v, lo, hi);
             if (len > kT * kWave && threadIdx.x == 0) {
                 // neighbouring tiles tend to be equally busy: mix the index so that every list gets its share
                 const uint32_t shard = (v ^ (v >> 5) ^ (v >> 10) ^ (v >> 15)) % kListShards;
@@ -1993,13 +2001,14 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(7))) void
 // A list of at most kAlonePairs pairs in few tiles: one workgroup per tile id, of which one wave does unless the segment has more than
 // 1024 pairs, so that no other launch is needed for those.
 static_assert(Short::kTile <= kCapSmall, "a list of one such block has no segment of the listed classes");
-__global__ __launch_bounds__(4 * kWave) void segment_sort_alone_kernel(Lists lists, const int* __restrict__ seg_start)
+__global__ __launch_bounds__(4 * kWave) void segment_sort_alone_kernel(Lists lists, const int* __restrict__ seg_start, TileNotes notes)
 {
     static_assert(kAlonePairs <= kCapMedium, "four waves hold any segment");
     __shared__ uint64_t s_w[4 * staging_words(kCapMedium / 4)];
     __shared__ Between<4> s_between;
     const uint32_t v = blockIdx.x;
     const int lo = seg_start[v], hi = seg_start[v + 1];
+    if (threadIdx.x == 0) note_tile(notes, v, lo, hi);
     if (hi - lo > kCapSmall) sort_segment_waves<4, kCapMedium, 8, true>(lists, v, lo, hi, s_w, s_between);
     else if (hi > lo && threadIdx.x < kWave) sort_segment_wave<kCapSmall / kWave, true>(lists, v, lo, hi, s_w);
 }
@@ -2133,37 +2142,38 @@ extern "C" size_t fgs_get_sort_buffer_size(int num_rendered)
     return fgs::workspace_for(num_rendered).total;
 }
 
-extern "C" int fgs_sort_gaussian(int num_rendered,
-                                 int width, int height, int block_x, int block_y,
-                                 char* list_sorting_space, size_t sorting_size,
-                                 const uint64_t* gaussian_keys_unsorted, const uint32_t* gaussian_values_unsorted,
-                                 uint64_t* gaussian_keys_sorted, uint32_t* gaussian_values_sorted, void* stream)
+namespace fgs {
+
+int sort_impl(int num_rendered, int width, int height, int block_x, int block_y, char* list_sorting_space, size_t sorting_size,
+              const uint64_t* gaussian_keys_unsorted, const uint32_t* gaussian_values_unsorted,
+              uint64_t* gaussian_keys_sorted, uint32_t* gaussian_values_sorted, FrameTables* frame, void* stream, const char* who)
 {
-    using namespace fgs;
+    FrameTables tables = {};
+    if (frame) std::swap(tables, *frame);           // what is written comes back
     if (num_rendered < 0)
-        return fail(FGS_E_INVALID, "fgs_sort_gaussian: num_rendered = %d is negative "
-                                   "(a negative count is what a failed preprocess leaves behind)", num_rendered);
+        return fail(FGS_E_INVALID, "%s: num_rendered = %d is negative "
+                                   "(a negative count is what a failed preprocess leaves behind)", who, num_rendered);
     if (num_rendered > FGS_MAX_RENDERED)
-        return fail(FGS_E_INVALID, "fgs_sort_gaussian: num_rendered = %d exceeds %d", num_rendered, FGS_MAX_RENDERED);
+        return fail(FGS_E_INVALID, "%s: num_rendered = %d exceeds %d", who, num_rendered, FGS_MAX_RENDERED);
     if (width <= 0 || height <= 0 || block_x <= 0 || block_y <= 0)
-        return fail(FGS_E_INVALID, "fgs_sort_gaussian: width/height/block must be positive");
+        return fail(FGS_E_INVALID, "%s: width/height/block must be positive", who);
     if (num_rendered == 0) return FGS_OK;
     if (!list_sorting_space || !gaussian_keys_unsorted || !gaussian_values_unsorted ||
         !gaussian_keys_sorted || !gaussian_values_sorted)
-        return fail(FGS_E_INVALID, "fgs_sort_gaussian: null buffer");
+        return fail(FGS_E_INVALID, "%s: null buffer", who);
     if ((uintptr_t)list_sorting_space % 256 != 0)
-        return fail(FGS_E_INVALID, "fgs_sort_gaussian: list_sorting_space must be 256-byte aligned");
+        return fail(FGS_E_INVALID, "%s: list_sorting_space must be 256-byte aligned", who);
     if (((uintptr_t)gaussian_keys_unsorted | (uintptr_t)gaussian_keys_sorted) % 8 != 0)
-        return fail(FGS_E_INVALID, "fgs_sort_gaussian: key buffers must be 8-byte aligned");
+        return fail(FGS_E_INVALID, "%s: key buffers must be 8-byte aligned", who);
 
     const int n = num_rendered;
     const Workspace ws = workspace_for(n);
     if (sorting_size < ws.total)
-        return fail(FGS_E_WORKSPACE, "fgs_sort_gaussian: list_sorting_space holds %zu bytes, %zu needed for %d pairs",
-                    sorting_size, ws.total, n);
+        return fail(FGS_E_WORKSPACE, "%s: list_sorting_space holds %zu bytes, %zu needed for %d pairs",
+                    who, sorting_size, ws.total, n);
 
     const long long tiles_xy = (long long)((width + block_x - 1) / block_x) * ((height + block_y - 1) / block_y);
-    if (tiles_xy >= (1LL << 30)) return fail(FGS_E_INVALID, "fgs_sort_gaussian: too many tiles");
+    if (tiles_xy >= (1LL << 30)) return fail(FGS_E_INVALID, "%s: too many tiles", who);
     const int tile_bits = bit_length((uint32_t)tiles_xy);         // sort.cu:34-39: bits [0, 32 + tile_bits)
     const uint32_t tile_mask = (1u << tile_bits) - 1u;
 
@@ -2191,6 +2201,7 @@ extern "C" int fgs_sort_gaussian(int num_rendered,
         seg_counts = (uint32_t*)(list_sorting_space + ws.seg_lists);
     }
     const bool words = tile_bits <= kWordsMaxTileBits;              // at most two passes
+    if (frame && words) frame->notes = tables.notes;
 
     // 1. stable partition by tile id, least significant tile digit first
     auto partition = [&](auto shape) {
@@ -2276,8 +2287,10 @@ extern "C" int fgs_sort_gaussian(int num_rendered,
         hipLaunchKernelGGL((tile_count_kernel<kItems>), dim3(blocks), dim3(kOnePassThreads), 0, st, gaussian_keys_unsorted, n, ids, rows, beyond, seg_counts);
         hipLaunchKernelGGL(tile_offsets_kernel, dim3(ids / kColumnTiles), dim3(kOnePassThreads), 0, st, (const uint16_t*)rows, blocks, ids, offsets, totals,
                            gaussian_keys_unsorted, (const uint32_t*)beyond, marks);
-        hipLaunchKernelGGL((tile_scatter_kernel<kItems>), dim3(blocks), dim3(kOnePassThreads), 0, st, gaussian_keys_unsorted, gaussian_values_unsorted,
-                           gaussian_keys_sorted, n, ids, (const uint32_t*)offsets, (const uint32_t*)totals, (const uint32_t*)marks, seg_start);
+        if (frame) frame->ranking = tables.ranking;
+        hipLaunchKernelGGL((tile_scatter_kernel<kItems>), dim3(blocks + (tables.ranking.order ? 1 : 0)), dim3(kOnePassThreads), 0, st, gaussian_keys_unsorted,
+                           gaussian_values_unsorted, gaussian_keys_sorted, n, ids, (const uint32_t*)offsets, (const uint32_t*)totals,
+                           (const uint32_t*)marks, seg_start, tables.ranking);
         return true;
     };
     const bool one_digit = tile_bits >= kOnePassLeastBits && tile_bits <= kOnePassBits;         // (up to 8 bits are one pass of that digit)
@@ -2323,7 +2336,7 @@ extern "C" int fgs_sort_gaussian(int num_rendered,
     hipLaunchKernelGGL((segment_sort_wave_kernel<(CAP) / kWave, WORDS>), dim3((ids + ids_per_wave - 1) / ids_per_wave), dim3(kWave),              \
                        0, st, lists, n, tile_mask, (const int*)seg_start,                                     \
                        kCapSmall, kCapMedium, kCapLarge, seg_counts, list_small, list_medium,                 \
-                       list_large, list_long, cap_small, cap_medium, cap_large, cap_long)
+                       list_large, list_long, cap_small, cap_medium, cap_large, cap_long, tables.notes)
 #define FGS_SEGMENT_CLASS(WAVES, CAP, LEAST, WORDS, MINLEN, GRID, LIST, COUNT, LISTCAP)                         \
     hipLaunchKernelGGL((segment_sort_kernel<WAVES, CAP, LEAST, WORDS>), dim3(GRID), dim3((WAVES) * kWave), 0, st,  \
                        lists, n, tile_mask, MINLEN, (const int*)seg_start,                                    \
@@ -2346,7 +2359,7 @@ extern "C" int fgs_sort_gaussian(int num_rendered,
     const int first_class = merged_tail ? 1 : merged_large ? 2 : 3;
     const unsigned medium_blocks = list_grid((unsigned)(n / (kCapSmall + 1) + 1), 4096u), large_blocks = list_grid((unsigned)(n / (kCapMedium + 1) + 1), 1024u);
     if (few_ids) {
-        hipLaunchKernelGGL(segment_sort_alone_kernel, dim3(ids), dim3(4 * kWave), 0, st, lists, (const int*)seg_start);
+        hipLaunchKernelGGL(segment_sort_alone_kernel, dim3(ids), dim3(4 * kWave), 0, st, lists, (const int*)seg_start, tables.notes);
     } else if (words) {
         // Up to 1024 pairs: one wave, network in registers; one tile id per wave on all but long lists (neighbouring
         // tiles tend to be equally busy, so a wave that took several of them would become the tail
@@ -2386,4 +2399,16 @@ extern "C" int fgs_sort_gaussian(int num_rendered,
 #undef FGS_SEGMENT_CLASS
 #undef FGS_SEGMENT_GENERAL
     return check_hip(hipGetLastError(), "sort launch");
+}
+
+} // namespace fgs
+
+extern "C" int fgs_sort_gaussian(int num_rendered,
+                                 int width, int height, int block_x, int block_y,
+                                 char* list_sorting_space, size_t sorting_size,
+                                 const uint64_t* gaussian_keys_unsorted, const uint32_t* gaussian_values_unsorted,
+                                 uint64_t* gaussian_keys_sorted, uint32_t* gaussian_values_sorted, void* stream)
+{
+    return fgs::sort_impl(num_rendered, width, height, block_x, block_y, list_sorting_space, sorting_size, gaussian_keys_unsorted,
+                          gaussian_values_unsorted, gaussian_keys_sorted, gaussian_values_sorted, nullptr, stream, "fgs_sort_gaussian");
 }

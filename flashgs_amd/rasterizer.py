@@ -1,5 +1,5 @@
 """Driver with the shape of FlashGS's ``example.py``: ``Scene``, ``Camera``, a statically allocated
-``Rasterizer`` whose ``forward`` runs preprocess -> pair count -> sort_gaussian -> render_16x16
+``Rasterizer`` whose ``forward`` runs preprocess -> pair count -> sort_gaussian -> render_16x16 (the latter two in one call)
 through ``flash_gaussian_splatting.ops``, ``savePpm`` and ``render_scene``.
 
 Differences from the reference driver: the output image is allocated once instead of per frame,
@@ -99,7 +99,7 @@ class Rasterizer:
     def __init__(self, scene, MAX_NUM_RENDERED, MAX_NUM_TILES, tile=(16, 16), max_width=0, max_height=0):
         dev = scene.device
         self.tile = tuple(tile)
-        self._render = getattr(ops(), self.RENDER[self.tile])
+        self._sort_render = getattr(ops(), "sort_" + self.RENDER[self.tile])
         self.gaussian_keys_unsorted = torch.zeros(MAX_NUM_RENDERED, device=dev, dtype=torch.int64)
         self.gaussian_values_unsorted = torch.zeros(MAX_NUM_RENDERED, device=dev, dtype=torch.int32)
         self.gaussian_keys_sorted = torch.zeros(MAX_NUM_RENDERED, device=dev, dtype=torch.int64)
@@ -191,14 +191,11 @@ class Rasterizer:
                              "(fgs_set_scan_spin_limit polls); the frame was not rendered")
         if num_rendered >= self.MAX_NUM_RENDERED:
             raise TooManyPairs("Too many k-v pairs! (%d, capacity %d)" % (num_rendered, self.MAX_NUM_RENDERED))
-        o.sort_gaussian(num_rendered, camera.width, camera.height, bx, by, self.list_sorting_space,
-                        self.gaussian_keys_unsorted, self.gaussian_values_unsorted,
-                        self.gaussian_keys_sorted, self.gaussian_values_sorted)
         out_color = self._image(camera, scene.device) if out is None else out
-        self._render(num_rendered, camera.width, camera.height,
-                     self.points_xy, self.rgb_depth, self.conic_opacity,
-                     self.gaussian_keys_sorted, self.gaussian_values_sorted,
-                     self.ranges, bg_color, out_color)
+        self._sort_render(num_rendered, camera.width, camera.height, self.list_sorting_space,
+                          self.gaussian_keys_unsorted, self.gaussian_values_unsorted,
+                          self.gaussian_keys_sorted, self.gaussian_values_sorted,
+                          self.points_xy, self.rgb_depth, self.conic_opacity, self.ranges, bg_color, out_color)
         return out_color
 
 

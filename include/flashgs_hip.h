@@ -168,7 +168,7 @@ size_t fgs_get_sort_buffer_size(int num_rendered);
  * those with a curvature along y beyond -3 (splats that were not widened by 0.3), saddles and non-finite ones take
  * slower paths.
  * A frame of at most 8192 tiles first ranks its tiles by list length into a table the library keeps per
- * (device, stream) (37 KB, allocated on the first call on that stream that uses it); fgs_render_* leaves the ranking out where
+ * (device, stream) (41 KB, allocated on the first call on that stream that uses it); fgs_render_* leaves the ranking out where
  * the frame is so small that all its workgroups are resident at once, and lists the long lists of a frame of 65536 tiles and 3 * 2^20 pairs or more
  * in the same memory, so that they are blended first.  Lists that are long for the frame are blended in
  * runs by several waves and folded front to back.  The run that holds the stop of render.cu:394-408 is walked again
@@ -205,6 +205,19 @@ int fgs_render_f32(int block_x, int block_y, int num_rendered, int width, int he
                    const uint64_t* gaussian_keys_sorted, const uint32_t* gaussian_values_sorted,
                    int* ranges, const float bg_color[3], uint8_t* out_color_u8, float* out_color_f32,
                    void* stream);
+
+/*
+ * No counterpart in the reference: fgs_sort_gaussian and then fgs_render_ex of one frame in one call, with the same arguments and the
+ * same results in every buffer, for keys as fgs_preprocess makes them (no bits set above the sorted range).  What the blend
+ * needs to know of the tiles is written by the launches of the sort, so there are up to two launches less.
+ */
+int fgs_sort_render(int block_x, int block_y, int num_rendered, int width, int height,
+                    char* list_sorting_space, size_t sorting_size,
+                    const uint64_t* gaussian_keys_unsorted, const uint32_t* gaussian_values_unsorted,
+                    uint64_t* gaussian_keys_sorted, uint32_t* gaussian_values_sorted,
+                    const float* points_xy, const float* rgb_depth, const float* conic_opacity,
+                    int* ranges, const float bg_color[3], uint8_t* out_color_u8, float* out_color_f32,
+                    int flags, void* stream);
 
 /*
  * The two halves of fgs_render_*, for callers that want them separately (per-stage timing, or

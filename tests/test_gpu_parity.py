@@ -572,6 +572,85 @@ def test_sort_and_render_replayed_from_a_captured_graph():
         torch.cuda.synchronize()
 
 
+def _frame_for_sort_render(kind):
+    """(W, H, block, tile, depth, splats): the tile id and depth of every pair of a frame, and of how many splats they are."""
+    rng = np.random.default_rng(len(kind))
+    W, H, block, n = {"empty": (320, 200, (16, 16), 0), "one pair": (320, 200, (16, 16), 1), "one block": (256, 192, (16, 16), 900),
+                      "one block, many tiles": (1920, 1080, (16, 16), 1000), "few tiles": (256, 192, (16, 16), 4000),
+                      "one digit": (160, 160, (16, 16), 30_000), "one pass": (1280, 720, (16, 16), 200_003),
+                      "one pass, 32x16": (1599, 901, (32, 16), 300_000), "one pass, 32x32": (2560, 1440, (32, 32), 600_000),
+                      "two passes, ranked": (1920, 1080, (16, 16), (1 << 22) + 5), "unranked": (2560, 1440, (16, 16), 300_000),
+                      "long lists": (4112, 4096, (16, 16), 3_400_000), "three passes": (8208, 8192, (16, 16), 60_000)}[kind]
+    tiles = ((W + block[0] - 1) // block[0]) * ((H + block[1] - 1) // block[1])
+    tile = (tiles * rng.random(n) ** 2).astype(np.int64)
+    if kind == "long lists":
+        tile[:9000] = np.repeat([5, tiles // 2, tiles - 1], 3000)
+    elif kind == "one pair":
+        tile[:] = tiles - 2
+    else:
+        tile[: n // 8] = tiles // 3             # shared out, and sorted by several waves
+    return W, H, block, tile, rng.random(n).astype(np.float32) + 1.0, 5000
+
+
+@pytest.mark.parametrize("kind", ["empty", "one pair", "one block", "one block, many tiles", "few tiles", "one digit", "one pass", "one pass, 32x16",
+                                  "one pass, 32x32", "two passes, ranked", "unranked", "long lists", "three passes"])
+def test_sort_render_is_sort_and_then_render(kind):
+    """fgs_sort_render, whose sort writes the tile ranges, ranks the tiles and lists the long lists where it can, against fgs_sort_gaussian
+    and fgs_render_ex: the same bits in every buffer, with fp32 and f16 sums, and three times from a captured graph."""
+    import gpu_pipeline as gp
+    import torch
+    from flashgs_amd import cabi
+    W, H, (bx, by), tile, depth, P = _frame_for_sort_render(kind)
+    n, rng = tile.size, np.random.default_rng(3)
+    keys = gp.dev(((tile.astype(np.uint64) << np.uint64(32)) | depth.view(np.uint32).astype(np.uint64)).view(np.int64)) if n else gp.dev(np.zeros(1, np.int64))
+    vals = gp.dev(rng.integers(0, P, max(n, 1)).astype(np.int32))
+    xy = gp.dev((rng.random((P, 2)) * [W, H]).astype(np.float32))
+    rgb = gp.dev(rng.random((P, 4)).astype(np.float32))
+    conic = gp.dev(np.tile(np.array([-0.01, 0.0, -0.01, -3.0], np.float32), (P, 1)))
+    bg = np.array([0.2, 0.4, 0.6], np.float32)
+    gx, gy = (W + bx - 1) // bx, (H + by - 1) // by
+    size = max(cabi.get_sort_buffer_size(n), 256)
+    space = torch.empty(size, device=gp.DEV, dtype=torch.uint8)
+
+    def buffers():
+        return [torch.full((max(n, 1),), -1, device=gp.DEV, dtype=torch.int64), torch.full((max(n, 1),), -1, device=gp.DEV, dtype=torch.int32),
+                torch.full((gx * gy, 2), -7, device=gp.DEV, dtype=torch.int32), torch.zeros((H, W, 3), device=gp.DEV, dtype=torch.uint8),
+                torch.zeros((H, W, 3), device=gp.DEV, dtype=torch.float32)]
+
+    def both(b, flags):
+        st = torch.cuda.current_stream().cuda_stream
+        cabi.sort_gaussian(n, W, H, bx, by, space.data_ptr(), size, keys.data_ptr(), vals.data_ptr(), b[0].data_ptr(), b[1].data_ptr(), st)
+        cabi.render_f32(bx, by, n, W, H, xy.data_ptr(), rgb.data_ptr(), conic.data_ptr(), b[0].data_ptr(), b[1].data_ptr(), b[2].data_ptr(), bg,
+                        b[3].data_ptr(), b[4].data_ptr(), st, flags=flags)
+
+    def one(b, flags):
+        cabi.sort_render(bx, by, n, W, H, space.data_ptr(), size, keys.data_ptr(), vals.data_ptr(), b[0].data_ptr(), b[1].data_ptr(), xy.data_ptr(),
+                         rgb.data_ptr(), conic.data_ptr(), b[2].data_ptr(), bg, b[3].data_ptr(), b[4].data_ptr(),
+                         torch.cuda.current_stream().cuda_stream, flags=flags)
+
+    for flags in (cabi.BLEND_FP32, cabi.BLEND_MATRIX_F16):
+        want, got = buffers(), buffers()
+        both(want, flags)
+        for again in range(2):                  # (the tables of long lists take turns)
+            for g in got: g.zero_()
+            one(got, flags)
+            torch.cuda.synchronize()
+            for w, g in zip(want, got):
+                assert torch.equal(w, g) or n == 0 and w is want[0] or n == 0 and w is want[1]
+    graph, got, side = torch.cuda.CUDAGraph(), buffers(), torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.graph(graph, stream=side):
+        one(got, cabi.BLEND_MATRIX_F16)
+    for replay in range(3):
+        for g in got[:4]: g.fill_(1)
+        graph.replay()
+        torch.cuda.synchronize()
+        for w, g in zip(want[2:], got[2:]):
+            assert torch.equal(w, g), "replay %d" % replay
+        both(buffers(), cabi.BLEND_FP32)        # eager work in between
+        torch.cuda.synchronize()
+
+
 @pytest.mark.parametrize("block", [(16, 16), (32, 16), (32, 32)])
 def test_blends_replayed_beside_each_other(block):
     """Blends hold no table of the library's in a captured graph: graphs of two frame sizes, replayed side
