@@ -175,7 +175,7 @@ template <class Shape, class In>
 struct Digits {
     static constexpr bool kKeys = sizeof(In) == 8;
     static constexpr int kItems = Shape::kCountItems;
-    static constexpr int kWords = kKeys ? 2 * kItems : kItems * (int)sizeof(In) / 4;
+    static constexpr int kWords = kKeys ? kItems : kItems * (int)sizeof(In) / 4;     // (of keys the upper halves alone)
     uint32_t w[kWords];
 
     __device__ __forceinline__ int index(int i, int tid) const { return kKeys ? i * kSortBlock + tid : tid * kItems + i; }
@@ -186,9 +186,7 @@ struct Digits {
 #pragma unroll
             for (int i = 0; i < kItems; i++) {
                 const int idx = base + i * kSortBlock + tid;
-                const uint64_t k = idx < n ? in[idx] : 0ull;
-                w[2 * i] = (uint32_t)k;
-                w[2 * i + 1] = (uint32_t)(k >> 32);
+                w[i] = idx < n ? ((const uint32_t*)in)[2 * (size_t)idx + 1] : 0u;
             }
         } else {
             const int first = base + tid * kItems;
@@ -206,11 +204,11 @@ struct Digits {
     }
     __device__ __forceinline__ uint32_t digit(int i, int shift, uint32_t mask) const
     {
-        if constexpr (kKeys) return (w[2 * i + 1] >> shift) & mask;
+        if constexpr (kKeys) return (w[i] >> shift) & mask;
         constexpr int kPer = 4 / (sizeof(In) < 4 ? (int)sizeof(In) : 4);
         return (w[i / kPer] >> (i % kPer * (32 / kPer))) & mask;
     }
-    __device__ __forceinline__ uint32_t field(int i) const { return kKeys ? w[2 * i + 1] : 0u; }
+    __device__ __forceinline__ uint32_t field(int i) const { return kKeys ? w[i] : 0u; }
 };
 
 // The tile field of the list's first key, whose bits above the sorted range are those of every key unless marked (kMarkBeyond).
@@ -261,7 +259,9 @@ __global__ __launch_bounds__(kSortBlock) void count_kernel(const In* __restrict_
 // The same for a list of more than kMostRowWords histogram entries: one workgroup counts a whole chunk of
 // `chunk` consecutive blocks, blockDim.x / kSortBlock of them at a time, and so also has the
 // chunk's digit sums, which the offsets launch needs (a launch of their own would read the rows
-// back just to add them up).
+// back just to add them up).  The digits of the next blocks are requested before those at hand are counted: second count of 110M pairs 76 -> 66 us, of 14.3M
+// 17.4 -> 15.3, first count of 4.9M 12.8 -> 11.3.  The first count of 110M pairs stays at 205: behind preprocess, whose pairs are still on their way to memory, no
+// order of its reads changes it (on a list that rests the same change is 251 -> 189, and a plain read of the 0.87 GB 138).
 constexpr int kCountGroups = 4;
 
 template <class Shape, class In>
@@ -271,7 +271,7 @@ __global__ __launch_bounds__(kCountGroups * kSortBlock) void count_chunk_kernel(
     uint32_t above, uint32_t* __restrict__ beyond, uint32_t* __restrict__ seg_counts)
 {
     constexpr int kB = Shape::kBinsP, kPer = Shape::kPerThread;
-    __shared__ uint32_t h[kCountGroups][kB];
+    __shared__ uint32_t h[2][kCountGroups][kB];         // in turn: while the one is written out the other counts
     __shared__ uint32_t s_beyond;
     const int tid = threadIdx.x % kSortBlock, group = threadIdx.x / kSortBlock;
     const int groups = (int)blockDim.x / kSortBlock;
@@ -281,22 +281,25 @@ __global__ __launch_bounds__(kCountGroups * kSortBlock) void count_chunk_kernel(
     }
     const uint32_t mask = (1u << nbits) - 1u;
     const int t0 = blockIdx.x * chunk, t1 = min(tiles, t0 + chunk);
+    Digits<Shape, In> next = {};
+    if (t0 + group < t1) next.load(in, (t0 + group) * Shape::kTile, tid, n);
     uint32_t sum[kPer];
 #pragma unroll
-    for (int q = 0; q < kPer; q++) { sum[q] = 0; h[group][q * kSortBlock + tid] = 0; }
+    for (int q = 0; q < kPer; q++) { sum[q] = 0; h[0][group][q * kSortBlock + tid] = 0; h[1][group][q * kSortBlock + tid] = 0; }
     if (threadIdx.x == 0) s_beyond = 0;
     __syncthreads();
     uint32_t seen = 0;
     const uint32_t field_of_first = beyond ? first_field(in) : 0u;
-    for (int first = t0; first < t1; first += groups) {      // the same trips for every group
+    int turn = 0;
+    for (int first = t0; first < t1; first += groups, turn ^= 1) {      // the same trips for every group
         const int row = first + group;
+        const Digits<Shape, In> digits = next;
+        if (row + groups < t1) next.load(in, (row + groups) * Shape::kTile, tid, n);
         if (row < t1) {
             const int base = row * Shape::kTile;
-            Digits<Shape, In> digits;
-            digits.load(in, base, tid, n);
 #pragma unroll
             for (int i = 0; i < Shape::kCountItems; i++) {
-                if (base + digits.index(i, tid) < n) atomicAdd(&h[group][digits.digit(i, shift, mask)], 1u);
+                if (base + digits.index(i, tid) < n) atomicAdd(&h[turn][group][digits.digit(i, shift, mask)], 1u);
                 if (base + digits.index(i, tid) < n) seen |= digits.field(i) ^ field_of_first;
             }
         }
@@ -304,23 +307,23 @@ __global__ __launch_bounds__(kCountGroups * kSortBlock) void count_chunk_kernel(
         if (row < t1) {
 #pragma unroll
             for (int q = 0; q < kPer; q++) {
-                const uint32_t c = h[group][q * kSortBlock + tid];
-                h[group][q * kSortBlock + tid] = 0;          // read and cleared by the same thread
+                const uint32_t c = h[turn][group][q * kSortBlock + tid];
+                h[turn][group][q * kSortBlock + tid] = 0;       // read and cleared by the same thread, a barrier in front of the next counts
                 hist[(size_t)row * kB + q * kSortBlock + tid] = c;
                 sum[q] += c;
             }
         }
-        __syncthreads();
     }
+    __syncthreads();
     if (beyond && (seen & above) != 0) s_beyond = 1;
 #pragma unroll
-    for (int q = 0; q < kPer; q++) h[group][q * kSortBlock + tid] = sum[q];
+    for (int q = 0; q < kPer; q++) h[0][group][q * kSortBlock + tid] = sum[q];
     __syncthreads();
     if (group == 0) {
 #pragma unroll
         for (int q = 0; q < kPer; q++) {
             uint32_t total = 0;
-            for (int g = 0; g < groups; g++) total += h[g][q * kSortBlock + tid];
+            for (int g = 0; g < groups; g++) total += h[0][g][q * kSortBlock + tid];
             chunk_sums[(size_t)blockIdx.x * kB + q * kSortBlock + tid] = total;
         }
     }
@@ -330,9 +333,9 @@ __global__ __launch_bounds__(kCountGroups * kSortBlock) void count_chunk_kernel(
 // ---- step 2: exclusive start of every (block, digit) run ----------------------------------------
 // start[b][d] = sum of hist[*][d' < d] + sum of hist[b' < b][d]   (digit-major, then block)
 
-// One workgroup per chunk, up to 1024 / bins threads per digit (blockDim.x / bins of them): the
-// chunk sums are few and the loop over them is latency-bound, so each group of `bins` threads
-// takes every groups-th batch of 16 independent loads.
+// One workgroup per chunk.  Every one of them adds up the sums of all chunks, four digits a thread and eight rows a trip to memory: two trips for 256 chunks of
+// 256 digits and four with 512, where a digit a thread took four and eight (8K / 14.3M pairs 14.1 -> 11.3 us a launch, 110M 29.6 -> 25.4, 4K / 8M 8.1 -> 8.0).  (Sixteen rows a trip, or the chunk's own rows requested in front of the
+// sums, are no faster.)
 constexpr int kOffsetThreads = 1024;
 
 template <class Shape>
@@ -340,55 +343,58 @@ __global__ __launch_bounds__(kOffsetThreads) void offsets_kernel(uint32_t* __res
                                                                  const uint32_t* __restrict__ chunk_sums, int chunks,
                                                                  uint32_t* marks)       // of the first pass, else null
 {
-    constexpr int kB = Shape::kBinsP;
-    constexpr int kMaxGroups = kOffsetThreads / kB;
-    __shared__ uint32_t s_total[kMaxGroups][kB], s_before[kMaxGroups][kB];
+    typedef uint32_t Four __attribute__((ext_vector_type(4)));
+    constexpr int kB = Shape::kBinsP, kQuads = kB / 4, kGroups = kOffsetThreads / kQuads, kSumsAtOnce = 8, kRowsAtOnce = 16;
+    __shared__ Four s_total[kGroups][kQuads], s_before[kGroups][kQuads];
     __shared__ uint32_t s_wave[kB / kWave];
-    const int d = threadIdx.x & (kB - 1), group = threadIdx.x / kB;
-    const int lane = d & (kWave - 1), wave = d / kWave;
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
     const int mine = (int)blockIdx.x;
-    const int groups = (int)blockDim.x / kB;
     if (marks && mine == 0) {       // one word out of the count workgroups' words
         uint32_t seen = 0;
-        for (int c = (int)threadIdx.x; c < chunks; c += (int)blockDim.x) seen |= marks[kMarkBeyond + c];
+        for (int c = tid; c < chunks; c += kOffsetThreads) seen |= marks[kMarkBeyond + c];
         const int any = __syncthreads_or(seen != 0);
-        if (threadIdx.x == 0) marks[kMarkByIndex] = any ? 1u : 0u;
+        if (tid == 0) marks[kMarkByIndex] = any ? 1u : 0u;
     }
-    uint32_t total = 0, before = 0;
-    for (int c0 = group * 16; c0 < chunks; c0 += 16 * groups) {
-        uint32_t v[16];
+    {
+        const int quad = tid & (kQuads - 1), group = tid / kQuads;
+        Four total = 0, before = 0;
+        for (int c0 = group * kSumsAtOnce; c0 < chunks; c0 += kSumsAtOnce * kGroups) {
+            Four v[kSumsAtOnce];
 #pragma unroll
-        for (int j = 0; j < 16; j++) v[j] = c0 + j < chunks ? chunk_sums[(size_t)(c0 + j) * kB + d] : 0u;
+            for (int j = 0; j < kSumsAtOnce; j++) {
+                v[j] = 0;
+                if (c0 + j < chunks) v[j] = ((const Four*)chunk_sums)[(size_t)(c0 + j) * kQuads + quad];
+            }
 #pragma unroll
-        for (int j = 0; j < 16; j++) {
-            if (c0 + j < mine) before += v[j];
-            total += v[j];
+            for (int j = 0; j < kSumsAtOnce; j++) {
+                if (c0 + j < mine) before += v[j];
+                total += v[j];
+            }
         }
+        s_total[group][quad] = total;
+        s_before[group][quad] = before;
     }
-    s_total[group][d] = total;
-    s_before[group][d] = before;
     __syncthreads();
-    total = 0; before = 0;
+    uint32_t total = 0, before = 0, incl = 0;
+    if (tid < kB) {
 #pragma unroll
-    for (int g = 0; g < kMaxGroups; g++)
-        if (g < groups) { total += s_total[g][d]; before += s_before[g][d]; }
-    // exclusive scan of the digit totals over the digits (every group does the same sums)
-    uint32_t incl = wave_inclusive_sum(total);
-    if (group == 0 && lane == kWave - 1) s_wave[wave] = incl;
+        for (int g = 0; g < kGroups; g++) { total += ((const uint32_t*)s_total[g])[tid]; before += ((const uint32_t*)s_before[g])[tid]; }
+        // exclusive scan of the digit totals over the digits
+        incl = wave_inclusive_sum(total);
+        if (lane == kWave - 1) s_wave[wave] = incl;
+    }
     __syncthreads();
-    if (group != 0) return;
-    uint32_t digit_base = incl - total;
-    for (int w = 0; w < wave; w++) digit_base += s_wave[w];
-
-    uint32_t run = digit_base + before;
+    if (tid >= kB) return;
+    uint32_t run = incl - total + before;
+    for (int w = 0; w < wave; w++) run += s_wave[w];
     const int t0 = mine * chunk, t1 = min(tiles, t0 + chunk);
-    for (int tb = t0; tb < t1; tb += 16) {
-        uint32_t c[16];
+    for (int row = t0; row < t1; row += kRowsAtOnce) {
+        uint32_t c[kRowsAtOnce];
 #pragma unroll
-        for (int j = 0; j < 16; j++) c[j] = tb + j < t1 ? hist[(size_t)(tb + j) * kB + d] : 0u;
+        for (int j = 0; j < kRowsAtOnce; j++) c[j] = row + j < t1 ? hist[(size_t)(row + j) * kB + tid] : 0u;
 #pragma unroll
-        for (int j = 0; j < 16; j++) {
-            if (tb + j < t1) hist[(size_t)(tb + j) * kB + d] = run;
+        for (int j = 0; j < kRowsAtOnce; j++) {
+            if (row + j < t1) hist[(size_t)(row + j) * kB + tid] = run;
             run += c[j];
         }
     }
@@ -2247,7 +2253,7 @@ int sort_impl(int num_rendered, int width, int height, int block_x, int block_y,
                         const int groups = g.chunk < kCountGroups ? g.chunk : kCountGroups;
                         hipLaunchKernelGGL((count_chunk_kernel<Shape, In>), dim3(g.chunks), dim3(groups * kSortBlock), 0, st,
                                            in, n, shift, nbits, hist, g.tiles, g.chunk, chunk_sums, ~tile_mask, beyond, clear);
-                        hipLaunchKernelGGL((offsets_kernel<Shape>), dim3(g.chunks), dim3(g.chunks > 16 ? kOffsetThreads : Shape::kBinsP), 0, st,
+                        hipLaunchKernelGGL((offsets_kernel<Shape>), dim3(g.chunks), dim3(kOffsetThreads), 0, st,
                                            hist, g.tiles, g.chunk, chunk_sums, g.chunks, first ? marks : nullptr);
                     }
                 };

@@ -1715,6 +1715,19 @@ def test_sort_around_the_list_lengths_where_the_partition_blocks_change(n, W, H)
     _sort_case(tile, depth, W, H, seed=n % 89, ascending=n % 2 == 0)
 
 
+@pytest.mark.parametrize("W,H,n", [(3840, 2160, 257 * 2048 - 5), (3840, 2160, (1 << 21) + 1), (3840, 2160, 1025 * 4096 + 1),
+                                   (3840, 2160, 4353 * 4096 - 4095), (7680, 4320, 129 * 4096 - 7), (7680, 4320, 257 * 4096 + 1),
+                                   (7680, 4320, 1281 * 4096)])
+def test_sort_around_the_blocks_that_a_count_workgroup_takes(W, H, n):
+    """Chunks of 1, 2, 3, 5, 6 and 18 blocks: fewer than a workgroup counts at a time, as many, a last trip and a last chunk with some of them, and more rows
+    than a trip of the offsets launch; digits of 8 and of 9 bits, half of the pairs in a corner of the frame."""
+    rng = np.random.default_rng(n % 1009)
+    tiles = ((W + 15) // 16) * ((H + 15) // 16)
+    tile = rng.integers(0, tiles, n)
+    tile[n // 2:] %= tiles // 16
+    _sort_case(tile.astype(np.uint32), rng.integers(0, 1 << 31, n, dtype=np.uint64).astype(np.uint32), W, H, None, seed=n % 89)
+
+
 @pytest.mark.parametrize("W,H,n", [(256, 255, 5000), (512, 254, 2048), (512, 254, 2049), (1000, 400, 1025), (1000, 400, 4097), (1280, 720, 150_001),
                                    (1920, 1080, 3000), (1920, 1080, 300_000), (1920, 1080, (1 << 19) - 1), (1920, 1080, (1 << 19) + 1),
                                    (1280, 720, 1_300_003), (1920, 1080, 1 << 22), (1920, 1080, (1 << 22) + 1), (2048, 1024, 100_000)])
