@@ -99,7 +99,7 @@ class Rasterizer:
     def __init__(self, scene, MAX_NUM_RENDERED, MAX_NUM_TILES, tile=(16, 16), max_width=0, max_height=0):
         dev = scene.device
         self.tile = tuple(tile)
-        self._sort_render = getattr(ops(), "sort_" + self.RENDER[self.tile])
+        self._frame = getattr(ops(), self.RENDER[self.tile].replace("render", "frame"))
         self.gaussian_keys_unsorted = torch.zeros(MAX_NUM_RENDERED, device=dev, dtype=torch.int64)
         self.gaussian_values_unsorted = torch.zeros(MAX_NUM_RENDERED, device=dev, dtype=torch.int32)
         self.gaussian_keys_sorted = torch.zeros(MAX_NUM_RENDERED, device=dev, dtype=torch.int64)
@@ -119,8 +119,9 @@ class Rasterizer:
         self.rgb_depth = torch.zeros((scene.num_vertex, 4), device=dev, dtype=torch.float32)
         self.conic_opacity = torch.zeros((scene.num_vertex, 4), device=dev, dtype=torch.float32)
         # the launch stores the pair count here as soon as it has it; forward polls this word
-        # instead of the blocking device-to-host copy of example.py:79
+        # instead of the blocking device-to-host copy of example.py:79 (_count_seen: the same memory)
         self._count = torch.zeros(1, dtype=torch.int32, pin_memory=True)
+        self._count_seen = self._count.numpy()
         self._out = None
         if max_width and max_height:
             self._out = torch.zeros((max_height, max_width, 3), device=dev, dtype=torch.uint8)
@@ -139,22 +140,18 @@ class Rasterizer:
     def curr_offset(self, word):
         self._curr_offset = word
 
-    def _preprocess(self, scene, camera):
-        bx, by = self.tile
-        arguments = (scene.position, scene.shs, scene.opacity, scene.cov3d, camera.width, camera.height, bx, by,
-                     camera.position, camera.rotation, camera.focal_x, camera.focal_y, camera.zFar, camera.zNear,
-                     self.points_xy, self.rgb_depth, self.conic_opacity,
-                     self.gaussian_keys_unsorted, self.gaussian_values_unsorted)
+    def _words(self):
+        """The word that a frame counts its pairs in, zero by the time its preprocess runs, and the one that it leaves zero for the
+        next frame (or None)."""
         cleared, self._cleared = self._cleared, False
         if self._curr_offset is not None:
             self._curr_offset.zero_()
-            ops().preprocess_mirrored(*arguments, self._curr_offset, self._count)
-            return
+            return self._curr_offset, None
         if cleared:
             self._turn ^= 1
         else:
             self._offsets[self._turn].zero_()
-        ops().preprocess_chained(*arguments, self._offsets[self._turn], self._count, self._offsets[self._turn ^ 1])
+        return self._offsets[self._turn], self._offsets[self._turn ^ 1]
 
     def _image(self, camera, device):
         if self._out is None or self._out.shape[0] != camera.height or self._out.shape[1] != camera.width:
@@ -169,17 +166,22 @@ class Rasterizer:
         tiles = ((camera.width + bx - 1) // bx) * ((camera.height + by - 1) // by)
         if tiles > self.MAX_NUM_TILES:
             raise ValueError("image needs %d tiles, MAX_NUM_TILES is %d" % (tiles, self.MAX_NUM_TILES))
-        if self.num_rendered >= 0 and int(self._count[0]) < 0:
+        if self.num_rendered >= 0 and self._count_seen[0] < 0:
             # the count of the last frame was good when it arrived, and a wait of one workgroup gave up after that
             self.num_rendered = -1
             o.reset_scan(self._offsets[0])
             raise ScanGaveUp("a workgroup of the previous frame's preprocess gave up waiting after the pair count "
                              "had been reported; that frame's image is not to be used")
+        out_color = self._image(camera, scene.device) if out is None else out
         for attempt in range(2):
-            self._preprocess(scene, camera)
-            # the count arrives while the launch is still writing keys; the sort below is enqueued
-            # behind it on the same stream
-            num_rendered = o.wait_count(self._count, 60.0)
+            offset, next_offset = self._words()
+            # the count arrives while the launch is still writing keys; the sort is enqueued behind it on the same stream
+            num_rendered = self._frame(scene.position, scene.shs, scene.opacity, scene.cov3d, camera.width, camera.height,
+                                       camera.position, camera.rotation, camera.focal_x, camera.focal_y, camera.zFar, camera.zNear,
+                                       self.points_xy, self.rgb_depth, self.conic_opacity,
+                                       self.gaussian_keys_unsorted, self.gaussian_values_unsorted, offset, self._count, next_offset,
+                                       60.0, self.MAX_NUM_RENDERED, self.list_sorting_space,
+                                       self.gaussian_keys_sorted, self.gaussian_values_sorted, self.ranges, bg_color, out_color)
             if num_rendered >= 0:
                 self._cleared = self._curr_offset is None
                 break
@@ -191,11 +193,6 @@ class Rasterizer:
                              "(fgs_set_scan_spin_limit polls); the frame was not rendered")
         if num_rendered >= self.MAX_NUM_RENDERED:
             raise TooManyPairs("Too many k-v pairs! (%d, capacity %d)" % (num_rendered, self.MAX_NUM_RENDERED))
-        out_color = self._image(camera, scene.device) if out is None else out
-        self._sort_render(num_rendered, camera.width, camera.height, self.list_sorting_space,
-                          self.gaussian_keys_unsorted, self.gaussian_values_unsorted,
-                          self.gaussian_keys_sorted, self.gaussian_values_sorted,
-                          self.points_xy, self.rgb_depth, self.conic_opacity, self.ranges, bg_color, out_color)
         return out_color
 
 

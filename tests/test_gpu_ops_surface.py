@@ -192,6 +192,51 @@ def test_the_next_offset_is_cleared_whatever_the_count():
         image = no_rast.forward(none, cam, torch.zeros(3))
 
 
+@pytest.mark.parametrize("tile", [(16, 16), (32, 16), (32, 32)])
+def test_a_frame_in_one_call_is_the_operators_one_by_one(tile):
+    """forward against preprocess, sort_gaussian and render on buffers of their own; an image that is refused leaves no count pending, too many pairs
+    are reported, and the next frame is whole either way."""
+    import flash_gaussian_splatting as fgs
+    from flashgs_amd.rasterizer import TooManyPairs
+    sc, scene, cam, _ = _setup(n=5000)
+    rast, apart = (Rasterizer(scene, 1 << 20, 1 << 14, tile=tile) for _ in range(2))
+    bg = torch.tensor([0.1, 0.2, 0.3])
+    fgs.ops.preprocess(scene.position, scene.shs, scene.opacity, scene.cov3d, cam.width, cam.height, *tile,
+                       cam.position, cam.rotation, cam.focal_x, cam.focal_y, cam.zFar, cam.zNear,
+                       apart.points_xy, apart.rgb_depth, apart.conic_opacity,
+                       apart.gaussian_keys_unsorted, apart.gaussian_values_unsorted, apart.curr_offset)
+    n = int(apart.curr_offset.cpu()[0])
+    fgs.ops.sort_gaussian(n, cam.width, cam.height, *tile, apart.list_sorting_space, apart.gaussian_keys_unsorted, apart.gaussian_values_unsorted,
+                          apart.gaussian_keys_sorted, apart.gaussian_values_sorted)
+    expected = torch.zeros((cam.height, cam.width, 3), device="cuda:0", dtype=torch.uint8)
+    getattr(fgs.ops, "render_%dx%d" % tile)(n, cam.width, cam.height, apart.points_xy, apart.rgb_depth, apart.conic_opacity,
+                                            apart.gaussian_keys_sorted, apart.gaussian_values_sorted, apart.ranges, bg, expected)
+    tiles = -(-cam.width // tile[0]) * -(-cam.height // tile[1])
+
+    def whole():
+        image = rast.forward(scene, cam, bg)
+        assert rast.num_rendered == n and torch.equal(image, expected)
+        for name in ("points_xy", "rgb_depth", "conic_opacity"):
+            assert torch.equal(getattr(rast, name), getattr(apart, name))
+        assert torch.equal(rast.gaussian_keys_sorted[:n], apart.gaussian_keys_sorted[:n])
+        assert torch.equal(rast.gaussian_values_sorted[:n], apart.gaussian_values_sorted[:n])
+        assert torch.equal(rast.ranges[:tiles], apart.ranges[:tiles])
+
+    whole()
+    for bad in (expected[:-1], expected.cpu(), expected[:, :, :2], expected.float()):
+        with pytest.raises(RuntimeError, match="out_color"):
+            rast.forward(scene, cam, bg, out=bad)
+        whole()
+    with pytest.raises(RuntimeError, match="bg_color"):
+        rast.forward(scene, cam, bg[:2])
+    whole()
+    rast.MAX_NUM_RENDERED = n
+    with pytest.raises(TooManyPairs, match="%d" % n):
+        rast.forward(scene, cam, bg)
+    rast.MAX_NUM_RENDERED = n + 1
+    whole()
+
+
 def _write_ply(path, recs):
     props = ["x", "y", "z", "nx", "ny", "nz"] + ["f_dc_%d" % i for i in range(3)] + ["f_rest_%d" % i for i in range(45)] \
         + ["opacity"] + ["scale_%d" % i for i in range(3)] + ["rot_%d" % i for i in range(4)]
