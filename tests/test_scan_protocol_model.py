@@ -36,7 +36,7 @@ class Words:
         self.offsets = [[0] * self.capacity for _ in range(2)]
 
 
-def workgroup(words, out, ticket, num_blocks, key_count, spin_limit, grid_threads):
+def workgroup(words, out, ticket, num_blocks, key_count, spin_limit):
     """One workgroup of the launch as a generator: yields at every access to a shared word."""
     control = words.control
     yield
@@ -46,10 +46,6 @@ def workgroup(words, out, ticket, num_blocks, key_count, spin_limit, grid_thread
         return
     which = control & GENERATION
     other = which ^ 1
-    # strided share of the clear of the other generation
-    for w in range(ticket + 1, 2 * words.capacity, grid_threads):
-        (words.counts[other] if w < words.capacity else words.offsets[other])[w % words.capacity] = 0
-        yield
     if ticket < 0:                                   # the scanner (workgroup 0 of the grid)
         start = out["curr"]
         yield
@@ -81,6 +77,10 @@ def workgroup(words, out, ticket, num_blocks, key_count, spin_limit, grid_thread
         return
     words.counts[which][ticket] = (COUNT, key_count)
     yield
+    # strided share of the clear of the other generation
+    for w in range(ticket, 2 * words.capacity, num_blocks):
+        (words.counts[other] if w < words.capacity else words.offsets[other])[w % words.capacity] = 0
+        yield
     spins = 0
     while True:
         word = words.offsets[which][ticket]
@@ -101,7 +101,7 @@ def launch(words, key_counts, residency, spin_limit, rng, start=0, slow_first=0)
     workgroup but the scanner may move (a scanner that polls while nobody has published)."""
     num_blocks = len(key_counts)
     out = dict(curr=start, slots={}, touched=set(range(num_blocks)))
-    todo = [workgroup(words, out, t, num_blocks, key_counts[t] if t >= 0 else 0, spin_limit, num_blocks + 1)
+    todo = [workgroup(words, out, t, num_blocks, key_counts[t] if t >= 0 else 0, spin_limit)
             for t in range(-1, num_blocks)]
     resident, nxt, burnt = [], 0, 0
     while resident or nxt < len(todo):
