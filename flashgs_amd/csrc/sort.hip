@@ -1035,7 +1035,11 @@ __global__ __launch_bounds__(kOnePassThreads) void tile_scatter_kernel(const uin
 constexpr int kCapTiny = 512, kCapSmall = 1024, kCapMedium = 4096, kCapLarge = 8192;
 constexpr int kMergedLargeMax = 1 << 24;     // up to this many pairs the last launch also takes the class of 4097 .. 8192 pairs
 constexpr int kManyPairs = 1 << 26;
-constexpr int kMergedTailMax = 1 << 19;      // up to this many pairs the last launch also takes the classes of 1025 .. 8192 pairs
+// Up to kMergedTailMax pairs the last launch also takes the classes of 1025 .. 8192 pairs, and up to kMergedTailSpread where a tile has at most kMergedTailEach on
+// average.  Sort, merged and not: 1M pairs of 3600 tiles, crowded, 68.5 and 82.3 us, of 8160 tiles, spread evenly, 39.7 and 41.4, 0.6M of 8160, crowded,
+// 169.5 and 178, the frame of 1599x901 in 32x16 tiles 174.6 and 180.5; 1M pairs of 704 tiles, nearly all of them in these classes, 51 and 42.  Up to 2^21: 1.5M pairs of 3600
+// tiles of 32x32 pixels 446 and 438.
+constexpr int kMergedTailMax = 1 << 19, kMergedTailSpread = 1 << 20, kMergedTailEach = 512;
 
 // First index in [0, n) whose tile field is >= v (n if none), found by the whole wave probing 64
 // evenly spaced positions per step.  `keys` is ordered by tile field.  All lanes return the same.
@@ -2361,7 +2365,7 @@ int sort_impl(int num_rendered, int width, int height, int block_x, int block_y,
                        (const uint32_t*)list_medium, cap_medium, (const uint32_t*)list_large, cap_large, FIRST, ranks)
     // A short list of pairs has few segments of more than 1024 pairs, or none: there the one
     // launch below takes those classes too (720p, 0.2M pairs: two launches less).
-    const bool merged_tail = seg_start && n <= kMergedTailMax;
+    const bool merged_tail = seg_start && (n <= kMergedTailMax || (n <= kMergedTailSpread && n <= kMergedTailEach * tiles_xy));
     // On a long list a wave takes several tile ids (a grid apart): its successor would start some 3 us after its end.  The segments of up
     // to 1024 pairs with 1, 2, 4 and 8 ids a wave: 110M pairs of an 8K frame 279, 256, 232, 224 us, 29M 113, 107, 109, 118, 36M of a 4K frame
     // 93, 76, 85, 103; below, the last waves' second segments count for more: 14.5M 82, 77, 80, 8M 34.7, 39.7, 41.1.

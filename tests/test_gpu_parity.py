@@ -1715,6 +1715,21 @@ def test_sort_around_the_list_lengths_where_the_partition_blocks_change(n, W, H)
     _sort_case(tile, depth, W, H, seed=n % 89, ascending=n % 2 == 0)
 
 
+@pytest.mark.parametrize("W,H,n", [(1024, 512, 1 << 20), (1024, 512, (1 << 20) + 1), (1008, 512, 1 << 20), (512, 512, (1 << 19) + 1),
+                                   (528, 512, (1 << 19) + 1), (528, 512, 540_672), (528, 512, 540_673), (16400, 16400, 600_000)])
+def test_sort_around_the_averages_where_the_last_launch_takes_every_class(W, H, n):
+    """512 pairs a tile and one more, 2^20 pairs and one more, on either side of 2^19; a frame of more tiles than carries words: segments of every class."""
+    rng = np.random.default_rng(n % 997 + W)
+    tiles = ((W + 15) // 16) * ((H + 15) // 16)
+    tile = rng.integers(0, tiles, n)
+    at = 0
+    for t, length in ((3, 1024), (5, 1025), (7, 4096), (11, 4097), (tiles // 2, 8192), (tiles // 2 + 1, 8193), (tiles - 2, 16384), (tiles - 1, 16385)):
+        tile[tile == t] = 0
+        tile[at:at + length] = t
+        at += length
+    _sort_case(rng.permutation(tile).astype(np.uint32), rng.integers(0, 1 << 31, n, dtype=np.uint64).astype(np.uint32), W, H, None, seed=n % 83)
+
+
 @pytest.mark.parametrize("W,H,n", [(3840, 2160, 257 * 2048 - 5), (3840, 2160, (1 << 21) + 1), (3840, 2160, 1025 * 4096 + 1),
                                    (3840, 2160, 4353 * 4096 - 4095), (7680, 4320, 129 * 4096 - 7), (7680, 4320, 257 * 4096 + 1),
                                    (7680, 4320, 1281 * 4096)])
