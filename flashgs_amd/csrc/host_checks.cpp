@@ -136,6 +136,24 @@ void check_arguments()
     refused(fgs_sort_render(16, 32, 5, 64, 64, ws, 1 << 20, k, v, k, v, f, f, f, i32, bg, u8, nullptr, 0, nullptr), "tile shape in sort_render");
     refused(fgs_sort_render(16, 16, 5, 64, 64, ws, 1 << 20, k, v, k, v, f, f, f, i32, bg, u8, nullptr, 7, nullptr), "flags in sort_render");
     expect(fgs_sort_render(16, 16, 100000, 64, 64, ws, 1000, k, v, k, v, f, f, f, i32, bg, u8, nullptr, 0, nullptr) < 0, "workspace too small in sort_render");
+    for (int pairs : {100000, 14000000}) {           // (a frame that is ranked and one that lists its long lists, were it taken)
+        const int w = pairs > 100000 ? 7680 : 1920, h = pairs > 100000 ? 4320 : 1080;
+        const size_t room = fgs_get_sort_buffer_size(pairs);
+        auto sort_render = [&](char* space, size_t size, uint64_t* ku, uint32_t* vu, uint64_t* ks, uint32_t* vs) {
+            return fgs_sort_render(16, 16, pairs, w, h, space, size, ku, vu, ks, vs, f, f, f, i32, bg, u8, nullptr, 0, nullptr);
+        };
+        expect(sort_render(ws, room - 1, k, v, k, v) == FGS_E_WORKSPACE, "a workspace one byte short in sort_render");
+        refused(sort_render(nullptr, room, k, v, k, v), "null workspace in sort_render");
+        refused(sort_render(ws + 8, room, k, v, k, v), "misaligned workspace in sort_render");
+        refused(sort_render(ws, room, nullptr, v, k, v), "null unsorted keys in sort_render");
+        refused(sort_render(ws, room, k, nullptr, k, v), "null unsorted values in sort_render");
+        refused(sort_render(ws, room, k, v, nullptr, v), "null sorted keys in sort_render");
+        refused(sort_render(ws, room, k, v, k, nullptr), "null sorted values in sort_render");
+        refused(sort_render(ws, room, (uint64_t*)(ws + 4), v, k, v), "misaligned unsorted keys in sort_render");
+        refused(sort_render(ws, room, k, v, (uint64_t*)(ws + 4), v), "misaligned sorted keys in sort_render");
+    }
+    refused(fgs_sort_render(16, 16, 1 << 30, 64, 64, ws, (size_t)1 << 40, k, v, k, v, f, f, f, i32, bg, u8, nullptr, 0, nullptr),
+            "pair count beyond FGS_MAX_RENDERED in sort_render");
     refused(fgs_render_16x16(-1, 64, 64, f, f, f, k, v, i32, bg, u8, nullptr), "negative pair count in render");
     refused(fgs_render_16x16(5, 64, 64, nullptr, f, f, k, v, i32, bg, u8, nullptr), "null attributes in render");
     refused(fgs_render_32x16(0, 64, 64, f, f, f, k, v, i32, bg, nullptr, nullptr), "null image");

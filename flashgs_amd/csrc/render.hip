@@ -1500,6 +1500,10 @@ int sort_render_impl(int block_x, int block_y, int num_rendered, int width, int 
     int rc = check_blend(block_x, block_y, width, height, points_xy, rgb_depth, conic_opacity, ranges, bg, out_u8, out_f32, flags, &sx, &sy, &mode, who);
     if (rc != FGS_OK) return rc;
     if (num_rendered > 0 && (!points_xy || !rgb_depth || !conic_opacity)) return fail(FGS_E_INVALID, "%s: null buffer", who);
+    // A call that is refused has asked the runtime for nothing and used up no turn of the tables.
+    rc = check_sort(num_rendered, width, height, block_x, block_y, list_sorting_space, sorting_size, keys_unsorted, values_unsorted,
+                    keys_sorted, values_sorted, who);
+    if (rc != FGS_OK) return rc;
     const int tiles_x = (width + block_x - 1) / block_x, tiles_y = (height + block_y - 1) / block_y, num_tiles = tiles_x * tiles_y;
     LongTable longer;
     std::unique_lock<std::mutex> enqueue, ranking;      // from the launch that writes a table to the blend that reads it

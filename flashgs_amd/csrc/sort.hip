@@ -156,6 +156,11 @@ Workspace workspace_for(int n)
     return w;
 }
 
+long long tiles_of(int width, int height, int block_x, int block_y)
+{
+    return (long long)((width + block_x - 1) / block_x) * ((height + block_y - 1) / block_y);
+}
+
 // What a partition pass reads and writes.
 enum class Form {
     kPairs,         // keys and values as the caller has them
@@ -2161,12 +2166,10 @@ extern "C" size_t fgs_get_sort_buffer_size(int num_rendered)
 
 namespace fgs {
 
-int sort_impl(int num_rendered, int width, int height, int block_x, int block_y, char* list_sorting_space, size_t sorting_size,
-              const uint64_t* gaussian_keys_unsorted, const uint32_t* gaussian_values_unsorted,
-              uint64_t* gaussian_keys_sorted, uint32_t* gaussian_values_sorted, FrameTables* frame, void* stream, const char* who)
+int check_sort(int num_rendered, int width, int height, int block_x, int block_y, const char* list_sorting_space, size_t sorting_size,
+               const uint64_t* gaussian_keys_unsorted, const uint32_t* gaussian_values_unsorted,
+               const uint64_t* gaussian_keys_sorted, const uint32_t* gaussian_values_sorted, const char* who)
 {
-    FrameTables tables = {};
-    if (frame) std::swap(tables, *frame);           // what is written comes back
     if (num_rendered < 0)
         return fail(FGS_E_INVALID, "%s: num_rendered = %d is negative "
                                    "(a negative count is what a failed preprocess leaves behind)", who, num_rendered);
@@ -2182,15 +2185,27 @@ int sort_impl(int num_rendered, int width, int height, int block_x, int block_y,
         return fail(FGS_E_INVALID, "%s: list_sorting_space must be 256-byte aligned", who);
     if (((uintptr_t)gaussian_keys_unsorted | (uintptr_t)gaussian_keys_sorted) % 8 != 0)
         return fail(FGS_E_INVALID, "%s: key buffers must be 8-byte aligned", who);
+    const size_t needed = workspace_for(num_rendered).total;
+    if (sorting_size < needed)
+        return fail(FGS_E_WORKSPACE, "%s: list_sorting_space holds %zu bytes, %zu needed for %d pairs",
+                    who, sorting_size, needed, num_rendered);
+    if (tiles_of(width, height, block_x, block_y) >= (1LL << 30)) return fail(FGS_E_INVALID, "%s: too many tiles", who);
+    return FGS_OK;
+}
+
+int sort_impl(int num_rendered, int width, int height, int block_x, int block_y, char* list_sorting_space, size_t sorting_size,
+              const uint64_t* gaussian_keys_unsorted, const uint32_t* gaussian_values_unsorted,
+              uint64_t* gaussian_keys_sorted, uint32_t* gaussian_values_sorted, FrameTables* frame, void* stream, const char* who)
+{
+    FrameTables tables = {};
+    if (frame) std::swap(tables, *frame);           // what is written comes back
+    int rc = check_sort(num_rendered, width, height, block_x, block_y, list_sorting_space, sorting_size, gaussian_keys_unsorted,
+                        gaussian_values_unsorted, gaussian_keys_sorted, gaussian_values_sorted, who);
+    if (rc != FGS_OK || num_rendered == 0) return rc;
 
     const int n = num_rendered;
     const Workspace ws = workspace_for(n);
-    if (sorting_size < ws.total)
-        return fail(FGS_E_WORKSPACE, "%s: list_sorting_space holds %zu bytes, %zu needed for %d pairs",
-                    who, sorting_size, ws.total, n);
-
-    const long long tiles_xy = (long long)((width + block_x - 1) / block_x) * ((height + block_y - 1) / block_y);
-    if (tiles_xy >= (1LL << 30)) return fail(FGS_E_INVALID, "%s: too many tiles", who);
+    const long long tiles_xy = tiles_of(width, height, block_x, block_y);
     const int tile_bits = bit_length((uint32_t)tiles_xy);         // sort.cu:34-39: bits [0, 32 + tile_bits)
     const uint32_t tile_mask = (1u << tile_bits) - 1u;
 
