@@ -52,7 +52,7 @@ __global__ __launch_bounds__(256) void fill_i32_kernel(int* p, size_t n, int v)
 struct OrderTable {
     std::mutex enqueue;
     uint32_t* ranks = nullptr;          // kOrderCap + 2 words, then two LongLists
-    int turn = 0;                       // which of those the next large frame uses
+    int turn = 0;                       // which of those the next large frame uses: cleared by the last blend that was enqueued
 };
 std::map<StreamKey, OrderTable> g_order_tables;      // (entries stay where they are)
 std::mutex g_order_mutex;
@@ -1296,6 +1296,7 @@ struct LongTable {
     LongLists *list = nullptr, *next = nullptr;
     int least = 0;
     int per_shard = kLongPerShard / 2;
+    OrderTable* taken_from = nullptr;       // whose turn ends when a blend that clears `next` is enqueued
 };
 
 // A list is long for its frame if it has a seventh of the entries that a SIMD has on average: it takes 166 ns per entry beside others
@@ -1322,7 +1323,7 @@ int long_table(hipStream_t stream, int num_rendered, int block_x, int block_y, i
     LongLists* const both = (LongLists*)(ranks + kOrderCap + 2);
     out->list = both + entry->turn;
     out->next = both + (entry->turn ^ 1);
-    entry->turn ^= 1;
+    out->taken_from = entry;
     out->least = (int)std::max(seventh, (long long)kLongLeast);
     return FGS_OK;
 }
@@ -1432,7 +1433,9 @@ int blend_impl(bool rank, uint32_t* ranked, const LongTable& longer, int block_x
         if (sx == 1 && sy == 1) launch(fp32 ? blend_kernel<1, 1, true> : blend_kernel<1, 1, false>);
         else if (sx == 2 && sy == 1) launch(fp32 ? blend_kernel<2, 1, true> : blend_kernel<2, 1, false>);
         else launch(fp32 ? blend_kernel<2, 2, true> : blend_kernel<2, 2, false>);
-        return check_hip(hipGetLastError(), who);
+        rc = check_hip(hipGetLastError(), who);
+        if (rc == FGS_OK && longer.taken_from) longer.taken_from->turn ^= 1;
+        return rc;
     }
     SharedGrid grid;
     rc = shared_grid(sx, sy, num_tiles, fp32, &grid);
@@ -1470,18 +1473,14 @@ int render_impl(int block_x, int block_y, int num_rendered, int width, int heigh
                 int* ranges, const float bg[3], uint8_t* out_u8, float* out_f32, int flags, void* stream, const char* who)
 {
     int sx = 0, sy = 0, mode = 0;
-    int rc = check_tile(block_x, block_y, &sx, &sy, who);
-    if (rc != FGS_OK) return rc;
-    rc = colour_mode(flags, &mode, who);        // before anything is launched
-    if (rc != FGS_OK) return rc;
+    int rc = check_blend(block_x, block_y, width, height, points_xy, rgb_depth, conic_opacity, ranges, bg, out_u8, out_f32, flags, &sx, &sy, &mode, who);
+    if (rc != FGS_OK) return rc;                // before anything is launched
     if (num_rendered > 0 && (!points_xy || !rgb_depth || !conic_opacity || !keys_sorted || !values_sorted))
         return fail(FGS_E_INVALID, "%s: null buffer", who);
     LongTable longer;
     std::unique_lock<std::mutex> enqueue;       // from the launch that lists them to the blend that reads the table
-    if (width > 0 && height > 0) {
-        rc = long_table((hipStream_t)stream, num_rendered, block_x, block_y, width, height, &longer, &enqueue);
-        if (rc != FGS_OK) return rc;
-    }
+    rc = long_table((hipStream_t)stream, num_rendered, block_x, block_y, width, height, &longer, &enqueue);
+    if (rc != FGS_OK) return rc;
     rc = ranges_impl(block_x, block_y, num_rendered, width, height, keys_sorted, ranges, longer, stream, who);
     if (rc != FGS_OK) return rc;
     return blend_impl(false, nullptr, longer, block_x, block_y, width, height, points_xy, rgb_depth, conic_opacity, values_sorted, ranges,
@@ -1500,7 +1499,7 @@ int sort_render_impl(int block_x, int block_y, int num_rendered, int width, int 
     int rc = check_blend(block_x, block_y, width, height, points_xy, rgb_depth, conic_opacity, ranges, bg, out_u8, out_f32, flags, &sx, &sy, &mode, who);
     if (rc != FGS_OK) return rc;
     if (num_rendered > 0 && (!points_xy || !rgb_depth || !conic_opacity)) return fail(FGS_E_INVALID, "%s: null buffer", who);
-    // A call that is refused has asked the runtime for nothing and used up no turn of the tables.
+    // (a call that is refused has asked the runtime for nothing)
     rc = check_sort(num_rendered, width, height, block_x, block_y, list_sorting_space, sorting_size, keys_unsorted, values_unsorted,
                     keys_sorted, values_sorted, who);
     if (rc != FGS_OK) return rc;

@@ -48,7 +48,7 @@ void __hipRegisterFunction(void **module, const void *function, char *host, cons
 
 int hipGetDevice(int *device) { asked++; *device = 0; return 0; }
 int hipDeviceGetAttribute(int *value, int attribute, int device) { (void)attribute; (void)device; asked++; *value = 256; return 0; }
-int hipGetLastError(void) { if (failing > 0) { failing--; return 1; } return 0; }
+int hipGetLastError(void) { const int failed = failing; failing = 0; return failed; }
 const char *hipGetErrorString(int error) { (void)error; return "made to fail"; }
 int hipMalloc(void **p, size_t bytes) { asked++; *p = no_memory ? NULL : malloc(bytes); return *p ? 0 : 2; }
 int hipGetSymbolAddress(void **p, const void *symbol) { *p = (void *)symbol; return 0; }
@@ -73,6 +73,7 @@ int hipLaunchKernel(const void *function, dim3 grid, dim3 block, void **args, si
     (void)grid; (void)block; (void)lds;
     const char *name = "";
     for (int i = 0; i < kernel_count; i++) if (kernels[i].function == function) name = kernels[i].name;
+    if (failing) return 1;
     Launch l = { 0, (size_t)stream, 0, 0, 0 };
     if (strstr(name, "tile_scatter_kernel")) {                  /* (TileRanking) */
         l.kind = kRanks; l.table = *(size_t *)args[9];
@@ -98,7 +99,7 @@ int hipLaunchKernel(const void *function, dim3 grid, dim3 block, void **args, si
 }
 
 void stand_in_set(int is_capturing, int is_out_of_memory) { capturing = is_capturing; no_memory = is_out_of_memory; }
-void stand_in_fail(int times) { failing = times; }
+void stand_in_fail(void) { failing = 1; }
 int stand_in_asked(void) { const int n = asked; asked = 0; return n; }
 int stand_in_launches(Launch *out)
 {
@@ -133,11 +134,11 @@ def frames(mine, calls):
     for how, bx, by, w, h, pairs, ranges, stream in calls:
         hip.stand_in_asked()
         room = lib.fgs_get_sort_buffer_size(pairs)
-        if how == "render" or how == "render fails":
-            if how == "render fails": hip.stand_in_fail(1)
-            rc = lib.fgs_render_f32(bx, by, pairs, w, h, 256, 256, 256, 256, 256, ranges, C.addressof(bg), 256, None, stream)
+        if how.endswith("fails"): hip.stand_in_fail()             # up to the first time that the library looks
+        if how.startswith("render"):
+            rc = lib.fgs_render_f32(bx, by, pairs, w, h, 256, 256, 256, 256 + 4 * (how == "render misaligned keys"), 256, ranges, C.addressof(bg),
+                                    None if how == "render without image" else 256, None, stream)
         else:
-            if how == "sort fails": hip.stand_in_fail(1)
             space = {"misaligned": 256 + 8, "no space": None}.get(how, 256)
             rc = lib.fgs_sort_render(bx, by, pairs, w, h, space, room - (how == "short of room"), 256, 256, None if how == "no keys" else 256, 256,
                                      256, 256, 256, ranges, C.addressof(bg), 256, None, 0, stream)
@@ -202,3 +203,14 @@ def test_a_refused_call_asks_the_runtime_for_nothing(runtime, how, frame):
     if frame is LONG:
         assert [l["kind"] for l in launches] == [LISTS, BLENDS] * 3
         check_turns(launches)
+
+
+@pytest.mark.parametrize("how, code", [("render without image", cabi.FGS_E_INVALID), ("render misaligned keys", cabi.FGS_E_INVALID),
+                                       ("render fails", cabi.FGS_E_HIP), ("sort_render fails", cabi.FGS_E_HIP)])
+def test_a_frame_without_a_blend_uses_up_no_turn(runtime, how, code):
+    """Refused, or ended by an error before its blend: nothing of it is enqueued, and the next frame lists in the table that was cleared last."""
+    calls = [["sort_render", *LONG, A, 0x70], [how, *LONG, B, 0x70], ["render", *LONG, A, 0x70], [how, *LONG, B, 0x70], ["sort_render", *LONG, A, 0x70]]
+    results, launches = enqueued(runtime, [calls])
+    assert [r for r, _ in results[0]] == [0, code, 0, code, 0]
+    assert [l["kind"] for l in launches] == [LISTS, BLENDS] * 3
+    check_turns(launches)
