@@ -214,3 +214,56 @@ def test_a_frame_without_a_blend_uses_up_no_turn(runtime, how, code):
     assert [r for r, _ in results[0]] == [0, code, 0, code, 0]
     assert [l["kind"] for l in launches] == [LISTS, BLENDS] * 3
     check_turns(launches)
+
+
+RANKED = [16, 16, 1920, 1080]                           # ranked: by the scatter, by the last launch of the sort, or by a launch of its own
+PAIRS = {"by the scatter": 200_000, "by the last launch": 5_000_000, "by itself": 1000}
+
+
+def check_tables(launches):
+    """The last launch that wrote a blend's table belongs to the blend's own frame.  Frames of one thread have one address of ranges; a ranking that
+    the sort makes knows none, but a frame's launches stand together."""
+    ranked = {}
+    for l in launches:
+        if l["kind"] == RANKS:
+            assert l["table"] not in ranked, "another frame's ranking between a ranking and the blend that reads it"
+            ranked[l["table"]] = l["ranges"]
+        else:
+            assert l["kind"] == BLENDS and l["table"] in ranked
+            assert ranked.pop(l["table"]) in (0, l["ranges"])
+    assert not ranked
+
+
+@pytest.mark.parametrize("first", sorted(PAIRS))
+@pytest.mark.parametrize("second", sorted(PAIRS) + ["render"])
+def test_threads_that_sort_and_render_on_one_stream_read_their_own_ranking(runtime, first, second):
+    one = [["sort_render", *RANKED, PAIRS[first], A, 0x70]] * 4
+    other = [["render", *RANKED, 200_000, B, 0x70] if second == "render" else ["sort_render", *RANKED, PAIRS[second], B, 0x70]] * 4
+    results, launches = enqueued(runtime, [one, other])
+    assert not any(rc for thread in results for rc, _ in thread)
+    assert len(launches) == 16
+    check_tables(launches)
+
+
+@pytest.mark.parametrize("other", ["sort_render", "render"])
+def test_threads_that_sort_and_render_on_one_stream_read_their_own_long_lists(runtime, other):
+    results, launches = enqueued(runtime, [[["sort_render", *LONG, A, 0x70]] * 6, [[other, *LONG, B, 0x70]] * 6])
+    assert not any(rc for thread in results for rc, _ in thread)
+    assert len(launches) == 24 and len({l["table"] for l in launches}) == 2
+    check_turns(launches)
+
+
+def test_frames_on_different_streams_have_tables_of_their_own(runtime):
+    calls = [[["sort_render", *frame, ranges, stream]] * 3 for stream, ranges in ((0x70, A), (0x80, B)) for frame in (LONG, [*RANKED, 200_000])]
+    results, launches = enqueued(runtime, calls)
+    assert not any(rc for thread in results for rc, _ in thread)
+    tables = {s: {l["table"] for l in launches if l["stream"] == s} for s in (0x70, 0x80)}
+    assert len(launches) == 24 and all(len(t) == 3 for t in tables.values()) and not tables[0x70] & tables[0x80]
+
+
+@pytest.mark.parametrize("why", ["capturing", "no_memory"])
+@pytest.mark.parametrize("frame", [LONG] + [[*RANKED, pairs] for pairs in PAIRS.values()])
+def test_no_table_under_capture_or_without_memory(runtime, why, frame):
+    results, launches = enqueued(runtime, [[["sort_render", *frame, A, 0x70]] * 2], **{why: True})
+    assert not any(rc for rc, _ in results[0])
+    assert [l["kind"] for l in launches] == [BLENDS] * 2 and not any(l["table"] or l["next"] for l in launches)
