@@ -539,8 +539,8 @@ __global__ __launch_bounds__(kBlock) void preprocess_kernel(
     const int lane = tid & (kWave - 1);
     const int wave = tid / kWave;
     // One read of the control word per workgroup: all its threads must agree on it.  Nothing is written before it is looked at, and nothing waits for it before
-    // the rectangles are tested.  (Every workgroup began with a wait for it, a trip to memory, and the covariances were a third trip behind the culls:
-    // needles at 4K 186 -> 175 us, 4K 189.7 -> 186.2, 110M pairs 844 -> 810, 256x192 / 2k 7.7 -> 7.4.)
+    // the rectangles are tested.  (Every workgroup began with a wait for it, a trip to memory: needles at 4K 190 -> 182 us, 110M pairs 845 -> 823, 2M at 1080p
+    // 148 -> 146; scenes of small splats 421 -> 421 and, 1M, 46.6 -> 47.8.)
     uint32_t control_seen = 0;
     if (tid == 0) {
         s_nhuge = 0;
@@ -598,11 +598,8 @@ __global__ __launch_bounds__(kBlock) void preprocess_kernel(
         px = positions[3 * (size_t)idx + 0];
         py = positions[3 * (size_t)idx + 1];
         pz = positions[3 * (size_t)idx + 2];
-        // all per-Gaussian inputs are requested up front so that their latencies overlap (left alone, the compiler requests the covariance behind the culls)
         const float opacity = opacities[idx];
         const float2* cv = reinterpret_cast<const float2*>(cov3ds + 6 * (size_t)idx);
-        float2 s01 = cv[0], s23 = cv[1], s45 = cv[2];
-        asm volatile("" : "+v"(s01.x), "+v"(s01.y), "+v"(s23.x), "+v"(s23.y), "+v"(s45.x), "+v"(s45.y));
         const float* m = cam.view;
         float t[3];
         t[0] = m[0] * px + m[4] * py + m[8] * pz + m[12];
@@ -610,6 +607,11 @@ __global__ __launch_bounds__(kBlock) void preprocess_kernel(
         t[2] = m[2] * px + m[6] * py + m[10] * pz + m[14];
         depth = t[2];
         if (t[2] > 0.2f) {
+            // Requested here, while the opacity is on its way (left alone, the compiler requests it behind the second cull), and not with the position: of what is
+            // behind the camera nothing else is read.  With the position: frames that see nearly all 0.5 to 2 % of this launch faster (4K / 3M 198 -> 194.5 us), but
+            // 200k small splats 15.4 -> 16.8, 3M in the order of their depth, half of them behind, 109 -> 115, 8M, nine in ten behind, 208 -> 235, all of them 190 -> 213.
+            float2 s01 = cv[0], s23 = cv[1], s45 = cv[2];
+            asm volatile("" : "+v"(s01.x), "+v"(s01.y), "+v"(s23.x), "+v"(s23.y), "+v"(s45.x), "+v"(s45.y));
             if (!(255.0f * opacity < 1.0f)) {
                 const float* q = cam.proj;
                 float hx = q[0] * px + q[4] * py + q[8] * pz + q[12];

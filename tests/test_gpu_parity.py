@@ -277,6 +277,37 @@ def test_start_offset_and_capacity_guard(oracle):
     assert np.all(gp.u64(keys)[cap:] == 0) and np.all(values.cpu().numpy()[cap:] == -1)   # nothing past the capacity
 
 
+def test_what_is_behind_the_camera_costs_its_position_and_opacity():
+    """8M Gaussians behind the camera, of which 16 bytes each are read, against as many in front of it and beside the frame, whose covariances (24 bytes)
+    are read too and projected: 0.86 of the time, 0.96 where the covariances of all are read."""
+    import gpu_pipeline as gp
+    import torch
+    from flashgs_amd import cabi
+    P = 8_000_000
+    z = 5.0 + 20.0 * torch.rand(P, device=gp.DEV)
+    opacity = torch.full((P,), 0.5, device=gp.DEV)
+    cov = torch.tensor([1e-4, 0, 0, 1e-4, 0, 1e-4], device=gp.DEV).repeat(P, 1)
+    shs = torch.zeros(P, 48, device=gp.DEV)
+    xy, rgbd, conic = (torch.zeros(P, c, device=gp.DEV) for c in (2, 4, 4))
+    keys, vals = torch.zeros(16, device=gp.DEV, dtype=torch.int64), torch.zeros(16, device=gp.DEV, dtype=torch.int32)
+    off = torch.zeros(1, device=gp.DEV, dtype=torch.int32)
+    places = {"behind": torch.stack([torch.zeros_like(z), torch.zeros_like(z), -z], 1).contiguous(),
+              "beside": torch.stack([torch.full_like(z, 1000.0), torch.zeros_like(z), z], 1).contiguous()}
+    times = {k: [] for k in places}
+    for _ in range(12):
+        for k, position in places.items():
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            cabi.preprocess(P, position.data_ptr(), shs.data_ptr(), opacity.data_ptr(), cov.data_ptr(), 1920, 1080, 16, 16, np.zeros(3, np.float32),
+                            np.eye(3, dtype=np.float32), 1200.0, 1200.0, 100.0, 0.01, xy.data_ptr(), rgbd.data_ptr(), conic.data_ptr(),
+                            keys.data_ptr(), vals.data_ptr(), off.data_ptr(), 16, torch.cuda.current_stream().cuda_stream)
+            b.record()
+            b.synchronize()
+            times[k].append(a.elapsed_time(b))
+    assert int(off.cpu()[0]) == 0
+    assert min(times["behind"]) < 0.91 * min(times["beside"]), {k: min(t) for k, t in times.items()}
+
+
 def test_mirrored_preprocess_stores_the_count_in_pinned_memory():
     """fgs_preprocess_mirrored: the word of pinned host memory receives the pair count the launch
     leaves in *curr_offset (with a starting offset too), everything else is what fgs_preprocess
