@@ -682,6 +682,63 @@ def test_sort_render_is_sort_and_then_render(kind):
         torch.cuda.synchronize()
 
 
+@pytest.mark.parametrize("kind", ["empty", "one pair", "one block", "one block, many tiles", "few tiles", "one pass", "one pass, 32x32",
+                                  "two passes, ranked", "unranked", "long lists", "three passes"])
+def test_a_replayed_sort_render_writes_every_buffer(kind):
+    """Every buffer is filled with something else before each of three replays and compared behind it: sorted keys and values, ranges and both images."""
+    import gpu_pipeline as gp
+    import torch
+    from flashgs_amd import cabi
+    W, H, block, tile, depth, P = _frame_for_sort_render(kind)
+    n, rng = tile.size, np.random.default_rng(4)
+    keys = gp.dev(((tile.astype(np.uint64) << np.uint64(32)) | depth.view(np.uint32).astype(np.uint64)).view(np.int64)) if n else gp.dev(np.zeros(1, np.int64))
+    vals = gp.dev(rng.integers(0, P, max(n, 1)).astype(np.int32))
+    points = [gp.dev((rng.random((P, 2)) * [W, H]).astype(np.float32)), gp.dev(rng.random((P, 4)).astype(np.float32)),
+              gp.dev(np.tile(np.array([-0.01, 0.0, -0.01, -3.0], np.float32), (P, 1)))]
+    bg = np.array([0.2, 0.4, 0.6], np.float32)
+    tiles = ((W + block[0] - 1) // block[0]) * ((H + block[1] - 1) // block[1])
+    size = max(cabi.get_sort_buffer_size(n), 256)
+    space = torch.empty(size, device=gp.DEV, dtype=torch.uint8)
+    buffers = [torch.empty(shape, device=gp.DEV, dtype=dtype) for shape, dtype in
+               (((max(n, 1),), torch.int64), ((max(n, 1),), torch.int32), ((tiles, 2), torch.int32), ((H, W, 3), torch.uint8), ((H, W, 3), torch.float32))]
+    ks, vs, ranges, u8, f32 = buffers
+    written = buffers[2:] if n == 0 else buffers
+
+    def sort(): cabi.sort_gaussian(n, W, H, *block, space.data_ptr(), size, keys.data_ptr(), vals.data_ptr(), ks.data_ptr(), vs.data_ptr(),
+                                   torch.cuda.current_stream().cuda_stream)
+
+    def render(): cabi.render_f32(*block, n, W, H, *[p.data_ptr() for p in points], ks.data_ptr(), vs.data_ptr(), ranges.data_ptr(), bg, u8.data_ptr(),
+                                  f32.data_ptr(), torch.cuda.current_stream().cuda_stream, flags=cabi.BLEND_FP32)
+
+    def both():
+        sort()
+        render()
+
+    def fill(with_what):
+        for t in buffers: t.fill_(with_what)
+
+    fill(7)
+    both()
+    torch.cuda.synchronize()
+    want = [t.clone() for t in written]
+    graph, side = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.graph(graph, stream=side):
+        cabi.sort_render(*block, n, W, H, space.data_ptr(), size, keys.data_ptr(), vals.data_ptr(), ks.data_ptr(), vs.data_ptr(),
+                         *[p.data_ptr() for p in points], ranges.data_ptr(), bg, u8.data_ptr(), f32.data_ptr(),
+                         torch.cuda.current_stream().cuda_stream, flags=cabi.BLEND_FP32)
+    for replay in range(3):
+        fill(11 + replay)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        for w, t in zip(want, written):
+            assert torch.equal(w, t), "replay %d" % replay
+        fill(3)
+        both()                                  # eager work in between
+        torch.cuda.synchronize()
+
+
 @pytest.mark.parametrize("block", [(16, 16), (32, 16), (32, 32)])
 def test_blends_replayed_beside_each_other(block):
     """Blends hold no table of the library's in a captured graph: graphs of two frame sizes, replayed side
