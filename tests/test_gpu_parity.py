@@ -1066,6 +1066,66 @@ def test_long_lists_of_large_frames_start_first(W, H, block, long_lists, fewest,
         assert torch.equal(listed, out)
 
 
+def _lists_around_the_places_of_a_shard(rng, T, shard):
+    places = rng.permutation(T)
+    crowded = np.concatenate([places[shard(places) == k][:many] for k, many in ((0, 40), (5, 16), (6, 17), (8, 31), (13, 32), (20, 33), (31, 64))])
+    return crowded, lambda least: least + 65 + np.arange(crowded.size) * 5
+
+
+@pytest.mark.parametrize("W,H,block", [(4096, 4111, (16, 16)), (8200, 4096, (32, 16)), (8192, 8223, (32, 32))])
+@pytest.mark.parametrize("flags", ["fp32", "f16"])
+def test_long_lists_behind_the_sort_start_first(W, H, block, flags):
+    """fgs_sort_render uses all 32 places of a shard, fgs_render 16 of the same tables: shards with 16, 17, 31, 32, 33 and more long lists, frames of either in turn
+    on a stream of its own, against fgs_blend, which lists none, bit for bit."""
+    import gpu_pipeline as gp
+    from flashgs_amd import cabi
+    import torch
+    bg = np.array([0.2, 0.4, 0.6], np.float32)
+    flags = {"fp32": cabi.BLEND_FP32, "f16": cabi.BLEND_MATRIX_F16}[flags]
+    stream = _fresh_stream()
+    st = stream.cuda_stream
+    for seed in range(2):
+        K, (xy, rgbd, co, keys, vals), ranges_of, n, in_shard = _long_lists_frame(W, H, block, _lists_around_the_places_of_a_shard, 7 * seed + block[1])
+        assert list(in_shard[[0, 5, 6, 8, 13, 20, 31]]) == [40, 16, 17, 31, 32, 33, 64] and in_shard.sum() == 233
+        T, size = n.size, cabi.get_sort_buffer_size(K)
+        place = torch.randperm(K, device=gp.DEV)
+        keys, vals = keys[place], vals[place]                   # (stable: the order of a tile's list, at one depth)
+        space = torch.empty(size, device=gp.DEV, dtype=torch.uint8)
+        ks, vs = torch.empty_like(keys), torch.empty_like(vals)
+        ranges = torch.empty((T, 2), device=gp.DEV, dtype=torch.int32)
+        image = torch.empty((H, W, 3), device=gp.DEV, dtype=torch.float32)
+        torch.cuda.synchronize()
+
+        def clear():
+            for t in (ks, vs, ranges): t.fill_(-1)
+            image.fill_(-1.0)
+            torch.cuda.synchronize()
+
+        def sort(): cabi.sort_gaussian(K, W, H, *block, space.data_ptr(), size, keys.data_ptr(), vals.data_ptr(), ks.data_ptr(), vs.data_ptr(), st)
+
+        clear()
+        with torch.cuda.stream(stream):
+            sort()
+            cabi.tile_ranges(*block, K, W, H, ks.data_ptr(), ranges.data_ptr(), st)
+            cabi.blend(*block, W, H, xy.data_ptr(), rgbd.data_ptr(), co.data_ptr(), vs.data_ptr(), ranges.data_ptr(), bg, 0, image.data_ptr(), st, flags=flags)
+        torch.cuda.synchronize()
+        want = [t.clone() for t in (ks, vs, ranges, image)]
+        assert np.array_equal(ranges.cpu().numpy()[n > 0], ranges_of[n > 0])
+        for how in ("one", "one", "both", "one", "both", "both", "one"):
+            clear()
+            with torch.cuda.stream(stream):
+                if how == "one":
+                    cabi.sort_render(*block, K, W, H, space.data_ptr(), size, keys.data_ptr(), vals.data_ptr(), ks.data_ptr(), vs.data_ptr(), xy.data_ptr(),
+                                     rgbd.data_ptr(), co.data_ptr(), ranges.data_ptr(), bg, None, image.data_ptr(), st, flags=flags)
+                else:
+                    sort()
+                    cabi.render_f32(*block, K, W, H, xy.data_ptr(), rgbd.data_ptr(), co.data_ptr(), ks.data_ptr(), vs.data_ptr(), ranges.data_ptr(), bg,
+                                    None, image.data_ptr(), st, flags=flags)
+            torch.cuda.synchronize()
+            for w, t in zip(want, (ks, vs, ranges, image)):
+                assert torch.equal(w, t), how
+
+
 def test_a_long_list_of_the_last_tile_starts_first():
     """300 entries in 65 792 tiles and some 6000, never opaque, in the last three: fgs_render starts those with the first workgroups, fgs_blend,
     which lists none, with the last ones, behind which they are walked alone."""
