@@ -767,12 +767,17 @@ __global__ __launch_bounds__(Shape::kThreads) void scatter_kernel(
 // (Instead of the two passes in LDS, pairs that put their places down by tile and count the smaller ones there, words written from
 // registers in any order: the scatter 21 -> 28 us, 12 -> 18 where some tiles are crowded.  Counters in memory in place of the rows, by atomic additions
 // of a block's counts and of bases taken from them: 0.4M and 1.7M pairs 17 and 45 us in all for 20 and 34, and an order to be mended behind it.)
-// Rows and offsets stand in the space of the copy that longer segments go through later, or behind what the sort needs if there is more.
+// With few ids the rows are many, and it still pays at the longest list that has any: 300 tiles 20M pairs 1574 -> 1520 us, 60M 4982 -> 4677 (14 649 rows of 512), 1000 tiles
+// 16.5M 806 -> 748, 2048 tiles 16M 376 -> 373, 3600 tiles 8.3M 200 -> 181.
+// Rows and offsets stand in the space of the copy that longer segments go through later, or, where that is too small, behind what the sort needs, in whatever more
+// space the caller has passed (with neither, larger blocks or two passes: see kOnePassShort).
 constexpr int kOnePassBits = 13, kOnePassIds = 1 << kOnePassBits, kOnePassLeastBits = 9;
 constexpr int kOnePassThreads = 1024, kOnePassWaves = kOnePassThreads / kWave;
 constexpr int kOnePassLow = 7;                  // bits of the tile id that the first sort of a block takes
 // Blocks of 2048 pairs up to this many pairs, of 4096 above: 3600 tiles 0.2M pairs 25 and 28 us, 0.8M 50 and 48; 8160 tiles 0.2M 26 and 28, 0.4M 32 and 31, 1.6M 73 and 62.
 // (Of 8192: 0.2M 33, 1.7M 1 % more.)
+// The rows of blocks of 2048 pairs and 8192 ids are 24 bytes a pair, twice the copy: a caller with no space to spare has blocks of 4096 there.  5700 tiles, 0.1M pairs: 23.3
+// us, 26.0 without, 27.1 by two passes; 8160 tiles 24.7, 27.5, 28.3; 0.4M 30.8, 30.7, 33.5.  With 4096 ids there is room as it is.
 constexpr int kOnePassShort = 1 << 19;
 constexpr size_t kOnePassCells = (size_t)1 << 23;       // the most cells of rows: 4.2M pairs with 8192 ids, 8.4M with 4096
 

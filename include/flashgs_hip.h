@@ -141,7 +141,9 @@ int fgs_wait_count(const int* count_mirror, double timeout_seconds, int* count);
  * stable ascending sort of num_rendered (key, value) pairs on key bits
  * [0, 32 + bit_length(tiles_x * tiles_y)).  Inputs are left untouched.
  * list_sorting_space must hold at least fgs_get_sort_buffer_size(num_rendered) bytes and be
- * 256-byte aligned.
+ * 256-byte aligned.  All of its sorting_size bytes are scratch: what there is beyond that least size may be written too, and lists
+ * of some 100 000 pairs in frames of 4096 to 8191 tiles are sorted up to a tenth faster where there is twice as much (as with a space
+ * sized for the most pairs that a caller expects).  The result does not depend on it.
  */
 int fgs_sort_gaussian(int num_rendered,
                       int width, int height, int block_x, int block_y,
@@ -170,7 +172,7 @@ size_t fgs_get_sort_buffer_size(int num_rendered);
  * A frame of at most 8192 tiles first ranks its tiles by list length into a table the library keeps per
  * (device, stream) (41 KB, allocated on the first call on that stream that uses it); fgs_render_* leaves the ranking out where
  * the frame is so small that all its workgroups are resident at once, and lists the long lists of a frame of 65536 tiles and 3 * 2^20 pairs or more
- * in the same memory, so that they are blended first.  Lists that are long for the frame are blended in
+ * in the same memory, so that they are blended first (fgs_sort_render does either with the launches of its sort).  Lists that are long for the frame are blended in
  * runs by several waves and folded front to back.  The run that holds the stop of render.cu:394-408 is walked again
  * pair by pair behind what precedes it, and so is one with weights above 1 in it or behind a transmittance that
  * such weights took out of 0 to 1, so the walk ends where the reference's does.  From which length on a list is cut
@@ -210,6 +212,7 @@ int fgs_render_f32(int block_x, int block_y, int num_rendered, int width, int he
  * No counterpart in the reference: fgs_sort_gaussian and then fgs_render_ex of one frame in one call, with the same arguments and the
  * same results in every buffer, for keys as fgs_preprocess makes them (no bits set above the sorted range).  What the blend
  * needs to know of the tiles is written by the launches of the sort, so there are up to two launches less.
+ * A call that is refused asks the runtime for nothing and launches nothing.
  */
 int fgs_sort_render(int block_x, int block_y, int num_rendered, int width, int height,
                     char* list_sorting_space, size_t sorting_size,
@@ -270,8 +273,8 @@ int fgs_blend_ex(int block_x, int block_y, int width, int height,
 /*
  * No counterpart in the reference.  Name of the kernel(s) fgs_blend(_ex) launches with these flags for this
  * tile and frame size outside stream capture (frames of at most 8192 tiles have their tiles ranked
- * first, by tile_order_kernel, which fgs_render_* leaves out where all workgroups are resident at once), as a
- * profiler lists them; "" for an unsupported tile size or unknown flags.  Lets a
+ * first, by tile_order_kernel, which fgs_render_* leaves out where all workgroups are resident at once, and fgs_sort_render
+ * there and where a launch of its sort has ranked them), as a profiler lists them; "" for an unsupported tile size or unknown flags.  Lets a
  * benchmark attribute its figures to the kernel that ran.
  */
 const char* fgs_blend_kernel_name(int block_x, int block_y, int width, int height, int flags);

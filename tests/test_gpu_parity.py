@@ -1918,6 +1918,18 @@ def test_sort_by_the_whole_tile_id(W, H, n, crowd, spare):
     _sort_case(tile.astype(np.uint32), depth, W, H, junk, seed=n % 97, space_for=max(n, 1 << 24) if spare else None)
 
 
+@pytest.mark.parametrize("W,H,n", [(400, 300, 20_000_003), (1280, 720, 1 << 23), (1280, 720, (1 << 23) + 1)])
+def test_sort_by_the_whole_tile_id_of_few_tiles_and_many_pairs(W, H, n):
+    """512 ids with 4883 rows, of which a workgroup of the offsets launch walks 153 a thread, and the longest list that has rows with 4096 ids, and one pair more."""
+    rng = np.random.default_rng(n % 1013)
+    tiles = ((W + 15) // 16) * ((H + 15) // 16)
+    tile = rng.integers(0, tiles, n, dtype=np.uint32)
+    tile[n // 3: n // 2] = tile[n // 3: n // 2] // 8 * 8        # some tiles with more
+    depth = rng.integers(0, 1 << 31, n, dtype=np.uint32)
+    depth[::5] = depth[n // 2]
+    _sort_case(tile, depth, W, H, None, seed=n % 97, ascending=True, space_for=1 << 25)
+
+
 def test_sort_bits_above_the_range_stay_with_their_pair():
     """Bits above 32 + bit_length(tiles) are outside the sorted range (sort.cu:34-39) but travel
     with the key."""
