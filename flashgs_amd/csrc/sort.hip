@@ -1978,7 +1978,8 @@ __global__ __launch_bounds__(kWaves * kWave) __attribute__((amdgpu_waves_per_eu(
 
 // One wave per workgroup: it sorts the segments of up to 64*kT pairs of one tile id or of several, a grid apart.  Their bounds come from
 // the table of segment starts or, without one, from a search.
-template <int kT, bool kWords>
+// kNotes: writes what it finds of the tiles too.  (Compiled apart: a sort by itself does not pay for the question, 8K frame 0.1M pairs 57.5 -> 56.2 us, 0.4M 80.4 -> 79.4.)
+template <int kT, bool kWords, bool kNotes>
 __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(7))) void segment_sort_wave_kernel(
     Lists lists, int n, uint32_t tile_mask, const int* __restrict__ seg_start,
     int list_max0, int list_max1, int list_max2,
@@ -1999,7 +2000,7 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(7))) void
             // (lengths up to list_max0, list_max1, list_max2, and everything longer), so that those
             // fewer, longer-running segments can be dealt out evenly by the launches that follow.
             const int len = hi - lo;
-            if (kWords && threadIdx.x == 0) note_tile(notes, v, lo, hi);
+            if (kNotes && threadIdx.x == 0) note_tile(notes, v, lo, hi);
             if (len > kT * kWave && threadIdx.x == 0) {
                 // neighbouring tiles tend to be equally busy: mix the index so that every list gets its share
                 const uint32_t shard = (v ^ (v >> 5) ^ (v >> 10) ^ (v >> 15)) % kListShards;
@@ -2369,8 +2370,8 @@ int sort_impl(int num_rendered, int width, int height, int block_x, int block_y,
         const unsigned g = most < limit ? most : limit;
         return (g + kListShards - 1) / kListShards * kListShards;
     };
-#define FGS_SEGMENT_WAVE(CAP, WORDS)                                                                          \
-    hipLaunchKernelGGL((segment_sort_wave_kernel<(CAP) / kWave, WORDS>), dim3((ids + ids_per_wave - 1) / ids_per_wave), dim3(kWave),              \
+#define FGS_SEGMENT_WAVE(CAP, WORDS, NOTES)                                                                   \
+    hipLaunchKernelGGL((segment_sort_wave_kernel<(CAP) / kWave, WORDS, NOTES>), dim3((ids + ids_per_wave - 1) / ids_per_wave), dim3(kWave),              \
                        0, st, lists, n, tile_mask, (const int*)seg_start,                                     \
                        kCapSmall, kCapMedium, kCapLarge, seg_counts, list_small, list_medium,                 \
                        list_large, list_long, cap_small, cap_medium, cap_large, cap_long, tables.notes)
@@ -2407,7 +2408,8 @@ int sort_impl(int num_rendered, int width, int height, int block_x, int block_y,
         // of the launch).  The launch also lists the longer segments.  Segments of 513..1024 pairs in a launch of
         // their own last as long as one such sort on a frame of few tiles, which has about one per SIMD (1080p: -15 us, 4K:
         // -8 us, 8K -12 us without it, and -0.28 ms on the 8K frame of 109M pairs).
-        FGS_SEGMENT_WAVE(kCapSmall, true);
+        if (tables.notes.ranges) FGS_SEGMENT_WAVE(kCapSmall, true, true);
+        else FGS_SEGMENT_WAVE(kCapSmall, true, false);
         if (n > kCapSmall && !merged_tail) {
             FGS_SEGMENT_CLASS(4, kCapMedium, 8, true, kCapSmall, medium_blocks, list_medium, seg_counts + kListShards, cap_medium);
             if (n > kCapMedium && !merged_large)
@@ -2416,7 +2418,7 @@ int sort_impl(int num_rendered, int width, int height, int block_x, int block_y,
         // longer segments from their list, one workgroup per segment
         if (tail_blocks) FGS_SEGMENT_GENERAL(true, true, tail_blocks, first_class);
     } else {
-        FGS_SEGMENT_WAVE(kCapTiny, false);
+        FGS_SEGMENT_WAVE(kCapTiny, false, false);
         if (seg_start) {
             if (n > kCapTiny)       // 513..1024: the same network over 16 register slots, from the lists
                 hipLaunchKernelGGL((segment_sort_wave_list_kernel<kCapSmall / kWave, false>),

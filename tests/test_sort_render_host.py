@@ -29,7 +29,7 @@ enum { kRanks = 1, kLists = 2, kBlends = 3 };
 
 static struct { const void *function; char name[160]; } kernels[512];
 static Launch launches[1024];
-static int kernel_count, count, capturing, no_memory, failing, asked;
+static int kernel_count, launched[512], count, capturing, no_memory, failing, asked;
 static pthread_mutex_t lock = PTHREAD_MUTEX_INITIALIZER;
 static __thread dim3 pushed_grid, pushed_block;
 static __thread void *pushed_stream;
@@ -72,8 +72,12 @@ int hipLaunchKernel(const void *function, dim3 grid, dim3 block, void **args, si
 {
     (void)grid; (void)block; (void)lds;
     const char *name = "";
-    for (int i = 0; i < kernel_count; i++) if (kernels[i].function == function) name = kernels[i].name;
     if (failing) return 1;
+    for (int i = 0; i < kernel_count; i++) {
+        if (kernels[i].function != function) continue;
+        name = kernels[i].name;
+        __sync_fetch_and_add(&launched[i], 1);
+    }
     Launch l = { 0, (size_t)stream, 0, 0, 0 };
     if (strstr(name, "tile_scatter_kernel")) {                  /* (TileRanking) */
         l.kind = kRanks; l.table = *(size_t *)args[9];
@@ -101,6 +105,12 @@ int hipLaunchKernel(const void *function, dim3 grid, dim3 block, void **args, si
 void stand_in_set(int is_capturing, int is_out_of_memory) { capturing = is_capturing; no_memory = is_out_of_memory; }
 void stand_in_fail(void) { failing = 1; }
 int stand_in_asked(void) { const int n = asked; asked = 0; return n; }
+int stand_in_launches_of(const char *part)
+{
+    int n = 0;
+    for (int i = 0; i < kernel_count; i++) if (strstr(kernels[i].name, part)) n += launched[i];
+    return n;
+}
 int stand_in_launches(Launch *out)
 {
     pthread_mutex_lock(&lock);
@@ -122,6 +132,7 @@ hip = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)         # in front of the runtime 
 lib = C.CDLL(sys.argv[2])
 threads_of, capturing, no_memory = json.loads(sys.argv[3]), int(sys.argv[4]), int(sys.argv[5])
 lib.fgs_sort_render.argtypes = [C.c_int] * 5 + [C.c_void_p, C.c_size_t] + [C.c_void_p] * 11 + [C.c_int, C.c_void_p]
+lib.fgs_sort_gaussian.argtypes = [C.c_int] * 5 + [C.c_void_p, C.c_size_t] + [C.c_void_p] * 5
 lib.fgs_render_f32.argtypes = [C.c_int] * 5 + [C.c_void_p] * 10
 lib.fgs_get_sort_buffer_size.restype = C.c_size_t
 lib.fgs_last_error.restype = C.c_char_p
@@ -135,7 +146,9 @@ def frames(mine, calls):
         hip.stand_in_asked()
         room = lib.fgs_get_sort_buffer_size(pairs)
         if how.endswith("fails"): hip.stand_in_fail()             # up to the first time that the library looks
-        if how.startswith("render"):
+        if how == "sort":
+            rc = lib.fgs_sort_gaussian(pairs, w, h, bx, by, 256, room, 256, 256, 256, 256, stream)
+        elif how.startswith("render"):
             rc = lib.fgs_render_f32(bx, by, pairs, w, h, 256, 256, 256, 256 + 4 * (how == "render misaligned keys"), 256, ranges, C.addressof(bg),
                                     None if how == "render without image" else 256, None, stream)
         else:
@@ -150,7 +163,8 @@ for t in threads: t.start()
 for t in threads: t.join()
 found = (Launch * 1024)()
 n = hip.stand_in_launches(found)
-print(json.dumps({"results": results, "launches": [{f: getattr(l, f) for f, _ in Launch._fields_} for l in found[:n]]}))
+noting, plain = (hip.stand_in_launches_of(b"segment_sort_wave_kernelILi16ELb1ELb%dEE" % notes) for notes in (1, 0))
+print(json.dumps({"noting": noting, "plain": plain, "results": results, "launches": [{f: getattr(l, f) for f, _ in Launch._fields_} for l in found[:n]]}))
 """
 
 RANKS, LISTS, BLENDS = 1, 2, 3
@@ -168,13 +182,16 @@ def runtime(tmp_path_factory):
     return str(library)
 
 
-def enqueued(runtime, threads, capturing=False, no_memory=False):
+def enqueued(runtime, threads, capturing=False, no_memory=False, count_segments=False):
     """(status and calls of the runtime, but for launches, of every frame; launches that write or read a table) of threads
-    that each make frames (how, bx, by, width, height, pairs, ranges, stream)."""
+    that each make frames (how, bx, by, width, height, pairs, ranges, stream).  count_segments: how often the first segment launch was the one
+    that writes ranges and lists, and how often the one that does not."""
     done = subprocess.run([sys.executable, "-c", PROGRAM, runtime, cabi.LIB_PATH, json.dumps(threads), str(int(capturing)),
                            str(int(no_memory))], capture_output=True, text=True, timeout=120, cwd=ROOT)
     assert done.returncode == 0, done.stderr[-2000:]
     found = json.loads(done.stdout.splitlines()[-1])
+    if count_segments:
+        return found["noting"], found["plain"]
     return found["results"], found["launches"]
 
 
@@ -267,3 +284,9 @@ def test_no_table_under_capture_or_without_memory(runtime, why, frame):
     results, launches = enqueued(runtime, [[["sort_render", *frame, A, 0x70]] * 2], **{why: True})
     assert not any(rc for rc, _ in results[0])
     assert [l["kind"] for l in launches] == [BLENDS] * 2 and not any(l["table"] or l["next"] for l in launches)
+
+
+@pytest.mark.parametrize("frame", [LONG, [16, 16, 1920, 1080, 200_000], [16, 16, 7680, 4320, 100_000]])
+def test_a_sort_by_itself_does_not_pay_for_the_ranges(runtime, frame):
+    """... and the call that needs them has the launch that writes them."""
+    assert enqueued(runtime, [[["sort", *frame, A, 0x70]] * 3 + [["sort_render", *frame, A, 0x70]] * 2], count_segments=True) == (2, 3)
