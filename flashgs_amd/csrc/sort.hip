@@ -759,8 +759,8 @@ __global__ __launch_bounds__(Shape::kThreads) void scatter_kernel(
 // a row of counts per block, 16 bits for every tile id, `tile_offsets_kernel` turns every column of the rows into what the blocks in front
 // hold of that tile, and `tile_scatter_kernel` sorts its block by tile id in LDS (two stable passes, seven bits first) and writes every pair's
 // word to its place.  The pairs travel once and there are three launches, where two passes of 8 bits take four to six, each of which lasts 3 to 14 us on
-// such a list whatever it moves: 3 + 4 + 8 us for 22 in all on 0.2M pairs of a 720p frame, 5 + 8 + 21 for 52 on 1.7M of a 1080p frame (that one reads 35 MB, of which
-// 14 are offsets, and writes 14 in runs of one or two pairs).  The whole sort, two passes -> one: 3600 tiles 0.1M pairs 27 -> 22 us, 0.4M 41 -> 35,
+// such a list whatever it moves: 3 + 4 + 8 us for 22 in all on 0.2M pairs of a 720p frame, 5 + 8 + 21 for 52 on 1.7M of a 1080p frame (that one reads 36 MB, of which
+// 14 are offsets, and writes 16 for 14 in runs of one or two pairs).  The whole sort, two passes -> one: 3600 tiles 0.1M pairs 27 -> 22 us, 0.4M 41 -> 35,
 // 1.6M 97 -> 77, 6.4M 275 -> 255; 8160 tiles 0.1M 28 -> 25, 0.8M 59 -> 48, 1.6M 78 -> 62, 3.2M 121 -> 113; 300 tiles 25k 27 -> 22, 0.8M 117 -> 96.
 // A block's rows cost 6 bytes per tile id, so it stops paying where blocks x ids do: 8160 tiles 6.4M pairs 170 -> 180 us, 14 400 tiles 0.2M 32 -> 34, 0.8M
 // 53 -> 48, 3.2M 100 -> 133.
